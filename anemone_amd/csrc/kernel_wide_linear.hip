@@ -23,6 +23,18 @@
 
 #include "wide_device.cuh"
 #include "wide_finish_device.cuh"
+#include "wide_order_device.cuh"
+
+/* The tile's pairs in LDS for the finish, each wavefront's sixteen from a lane's registers, once the stages are done
+ * with: the window is all of a third of a CU's LDS (42 of its units of 1,280 bytes), so that there is no room beside it.
+ * The whole block calls. */
+__device__ static __forceinline__ const struct wide_pair *wide_columns_in(unsigned char *window, uint32_t column, const struct wide_pair &pair)
+{
+    __syncthreads();
+    ((struct wide_pair *)window)[column] = pair;
+    __syncthreads();
+    return (const struct wide_pair *)window;
+}
 
 /* grid (ceil(output_size / (4 strips)), tile_count), block 256; a strip is STRIP tiles of gate and STRIP of up */
 template <bool BYTES, uint32_t STRIP, uint32_t DEPTH, bool B128 = false>
@@ -32,26 +44,28 @@ __device__ static __forceinline__ void wide_expert_gate_up(const struct wide_exp
     constexpr uint32_t TILES = chain_type::TILES, STRIP_OUTPUTS = STRIP * 16u;
     static_assert(STRIP == 1u || STRIP == 2u, "a quantizer block of 32 outputs is one strip or two");
     extern __shared__ __attribute__((aligned(16))) unsigned char window[];
-    const struct wide_expert_tile tile = ((const struct wide_expert_tile *)(arena + arguments.tiles_offset))[blockIdx.y];
-    if (tile.pair_count == 0u) {
+    const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    struct wide_expert_tile tile;
+    uint32_t pair_count = 0, block_strip = 0;
+    if (!order_block_of<1u, false, !BYTES>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count)) {
         return;
     }
-    const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const struct wide_pair *pairs = (const struct wide_pair *)(arena + arguments.pairs_offset) + tile.first_pair;
     /* columns past the tile's last pair read its first pair's vector; their sums are never stored */
     uint32_t code_vectors[2];
 #pragma unroll
     for (uint32_t part = 0; part < 2u; part++) {
         const uint32_t column = 8u * (2u * wave + part) + lane / 8u;
-        code_vectors[part] = pairs[column < tile.pair_count ? column : 0u].pair_index / arguments.pairs_per_row;
+        code_vectors[part] = pairs[column < pair_count ? column : 0u].pair_index / arguments.pairs_per_row;
     }
     const uint32_t scale_column = 16u * wave + lane % 16u;
-    const uint32_t exponent_vector = pairs[scale_column < tile.pair_count ? scale_column : 0u].pair_index / arguments.pairs_per_row;
+    const struct wide_pair scale_pair = pairs[scale_column < pair_count ? scale_column : 0u];
+    const uint32_t exponent_vector = scale_pair.pair_index / arguments.pairs_per_row;
     chain_type chain_of;
     const unsigned char *const matrices[2] = {arena + tile.gate_offset, arena + tile.up_offset};
     const uint32_t window_address = (uint32_t)(uintptr_t)(lds_pointer)window;
     uint32_t tile0 = 0;
-    chain_of.place(matrices, arguments.output_size, arguments.input_size, blockIdx.x, arena + arguments.codes_offset,
+    chain_of.place(matrices, arguments.output_size, arguments.input_size, block_strip, arena + arguments.codes_offset,
                    arena + arguments.exponents_offset, code_vectors, exponent_vector, window_address, wave, lane, tile0);
     float4_t chain[TILES][WIDE_COLUMN_BLOCKS];
 #pragma unroll
@@ -61,9 +75,10 @@ __device__ static __forceinline__ void wide_expert_gate_up(const struct wide_exp
             chain[t][j] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
         }
     }
-    const uint32_t live_blocks = (tile.pair_count + 15u) / 16u;
+    const uint32_t live_blocks = (pair_count + 15u) / 16u;
     chain_of.whole(arguments.input_size / 128u, live_blocks, chain);
-    wide_gate_up_finish<STRIP, WIDE_COLUMN_BLOCKS, B128>(arguments, arena, window, pairs, tile.pair_count, blockIdx.x, tile0, wave, lane, chain);
+    const struct wide_pair *columns = wide_columns_in(window, scale_column, scale_pair);
+    wide_gate_up_finish<STRIP, WIDE_COLUMN_BLOCKS, B128>(arguments, arena, window + WIDE_TILE_PAIRS * sizeof(struct wide_pair), columns, pair_count, block_strip, tile0, wave, lane, chain);
 }
 
 template <bool BYTES, bool B128 = false>
@@ -72,24 +87,28 @@ __device__ static __forceinline__ void wide_expert_down(const struct wide_expert
     typedef wide_chain<1, BYTES, (BYTES ? 2u : 4u), 2u, B128> chain_type;
     constexpr uint32_t TILES = chain_type::TILES, STRIP = chain_type::STRIP, STRIP_OUTPUTS = STRIP * 16u;
     extern __shared__ __attribute__((aligned(16))) unsigned char window[];
-    const struct wide_expert_tile tile = ((const struct wide_expert_tile *)(arena + arguments.tiles_offset))[blockIdx.y];
-    if (tile.pair_count == 0u) {
+    __shared__ struct wide_pair columns[WIDE_TILE_PAIRS]; /* beside the window: 41 of a CU's 128 units of LDS with it */
+    const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    struct wide_expert_tile tile;
+    uint32_t pair_count = 0, block_strip = 0;
+    if (!order_block_of<1u, true, !BYTES>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count)) {
         return;
     }
-    const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const struct wide_pair *pairs = (const struct wide_pair *)(arena + arguments.pairs_offset) + tile.first_pair;
     uint32_t code_vectors[2]; /* the vectors are the pairs' hidden vectors */
 #pragma unroll
     for (uint32_t part = 0; part < 2u; part++) {
         const uint32_t column = 8u * (2u * wave + part) + lane / 8u;
-        code_vectors[part] = pairs[column < tile.pair_count ? column : 0u].pair_index;
+        code_vectors[part] = pairs[column < pair_count ? column : 0u].pair_index;
     }
     const uint32_t scale_column = 16u * wave + lane % 16u;
-    const uint32_t exponent_vector = pairs[scale_column < tile.pair_count ? scale_column : 0u].pair_index;
+    const struct wide_pair scale_pair = pairs[scale_column < pair_count ? scale_column : 0u];
+    const uint32_t exponent_vector = scale_pair.pair_index;
+    columns[scale_column] = scale_pair; /* for the finish, behind the chain's barriers */
     chain_type chain_of;
     const unsigned char *const matrices[1] = {arena + tile.down_offset};
     uint32_t tile0 = 0;
-    chain_of.place(matrices, arguments.output_size, arguments.input_size, blockIdx.x, arena + arguments.codes_offset,
+    chain_of.place(matrices, arguments.output_size, arguments.input_size, block_strip, arena + arguments.codes_offset,
                    arena + arguments.exponents_offset, code_vectors, exponent_vector, (uint32_t)(uintptr_t)(lds_pointer)window, wave, lane, tile0);
     float4_t chain[TILES][WIDE_COLUMN_BLOCKS];
 #pragma unroll
@@ -99,8 +118,8 @@ __device__ static __forceinline__ void wide_expert_down(const struct wide_expert
             chain[t][j] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
         }
     }
-    chain_of.whole(arguments.input_size / 128u, (tile.pair_count + 15u) / 16u, chain);
-    wide_down_finish<STRIP, WIDE_COLUMN_BLOCKS>(arguments, arena, pairs, tile.pair_count, blockIdx.x, tile0, wave, lane, chain);
+    chain_of.whole(arguments.input_size / 128u, (pair_count + 15u) / 16u, chain);
+    wide_down_finish<STRIP, WIDE_COLUMN_BLOCKS>(arguments, arena, columns, pair_count, block_strip, tile0, wave, lane, chain);
 }
 
 /* wide_expert_gate_up_1, wide_expert_down_1: the reference's entries, of WEIGHT_FORMAT_E2M1_SCALED experts; the _e4m3_

@@ -94,9 +94,11 @@ struct native_chain {
     /* scale codes: of one-byte weights a byte a lane a tile (a row of 32 outputs' codes, as the reference stores them); of
      * 4-bit weights a word a lane a matrix: its bytes are the codes of the lane's row and inputs in the four tiles of a group
      * of 64 outputs, which the matrix instruction picks by number */
-    static constexpr uint32_t SCALE_LOADS = BYTES && !B128 ? TILES : MATRICES;
+    static constexpr uint32_t GROUP_TILES = STRIP < 4u ? STRIP : 4u; /* tiles of a strip that share a word of 4-bit weights' codes */
+    static constexpr uint32_t GROUPS = BYTES ? 1u : STRIP / GROUP_TILES;
+    static constexpr uint32_t SCALE_LOADS = BYTES && !B128 ? TILES : MATRICES * GROUPS;
     static constexpr uint32_t WEIGHT_LOADS = TILES * HALVES + SCALE_LOADS;
-    static_assert(BYTES || STRIP == 2u || STRIP == 4u, "a strip of 4-bit weights is half a group of four tiles, or a whole one");
+    static_assert(BYTES || STRIP == 2u || STRIP % 4u == 0u, "a strip of 4-bit weights is half a group of four tiles, or whole ones");
     static_assert((DEPTH - 1u) * VECTOR_LOADS + (SLOTS - 1u) * WEIGHT_LOADS < 64u, "vmcnt has six bits");
 
     struct slot {
@@ -105,8 +107,8 @@ struct native_chain {
     };
 
     const unsigned char *words[MATRICES], *scales[MATRICES], *codes, *exponents;
-    uint32_t step_stride; /* from a tile's K step to its next */
-    uint32_t window, wave, word_offset[STRIP], scale_offset[STRIP], codes_offset[WAVE_BLOCKS][2], exponents_offset;
+    uint32_t step_stride, scale_stride; /* from a tile's K step to its next; from a group's scale words to the next group's */
+    uint32_t window, wave, tile_bytes, group_bytes, word_offset, scale_offset[BYTES && !B128 ? STRIP : 1], codes_offset[WAVE_BLOCKS][2], exponents_offset;
     uint32_t vector_at[BYTES ? 8 : 4], vector_scale_at, operand_at, scale_shift;
     bool scale_lane;
 
@@ -146,9 +148,11 @@ struct native_chain {
             const unsigned char *step_words = words[m] + (uint64_t)at * step_stride;
 #pragma unroll
             for (uint32_t n = 0; n < STRIP; n++) {
-                load_16<BYTES>(into.words[m * STRIP + n][0], step_words, word_offset[n]);
+                /* the tile's place is scalar: one register of lane offsets serves every tile */
+                const unsigned char *tile_words = step_words + n / 4u * group_bytes + n % 4u * tile_bytes;
+                load_16<BYTES>(into.words[m * STRIP + n][0], tile_words, word_offset);
                 if constexpr (BYTES) {
-                    load_16_second<BYTES>(into.words[m * STRIP + n][1], step_words, word_offset[n]);
+                    load_16_second<BYTES>(into.words[m * STRIP + n][1], tile_words, word_offset);
                 }
             }
         }
@@ -161,7 +165,10 @@ struct native_chain {
                     load_1(into.scale[m * STRIP + n], step_scales, scale_offset[n]);
                 }
             } else { /* a word a lane of a group of four tiles' codes, or the strip's one float32 scale in every lane */
-                load_4(into.scale[m], step_scales, scale_offset[0]);
+#pragma unroll
+                for (uint32_t group = 0; group < GROUPS; group++) {
+                    load_4(into.scale[m * GROUPS + group], step_scales + group * scale_stride, scale_offset[0]);
+                }
             }
         }
     }
@@ -232,7 +239,7 @@ struct native_chain {
         } else {
             const uint4_t w = set.words[T][0];
             const int8_vector a = {(int)w.x, (int)w.y, (int)w.z, (int)w.w, 0, 0, 0, 0};
-            chain[T][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, chain[T][j], 4, 0, T % STRIP, (int)scale_a[T / STRIP], 0, (int)scale_b);
+            chain[T][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, chain[T][j], 4, 0, T % GROUP_TILES, (int)scale_a[T / GROUP_TILES], 0, (int)scale_b);
         }
         if constexpr (T + 1u < TILES) {
             multiply_tiles<T + 1u>(set, scale_a, b, scale_b, j, chain);
@@ -409,9 +416,12 @@ struct native_chain {
         const uint32_t o = lane % 16u, g = lane / 16u;
         const uint32_t strip = block_strip * NATIVE_WAVES + wave_index;
         /* a strip that reaches past the last tile reads the last tiles again; its surplus sums are not stored */
-        const uint32_t tile0 = strip * STRIP + STRIP <= tiles ? strip * STRIP : tiles - STRIP;
+        const uint32_t tile0 = strip * STRIP + STRIP <= tiles ? strip * STRIP : tiles > STRIP ? tiles - STRIP : 0u;
         tile0_out = tile0;
-        const uint32_t tile_bytes = steps * STEP_BYTES;
+        tile_bytes = steps * STEP_BYTES;
+        /* a matrix of one group of four tiles under strips of two groups: the second reads the first again */
+        group_bytes = STRIP > 4u && tiles < STRIP ? 0u : 4u * tile_bytes;
+        scale_stride = STRIP > 4u && tiles < STRIP ? 0u : steps * 256u;
         step_stride = STEP_BYTES;
         window = window_address;
         wave = wave_index;
@@ -428,10 +438,14 @@ struct native_chain {
                 scales[m] = matrices[m] + (uint64_t)outputs * inputs / 2u + (uint64_t)(tile0 / 4u) * steps * 256u;
             }
         }
+        word_offset = 16u * lane;
+        if constexpr (BYTES && !B128) {
 #pragma unroll
-        for (uint32_t n = 0; n < STRIP; n++) {
-            word_offset[n] = n * tile_bytes + 16u * lane;
-            scale_offset[n] = B128 ? 0u : BYTES ? ((tile0 + n) / 2u - tile0 / 2u) * (inputs / 32u) + g : 4u * lane;
+            for (uint32_t n = 0; n < STRIP; n++) {
+                scale_offset[n] = ((tile0 + n) / 2u - tile0 / 2u) * (inputs / 32u) + g;
+            }
+        } else {
+            scale_offset[0] = B128 ? 0u : 4u * lane;
         }
 #pragma unroll
         for (uint32_t i = 0; i < WAVE_BLOCKS; i++) {

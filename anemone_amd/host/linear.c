@@ -682,8 +682,9 @@ static result_status wide_experts_prepare(const struct linear_wide_experts_descr
         down->output_size, down->input_size, description->tile_count, (uint32_t)pairs};
     const struct expert_row_sum_arguments row_sum_record = {experts->pair_output.byte_offset, experts->row_output.byte_offset,
                                                             down->output_size, experts->pairs_per_row};
-    const uint32_t block_outputs = 4u * strip_outputs;
-    const uint32_t gate_up_outputs = bytes ? WIDE_GATE_UP_E4M3_BLOCK_OUTPUTS : WIDE_GATE_UP_BLOCK_OUTPUTS;
+    const uint32_t wider = native && !bytes ? 2u : 1u; /* 4-bit weights in gfx950's lane order: strips of twice the tiles */
+    const uint32_t block_outputs = wider * 4u * strip_outputs;
+    const uint32_t gate_up_outputs = bytes ? WIDE_GATE_UP_E4M3_BLOCK_OUTPUTS : wider * WIDE_GATE_UP_BLOCK_OUTPUTS;
     struct kernel_launch launches[LINEAR_WIDE_EXPERTS_BLOCK128_LAUNCH_COUNT];
     uint32_t at = 0;
     launch_fill(&launches[at++], gate_up_kernel,
