@@ -224,138 +224,4 @@ __device__ static __forceinline__ uint16_t exl3_decode_one(uint32_t state)
     return (uint16_t)exl3_decode_pair(state & 0xFFFFu, 0u);
 }
 
-/* the geometry of one width, all compile time */
-template <uint32_t bits_x2> struct exl3_width {
-    static constexpr uint32_t ring_bits = EXL3_TILE_VALUES * bits_x2 / 2u;
-    static constexpr uint32_t tile_words = ring_bits / 32u;
-    static constexpr uint32_t tile_bytes = ring_bits / 8u;
-    /* bits from the end of a run's first window to the end of symbol j's; a run starts at an even position */
-    __host__ __device__ static constexpr uint32_t step(uint32_t j)
-    {
-        return (j + 1u) * bits_x2 / 2u - bits_x2 / 2u;
-    }
-    static_assert(16u + step(3) <= 32u, "a run of four windows fits one 32-bit funnel");
-};
-
-/* Where lane (row o, chunk t) finds its run of four symbols in a tile: two word indices and a funnel shift */
-struct exl3_run_place {
-    uint32_t word0, word1, shift; /* F = alignbit(word0, word1, shift): 32 stream bits from the run's start */
-};
-
-template <uint32_t bits_x2>
-__device__ static __forceinline__ exl3_run_place exl3_run_of(uint32_t o, uint32_t t)
-{
-    typedef exl3_width<bits_x2> W;
-    const uint32_t position = 8u * (4u * (o % 8u) + t) + 4u * (o / 8u);
-    const uint32_t begin = (exl3_window_end(position, bits_x2) + W::ring_bits - 16u) % W::ring_bits;
-    const uint32_t word = begin / 32u, offset = begin % 32u;
-    exl3_run_place place;
-    place.word0 = word;
-    /* v_alignbit(hi, lo, s) takes ({hi, lo} >> s)[31:0] with s in 0..31: offset 0 needs lo = hi = word */
-    place.word1 = offset == 0u ? word : (word + 1u) % W::tile_words;
-    place.shift = (32u - offset) % 32u;
-    return place;
-}
-
-/* four symbols of a run from its funnel word F -> two registers of two fp16 weights: (j = 0, 1) and (j = 2, 3) */
-template <uint32_t bits_x2>
-__device__ static __forceinline__ void exl3_decode_run(uint32_t funnel, uint32_t &first, uint32_t &second)
-{
-    typedef exl3_width<bits_x2> W;
-    const uint32_t s0 = funnel >> 16;
-    const uint32_t s1 = (funnel >> (16u - W::step(1))) & 0xFFFFu;
-    const uint32_t s2 = (funnel >> (16u - W::step(2))) & 0xFFFFu;
-    const uint32_t s3 = (funnel >> (16u - W::step(3))) & 0xFFFFu;
-    first = exl3_decode_pair(s0, s1);
-    second = exl3_decode_pair(s2, s3);
-}
-
-/* ---- the wavefront product ----
- *
- * One wavefront multiplies a strip of NT adjacent output tiles by the K tiles [first_tile, last_tile) against up to
- * 16 operand columns and returns, per output tile, the MFMA accumulator (lane l: outputs 4 (l / 16) + i, i = 0..3,
- * of column l % 16). Tile rows of the strip are contiguous in memory (NT tile_bytes bytes), so each K tile row is
- * one coalesced 16-byte-per-lane load; two rows make an MFMA step; the next step's rows are in flight while the
- * current ones are decoded. The rows pass through a private LDS window of the wavefront (no block barrier).
- *
- *   codes        the matrix's trellis, [inputs / 16][out_tiles][tile_words] uint32
- *   out_tiles    output tiles of the whole matrix; strip_tile the first of this strip
- *   operand      per lane: pointer to the fp16 operand row of column l % 16 (NULL: the column is zero)
- *   lds          this wavefront's 2 * NT * tile_bytes bytes of LDS, 16-byte aligned
- */
-template <uint32_t bits_x2, uint32_t NT>
-__device__ static __forceinline__ void
-exl3_wave_product(const uint32_t *__restrict__ codes, uint32_t out_tiles, uint32_t strip_tile, uint32_t first_tile,
-                  uint32_t last_tile, const half_t *__restrict__ operand, uint32_t *lds, uint32_t lane,
-                  float4_t (&accumulator)[NT])
-{
-    typedef exl3_width<bits_x2> W;
-    constexpr uint32_t row_bytes = NT * W::tile_bytes;      /* one K tile row of the strip */
-    constexpr uint32_t row_lanes = row_bytes / 16u;         /* lanes that carry a 16-byte piece of it */
-    static_assert(row_bytes % 16u == 0u && row_lanes <= WAVE, "a strip row is at most one load of the wavefront");
-    const uint32_t o = lane % 16u, g = lane / 16u, tau = g / 2u, q = g % 2u;
-    const exl3_run_place run0 = exl3_run_of<bits_x2>(o, 2u * q), run1 = exl3_run_of<bits_x2>(o, 2u * q + 1u);
-    const uint32_t lane_base = tau * (row_bytes / 4u); /* the lane's tile row inside the LDS window, in words */
-    const uint64_t row_stride = (uint64_t)out_tiles * W::tile_words; /* words between K tile rows */
-    const uint32_t *source = codes + (uint64_t)first_tile * row_stride + (uint64_t)strip_tile * W::tile_words +
-                             lane * 4u;
-    const bool carries = lane < row_lanes;
-    /* the operand's eight inputs of this lane in a step: 16 tau + 4 q + {0..3} and + {8..11}. They are asked for a
-     * step ahead with the weights: loads return in order, so an operand asked for inside the step that uses it would
-     * make that step wait for the weights prefetched just before it */
-    const half_t *x = operand == nullptr ? nullptr : operand + (first_tile * 16u + 16u * tau + 4u * q);
-    uint4_t next0 = {0, 0, 0, 0}, next1 = {0, 0, 0, 0};
-    uint2_t next_low = {0, 0}, next_high = {0, 0};
-    if (first_tile < last_tile) {
-        if (carries) {
-            next0 = *(const uint4_t *)source;
-            next1 = *(const uint4_t *)(source + row_stride);
-        }
-        if (x != nullptr) {
-            next_low = *(const uint2_t *)x;
-            next_high = *(const uint2_t *)(x + 8);
-        }
-    }
-#pragma unroll
-    for (uint32_t n = 0; n < NT; n++) {
-        accumulator[n] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    for (uint32_t tile = first_tile; tile < last_tile; tile += 2u) {
-        const uint4_t row0 = next0, row1 = next1;
-        const uint2_t b_low = next_low, b_high = next_high;
-        source += 2u * row_stride;
-        if (tile + 2u < last_tile) {
-            if (carries) {
-                next0 = *(const uint4_t *)source;
-                next1 = *(const uint4_t *)(source + row_stride);
-            }
-            if (x != nullptr) {
-                x += 32;
-                next_low = *(const uint2_t *)x;
-                next_high = *(const uint2_t *)(x + 8);
-            }
-        }
-        if (carries) {
-            *(uint4_t *)(lds + lane * 4u) = row0;
-            *(uint4_t *)(lds + row_bytes / 4u + lane * 4u) = row1;
-        }
-        __builtin_amdgcn_s_waitcnt(0xc07f); /* lgkmcnt(0): the wavefront's own LDS writes have landed */
-        __builtin_amdgcn_wave_barrier();
-        const uint32_t b[4] = {b_low.x, b_low.y, b_high.x, b_high.y};
-        const half8_t operand_b = __builtin_bit_cast(half8_t, *(const uint4_t *)b);
-#pragma unroll
-        for (uint32_t n = 0; n < NT; n++) {
-            const uint32_t *tile_words = lds + lane_base + n * W::tile_words;
-            const uint32_t f0 = __builtin_amdgcn_alignbit(tile_words[run0.word0], tile_words[run0.word1], run0.shift);
-            const uint32_t f1 = __builtin_amdgcn_alignbit(tile_words[run1.word0], tile_words[run1.word1], run1.shift);
-            uint32_t a[4];
-            exl3_decode_run<bits_x2>(f0, a[0], a[2]); /* run 0: inputs 4 q + {0, 1} and {8, 9} */
-            exl3_decode_run<bits_x2>(f1, a[1], a[3]); /* run 1: inputs 4 q + {2, 3} and {10, 11} */
-            const half8_t weights = __builtin_bit_cast(half8_t, *(const uint4_t *)a);
-            accumulator[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(weights, operand_b, accumulator[n], 0, 0, 0);
-        }
-        __builtin_amdgcn_wave_barrier(); /* the next step's writes stay behind these reads */
-    }
-}
-
 #endif

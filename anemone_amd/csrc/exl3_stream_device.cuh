@@ -256,6 +256,84 @@ exl3_stream_product(const uint32_t *__restrict__ codes, uint32_t out_tiles, uint
     }
 }
 
+/*
+ * One wavefront multiplies ONE output tile by the K tiles [first_tile, last_tile) (as above): the form of a launch too
+ * small to fill the card, where a wavefront has a SIMD to itself and what counts is the length of its own chain.
+ *
+ * Lane 16 g + i decodes one half of chunk i % 8 of K tile g: the sixteen symbols of output i % 8 + 8 (i / 8), which is row
+ * i of the matrix instruction. The upper half's symbols lie four further in the ring: those lanes bring them to the lower
+ * half's places (one shift of the chunk a step), so that every lane's fields are constants. Each output's sums run over the
+ * same operands in the same order as exl3_stream_product's: the same bits.
+ * The loads run STEPS_AHEAD steps ahead: a step is two loads of codes and two of operands, and a chain of sixteen steps
+ * (4,096 inputs in four slices) waits for memory once.
+ *   accumulator  lane 16 g' + j: outputs 4 g' + {0..3} of the tile, column j
+ */
+template <uint32_t bits_x2>
+__device__ static __forceinline__ void exl3_stream_tile_product(const uint32_t *__restrict__ codes, uint32_t out_tiles, uint32_t out_tile, uint32_t first_tile,
+                                                                uint32_t last_tile, const half_t *__restrict__ operand, uint32_t lane, float4_t &accumulator)
+{
+    typedef exl3_chunk<bits_x2> C;
+    constexpr uint32_t STEPS_AHEAD = 8u, FOUR_SYMBOLS = 2u * bits_x2; /* bits */
+    const uint32_t g = lane / 16u, i = lane % 16u, c = i % 8u;
+    const bool odd = (c & 1u) != 0u, upper = i >= 8u;
+    uint32_t own, front;
+    exl3_chunk_place<bits_x2>(c, own, front);
+    const uint64_t step_stride = 4u * (uint64_t)out_tiles * C::tile_words; /* words between steps */
+    const uint32_t *tile = codes + ((uint64_t)(first_tile + g) * out_tiles + out_tile) * C::tile_words;
+    const half_t *x = operand + (first_tile + g) * EXL3_TILE;
+    const uint32_t steps = (last_tile - first_tile) / 4u;
+    accumulator = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
+    exl3_chunk_words<bits_x2> held[STEPS_AHEAD];
+    uint4_t values[STEPS_AHEAD][2];
+    const auto load = [&](uint32_t step, uint32_t set) {
+        exl3_chunk_load<bits_x2>(tile + step * step_stride, own, front, held[set]);
+        values[set][0] = *(const uint4_t *)(x + step * 4u * EXL3_TILE);
+        values[set][1] = *(const uint4_t *)(x + step * 4u * EXL3_TILE + 8u);
+    };
+#pragma unroll
+    for (uint32_t set = 0; set < STEPS_AHEAD; set++) {
+        if (set < steps) { /* the same in every lane */
+            load(set, set);
+        }
+    }
+    for (uint32_t first = 0; first < steps; first += STEPS_AHEAD) {
+#pragma unroll
+        for (uint32_t set = 0; set < STEPS_AHEAD; set++) {
+            if (first + set >= steps) {
+                break;
+            }
+            exl3_chunk_words<bits_x2> now = held[set];
+            const uint4_t now_values[2] = {values[set][0], values[set][1]};
+            if (first + set + STEPS_AHEAD < steps) {
+                load(first + set + STEPS_AHEAD, set);
+            }
+            exl3_chunk_align<bits_x2>(now, odd);
+#pragma unroll
+            for (uint32_t k = 0; k < C::words; k++) {
+                const uint32_t moved = __builtin_amdgcn_alignbit(now.z[k], now.z[k + 1u], 32u - FOUR_SYMBOLS);
+                now.z[k] = upper ? moved : now.z[k];
+            }
+            now.z[C::words] = upper ? now.z[C::words] << FOUR_SYMBOLS : now.z[C::words];
+            uint32_t funnel[C::words];
+#pragma unroll
+            for (uint32_t k = 0; k < C::words; k++) {
+                funnel[k] = __builtin_amdgcn_alignbit(now.z[k], now.z[k + 1u], 16u);
+            }
+#pragma unroll
+            for (uint32_t v = 0; v < 2u; v++) {
+                uint32_t a[4];
+#pragma unroll
+                for (uint32_t t = 0; t < 4u; t++) {
+                    a[t] = exl3_decode_pair(exl3_chunk_state<bits_x2>(now.z, funnel, 8u * t + 2u * v),
+                                            exl3_chunk_state<bits_x2>(now.z, funnel, 8u * t + 2u * v + 1u));
+                }
+                const uint4_t packed = {a[0], a[1], a[2], a[3]};
+                accumulator = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, packed), __builtin_bit_cast(half8_t, now_values[v]), accumulator, 0, 0, 0);
+            }
+        }
+    }
+}
+
 /* where lane (g', column) stores accumulator [p][h] of a strip: four consecutive outputs from this one */
 __device__ static __forceinline__ uint32_t exl3_stream_output(uint32_t strip_tile, uint32_t p, uint32_t h, uint32_t lane)
 {

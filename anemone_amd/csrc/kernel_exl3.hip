@@ -1,8 +1,8 @@
 /*
  * kernel_exl3.hip -- EXL3 (trellis, codebook mul1) reconstruction and the routed experts' five-launch chain for
  * gfx950. Entry names and records are the reference's (source/kernel_exl3.cu, include/anemone/exl3_records.h);
- * the work mapping is this build's: one wavefront per 128-value transform block, and products by wavefronts that
- * stream strips of eight output tiles through LDS into v_mfma_f32_16x16x32_f16 (exl3_device.cuh).
+ * the work mapping is this build's: one wavefront per 128-value transform block, and products by wavefronts whose lanes
+ * take their codes from memory and decode them for v_mfma_f32_16x16x32_f16 (exl3_stream_device.cuh).
  *
  * Arithmetic contract (source/kernel_exl3.cu:133-424): operands fp16( H128(bf16 x . fp16 suh) . norm ); products
  * float32 in four contiguous K slices added in slice order from +0; hidden bf16( min(g, L) / (1 + e^-g) . clamp(u) )
@@ -10,7 +10,7 @@
  * H128(down product) . norm . svh . route weight, in place of the down products; row sum in slot order from +0.
  * Inside a slice the MFMA adds 32 products at a time in its own order, which no host reference has bit for bit.
  */
-#include "exl3_device.cuh"
+#include "exl3_stream_device.cuh"
 #include "kernel_registry.h"
 
 #define PRODUCT_WAVES EXL3_PRODUCT_SLICES
@@ -76,42 +76,48 @@ extern "C" __global__ void exl3_input(struct exl3_expert_record record, unsigned
 }
 ANEMONE_KERNEL(EXL3_KERNEL_FILE, exl3_input, exl3_expert_record);
 
-/* Products of one job: block = four wavefronts = the four K slices of one strip of STRIP_TILES output tiles (eight; one
- * in the thin instances, which a launch of few jobs takes so that its blocks cover the card: the same slices and the
- * same order of sums, so the same bits). */
+/* Products of one job: block = four wavefronts = the four K slices (whole steps of four K tiles) of one strip of
+ * STRIP_TILES output tiles: eight (the stream product), or one in the thin instances, which a launch of few jobs takes so
+ * that its blocks cover the card (the same slices and the same order of sums, so the same bits).
+ * A thin launch has a wavefront a SIMD, so its time is the chain of one wavefront: its codes' loads run eight steps ahead
+ * and pass through no LDS. One 4096 x 4096 matrix of K 4 by one vector: 7.8 us (13.4 with two K tiles a step, a step ahead
+ * through an LDS window); the input, product and finish launches 10.8 us (16.5). */
 template <uint32_t bits_x2, bool down, uint32_t STRIP_TILES>
 __device__ static __forceinline__ void chain_product(const struct exl3_expert_record &record, unsigned char *arena,
-                                                     const struct expert_job_record *job, uint32_t *staging,
-                                                     float *partial)
+                                                     const struct expert_job_record *job, float *partial)
 {
-    typedef exl3_width<bits_x2> W;
     const uint32_t projection = blockIdx.z;
     const uint32_t inputs = down ? record.inner_size : record.input_size;
     const uint32_t outputs = down ? record.input_size : record.inner_size;
-    const uint32_t lane = threadIdx.x % WAVE, slice = threadIdx.x / WAVE;
+    const uint32_t lane = threadIdx.x % WAVE, slice = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const uint64_t matrix = down ? job->down_offset : projection == 0u ? job->gate_offset : job->up_offset;
     const uint32_t column = lane % 16u;
-    const half_t *operand = nullptr;
-    if (column < job->row_count) {
-        operand = (const half_t *)(arena + record.operands_offset) +
-                  ((uint64_t)projection * record.pair_count + job->pair_index[column]) * inputs;
+    /* a column that is not live reads the first column's operand: its sums are not stored */
+    const uint32_t pair = job->pair_index[column < job->row_count ? column : 0u];
+    const half_t *operand = (const half_t *)(arena + record.operands_offset) + ((uint64_t)projection * record.pair_count + pair) * inputs;
+    const uint32_t steps = inputs / (4u * EXL3_TILE), strip_tile = blockIdx.x * STRIP_TILES;
+    const uint32_t first_tile = 4u * (steps * slice / PRODUCT_WAVES), last_tile = 4u * (steps * (slice + 1u) / PRODUCT_WAVES);
+    const uint32_t *codes = (const uint32_t *)(arena + matrix);
+    float4_t sums[STRIP_TILES];
+    if constexpr (STRIP_TILES == 1u) {
+        exl3_stream_tile_product<bits_x2>(codes, outputs / EXL3_TILE, strip_tile, first_tile, last_tile, operand, lane, sums[0]);
+    } else {
+        float4_t accumulator[STRIP_TILES / 2u][2];
+        exl3_stream_product<bits_x2, STRIP_TILES / 2u, true>(codes, outputs / EXL3_TILE, strip_tile, first_tile, last_tile, operand, lane, accumulator);
+#pragma unroll
+        for (uint32_t n = 0; n < STRIP_TILES; n++) {
+            sums[n] = accumulator[n / 2u][n % 2u];
+        }
     }
-    const uint32_t tiles = inputs / EXL3_TILE;
-    float4_t accumulator[STRIP_TILES];
-    exl3_wave_product<bits_x2, STRIP_TILES>((const uint32_t *)(arena + matrix), outputs / EXL3_TILE,
-                                            blockIdx.x * STRIP_TILES, tiles * slice / PRODUCT_WAVES,
-                                            tiles * (slice + 1u) / PRODUCT_WAVES, operand,
-                                            staging + slice * (2u * STRIP_TILES * W::tile_words), lane, accumulator);
-    /* partial [slice][tile][lane] as float4; slice 0 then adds the four in order from +0 */
+    /* partial [slice][n][lane] as float4; slice 0 then adds the four in order from +0 */
     float4_t *mine = (float4_t *)partial + (slice * STRIP_TILES) * WAVE + lane;
 #pragma unroll
     for (uint32_t n = 0; n < STRIP_TILES; n++) {
-        mine[n * WAVE] = accumulator[n];
+        mine[n * WAVE] = sums[n];
     }
     __syncthreads();
     if (slice == 0u && column < job->row_count) {
-        float *products = (float *)(arena + record.products_offset) +
-                          ((uint64_t)projection * record.pair_count + job->pair_index[column]) * outputs;
+        float *products = (float *)(arena + record.products_offset) + ((uint64_t)projection * record.pair_count + pair) * outputs;
 #pragma unroll
         for (uint32_t n = 0; n < STRIP_TILES; n++) {
             float4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -123,8 +129,10 @@ __device__ static __forceinline__ void chain_product(const struct exl3_expert_re
                 sum.z = __fadd_rn(sum.z, value.z);
                 sum.w = __fadd_rn(sum.w, value.w);
             }
-            /* lane: outputs 4 (lane / 16) + 0..3 of tile n of the strip */
-            *(float4_t *)(products + (blockIdx.x * STRIP_TILES + n) * EXL3_TILE + 4u * (lane / 16u)) = sum;
+            /* four outputs a lane, from where the product's form keeps them */
+            const uint32_t output = STRIP_TILES == 1u ? strip_tile * EXL3_TILE + 4u * (lane / 16u)
+                                                      : exl3_stream_output(strip_tile, n / 2u, n % 2u, lane);
+            *(float4_t *)(products + output) = sum;
         }
     }
 }
@@ -133,7 +141,6 @@ template <uint32_t fixed_bits_x2, bool down, uint32_t STRIP_TILES>
 __device__ static __forceinline__ void chain_product_entry(const struct exl3_expert_record &record,
                                                            unsigned char *arena)
 {
-    __shared__ __attribute__((aligned(16))) uint32_t staging[PRODUCT_WAVES * 2u * STRIP_TILES * exl3_width<8>::tile_words];
     __shared__ __attribute__((aligned(16))) float partial[PRODUCT_WAVES * STRIP_TILES * WAVE * 4u];
     const struct expert_job_record *job = (const struct expert_job_record *)(arena + record.jobs_offset) + blockIdx.y;
     if (job->row_count == 0u) {
@@ -144,10 +151,10 @@ __device__ static __forceinline__ void chain_product_entry(const struct exl3_exp
         bits_x2 = exl3_bits_x2(chain_width(record, arena, job->expert, down ? 2u : blockIdx.z));
     }
     switch (bits_x2) {
-    case 4u: chain_product<4u, down, STRIP_TILES>(record, arena, job, staging, partial); break;
-    case 5u: chain_product<5u, down, STRIP_TILES>(record, arena, job, staging, partial); break;
-    case 6u: chain_product<6u, down, STRIP_TILES>(record, arena, job, staging, partial); break;
-    case 8u: chain_product<8u, down, STRIP_TILES>(record, arena, job, staging, partial); break;
+    case 4u: chain_product<4u, down, STRIP_TILES>(record, arena, job, partial); break;
+    case 5u: chain_product<5u, down, STRIP_TILES>(record, arena, job, partial); break;
+    case 6u: chain_product<6u, down, STRIP_TILES>(record, arena, job, partial); break;
+    case 8u: chain_product<8u, down, STRIP_TILES>(record, arena, job, partial); break;
     default: break;
     }
 }

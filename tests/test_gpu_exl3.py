@@ -345,3 +345,40 @@ def test_a_slice_of_outputs_gives_the_whole_matrix_bits(amd, card, width):
     whole, part = products_of(matrix, outputs), products_of(sliced, count)
     assert np.array_equal(part.view(np.uint32), whole[begin:begin + count].view(np.uint32))
     assert np.any(part != 0)
+
+
+@pytest.mark.parametrize("width", [2, 40, 3, 4])
+@pytest.mark.parametrize("inputs", [128, 384, 2304])
+def test_thin_product_of_short_and_long_slices(amd, card, inputs, width):
+    """The product of one output tile a block where its K slices are empty or one step (128 inputs are two steps of 64 for
+    four slices), of unequal lengths (384), and longer than the eight steps its loads run ahead (2304: nine); three rows,
+    against the codebook's weights (the oracle's reconstruction) in float64. An output's sum of `inputs` products in float32
+    is off by at most inputs 2^-24 of the sum of their magnitudes, whatever the order."""
+    say("thin product", inputs, width)
+    outputs, rows = max(256, inputs), 3
+    matrix, spare = exl3_matrix(0x7300 + width, inputs, outputs, width), exl3_matrix(0x7400 + width, outputs, inputs, width)
+    weights = np.zeros((inputs, outputs), dtype=np.uint16)
+    orc.orc_exl3_decode_matrix(ptr(matrix, u8p), inputs, outputs, width, ptr(weights, u16p))
+    weights = weights.view(np.float16).astype(np.float64)
+    jobs = np.zeros(1, dtype=JOB_DTYPE)
+    jobs[0]["gate_offset"] = jobs[0]["up_offset"] = card.place(spare, 256)
+    jobs[0]["down_offset"] = card.place(matrix, 256)
+    jobs[0]["row_count"], jobs[0]["pair_index"][:rows], jobs[0]["route_weight"][:rows] = rows, np.arange(rows), 1.0
+    operands = normals(0x7500 + inputs, rows * inputs).astype(np.float16).reshape(rows, inputs)
+    record = amd.Exl3ExpertRecord()
+    record.jobs_offset = card.place(jobs.view(np.uint8))
+    record.input_offset = card.reserve(rows * outputs * 2)
+    record.operands_offset = card.reserve(rows * outputs * 4)
+    record.products_offset = record.output_offset = card.reserve(rows * outputs * 8)
+    record.hidden_offset = card.reserve(rows * inputs * 2)
+    record.input_size, record.inner_size = outputs, inputs
+    record.pair_count, record.pairs_per_row, record.job_count = rows, 1, 1
+    record.bits_per_weight, record.activation_limit = width, 10.0
+    launches = amd.launches_of(5)
+    amd.check(card.lib.exl3_experts_prepare(C.byref(record), card.arena_bytes, amd.backend_table(), card.handle, 950, launches), "prepare")
+    assert list(launches[3].grid) == [outputs // 16, 1, 1]
+    card.upload(record.operands_offset, operands)
+    card.run(launches[3:4])
+    got = card.download(record.products_offset, rows * outputs * 4, np.float32).reshape(rows, outputs)
+    want, magnitudes = operands.astype(np.float64) @ weights, np.abs(operands.astype(np.float64)) @ np.abs(weights)
+    assert np.all(np.abs(got - want) <= inputs * 2.0 ** -24 * magnitudes)
