@@ -7,7 +7,8 @@
  *
  * Arithmetic: the chain's (kernel_exl3.hip): fp16 operands from a float32 Hadamard transform, exactly decoded fp16
  * weights, float32 MFMA sums over increasing k (one chain an output: the GEMM is not cut along k), SwiGLU in float32,
- * a row's weighted pair outputs added in slot order. A pair's result does not depend on the other pairs of the call.
+ * a row's weighted pair outputs added in slot order. A pair's result does not depend on the other pairs of the call; the
+ * two forms of the GEMM, which the call's sizes choose between (exl3_tcp_is_thin), add in an order of their own each.
  *
  * The GEMM block: 256 outputs (four wavefronts of four 16 x 16 tiles) by one chunk of at most EXL3_TCP_CHUNK_PAIRS (160)
  * pairs of one expert. A K step is 64 inputs: the chunk's operand columns (160 x 64 fp16, 20 KB) go from memory straight
@@ -514,6 +515,178 @@ extern "C" __global__ void __launch_bounds__(TCP_GEMM_THREADS, 2) exl3_tcp_gemm(
 #undef TCP_GEMM_OF
 }
 ANEMONE_KERNEL(EXL3_TCP_KERNEL_FILE, exl3_tcp_gemm, exl3_tcp_record);
+
+/*
+ * The GEMM of few pairs an expert. The launch above is written for chunks of up to 160 pairs: their sums (160 registers)
+ * leave room for two wavefronts a SIMD, and at two the vector unit issues an instruction every 5 to 6 cycles where it
+ * issues one every 4.5 at four; with a handful of pairs an expert the launch is nothing but decoding, and the step's
+ * barrier and wait are paid for columns that are not there. This form keeps its operands to itself: codes and operand
+ * columns go from memory straight into a wavefront's registers, no LDS and no barrier, at four wavefronts a SIMD.
+ * Lanes and decode are the stream product's (exl3_stream_device.cuh), and so is the matrix instruction of 16 x 16 outputs:
+ * a decoded operand feeds one for every sixteen pairs. (On the 32 x 32 instruction above, with the same bits as above, the
+ * half-empty columns cost: 1012 us for the first call below.)
+ * What bounds it is the vector unit (3.75 instructions a weight). Whole calls, hidden 4096, intermediate 2048, 256 experts,
+ * 8 picks, this form against the one above: 203 rows 947 / 1120 us, 66 rows 838 / 992, 512 rows 1063 / 1197; 203 rows of
+ * Zipf(1.1) loads 960 / 1061. Four wavefronts with room for 32, 48 and 64 pairs a block (three wavefronts): 955, 947 and
+ * 975 us at 203 rows, 1002, 960 and 984 at the Zipf loads; two pairs of tiles or four a wavefront: the same.
+ */
+
+/* A wavefront's product of TCP_WAVE_PAIRS pairs of adjacent output tiles by CB blocks of sixteen columns. The inner half v
+ * of the operands' values is outermost in a step, so that one set of registers holds them: a half's values of the next
+ * step are asked for behind its last use, half a step ahead. */
+template <uint32_t bits_x2, uint32_t CB>
+__device__ static __forceinline__ void tcp_thin_item(const uint32_t *__restrict__ codes, uint32_t inputs, uint32_t outputs, uint32_t strip_tile,
+                                                     const half_t *__restrict__ columns, uint32_t column_count, float *__restrict__ products, uint32_t lane)
+{
+    typedef exl3_chunk<bits_x2> C;
+    const uint32_t out_tiles = outputs / EXL3_TILE, g = lane / 16u, i = lane % 16u, c = i % 8u;
+    const bool odd = (c & 1u) != 0u;
+    uint32_t own, front;
+    exl3_chunk_place<bits_x2>(c, own, front);
+    const uint64_t step_stride = 4u * (uint64_t)out_tiles * C::tile_words; /* words between steps */
+    const uint32_t *tile = codes + ((uint64_t)g * out_tiles + strip_tile + i / 8u) * C::tile_words;
+    /* the lane's column of each block at its K tile's values, in bytes (EXL3_TCP_THIN_WIDTH keeps 48 columns within 32
+     * bits); a column past the pairs names the first: its sums are not stored, and the instruction keeps columns apart */
+    const unsigned char *x = (const unsigned char *)columns;
+    uint32_t column_at[CB];
+#pragma unroll
+    for (uint32_t b = 0; b < CB; b++) {
+        const uint32_t column = 16u * b + i;
+        column_at[b] = ((column < column_count ? column : 0u) * inputs + g * EXL3_TILE) * 2u;
+    }
+    float4_t accumulator[TCP_WAVE_PAIRS][2][CB];
+#pragma unroll
+    for (uint32_t p = 0; p < TCP_WAVE_PAIRS; p++) {
+#pragma unroll
+        for (uint32_t b = 0; b < CB; b++) {
+            accumulator[p][0][b] = accumulator[p][1][b] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
+    exl3_chunk_words<bits_x2> held[2][TCP_WAVE_PAIRS];
+    uint4_t operand[2][CB];
+    const auto load_codes = [&](exl3_chunk_words<bits_x2> (&into)[TCP_WAVE_PAIRS]) {
+#pragma unroll
+        for (uint32_t p = 0; p < TCP_WAVE_PAIRS; p++) {
+            exl3_chunk_load<bits_x2>(tile + p * 2u * C::tile_words, own, front, into[p]);
+        }
+    };
+    const auto load_operands = [&](uint32_t v) {
+#pragma unroll
+        for (uint32_t b = 0; b < CB; b++) {
+            operand[v][b] = *(const uint4_t *)(x + column_at[b] + 16u * v);
+        }
+    };
+    const uint32_t steps = inputs / TCP_STEP_INPUTS;
+    load_codes(held[0]);
+    load_operands(0u);
+    load_operands(1u);
+    const auto one_step = [&](uint32_t step, exl3_chunk_words<bits_x2> (&now)[TCP_WAVE_PAIRS], exl3_chunk_words<bits_x2> (&next)[TCP_WAVE_PAIRS]) {
+        const bool more = step + 1u < steps; /* the same in every lane */
+        if (more) {
+            tile += step_stride;
+            load_codes(next);
+        }
+        x += more ? TCP_STEP_INPUTS * 2u : 0u; /* the last step asks for its own values again: no branch around the loads */
+        uint32_t funnel[TCP_WAVE_PAIRS][C::words];
+#pragma unroll
+        for (uint32_t p = 0; p < TCP_WAVE_PAIRS; p++) {
+            exl3_chunk_align<bits_x2>(now[p], odd);
+#pragma unroll
+            for (uint32_t word = 0; word < C::words; word++) {
+                funnel[p][word] = __builtin_amdgcn_alignbit(now[p].z[word], now[p].z[word + 1u], 16u);
+            }
+        }
+#pragma unroll
+        for (uint32_t v = 0; v < 2u; v++) {
+#pragma unroll
+            for (uint32_t p = 0; p < TCP_WAVE_PAIRS; p++) {
+#pragma unroll
+                for (uint32_t h = 0; h < 2u; h++) {
+                    uint32_t a[4];
+#pragma unroll
+                    for (uint32_t t = 0; t < 4u; t++) {
+                        const uint32_t m = 8u * t + 4u * h + 2u * v;
+                        a[t] = exl3_decode_pair(exl3_chunk_state<bits_x2>(now[p].z, funnel[p], m), exl3_chunk_state<bits_x2>(now[p].z, funnel[p], m + 1u));
+                    }
+                    const uint4_t packed = {a[0], a[1], a[2], a[3]};
+                    const half8_t weights = __builtin_bit_cast(half8_t, packed);
+#pragma unroll
+                    for (uint32_t b = 0; b < CB; b++) {
+                        accumulator[p][h][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(weights, __builtin_bit_cast(half8_t, operand[v][b]), accumulator[p][h][b], 0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0); /* the next operand's decoding, hoisted above, spills */
+                }
+            }
+            load_operands(v);
+        }
+    };
+    for (uint32_t step = 0; step < steps; step += 2u) {
+        one_step(step, held[0], held[1]);
+        if (step + 1u < steps) {
+            one_step(step + 1u, held[1], held[0]);
+        }
+    }
+#pragma unroll
+    for (uint32_t b = 0; b < CB; b++) {
+        const uint32_t column = 16u * b + i;
+        if (column < column_count) {
+            float *out = products + (uint64_t)column * outputs;
+#pragma unroll
+            for (uint32_t p = 0; p < TCP_WAVE_PAIRS; p++) {
+#pragma unroll
+                for (uint32_t h = 0; h < 2u; h++) {
+                    *(float4_t *)(out + exl3_stream_output(strip_tile, p, h, lane)) = accumulator[p][h][b];
+                }
+            }
+        }
+    }
+}
+
+/* launches 3 and 5 of a call of few pairs an expert (exl3_tcp_is_thin): grid (ceil(outputs / 256), chunk capacity,
+ * projections x EXL3_TCP_THIN_PARTS), block 256. A block takes EXL3_TCP_THIN_COLUMNS pairs of a chunk, so that a busy
+ * expert's chunk is several blocks side by side and not a long one at the launch's end. */
+extern "C" __global__ void __launch_bounds__(TCP_GEMM_THREADS, 4) exl3_tcp_gemm_thin(struct exl3_tcp_record record, unsigned char *arena)
+{
+    const tcp_shape shape = tcp_shape_of(record);
+    unsigned char *workspace = arena + record.workspace_offset;
+    const struct exl3_tcp_chunk chunk = tcp_chunk_of(shape, workspace, blockIdx.y);
+    const bool down = record.pass == EXL3_TCP_DOWN;
+    const uint32_t projection = down ? 2u : blockIdx.z % 2u, first = (down ? blockIdx.z : blockIdx.z / 2u) * EXL3_TCP_THIN_COLUMNS;
+    if (first >= chunk.pair_count) {
+        return;
+    }
+    const uint32_t left = chunk.pair_count - first, count = left < EXL3_TCP_THIN_COLUMNS ? left : EXL3_TCP_THIN_COLUMNS;
+    const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const uint32_t inputs = down ? shape.intermediate : shape.hidden, outputs = down ? shape.hidden : shape.intermediate;
+    const uint32_t strip_tile = (blockIdx.x * EXL3_TCP_BLOCK_OUTPUTS) / EXL3_TILE + wave * 2u * TCP_WAVE_PAIRS;
+    if (strip_tile * EXL3_TILE >= outputs) {
+        return;
+    }
+    const uint32_t bits_x2 = tcp_bits_x2(record, arena, chunk.expert, projection);
+    const uint32_t *codes = (const uint32_t *)(arena + tcp_matrix_of(record, arena, chunk.expert, projection));
+    const uint64_t place = chunk.first_pair + first;
+    const half_t *columns = (const half_t *)(workspace + shape.layout.operands) + ((uint64_t)(down ? 0u : projection) * shape.pairs + place) * inputs;
+    float *products = down ? (float *)(workspace + shape.layout.down) + place * outputs
+                           : (float *)(workspace + shape.layout.gate_up) + ((uint64_t)projection * shape.pairs + place) * outputs;
+    /* one instance a width and a count of blocks of sixteen columns */
+#define TCP_THIN_WIDTH(bits)                                                                         \
+    if (count <= 16u) {                                                                              \
+        tcp_thin_item<bits, 1u>(codes, inputs, outputs, strip_tile, columns, count, products, lane); \
+    } else if (count <= 32u) {                                                                       \
+        tcp_thin_item<bits, 2u>(codes, inputs, outputs, strip_tile, columns, count, products, lane); \
+    } else {                                                                                         \
+        tcp_thin_item<bits, EXL3_TCP_THIN_COLUMNS / 16u>(codes, inputs, outputs, strip_tile, columns, count, products, lane); \
+    }
+    switch (bits_x2) {
+    case 4u: TCP_THIN_WIDTH(4u) break;
+    case 5u: TCP_THIN_WIDTH(5u) break;
+    case 6u: TCP_THIN_WIDTH(6u) break;
+    case 8u: TCP_THIN_WIDTH(8u) break;
+    default: return; /* no width of the format: the prepare refuses such a record */
+    }
+#undef TCP_THIN_WIDTH
+}
+ANEMONE_KERNEL(EXL3_TCP_KERNEL_FILE, exl3_tcp_gemm_thin, exl3_tcp_record);
 
 /* launch 4: grid (ceil(intermediate / 512), chunk capacity, EXL3_TCP_COLUMN_PARTS), block 64: per pair of a part of the chunk, gate = H128(gate products) /
  * sqrt(128) x svh, up the same, the SwiGLU with its limit, x the down matrix's suh, H128 -> the fp16 down operand */

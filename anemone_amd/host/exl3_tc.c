@@ -197,8 +197,14 @@ result_status exl3_tc_prepare_detached(const struct exl3_tc_record *record, uint
  *   down        exl3_tcp_gemm       (ceil(hidden / 256), chunk capacity, 1)          256   pass EXL3_TCP_DOWN
  *   combine     exl3_tcp_combine    (hidden / 128, rows, 1)                          64
  * chunk capacity = pairs / EXL3_TCP_CHUNK_PAIRS + experts: an expert's pairs cut in chunks of EXL3_TCP_CHUNK_PAIRS (160), the
- * last ragged.
+ * last ragged. A thin call (exl3_tcp_is_thin) takes exl3_tcp_gemm_thin for both GEMM passes, its grid's z
+ * EXL3_TCP_THIN_PARTS times as many.
  */
+static bool exl3_tcp_is_thin(uint64_t pairs, uint64_t experts, uint32_t hidden, uint32_t intermediate)
+{
+    return pairs <= EXL3_TCP_THIN_PAIRS * experts && hidden <= EXL3_TCP_THIN_WIDTH && intermediate <= EXL3_TCP_THIN_WIDTH;
+}
+
 static result_status tcp_prepare(const struct exl3_tcp_record *record, uint64_t arena_byte_count,
                                  const struct backend_operations *backend, struct device_card *card,
                                  struct kernel_launch launches_out[EXL3_TCP_MOST_LAUNCHES], uint32_t *launch_count_out)
@@ -255,14 +261,17 @@ static result_status tcp_prepare(const struct exl3_tcp_record *record, uint64_t 
         }
         return STATUS_INVALID_ARGUMENT;
     }
-    static const char *const names[EXL3_TCP_LAUNCHES] = {"exl3_tcp_count",    "exl3_tcp_place", "exl3_tcp_operands", "exl3_tcp_gemm",
-                                                         "exl3_tcp_activate", "exl3_tcp_gemm",  "exl3_tcp_combine"};
+    const bool thin = exl3_tcp_is_thin(pairs, E, H, I);
+    const char *const gemm = thin ? "exl3_tcp_gemm_thin" : "exl3_tcp_gemm";
+    const uint32_t parts = thin ? EXL3_TCP_THIN_PARTS : 1u;
+    const char *const names[EXL3_TCP_LAUNCHES] = {"exl3_tcp_count",    "exl3_tcp_place", "exl3_tcp_operands", gemm,
+                                                  "exl3_tcp_activate", gemm,             "exl3_tcp_combine"};
     const uint32_t blocks = (uint32_t)((rows + ROUTER_SORT_ROWS - 1u) / ROUTER_SORT_ROWS), capacity = layout.chunk_capacity;
     /* an element-wise launch's wavefront takes four blocks of 128 channels */
     const uint32_t grid_x[EXL3_TCP_LAUNCHES] = {blocks, blocks, (H + 511u) / 512u, (I + EXL3_TCP_BLOCK_OUTPUTS - 1u) / EXL3_TCP_BLOCK_OUTPUTS,
                                                 (I + 511u) / 512u, (H + EXL3_TCP_BLOCK_OUTPUTS - 1u) / EXL3_TCP_BLOCK_OUTPUTS, (H + 511u) / 512u};
     const uint32_t grid_y[EXL3_TCP_LAUNCHES] = {1u, 1u, capacity, capacity, capacity, capacity, record->row_count};
-    const uint32_t grid_z[EXL3_TCP_LAUNCHES] = {1u, 1u, EXL3_TCP_COLUMN_PARTS, 2u, EXL3_TCP_COLUMN_PARTS, 1u, 1u};
+    const uint32_t grid_z[EXL3_TCP_LAUNCHES] = {1u, 1u, EXL3_TCP_COLUMN_PARTS, 2u * parts, EXL3_TCP_COLUMN_PARTS, parts, 1u};
     const uint32_t threads[EXL3_TCP_LAUNCHES] = {512u, 512u, WAVE_THREADS, PRODUCT_THREADS, WAVE_THREADS, PRODUCT_THREADS, WAVE_THREADS};
     struct kernel_launch launches[EXL3_TCP_LAUNCHES];
     for (uint32_t index = 0; index < EXL3_TCP_LAUNCHES; index++) {

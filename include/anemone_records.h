@@ -342,6 +342,14 @@ ANEMONE_INLINE uint64_t exl3_tc_workspace_bytes(uint64_t pairs, uint64_t hidden,
  * the combine of a row's pairs in slot order. */
 #define EXL3_TCP_KERNEL_FILE "kernel_exl3_tcp"
 #define EXL3_TCP_CHUNK_PAIRS 160u  /* columns of one GEMM block: pairs of one expert (ten MFMA column blocks) */
+/* a call of few pairs an expert on average takes the GEMM whose blocks hold THIN_COLUMNS pairs (kernel_exl3_tcp.hip,
+ * exl3_tcp_gemm_thin), THIN_PARTS of them a chunk. Whole calls of 256 experts, 8 picks, that form against the other, us:
+ * 12.5 pairs an expert 1009 / 1170, 16 1064 / 1197, 20 1164 / 1223, 32 1388 / 1395; of Zipf(1.1) loads 6.3 pairs 960 /
+ * 1061, 12.5 1175 / 1223, 20 1392 / 1373: the line lies where no load tried is slower */
+#define EXL3_TCP_THIN_PAIRS 16u
+#define EXL3_TCP_THIN_COLUMNS 48u
+#define EXL3_TCP_THIN_WIDTH (1u << 20) /* and sizes up to this: a block's operand columns are addressed in 32 bits */
+#define EXL3_TCP_THIN_PARTS ((EXL3_TCP_CHUNK_PAIRS + EXL3_TCP_THIN_COLUMNS - 1u) / EXL3_TCP_THIN_COLUMNS)
 #define EXL3_TCP_PART_COLUMNS 16u /* pairs of a chunk a block of the element-wise launches (operands, activate) takes */
 #define EXL3_TCP_COLUMN_PARTS ((EXL3_TCP_CHUNK_PAIRS + EXL3_TCP_PART_COLUMNS - 1u) / EXL3_TCP_PART_COLUMNS)
 #define EXL3_TCP_BLOCK_OUTPUTS 256u /* outputs of one GEMM block: four wavefronts of four tiles */

@@ -485,6 +485,18 @@ def tcp_record(**changes):
     return r
 
 
+@pytest.mark.parametrize("rows,changes,thin", [(512, {}, True), (513, {}, False), (1, dict(hidden=1 << 20, intermediate=128), True),
+                                               (1, dict(hidden=(1 << 20) + 128, intermediate=128), False)])
+def test_tcp_prepare_takes_the_thin_gemm_up_to_sixteen_pairs_an_expert(fake, rows, changes, thin):
+    launches, count, arena = amd.launches_of(8), C.c_uint32(0), 1 << 40
+    record = tcp_record(row_count=rows, output_offset=1 << 32, workspace_offset=1 << 33, **changes)
+    assert amd.library().exl3_tcp_prepare(C.byref(record), arena, fake.address, fake.card, launches, C.byref(count)) == 0
+    capacity = rows * 8 // amd.EXL3_TCP_CHUNK_PAIRS + 256
+    for index, outputs, matrices in ((3, record.intermediate, 2), (5, record.hidden, 1)):
+        assert fake.handles[launches[index].kernel][1] == ("exl3_tcp_gemm_thin" if thin else "exl3_tcp_gemm")
+        assert list(launches[index].grid) == [(outputs + 255) // 256, capacity, matrices * (4 if thin else 1)] and launches[index].block[0] == 256
+
+
 def test_tcp_prepare_geometry_and_refusals(fake):
     lib = amd.library()
     launches, count = amd.launches_of(8), C.c_uint32(0)

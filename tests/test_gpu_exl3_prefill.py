@@ -122,6 +122,40 @@ def test_prefill_layer_against_oracle(amd, card, hidden, inner, experts_n, picks
     assert error <= 4e-3
 
 
+@pytest.mark.parametrize("hidden,inner,width_choices", [(512, 384, [2, 3, 4]), (128, 128, [40])])
+def test_thin_gemm_at_the_edges_of_its_blocks(amd, card, hidden, inner, width_choices):
+    """A call of few pairs an expert (exl3_tcp_gemm_thin: blocks of 48 pairs, instances of one to three blocks of sixteen):
+    experts of 15, 16, 17, 32, 33, 47, 48, 49 and 161 pairs, others with none; against the oracle (the bound of the layer
+    test above), and the same rows in a call of more pairs an expert (exl3_tcp_gemm: the same operands and weights, the
+    float32 sums in another order). What the order moves: here and there a down operand's fp16 rounding by a place, 2^-10 of
+    a value; one of five times the operands' rms among `inner` of them moves an output by 5 2^-10 / sqrt(inner) of its rms
+    (2.5e-4 at 384). Four such in one output are allowed."""
+    say("thin prefill", hidden, inner, width_choices)
+    experts_n, picks, rows = 64, 2, 256
+    first = np.repeat(np.arange(8), [15, 16, 17, 32, 33, 47, 48, 48])
+    second = np.repeat([40, 41, 63], [161, 49, 46])
+    layer, matrices, widths = build_layer(amd, card, hidden, inner, experts_n, picks, 3 * rows, 23, width_choices)
+    x = to_bf16(normals(35, 3 * rows * hidden)).reshape(3 * rows, hidden)
+    table = np.zeros((3 * rows, picks), dtype=np.dtype([("expert", "<u4"), ("route_weight", "<f4")]))
+    table["expert"] = np.tile(np.stack([first, np.random.default_rng(3).permutation(second)], axis=1), (3, 1))
+    table["route_weight"] = np.random.default_rng(4).uniform(0.1, 1.0, (3 * rows, picks)).astype(np.float32)
+    picks_at, got = card.place(table.view(np.uint8).reshape(-1)), {}
+    for count in (rows, 3 * rows):  # 8 and 24 pairs an expert on average
+        layer.rows, layer.tcp_workspace_offset = count, None
+        layer.set_rows(x[:count], count)
+        card.upload(layer.out_offset, np.full(count * hidden * 4, 0xFF, dtype=np.uint8))
+        launches = layer.tcp_launches(picks_at)
+        assert launches[3].grid[2] == (8 if count == rows else 2) and launches[5].grid[2] == (4 if count == rows else 1)
+        card.run(launches)
+        got[count] = layer.output()[:rows].copy()
+    layer.rows = rows
+    want = oracle_layer(layer, x[:rows], np.ascontiguousarray(table["expert"][:rows]), np.ascontiguousarray(table["route_weight"][:rows]), matrices, widths)
+    scale = float(np.sqrt(np.mean(want.astype(np.float64) ** 2)))
+    error, apart = (float(np.max(np.abs(got[rows] - other))) / scale for other in (want, got[3 * rows]))
+    say("  max error %.2e of the output's rms, the two forms %.2e apart" % (error, apart))
+    assert error <= 4e-3 and apart <= 4 * 5 * 2.0 ** -10 / inner ** 0.5
+
+
 def test_prefill_equals_fused_decode_on_the_same_rows(amd, card):
     """Eight rows through the fused decode and through the prefill form: the same operands, weights and float32 chains
     cut differently along k (the decode's slices against one chain): equal within float32 rounding of the sums."""
