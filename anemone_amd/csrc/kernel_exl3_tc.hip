@@ -22,6 +22,7 @@
 #include <string.h>
 
 #define STRIP_PAIRS (EXL3_TC_STRIP_OUTPUTS / 32u) /* a strip: pairs of adjacent output tiles */
+#define NARROW_STRIP_PAIRS (EXL3_TC_NARROW_STRIP_OUTPUTS / 32u)
 /* false: the matrix instruction takes the codebook values before their scale and bias (1024 + b), which enter once a
  * sum; the weights' own rounding to fp16 is then left out of the product (within the products' stated tolerance) */
 #define EXACT_WEIGHTS true
@@ -83,8 +84,8 @@ extern "C" __global__ void exl3_tc_operands(struct exl3_tc_record record, unsign
 }
 ANEMONE_KERNEL(EXL3_TC_KERNEL_FILE, exl3_tc_operands, exl3_tc_record);
 
-/* one wavefront item: a strip of EXL3_TC_STRIP_OUTPUTS outputs by one K slice of one matrix of one job */
-template <uint32_t bits_x2>
+/* one wavefront item: a strip of NP pairs of output tiles by one K slice of one matrix of one job */
+template <uint32_t bits_x2, uint32_t NP>
 __device__ static __forceinline__ void tc_item(const uint32_t *codes, uint32_t inputs, uint32_t outputs,
                                                uint32_t strip, uint32_t slice, uint32_t slices,
                                                const struct expert_job_record *job, const half_t *operands,
@@ -95,26 +96,29 @@ __device__ static __forceinline__ void tc_item(const uint32_t *codes, uint32_t i
     /* a column that is not live reads the first column's operand: its sums are not stored */
     const uint32_t pair = job->pair_index[live ? column : 0u];
     const uint32_t steps = inputs / (4u * EXL3_TILE); /* a slice is a whole number of steps of four K tiles */
-    float4_t accumulator[STRIP_PAIRS][2];
-    exl3_stream_product<bits_x2, STRIP_PAIRS, EXACT_WEIGHTS>(codes, outputs / EXL3_TILE, strip * 2u * STRIP_PAIRS, 4u * (steps * slice / slices),
+    float4_t accumulator[NP][2];
+    exl3_stream_product<bits_x2, NP, EXACT_WEIGHTS>(codes, outputs / EXL3_TILE, strip * 2u * NP, 4u * (steps * slice / slices),
                                                              4u * (steps * (slice + 1u) / slices), operands + (uint64_t)pair * inputs, lane,
                                                              accumulator);
     if (live) {
         float *out = partials + (uint64_t)pair * outputs;
 #pragma unroll
-        for (uint32_t p = 0; p < STRIP_PAIRS; p++) {
+        for (uint32_t p = 0; p < NP; p++) {
 #pragma unroll
             for (uint32_t h = 0; h < 2u; h++) {
-                *(float4_t *)(out + exl3_stream_output(strip * 2u * STRIP_PAIRS, p, h, lane)) = accumulator[p][h];
+                *(float4_t *)(out + exl3_stream_output(strip * 2u * NP, p, h, lane)) = accumulator[p][h];
             }
         }
     }
 }
 
-/* launches 1 and 3: grid (outputs / EXL3_TC_STRIP_OUTPUTS, job_capacity, matrices * slices / 4), block 256: the block's four
+/* launches 1 and 3: grid (strips, job_capacity, matrices * slices / 4), block 256; a strip is EXL3_TC_STRIP_OUTPUTS outputs,
+ * or EXL3_TC_NARROW_STRIP_OUTPUTS where the grid's x says so (the same sums: a launch of few jobs, whose wide
+ * strips leave a SIMD one wavefront or none and which waits for each wavefront's own chain). The block's four
  * wavefronts take four consecutive (matrix, slice) items of one strip (a strip of fewer than four items: the items of
  * adjacent strips, the grid's x that many times smaller and its z 1). pass 0: gate and up; pass 1: down. A slice is
  * a whole number of steps of four K tiles. */
+template <uint32_t NP>
 __device__ static __forceinline__ void tc_products_block(const struct exl3_tc_record &record, unsigned char *arena, uint32_t block_x,
                                                          uint32_t block_y, uint32_t block_z, uint32_t lane, uint32_t wave)
 {
@@ -148,20 +152,20 @@ __device__ static __forceinline__ void tc_products_block(const struct exl3_tc_re
     }
     const uint32_t *codes = (const uint32_t *)(arena + matrix);
     switch (bits_x2) {
-    case 4u: tc_item<4u>(codes, inputs, outputs, strip, slice, slices, job, operands, partials, lane); break;
-    case 5u: tc_item<5u>(codes, inputs, outputs, strip, slice, slices, job, operands, partials, lane); break;
-    case 6u: tc_item<6u>(codes, inputs, outputs, strip, slice, slices, job, operands, partials, lane); break;
-    case 8u: tc_item<8u>(codes, inputs, outputs, strip, slice, slices, job, operands, partials, lane); break;
+    case 4u: tc_item<4u, NP>(codes, inputs, outputs, strip, slice, slices, job, operands, partials, lane); break;
+    case 5u: tc_item<5u, NP>(codes, inputs, outputs, strip, slice, slices, job, operands, partials, lane); break;
+    case 6u: tc_item<6u, NP>(codes, inputs, outputs, strip, slice, slices, job, operands, partials, lane); break;
+    case 8u: tc_item<8u, NP>(codes, inputs, outputs, strip, slice, slices, job, operands, partials, lane); break;
     default:
         /* a width this build does not decode (the prepare function refuses the one width of a record; a table's widths
          * are the caller's): zeros, so that the launches behind this one add nothing stale */
         if (lane % 16u < job->row_count) {
             float *out = partials + (uint64_t)job->pair_index[lane % 16u] * outputs;
 #pragma unroll
-            for (uint32_t p = 0; p < STRIP_PAIRS; p++) {
+            for (uint32_t p = 0; p < NP; p++) {
 #pragma unroll
                 for (uint32_t h = 0; h < 2u; h++) {
-                    *(float4_t *)(out + exl3_stream_output(strip * 2u * STRIP_PAIRS, p, h, lane)) = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
+                    *(float4_t *)(out + exl3_stream_output(strip * 2u * NP, p, h, lane)) = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
                 }
             }
         }
@@ -172,7 +176,13 @@ __device__ static __forceinline__ void tc_products_block(const struct exl3_tc_re
 extern "C" __global__ void __launch_bounds__(PRODUCT_THREADS, 4)
     exl3_tc_products(struct exl3_tc_record record, unsigned char *arena)
 {
-    tc_products_block(record, arena, blockIdx.x, blockIdx.y, blockIdx.z, threadIdx.x % WAVE, __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE));
+    const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const uint32_t outputs = record.pass != 0u ? tc_shape_of(record).hidden : record.intermediate;
+    if (gridDim.x * EXL3_TC_STRIP_OUTPUTS > outputs) { /* the same in every block */
+        tc_products_block<NARROW_STRIP_PAIRS>(record, arena, blockIdx.x, blockIdx.y, blockIdx.z, lane, wave);
+    } else {
+        tc_products_block<STRIP_PAIRS>(record, arena, blockIdx.x, blockIdx.y, blockIdx.z, lane, wave);
+    }
 }
 ANEMONE_KERNEL(EXL3_TC_KERNEL_FILE, exl3_tc_products, exl3_tc_record);
 

@@ -46,6 +46,14 @@ const char *exl3_tc_geometry_refusal(uint32_t hidden, uint32_t intermediate)
     return NULL;
 }
 
+/* the x of a products launch whose strips of EXL3_TC_STRIP_OUTPUTS fill `blocks` blocks a job: twice as many narrow strips
+ * where the whole launch is fewer than EXL3_TC_NARROW_BELOW_BLOCKS blocks */
+static uint32_t products_blocks(uint32_t blocks, uint32_t jobs, uint32_t items)
+{
+    const uint64_t z = (items + PRODUCT_WAVES - 1u) / PRODUCT_WAVES;
+    return blocks * jobs * z < EXL3_TC_NARROW_BELOW_BLOCKS ? blocks * (EXL3_TC_STRIP_OUTPUTS / EXL3_TC_NARROW_STRIP_OUTPUTS) : blocks;
+}
+
 /* detached_workspace: the workspace is not a range of the arena (exl3_tc_run_static names it by an offset of its own) */
 static result_status tc_prepare(const struct exl3_tc_record *record, uint64_t arena_byte_count,
                                 const struct backend_operations *backend, struct device_card *card,
@@ -129,8 +137,9 @@ static result_status tc_prepare(const struct exl3_tc_record *record, uint64_t ar
                EXL3_TC_STRIP_OUTPUTS * gate_up_strips, EXL3_TC_STRIP_OUTPUTS * down_strips);
         return STATUS_INVALID_ARGUMENT;
     }
-    const uint32_t grid_x[EXL3_TC_LAUNCHES] = {hidden / 128u, I / (EXL3_TC_STRIP_OUTPUTS * gate_up_strips), I / 128u,
-                                               hidden / (EXL3_TC_STRIP_OUTPUTS * down_strips), hidden / 128u};
+    const uint32_t gate_up_blocks = products_blocks(I / (EXL3_TC_STRIP_OUTPUTS * gate_up_strips), record->job_capacity, GATE_UP_ITEMS);
+    const uint32_t down_blocks = products_blocks(hidden / (EXL3_TC_STRIP_OUTPUTS * down_strips), record->job_capacity, DOWN_ITEMS);
+    const uint32_t grid_x[EXL3_TC_LAUNCHES] = {hidden / 128u, gate_up_blocks, I / 128u, down_blocks, hidden / 128u};
     const uint32_t grid_y[EXL3_TC_LAUNCHES] = {record->job_capacity, record->job_capacity, record->job_capacity,
                                                record->job_capacity, record->row_count};
     const uint32_t grid_z[EXL3_TC_LAUNCHES] = {2u, (GATE_UP_ITEMS + PRODUCT_WAVES - 1u) / PRODUCT_WAVES, 1u,

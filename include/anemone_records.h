@@ -290,6 +290,10 @@ ANEMONE_RECORD_HAS(expert_row_sum_arguments, 24);
 #define EXL3_TC_GATE_UP_SLICES 4u /* K slices of a gate/up product: partial sums kept apart, added in order */
 #define EXL3_TC_DOWN_SLICES 4u
 #define EXL3_TC_STRIP_OUTPUTS 64u /* outputs of one wavefront item of the products launches */
+#define EXL3_TC_NARROW_STRIP_OUTPUTS 32u /* of a launch of fewer than NARROW_BELOW_BLOCKS blocks: two wavefronts a SIMD */
+/* whole steps, narrow against wide, us: 96 and 128 blocks 27.8 / 30.4, 288 and 480 blocks 53.3 / 56.8, 512 blocks 54.9 /
+ * 54.3, 768 blocks 48.5 / 46.4 (hidden 2048 and intermediate 768, 5120 and 1536, 4096 and 2048, 2048 and 1024) */
+#define EXL3_TC_NARROW_BELOW_BLOCKS 512u
 
 struct exl3_tc_record {
     uint64_t jobs_offset;      /* read: struct expert_job_record [job_capacity], empty ones anywhere */

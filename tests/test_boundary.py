@@ -180,6 +180,13 @@ def tc_record(**changes):
     return r
 
 
+@pytest.mark.parametrize("jobs,grids", [(3, [64, 128]), (7, [64, 128]), (8, [32, 64]), (64, [32, 64])])
+def test_tc_prepare_takes_narrow_strips_below_512_blocks(fake, jobs, grids):
+    launches = amd.launches_of(5)
+    assert amd.library().exl3_tc_prepare(C.byref(tc_record(job_capacity=jobs)), ARENA, fake.address, fake.card, launches) == 0
+    assert [list(launches[index].grid) for index in (1, 3)] == [[grids[0], jobs, 2], [grids[1], jobs, 1]]
+
+
 def test_tc_prepare_geometry_and_refusals(fake):
     lib = amd.library()
     launches = amd.launches_of(5)

@@ -382,3 +382,23 @@ def test_thin_product_of_short_and_long_slices(amd, card, inputs, width):
     got = card.download(record.products_offset, rows * outputs * 4, np.float32).reshape(rows, outputs)
     want, magnitudes = operands.astype(np.float64) @ weights, np.abs(operands.astype(np.float64)) @ np.abs(weights)
     assert np.all(np.abs(got - want) <= inputs * 2.0 ** -24 * magnitudes)
+
+
+@pytest.mark.parametrize("hidden,inner,width_choices", [(512, 384, [2, 3, 4]), (256, 128, [40])])
+def test_narrow_strips_of_the_fused_decode_give_the_same_bits(amd, card, hidden, inner, width_choices):
+    """A products launch of few blocks takes strips of 32 outputs in place of 64 (anemone_amd/host/exl3_tc.c); the kernel
+    reads which off its grid: the same launches with the grids of the wide strips give every output's bits."""
+    say("narrow strips", hidden, inner, width_choices)
+    rows, picks = 3, 4
+    layer, _, _, _ = build_layer(amd, card, hidden, inner, 64, picks, rows, 13, width_choices)
+    layer.set_rows(to_bf16(normals(29, rows * hidden)).reshape(rows, hidden), rows)
+    card.run(layer.projection_launch())
+    card.run(layer.select_launch(0))
+    launches, outputs = layer.tc_launches(), []
+    assert [launches[index].grid[0] for index in (1, 3)] == [inner // 32, hidden // 32]
+    for _ in range(2):
+        card.upload(layer.out_offset, np.full(rows * hidden * 4, 0xEE, dtype=np.uint8))
+        card.run(launches)
+        outputs.append(layer.output().view(np.uint32).copy())
+        launches[1].grid[0], launches[3].grid[0] = inner // 64, hidden // 64
+    assert np.array_equal(outputs[0], outputs[1]) and not np.all(outputs[0] == 0xEEEEEEEE)
