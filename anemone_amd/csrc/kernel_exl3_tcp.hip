@@ -29,6 +29,7 @@
 #define TCP_STEP_INPUTS 64u
 #define TCP_DIES 8u         /* the card's dies (XCDs), each with a level-2 cache of its own: blocks are dealt to them in turn */
 #define TCP_BATCH 4u        /* columns the element-wise launches take at a time */
+#define TCP_THIN_PLACES 4u  /* places of a block of a thin call's element-wise launches: one a wavefront */
 #define TCP_WAVE_BLOCKS 4u  /* blocks of 128 channels a wavefront of an element-wise launch takes: a row of sixteen lanes each */
 
 struct tcp_shape {
@@ -181,6 +182,23 @@ __device__ static __forceinline__ bool tcp_lane_channels(uint32_t width, uint32_
     return channel < width;
 }
 
+/* eight values of a row as an operand of one matrix: fp16(H128(x suh) / sqrt(128)) */
+__device__ static __forceinline__ uint4_t tcp_operand(uint4_t load, const float (&scale)[8], uint32_t lane)
+{
+    float v[8];
+    unpack_bf16x8(load, v);
+#pragma unroll
+    for (uint32_t j = 0; j < 8u; j++) {
+        v[j] = __fmul_rn(v[j], scale[j]);
+    }
+    row_hadamard128(v, lane);
+#pragma unroll
+    for (uint32_t j = 0; j < 8u; j++) {
+        v[j] = __fmul_rn(v[j], EXL3_NORMALIZATION);
+    }
+    return pack_half8(v);
+}
+
 /* launch 2: grid (ceil(hidden / 512), chunk capacity, EXL3_TCP_COLUMN_PARTS), block 64: the gate and the up operands of
  * a part of a chunk's pairs, by place: fp16(H128(x suh) / sqrt(128)); a row is read once for both */
 extern "C" __global__ void exl3_tcp_operands(struct exl3_tcp_record record, unsigned char *arena)
@@ -220,28 +238,62 @@ extern "C" __global__ void exl3_tcp_operands(struct exl3_tcp_record record, unsi
         }
 #pragma unroll
         for (uint32_t i = 0; i < TCP_BATCH; i++) {
-            float x[8];
-            unpack_bf16x8(loads[i], x);
+            const bool kept = first + i < last_column;
 #pragma unroll
             for (uint32_t projection = 0; projection < 2u; projection++) {
-                float v[8];
-#pragma unroll
-                for (uint32_t j = 0; j < 8u; j++) {
-                    v[j] = __fmul_rn(x[j], scale[projection][j]);
-                }
-                row_hadamard128(v, lane);
-#pragma unroll
-                for (uint32_t j = 0; j < 8u; j++) {
-                    v[j] = __fmul_rn(v[j], EXL3_NORMALIZATION);
-                }
-                if (first + i < last_column) {
-                    *(uint4_t *)(operands + ((uint64_t)projection * shape.pairs + place[i]) * shape.hidden + channel) = pack_half8(v);
+                const uint4_t operand = tcp_operand(loads[i], scale[projection], lane);
+                if (kept) {
+                    *(uint4_t *)(operands + ((uint64_t)projection * shape.pairs + place[i]) * shape.hidden + channel) = operand;
                 }
             }
         }
     }
 }
 ANEMONE_KERNEL(EXL3_TCP_KERNEL_FILE, exl3_tcp_operands, exl3_tcp_record);
+
+/* The element-wise launches of a thin call (exl3_tcp_is_thin): grid (ceil(width / 512), ceil(pairs / 4)), block 256: a
+ * wavefront a place. By chunks, as above, a handful of pairs an expert is a wavefront or two a SIMD that walk their columns
+ * one batch behind the other, among ten times as many blocks that find none; by places every pair is a wavefront of its
+ * own and reads its expert's scales itself. The same operands. 203 rows of 256 experts,
+ * 8 picks, hidden 4096, intermediate 2048: operands 25 -> 14 us, activate 35 -> 17, the call 881 -> 851.
+ * false past the pairs or the width */
+__device__ static __forceinline__ bool tcp_thin_place(const tcp_shape &shape, const struct exl3_tcp_record &record, const unsigned char *arena,
+                                                      uint32_t width, uint32_t &place, uint32_t &pair, uint32_t &expert, uint32_t &channel, uint32_t &lane)
+{
+    lane = threadIdx.x % WAVE;
+    place = blockIdx.y * TCP_THIN_PLACES + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    channel = (blockIdx.x * TCP_WAVE_BLOCKS + lane / 16u) * EXL3_TRANSFORM + 8u * (lane % 16u);
+    if (place >= shape.pairs || channel >= width) {
+        return false;
+    }
+    pair = ((const uint32_t *)(arena + record.workspace_offset + shape.layout.sorted))[place];
+    expert = ((const struct router_pick *)(arena + record.picks_offset))[pair].expert;
+    return true;
+}
+
+extern "C" __global__ void __launch_bounds__(TCP_THIN_PLACES * WAVE) exl3_tcp_operands_thin(struct exl3_tcp_record record, unsigned char *arena)
+{
+    const tcp_shape shape = tcp_shape_of(record);
+    uint32_t place, pair, expert, channel, lane;
+    if (!tcp_thin_place(shape, record, arena, shape.hidden, place, pair, expert, channel, lane)) {
+        return;
+    }
+    const uint4_t load = *(const uint4_t *)((const uint16_t *)(arena + record.hidden_offset) + (uint64_t)(pair / shape.picks) * shape.hidden + channel);
+    uint16_t *operands = (uint16_t *)(arena + record.workspace_offset + shape.layout.operands);
+    uint4_t scales[2];
+#pragma unroll
+    for (uint32_t projection = 0; projection < 2u; projection++) {
+        scales[projection] = *(const uint4_t *)((const uint16_t *)(arena + tcp_matrix_of(record, arena, expert, projection) +
+                                                                   exl3_code_bytes(shape.hidden, shape.intermediate, tcp_bits_x2(record, arena, expert, projection))) + channel);
+    }
+#pragma unroll
+    for (uint32_t projection = 0; projection < 2u; projection++) {
+        float scale[8];
+        unpack_half8(scales[projection], scale);
+        *(uint4_t *)(operands + ((uint64_t)projection * shape.pairs + place) * shape.hidden + channel) = tcp_operand(load, scale, lane);
+    }
+}
+ANEMONE_KERNEL(EXL3_TCP_KERNEL_FILE, exl3_tcp_operands_thin, exl3_tcp_record);
 
 /*
  * The GEMM block: 256 outputs by one chunk of at most EXL3_TCP_CHUNK_PAIRS pairs of one expert, four wavefronts of 64
@@ -688,6 +740,36 @@ extern "C" __global__ void __launch_bounds__(TCP_GEMM_THREADS, 4) exl3_tcp_gemm_
 }
 ANEMONE_KERNEL(EXL3_TCP_KERNEL_FILE, exl3_tcp_gemm_thin, exl3_tcp_record);
 
+/* eight gate and eight up products as a down operand: gate = H128(gate products) / sqrt(128) x svh, up the same, the SwiGLU
+ * with its limit, x the down matrix's suh, H128, fp16 */
+__device__ static __forceinline__ uint4_t tcp_activated(const float4_t (&loads)[4], const float (&gs)[8], const float (&us)[8], const float (&ds)[8],
+                                                        float limit, uint32_t lane)
+{
+    float g[8], u[8], v[8];
+#pragma unroll
+    for (uint32_t j = 0; j < 8u; j++) {
+        g[j] = loads[j / 4u][j % 4u];
+        u[j] = loads[2u + j / 4u][j % 4u];
+    }
+    row_hadamard128(g, lane);
+    row_hadamard128(u, lane);
+#pragma unroll
+    for (uint32_t j = 0; j < 8u; j++) {
+        const float gate = __fmul_rn(__fmul_rn(g[j], EXL3_NORMALIZATION), gs[j]);
+        const float up = __fmul_rn(__fmul_rn(u[j], EXL3_NORMALIZATION), us[j]);
+        const float bounded_gate = limit > 0.0f ? fminf(gate, limit) : gate;
+        const float bounded_up = limit > 0.0f ? fminf(fmaxf(up, -limit), limit) : up;
+        const float hidden = __fmul_rn(det_silu(bounded_gate), bounded_up);
+        v[j] = __fmul_rn(hidden, ds[j]);
+    }
+    row_hadamard128(v, lane);
+#pragma unroll
+    for (uint32_t j = 0; j < 8u; j++) {
+        v[j] = __fmul_rn(v[j], EXL3_NORMALIZATION);
+    }
+    return pack_half8(v);
+}
+
 /* launch 4: grid (ceil(intermediate / 512), chunk capacity, EXL3_TCP_COLUMN_PARTS), block 64: per pair of a part of the chunk, gate = H128(gate products) /
  * sqrt(128) x svh, up the same, the SwiGLU with its limit, x the down matrix's suh, H128 -> the fp16 down operand */
 extern "C" __global__ void exl3_tcp_activate(struct exl3_tcp_record record, unsigned char *arena)
@@ -730,35 +812,38 @@ extern "C" __global__ void exl3_tcp_activate(struct exl3_tcp_record record, unsi
         }
 #pragma unroll
         for (uint32_t i = 0; i < BATCH; i++) {
-            float g[8], u[8], v[8];
-#pragma unroll
-            for (uint32_t j = 0; j < 8u; j++) {
-                g[j] = loads[i][j / 4u][j % 4u];
-                u[j] = loads[i][2u + j / 4u][j % 4u];
-            }
-            row_hadamard128(g, lane);
-            row_hadamard128(u, lane);
-#pragma unroll
-            for (uint32_t j = 0; j < 8u; j++) {
-                const float gate = __fmul_rn(__fmul_rn(g[j], EXL3_NORMALIZATION), gs[j]);
-                const float up = __fmul_rn(__fmul_rn(u[j], EXL3_NORMALIZATION), us[j]);
-                const float bounded_gate = limit > 0.0f ? fminf(gate, limit) : gate;
-                const float bounded_up = limit > 0.0f ? fminf(fmaxf(up, -limit), limit) : up;
-                const float hidden = __fmul_rn(det_silu(bounded_gate), bounded_up);
-                v[j] = __fmul_rn(hidden, ds[j]);
-            }
-            row_hadamard128(v, lane);
-#pragma unroll
-            for (uint32_t j = 0; j < 8u; j++) {
-                v[j] = __fmul_rn(v[j], EXL3_NORMALIZATION);
-            }
+            const uint4_t operand = tcp_activated(loads[i], gs, us, ds, limit, lane);
             if (first + i < last_column) {
-                *(uint4_t *)(operands + place[i] * I + channel) = pack_half8(v);
+                *(uint4_t *)(operands + place[i] * I + channel) = operand;
             }
         }
     }
 }
 ANEMONE_KERNEL(EXL3_TCP_KERNEL_FILE, exl3_tcp_activate, exl3_tcp_record);
+
+extern "C" __global__ void __launch_bounds__(TCP_THIN_PLACES * WAVE) exl3_tcp_activate_thin(struct exl3_tcp_record record, unsigned char *arena)
+{
+    const tcp_shape shape = tcp_shape_of(record);
+    const uint32_t H = shape.hidden, I = shape.intermediate;
+    uint32_t place, pair, expert, channel, lane;
+    if (!tcp_thin_place(shape, record, arena, I, place, pair, expert, channel, lane)) {
+        return;
+    }
+    unsigned char *workspace = arena + record.workspace_offset;
+    const float *products = (const float *)(workspace + shape.layout.gate_up);
+    const float4_t *gate = (const float4_t *)(products + (uint64_t)place * I + channel), *up = (const float4_t *)(products + ((uint64_t)shape.pairs + place) * I + channel);
+    const float4_t loads[4] = {gate[0], gate[1], up[0], up[1]};
+    const uint4_t scales[3] = {
+        *(const uint4_t *)((const uint16_t *)(arena + tcp_matrix_of(record, arena, expert, 0u) + exl3_code_bytes(H, I, tcp_bits_x2(record, arena, expert, 0u))) + H + channel),
+        *(const uint4_t *)((const uint16_t *)(arena + tcp_matrix_of(record, arena, expert, 1u) + exl3_code_bytes(H, I, tcp_bits_x2(record, arena, expert, 1u))) + H + channel),
+        *(const uint4_t *)((const uint16_t *)(arena + tcp_matrix_of(record, arena, expert, 2u) + exl3_code_bytes(I, H, tcp_bits_x2(record, arena, expert, 2u))) + channel)};
+    float gs[8], us[8], ds[8];
+    unpack_half8(scales[0], gs);
+    unpack_half8(scales[1], us);
+    unpack_half8(scales[2], ds);
+    *(uint4_t *)((uint16_t *)(workspace + shape.layout.operands) + (uint64_t)place * I + channel) = tcp_activated(loads, gs, us, ds, record.activation_limit, lane);
+}
+ANEMONE_KERNEL(EXL3_TCP_KERNEL_FILE, exl3_tcp_activate_thin, exl3_tcp_record);
 
 /* launch 6: grid (ceil(hidden / 512), row_count), block 64: a row's pairs in slot order */
 extern "C" __global__ void exl3_tcp_combine(struct exl3_tcp_record record, unsigned char *arena)

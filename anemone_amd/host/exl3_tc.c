@@ -21,6 +21,7 @@
 #define PRODUCT_THREADS 256u
 #define PRODUCT_WAVES 4u
 #define MOST_GRID_ROWS 65535u
+#define THIN_PLACES 4u /* pairs of a block of a thin prefill's element-wise launches: one a wavefront */
 
 /* a block's four wavefronts take four items: of one strip (its matrices x slices a multiple of four: z blocks a strip)
  * or of adjacent strips (a divisor of four: that many strips a block) */
@@ -207,7 +208,8 @@ result_status exl3_tc_prepare_detached(const struct exl3_tc_record *record, uint
  *   combine     exl3_tcp_combine    (hidden / 128, rows, 1)                          64
  * chunk capacity = pairs / EXL3_TCP_CHUNK_PAIRS + experts: an expert's pairs cut in chunks of EXL3_TCP_CHUNK_PAIRS (160), the
  * last ragged. A thin call (exl3_tcp_is_thin) takes exl3_tcp_gemm_thin for both GEMM passes, its grid's z
- * EXL3_TCP_THIN_PARTS times as many.
+ * EXL3_TCP_THIN_PARTS times as many, and exl3_tcp_operands_thin and exl3_tcp_activate_thin of (width / 512, pairs / 4)
+ * blocks of 256.
  */
 static bool exl3_tcp_is_thin(uint64_t pairs, uint64_t experts, uint32_t hidden, uint32_t intermediate)
 {
@@ -270,18 +272,21 @@ static result_status tcp_prepare(const struct exl3_tcp_record *record, uint64_t 
         }
         return STATUS_INVALID_ARGUMENT;
     }
+    static const char *const names_of[2][EXL3_TCP_LAUNCHES] = {
+        {"exl3_tcp_count", "exl3_tcp_place", "exl3_tcp_operands", "exl3_tcp_gemm", "exl3_tcp_activate", "exl3_tcp_gemm", "exl3_tcp_combine"},
+        {"exl3_tcp_count", "exl3_tcp_place", "exl3_tcp_operands_thin", "exl3_tcp_gemm_thin", "exl3_tcp_activate_thin", "exl3_tcp_gemm_thin",
+         "exl3_tcp_combine"}};
     const bool thin = exl3_tcp_is_thin(pairs, E, H, I);
-    const char *const gemm = thin ? "exl3_tcp_gemm_thin" : "exl3_tcp_gemm";
-    const uint32_t parts = thin ? EXL3_TCP_THIN_PARTS : 1u;
-    const char *const names[EXL3_TCP_LAUNCHES] = {"exl3_tcp_count",    "exl3_tcp_place", "exl3_tcp_operands", gemm,
-                                                  "exl3_tcp_activate", gemm,             "exl3_tcp_combine"};
+    const char *const *const names = names_of[thin ? 1 : 0];
     const uint32_t blocks = (uint32_t)((rows + ROUTER_SORT_ROWS - 1u) / ROUTER_SORT_ROWS), capacity = layout.chunk_capacity;
-    /* an element-wise launch's wavefront takes four blocks of 128 channels */
+    /* an element-wise launch's wavefront takes four blocks of 128 channels, of a part of a chunk's pairs or of one pair */
     const uint32_t grid_x[EXL3_TCP_LAUNCHES] = {blocks, blocks, (H + 511u) / 512u, (I + EXL3_TCP_BLOCK_OUTPUTS - 1u) / EXL3_TCP_BLOCK_OUTPUTS,
                                                 (I + 511u) / 512u, (H + EXL3_TCP_BLOCK_OUTPUTS - 1u) / EXL3_TCP_BLOCK_OUTPUTS, (H + 511u) / 512u};
-    const uint32_t grid_y[EXL3_TCP_LAUNCHES] = {1u, 1u, capacity, capacity, capacity, capacity, record->row_count};
-    const uint32_t grid_z[EXL3_TCP_LAUNCHES] = {1u, 1u, EXL3_TCP_COLUMN_PARTS, 2u * parts, EXL3_TCP_COLUMN_PARTS, parts, 1u};
-    const uint32_t threads[EXL3_TCP_LAUNCHES] = {512u, 512u, WAVE_THREADS, PRODUCT_THREADS, WAVE_THREADS, PRODUCT_THREADS, WAVE_THREADS};
+    const uint32_t element_y = thin ? (uint32_t)((pairs + THIN_PLACES - 1u) / THIN_PLACES) : capacity, element_z = thin ? 1u : EXL3_TCP_COLUMN_PARTS;
+    const uint32_t element_threads = thin ? THIN_PLACES * WAVE_THREADS : WAVE_THREADS, gemm_z = thin ? EXL3_TCP_THIN_PARTS : 1u;
+    const uint32_t grid_y[EXL3_TCP_LAUNCHES] = {1u, 1u, element_y, capacity, element_y, capacity, record->row_count};
+    const uint32_t grid_z[EXL3_TCP_LAUNCHES] = {1u, 1u, element_z, 2u * gemm_z, element_z, gemm_z, 1u};
+    const uint32_t threads[EXL3_TCP_LAUNCHES] = {512u, 512u, element_threads, PRODUCT_THREADS, element_threads, PRODUCT_THREADS, WAVE_THREADS};
     struct kernel_launch launches[EXL3_TCP_LAUNCHES];
     for (uint32_t index = 0; index < EXL3_TCP_LAUNCHES; index++) {
         uint32_t kernel = BACKEND_NO_KERNEL;

@@ -502,6 +502,9 @@ def test_tcp_prepare_takes_the_thin_gemm_up_to_sixteen_pairs_an_expert(fake, row
     for index, outputs, matrices in ((3, record.intermediate, 2), (5, record.hidden, 1)):
         assert fake.handles[launches[index].kernel][1] == ("exl3_tcp_gemm_thin" if thin else "exl3_tcp_gemm")
         assert list(launches[index].grid) == [(outputs + 255) // 256, capacity, matrices * (4 if thin else 1)] and launches[index].block[0] == 256
+    for index, name, width in ((2, "exl3_tcp_operands", record.hidden), (4, "exl3_tcp_activate", record.intermediate)):
+        assert fake.handles[launches[index].kernel][1] == name + ("_thin" if thin else "")
+        assert list(launches[index].grid) == [(width + 511) // 512] + ([rows * 2, 1] if thin else [capacity, 10])
 
 
 def test_tcp_prepare_geometry_and_refusals(fake):
