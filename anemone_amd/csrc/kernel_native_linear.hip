@@ -54,16 +54,17 @@ __device__ static __forceinline__ void native_vectors_of(const struct wide_pair 
 #define NATIVE_B128_SLOTS 3u
 #define NATIVE_B128_GATE_UP_WAVES 2
 #define NATIVE_B128_DOWN_WAVES 2
-template <bool BYTES, bool B128 = false>
+template <bool BYTES, uint32_t TILES> /* tiles of a wavefront, of its matrices together */
 struct native_depths {
-    static constexpr uint32_t SLOTS = BYTES ? 3u : 2u, DEPTH = BYTES ? NATIVE_E4M3_STAGES : NATIVE_E2M1_STAGES;
+    static constexpr uint32_t SLOTS = !BYTES && TILES == 8u ? 2u : 3u, DEPTH = BYTES ? NATIVE_E4M3_STAGES : NATIVE_E2M1_STAGES;
 };
 
 template <bool BYTES, uint32_t STRIP, uint32_t GROUP, bool B128 = false>
 __device__ static __forceinline__ void native_expert_gate_up(const struct wide_expert_gate_up_arguments &arguments, unsigned char *arena)
 {
     constexpr uint32_t COLUMN_BLOCKS = 4u * GROUP;
-    typedef native_chain<2, BYTES, STRIP, COLUMN_BLOCKS, native_depths<BYTES, B128>::SLOTS, native_depths<BYTES, B128>::DEPTH, B128> chain_type;
+    typedef native_depths<BYTES, 2u * STRIP> depths;
+    typedef native_chain<2, BYTES, STRIP, COLUMN_BLOCKS, depths::SLOTS, depths::DEPTH, B128> chain_type;
     constexpr uint32_t TILES = chain_type::TILES;
     static_assert(STRIP == 1u || STRIP % 2u == 0u, "a quantizer block of 32 outputs is two strips, or strips are whole blocks");
     extern __shared__ __attribute__((aligned(16))) unsigned char window[];
@@ -94,11 +95,12 @@ __device__ static __forceinline__ void native_expert_gate_up(const struct wide_e
     wide_gate_up_finish<STRIP, COLUMN_BLOCKS, B128>(arguments, arena, window, columns, pair_count, block_strip, tile0, wave, lane, chain);
 }
 
-template <bool BYTES, uint32_t GROUP, bool B128 = false>
+template <bool BYTES, uint32_t DOWN_STRIP, uint32_t GROUP, bool B128 = false>
 __device__ static __forceinline__ void native_expert_down(const struct wide_expert_down_arguments &arguments, unsigned char *arena)
 {
     constexpr uint32_t COLUMN_BLOCKS = 4u * GROUP;
-    typedef native_chain<1, BYTES, (BYTES ? 2u : 8u), COLUMN_BLOCKS, native_depths<BYTES, B128>::SLOTS, native_depths<BYTES, B128>::DEPTH, B128> chain_type;
+    typedef native_depths<BYTES, DOWN_STRIP> depths;
+    typedef native_chain<1, BYTES, DOWN_STRIP, COLUMN_BLOCKS, depths::SLOTS, depths::DEPTH, B128> chain_type;
     constexpr uint32_t TILES = chain_type::TILES, STRIP = chain_type::STRIP;
     extern __shared__ __attribute__((aligned(16))) unsigned char window[];
     __shared__ struct wide_pair columns[COLUMN_BLOCKS * 16u];
@@ -138,9 +140,22 @@ extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_E2M1_WAVES) 
 ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_gate_up_1, wide_expert_gate_up_arguments);
 extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_E2M1_WAVES) native_expert_down_1(struct wide_expert_down_arguments arguments, unsigned char *arena)
 {
-    native_expert_down<false, NATIVE_E2M1_COLUMN_BLOCKS / 4u>(arguments, arena);
+    native_expert_down<false, 8u, NATIVE_E2M1_COLUMN_BLOCKS / 4u>(arguments, arena);
 }
 ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_down_1, wide_expert_down_arguments);
+/* the same of half the strips, at three wavefronts a SIMD: for launches of few pairs an expert whose blocks fill their last
+ * round better so (anemone_amd/host/linear.c, native_takes_narrow, holds both sides' times) */
+#define NATIVE_E2M1_NARROW_WAVES 3 /* 168 registers */
+extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_E2M1_NARROW_WAVES) native_expert_gate_up_narrow_1(struct wide_expert_gate_up_arguments arguments, unsigned char *arena)
+{
+    native_expert_gate_up<false, 2u, NATIVE_E2M1_COLUMN_BLOCKS / 4u>(arguments, arena);
+}
+ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_gate_up_narrow_1, wide_expert_gate_up_arguments);
+extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_E2M1_NARROW_WAVES) native_expert_down_narrow_1(struct wide_expert_down_arguments arguments, unsigned char *arena)
+{
+    native_expert_down<false, 4u, NATIVE_E2M1_COLUMN_BLOCKS / 4u>(arguments, arena);
+}
+ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_down_narrow_1, wide_expert_down_arguments);
 #define NATIVE_E4M3_WAVES 3 /* 150 and 152 registers (with four sets of weight registers the down launch took 170 left to itself, and at two wavefronts a SIMD 487 against 461 us) */
 extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_E4M3_WAVES) native_expert_gate_up_e4m3_1(struct wide_expert_gate_up_arguments arguments, unsigned char *arena)
 {
@@ -149,7 +164,7 @@ extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_E4M3_WAVES) 
 ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_gate_up_e4m3_1, wide_expert_gate_up_arguments);
 extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_E4M3_WAVES) native_expert_down_e4m3_1(struct wide_expert_down_arguments arguments, unsigned char *arena)
 {
-    native_expert_down<true, NATIVE_E4M3_COLUMN_BLOCKS / 4u>(arguments, arena);
+    native_expert_down<true, 2u, NATIVE_E4M3_COLUMN_BLOCKS / 4u>(arguments, arena);
 }
 ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_down_e4m3_1, wide_expert_down_arguments);
 
@@ -163,7 +178,7 @@ extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_B128_GATE_UP
 ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_gate_up_b128_1, wide_expert_gate_up_arguments);
 extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_B128_DOWN_WAVES) native_expert_down_b128_1(struct wide_expert_down_arguments arguments, unsigned char *arena)
 {
-    native_expert_down<true, NATIVE_E4M3_COLUMN_BLOCKS / 4u, true>(arguments, arena);
+    native_expert_down<true, 2u, NATIVE_E4M3_COLUMN_BLOCKS / 4u, true>(arguments, arena);
 }
 ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_down_b128_1, wide_expert_down_arguments);
 

@@ -592,6 +592,25 @@ result_status linear_wide_kernels_prepare(const struct backend_operations *backe
 
 /* block128: the launches of WEIGHT_FORMAT_E4M3_BLOCK128 experts (four: the hidden vectors' quantizer is a launch of its
  * own between the products); else those of the reference's formats (three) */
+/* Whether a launch of the 4-bit native kernels takes strips of `outputs` a block (three blocks a CU) in place of twice as
+ * many (two). At up to 32 pairs an expert, a tile of pairs an expert, the launch is its weights' way from memory, and what
+ * differs is how full its last round of blocks is: 768 blocks of one unit, or 512 of two. Strips of half the tiles against
+ * whole ones, us: gate/up of 5120 x 1536 x 64 experts (384 whole blocks) 95.5 / 97.0, of 4096 x 1152 x 256 (1280) 196 / 214,
+ * of 5120 x 1024 x 128 (512) 128 / 120, of 4096 x 1664 x 128 (896) 165 / 159; down of 1536 x 5120 x 64 (640) 54 / 63, of
+ * 768 x 2048 x 128 (512) 23.7 / 20.7. Beyond 32 pairs whole strips read LDS half as often (70 an expert: 104 / 113);
+ * fewer than 1,024 inputs are blocks that are mostly start and finish (down of 896 x 3072 x 128, 768 whole blocks: the step
+ * 155 / 149). */
+static bool native_takes_narrow(const struct matrix_shape_record *shape, uint32_t outputs, uint32_t tile_count, uint64_t pairs)
+{
+    const uint64_t full_tiles = pairs / WIDE_TILE_PAIRS, experts = tile_count > full_tiles ? tile_count - full_tiles : 1u;
+    if (pairs > 32u * experts || shape->input_size < 1024u) {
+        return false;
+    }
+    const uint64_t narrow = ((uint64_t)shape->output_size + outputs - 1u) / outputs * experts;
+    const uint64_t whole = ((uint64_t)shape->output_size + 2u * outputs - 1u) / (2u * outputs) * experts;
+    return (narrow + 767u) / 768u * 768u < (whole + 511u) / 512u * 1024u;
+}
+
 static result_status wide_experts_prepare(const struct linear_wide_experts_description *description, uint64_t arena_byte_count,
                                           const struct linear_kernels_record *linear_kernels,
                                           const struct linear_wide_kernels_record *kernels, const struct linear_native_kernels_record *native_kernels,
@@ -682,9 +701,21 @@ static result_status wide_experts_prepare(const struct linear_wide_experts_descr
         down->output_size, down->input_size, description->tile_count, (uint32_t)pairs};
     const struct expert_row_sum_arguments row_sum_record = {experts->pair_output.byte_offset, experts->row_output.byte_offset,
                                                             down->output_size, experts->pairs_per_row};
-    const uint32_t wider = native && !bytes ? 2u : 1u; /* 4-bit weights in gfx950's lane order: strips of twice the tiles */
-    const uint32_t block_outputs = wider * 4u * strip_outputs;
-    const uint32_t gate_up_outputs = bytes ? WIDE_GATE_UP_E4M3_BLOCK_OUTPUTS : wider * WIDE_GATE_UP_BLOCK_OUTPUTS;
+    uint32_t block_outputs = 4u * strip_outputs, gate_up_outputs = bytes ? WIDE_GATE_UP_E4M3_BLOCK_OUTPUTS : WIDE_GATE_UP_BLOCK_OUTPUTS;
+    if (native && !bytes) { /* 4-bit weights in gfx950's lane order: strips of twice the tiles, or of as many */
+        if (native_kernels->native_expert_gate_up_narrow != BACKEND_NO_KERNEL &&
+            native_takes_narrow(gate_up, gate_up_outputs, description->tile_count, pairs)) {
+            gate_up_kernel = native_kernels->native_expert_gate_up_narrow;
+        } else {
+            gate_up_outputs *= 2u;
+        }
+        if (native_kernels->native_expert_down_narrow != BACKEND_NO_KERNEL &&
+            native_takes_narrow(down, block_outputs, description->tile_count, pairs)) {
+            down_kernel = native_kernels->native_expert_down_narrow;
+        } else {
+            block_outputs *= 2u;
+        }
+    }
     struct kernel_launch launches[LINEAR_WIDE_EXPERTS_BLOCK128_LAUNCH_COUNT];
     uint32_t at = 0;
     launch_fill(&launches[at++], gate_up_kernel,
@@ -733,15 +764,18 @@ result_status linear_native_kernels_prepare(const struct backend_operations *bac
     static const struct {
         const char *name;
         uint32_t record_bytes;
-    } wanted[6] = {{KERNEL_NATIVE_EXPERT_GATE_UP_STEM "1", sizeof(struct wide_expert_gate_up_arguments)},
-                   {KERNEL_NATIVE_EXPERT_DOWN_STEM "1", sizeof(struct wide_expert_down_arguments)},
-                   {KERNEL_NATIVE_EXPERT_GATE_UP_STEM "e4m3_1", sizeof(struct wide_expert_gate_up_arguments)},
-                   {KERNEL_NATIVE_EXPERT_DOWN_STEM "e4m3_1", sizeof(struct wide_expert_down_arguments)},
-                   {KERNEL_NATIVE_EXPERT_GATE_UP_STEM "b128_1", sizeof(struct wide_expert_gate_up_arguments)},
-                   {KERNEL_NATIVE_EXPERT_DOWN_STEM "b128_1", sizeof(struct wide_expert_down_arguments)}};
-    uint32_t handles[6];
+    } wanted[] = {{KERNEL_NATIVE_EXPERT_GATE_UP_STEM "1", sizeof(struct wide_expert_gate_up_arguments)},
+                  {KERNEL_NATIVE_EXPERT_DOWN_STEM "1", sizeof(struct wide_expert_down_arguments)},
+                  {KERNEL_NATIVE_EXPERT_GATE_UP_STEM "e4m3_1", sizeof(struct wide_expert_gate_up_arguments)},
+                  {KERNEL_NATIVE_EXPERT_DOWN_STEM "e4m3_1", sizeof(struct wide_expert_down_arguments)},
+                  {KERNEL_NATIVE_EXPERT_GATE_UP_STEM "b128_1", sizeof(struct wide_expert_gate_up_arguments)},
+                  {KERNEL_NATIVE_EXPERT_DOWN_STEM "b128_1", sizeof(struct wide_expert_down_arguments)},
+                  {KERNEL_NATIVE_EXPERT_GATE_UP_STEM "narrow_1", sizeof(struct wide_expert_gate_up_arguments)},
+                  {KERNEL_NATIVE_EXPERT_DOWN_STEM "narrow_1", sizeof(struct wide_expert_down_arguments)}};
+    enum { WANTED = sizeof wanted / sizeof wanted[0] };
+    uint32_t handles[WANTED];
     _Static_assert(sizeof(struct linear_native_kernels_record) == sizeof handles, "a handle a member, in the members' order");
-    for (uint32_t i = 0; i < 6u; i++) {
+    for (uint32_t i = 0; i < WANTED; i++) {
         const result_status status = backend->kernel_prepare(card, KERNEL_FILE_NATIVE_LINEAR, wanted[i].name, wanted[i].record_bytes, &handles[i]);
         if (status != STATUS_OK) {
             REFUSE("linear_native_kernels_prepare: %s: %s", wanted[i].name, status_text(status));

@@ -607,6 +607,8 @@ struct linear_native_kernels_record {
     uint32_t native_expert_down_e4m3;
     uint32_t native_expert_gate_up_b128; /* E4M3_BLOCK128_GFX950 */
     uint32_t native_expert_down_b128;
+    uint32_t native_expert_gate_up_narrow; /* E2M1_GFX950, strips of half the tiles */
+    uint32_t native_expert_down_narrow;
 };
 MUST_CHECK result_status linear_native_kernels_prepare(const struct backend_operations *backend, struct device_card *card,
                                                        uint32_t arithmetic_class, struct linear_native_kernels_record *kernels_out);

@@ -202,3 +202,30 @@ def test_native_job_table_kernels_equal_the_reference_lay_out(amd, card, hidden,
         assert differing.size == 0, (name, differing[:8], per)
         if not (fmt == B128 and name == "hidden_operands"):  # the quantizer of 128 values a scale writes no operands
             assert a.reshape(-1)[:count].tobytes() != bytes([0xEE]) * count, "the launches wrote"
+
+
+@pytest.mark.parametrize("hidden,inner,rows,live", [(512, 384, 100, 100), (640, 128, 70, 67)])
+def test_narrow_and_whole_strips_give_the_same_bytes(amd, card, hidden, inner, rows, live):
+    """The 4-bit wide launches of strips of half the tiles (native_expert_gate_up_narrow_1, native_expert_down_narrow_1) and
+    of whole strips, over the same rows: every output byte. Widths that end inside a block of either."""
+    say("narrow and whole strips", hidden, inner, rows, live)
+    experts_n, picks = 64, 2
+    router = to_bf16(normals(81, experts_n * hidden) * 0.02).reshape(experts_n, hidden)
+    layer = amd.Fp4Layer(card, hidden, inner, experts_n, picks, rows, matrices_of(hidden, inner, experts_n, 83, E2M1),
+                         router_weights_bf16=router, weight_format=E2M1_GFX950)
+    x = to_bf16(normals(85, rows * hidden)).reshape(rows, hidden)
+    _, wide = run_wide(card, layer, x, live)
+    native = amd.LinearNativeKernels()
+    amd.check(card.lib.linear_native_kernels_prepare(amd.backend_table(), card.handle, amd.ARITHMETIC_CLASS_GFX950, C.byref(native)), "prepare")
+    launches, outputs = layer.wide_expert_launches(wide), []
+    for gate_up, down, tiles in ((native.native_expert_gate_up_narrow, native.native_expert_down_narrow, 1),
+                                 (native.native_expert_gate_up, native.native_expert_down, 2)):
+        launches[0].kernel, launches[1].kernel = gate_up, down
+        launches[0].grid[0], launches[1].grid[0] = -(-inner // (128 * tiles)), -(-hidden // (256 * tiles))
+        for name in NAMES:
+            card.upload(layer.ranges[name].byte_offset, np.full(layer.ranges[name].byte_count, 0xEE, dtype=np.uint8))
+        card.run(launches)
+        outputs.append([layer.read(name).copy() for name in NAMES])
+    for name, a, b in zip(NAMES, *outputs):
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), name
+        assert not np.all(a.view(np.uint8) == 0xEE)

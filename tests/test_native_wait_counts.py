@@ -15,6 +15,8 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 # 2 loads a column block a wavefront brings (one or two) and one of scale words; WEIGHT_LOADS the tiles' halves and the
 # scale loads of a wavefront's strip
 INSTANCES = {
+    "E2M1 gate/up of whole strips (8 tiles, 2 scale words; 64 columns)": (2, 2, False, 3, 10),
+    "E2M1 down of whole strips (8 tiles, 2 scale words)": (2, 2, False, 3, 10),
     "E2M1 gate/up (4 tiles, 2 scale words; 64 columns)": (3, 2, False, 3, 6),
     "E2M1 down (4 tiles, 1 scale word)": (3, 2, False, 3, 5),
     "E4M3 gate/up and down (2 tiles of two halves, 2 scale bytes; 128 columns)": (3, 3, True, 5, 6),
