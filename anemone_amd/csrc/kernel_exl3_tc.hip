@@ -113,7 +113,7 @@ __device__ static __forceinline__ void tc_item(const uint32_t *codes, uint32_t i
 }
 
 /* launches 1 and 3: grid (strips, job_capacity, matrices * slices / 4), block 256; a strip is EXL3_TC_STRIP_OUTPUTS outputs,
- * or EXL3_TC_NARROW_STRIP_OUTPUTS where the grid's x says so (the same sums: a launch of few jobs, whose wide
+ * or EXL3_TC_NARROW_STRIP_OUTPUTS of the narrow kernel (the same sums: a launch of few jobs, whose wide
  * strips leave a SIMD one wavefront or none and which waits for each wavefront's own chain). The block's four
  * wavefronts take four consecutive (matrix, slice) items of one strip (a strip of fewer than four items: the items of
  * adjacent strips, the grid's x that many times smaller and its z 1). pass 0: gate and up; pass 1: down. A slice is
@@ -176,15 +176,17 @@ __device__ static __forceinline__ void tc_products_block(const struct exl3_tc_re
 extern "C" __global__ void __launch_bounds__(PRODUCT_THREADS, 4)
     exl3_tc_products(struct exl3_tc_record record, unsigned char *arena)
 {
-    const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const uint32_t outputs = record.pass != 0u ? tc_shape_of(record).hidden : record.intermediate;
-    if (gridDim.x * EXL3_TC_STRIP_OUTPUTS > outputs) { /* the same in every block */
-        tc_products_block<NARROW_STRIP_PAIRS>(record, arena, blockIdx.x, blockIdx.y, blockIdx.z, lane, wave);
-    } else {
-        tc_products_block<STRIP_PAIRS>(record, arena, blockIdx.x, blockIdx.y, blockIdx.z, lane, wave);
-    }
+    tc_products_block<STRIP_PAIRS>(record, arena, blockIdx.x, blockIdx.y, blockIdx.z, threadIdx.x % WAVE, __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE));
 }
 ANEMONE_KERNEL(EXL3_TC_KERNEL_FILE, exl3_tc_products, exl3_tc_record);
+
+/* a kernel of its own: as a branch of the one above it made a step of one row 1.5 % longer */
+extern "C" __global__ void __launch_bounds__(PRODUCT_THREADS, 4)
+    exl3_tc_products_narrow(struct exl3_tc_record record, unsigned char *arena)
+{
+    tc_products_block<NARROW_STRIP_PAIRS>(record, arena, blockIdx.x, blockIdx.y, blockIdx.z, threadIdx.x % WAVE, __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE));
+}
+ANEMONE_KERNEL(EXL3_TC_KERNEL_FILE, exl3_tc_products_narrow, exl3_tc_record);
 
 /* launch 2: grid (intermediate / 128, job_capacity), block 64 */
 extern "C" __global__ void exl3_tc_activate(struct exl3_tc_record record, unsigned char *arena)
@@ -387,8 +389,9 @@ extern "C" result_status exl3_tc_static_scratch_resolve(void)
     return static_scratch_of(&address);
 }
 
-/* kernel_prepare of a table that launches nothing: the four kernels of this file by number */
-static const char *const static_kernel_names[] = {"exl3_tc_operands", "exl3_tc_products", "exl3_tc_activate", "exl3_tc_combine"};
+/* kernel_prepare of a table that launches nothing: the kernels of this file by number */
+static const char *const static_kernel_names[] = {"exl3_tc_operands", "exl3_tc_products", "exl3_tc_activate", "exl3_tc_combine", "exl3_tc_products_narrow"};
+#define STATIC_KERNELS (sizeof static_kernel_names / sizeof static_kernel_names[0])
 
 static result_status static_kernel_prepare(struct device_card *, const char *file, const char *function, uint32_t record_bytes,
                                            uint32_t *kernel_out)
@@ -396,7 +399,7 @@ static result_status static_kernel_prepare(struct device_card *, const char *fil
     if (strcmp(file, EXL3_TC_KERNEL_FILE) != 0 || record_bytes != sizeof(struct exl3_tc_record)) {
         return STATUS_INVALID_ARGUMENT;
     }
-    for (uint32_t index = 0; index < 4u; index++) {
+    for (uint32_t index = 0; index < STATIC_KERNELS; index++) {
         if (strcmp(function, static_kernel_names[index]) == 0) {
             *kernel_out = index;
             return STATUS_OK;
@@ -442,7 +445,7 @@ extern "C" result_status exl3_tc_run_static(const struct exl3_tc_record *record,
      * arena whichever lies higher */
     const uint64_t offset = (uint64_t)(uintptr_t)workspace - (uint64_t)(uintptr_t)arena_device;
     typedef void (*entry)(struct exl3_tc_record, unsigned char *);
-    const entry entries[4] = {exl3_tc_operands, exl3_tc_products, exl3_tc_activate, exl3_tc_combine};
+    const entry entries[STATIC_KERNELS] = {exl3_tc_operands, exl3_tc_products, exl3_tc_activate, exl3_tc_combine, exl3_tc_products_narrow};
     for (uint32_t index = 0; index < EXL3_TC_LAUNCHES; index++) {
         struct exl3_tc_record argument;
         memcpy(&argument, launches[index].argument, sizeof argument);

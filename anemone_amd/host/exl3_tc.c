@@ -130,8 +130,6 @@ static result_status tc_prepare(const struct exl3_tc_record *record, uint64_t ar
         }
         return STATUS_INVALID_ARGUMENT;
     }
-    static const char *const names[EXL3_TC_LAUNCHES] = {"exl3_tc_operands", "exl3_tc_products", "exl3_tc_activate",
-                                                        "exl3_tc_products", "exl3_tc_combine"};
     const uint32_t gate_up_strips = GATE_UP_STRIPS, down_strips = DOWN_STRIPS;
     if (I % (EXL3_TC_STRIP_OUTPUTS * gate_up_strips) != 0 || hidden % (EXL3_TC_STRIP_OUTPUTS * down_strips) != 0) {
         REFUSE("%s: sizes that are no whole number of the products' blocks (%u and %u outputs)", what,
@@ -140,6 +138,10 @@ static result_status tc_prepare(const struct exl3_tc_record *record, uint64_t ar
     }
     const uint32_t gate_up_blocks = products_blocks(I / (EXL3_TC_STRIP_OUTPUTS * gate_up_strips), record->job_capacity, GATE_UP_ITEMS);
     const uint32_t down_blocks = products_blocks(hidden / (EXL3_TC_STRIP_OUTPUTS * down_strips), record->job_capacity, DOWN_ITEMS);
+    const char *const names[EXL3_TC_LAUNCHES] = {
+        "exl3_tc_operands", gate_up_blocks > I / (EXL3_TC_STRIP_OUTPUTS * gate_up_strips) ? "exl3_tc_products_narrow" : "exl3_tc_products",
+        "exl3_tc_activate", down_blocks > hidden / (EXL3_TC_STRIP_OUTPUTS * down_strips) ? "exl3_tc_products_narrow" : "exl3_tc_products",
+        "exl3_tc_combine"};
     const uint32_t grid_x[EXL3_TC_LAUNCHES] = {hidden / 128u, gate_up_blocks, I / 128u, down_blocks, hidden / 128u};
     const uint32_t grid_y[EXL3_TC_LAUNCHES] = {record->job_capacity, record->job_capacity, record->job_capacity,
                                                record->job_capacity, record->row_count};

@@ -185,6 +185,7 @@ def test_tc_prepare_takes_narrow_strips_below_512_blocks(fake, jobs, grids):
     launches = amd.launches_of(5)
     assert amd.library().exl3_tc_prepare(C.byref(tc_record(job_capacity=jobs)), ARENA, fake.address, fake.card, launches) == 0
     assert [list(launches[index].grid) for index in (1, 3)] == [[grids[0], jobs, 2], [grids[1], jobs, 1]]
+    assert [fake.handles[launches[index].kernel][1] for index in (1, 3)] == ["exl3_tc_products" + ("_narrow" if jobs < 8 else "")] * 2
 
 
 def test_tc_prepare_geometry_and_refusals(fake):

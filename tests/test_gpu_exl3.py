@@ -386,8 +386,8 @@ def test_thin_product_of_short_and_long_slices(amd, card, inputs, width):
 
 @pytest.mark.parametrize("hidden,inner,width_choices", [(512, 384, [2, 3, 4]), (256, 128, [40])])
 def test_narrow_strips_of_the_fused_decode_give_the_same_bits(amd, card, hidden, inner, width_choices):
-    """A products launch of few blocks takes strips of 32 outputs in place of 64 (anemone_amd/host/exl3_tc.c); the kernel
-    reads which off its grid: the same launches with the grids of the wide strips give every output's bits."""
+    """A products launch of few blocks takes strips of 32 outputs in place of 64 (exl3_tc_products_narrow): the same
+    launches with the kernel and the grids of the wide strips give every output's bits."""
     say("narrow strips", hidden, inner, width_choices)
     rows, picks = 3, 4
     layer, _, _, _ = build_layer(amd, card, hidden, inner, 64, picks, rows, 13, width_choices)
@@ -401,4 +401,5 @@ def test_narrow_strips_of_the_fused_decode_give_the_same_bits(amd, card, hidden,
         card.run(launches)
         outputs.append(layer.output().view(np.uint32).copy())
         launches[1].grid[0], launches[3].grid[0] = inner // 64, hidden // 64
+        launches[1].kernel = launches[3].kernel = card.kernel("kernel_exl3_tc", "exl3_tc_products", C.sizeof(amd.Exl3TcRecord))
     assert np.array_equal(outputs[0], outputs[1]) and not np.all(outputs[0] == 0xEEEEEEEE)
