@@ -258,22 +258,22 @@ exl3_stream_product(const uint32_t *__restrict__ codes, uint32_t out_tiles, uint
 
 /*
  * One wavefront multiplies ONE output tile by the K tiles [first_tile, last_tile) (as above): the form of a launch too
- * small to fill the card, where a wavefront has a SIMD to itself and what counts is the length of its own chain.
+ * small to fill the card, where a SIMD has one to a few wavefronts and what counts is the length of a wavefront's chain.
  *
  * Lane 16 g + i decodes one half of chunk i % 8 of K tile g: the sixteen symbols of output i % 8 + 8 (i / 8), which is row
  * i of the matrix instruction. The upper half's symbols lie four further in the ring: those lanes bring them to the lower
  * half's places (one shift of the chunk a step), so that every lane's fields are constants. Each output's sums run over the
  * same operands in the same order as exl3_stream_product's: the same bits.
- * The loads run STEPS_AHEAD steps ahead: a step is two loads of codes and two of operands, and a chain of sixteen steps
- * (4,096 inputs in four slices) waits for memory once.
+ * The loads run STEPS_AHEAD steps ahead (a step is two loads of codes and two of operands): the more, the fewer of a lone
+ * chain's waits for memory; each costs 13 to 17 registers, and a launch of several wavefronts a SIMD needs the wavefronts.
  *   accumulator  lane 16 g' + j: outputs 4 g' + {0..3} of the tile, column j
  */
-template <uint32_t bits_x2>
+template <uint32_t bits_x2, uint32_t STEPS_AHEAD>
 __device__ static __forceinline__ void exl3_stream_tile_product(const uint32_t *__restrict__ codes, uint32_t out_tiles, uint32_t out_tile, uint32_t first_tile,
                                                                 uint32_t last_tile, const half_t *__restrict__ operand, uint32_t lane, float4_t &accumulator)
 {
     typedef exl3_chunk<bits_x2> C;
-    constexpr uint32_t STEPS_AHEAD = 8u, FOUR_SYMBOLS = 2u * bits_x2; /* bits */
+    constexpr uint32_t FOUR_SYMBOLS = 2u * bits_x2; /* bits */
     const uint32_t g = lane / 16u, i = lane % 16u, c = i % 8u;
     const bool odd = (c & 1u) != 0u, upper = i >= 8u;
     uint32_t own, front;

@@ -79,10 +79,17 @@ ANEMONE_KERNEL(EXL3_KERNEL_FILE, exl3_input, exl3_expert_record);
 /* Products of one job: block = four wavefronts = the four K slices (whole steps of four K tiles) of one strip of
  * STRIP_TILES output tiles: eight (the stream product), or one in the thin instances, which a launch of few jobs takes so
  * that its blocks cover the card (the same slices and the same order of sums, so the same bits).
- * A thin launch has a wavefront a SIMD, so its time is the chain of one wavefront: its codes' loads run eight steps ahead
- * and pass through no LDS. One 4096 x 4096 matrix of K 4 by one vector: 7.8 us (13.4 with two K tiles a step, a step ahead
- * through an LDS window); the input, product and finish launches 10.8 us (16.5). */
-template <uint32_t bits_x2, bool down, uint32_t STRIP_TILES>
+ * A thin launch of at most a block a CU has a wavefront a SIMD, so its time is the chain of one wavefront: its codes' loads
+ * run eight steps ahead and pass through no LDS. One 4096 x 4096 matrix of K 4 by one vector: 7.8 us (13.4 with two K tiles a
+ * step, a step ahead through an LDS window); the input, product and finish launches 10.8 us (16.5).
+ * The thin instances of more blocks (_thin_many) run five steps ahead: 108 to 122 registers, four wavefronts a SIMD, where
+ * eight ahead take 157 to 177 and leave two or three. K 4, us, eight | five | the LDS form: 512 blocks of 4096 inputs 11.8 |
+ * 11.2 | 23.9; 1,024 of 4096 20.3 | 18.7 | 27.9, of 512 5.6 | 4.2 | 5.2; 1,280 of 512 7.1 | 5.3 | 5.9. Four steps ahead are
+ * within 3 % of five either way, six (three wavefronts) slower from 1,024 blocks up.
+ * The eight-tile instances are held to three wavefronts a SIMD: left to itself the compiler keeps the sums in accumulation
+ * registers and copies beside them (175 registers, two wavefronts, for K 4): down of 32 jobs at 1536 x 5120 40.5 -> 39.0 us,
+ * of 64 at 2048 x 4096 79.7 -> 74.6. */
+template <uint32_t bits_x2, bool down, uint32_t STRIP_TILES, uint32_t STEPS_AHEAD>
 __device__ static __forceinline__ void chain_product(const struct exl3_expert_record &record, unsigned char *arena,
                                                      const struct expert_job_record *job, float *partial)
 {
@@ -100,7 +107,7 @@ __device__ static __forceinline__ void chain_product(const struct exl3_expert_re
     const uint32_t *codes = (const uint32_t *)(arena + matrix);
     float4_t sums[STRIP_TILES];
     if constexpr (STRIP_TILES == 1u) {
-        exl3_stream_tile_product<bits_x2>(codes, outputs / EXL3_TILE, strip_tile, first_tile, last_tile, operand, lane, sums[0]);
+        exl3_stream_tile_product<bits_x2, STEPS_AHEAD>(codes, outputs / EXL3_TILE, strip_tile, first_tile, last_tile, operand, lane, sums[0]);
     } else {
         float4_t accumulator[STRIP_TILES / 2u][2];
         exl3_stream_product<bits_x2, STRIP_TILES / 2u, true>(codes, outputs / EXL3_TILE, strip_tile, first_tile, last_tile, operand, lane, accumulator);
@@ -137,7 +144,7 @@ __device__ static __forceinline__ void chain_product(const struct exl3_expert_re
     }
 }
 
-template <uint32_t fixed_bits_x2, bool down, uint32_t STRIP_TILES>
+template <uint32_t fixed_bits_x2, bool down, uint32_t STRIP_TILES, uint32_t STEPS_AHEAD = 0u>
 __device__ static __forceinline__ void chain_product_entry(const struct exl3_expert_record &record,
                                                            unsigned char *arena)
 {
@@ -151,39 +158,28 @@ __device__ static __forceinline__ void chain_product_entry(const struct exl3_exp
         bits_x2 = exl3_bits_x2(chain_width(record, arena, job->expert, down ? 2u : blockIdx.z));
     }
     switch (bits_x2) {
-    case 4u: chain_product<4u, down, STRIP_TILES>(record, arena, job, partial); break;
-    case 5u: chain_product<5u, down, STRIP_TILES>(record, arena, job, partial); break;
-    case 6u: chain_product<6u, down, STRIP_TILES>(record, arena, job, partial); break;
-    case 8u: chain_product<8u, down, STRIP_TILES>(record, arena, job, partial); break;
+    case 4u: chain_product<4u, down, STRIP_TILES, STEPS_AHEAD>(record, arena, job, partial); break;
+    case 5u: chain_product<5u, down, STRIP_TILES, STEPS_AHEAD>(record, arena, job, partial); break;
+    case 6u: chain_product<6u, down, STRIP_TILES, STEPS_AHEAD>(record, arena, job, partial); break;
+    case 8u: chain_product<8u, down, STRIP_TILES, STEPS_AHEAD>(record, arena, job, partial); break;
     default: break;
     }
 }
 
+#define EXL3_PRODUCT_ENTRY(entry, bits_x2, down, wavefronts, ...)                                            \
+    extern "C" __global__ void __launch_bounds__(PRODUCT_THREADS, wavefronts)                                \
+        entry(struct exl3_expert_record record, unsigned char *arena)                                        \
+    {                                                                                                        \
+        chain_product_entry<bits_x2, down, __VA_ARGS__>(record, arena);                                      \
+    }                                                                                                        \
+    ANEMONE_KERNEL(EXL3_KERNEL_FILE, entry, exl3_expert_record)
 #define EXL3_PRODUCT_ENTRIES(name, bits_x2)                                                                  \
-    extern "C" __global__ void __launch_bounds__(PRODUCT_THREADS)                                            \
-        exl3_gate_up_##name(struct exl3_expert_record record, unsigned char *arena)                         \
-    {                                                                                                        \
-        chain_product_entry<bits_x2, false, EXL3_STRIP_TILES>(record, arena);                                \
-    }                                                                                                        \
-    ANEMONE_KERNEL(EXL3_KERNEL_FILE, exl3_gate_up_##name, exl3_expert_record);                               \
-    extern "C" __global__ void __launch_bounds__(PRODUCT_THREADS)                                            \
-        exl3_down_##name(struct exl3_expert_record record, unsigned char *arena)                            \
-    {                                                                                                        \
-        chain_product_entry<bits_x2, true, EXL3_STRIP_TILES>(record, arena);                                 \
-    }                                                                                                        \
-    ANEMONE_KERNEL(EXL3_KERNEL_FILE, exl3_down_##name, exl3_expert_record);                                  \
-    extern "C" __global__ void __launch_bounds__(PRODUCT_THREADS)                                            \
-        exl3_gate_up_##name##_thin(struct exl3_expert_record record, unsigned char *arena)                  \
-    {                                                                                                        \
-        chain_product_entry<bits_x2, false, EXL3_THIN_STRIP_TILES>(record, arena);                           \
-    }                                                                                                        \
-    ANEMONE_KERNEL(EXL3_KERNEL_FILE, exl3_gate_up_##name##_thin, exl3_expert_record);                        \
-    extern "C" __global__ void __launch_bounds__(PRODUCT_THREADS)                                            \
-        exl3_down_##name##_thin(struct exl3_expert_record record, unsigned char *arena)                     \
-    {                                                                                                        \
-        chain_product_entry<bits_x2, true, EXL3_THIN_STRIP_TILES>(record, arena);                            \
-    }                                                                                                        \
-    ANEMONE_KERNEL(EXL3_KERNEL_FILE, exl3_down_##name##_thin, exl3_expert_record)
+    EXL3_PRODUCT_ENTRY(exl3_gate_up_##name, bits_x2, false, 3, EXL3_STRIP_TILES);                            \
+    EXL3_PRODUCT_ENTRY(exl3_down_##name, bits_x2, true, 3, EXL3_STRIP_TILES);                                \
+    EXL3_PRODUCT_ENTRY(exl3_gate_up_##name##_thin, bits_x2, false, 1, EXL3_THIN_STRIP_TILES, 8u);            \
+    EXL3_PRODUCT_ENTRY(exl3_down_##name##_thin, bits_x2, true, 1, EXL3_THIN_STRIP_TILES, 8u);                \
+    EXL3_PRODUCT_ENTRY(exl3_gate_up_##name##_thin_many, bits_x2, false, 4, EXL3_THIN_STRIP_TILES, 5u);       \
+    EXL3_PRODUCT_ENTRY(exl3_down_##name##_thin_many, bits_x2, true, 4, EXL3_THIN_STRIP_TILES, 5u)
 EXL3_PRODUCT_ENTRIES(k2, 4u);
 EXL3_PRODUCT_ENTRIES(k2_5, 5u);
 EXL3_PRODUCT_ENTRIES(k3, 6u);

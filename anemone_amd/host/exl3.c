@@ -8,7 +8,8 @@
  *   gate/up         exl3_gate_up_<k>|_mixed     (inner_size / 128, jobs, 2)           256  4 K slices x 8 output tiles
  *   activate        exl3_activate               (inner_size / 128, jobs, 1)           64
  *   down            exl3_down_<k>|_mixed        (input_size / 128, jobs, 1)           256
- *   (a product launch of fewer than EXL3_THIN_BELOW_BLOCKS such blocks: the _thin instance, x = size / 16)
+ *   (a product launch of at most EXL3_THIN_BLOCKS, EXL3_THIN_MANY_BLOCKS blocks of one output tile: the _thin, _thin_many
+ *   instance, x = size / 16)
  *   finish          exl3_finish                 (input_size / 128, jobs, 1)           64
  *   row sum         exl3_row_sum                (ceil(width / 256), rows, 1)          256
  *
@@ -69,6 +70,19 @@ result_status exl3_reconstruct_prepare(const struct exl3_reconstruct_record *rec
     return STATUS_OK;
 }
 
+/* the form of a product launch over `projections` matrices of `outputs` outputs for each of `jobs` jobs (the lines:
+ * anemone_records.h). Every form gives the same sums. */
+static struct product_form {
+    const char *suffix;
+    uint32_t block_outputs;
+} product_form_of(uint32_t outputs, uint32_t jobs, uint32_t projections)
+{
+    const uint64_t thin_blocks = (uint64_t)(outputs / (EXL3_THIN_STRIP_TILES * EXL3_TILE)) * jobs * projections;
+    return thin_blocks <= EXL3_THIN_BLOCKS        ? (struct product_form){"_thin", EXL3_THIN_STRIP_TILES * EXL3_TILE}
+           : thin_blocks <= EXL3_THIN_MANY_BLOCKS ? (struct product_form){"_thin_many", EXL3_THIN_STRIP_TILES * EXL3_TILE}
+                                                  : (struct product_form){"", STRIP_OUTPUTS};
+}
+
 static result_status chain_prepare(const struct exl3_expert_record *record, uint64_t arena_byte_count,
                                    const struct backend_operations *backend, struct device_card *card,
                                    uint32_t arithmetic_class, struct kernel_launch *launches_out)
@@ -125,20 +139,18 @@ static result_status chain_prepare(const struct exl3_expert_record *record, uint
     }
     char gate_up_name[40], down_name[40];
     const char *width = mixed ? "mixed" : exl3_width_name(exl3_bits_x2(record->bits_per_weight));
-    /* a product launch of few blocks (a job or two) takes the instances of one output tile a block: eight times the
-     * blocks, the same sums */
-    const bool thin_gate_up = (uint64_t)record->inner_size / STRIP_OUTPUTS * record->job_count * 2u < EXL3_THIN_BELOW_BLOCKS;
-    const bool thin_down = (uint64_t)record->input_size / STRIP_OUTPUTS * record->job_count < EXL3_THIN_BELOW_BLOCKS;
-    (void)snprintf(gate_up_name, sizeof gate_up_name, "exl3_gate_up_%s%s", width, thin_gate_up ? "_thin" : "");
-    (void)snprintf(down_name, sizeof down_name, "exl3_down_%s%s", width, thin_down ? "_thin" : "");
+    const struct product_form gate_up = product_form_of(record->inner_size, record->job_count, 2u);
+    const struct product_form down = product_form_of(record->input_size, record->job_count, 1u);
+    (void)snprintf(gate_up_name, sizeof gate_up_name, "exl3_gate_up_%s%s", width, gate_up.suffix);
+    (void)snprintf(down_name, sizeof down_name, "exl3_down_%s%s", width, down.suffix);
     const struct {
         const char *name;
         uint32_t width, threads, projections, block_outputs;
     } stages[EXL3_EXPERT_LAUNCHES] = {
         {"exl3_input", record->input_size, WAVE_THREADS, 2u, EXL3_TRANSFORM},
-        {gate_up_name, record->inner_size, PRODUCT_THREADS, 2u, (thin_gate_up ? EXL3_THIN_STRIP_TILES : EXL3_STRIP_TILES) * EXL3_TILE},
+        {gate_up_name, record->inner_size, PRODUCT_THREADS, 2u, gate_up.block_outputs},
         {"exl3_activate", record->inner_size, WAVE_THREADS, 1u, EXL3_TRANSFORM},
-        {down_name, record->input_size, PRODUCT_THREADS, 1u, (thin_down ? EXL3_THIN_STRIP_TILES : EXL3_STRIP_TILES) * EXL3_TILE},
+        {down_name, record->input_size, PRODUCT_THREADS, 1u, down.block_outputs},
         {"exl3_finish", record->input_size, WAVE_THREADS, 1u, EXL3_TRANSFORM},
     };
     struct kernel_launch launches[EXL3_EXPERT_LAUNCHES];

@@ -203,8 +203,13 @@ ANEMONE_RECORD_HAS(router_wide_arguments, 136);
 #define EXL3_EXPERT_LAUNCHES 5u
 #define EXL3_PRODUCT_SLICES 4u
 #define EXL3_STRIP_TILES 8u      /* output tiles of a block of the chain's product launches: 128 outputs */
-#define EXL3_THIN_STRIP_TILES 1u /* of the _thin instances, which a launch of fewer than EXL3_THIN_BELOW_BLOCKS blocks takes */
-#define EXL3_THIN_BELOW_BLOCKS 256u
+#define EXL3_THIN_STRIP_TILES 1u /* of the _thin and _thin_many instances */
+/* A product launch takes one tile a block while that makes at most this many blocks. By 256 of them, a block a CU, a wavefront
+ * has a SIMD to itself (_thin). Beyond, four blocks a CU run side by side (_thin_many), and the launch takes as long as its
+ * rounds of 1,024 where the eight-tile form takes one chain up to 256 blocks of eight: K 4, us, one tile | eight: 1,024 blocks
+ * of 4096 inputs 18.7 | 24.0, 1,408 of 2048 inputs 13.9 | 14.1, 1,536 of 4096 inputs 25.0 | 24.1, 1,984 of 1024 inputs 10.9 | 9.4. */
+#define EXL3_THIN_BLOCKS 256u
+#define EXL3_THIN_MANY_BLOCKS 1408u
 
 #ifdef __cplusplus
 #define ANEMONE_INLINE __host__ __device__ static constexpr inline

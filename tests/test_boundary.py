@@ -130,9 +130,11 @@ def test_chain_prepare_geometry(fake):
     mixed = amd.launches_of(5)
     assert lib.exl3_experts_prepare(C.byref(chain_record(widths_offset=1 << 30)), ARENA, fake.address, fake.card, 950, mixed) == 0
     assert fake.handles[mixed[1].kernel][1] == "exl3_gate_up_mixed" and fake.handles[mixed[3].kernel][1] == "exl3_down_mixed"
-    # product launches of fewer than 256 blocks take the instances of one output tile a block (eight times the blocks)
+    # product launches of at most 256 (1408) blocks of one output tile a block take the instances of that form
     for jobs, pairs, names, grids in ((1, 8, ["exl3_gate_up_k3_thin", "exl3_down_k3_thin"], [[128, 1, 2], [256, 1, 1]]),
-                                      (7, 8, ["exl3_gate_up_k3_thin", "exl3_down_k3_thin"], [[128, 7, 2], [256, 7, 1]]),
+                                      (2, 8, ["exl3_gate_up_k3_thin_many", "exl3_down_k3_thin_many"], [[128, 2, 2], [256, 2, 1]]),
+                                      (5, 8, ["exl3_gate_up_k3_thin_many", "exl3_down_k3_thin_many"], [[128, 5, 2], [256, 5, 1]]),
+                                      (6, 8, ["exl3_gate_up_k3", "exl3_down_k3"], [[16, 6, 2], [32, 6, 1]]),
                                       (8, 8, ["exl3_gate_up_k3", "exl3_down_k3"], [[16, 8, 2], [32, 8, 1]])):
         few = amd.launches_of(5)
         assert lib.exl3_experts_prepare(C.byref(chain_record(job_count=jobs, pair_count=pairs)), ARENA, fake.address, fake.card, 950, few) == 0

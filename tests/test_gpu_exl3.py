@@ -384,6 +384,45 @@ def test_thin_product_of_short_and_long_slices(amd, card, inputs, width):
     assert np.all(np.abs(got - want) <= inputs * 2.0 ** -24 * magnitudes)
 
 
+@pytest.mark.parametrize("width", [2, 40, 3, 4, (3, 2, 4)])
+@pytest.mark.parametrize("inputs", [128, 1280, 2816])
+def test_thin_products_of_many_blocks_give_the_same_bits(amd, card, inputs, width):
+    """A product launch of 257 to 1408 blocks of one tile (exl3_down_<k>_thin_many, loads five steps ahead) with K slices of no
+    or one step, of five, and of eleven: the float32 products of the eight-tile kernel and of the eight-steps-ahead one."""
+    say("thin products of many blocks", inputs, width)
+    hidden = max(512, inputs)
+    job_count, rows = 256 // (hidden // 16) + 1, 3
+    mixed, down_width = isinstance(width, tuple), width[2] if isinstance(width, tuple) else width
+    matrix = exl3_matrix(0x7600 + down_width, inputs, hidden, down_width)
+    jobs, pairs = np.zeros(job_count, dtype=JOB_DTYPE), job_count * rows
+    jobs["gate_offset"] = jobs["up_offset"] = jobs["down_offset"] = card.place(matrix, 256)
+    jobs["row_count"] = rows
+    jobs["pair_index"][:, :rows] = np.arange(pairs).reshape(job_count, rows)
+    record = amd.Exl3ExpertRecord()
+    record.jobs_offset = card.place(jobs.view(np.uint8))
+    record.input_offset, record.hidden_offset = card.reserve(pairs * hidden * 2), card.reserve(pairs * inputs * 2)
+    record.operands_offset = card.reserve(pairs * hidden * 4)
+    record.products_offset = record.output_offset = card.reserve(pairs * hidden * 8)
+    record.input_size, record.inner_size = hidden, inputs
+    record.pair_count, record.pairs_per_row, record.job_count = pairs, 1, job_count
+    record.bits_per_weight, record.activation_limit = down_width, 10.0
+    if mixed:
+        record.widths_offset = card.place(np.full(1, width[0] | width[1] << 8 | width[2] << 16, dtype=np.uint32))
+    launches = amd.launches_of(5)
+    amd.check(card.lib.exl3_experts_prepare(C.byref(record), card.arena_bytes, amd.backend_table(), card.handle, 950, launches), "prepare")
+    assert list(launches[3].grid) == [hidden // 16, job_count, 1]
+    card.upload(record.operands_offset, normals(0x7700 + inputs, pairs * inputs).astype(np.float16))
+    name = "exl3_down_" + ("mixed" if mixed else {2: "k2", 40: "k2_5", 3: "k3", 4: "k4"}[width])
+    outputs = []
+    for suffix, tiles in (("_thin_many", 1), ("_thin", 1), ("", 8)):
+        launches[3].kernel, launches[3].grid[0] = card.kernel("kernel_exl3", name + suffix, C.sizeof(record)), hidden // 16 // tiles
+        card.upload(record.products_offset, np.full(pairs * hidden * 4, 0xEE, dtype=np.uint8))
+        card.run(launches[3:4])
+        outputs.append(card.download(record.products_offset, pairs * hidden * 4, np.uint32).copy())
+    assert np.array_equal(outputs[0], outputs[1]) and np.array_equal(outputs[0], outputs[2])
+    assert not np.any(outputs[0] == 0xEEEEEEEE) and np.any(outputs[0] != 0)
+
+
 @pytest.mark.parametrize("hidden,inner,width_choices", [(512, 384, [2, 3, 4]), (256, 128, [40])])
 def test_narrow_strips_of_the_fused_decode_give_the_same_bits(amd, card, hidden, inner, width_choices):
     """A products launch of few blocks takes strips of 32 outputs in place of 64 (exl3_tc_products_narrow): the same
