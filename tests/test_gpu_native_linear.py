@@ -78,6 +78,12 @@ def run_wide(card, layer, x, live):
     (640, 384, 64, 2, 450, 449, B128),
     (512, 256, 64, 8, 1500, 1401, B128),
     (512, 256, 64, 1, 4300, 4300, -B128),
+    # 4-bit weights, whose blocks go in the order of runs: one expert takes every row (a run of 68 tiles: cut in pieces of 16
+    # and where a window of 64 tiles ends), the same with the other experts' tiles around it, and few rows of many experts
+    # (more unused tiles behind the used ones than the first look takes)
+    (512, 256, 64, 1, 4300, 4300, -E2M1),
+    (640, 384, 64, 3, 4300, 4287, -E2M1),
+    (256, 128, 384, 1, 100, 100, -E2M1),
     # chains of one, two and three K steps: fewer steps than sets of weight registers and stages of columns
     (128, 128, 64, 4, 300, 300, E2M1),
     (256, 128, 64, 4, 300, 297, E2M1),
@@ -148,6 +154,116 @@ def test_native_layer_against_oracle(amd, card, fmt):
     error = np.sqrt(np.mean((row_output - want) ** 2) / np.mean(want.astype(np.float64) ** 2))
     say("  layer rms error vs oracle: %.2e" % error)
     assert error < 2e-2
+
+
+def special_rows(rows, hidden):
+    """Rows of ordinary values; of values whose sums overflow (a gate of minus infinity makes a hidden value that is not a
+    number); with infinities (a scale code of 255: every sum is not a number); of 1e30; with a value that is not a number."""
+    x = normals(91, rows * hidden).reshape(rows, hidden).astype(np.float64)
+    x[1::5] *= 1e38
+    x[3::5] *= 1e30
+    x = to_bf16(np.clip(x, -3e38, 3e38).astype(np.float32)).reshape(rows, hidden)
+    x[2::5, 7] = 0x7F80
+    x[4::5, 9] = 0x7FC1
+    return x
+
+
+@pytest.mark.parametrize("fmt", [E2M1, E4M3, B128])
+@pytest.mark.parametrize("limit", [10.0, 1e12, 1e30])
+def test_finishes_of_values_without_order_and_of_large_scales(amd, card, fmt, limit):
+    """The finishes' side paths: hidden values and down sums that are not numbers, scale codes of the hidden values above 146
+    (an activation limit of 1e12 and 1e30 lets them through), in column blocks beside ordinary ones: the wide launches byte
+    for byte the job-table kernels', the native launches byte for byte theirs."""
+    say("finishes of special values", fmt, limit)
+    hidden, inner, experts_n, picks, rows = 256, 128, 64, 4, 120
+    from anemone_amd import workloads
+    # gates and ups of deviation 16 times the rows' values and more: sums of the second kind of row overflow
+    matrix, loud = {E2M1: (workloads.fp4_matrix, dict(scale_code=126)), E4M3: (workloads.fp8_matrix, dict(deviation=1.5)),
+                    B128: (workloads.fp8_block128_matrix, dict(deviation=1.5))}[fmt]
+    trios = [[matrix(9300 + 3 * e, inner, hidden, **loud), matrix(9301 + 3 * e, inner, hidden, **loud), matrix(9302 + 3 * e, hidden, inner)] for e in range(8)]
+    matrices = [trios[e % 8] for e in range(experts_n)]
+    router = to_bf16(normals(95, experts_n * hidden) * 0.02).reshape(experts_n, hidden)
+    x = special_rows(rows, hidden)
+    made = [amd.Fp4Layer(card, hidden, inner, experts_n, picks, rows, matrices, router_weights_bf16=router, limit=limit,
+                         weight_format=weight_format, gate_up_slices=1, down_slices=1) for weight_format in (fmt, NATIVE_OF[fmt])]
+    scores = normals(97, rows * experts_n).astype(np.float32)  # the rows' own scores would not be numbers
+    outputs = []
+    for layer, wide_form in ((made[0], False), (made[0], True), (made[1], True)):
+        layer.set_rows(x, rows)
+        card.upload(layer.scores_offset, scores)
+        wide = layer.wide_router()
+        card.run(wide.launches())
+        card.run(layer.quantize_launch())
+        for name in ("hidden",) + NAMES:
+            card.upload(layer.ranges[name].byte_offset, np.full(layer.ranges[name].byte_count, 0xEE, dtype=np.uint8))
+        card.run(layer.wide_expert_launches(wide) if wide_form else layer.expert_launches(wide))
+        outputs.append([layer.read(name).copy() for name in NAMES])
+        if not wide_form:
+            values, sums = layer.read("hidden", np.uint16), layer.read("pair_output", np.uint16)
+            exponents = layer.read("hidden_exponents", np.uint32 if fmt == B128 else np.uint8)
+            say("  hidden values that are not numbers %d, down sums %d, largest scale %d" %
+                (np.count_nonzero(values == 0x7FC0), np.count_nonzero(sums == 0x7FC0), int(exponents.max())))
+            assert np.any(values == 0x7FC0)
+            if limit > 10.0:
+                assert fmt == B128 or np.any(exponents > 146)
+            if limit == 1e30:
+                assert np.any(sums == 0x7FC0)
+    for name, narrow, wide, native in zip(NAMES, *outputs):
+        if fmt == B128 and name == "hidden_operands":
+            continue  # the wide launches leave the hidden values there, the job-table kernels nothing
+        assert np.array_equal(narrow, wide), name
+        assert np.array_equal(narrow, native), name
+
+
+@pytest.mark.parametrize("fmt,outputs", [(E2M1, 64), (E2M1, 192), (E2M1, 320), (E2M1, 576), (E4M3, 32), (E4M3, 96), (E4M3, 160)])
+def test_down_outputs_of_half_a_strip(amd, card, fmt, outputs):
+    """Down products of any outputs the formats store (4-bit: 64 k; one byte: 32 k), not of whole strips of 128: a strip that
+    begins at the last tiles again, a matrix of fewer tiles than a strip; the reference's lay-out through the wide and the
+    job-table kernels, gfx950's through whole and narrow strips."""
+    say("down outputs", fmt, outputs)
+    from anemone_amd import workloads
+    hidden, inner, experts_n, picks, rows = 640, 256, 64, 2, 150
+
+    class Layer(amd.Fp4Layer):
+        def experts_description(self, wide=None):
+            description = super().experts_description(wide)
+            description.down_shape = amd.Shape(outputs, self.I, self.bits, 0)
+            return description
+
+        def wide_router(self):
+            return amd.WideRouter(self, self.rows, self.weight_format, amd.Shape(self.I, self.H, self.bits, 0), amd.Shape(outputs, self.I, self.bits, 0))
+    down = workloads.fp4_matrix if fmt == E2M1 else workloads.fp8_matrix
+    trios = [trio[:2] + [down(5100 + e, outputs, inner)] for e, trio in enumerate(matrices_of(hidden, inner, 8, 99, fmt))]
+    router = to_bf16(normals(101, experts_n * hidden) * 0.02).reshape(experts_n, hidden)
+    x = to_bf16(normals(103, rows * hidden)).reshape(rows, hidden)
+    packed = [[amd.gfx950_pack(NATIVE_OF[fmt], *((inner, hidden) if m < 2 else (outputs, inner)), matrix) for m, matrix in enumerate(trio)] for trio in trios]
+    count, results = rows * picks, {}
+    for native, matrices in ((False, trios), (True, packed)):
+        layer = Layer(card, hidden, inner, experts_n, picks, rows, [matrices[e % 8] for e in range(experts_n)], router_weights_bf16=router,
+                      weight_format=fmt, gate_up_slices=1, down_slices=1)
+        if native:  # the matrices are packed already, in shapes of their own
+            layer.weight_format, layer.native = NATIVE_OF[fmt], True
+        _, wide = run_wide(card, layer, x, rows)
+        forms = {"wide": layer.wide_expert_launches(wide)}
+        if not native:
+            forms["jobs"] = layer.expert_launches(wide)
+        elif fmt == E2M1:
+            narrow = forms["narrow"] = layer.wide_expert_launches(wide)
+            narrow[0].kernel, narrow[1].kernel = layer.native_kernels.native_expert_gate_up_narrow, layer.native_kernels.native_expert_down_narrow
+            narrow[0].grid[0], narrow[1].grid[0] = -(-inner // 128), -(-outputs // 256)
+            forms["wide"][0].kernel, forms["wide"][1].kernel = layer.native_kernels.native_expert_gate_up, layer.native_kernels.native_expert_down
+            forms["wide"][0].grid[0], forms["wide"][1].grid[0] = -(-inner // 256), -(-outputs // 512)
+        for form, launches in forms.items():
+            for name in NAMES:
+                card.upload(layer.ranges[name].byte_offset, np.full(layer.ranges[name].byte_count, 0xEE, dtype=np.uint8))
+            card.run(launches)
+            sums, sums_of_rows = layer.read("pair_output"), layer.read("row_output")
+            assert np.all(sums[count * outputs * 2:] == 0xEE) and np.all(sums_of_rows[rows * outputs * 4:] == 0xEE), (native, form)
+            results[native, form] = (sums[:count * outputs * 2].copy(), sums_of_rows[:rows * outputs * 4].copy())
+    first = results[False, "jobs"]
+    assert np.any(first[0] != 0xEE)
+    for which, result in results.items():
+        assert all(np.array_equal(a, b) for a, b in zip(first, result)), which
 
 
 def run_jobs(card, layer, x, live):

@@ -61,12 +61,22 @@ def build(amd, card, hidden, inner, experts_n, picks, rows, seed, fmt, distinct=
     (512, 256, 64, 8, 1500, 1500, E2M1),  # runs of three tiles and more: blocks of two tiles of one expert, and a run's odd last tile
     (640, 384, 64, 8, 1100, 1003, E2M1),
     (512, 256, 64, 8, 1500, 1401, E4M3),
+    # one expert takes every row: a run of 64 tiles, cut in pieces of 16, alone and among others' tiles (and so where a window
+    # of 64 tiles ends); more unused tiles behind the used ones than the first look takes
+    (512, 256, 64, 1, 4090, 4090, -E2M1),
+    (640, 384, 64, 3, 4090, 4077, -E2M1),
+    (512, 256, 384, 1, 100, 100, -E2M1),
 ])
 def test_wide_equals_the_job_table_kernels_byte_for_byte(amd, card, hidden, inner, experts_n, picks, rows, live, fmt):
     say("wide experts", hidden, inner, experts_n, picks, rows, live, fmt)
+    one_expert, fmt = fmt < 0, abs(fmt)
     layer, _ = build(amd, card, hidden, inner, experts_n, picks, rows, 21, fmt)
     x = to_bf16(normals(31, rows * hidden)).reshape(rows, hidden)
     layer.set_rows(x, live)
+    if one_expert:
+        bias = np.zeros(experts_n, dtype=np.float32)
+        bias[5] = 100.0
+        card.upload(layer.bias_offset, bias)
     card.run(layer.projection_launch())
     wide = layer.wide_router()
     card.run(wide.launches())
