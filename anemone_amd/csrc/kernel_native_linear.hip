@@ -95,7 +95,7 @@ __device__ static __forceinline__ void native_expert_gate_up(const struct wide_e
     wide_gate_up_finish<STRIP, COLUMN_BLOCKS, B128>(arguments, arena, window, columns, pair_count, block_strip, tile0, wave, lane, chain);
 }
 
-template <bool BYTES, uint32_t DOWN_STRIP, uint32_t GROUP, bool B128 = false>
+template <bool BYTES, uint32_t DOWN_STRIP, uint32_t GROUP, bool B128 = false, bool BY_RUN = !BYTES>
 __device__ static __forceinline__ void native_expert_down(const struct wide_expert_down_arguments &arguments, unsigned char *arena)
 {
     constexpr uint32_t COLUMN_BLOCKS = 4u * GROUP;
@@ -107,7 +107,7 @@ __device__ static __forceinline__ void native_expert_down(const struct wide_expe
     const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     struct wide_expert_tile tile;
     uint32_t pair_count = 0, block_strip = 0;
-    if (!order_block_of<GROUP, true, !BYTES>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count)) {
+    if (!order_block_of<GROUP, true, BY_RUN>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count)) {
         return;
     }
     const struct wide_pair *pairs = (const struct wide_pair *)(arena + arguments.pairs_offset) + tile.first_pair;
@@ -144,7 +144,10 @@ extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_E2M1_WAVES) 
 }
 ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_down_1, wide_expert_down_arguments);
 /* the same of half the strips, at three wavefronts a SIMD: for launches of few pairs an expert whose blocks fill their last
- * round better so (anemone_amd/host/linear.c, native_takes_narrow, holds both sides' times) */
+ * round better so (anemone_amd/host/linear.c, native_takes_narrow, holds both sides' times). Down's blocks go as they are
+ * dealt: its chains are short and its runs a tile, so that the two looks at the table for an order of runs cost more than
+ * the order gives (down of 896 x 3072 x 128 experts, 4 pairs an expert: 42.2 -> 40.0 us; of 768 x 2048 x 384, 3: 65.5 -> 61.9;
+ * loads of Zipf(1.1), 24 on average: 40.4..92.9 -> 38.0..89.5); gate/up's gain 0 to 6 % from it at 24 pairs. */
 #define NATIVE_E2M1_NARROW_WAVES 3 /* 168 registers */
 extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_E2M1_NARROW_WAVES) native_expert_gate_up_narrow_1(struct wide_expert_gate_up_arguments arguments, unsigned char *arena)
 {
@@ -153,7 +156,7 @@ extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_E2M1_NARROW_
 ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_gate_up_narrow_1, wide_expert_gate_up_arguments);
 extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_E2M1_NARROW_WAVES) native_expert_down_narrow_1(struct wide_expert_down_arguments arguments, unsigned char *arena)
 {
-    native_expert_down<false, 4u, NATIVE_E2M1_COLUMN_BLOCKS / 4u>(arguments, arena);
+    native_expert_down<false, 4u, NATIVE_E2M1_COLUMN_BLOCKS / 4u, false, false>(arguments, arena);
 }
 ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_down_narrow_1, wide_expert_down_arguments);
 #define NATIVE_E4M3_WAVES 3 /* 150 and 152 registers (with four sets of weight registers the down launch took 170 left to itself, and at two wavefronts a SIMD 487 against 461 us) */

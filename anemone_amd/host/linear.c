@@ -590,27 +590,33 @@ result_status linear_wide_kernels_prepare(const struct backend_operations *backe
     return STATUS_OK;
 }
 
-/* block128: the launches of WEIGHT_FORMAT_E4M3_BLOCK128 experts (four: the hidden vectors' quantizer is a launch of its
- * own between the products); else those of the reference's formats (three) */
 /* Whether a launch of the 4-bit native kernels takes strips of `outputs` a block (three blocks a CU) in place of twice as
- * many (two). At up to 32 pairs an expert, a tile of pairs an expert, the launch is its weights' way from memory, and what
- * differs is how full its last round of blocks is: 768 blocks of one unit, or 512 of two. Strips of half the tiles against
- * whole ones, us: gate/up of 5120 x 1536 x 64 experts (384 whole blocks) 95.5 / 97.0, of 4096 x 1152 x 256 (1280) 196 / 214,
- * of 5120 x 1024 x 128 (512) 128 / 120, of 4096 x 1664 x 128 (896) 165 / 159; down of 1536 x 5120 x 64 (640) 54 / 63, of
- * 768 x 2048 x 128 (512) 23.7 / 20.7. Beyond 32 pairs whole strips read LDS half as often (70 an expert: 104 / 113);
- * fewer than 1,024 inputs are blocks that are mostly start and finish (down of 896 x 3072 x 128, 768 whole blocks: the step
- * 155 / 149). */
+ * many (two). By a tile of pairs an expert the launch is its weights' way from memory, and what differs is how full its last
+ * round of blocks is: 768 blocks of one unit, or 512 of two. Strips of half the tiles against whole ones, us, even loads of
+ * 24 pairs an expert unless said: gate/up of 3072 x 640 x 128 experts (640 narrow, 384 whole blocks) 67 / 73, of
+ * 4096 x 1152 x 256 at 3 pairs (2304, 1280) 207 / 221, of 4096 x 1664 x 128 (1664, 896) 182 / 178; down of 1536 x 5120 x 64
+ * (1280, 640) 61 / 68, of 896 x 3072 x 128 at 4 pairs (1536, 768) 40 / 45, of 768 x 2048 x 384 at 3 (3072, 1536: as full) 62 / 66.
+ * A second tile of a busy expert spills what exactly fills its rounds: 3072 x 896 x 128 (896, 512) 94 / 87 even, 95 / 107 under
+ * loads of Zipf(1.1); 5120 x 1536 x 64 (768, 384) 108 / 113 and 127 / 116. So the rounds are counted for a tile an expert and
+ * with a sixteenth of the experts at a second one, but for few pairs, which leave experts without a tile.
+ * Whole strips read LDS half as often, which counts from 28 pairs an expert on; above 32 narrow ones are taken where a
+ * quarter is gained (34 an expert: gate/up of 3072 x 512 x 128 55.9 / 60.2, of 3072 x 1280 x 384, a sixteenth gained, 335 / 322);
+ * from 52 whole ones are as fast. */
 static bool native_takes_narrow(const struct matrix_shape_record *shape, uint32_t outputs, uint32_t tile_count, uint64_t pairs)
 {
-    const uint64_t full_tiles = pairs / WIDE_TILE_PAIRS, experts = tile_count > full_tiles ? tile_count - full_tiles : 1u;
-    if (pairs > 32u * experts || shape->input_size < 1024u) {
-        return false;
-    }
-    const uint64_t narrow = ((uint64_t)shape->output_size + outputs - 1u) / outputs * experts;
-    const uint64_t whole = ((uint64_t)shape->output_size + 2u * outputs - 1u) / (2u * outputs) * experts;
-    return (narrow + 767u) / 768u * 768u < (whole + 511u) / 512u * 1024u;
+    const uint64_t pairs_tiles = (pairs + WIDE_TILE_PAIRS - 1u) / WIDE_TILE_PAIRS; /* tile_count: these and the experts (ROUTER_WIDE_TILES_OF) */
+    const uint64_t experts = tile_count > pairs_tiles ? tile_count - pairs_tiles : 1u;
+    const uint64_t narrow_strips = ((uint64_t)shape->output_size + outputs - 1u) / outputs, whole_strips = (narrow_strips + 1u) / 2u;
+    const uint64_t busy = pairs <= 4u * experts ? experts : experts + experts / 16u; /* tiles when some experts have two */
+    const uint64_t narrow = (narrow_strips * experts + 767u) / 768u * 768u, narrow_busy = (narrow_strips * busy + 767u) / 768u * 768u;
+    const uint64_t whole = (whole_strips * experts + 511u) / 512u * 1024u, whole_busy = (whole_strips * busy + 511u) / 512u * 1024u;
+    return pairs <= 28u * experts   ? narrow + narrow_busy <= whole + whole_busy
+           : pairs <= 32u * experts ? narrow + narrow_busy < whole + whole_busy
+                                    : pairs <= 48u * experts && 4u * narrow_busy <= 3u * whole;
 }
 
+/* block128: the launches of WEIGHT_FORMAT_E4M3_BLOCK128 experts (four: the hidden vectors' quantizer is a launch of its
+ * own between the products); else those of the reference's formats (three) */
 static result_status wide_experts_prepare(const struct linear_wide_experts_description *description, uint64_t arena_byte_count,
                                           const struct linear_kernels_record *linear_kernels,
                                           const struct linear_wide_kernels_record *kernels, const struct linear_native_kernels_record *native_kernels,

@@ -863,15 +863,21 @@ def test_block128_prepare_geometry_and_refusals(fake):
 
 @pytest.mark.parametrize("experts_n,rows,down_input,gate_up,down", [
     (256, 1024, 2048, "native_expert_gate_up_1", "native_expert_down_1"),                # whole blocks fill whole rounds of 512
-    (64, 128, 1536, "native_expert_gate_up_narrow_1", "native_expert_down_1"),           # 384 whole blocks, 768 narrow ones
-    (64, 256, 1536, "native_expert_gate_up_narrow_1", "native_expert_down_1"),           # 32 pairs an expert
-    (64, 257, 1536, "native_expert_gate_up_1", "native_expert_down_1")])                 # more
+    (64, 128, 1536, "native_expert_gate_up_1", "native_expert_down_narrow_1"),           # 768 narrow blocks, but for second tiles
+    (64, 256, 1152, "native_expert_gate_up_narrow_1", "native_expert_down_1"),           # 32 pairs an expert: 576 narrow blocks, 320 whole
+    (64, 257, 1536, "native_expert_gate_up_1", "native_expert_down_1"),                  # more, and no quarter gained
+    (256, 70, 1152, "native_expert_gate_up_narrow_1", "native_expert_down_1"),           # pairs of no whole tiles: 2304 narrow blocks, three rounds
+    (128, 64, 896, "native_expert_gate_up_1", "native_expert_down_1"),                   # few pairs: 512 whole blocks, one round
+    (128, 65, 896, "native_expert_gate_up_narrow_1", "native_expert_down_narrow_1"),     # more than four an expert: second tiles
+    (192, 73, 896, "native_expert_gate_up_narrow_1", "native_expert_down_narrow_1"),     # down: as full either way
+    (128, 545, 512, "native_expert_gate_up_narrow_1", "native_expert_down_1"),           # 34 pairs an expert, a quarter gained
+    (128, 769, 512, "native_expert_gate_up_1", "native_expert_down_1")])                 # above 48
 def test_native_strips_by_how_full_their_last_round_is(fake, experts_n, rows, down_input, gate_up, down):
     lib, linear, native, launches = amd.library(), amd.LinearKernels(), amd.LinearNativeKernels(), amd.launches_of(4)
     assert lib.linear_kernels_prepare(fake.address, fake.card, 950, C.byref(linear)) == 0
     assert lib.linear_native_kernels_prepare(fake.address, fake.card, 950, C.byref(native)) == 0
     d = wide_experts_description(amd.WEIGHT_FORMAT_E2M1_GFX950, gate_up_shape=amd.Shape(down_input, 4096, 4, 0), down_shape=amd.Shape(4096, down_input, 4, 0),
-                                 row_count=rows, tile_count=rows * 8 // 64 + experts_n)
+                                 row_count=rows, tile_count=amd.wide_tile_count(rows, 8, experts_n))
     assert lib.linear_native_experts_prepare(C.byref(d), 8 << 30, C.byref(linear), C.byref(native), launches) == 0
     assert [fake.handles[launches[i].kernel][1] for i in (0, 1)] == [gate_up, down]
     assert launches[0].grid[0] == -(-down_input // (128 if "narrow" in gate_up else 256)) and launches[1].grid[0] == -(-4096 // (256 if "narrow" in down else 512))
