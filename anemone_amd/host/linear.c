@@ -778,12 +778,15 @@ result_status linear_native_kernels_prepare(const struct backend_operations *bac
                   {KERNEL_NATIVE_EXPERT_DOWN_STEM "b128_1", sizeof(struct wide_expert_down_arguments)},
                   {KERNEL_NATIVE_EXPERT_GATE_UP_STEM "narrow_1", sizeof(struct wide_expert_gate_up_arguments)},
                   {KERNEL_NATIVE_EXPERT_DOWN_STEM "narrow_1", sizeof(struct wide_expert_down_arguments)}};
-    enum { WANTED = sizeof wanted / sizeof wanted[0] };
+    enum { WANTED = sizeof wanted / sizeof wanted[0], REQUIRED = WANTED - 2 }; /* without the narrow ones every launch is of whole strips */
     uint32_t handles[WANTED];
     _Static_assert(sizeof(struct linear_native_kernels_record) == sizeof handles, "a handle a member, in the members' order");
     for (uint32_t i = 0; i < WANTED; i++) {
+        handles[i] = BACKEND_NO_KERNEL;
         const result_status status = backend->kernel_prepare(card, KERNEL_FILE_NATIVE_LINEAR, wanted[i].name, wanted[i].record_bytes, &handles[i]);
-        if (status != STATUS_OK) {
+        if (status != STATUS_OK && i >= REQUIRED) {
+            handles[i] = BACKEND_NO_KERNEL;
+        } else if (status != STATUS_OK) {
             REFUSE("linear_native_kernels_prepare: %s: %s", wanted[i].name, status_text(status));
             return status;
         }

@@ -607,7 +607,7 @@ struct linear_native_kernels_record {
     uint32_t native_expert_down_e4m3;
     uint32_t native_expert_gate_up_b128; /* E4M3_BLOCK128_GFX950 */
     uint32_t native_expert_down_b128;
-    uint32_t native_expert_gate_up_narrow; /* E2M1_GFX950, strips of half the tiles */
+    uint32_t native_expert_gate_up_narrow; /* E2M1_GFX950, strips of half the tiles; BACKEND_NO_KERNEL: launches of whole strips alone */
     uint32_t native_expert_down_narrow;
 };
 MUST_CHECK result_status linear_native_kernels_prepare(const struct backend_operations *backend, struct device_card *card,

@@ -883,6 +883,23 @@ def test_native_strips_by_how_full_their_last_round_is(fake, experts_n, rows, do
     assert launches[0].grid[0] == -(-down_input // (128 if "narrow" in gate_up else 256)) and launches[1].grid[0] == -(-4096 // (256 if "narrow" in down else 512))
 
 
+def test_native_kernels_without_the_narrow_ones(fake):
+    """A backend without the kernels of narrow strips prepares the others, and every launch is of whole strips."""
+    lib, linear, native, launches = amd.library(), amd.LinearKernels(), amd.LinearNativeKernels(), amd.launches_of(4)
+    for function in ("native_expert_gate_up_narrow_1", "native_expert_down_narrow_1"):
+        del fake.table["kernel_native_linear", function]
+    assert lib.linear_kernels_prepare(fake.address, fake.card, 950, C.byref(linear)) == 0
+    assert lib.linear_native_kernels_prepare(fake.address, fake.card, 950, C.byref(native)) == 0
+    assert native.native_expert_gate_up_narrow == native.native_expert_down_narrow == amd.BACKEND_NO_KERNEL
+    d = wide_experts_description(amd.WEIGHT_FORMAT_E2M1_GFX950, gate_up_shape=amd.Shape(1152, 4096, 4, 0), down_shape=amd.Shape(4096, 1152, 4, 0),
+                                 row_count=70, tile_count=amd.wide_tile_count(70, 8, 256))
+    assert lib.linear_native_experts_prepare(C.byref(d), 8 << 30, C.byref(linear), C.byref(native), launches) == 0
+    assert fake.handles[launches[0].kernel][1] == "native_expert_gate_up_1" and launches[0].grid[0] == 5
+    del fake.table["kernel_native_linear", "native_expert_down_1"]  # a kernel that every launch needs
+    other = amd.LinearNativeKernels()
+    assert lib.linear_native_kernels_prepare(fake.address, fake.card, 950, C.byref(other)) != 0 and not any(bytes(other))
+
+
 def test_gfx950_formats_prepare_geometry_and_refusals(fake):
     """The formats in gfx950's lane order (7, 8, 9): the job-table launches by the expert_*_gfx950_<S> kernels on the
     reference formats' grids, the wide form by linear_native_experts_prepare alone, the producer refused."""
