@@ -213,6 +213,7 @@ result_status exl3_tc_prepare_detached(const struct exl3_tc_record *record, uint
  * EXL3_TCP_THIN_PARTS times as many, and exl3_tcp_operands_thin and exl3_tcp_activate_thin of (width / 512, pairs / 4)
  * blocks of 256.
  */
+/* the forms' float32 sums differ in order: a row's bits are the same in every call on one side of this line, not across it */
 static bool exl3_tcp_is_thin(uint64_t pairs, uint64_t experts, uint32_t hidden, uint32_t intermediate)
 {
     return pairs <= EXL3_TCP_THIN_PAIRS * experts && hidden <= EXL3_TCP_THIN_WIDTH && intermediate <= EXL3_TCP_THIN_WIDTH;
@@ -316,7 +317,7 @@ result_status exl3_tcp_prepare(const struct exl3_tcp_record *record, uint64_t ar
 }
 
 /* the reference's _base and _hybrid forms pick between two GEMM forms of its 640-column geometry that give the same
- * bits; here there is one form */
+ * bits; here the call's sizes pick (exl3_tcp_is_thin), under every name */
 result_status exl3_tcp_prepare_base(const struct exl3_tcp_record *record, uint64_t arena_byte_count,
                                     const struct backend_operations *backend, struct device_card *card,
                                     struct kernel_launch launches_out[EXL3_TCP_MOST_LAUNCHES], uint32_t *launch_count_out)

@@ -135,8 +135,11 @@ MUST_CHECK result_status exl3_tc_run_static(const struct exl3_tc_record *record,
                                             uint64_t arena_byte_count, void *stream);
 
 /* The prefill form (include/anemone/exl3_tc.h:40-59 of the reference): fills launches_out and *launch_count_out
- * (EXL3_TCP_LAUNCHES here). The reference's _base and _hybrid choose between two GEMM forms of the same bits; this
- * library has one form behind all three names. */
+ * (EXL3_TCP_LAUNCHES here). The reference's _base and _hybrid choose between two GEMM forms of the same bits; here all
+ * three names fill the same launches, and which of two GEMM forms those are follows from the call's sizes: at most
+ * EXL3_TCP_THIN_PAIRS pairs an expert on average, or more. Either form adds an output's float32 products in a fixed order of its
+ * own, so a row's bits do not depend on the other rows of a call, and they are the same in every call on the same side of that
+ * line; across it they differ by the rounding of the sums (2.6e-4 of the output's root mean square at the most seen). */
 MUST_CHECK result_status exl3_tcp_prepare(const struct exl3_tcp_record *record, uint64_t arena_byte_count,
                                           const struct backend_operations *backend, struct device_card *card,
                                           struct kernel_launch launches_out[EXL3_TCP_MOST_LAUNCHES],

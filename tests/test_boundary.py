@@ -510,6 +510,19 @@ def test_tcp_prepare_takes_the_thin_gemm_up_to_sixteen_pairs_an_expert(fake, row
         assert list(launches[index].grid) == [(width + 511) // 512] + ([rows * 2, 1] if thin else [capacity, 10])
 
 
+@pytest.mark.parametrize("rows", [512, 513])
+def test_tcp_prepare_fills_the_same_launches_under_its_three_names(fake, rows):
+    """On either side of the thin GEMM's line: which form a call takes follows from its sizes alone."""
+    lib, filled = amd.library(), []
+    record = tcp_record(row_count=rows, output_offset=1 << 32, workspace_offset=1 << 33)
+    for prepare in (lib.exl3_tcp_prepare, lib.exl3_tcp_prepare_base, lib.exl3_tcp_prepare_hybrid):
+        prepare.restype, prepare.argtypes = lib.exl3_tcp_prepare.restype, lib.exl3_tcp_prepare.argtypes
+        launches, count = amd.launches_of(8), C.c_uint32(0)
+        assert prepare(C.byref(record), 1 << 40, fake.address, fake.card, launches, C.byref(count)) == 0 and count.value == 7
+        filled.append(bytes(launches))
+    assert filled[0] == filled[1] == filled[2]
+
+
 def test_tcp_prepare_geometry_and_refusals(fake):
     lib = amd.library()
     launches, count = amd.launches_of(8), C.c_uint32(0)

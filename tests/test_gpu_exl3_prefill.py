@@ -156,6 +156,31 @@ def test_thin_gemm_at_the_edges_of_its_blocks(amd, card, hidden, inner, width_ch
     assert error <= 4e-3 and apart <= 4 * 5 * 2.0 ** -10 / inner ** 0.5
 
 
+@pytest.mark.parametrize("counts,thin", [((70, 301, 512), True), ((513, 700), False)])
+def test_a_rows_bits_do_not_depend_on_the_calls_other_rows(amd, card, counts, thin):
+    """The same seventy rows in calls of several sizes on one side of the line between the two GEMM forms (16 pairs an expert on
+    average): every output bit."""
+    say("prefill rows of other calls", counts)
+    hidden, inner, experts_n, picks, kept = 512, 384, 64, 2, 70
+    layer, _, _ = build_layer(amd, card, hidden, inner, experts_n, picks, counts[-1], 27, [2, 3, 4])
+    x = to_bf16(normals(37, counts[-1] * hidden)).reshape(counts[-1], hidden)
+    table = np.zeros((counts[-1], picks), dtype=np.dtype([("expert", "<u4"), ("route_weight", "<f4")]))
+    rng = np.random.default_rng(5)
+    table["expert"] = np.argsort(rng.random((counts[-1], experts_n)), axis=1)[:, :picks]
+    table["route_weight"] = rng.uniform(0.1, 1.0, table.shape).astype(np.float32)
+    outputs = []
+    for count in counts:
+        order = np.concatenate([np.arange(kept, count), np.arange(kept)])  # the kept rows last: other places, other chunks' columns
+        picks_at = card.place(np.ascontiguousarray(table[order]).view(np.uint8).reshape(-1))
+        layer.rows, layer.tcp_workspace_offset = count, None
+        layer.set_rows(np.ascontiguousarray(x[order]), count)
+        launches = layer.tcp_launches(picks_at)
+        assert launches[5].grid[2] == (4 if thin else 1)
+        card.run(launches)
+        outputs.append(layer.output()[count - kept:].view(np.uint32).copy())
+    assert all(np.array_equal(outputs[0], other) for other in outputs[1:]) and np.any(outputs[0] != 0)
+
+
 def test_prefill_equals_fused_decode_on_the_same_rows(amd, card):
     """Eight rows through the fused decode and through the prefill form: the same operands, weights and float32 chains
     cut differently along k (the decode's slices against one chain): equal within float32 rounding of the sums."""
