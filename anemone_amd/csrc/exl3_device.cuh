@@ -1,20 +1,10 @@
 /*
- * exl3_device.cuh -- device code shared by the EXL3 kernels of gfx950: the mul1 codebook in registers, the
- * 128-point Hadamard transform of one wavefront, the deterministic exponential, and the wavefront product routine
- * that streams trellis tiles through LDS into MFMA.
+ * exl3_device.cuh -- device code shared by the EXL3 kernels of gfx950, and by the others for its conversions: the mul1
+ * codebook in registers, the 128-point Hadamard transform of one wavefront and of a row of sixteen lanes, and the
+ * deterministic exponential. The product routines, which say which lane decodes what, are exl3_stream_device.cuh's.
  *
- * Definitions followed (reference tree): codebook source/kernel_exl3.cu:58-65; tile placement
- * tools/measure/trellis_reference.h:10-11; window end include/anemone/exl3_records.h:111-119; transform order
- * source/kernel_exl3.cu:104-124. The lane mapping below is this build's own (wave64, v_mfma_f32_16x16x32_f16).
- *
- * Lane mapping of one MFMA step. A step multiplies 16 outputs by 32 inputs (two stacked 16 x 16 tiles, tau = 0, 1)
- * with up to 16 operand columns. Lane l owns output row o = l % 16 and input group g = l / 16; it takes from tile
- * tau = g / 2 the two runs of four consecutive ring symbols that belong to row o and to chunks t = 2 q, 2 q + 1,
- * q = g % 2: ring positions 8 (4 (o % 8) + t) + 4 (o / 8) + j, j = 0..3, which are the tile's inputs
- * 2 t + j % 2 + 8 (j / 2). So every symbol of both tiles is decoded by exactly one lane and never moves between
- * lanes. Ordered as (run 0: j = 0, 1), (run 1: j = 0, 1), (run 0: j = 2, 3), (run 1: j = 2, 3) the lane's eight
- * weights are the inputs 16 tau + 4 q + {0, 1, 2, 3, 8, 9, 10, 11}: two runs of four consecutive inputs, which the
- * operand side loads as two 8-byte words.
+ * Definitions followed (reference tree): codebook source/kernel_exl3.cu:58-65; transform order
+ * source/kernel_exl3.cu:104-124.
  */
 #ifndef EXL3_DEVICE_CUH
 #define EXL3_DEVICE_CUH

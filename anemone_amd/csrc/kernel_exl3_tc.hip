@@ -5,9 +5,10 @@
  *
  * The arithmetic is the chain's (kernel_exl3.hip): fp16 operands from a float32 Hadamard transform, the codebook's
  * weights (see EXACT_WEIGHTS), float32 MFMA sums, SwiGLU in float32, the weighted pair outputs added in slot order. What
- * differs is the work mapping: every (job, matrix, strip of eight output tiles, K slice) is an independent wavefront item
- * that streams its bytes once, from memory straight into the registers of the lanes that decode them; K-slice partial sums are kept apart in the workspace and added in slice order by the next
- * launch, so a result does not depend on scheduling, on the other rows of the step or on the grid.
+ * differs is the work mapping: every (job, matrix, strip of four output tiles, or of two in a launch of few blocks, K slice) is
+ * an independent wavefront item that streams its bytes once, from memory straight into the registers of the lanes that decode
+ * them; K-slice partial sums are kept apart in the workspace and added in slice order by the next launch, so a result does not
+ * depend on scheduling, on the other rows of the step or on the grid.
  *
  * Workspace (exl3_tc_workspace_bytes): fp16 operands [2][pairs][hidden], reused as [pairs][intermediate] for the
  * down operands; float32 gate/up partials [GATE_UP_SLICES][2][pairs][intermediate]; float32 down partials

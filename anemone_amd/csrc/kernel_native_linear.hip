@@ -49,8 +49,9 @@ __device__ static __forceinline__ void native_vectors_of(const struct wide_pair 
  * registers; 4 and 3, at 168, and 6 and 3 measured the same) */
 /* float32 block scales: a step's products start from zero and are added times the scales, which takes registers the
  * E8M0 forms leave free. Three sets of weight registers for either product; gate/up two wavefronts a SIMD (901 us a
- * launch of 2048 tokens, against 915 to 940 with four sets, and 1065 with four sets held to 168 registers by spills),
- * down three (459 us, against 484 at two wavefronts and 529 with four sets) */
+ * launch of 2048 tokens, against 915 to 940 with four sets, and 1065 with four sets held to 168 registers by spills), and
+ * down two (216 registers; held to three wavefronts it spills, which the build refuses; 529 us with four sets, 450 to 484
+ * with three) */
 #define NATIVE_B128_SLOTS 3u
 #define NATIVE_B128_GATE_UP_WAVES 2
 #define NATIVE_B128_DOWN_WAVES 2

@@ -13,7 +13,7 @@
  * K steps side by side: the weights come from memory once a run, and the run's columns (256 KB a tile of 4,096 inputs)
  * stay in that die's cache for the strips after the first.
  *
- * The 4-bit launches take this order, but for the narrow down's (BY_RUN; 8192 rows of 4096 x 2048 x 256 experts in gfx950's lane order: 5.6 -> 3.2 GB
+ * The 4-bit launches take this order, but for the narrow down's (BY_RUN; 8192 rows of 4096 x 2048 x 256 experts in gfx950's lane order: 5.5 -> 3.4 GB
  * fetched by a gate/up launch). One-byte launches keep the blocks as dealt: their tiles are taken two at a time, so that
  * an expert's matrix is read about once either way, and the second look at the table costs more (2 to 4 %).
  *
