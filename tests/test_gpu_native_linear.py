@@ -320,10 +320,10 @@ def test_native_job_table_kernels_equal_the_reference_lay_out(amd, card, hidden,
             assert a.reshape(-1)[:count].tobytes() != bytes([0xEE]) * count, "the launches wrote"
 
 
-@pytest.mark.parametrize("hidden,inner,rows,live", [(512, 384, 100, 100), (640, 128, 70, 67)])
+@pytest.mark.parametrize("hidden,inner,rows,live", [(512, 384, 100, 100), (640, 128, 70, 67), (256, 128, 2500, 2497)])
 def test_narrow_and_whole_strips_give_the_same_bytes(amd, card, hidden, inner, rows, live):
     """The 4-bit wide launches of strips of half the tiles (native_expert_gate_up_narrow_1, native_expert_down_narrow_1) and
-    of whole strips, over the same rows: every output byte. Widths that end inside a block of either."""
+    of whole strips, over the same rows: every output byte. Widths that end inside a block of either; runs of two tiles."""
     say("narrow and whole strips", hidden, inner, rows, live)
     experts_n, picks = 64, 2
     router = to_bf16(normals(81, experts_n * hidden) * 0.02).reshape(experts_n, hidden)
