@@ -306,13 +306,35 @@ ANEMONE_KERNEL(EXL3_TCP_KERNEL_FILE, exl3_tcp_operands_thin, exl3_tcp_record);
  * at the slots piece ^ ((column / 2) % 8) so that sixteen lanes of one read (sixteen columns, one piece) meet sixteen
  * different bank groups. Each wavefront brings a share of the stage by LDS DMA a step ahead, one barrier a step; the
  * reader of column block j takes piece 4 s + 2 (lane / 32) + v of column 32 j + lane % 32 as the instruction's B operand.
+ *
+ * What bounds it: the vector unit's decoding and the matrix unit, at the clock the card holds under both (1.8 GHz), and
+ * the cycles in which a wavefront has neither to issue. The step's one barrier therefore stands ahead of its last two
+ * operands' matrix instructions (all of the step's columns are in registers by then): the next step's first columns are
+ * read and its first operand is decoded in their shadow, where both stood bare behind a barrier at the step's end.
+ * 4096 rows of 4096 x 2048 x 256 experts, Zipf(1.1) loads, builds in turns on one card: gate/up 1525 -> 1475 us, down
+ * 855 -> 815. The addresses are kept as a base common to the wavefront and one offset a lane, which makes the registers
+ * for that (24 spilled with an address a lane, 2 now, neither in the loop over the steps).
  */
 /* 16 bytes a lane from memory straight into LDS (lane L lands at lds_base + 16 L), no register in between. Written as
  * assembly: the compiler keeps no book on it, so the wait that ends a step (every load of the wavefront, then the block's
  * barrier) is written out below. */
-__device__ static __forceinline__ void tcp_load_to_lds(const void *lane_address, uint32_t lds_base)
+__device__ static __forceinline__ void tcp_load_to_lds(const unsigned char *base, uint32_t lane_offset, uint32_t lds_base)
 {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(lane_address), "s"(lds_base) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_offset), "s"(base), "s"(lds_base) : "memory", "m0");
+}
+
+/* exl3_chunk_load of a base common to the wavefront and the lane's own byte offsets from it */
+template <uint32_t bits_x2>
+__device__ static __forceinline__ void tcp_chunk_load(const unsigned char *base, uint32_t own, uint32_t front, exl3_chunk_words<bits_x2> &out)
+{
+    typedef exl3_chunk<bits_x2> C;
+    typedef uint32_t words_t __attribute__((ext_vector_type(C::words)));
+    out.z[0] = *(const uint32_t *)(base + front);
+    const words_t load = *(const words_t *)(base + own);
+#pragma unroll
+    for (uint32_t word = 0; word < C::words; word++) {
+        out.z[word + 1u] = load[word];
+    }
 }
 
 #define TCP_STAGE_COLUMN_BYTES (TCP_STEP_INPUTS * 2u)
@@ -342,26 +364,22 @@ tcp_wave_gemm(const uint32_t *__restrict__ codes, uint32_t out_tiles, uint32_t s
     const bool odd = (c & 1u) != 0u;
     uint32_t own, front;
     exl3_chunk_place<bits_x2>(c, own, front);
-    const uint64_t step_stride = 4u * (uint64_t)out_tiles * C::tile_words, half_stride = 2u * (uint64_t)out_tiles * C::tile_words;
+    const uint64_t step_stride = 16u * (uint64_t)out_tiles * C::tile_words, half_stride = 8u * (uint64_t)out_tiles * C::tile_words; /* bytes */
     /* a strip past the matrix reads the matrix's first strip (its sums are not stored): every wavefront runs the same loop */
-    const uint32_t *tile = codes + ((uint64_t)(g / 2u) * out_tiles + (strip_is_live ? strip_tile : 0u) + i / 8u + 2u * (g % 2u)) * C::tile_words;
+    const unsigned char *tile = (const unsigned char *)(codes + (uint64_t)(strip_is_live ? strip_tile : 0u) * C::tile_words);
+    const uint32_t lane_tile = ((g / 2u) * out_tiles + i / 8u + 2u * (g % 2u)) * C::tile_words;
+    own = (own + lane_tile) * 4u;
+    front = (front + lane_tile) * 4u;
     /* the stage's groups this wavefront brings: wave, wave + 4, ...: lane L column 8 G + L / 8, slot L % 8 */
-    const unsigned char *operand_source[wave_groups];
+    uint32_t operand_source[wave_groups];
 #pragma unroll
     for (uint32_t part = 0; part < wave_groups; part++) {
         const uint32_t group = wave + TCP_GEMM_WAVES * part, column = 8u * group + lane / 8u;
         const uint32_t piece = (lane % 8u) ^ ((column / 2u) % 8u);
-        operand_source[part] = (const unsigned char *)(columns + (uint64_t)(column < column_count ? column : 0u) * inputs) + piece * 16u;
+        operand_source[part] = (column < column_count ? column : 0u) * inputs * 2u + piece * 16u;
     }
     /* where this lane reads its B operand (half s, inputs v) of column block j: column 32 j + row, piece 4 s + 2 upper + v */
-    uint32_t read_at[2][2];
-#pragma unroll
-    for (uint32_t s = 0; s < 2u; s++) {
-#pragma unroll
-        for (uint32_t v = 0; v < 2u; v++) {
-            read_at[s][v] = row * TCP_STAGE_COLUMN_BYTES + (((4u * s + 2u * upper + v) ^ ((row / 2u) % 8u)) * 16u);
-        }
-    }
+    const uint32_t read_at = stages + row * TCP_STAGE_COLUMN_BYTES + (((2u * upper) ^ ((row / 2u) % 8u)) * 16u);
 #pragma unroll
     for (uint32_t h = 0; h < 2u; h++) {
 #pragma unroll
@@ -376,76 +394,91 @@ tcp_wave_gemm(const uint32_t *__restrict__ codes, uint32_t out_tiles, uint32_t s
     exl3_chunk_words<bits_x2> held[2][2];
 #pragma unroll
     for (uint32_t s = 0; s < 2u; s++) {
-        exl3_chunk_load<bits_x2>(tile + s * half_stride, own, front, held[0][s]);
+        tcp_chunk_load<bits_x2>(tile + s * half_stride, own, front, held[0][s]);
     }
 #pragma unroll
     for (uint32_t part = 0; part < wave_groups; part++) {
         if (wave + TCP_GEMM_WAVES * part < live_groups) {
-            tcp_load_to_lds(operand_source[part], stages + (wave + TCP_GEMM_WAVES * part) * 1024u);
+            tcp_load_to_lds((const unsigned char *)columns, operand_source[part], stages + (wave + TCP_GEMM_WAVES * part) * 1024u);
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    auto one_step = [&](uint32_t step, exl3_chunk_words<bits_x2> (&now)[2], exl3_chunk_words<bits_x2> (&next)[2]) {
-        const bool more = step + 1u < steps; /* the same in every lane */
-        const uint32_t stage = stages + (step % 2u) * TCP_STAGE_BYTES, other = stages + ((step + 1u) % 2u) * TCP_STAGE_BYTES;
-        if (more) {
-            tile += step_stride;
+    /* A step is eight operands of eight weights a lane: k = 4 s + 2 v + h (the B operands of (s, v) serve both h and are
+     * read a pair of operands ahead). An operand's LIVE matrix instructions are issued with the next operand's decoding
+     * between them: the decoding runs in the products' shadow, across the steps as inside one. */
+    half8_t operand_b[2][LIVE];
+    uint32_t a[4], ahead[4]; /* the operand being multiplied, the one being decoded */
+    auto read_operands = [&](uint32_t parity, uint32_t k) { /* those of operands k and k + 1 of a step, out of the stage of its parity */
+        const uint32_t at = read_at ^ (64u * (k / 4u) + 16u * (k / 2u % 2u)); /* the piece's number lies in bits 4 to 6 */
 #pragma unroll
-            for (uint32_t s = 0; s < 2u; s++) {
-                exl3_chunk_load<bits_x2>(tile + s * half_stride, own, front, next[s]);
-            }
-#pragma unroll
-            for (uint32_t part = 0; part < wave_groups; part++) {
-                if (wave + TCP_GEMM_WAVES * part < live_groups) {
-                    tcp_load_to_lds(operand_source[part] + (uint64_t)(step + 1u) * TCP_STAGE_COLUMN_BYTES,
-                                    other + (wave + TCP_GEMM_WAVES * part) * 1024u);
-                }
-            }
+        for (uint32_t j = 0; j < LIVE; j++) {
+            operand_b[k / 2u % 2u][j] = __builtin_bit_cast(half8_t, *(const __attribute__((address_space(3))) uint4_t *)(uintptr_t)(at + parity * TCP_STAGE_BYTES + j * (32u * TCP_STAGE_COLUMN_BYTES)));
         }
+    };
+    auto decode_weight = [&](const exl3_chunk_words<bits_x2> (&now)[2], uint32_t k, uint32_t w, uint32_t (&into)[4]) {
+        const uint32_t s = k / 4u, v = k / 2u % 2u, h = k % 2u, t = w / 2u, m = 8u * t + 4u * h + 2u * v + w % 2u;
+        uint32_t funnel[C::words];
+#pragma unroll
+        for (uint32_t word = 0; word < C::words; word++) {
+            funnel[word] = __builtin_amdgcn_alignbit(now[s].z[word], now[s].z[word + 1u], 16u);
+        }
+        const uint32_t product = exl3_chunk_state<bits_x2>(now[s].z, funnel, m) * EXL3_MUL1_MULTIPLIER;
+        if (w % 2u == 0u) {
+            into[t] = __builtin_amdgcn_sad_u8(product, 0u, (uint32_t)EXL3_MUL1_BASE * 0x10001u);
+        } else {
+            const uint32_t sums = __builtin_amdgcn_sad_hi_u8(product, 0u, into[t]);
+            const half2_t scale = __builtin_bit_cast(half2_t, (uint32_t)EXL3_MUL1_SCALE * 0x10001u);
+            const half2_t bias = __builtin_bit_cast(half2_t, (uint32_t)EXL3_MUL1_BIAS * 0x10001u);
+            into[t] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(half2_t, sums), scale, bias));
+        }
+    };
+    auto ask = [&](uint32_t step, exl3_chunk_words<bits_x2> (&next)[2]) { /* the codes and columns of `step` */
+        tile += step_stride;
 #pragma unroll
         for (uint32_t s = 0; s < 2u; s++) {
-            exl3_chunk_align<bits_x2>(now[s], odd);
+            tcp_chunk_load<bits_x2>(tile + s * half_stride, own, front, next[s]);
         }
-        /* Eight operands of eight weights a lane: k = 4 s + 2 v + h (the B operands of (s, v) serve both h and are read a
-         * pair of operands ahead). An operand's LIVE matrix instructions are issued with the next operand's decoding
-         * between them: the decoding runs in the products' shadow. */
-        auto decode_weight = [&](uint32_t k, uint32_t w, uint32_t (&into)[4]) {
-            const uint32_t s = k / 4u, v = k / 2u % 2u, h = k % 2u, t = w / 2u, m = 8u * t + 4u * h + 2u * v + w % 2u;
-            uint32_t funnel[C::words];
 #pragma unroll
-            for (uint32_t word = 0; word < C::words; word++) {
-                funnel[word] = __builtin_amdgcn_alignbit(now[s].z[word], now[s].z[word + 1u], 16u);
+        for (uint32_t part = 0; part < wave_groups; part++) {
+            if (wave + TCP_GEMM_WAVES * part < live_groups) {
+                tcp_load_to_lds((const unsigned char *)columns + (uint64_t)step * TCP_STAGE_COLUMN_BYTES, operand_source[part],
+                                stages + (step % 2u) * TCP_STAGE_BYTES + (wave + TCP_GEMM_WAVES * part) * 1024u);
             }
-            const uint32_t product = exl3_chunk_state<bits_x2>(now[s].z, funnel, m) * EXL3_MUL1_MULTIPLIER;
-            if (w % 2u == 0u) {
-                into[t] = __builtin_amdgcn_sad_u8(product, 0u, (uint32_t)EXL3_MUL1_BASE * 0x10001u);
-            } else {
-                const uint32_t sums = __builtin_amdgcn_sad_hi_u8(product, 0u, into[t]);
-                const half2_t scale = __builtin_bit_cast(half2_t, (uint32_t)EXL3_MUL1_SCALE * 0x10001u);
-                const half2_t bias = __builtin_bit_cast(half2_t, (uint32_t)EXL3_MUL1_BIAS * 0x10001u);
-                into[t] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(half2_t, sums), scale, bias));
-            }
-        };
-        half8_t operand_b[2][LIVE];
-        uint32_t a[4], ahead[4];
-        auto read_operands = [&](uint32_t k) { /* those of operands k and k + 1 */
+        }
+    };
 #pragma unroll
-            for (uint32_t j = 0; j < LIVE; j++) {
-                operand_b[k / 2u % 2u][j] = __builtin_bit_cast(half8_t, *(const __attribute__((address_space(3))) uint4_t *)(uintptr_t)(stage + j * (32u * TCP_STAGE_COLUMN_BYTES) + read_at[k / 4u][k / 2u % 2u]));
-            }
-        };
-        read_operands(0u); /* on their way while the first operand is decoded */
-        __builtin_amdgcn_sched_barrier(0);
+    for (uint32_t s = 0; s < 2u; s++) {
+        exl3_chunk_align<bits_x2>(held[0][s], odd);
+    }
+    read_operands(0u, 0u);
 #pragma unroll
-        for (uint32_t w = 0; w < 8u; w++) {
-            decode_weight(0u, w, a);
+    for (uint32_t w = 0; w < 8u; w++) {
+        decode_weight(held[0], 0u, w, a);
+    }
+    auto one_step = [&](uint32_t step, uint32_t parity, exl3_chunk_words<bits_x2> (&now)[2], exl3_chunk_words<bits_x2> (&next)[2]) {
+        const bool more = step + 1u < steps; /* the same in every lane */
+        if (more) {
+            ask(step + 1u, next);
         }
 #pragma unroll
         for (uint32_t k = 0; k < 8u; k++) {
             const uint32_t h = k % 2u;
             if (k % 2u == 0u && k + 2u < 8u) {
-                read_operands(k + 2u);
+                read_operands(parity, k + 2u);
+            }
+            if (k == 6u) {
+                /* every load of this wavefront has landed (the next step's codes and its share of the next stage), and it
+                 * has read this step's stage, which the step after the next takes */
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+                __syncthreads();
+                if (more) {
+#pragma unroll
+                    for (uint32_t s = 0; s < 2u; s++) {
+                        exl3_chunk_align<bits_x2>(next[s], odd);
+                    }
+                }
+                read_operands(1u - parity, 0u); /* operand_b[0]: operands 4 and 5 are done with it */
             }
             const uint4_t packed = {a[0], a[1], a[2], a[3]};
             const half8_t weights = __builtin_bit_cast(half8_t, packed);
@@ -453,11 +486,13 @@ tcp_wave_gemm(const uint32_t *__restrict__ codes, uint32_t out_tiles, uint32_t s
             for (uint32_t j = 0; j < LIVE; j++) {
                 accumulator[h][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(weights, operand_b[k / 2u % 2u][j], accumulator[h][j], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
-                if (k + 1u < 8u) {
 #pragma unroll
-                    for (uint32_t w = 0; w < 8u; w++) {
-                        if (w * LIVE / 8u == j) {
-                            decode_weight(k + 1u, w, ahead);
+                for (uint32_t w = 0; w < 8u; w++) {
+                    if (w * LIVE / 8u == j) {
+                        if (k + 1u < 8u) {
+                            decode_weight(now, k + 1u, w, ahead);
+                        } else {
+                            decode_weight(next, 0u, w, ahead);
                         }
                     }
                 }
@@ -468,14 +503,11 @@ tcp_wave_gemm(const uint32_t *__restrict__ codes, uint32_t out_tiles, uint32_t s
                 a[t] = ahead[t];
             }
         }
-        /* every load of this wavefront has landed (the next step's stage among them), this step's stage is read */
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        __syncthreads();
     };
     for (uint32_t step = 0; step < steps; step += 2u) {
-        one_step(step, held[0], held[1]);
+        one_step(step, 0u, held[0], held[1]);
         if (step + 1u < steps) {
-            one_step(step + 1u, held[1], held[0]);
+            one_step(step + 1u, 1u, held[1], held[0]);
         }
     }
 }
@@ -485,7 +517,7 @@ tcp_wave_gemm(const uint32_t *__restrict__ codes, uint32_t out_tiles, uint32_t s
  * products [place][hidden]. */
 extern "C" __global__ void __launch_bounds__(TCP_GEMM_THREADS, 2) exl3_tcp_gemm(struct exl3_tcp_record record, unsigned char *arena)
 {
-    __shared__ __attribute__((aligned(16))) unsigned char stages[2u * TCP_STAGE_BYTES];
+    __shared__ __attribute__((aligned(128))) unsigned char stages[2u * TCP_STAGE_BYTES];
     const tcp_shape shape = tcp_shape_of(record);
     unsigned char *workspace = arena + record.workspace_offset;
     /* Which (strip of 256 outputs, chunk, projection) this block takes. The card deals blocks to its eight dies in turn by
