@@ -19,52 +19,47 @@
 #include "wide_finish_device.cuh"
 #include "wide_order_device.cuh"
 
-/* the vectors of the columns a wavefront brings: code_vectors[i][part] of column 8 (2 (WAVE_BLOCKS wave + i) + part) +
- * lane / 8, exponent_vector of column 16 WAVE_BLOCKS wave + lane; columns past the last pair read the first pair's. The
+/* the vectors of the columns a wavefront brings: code_vectors[part] of column lane / 8 of its group `part` of eight,
+ * exponent_vectors[i] of column 16 (WAVE_BLOCKS wave + i) + lane / 4; columns past the last pair read the first pair's. The
  * wavefront leaves the pairs of its columns in LDS for the finish (behind the chain's barriers). */
-template <uint32_t WAVE_BLOCKS>
+template <typename CHAIN>
 __device__ static __forceinline__ void native_vectors_of(const struct wide_pair *pairs, uint32_t pair_count, uint32_t divisor, uint32_t wave,
-                                                         uint32_t lane, uint32_t (&code_vectors)[WAVE_BLOCKS][2], uint32_t &exponent_vector,
-                                                         struct wide_pair *columns)
+                                                         uint32_t lane, uint32_t (&code_vectors)[2u * CHAIN::WAVE_BLOCKS],
+                                                         uint32_t (&exponent_vectors)[CHAIN::WAVE_BLOCKS], struct wide_pair *columns)
 {
+    constexpr uint32_t WAVE_BLOCKS = CHAIN::WAVE_BLOCKS;
+#pragma unroll
+    for (uint32_t part = 0; part < 2u * WAVE_BLOCKS; part++) {
+        const uint32_t column = 8u * CHAIN::group_of(wave, part) + lane / 8u;
+        code_vectors[part] = pairs[column < pair_count ? column : 0u].pair_index / divisor;
+    }
 #pragma unroll
     for (uint32_t i = 0; i < WAVE_BLOCKS; i++) {
-#pragma unroll
-        for (uint32_t part = 0; part < 2u; part++) {
-            const uint32_t column = 8u * (2u * (WAVE_BLOCKS * wave + i) + part) + lane / 8u;
-            code_vectors[i][part] = pairs[column < pair_count ? column : 0u].pair_index / divisor;
-        }
+        const uint32_t column = 16u * (WAVE_BLOCKS * wave + i) + lane / 4u;
+        exponent_vectors[i] = pairs[column < pair_count ? column : 0u].pair_index / divisor;
     }
-    const uint32_t scale_column = 16u * WAVE_BLOCKS * wave + lane % (16u * WAVE_BLOCKS);
-    const struct wide_pair pair = pairs[scale_column < pair_count ? scale_column : 0u];
-    exponent_vector = pair.pair_index / divisor;
-    columns[scale_column] = pair;
+    const uint32_t own_column = 16u * WAVE_BLOCKS * wave + lane % (16u * WAVE_BLOCKS);
+    columns[own_column] = pairs[own_column < pair_count ? own_column : 0u];
 }
 
 /* grid (ceil(output_size / (4 strips)), tile_count), block 256; a strip is STRIP tiles of gate and STRIP of up */
 /* sets of weight registers and stages of columns: 4-bit weights 2 and 2, with strips of four gate and four up tiles (eight
- * of down) at two wavefronts a SIMD (242 registers, 128 of them sums): a column block's operand read from LDS and its
+ * of down) at two wavefronts a SIMD (243 registers, 128 of them sums): a column block's operand read from LDS and its
  * preparation serve eight matrix instructions and not four (8192 rows of 4096 x 2048 x 256 experts: gate/up 1157 -> 1096
- * us, down 651 -> 625, against strips of half as many, three sets and three wavefronts); one-byte weights 3 and 3 (150
- * registers; 4 and 3, at 168, and 6 and 3 measured the same) */
-/* float32 block scales: a step's products start from zero and are added times the scales, which takes registers the
- * E8M0 forms leave free. Three sets of weight registers for either product; gate/up two wavefronts a SIMD (901 us a
- * launch of 2048 tokens, against 915 to 940 with four sets, and 1065 with four sets held to 168 registers by spills), and
- * down two (216 registers; held to three wavefronts it spills, which the build refuses; 529 us with four sets, 450 to 484
- * with three) */
-#define NATIVE_B128_SLOTS 3u
-#define NATIVE_B128_GATE_UP_WAVES 2
-#define NATIVE_B128_DOWN_WAVES 2
-template <bool BYTES, uint32_t TILES> /* tiles of a wavefront, of its matrices together */
+ * us, down 651 -> 625, against strips of half as many, three sets and three wavefronts). One-byte weights: gate/up 2 and 2
+ * at three wavefronts a SIMD (143 registers, 165 with float32 scales), down 3 and 3 at two (215 and 222): 2048 rows of
+ * 4096 x 2048 x 256 experts, gate/up 880 us against 900 (float32 scales 850 / 864), down 433 against 444 (444 / 453). */
+template <bool BYTES, bool DOWN, uint32_t TILES> /* tiles of a wavefront, of its matrices together */
 struct native_depths {
-    static constexpr uint32_t SLOTS = !BYTES && TILES == 8u ? 2u : 3u, DEPTH = BYTES ? NATIVE_E4M3_STAGES : NATIVE_E2M1_STAGES;
+    static constexpr uint32_t SLOTS = BYTES ? (DOWN ? 3u : 2u) : TILES == 8u ? 2u : 3u;
+    static constexpr uint32_t DEPTH = BYTES ? (DOWN ? NATIVE_E4M3_DOWN_STAGES : NATIVE_E4M3_GATE_UP_STAGES) : NATIVE_E2M1_STAGES;
 };
 
 template <bool BYTES, uint32_t STRIP, uint32_t GROUP, bool B128 = false>
 __device__ static __forceinline__ void native_expert_gate_up(const struct wide_expert_gate_up_arguments &arguments, unsigned char *arena)
 {
     constexpr uint32_t COLUMN_BLOCKS = 4u * GROUP;
-    typedef native_depths<BYTES, 2u * STRIP> depths;
+    typedef native_depths<BYTES, false, 2u * STRIP> depths;
     typedef native_chain<2, BYTES, STRIP, COLUMN_BLOCKS, depths::SLOTS, depths::DEPTH, B128> chain_type;
     constexpr uint32_t TILES = chain_type::TILES;
     static_assert(STRIP == 1u || STRIP % 2u == 0u, "a quantizer block of 32 outputs is two strips, or strips are whole blocks");
@@ -77,13 +72,13 @@ __device__ static __forceinline__ void native_expert_gate_up(const struct wide_e
         return;
     }
     const struct wide_pair *pairs = (const struct wide_pair *)(arena + arguments.pairs_offset) + tile.first_pair;
-    uint32_t code_vectors[chain_type::WAVE_BLOCKS][2], exponent_vector = 0;
-    native_vectors_of<chain_type::WAVE_BLOCKS>(pairs, pair_count, arguments.pairs_per_row, wave, lane, code_vectors, exponent_vector, columns);
+    uint32_t code_vectors[2u * chain_type::WAVE_BLOCKS], exponent_vectors[chain_type::WAVE_BLOCKS];
+    native_vectors_of<chain_type>(pairs, pair_count, arguments.pairs_per_row, wave, lane, code_vectors, exponent_vectors, columns);
     chain_type chain_of;
     const unsigned char *const matrices[2] = {arena + tile.gate_offset, arena + tile.up_offset};
     uint32_t tile0 = 0;
     chain_of.place(matrices, arguments.output_size, arguments.input_size, block_strip, arena + arguments.codes_offset,
-                   arena + arguments.exponents_offset, code_vectors, exponent_vector, (uint32_t)(uintptr_t)(lds_pointer)window, wave, lane, tile0);
+                   arena + arguments.exponents_offset, code_vectors, exponent_vectors, (uint32_t)(uintptr_t)(lds_pointer)window, wave, lane, tile0);
     float4_t chain[TILES][COLUMN_BLOCKS];
 #pragma unroll
     for (uint32_t t = 0; t < TILES; t++) {
@@ -100,7 +95,7 @@ template <bool BYTES, uint32_t DOWN_STRIP, uint32_t GROUP, bool B128 = false, bo
 __device__ static __forceinline__ void native_expert_down(const struct wide_expert_down_arguments &arguments, unsigned char *arena)
 {
     constexpr uint32_t COLUMN_BLOCKS = 4u * GROUP;
-    typedef native_depths<BYTES, DOWN_STRIP> depths;
+    typedef native_depths<BYTES, true, DOWN_STRIP> depths;
     typedef native_chain<1, BYTES, DOWN_STRIP, COLUMN_BLOCKS, depths::SLOTS, depths::DEPTH, B128> chain_type;
     constexpr uint32_t TILES = chain_type::TILES, STRIP = chain_type::STRIP;
     extern __shared__ __attribute__((aligned(16))) unsigned char window[];
@@ -112,13 +107,13 @@ __device__ static __forceinline__ void native_expert_down(const struct wide_expe
         return;
     }
     const struct wide_pair *pairs = (const struct wide_pair *)(arena + arguments.pairs_offset) + tile.first_pair;
-    uint32_t code_vectors[chain_type::WAVE_BLOCKS][2], exponent_vector = 0; /* the vectors are the pairs' hidden vectors */
-    native_vectors_of<chain_type::WAVE_BLOCKS>(pairs, pair_count, 1u, wave, lane, code_vectors, exponent_vector, columns);
+    uint32_t code_vectors[2u * chain_type::WAVE_BLOCKS], exponent_vectors[chain_type::WAVE_BLOCKS]; /* the vectors are the pairs' hidden vectors */
+    native_vectors_of<chain_type>(pairs, pair_count, 1u, wave, lane, code_vectors, exponent_vectors, columns);
     chain_type chain_of;
     const unsigned char *const matrices[1] = {arena + tile.down_offset};
     uint32_t tile0 = 0;
     chain_of.place(matrices, arguments.output_size, arguments.input_size, block_strip, arena + arguments.codes_offset,
-                   arena + arguments.exponents_offset, code_vectors, exponent_vector, (uint32_t)(uintptr_t)(lds_pointer)window, wave, lane, tile0);
+                   arena + arguments.exponents_offset, code_vectors, exponent_vectors, (uint32_t)(uintptr_t)(lds_pointer)window, wave, lane, tile0);
     float4_t chain[TILES][COLUMN_BLOCKS];
 #pragma unroll
     for (uint32_t t = 0; t < TILES; t++) {
@@ -160,13 +155,14 @@ extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_E2M1_NARROW_
     native_expert_down<false, 4u, NATIVE_E2M1_COLUMN_BLOCKS / 4u, false, false>(arguments, arena);
 }
 ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_down_narrow_1, wide_expert_down_arguments);
-#define NATIVE_E4M3_WAVES 3 /* 150 and 152 registers (with four sets of weight registers the down launch took 170 left to itself, and at two wavefronts a SIMD 487 against 461 us) */
-extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_E4M3_WAVES) native_expert_gate_up_e4m3_1(struct wide_expert_gate_up_arguments arguments, unsigned char *arena)
+#define NATIVE_BYTES_GATE_UP_WAVES 3
+#define NATIVE_BYTES_DOWN_WAVES 2
+extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_BYTES_GATE_UP_WAVES) native_expert_gate_up_e4m3_1(struct wide_expert_gate_up_arguments arguments, unsigned char *arena)
 {
     native_expert_gate_up<true, 1u, NATIVE_E4M3_COLUMN_BLOCKS / 4u>(arguments, arena);
 }
 ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_gate_up_e4m3_1, wide_expert_gate_up_arguments);
-extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_E4M3_WAVES) native_expert_down_e4m3_1(struct wide_expert_down_arguments arguments, unsigned char *arena)
+extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_BYTES_DOWN_WAVES) native_expert_down_e4m3_1(struct wide_expert_down_arguments arguments, unsigned char *arena)
 {
     native_expert_down<true, 2u, NATIVE_E4M3_COLUMN_BLOCKS / 4u>(arguments, arena);
 }
@@ -175,18 +171,18 @@ ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_down_e4m3_1, wide_expert
 /* E4M3_BLOCK128_GFX950 experts (float32 scales of 128 x 128 blocks, columns of 128-value float32 scales): the E4M3_GFX950
  * launches' shape; the gate/up launch leaves the hidden VALUES where the record names the hidden operands, and their
  * quantizer (activation_quantize_128_entry) is a launch of its own */
-extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_B128_GATE_UP_WAVES) native_expert_gate_up_b128_1(struct wide_expert_gate_up_arguments arguments, unsigned char *arena)
+extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_BYTES_GATE_UP_WAVES) native_expert_gate_up_b128_1(struct wide_expert_gate_up_arguments arguments, unsigned char *arena)
 {
     native_expert_gate_up<true, 1u, NATIVE_E4M3_COLUMN_BLOCKS / 4u, true>(arguments, arena);
 }
 ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_gate_up_b128_1, wide_expert_gate_up_arguments);
-extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_B128_DOWN_WAVES) native_expert_down_b128_1(struct wide_expert_down_arguments arguments, unsigned char *arena)
+extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_BYTES_DOWN_WAVES) native_expert_down_b128_1(struct wide_expert_down_arguments arguments, unsigned char *arena)
 {
     native_expert_down<true, 2u, NATIVE_E4M3_COLUMN_BLOCKS / 4u, true>(arguments, arena);
 }
 ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_down_b128_1, wide_expert_down_arguments);
 
 static_assert(native_chain<2, false, 2u, NATIVE_E2M1_COLUMN_BLOCKS, 3u, NATIVE_E2M1_STAGES>::WINDOW_BYTES == NATIVE_WINDOW_BYTES(NATIVE_E2M1_COLUMN_BLOCKS, NATIVE_E2M1_STAGES) &&
-                  native_chain<1, true, 2u, NATIVE_E4M3_COLUMN_BLOCKS, 4u, NATIVE_E4M3_STAGES>::WINDOW_BYTES == NATIVE_WINDOW_BYTES(NATIVE_E4M3_COLUMN_BLOCKS, NATIVE_E4M3_STAGES),
+                  native_chain<2, true, 1u, NATIVE_E4M3_COLUMN_BLOCKS, 2u, NATIVE_E4M3_GATE_UP_STAGES>::WINDOW_BYTES == NATIVE_WINDOW_BYTES(NATIVE_E4M3_COLUMN_BLOCKS, NATIVE_E4M3_GATE_UP_STAGES) &&
+                  native_chain<1, true, 2u, NATIVE_E4M3_COLUMN_BLOCKS, 3u, NATIVE_E4M3_DOWN_STAGES>::WINDOW_BYTES == NATIVE_WINDOW_BYTES(NATIVE_E4M3_COLUMN_BLOCKS, NATIVE_E4M3_DOWN_STAGES),
               "the windows the host asks for are the kernels'");
-

@@ -3,12 +3,20 @@
  * WEIGHT_FORMAT_E4M3_GFX950): a tile's K step of 128 inputs lies in memory as the 64 lanes' A operand of
  * v_mfma_scale_f32_16x16x128_f8f6f4, 16 bytes a lane (32 of one-byte weights, as two halves of 16), and goes from memory
  * into the wavefront's registers with one 16-byte load a lane and half: no LDS stage, no vector instruction between the
- * load and the matrix instruction. A tile's scale codes of a K step are one byte a lane, loaded as such. Only the
- * columns (the vectors' codes, which every wavefront of the block reads) pass through LDS, as in wide_device.cuh: brought
- * by LDS DMA, turned into the B operand's order in place by the wavefront that brought them.
+ * load and the matrix instruction. Only the columns (the vectors' codes, which every wavefront of the block reads) pass
+ * through LDS, as in wide_device.cuh: brought by LDS DMA; those of a block of 4-bit weights are turned into the B operand's
+ * order in place by the wavefront that brought them, a block of one-byte weights reads them as they landed.
  *
  * A block is COLUMN_BLOCKS x 16 columns (pairs of one expert) by four wavefronts' strips of weight tiles. A wavefront
  * keeps several sets of weight registers: while one step is multiplied, the loads of the steps behind it are on their way.
+ *
+ * What bounds the one-byte launches, beside the weights' way from memory, is the number of loads: with the clock read
+ * around a step's parts, a third of a wavefront's time went into asking for them (six of weights and five of columns a
+ * step, about 130 cycles each: the memory pipeline takes a wavefront's load a cache line a cycle and keeps a limited number
+ * of lines on their way). So the words of scales, which are a line each for four bytes, come in fewer loads -- the columns'
+ * four K steps together, the weights' sixty-four together, a lane a step -- and columns that hold no pair are not brought:
+ * 2048 rows of 4096 x 2048 x 256 experts, float32 scales: gate/up 930 -> 852 us, down 483 -> 446; E8M0 scales: 930 -> 897,
+ * 455 -> 435; 4-bit weights, 8192 rows: 1 %.
  */
 #ifndef NATIVE_DEVICE_CUH
 #define NATIVE_DEVICE_CUH
@@ -88,29 +96,43 @@ struct native_chain {
     static constexpr uint32_t HALVES = STEP_BYTES / 1024u;
     static constexpr uint32_t WAVE_BLOCKS = COLUMN_BLOCKS / NATIVE_WAVES;     /* column blocks a wavefront brings and prepares */
     static constexpr uint32_t VECTOR_BYTES = COLUMN_BLOCKS * 2048u;            /* a K step of the block's columns' codes */
-    static constexpr uint32_t STAGE_BYTES = VECTOR_BYTES + COLUMN_BLOCKS * 64u; /* and their scale words behind them */
-    static constexpr uint32_t WINDOW_BYTES = DEPTH * STAGE_BYTES;
-    static constexpr uint32_t VECTOR_LOADS = 2u * WAVE_BLOCKS + 1u;
-    /* scale codes: of one-byte weights a byte a lane a tile (a row of 32 outputs' codes, as the reference stores them); of
+    static constexpr uint32_t STAGE_BYTES = VECTOR_BYTES;
+    static constexpr uint32_t SCALE_STEPS = 4u; /* K steps whose scale words of the columns come together */
+    static constexpr uint32_t CHUNK_BYTES = COLUMN_BLOCKS * 16u * SCALE_STEPS * 4u; /* [column][step of the chunk] */
+    static constexpr uint32_t SCALES_AT = DEPTH * STAGE_BYTES; /* two chunks behind the stages: one in use, the next on its way */
+    static constexpr uint32_t WINDOW_BYTES = SCALES_AT + 2u * CHUNK_BYTES;
+    /* loads of a wavefront for a step's columns of LIVE column blocks: groups of eight columns (one-byte weights: a wavefront
+     * brings the groups wave, wave + 4, ... that LIVE blocks need; 4-bit weights: the two of its own block, which it also
+     * prepares), and one of scale words */
+    static constexpr uint32_t groups_of(uint32_t live)
+    {
+        return BYTES ? (live + 1u) / 2u : 2u * WAVE_BLOCKS;
+    }
+    static constexpr uint32_t vector_loads(uint32_t live)
+    {
+        return groups_of(live) + 1u;
+    }
+    /* scales: of one-byte weights a word a tile or a matrix a K step (a row of 32 outputs' four codes, as the reference stores
+     * them, or one float32), which a lane a step holds for SCALE_ROUND steps and a step takes from its lane; of
      * 4-bit weights a word a lane a matrix: its bytes are the codes of the lane's row and inputs in the four tiles of a group
      * of 64 outputs, which the matrix instruction picks by number */
     static constexpr uint32_t GROUP_TILES = STRIP < 4u ? STRIP : 4u; /* tiles of a strip that share a word of 4-bit weights' codes */
     static constexpr uint32_t GROUPS = BYTES ? 1u : STRIP / GROUP_TILES;
     static constexpr uint32_t SCALE_LOADS = BYTES && !B128 ? TILES : MATRICES * GROUPS;
-    static constexpr uint32_t WEIGHT_LOADS = TILES * HALVES + SCALE_LOADS;
+    static constexpr uint32_t WEIGHT_LOADS = TILES * HALVES + (BYTES ? 0u : SCALE_LOADS);
+    static constexpr uint32_t SCALE_ROUND = WAVE / SLOTS * SLOTS;
     static_assert(BYTES || STRIP == 2u || STRIP % 4u == 0u, "a strip of 4-bit weights is half a group of four tiles, or whole ones");
-    static_assert((DEPTH - 1u) * VECTOR_LOADS + (SLOTS - 1u) * WEIGHT_LOADS < 64u, "vmcnt has six bits");
+    static_assert((DEPTH - 1u) * vector_loads(COLUMN_BLOCKS) + (SLOTS - 1u) * WEIGHT_LOADS < 64u, "vmcnt has six bits");
 
     struct slot {
         uint4_t words[TILES][HALVES];
-        uint32_t scale[SCALE_LOADS];
+        uint32_t scale[BYTES ? 1 : SCALE_LOADS]; /* 4-bit weights */
     };
 
     const unsigned char *words[MATRICES], *scales[MATRICES], *codes, *exponents;
     uint32_t step_stride, scale_stride; /* from a tile's K step to its next; from a group's scale words to the next group's */
-    uint32_t window, wave, tile_bytes, group_bytes, word_offset, scale_offset[BYTES && !B128 ? STRIP : 1], codes_offset[WAVE_BLOCKS][2], exponents_offset;
-    uint32_t vector_at[BYTES ? 8 : 4], vector_scale_at, operand_at, scale_shift;
-    bool scale_lane;
+    uint32_t window, wave, tile_bytes, group_bytes, word_offset, scale_offset[BYTES && !B128 ? STRIP : 1], code_shift, codes_offset[2u * WAVE_BLOCKS], exponents_offset[WAVE_BLOCKS];
+    uint32_t vector_at[BYTES ? 8 : 4], vector_scale_at, operand_at, scale_shift, last_step, lane_of;
 
     template <typename T>
     __device__ static __forceinline__ T lds_read(uint32_t address)
@@ -124,19 +146,39 @@ struct native_chain {
         *(__attribute__((address_space(3))) T *)(uintptr_t)address = value;
     }
 
-    /* the block's columns of K step `at` into stage `stage`: this wavefront's column blocks and their scale words */
+    /* The scale words of a column lie in that column's own row: asked for a step at a time they are a cache line a column for
+     * four bytes, as many lines as the columns' codes. So the words of four K steps come together, a lane a step of a
+     * column: a quarter of the lines. Column block `block` of this wavefront, chunk `chunk` of four steps (a step past the
+     * last repeats the last). */
+    __device__ __forceinline__ void issue_scales(uint32_t chunk, uint32_t block) const
+    {
+        const uint32_t step = SCALE_STEPS * chunk + lane_of % SCALE_STEPS;
+        const uint32_t offset = (block == 0u ? exponents_offset[0] : exponents_offset[WAVE_BLOCKS - 1u]) + 4u * (step < last_step ? step : last_step);
+        load_to_lds_4(exponents, offset, window + SCALES_AT + chunk % 2u * CHUNK_BYTES + (wave * WAVE_BLOCKS + block) * (16u * SCALE_STEPS * 4u));
+    }
+
+    /* the group of eight columns that is this wavefront's part `part` */
+    __device__ __forceinline__ static uint32_t group_of(uint32_t wave_index, uint32_t part)
+    {
+        return BYTES ? wave_index + NATIVE_WAVES * part : 2u * WAVE_BLOCKS * wave_index + part;
+    }
+
+    /* the block's columns of K step `at` into stage `stage`, this wavefront's groups; and one load of scale words: the
+     * next chunk's are asked for behind the barrier of a chunk's first steps, a column block a step, when every wavefront is
+     * done with the chunk whose place they take (in the other steps one lane reads a word again, so that every step's loads
+     * are as many) */
+    template <uint32_t LIVE>
     __device__ __forceinline__ void issue_vectors(uint32_t stage, uint32_t at) const
     {
         const uint32_t base = window + stage * STAGE_BYTES;
 #pragma unroll
-        for (uint32_t i = 0; i < WAVE_BLOCKS; i++) {
-#pragma unroll
-            for (uint32_t part = 0; part < 2u; part++) {
-                load_to_lds_16(codes + (uint64_t)at * 128u, codes_offset[i][part], base + (wave * WAVE_BLOCKS + i) * 2048u + part * 1024u);
-            }
+        for (uint32_t part = 0; part < groups_of(LIVE); part++) {
+            load_to_lds_16(codes + (uint64_t)at * 128u, codes_offset[part], base + group_of(wave, part) * 1024u);
         }
-        if (scale_lane) { /* a lane a column: sixteen cache lines a column block */
-            load_to_lds_4(exponents + (uint64_t)at * 4u, exponents_offset, base + VECTOR_BYTES + wave * WAVE_BLOCKS * 64u);
+        const uint32_t now = at < DEPTH - 1u ? SCALE_STEPS - 1u : at - (DEPTH - 1u); /* the step that asks; ahead of the first: no chunk's first steps */
+        const bool next = now % SCALE_STEPS < WAVE_BLOCKS;
+        if (next || lane_of == 0u) {
+            issue_scales(at < DEPTH - 1u ? 0u : now / SCALE_STEPS + (next ? 1u : 0u), next ? now % SCALE_STEPS : 0u);
         }
     }
 
@@ -156,20 +198,25 @@ struct native_chain {
                 }
             }
         }
+        if constexpr (!BYTES) {
 #pragma unroll
-        for (uint32_t m = 0; m < MATRICES; m++) {
-            const unsigned char *step_scales = scales[m] + (uint64_t)at * (BYTES ? 4u : 256u);
-            if constexpr (BYTES && !B128) {
+            for (uint32_t m = 0; m < MATRICES; m++) {
 #pragma unroll
-                for (uint32_t n = 0; n < STRIP; n++) {
-                    load_1(into.scale[m * STRIP + n], step_scales, scale_offset[n]);
-                }
-            } else { /* a word a lane of a group of four tiles' codes, or the strip's one float32 scale in every lane */
-#pragma unroll
-                for (uint32_t group = 0; group < GROUPS; group++) {
-                    load_4(into.scale[m * GROUPS + group], step_scales + group * scale_stride, scale_offset[0]);
+                for (uint32_t group = 0; group < GROUPS; group++) { /* a word a lane of a group of four tiles' codes */
+                    load_4(into.scale[m * GROUPS + group], scales[m] + (uint64_t)at * 256u + group * scale_stride, scale_offset[0]);
                 }
             }
+        }
+    }
+
+    /* one-byte weights: the scale words of the steps first .. first + SCALE_ROUND - 1, a lane a step (past the last: the
+     * last's). A load a step of words that every lane shares would cost the memory pipeline as much as a tile's */
+    __device__ __forceinline__ void issue_weight_scales(uint32_t (&into)[SCALE_LOADS], uint32_t first) const
+    {
+        const uint32_t step = first + lane_of < last_step ? first + lane_of : last_step;
+#pragma unroll
+        for (uint32_t k = 0; k < SCALE_LOADS; k++) {
+            load_4(into[k], scales[B128 ? k : k / STRIP], scale_offset[B128 ? 0u : k % STRIP] + 4u * step);
         }
     }
 
@@ -183,13 +230,13 @@ struct native_chain {
             }
         }
 #pragma unroll
-        for (uint32_t k = 0; k < SCALE_LOADS; k++) {
+        for (uint32_t k = 0; k < (BYTES ? 0u : SCALE_LOADS); k++) {
             native_landed(set.scale[k]);
         }
     }
 
-    /* this wavefront's column blocks of a stage, from the codes as they landed (a column's 128 bytes in the order the
-     * quantizer writes them) to the B operand, in place: [half of the operand][lane][16 bytes]; only this wavefront
+    /* 4-bit weights: this wavefront's column blocks of a stage, from the codes as they landed (a column's 128 bytes in the
+     * order the quantizer writes them) to the B operand, in place: [half of the operand][lane][16 bytes]; only this wavefront
      * touches them before the next barrier */
     __device__ __forceinline__ void prepare_columns(uint32_t stage) const
     {
@@ -198,18 +245,11 @@ struct native_chain {
             uint32_t at = window + stage * STAGE_BYTES + (wave * WAVE_BLOCKS + i) * 2048u;
             asm volatile("" : "+s"(at));
             int8_vector b;
-            if constexpr (BYTES) {
 #pragma unroll
-                for (uint32_t v = 0; v < 8u; v++) {
-                    b[v] = (int)lds_read<uint32_t>(at + vector_at[v]);
-                }
-            } else {
-#pragma unroll
-                for (uint32_t part = 0; part < 4u; part++) {
-                    const uint2_t pair = lds_read<uint2_t>(at + vector_at[part]);
-                    b[2u * part] = (int)__builtin_amdgcn_perm(pair.y, pair.x, 0x05010400u);
-                    b[2u * part + 1u] = (int)__builtin_amdgcn_perm(pair.y, pair.x, 0x07030602u);
-                }
+            for (uint32_t part = 0; part < 4u; part++) {
+                const uint2_t pair = lds_read<uint2_t>(at + vector_at[part]);
+                b[2u * part] = (int)__builtin_amdgcn_perm(pair.y, pair.x, 0x05010400u);
+                b[2u * part + 1u] = (int)__builtin_amdgcn_perm(pair.y, pair.x, 0x07030602u);
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); /* every lane has read before any lane writes */
             lds_write<uint4_t>(at + operand_at, (uint4_t){(uint32_t)b[0], (uint32_t)b[1], (uint32_t)b[2], (uint32_t)b[3]});
@@ -217,30 +257,21 @@ struct native_chain {
         }
     }
 
-    /* tile T and the tiles behind it of the wavefront's strip against column block j (the number of the scale code's byte
-     * is part of the instruction: a constant) */
+    /* the scale words of step `step` of the columns, this lane's part aside */
+    __device__ __forceinline__ uint32_t scales_of(uint32_t step) const
+    {
+        return SCALES_AT + step / SCALE_STEPS % 2u * CHUNK_BYTES + 4u * (step % SCALE_STEPS);
+    }
+
+    /* 4-bit weights: tile T and the tiles behind it of the wavefront's strip against column block j (the number of the scale
+     * code's byte is part of the instruction: a constant) */
     template <uint32_t T>
     __device__ static __forceinline__ void multiply_tiles(const slot &set, const uint32_t (&scale_a)[SCALE_LOADS], const int8_vector &b,
                                                           uint32_t scale_b, uint32_t j, float4_t (&chain)[TILES][COLUMN_BLOCKS])
     {
-        if constexpr (B128) {
-            const uint4_t first = set.words[T][0], second = set.words[T][HALVES - 1u];
-            const int8_vector a = {(int)first.x, (int)first.y, (int)first.z, (int)first.w, (int)second.x, (int)second.y, (int)second.z, (int)second.w};
-            const float scale = __fmul_rn(__uint_as_float(scale_a[T / STRIP]), __uint_as_float(scale_b));
-            const float4_t step = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, (float4_t){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0, 127, 0, 127);
-#pragma unroll
-            for (uint32_t v = 0; v < 4u; v++) {
-                chain[T][j][v] = __fmaf_rn(step[v], scale, chain[T][j][v]);
-            }
-        } else if constexpr (BYTES) {
-            const uint4_t first = set.words[T][0], second = set.words[T][HALVES - 1u];
-            const int8_vector a = {(int)first.x, (int)first.y, (int)first.z, (int)first.w, (int)second.x, (int)second.y, (int)second.z, (int)second.w};
-            chain[T][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, chain[T][j], 0, 0, 0, (int)scale_a[T], 0, (int)scale_b);
-        } else {
-            const uint4_t w = set.words[T][0];
-            const int8_vector a = {(int)w.x, (int)w.y, (int)w.z, (int)w.w, 0, 0, 0, 0};
-            chain[T][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, chain[T][j], 4, 0, T % GROUP_TILES, (int)scale_a[T / GROUP_TILES], 0, (int)scale_b);
-        }
+        const uint4_t w = set.words[T][0];
+        const int8_vector a = {(int)w.x, (int)w.y, (int)w.z, (int)w.w, 0, 0, 0, 0};
+        chain[T][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, chain[T][j], 4, 0, T % GROUP_TILES, (int)scale_a[T / GROUP_TILES], 0, (int)scale_b);
         if constexpr (T + 1u < TILES) {
             multiply_tiles<T + 1u>(set, scale_a, b, scale_b, j, chain);
         }
@@ -249,21 +280,21 @@ struct native_chain {
     /* one K step of LIVE column blocks from a stage's columns and a set of weight registers; `between` runs behind the
      * middle column block's matrix instructions */
     template <uint32_t LIVE, typename BETWEEN>
-    __device__ __forceinline__ void consume(uint32_t stage, const slot &set, float4_t (&chain)[TILES][COLUMN_BLOCKS], BETWEEN between) const
+    __device__ __forceinline__ void consume(uint32_t stage, uint32_t step, const slot &set, float4_t (&chain)[TILES][COLUMN_BLOCKS], BETWEEN between) const
     {
-        uint32_t base = window + stage * STAGE_BYTES;
-        asm volatile("" : "+s"(base));
-        uint32_t b_at = base + operand_at, b_scale_at = base + VECTOR_BYTES + vector_scale_at;
+        uint32_t base = window + stage * STAGE_BYTES, scales = window + scales_of(step);
+        asm volatile("" : "+s"(base), "+s"(scales));
+        uint32_t b_at = base + operand_at, b_scale_at = scales + vector_scale_at;
         asm volatile("" : "+v"(b_at), "+v"(b_scale_at));
         uint32_t scale_a[SCALE_LOADS];
 #pragma unroll
-        for (uint32_t k = 0; k < SCALE_LOADS; k++) { /* 4-bit weights, two tiles a strip: the group's upper two tiles' codes down */
-            scale_a[k] = BYTES ? set.scale[k] : set.scale[k] >> scale_shift;
+        for (uint32_t k = 0; k < SCALE_LOADS; k++) { /* two tiles a strip: the group's upper two tiles' codes down */
+            scale_a[k] = set.scale[k] >> scale_shift;
         }
         __builtin_amdgcn_s_setprio(1);
         /* a column block's operand is read while the block before it is multiplied: two blocks' registers, not LIVE */
         uint4_t low = lds_read<uint4_t>(b_at), high = lds_read<uint4_t>(b_at + 1024u);
-        uint32_t scale_b = B128 ? lds_read<uint32_t>(b_scale_at) : lds_read<unsigned char>(b_scale_at); /* a code, or a float32's bits */
+        uint32_t scale_b = lds_read<unsigned char>(b_scale_at);
 #pragma unroll
         for (uint32_t j = 0; j < LIVE; j++) {
             const int8_vector b = {(int)low.x, (int)low.y, (int)low.z, (int)low.w, (int)high.x, (int)high.y, (int)high.z, (int)high.w};
@@ -272,7 +303,7 @@ struct native_chain {
             if (j + 1u < LIVE) {
                 low = lds_read<uint4_t>(b_at + (j + 1u) * 2048u);
                 high = lds_read<uint4_t>(b_at + (j + 1u) * 2048u + 1024u);
-                scale_b = B128 ? lds_read<uint32_t>(b_scale_at + (j + 1u) * 64u) : lds_read<unsigned char>(b_scale_at + (j + 1u) * 64u);
+                scale_b = lds_read<unsigned char>(b_scale_at + (j + 1u) * (16u * SCALE_STEPS * 4u));
             }
             multiply_tiles<0>(set, scale_a, b, scale_now, j, chain);
             if (j == (LIVE - 1u) / 2u) {
@@ -283,26 +314,94 @@ struct native_chain {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); /* the stage is read before the next barrier */
     }
 
-    /* how many loads may be outstanding at the top of a K step for its columns and weights to have landed: native_waits.h */
-    static constexpr bool WEIGHTS_FIRST = NATIVE_WEIGHTS_FIRST_OF(BYTES); /* inside a step: the weights asked for ahead of the columns */
-    typedef native_waits<SLOTS, DEPTH, WEIGHTS_FIRST, VECTOR_LOADS, WEIGHT_LOADS> waits;
-    __device__ static __forceinline__ uint32_t loads_behind(uint32_t step, uint32_t total)
+    /* one-byte weights: a column block's B operand, read from the stage as the codes landed: the lane's eight words lie four
+     * words apart, and the slots of the pieces put the 64 lanes of a word on every bank twice */
+    __device__ __forceinline__ void read_block(uint32_t at, uint32_t scales, uint32_t j, int8_vector &b, uint32_t &scale_b) const
     {
-        return waits::loads_behind(step, total);
+#pragma unroll
+        for (uint32_t v = 0; v < 8u; v++) {
+            b[v] = (int)lds_read<uint32_t>(vector_at[v] + at + j * 2048u);
+        }
+        const uint32_t scale_at = vector_scale_at + scales + j * (16u * SCALE_STEPS * 4u);
+        scale_b = B128 ? lds_read<uint32_t>(scale_at) : lds_read<unsigned char>(scale_at); /* a float32's bits, or a code */
     }
 
+    /* The same step of one-byte weights. A column block's operand is read while the block before it is multiplied (two or
+     * three blocks ahead: the same time, and more registers); under float32 scales a block's products enter its chains while
+     * the next block is multiplied. */
+    template <uint32_t LIVE>
+    __device__ __forceinline__ void consume_bytes(uint32_t stage, uint32_t step, const slot &set, const uint32_t (&held)[SCALE_LOADS], uint32_t holder,
+                                                  float4_t (&chain)[TILES][COLUMN_BLOCKS]) const
+    {
+        uint32_t scale_a[SCALE_LOADS];
+#pragma unroll
+        for (uint32_t k = 0; k < SCALE_LOADS; k++) {
+            const uint32_t word = (uint32_t)__builtin_amdgcn_readlane((int)held[k], (int)holder);
+            scale_a[k] = B128 ? word : word >> code_shift; /* a code: the instruction takes the lowest byte */
+        }
+        const uint32_t at = stage * STAGE_BYTES, scales = scales_of(step);
+        int8_vector b[LIVE];
+        uint32_t scale_b[LIVE];
+        float4_t products[2][TILES];
+        const auto add = [&](uint32_t j) {
+#pragma unroll
+            for (uint32_t t = 0; t < TILES; t++) {
+                const float scale = __fmul_rn(__uint_as_float(scale_a[t / STRIP]), __uint_as_float(scale_b[j]));
+#pragma unroll
+                for (uint32_t v = 0; v < 4u; v++) {
+                    chain[t][j][v] = __fmaf_rn(products[j % 2u][t][v], scale, chain[t][j][v]);
+                }
+            }
+        };
+        __builtin_amdgcn_s_setprio(1);
+        read_block(at, scales, 0u, b[0], scale_b[0]);
+#pragma unroll
+        for (uint32_t j = 0; j < LIVE; j++) {
+            asm volatile("" ::: "memory"); /* the reads below stay below the reads above, and above those of the next block */
+            if (j + 1u < LIVE) {
+                read_block(at, scales, j + 1u, b[j + 1u], scale_b[j + 1u]);
+            }
+#pragma unroll
+            for (uint32_t t = 0; t < TILES; t++) {
+                const uint4_t first = set.words[t][0], second = set.words[t][HALVES - 1u];
+                const int8_vector a = {(int)first.x, (int)first.y, (int)first.z, (int)first.w, (int)second.x, (int)second.y, (int)second.z, (int)second.w};
+                if constexpr (B128) {
+                    products[j % 2u][t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[j], (float4_t){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0, 127, 0, 127);
+                } else {
+                    chain[t][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[j], chain[t][j], 0, 0, 0, (int)scale_a[t], 0, (int)scale_b[j]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (B128) {
+                if (j != 0u) {
+                    add(j - 1u);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if constexpr (B128) {
+            add(LIVE - 1u);
+        }
+        __builtin_amdgcn_s_setprio(0);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); /* the stage is read before the next barrier */
+    }
+
+    /* how many loads may be outstanding at the top of a K step for its columns and weights to have landed: native_waits.h */
+    static constexpr bool WEIGHTS_FIRST = NATIVE_WEIGHTS_FIRST_OF(BYTES); /* inside a step: the weights asked for ahead of the columns */
+    template <uint32_t LIVE> using waits = native_waits<SLOTS, DEPTH, WEIGHTS_FIRST, vector_loads(LIVE), WEIGHT_LOADS>;
+
     /* s_waitcnt takes its count as a constant: one instruction a count that loads_behind can come to */
-    template <uint32_t WEIGHTS = 0, uint32_t VECTORS = 0>
+    template <uint32_t LIVE, uint32_t WEIGHTS = 0, uint32_t VECTORS = 0>
     __device__ static __forceinline__ void wait_behind(uint32_t count)
     {
-        if (count == WEIGHTS * WEIGHT_LOADS + VECTORS * VECTOR_LOADS) {
-            wait_loads<WEIGHTS * WEIGHT_LOADS + VECTORS * VECTOR_LOADS>();
+        if (count == WEIGHTS * WEIGHT_LOADS + VECTORS * vector_loads(LIVE)) {
+            wait_loads<WEIGHTS * WEIGHT_LOADS + VECTORS * vector_loads(LIVE)>();
             return;
         }
         if constexpr (VECTORS + 1u < DEPTH - 1u) {
-            wait_behind<WEIGHTS, VECTORS + 1u>(count);
+            wait_behind<LIVE, WEIGHTS, VECTORS + 1u>(count);
         } else if constexpr (WEIGHTS + 1u < SLOTS) {
-            wait_behind<WEIGHTS + 1u, 0u>(count);
+            wait_behind<LIVE, WEIGHTS + 1u, 0u>(count);
         } else {
             wait_loads<0>(); /* not reached: every count is one of the above */
         }
@@ -311,10 +410,16 @@ struct native_chain {
     /* K step `step` of `total` out of set K of the wavefront's sets of weight registers; the weights of step
      * `step` + SLOTS - 1 take the set the step before this one used */
     template <uint32_t LIVE, uint32_t K>
-    __device__ __forceinline__ void one_step(uint32_t step, uint32_t total, slot (&sets)[SLOTS], float4_t (&chain)[TILES][COLUMN_BLOCKS]) const
+    __device__ __forceinline__ void one_step(uint32_t step, uint32_t total, slot (&sets)[SLOTS], uint32_t (&held)[SCALE_LOADS], uint32_t round, float4_t (&chain)[TILES][COLUMN_BLOCKS]) const
     {
-        wait_behind(loads_behind(step, total));
+        wait_behind<LIVE>(waits<LIVE>::loads_behind(step, total));
         landed(sets[K]);
+        if constexpr (BYTES && K == 0u) { /* the words were asked for ahead of the first round's weights, or have been waited for */
+#pragma unroll
+            for (uint32_t k = 0; k < SCALE_LOADS; k++) {
+                native_landed(held[k]);
+            }
+        }
         const auto ask = [&]() {
             if (step + SLOTS - 1u < total) {
                 issue_weights(sets[(K + SLOTS - 1u) % SLOTS], step + SLOTS - 1u);
@@ -325,32 +430,31 @@ struct native_chain {
         }
         /* where the sets and the stages go round together the stage is a constant of the instance */
         const uint32_t stage = SLOTS % DEPTH == 0u ? K % DEPTH : step % DEPTH;
-        prepare_columns(stage);
-        __syncthreads(); /* every wavefront has read the step before and prepared its columns of this one */
+        if constexpr (!BYTES) {
+            prepare_columns(stage);
+        }
+        __syncthreads(); /* every wavefront has read the step before; its columns of this one have landed and are prepared */
         if (step + DEPTH - 1u < total) {
-            issue_vectors((stage + DEPTH - 1u) % DEPTH, step + DEPTH - 1u);
+            issue_vectors<LIVE>((stage + DEPTH - 1u) % DEPTH, step + DEPTH - 1u);
         }
         /* 4-bit weights: the next weights are asked for in the middle of the step's matrix instructions (a launch 1.7 %
          * shorter than asking ahead of them: the requests spread over the step); one-byte weights in the middle: a quarter
          * slower */
         if constexpr (WEIGHTS_FIRST) {
-            consume<LIVE>(stage, sets[K], chain, []() {});
-        } else if constexpr (BYTES) {
-            ask();
-            consume<LIVE>(stage, sets[K], chain, []() {});
+            consume_bytes<LIVE>(stage, step, sets[K], held, step - round, chain);
         } else {
-            consume<LIVE>(stage, sets[K], chain, ask);
+            consume<LIVE>(stage, step, sets[K], chain, ask);
         }
     }
 
     template <uint32_t LIVE, uint32_t K>
-    __device__ __forceinline__ void round_of_steps(uint32_t step, uint32_t total, slot (&sets)[SLOTS], float4_t (&chain)[TILES][COLUMN_BLOCKS]) const
+    __device__ __forceinline__ void round_of_steps(uint32_t step, uint32_t total, slot (&sets)[SLOTS], uint32_t (&held)[SCALE_LOADS], uint32_t round, float4_t (&chain)[TILES][COLUMN_BLOCKS]) const
     {
         if (step + K < total) {
-            one_step<LIVE, K>(step + K, total, sets, chain);
+            one_step<LIVE, K>(step + K, total, sets, held, round, chain);
         }
         if constexpr (K + 1u < SLOTS) {
-            round_of_steps<LIVE, K + 1u>(step, total, sets, chain);
+            round_of_steps<LIVE, K + 1u>(step, total, sets, held, round, chain);
         }
     }
 
@@ -369,15 +473,28 @@ struct native_chain {
     __device__ __forceinline__ void steps(uint32_t total, float4_t (&chain)[TILES][COLUMN_BLOCKS]) const
     {
         slot sets[SLOTS];
+        uint32_t held[SCALE_LOADS], round = 0; /* one-byte weights: the scale words of the steps from `round` on */
+        if constexpr (BYTES) {
+            issue_weight_scales(held, 0u);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < WAVE_BLOCKS; i++) {
+            issue_scales(0u, i);
+        }
 #pragma unroll
         for (uint32_t k = 0; k + 1u < DEPTH; k++) {
             if (k < total) {
-                issue_vectors(k, k);
+                issue_vectors<LIVE>(k, k);
             }
         }
         first_weights<0>(total, sets);
         for (uint32_t step = 0; step < total; step += SLOTS) {
-            round_of_steps<LIVE, 0>(step, total, sets, chain);
+            if (BYTES && step == round + SCALE_ROUND) { /* inputs past 128 SCALE_ROUND */
+                round = step;
+                issue_weight_scales(held, round);
+                wait_loads<0>();
+            }
+            round_of_steps<LIVE, 0>(step, total, sets, held, round, chain);
         }
     }
 
@@ -391,25 +508,26 @@ struct native_chain {
             case 3u: steps<3>(total, chain); break;
             default: steps<4>(total, chain); break;
             }
-        } else { /* five and seven run as six and eight: a block of columns past the last pair reads the first pair's again */
+        } else {
             switch (live_blocks) {
             case 1u: steps<1>(total, chain); break;
             case 2u: steps<2>(total, chain); break;
             case 3u: steps<3>(total, chain); break;
             case 4u: steps<4>(total, chain); break;
-            case 5u:
+            case 5u: steps<5>(total, chain); break;
             case 6u: steps<6>(total, chain); break;
+            case 7u: steps<7>(total, chain); break;
             default: steps<8>(total, chain); break;
             }
         }
     }
 
     /* matrices: arena addresses of the stored matrices; the block's first strip is NATIVE_WAVES block_strip;
-     * code_vectors[i][part]: the vector of column lane / 8 of group `part` of this wavefront's i-th column block;
-     * exponent_vector: the vector of column lane of this wavefront's column blocks (lanes below 16 WAVE_BLOCKS) */
+     * code_vectors[part]: the vector of column lane / 8 of this wavefront's group `part` of eight columns (group_of);
+     * exponent_vectors[i]: the vector of column lane / 4 of its i-th column block */
     __device__ __forceinline__ void place(const unsigned char *const (&matrices)[MATRICES], uint32_t outputs, uint32_t inputs,
                                           uint32_t block_strip, const unsigned char *vector_codes, const unsigned char *vector_exponents,
-                                          const uint32_t (&code_vectors)[WAVE_BLOCKS][2], uint32_t exponent_vector, uint32_t window_address,
+                                          const uint32_t (&code_vectors)[2u * WAVE_BLOCKS], const uint32_t (&exponent_vectors)[WAVE_BLOCKS], uint32_t window_address,
                                           uint32_t wave_index, uint32_t lane, uint32_t &tile0_out)
     {
         const uint32_t tiles = outputs / 16u, steps = inputs / 128u;
@@ -442,25 +560,27 @@ struct native_chain {
         if constexpr (BYTES && !B128) {
 #pragma unroll
             for (uint32_t n = 0; n < STRIP; n++) {
-                scale_offset[n] = ((tile0 + n) / 2u - tile0 / 2u) * (inputs / 32u) + g;
+                scale_offset[n] = ((tile0 + n) / 2u - tile0 / 2u) * (inputs / 32u);
             }
         } else {
             scale_offset[0] = B128 ? 0u : 4u * lane;
         }
+        code_shift = 8u * g;
+#pragma unroll
+        for (uint32_t part = 0; part < 2u * WAVE_BLOCKS; part++) {
+            codes_offset[part] = code_vectors[part] * inputs + 16u * ((lane % 8u) ^ (lane / 8u) ^ (group_of(wave_index, part) % 2u));
+        }
 #pragma unroll
         for (uint32_t i = 0; i < WAVE_BLOCKS; i++) {
-#pragma unroll
-            for (uint32_t part = 0; part < 2u; part++) {
-                codes_offset[i][part] = code_vectors[i][part] * inputs + 16u * ((lane % 8u) ^ (lane / 8u) ^ part);
-            }
+            exponents_offset[i] = exponent_vectors[i] * (inputs / 32u);
         }
-        exponents_offset = exponent_vector * (inputs / 32u);
-        scale_lane = lane < 16u * WAVE_BLOCKS;
+        last_step = steps - 1u;
+        lane_of = lane;
         const uint32_t column = o % 8u, group_bytes = (o / 8u) * 1024u;
         if constexpr (BYTES) {
 #pragma unroll
             for (uint32_t v = 0; v < 8u; v++) {
-                vector_at[v] = group_bytes + 16u * (8u * column + (v ^ column ^ (o / 8u))) + 4u * g;
+                vector_at[v] = window + group_bytes + 16u * (8u * column + (v ^ column ^ (o / 8u))) + 4u * g;
             }
         } else {
 #pragma unroll
@@ -469,7 +589,7 @@ struct native_chain {
                 vector_at[part] = group_bytes + 16u * (8u * column + (piece ^ column ^ (o / 8u))) + 8u * (g / 2u);
             }
         }
-        vector_scale_at = B128 ? 4u * o : 4u * o + g;
+        vector_scale_at = (BYTES ? window : 0u) + 4u * SCALE_STEPS * o + (B128 ? 0u : g);
         operand_at = 16u * lane;
         scale_shift = 8u * (tile0 % 4u);
     }

@@ -517,9 +517,11 @@ ANEMONE_RECORD_HAS(expert_gate_up_quantize_arguments, 96);
 #define NATIVE_E2M1_COLUMN_BLOCKS 4u /* a block of the E2M1_GFX950 launches: one tile of the wide select (64 pairs) */
 #define NATIVE_E4M3_COLUMN_BLOCKS 8u /* of the E4M3_GFX950 launches: two tiles of one expert (128 pairs), read once */
 #define NATIVE_E2M1_STAGES 2u /* stages of columns in LDS: a K step in use, the next on its way */
-#define NATIVE_E4M3_STAGES 3u
-/* dynamic LDS: the stages of a K step of the block's columns (128 bytes of codes a column, 4 of scale codes) */
-#define NATIVE_WINDOW_BYTES(column_blocks, stages) ((stages) * ((column_blocks) * 2048u + (column_blocks) * 64u))
+#define NATIVE_E4M3_GATE_UP_STAGES 2u
+#define NATIVE_E4M3_DOWN_STAGES 3u
+/* dynamic LDS: the stages of a K step of the block's columns (128 bytes of codes a column), and two chunks of their scale
+ * words (four K steps of 4 bytes a column each) */
+#define NATIVE_WINDOW_BYTES(column_blocks, stages) ((stages) * (column_blocks) * 2048u + 2u * (column_blocks) * 256u)
 struct wide_expert_gate_up_arguments {
     uint64_t tiles_offset;            /* read: struct wide_expert_tile [tile_count] */
     uint64_t pairs_offset;            /* read: struct wide_pair [pair_count] */

@@ -129,6 +129,21 @@ def test_native_equals_the_reference_lay_out_byte_for_byte(amd, card, hidden, in
             assert np.all(b.reshape(-1)[pairs * per:] == 0xEE), name
 
 
+@pytest.mark.parametrize("hidden,inner,picks,rows,fmt", [
+    # the columns' scale words come four K steps at a time: chains that end inside a chunk, with one, at its first step
+    (640, 896, 2, 100, E2M1), (1152, 1024, 2, 100, E2M1),
+    (640, 896, 2, 100, E4M3), (1152, 1024, 2, 100, E4M3),
+    (640, 896, 2, 100, B128), (1152, 1024, 2, 100, B128),
+    # a lane holds the weights' scale words of a step: chains of more steps than the lanes that do
+    (8320, 128, 2, 70, E4M3), (128, 8320, 2, 70, E4M3),
+    (8320, 128, 2, 70, B128), (128, 8320, 2, 70, B128),
+    # one expert's pairs: every number of column blocks of a block of two tiles, each with its own share of a wavefront's loads
+    *[(512, 256, 1, rows, -fmt) for rows in (9, 30, 41, 64, 70, 96, 100, 128) for fmt in (E4M3, B128)],
+])
+def test_native_chunks_of_scale_words(amd, card, hidden, inner, picks, rows, fmt):
+    test_native_equals_the_reference_lay_out_byte_for_byte(amd, card, hidden, inner, 64, picks, rows, rows, fmt)
+
+
 @pytest.mark.parametrize("fmt", [E2M1, E4M3, B128])
 def test_native_layer_against_oracle(amd, card, fmt):
     """The layer in gfx950's lay-out against the CPU oracle reading the SAME re-laid-out bytes (its own reading of the

@@ -21,6 +21,8 @@ INSTANCES = {
     "E2M1 down (4 tiles, 1 scale word)": (3, 2, False, 3, 5),
     "E4M3 gate/up and down (2 tiles of two halves, 2 scale bytes; 128 columns)": (3, 3, True, 5, 6),
     "E4M3_BLOCK128 down (2 tiles of two halves, 1 scale)": (3, 3, True, 5, 5),
+    **{"one-byte gate/up, %d loads of columns" % loads: (2, 2, True, loads, 4) for loads in (2, 3, 4, 5)},
+    **{"one-byte down, %d loads of columns" % loads: (3, 3, True, loads, 4) for loads in (2, 3, 4, 5)},
     "four sets of weight registers (measured, not kept)": (4, 3, True, 5, 6),
     "six sets": (6, 3, True, 5, 6),
     "weights behind the columns at three stages": (4, 3, False, 5, 6),
