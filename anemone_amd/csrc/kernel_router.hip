@@ -145,21 +145,25 @@ ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_projection, router_projection_argument
  * three blocks a CU, which measured faster than three stages and two blocks): the next stage is asked for behind the
  * barrier that ends the stage before the current one. */
 typedef __attribute__((ext_vector_type(16))) float float16_t;
+typedef __attribute__((address_space(3))) void *lds_bytes;
 #define PROJECTION_STAGE_ROW_BYTES (PROJECTION_STAGE_INPUTS * 2u)
 #define PROJECTION_STAGE_ROWS (16u + PROJECTION_TILE_ROWS)
 #define PROJECTION_STAGE_BYTES (PROJECTION_STAGE_ROWS * PROJECTION_STAGE_ROW_BYTES)
 #define PROJECTION_STAGES 2u
 #define PROJECTION_WAVE_LOADS (PROJECTION_STAGE_BYTES / 1024u / (PROJECTION_TILE_THREADS / WAVE)) /* 5 */
 
-/* a group of 32 inputs: eight instructions, each one input further on the four chains it takes */
-__device__ static __forceinline__ void projection_tile_group(const uint4_t &w_now, const uint4_t &x_now, float16_t (&chain)[8])
+/* COUNT words of two bfloat16 each as float32. The float32 matrix instruction runs on the vector unit's own multipliers:
+ * nothing else of the unit runs beside it, and every change between the two costs cycles of its own. By a probe of this
+ * instruction (33.2 cycles alone, at one to three wavefronts a SIMD alike): 57 cycles with its two operands converted in
+ * front of it, 53 with those of a later instruction converted behind it, 42 where the operands of eight instructions are
+ * converted together and then multiplied. So conversions and matrix instructions go in blocks, fenced from each other. */
+template <uint32_t COUNT>
+__device__ static __forceinline__ void projection_convert(const uint32_t (&words)[COUNT], float (&values)[2u * COUNT])
 {
-    const uint32_t w_words[4] = {w_now.x, w_now.y, w_now.z, w_now.w}, x_words[4] = {x_now.x, x_now.y, x_now.z, x_now.w};
 #pragma unroll
-    for (uint32_t q = 0; q < 8u; q++) {
-        const float a = __uint_as_float(q % 2u == 0u ? w_words[q / 2u] << 16 : w_words[q / 2u] & 0xFFFF0000u);
-        const float b = __uint_as_float(q % 2u == 0u ? x_words[q / 2u] << 16 : x_words[q / 2u] & 0xFFFF0000u);
-        chain[q] = __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, chain[q], 0, 0, 0);
+    for (uint32_t k = 0; k < 2u * COUNT; k++) {
+        values[k] = __uint_as_float(k % 2u == 0u ? words[k / 2u] << 16 : words[k / 2u] & 0xFFFF0000u);
+        asm volatile("" : "+v"(values[k]));
     }
 }
 
@@ -229,14 +233,22 @@ extern "C" __global__ void __launch_bounds__(PROJECTION_TILE_THREADS, 3) /* thre
         const unsigned char *now = window + (stage % PROJECTION_STAGES) * PROJECTION_STAGE_BYTES;
         uint4_t w_now = *(const uint4_t *)(now + w_at[0]), x_now = *(const uint4_t *)(now + x_at[0]);
 #pragma unroll
-        for (uint32_t i = 0; i < 4u; i++) {
-            const uint4_t w_use = w_now, x_use = x_now;
+        for (uint32_t i = 0; i < 4u; i++) { /* a group of 32 inputs: eight instructions, each one input further on the four chains it takes */
+            const uint32_t w_words[4] = {w_now.x, w_now.y, w_now.z, w_now.w}, x_words[4] = {x_now.x, x_now.y, x_now.z, x_now.w};
+            float w_values[8], x_values[8];
+            projection_convert(w_words, w_values);
+            projection_convert(x_words, x_values);
+            __builtin_amdgcn_sched_barrier(0);
             if (i + 1u < 4u) { /* the next group's pieces are on their way behind this group's instructions */
                 w_now = *(const uint4_t *)(now + w_at[i + 1u]);
                 x_now = *(const uint4_t *)(now + x_at[i + 1u]);
-                __builtin_amdgcn_sched_barrier(0); /* asked for here, not behind the group's instructions */
             }
-            projection_tile_group(w_use, x_use, chain);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (uint32_t q = 0; q < 8u; q++) {
+                chain[q] = __builtin_amdgcn_mfma_f32_16x16x1f32(w_values[q], x_values[q], chain[q], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
     /* register v = 4 b + r of chain[q] is chain 8 b + q of expert 4 (lane / 16) + r and row lane % 16. The fold, as the
@@ -269,6 +281,123 @@ extern "C" __global__ void __launch_bounds__(PROJECTION_TILE_THREADS, 3) /* thre
     }
 }
 ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_projection_tiles, router_projection_arguments);
+
+/* The same scores for steps of 9 to 256 rows, whose tiles of 16 experts by 64 rows are fewer than the card's CUs: a block
+ * is one 16 x 16 tile, and its four wavefronts take eight chains each, so that a CU's four vector units work on every
+ * score. Instruction t of a group of 32 inputs takes the chains 8 wave + 2 b + t of the blocks b = 0 .. 3: lane (b, n)
+ * needs the two inputs 32 i + 8 wave + 2 b + {0, 1} of expert n and of row n, one word each. A stage is the 16 + 16 rows'
+ * 128 inputs (8 KB, laid out and swizzled as above); PROJECTION_SPLIT_STAGES of them are in LDS or on their way (three blocks
+ * a CU; five to sixteen measured within 10 %), and a stage is read behind the instructions of the one before it. The
+ * wavefronts' sums meet in LDS at the end, each wavefront folding a quarter of the scores. What is left is a wavefront's 256
+ * instructions of 4096 inputs and their conversions (10,900 cycles, 5 us), the first loads' way from memory and the
+ * launch. By router_projection / so, us, 256 experts of 4096 inputs: 203 rows 38 / 13.5, 100 rows 25 / 12.7, 64 rows 14.3 /
+ * 12, 37 rows 15 / 13.2, 16 rows 13 / 12.6; up to eight rows router_projection takes a row a block (7 to 11).
+ * grid (E / 16, ceil(rows / 16)), block 256. */
+#define PROJECTION_SPLIT_STAGE_BYTES (32u * PROJECTION_STAGE_ROW_BYTES)
+#define PROJECTION_SPLIT_STAGES 6u
+extern "C" __global__ void __launch_bounds__(PROJECTION_TILE_THREADS)
+    router_projection_split(struct router_projection_arguments arguments, unsigned char *arena)
+{
+    __shared__ __attribute__((aligned(1024))) unsigned char window[PROJECTION_SPLIT_STAGES * PROJECTION_SPLIT_STAGE_BYTES];
+    const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), block = lane / 16u, index = lane % 16u;
+    const uint32_t H = arguments.hidden, stages = H / PROJECTION_STAGE_INPUTS;
+    const uint32_t first_expert = blockIdx.x * 16u, first_row = blockIdx.y * 16u;
+    const uint32_t window_address = (uint32_t)(uintptr_t)(lds_bytes)window;
+    /* this wavefront brings four experts' rows and four rows of a stage (a row past the last repeats the last) */
+    const uint32_t line = 4u * wave + lane / 16u, row = first_row + line < arguments.row_count ? first_row + line : arguments.row_count - 1u;
+    const uint32_t piece_bytes = 16u * ((lane % 16u) ^ line);
+    const unsigned char *w_source = arena + arguments.weights_offset + (uint64_t)(first_expert + line) * H * 2u + piece_bytes;
+    const unsigned char *x_source = arena + arguments.rows_offset + (uint64_t)row * H * 2u + piece_bytes;
+    auto ask = [&](uint32_t stage, uint32_t place) {
+        const uint32_t base = window_address + place * PROJECTION_SPLIT_STAGE_BYTES + wave * 1024u;
+        projection_load_to_lds(w_source + (uint64_t)stage * PROJECTION_STAGE_ROW_BYTES, base);
+        projection_load_to_lds(x_source + (uint64_t)stage * PROJECTION_STAGE_ROW_BYTES, base + 16u * PROJECTION_STAGE_ROW_BYTES);
+    };
+    /* past the last stage the last is asked for again, into a place that nobody reads any more: every wait counts the same */
+    for (uint32_t stage = 0; stage < PROJECTION_SPLIT_STAGES; stage++) {
+        ask(stage < stages ? stage : stages - 1u, stage);
+    }
+    float16_t chain[2];
+#pragma unroll
+    for (uint32_t v = 0; v < 16u; v++) {
+        chain[0][v] = chain[1][v] = 0.0f;
+    }
+    uint32_t w_words[4], x_words[4];
+    auto read = [&](uint32_t place) {
+        const unsigned char *now = window + place * PROJECTION_SPLIT_STAGE_BYTES + index * PROJECTION_STAGE_ROW_BYTES + 4u * block;
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; i++) {
+            const uint32_t slot = 16u * ((4u * i + wave) ^ index);
+            w_words[i] = *(const uint32_t *)(now + slot);
+            x_words[i] = *(const uint32_t *)(now + 16u * PROJECTION_STAGE_ROW_BYTES + slot);
+        }
+    };
+    /* this wavefront's loads of the oldest stage have landed, then every wavefront's */
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2u * (PROJECTION_SPLIT_STAGES - 1u)) : "memory");
+    __syncthreads();
+    read(0u);
+    uint32_t place = 0;
+    for (uint32_t stage = 0; stage < stages; stage++) {
+        float w_values[8], x_values[8];
+        projection_convert(w_words, w_values);
+        projection_convert(x_words, x_values);
+        /* the next stage is read behind this one's instructions; every wavefront has read this one, whose place the one to
+         * ask for takes */
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2u * (PROJECTION_SPLIT_STAGES - 2u)) : "memory");
+        __syncthreads();
+        const uint32_t ahead = stage + PROJECTION_SPLIT_STAGES;
+        ask(ahead < stages ? ahead : stages - 1u, place);
+        place = place + 1u < PROJECTION_SPLIT_STAGES ? place + 1u : 0u;
+        read(place);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; k++) {
+            chain[k % 2u] = __builtin_amdgcn_mfma_f32_16x16x1f32(w_values[k], x_values[k], chain[k % 2u], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    /* register v = 4 b + r of chain[t] is chain 8 wave + 2 b + t of expert 4 (lane / 16) + r and row lane % 16. Every
+     * wavefront leaves its eight chains of the experts r, [r][b][t] a lane; wavefront r then folds those of expert 4 (lane / 16) + r
+     * as the definition orders it: + 0 first, then the distances 16 and 8 (wavefronts), 4 and 2 (blocks), 1 (instructions) */
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* the last stage's repeats */
+    __syncthreads();
+    float *exchange = (float *)window; /* [wavefront][r][lane][8] */
+#pragma unroll
+    for (uint32_t r = 0; r < 4u; r++) {
+        float *to = exchange + ((wave * 4u + r) * WAVE + lane) * 8u;
+#pragma unroll
+        for (uint32_t b = 0; b < 4u; b += 2u) {
+            *(float4_t *)(to + 2u * b) = (float4_t){__fadd_rn(0.0f, chain[0][4u * b + r]), __fadd_rn(0.0f, chain[1][4u * b + r]),
+                                                   __fadd_rn(0.0f, chain[0][4u * b + 4u + r]), __fadd_rn(0.0f, chain[1][4u * b + 4u + r])};
+        }
+    }
+    __syncthreads();
+    float sums[8];
+#pragma unroll
+    for (uint32_t k = 0; k < 8u; k += 4u) {
+        float4_t part[4];
+#pragma unroll
+        for (uint32_t from = 0; from < 4u; from++) {
+            part[from] = *(const float4_t *)(exchange + ((from * 4u + wave) * WAVE + lane) * 8u + k);
+        }
+#pragma unroll
+        for (uint32_t v = 0; v < 4u; v++) {
+            sums[k + v] = __fadd_rn(__fadd_rn(part[0][v], part[2][v]), __fadd_rn(part[1][v], part[3][v]));
+        }
+    }
+#pragma unroll
+    for (uint32_t distance = 4u; distance != 0u; distance >>= 1u) {
+#pragma unroll
+        for (uint32_t k = 0; k < distance; k++) {
+            sums[k] = __fadd_rn(sums[k], sums[k + distance]);
+        }
+    }
+    if (first_row + index < arguments.row_count) {
+        ((float *)(arena + arguments.output_offset))[(uint64_t)(first_row + index) * arguments.expert_count + first_expert + 4u * block + wave] =
+            __fadd_rn(0.0f, sums[0]);
+    }
+}
+ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_projection_split, router_projection_arguments);
 
 extern "C" __global__ void __launch_bounds__(SELECT_THREADS)
     router_select_entry(struct router_select_arguments arguments, unsigned char *arena)

@@ -9,6 +9,8 @@
  *   projection    router_projection     (ceil(E / 8), ceil(rows / 4), 1)   128   eight experts and four rows a block
  *                 router_projection_tiles (E / 16, ceil(rows / 64), 1)     256   257 rows and more of a width in whole 128, E in whole 16:
  *                                                                                16 experts by 64 rows a block
+ *                 router_projection_split (E / 16, ceil(rows / 16), 1)     256   9 to 256 rows of such a width and E: 16 experts by 16 rows a
+ *                                                                                block (beside its kernel: both sides' times)
  *   select        router_select_entry   (1, 1, 1)                   512   a wavefront a row
  *   wide select   router_wide_select    (ceil(rows / 8), 1, 1)      512   a wavefront a row
  *   wide count    router_wide_count     (ceil(rows / 384), 1, 1)    512   a thread an expert
@@ -67,13 +69,18 @@ result_status router_kernels_prepare(const struct backend_operations *backend, s
     if (projected != STATUS_OK) {
         return projected;
     }
-    uint32_t tiles = BACKEND_NO_KERNEL;
+    uint32_t tiles = BACKEND_NO_KERNEL, split = BACKEND_NO_KERNEL;
     if (backend->kernel_prepare(card, KERNEL_FILE_ROUTER, KERNEL_ROUTER_PROJECTION_TILES, sizeof(struct router_projection_arguments),
                                 &tiles) != STATUS_OK) {
         tiles = BACKEND_NO_KERNEL; /* every row count then takes router_projection */
     }
+    if (backend->kernel_prepare(card, KERNEL_FILE_ROUTER, KERNEL_ROUTER_PROJECTION_SPLIT, sizeof(struct router_projection_arguments),
+                                &split) != STATUS_OK) {
+        split = BACKEND_NO_KERNEL; /* so do then 9 to 256 rows */
+    }
     memcpy(kernels_out, handles, sizeof handles);
     kernels_out->projection_tiles = tiles;
+    kernels_out->projection_split = split;
     return STATUS_OK;
 }
 
@@ -256,6 +263,14 @@ result_status router_projection_prepare(const struct router_projection_descripti
         description->hidden % PROJECTION_STAGE_INPUTS == 0) { /* many rows: the chains on the matrix unit, 16 experts by 64 rows a block */
         launch_fill(launch_out, kernels->projection_tiles, description->expert_count / 16u,
                     (description->row_count + PROJECTION_TILE_ROWS - 1u) / PROJECTION_TILE_ROWS, 1, PROJECTION_TILE_THREADS, 0, &record,
+                    sizeof record);
+        return STATUS_OK;
+    }
+    if (kernels->projection_split != BACKEND_NO_KERNEL && description->row_count >= PROJECTION_SPLIT_LEAST_ROWS &&
+        description->row_count < PROJECTION_TILE_LEAST_ROWS && description->expert_count % 16u == 0 &&
+        description->hidden % PROJECTION_STAGE_INPUTS == 0) { /* 16 experts by 16 rows a block, their chains over its wavefronts */
+        launch_fill(launch_out, kernels->projection_split, description->expert_count / 16u,
+                    (description->row_count + PROJECTION_SPLIT_ROWS - 1u) / PROJECTION_SPLIT_ROWS, 1, PROJECTION_TILE_THREADS, 0, &record,
                     sizeof record);
         return STATUS_OK;
     }

@@ -107,7 +107,10 @@ ANEMONE_RECORD_HAS(wide_expert_tile, 32);
 #define KERNEL_ROUTER_PROJECTION_TILES "router_projection_tiles" /* the same scores on the matrix unit: steps of many rows */
 #define PROJECTION_TILE_THREADS 256u
 #define PROJECTION_TILE_ROWS 64u   /* rows of a block of router_projection_tiles: 16 a wavefront */
-#define PROJECTION_TILE_LEAST_ROWS 257u /* fewer rows take router_projection: its blocks are smaller and more */
+#define PROJECTION_TILE_LEAST_ROWS 257u /* fewer rows take router_projection_split or router_projection: their blocks are smaller and more */
+#define KERNEL_ROUTER_PROJECTION_SPLIT "router_projection_split" /* and with a tile's chains over a block's wavefronts: few rows */
+#define PROJECTION_SPLIT_ROWS 16u       /* rows of a block of router_projection_split */
+#define PROJECTION_SPLIT_LEAST_ROWS 9u  /* up to eight rows router_projection takes a row a block, in blocks of eight experts */
 #define PROJECTION_STAGE_INPUTS 128u     /* inputs of a stage of router_projection_tiles: the width is a whole number of them */
 #define KERNEL_ROUTER_SELECT "router_select_entry"
 #define KERNEL_ROUTER_WIDE_SELECT "router_wide_select"

@@ -306,6 +306,12 @@ def test_router_projection_prepare_geometry(fake):
     assert (status, name, grid) == (0, "router_projection", [8, 75, 1])
     status, name, grid, block = prepared(300, 512, 72)  # no whole number of 16 experts
     assert (status, name, grid) == (0, "router_projection", [9, 75, 1])
+    for rows in (9, 16, 17, 203, 256):  # few rows: 16 experts by 16 rows a block
+        assert prepared(rows, 4096, 256) == (0, "router_projection_split", [16, (rows + 15) // 16, 1], 256)
+    assert prepared(257, 4096, 256)[1] == "router_projection_tiles"
+    assert prepared(100, 160, 64)[1:3] == ("router_projection", [8, 25, 1]) and prepared(100, 512, 72)[1:3] == ("router_projection", [9, 25, 1])
+    kernels.projection_split = amd.BACKEND_NO_KERNEL  # a backend without it
+    assert prepared(100, 512, 64)[1:3] == ("router_projection", [8, 25, 1])
     status, name, grid, block = prepared(8, 4096, 256)  # a thin step: a row a block
     assert (status, name, grid) == (0, "router_projection", [32, 8, 1])
     assert prepared(300, 48, 64)[0] == 1 and prepared(0, 512, 64)[0] == 1  # a width that is no multiple of 32; no row

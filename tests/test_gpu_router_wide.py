@@ -182,6 +182,34 @@ def test_projection_of_many_rows_bit_exact(amd, card, experts_n, rows, hidden, s
     assert differing.size == 0
 
 
+@pytest.mark.parametrize("experts_n,rows,hidden,scale", [
+    (64, 9, 128, 1.0),       # one stage: fewer than the kernel keeps on their way
+    (64, 16, 640, 1e-18), (128, 17, 768, 1.0), (256, 33, 896, 1.0),  # as many stages as places, and around it; a tile's last rows
+    (384, 63, 1024, 3e18), (256, 203, 4096, 1.0), (64, 256, 5120, 1.0),
+])
+def test_projection_of_few_rows_bit_exact(amd, card, experts_n, rows, hidden, scale):
+    """router_projection_split (9 to 256 rows: a tile's chains over a block's wavefronts) against the oracle's chains, every
+    bit, nothing written behind the scores."""
+    say("projection, few rows", experts_n, rows, hidden, scale)
+    layer, _ = small_layer(amd, card, experts_n, 2, rows, hidden=hidden)
+    router = to_bf16(normals(51, experts_n * hidden) * scale).reshape(experts_n, hidden)
+    x = to_bf16(normals(52, rows * hidden) * scale).reshape(rows, hidden)
+    card.upload(layer.router_offset, router)
+    layer.set_rows(x, rows)
+    launch = layer.projection_launch()
+    assert list(launch[0].block)[0] == 256 and list(launch[0].grid) == [experts_n // 16, (rows + 15) // 16, 1]
+    card.upload(layer.affinities_offset, np.full(rows * experts_n * 4, 0xEE, dtype=np.uint8))
+    card.upload(layer.scores_offset, np.full(rows * experts_n * 4, 0xEE, dtype=np.uint8))
+    card.run(launch)
+    got = card.download(layer.scores_offset, rows * experts_n * 4, np.float32).reshape(rows, experts_n)
+    want = np.zeros((rows, experts_n), dtype=np.float32)
+    orc.orc_router_projection(ptr(x, u16p), ptr(router, u16p), rows, hidden, experts_n, ptr(want, f32p))
+    differing = np.flatnonzero(got.view(np.uint32) != want.view(np.uint32))
+    say("  %d of %d scores differ" % (differing.size, got.size))
+    assert differing.size == 0
+    assert np.all(card.download(layer.affinities_offset, rows * experts_n * 4, np.uint8) == 0xEE)
+
+
 def test_fp4_layer_through_the_wide_job_table(amd, card):
     """40 rows (37 live) routed by the wide select, then the FP4 experts over its job table, against the oracle."""
     say("fp4 layer, wide")
