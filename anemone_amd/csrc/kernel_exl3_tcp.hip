@@ -88,7 +88,7 @@ extern "C" __global__ void __launch_bounds__(TCP_SORT_THREADS) exl3_tcp_place(st
     __shared__ __attribute__((aligned(16))) uint32_t block_experts[ROUTER_SORT_ROWS * ROUTER_MOST_PICKS];
     __shared__ uint32_t block_places[ROUTER_SORT_ROWS * ROUTER_MOST_PICKS];
     __shared__ uint32_t totals[ROUTER_MOST_EXPERTS], starts[ROUTER_MOST_EXPERTS], before[ROUTER_MOST_EXPERTS];
-    __shared__ uint32_t chunk_starts[ROUTER_MOST_EXPERTS + 1u], scratch[ROUTER_MOST_EXPERTS];
+    __shared__ uint32_t chunk_starts[ROUTER_MOST_EXPERTS + 1u], scratch[SORT_MOST_WAVES];
     __shared__ uint32_t first_places[ROUTER_MOST_EXPERTS], cursors[SORT_MOST_WAVES * ROUTER_MOST_EXPERTS];
     const tcp_shape shape = tcp_shape_of(record);
     const uint32_t experts = shape.experts;
@@ -99,6 +99,7 @@ extern "C" __global__ void __launch_bounds__(TCP_SORT_THREADS) exl3_tcp_place(st
     const uint32_t *counts = (const uint32_t *)(workspace + shape.layout.counts);
     for (uint32_t expert = threadIdx.x; expert < experts; expert += blockDim.x) {
         uint32_t total = 0, lower = 0;
+#pragma unroll 8
         for (uint32_t block = 0; block < blocks; block++) {
             const uint32_t count = counts[(uint64_t)block * experts + expert];
             total += count;

@@ -547,7 +547,7 @@ extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
     __shared__ __attribute__((aligned(16))) uint32_t block_experts[ROUTER_SORT_ROWS * ROUTER_MOST_PICKS];
     __shared__ uint32_t place_of[ROUTER_SORT_ROWS * ROUTER_MOST_PICKS];
     __shared__ uint32_t totals[ROUTER_MOST_EXPERTS], starts[ROUTER_MOST_EXPERTS], before[ROUTER_MOST_EXPERTS];
-    __shared__ uint32_t tile_starts[ROUTER_MOST_EXPERTS + 1u], scratch[ROUTER_MOST_EXPERTS];
+    __shared__ uint32_t tile_starts[ROUTER_MOST_EXPERTS + 1u], scratch[SORT_MOST_WAVES];
     __shared__ uint32_t first_places[ROUTER_MOST_EXPERTS], cursors[SORT_MOST_WAVES * ROUTER_MOST_EXPERTS];
     const uint32_t experts = arguments.expert_count;
     const uint32_t live_rows = wide_live_rows(arguments, arena);
@@ -559,6 +559,7 @@ extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
     const uint32_t *counts = (const uint32_t *)(arena + arguments.counts_offset);
     for (uint32_t expert = threadIdx.x; expert < experts; expert += blockDim.x) {
         uint32_t total = 0, lower = 0;
+#pragma unroll 8
         for (uint32_t block = 0; block < live_blocks; block++) {
             const uint32_t count = counts[(uint64_t)block * experts + expert];
             total += count;
@@ -575,29 +576,46 @@ extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
 }
 ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_wide_place, router_wide_arguments);
 
-/* The job table of the runs, a thread a job; job_starts holds every expert's jobs. The whole block calls it after a
- * barrier that follows the writing of the runs and the sorted pairs. */
-__device__ static __forceinline__ void wide_jobs_block(const struct router_wide_arguments &arguments, unsigned char *arena,
-                                                       uint32_t *job_starts, uint32_t *scratch)
+/* Job `job` of an expert whose jobs begin at job_start and whose `total` pairs begin at first_pair of the sorted pairs:
+ * pair(place, index, weight) reads one. The eight reads go together (those past the job's pairs repeat its first). */
+template <typename PAIR>
+__device__ static __forceinline__ void wide_job(uint32_t job, uint32_t job_start, uint32_t expert, uint32_t first_pair, uint32_t total,
+                                                const uint64_t *offsets, struct expert_job_record &value, PAIR pair)
 {
-    const uint32_t experts = arguments.expert_count, picks = arguments.pick_count;
+    const uint32_t taken = (job - job_start) * LINEAR_MAXIMUM_ROWS, left = total - taken;
+    value.gate_offset = offsets[0];
+    value.up_offset = offsets[1];
+    value.down_offset = offsets[2];
+    value.row_count = left < LINEAR_MAXIMUM_ROWS ? left : LINEAR_MAXIMUM_ROWS;
+    value.expert = expert;
+#pragma unroll
+    for (uint32_t column = 0; column < LINEAR_MAXIMUM_ROWS; column++) {
+        uint32_t index;
+        float weight;
+        pair(first_pair + taken + (column < value.row_count ? column : 0u), index, weight);
+        value.pair_index[column] = column < value.row_count ? index : 0u;
+        value.route_weight[column] = column < value.row_count ? weight : 0.0f;
+    }
+}
+
+/* grid (1): the job table of the runs, a thread a job */
+extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
+    router_wide_jobs(struct router_wide_arguments arguments, unsigned char *arena)
+{
+    __shared__ uint32_t job_starts[ROUTER_MOST_EXPERTS + 1u], scratch[SORT_MOST_WAVES];
+    const uint32_t experts = arguments.expert_count;
     const struct wide_run *runs = (const struct wide_run *)(arena + arguments.runs_offset);
-    const uint32_t used_jobs = block_exclusive_scan(job_starts, experts, scratch);
-    if (threadIdx.x == 0u) {
-        job_starts[experts] = used_jobs;
+    if (threadIdx.x < experts) {
+        job_starts[threadIdx.x] = (runs[threadIdx.x].pair_count + LINEAR_MAXIMUM_ROWS - 1u) / LINEAR_MAXIMUM_ROWS;
     }
     __syncthreads();
-    const uint32_t all_jobs = ROUTER_WIDE_JOBS_OF(arguments.row_count, picks, experts);
+    const uint32_t used_jobs = block_exclusive_scan(job_starts, experts, scratch);
+    const uint32_t all_jobs = ROUTER_WIDE_JOBS_OF(arguments.row_count, arguments.pick_count, experts);
     const struct wide_pair *sorted = (const struct wide_pair *)(arena + arguments.pairs_offset);
     const uint64_t *offsets = (const uint64_t *)(arena + arguments.expert_offsets_offset);
     struct expert_job_record *jobs = (struct expert_job_record *)(arena + arguments.jobs_offset);
     for (uint32_t job = threadIdx.x; job < all_jobs; job += blockDim.x) {
-        struct expert_job_record value;
-        uint32_t *words = (uint32_t *)&value;
-#pragma unroll
-        for (uint32_t word = 0; word < JOB_WORDS; word++) {
-            words[word] = 0u;
-        }
+        struct expert_job_record value = {};
         if (job < used_jobs) {
             uint32_t low = 0, high = experts;
             while (high - low > 1u) {
@@ -609,63 +627,127 @@ __device__ static __forceinline__ void wide_jobs_block(const struct router_wide_
                 }
             }
             const struct wide_run run = runs[low];
-            const uint32_t taken = (job - job_starts[low]) * LINEAR_MAXIMUM_ROWS, left = run.pair_count - taken;
-            value.gate_offset = offsets[(uint64_t)low * MODEL_EXPERT_MATRICES + 0u];
-            value.up_offset = offsets[(uint64_t)low * MODEL_EXPERT_MATRICES + 1u];
-            value.down_offset = offsets[(uint64_t)low * MODEL_EXPERT_MATRICES + 2u];
-            value.row_count = left < LINEAR_MAXIMUM_ROWS ? left : LINEAR_MAXIMUM_ROWS;
-            value.expert = low;
-            for (uint32_t column = 0; column < value.row_count; column++) {
-                const struct wide_pair pair = sorted[run.first_pair + taken + column];
-                value.pair_index[column] = pair.pair_index;
-                value.route_weight[column] = pair.route_weight;
-            }
+            wide_job(job, job_starts[low], low, run.first_pair, run.pair_count, offsets + (uint64_t)low * MODEL_EXPERT_MATRICES, value,
+                     [&](uint32_t place, uint32_t &index, float &weight) {
+                         const struct wide_pair pair = sorted[place];
+                         index = pair.pair_index;
+                         weight = pair.route_weight;
+                     });
         }
         jobs[job] = value;
     }
-}
-
-/* grid (1): the job table of the runs, a thread a job */
-extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
-    router_wide_jobs(struct router_wide_arguments arguments, unsigned char *arena)
-{
-    __shared__ uint32_t job_starts[ROUTER_MOST_EXPERTS + 1u], scratch[ROUTER_MOST_EXPERTS];
-    const struct wide_run *runs = (const struct wide_run *)(arena + arguments.runs_offset);
-    for (uint32_t expert = threadIdx.x; expert < arguments.expert_count; expert += blockDim.x) {
-        job_starts[expert] = (runs[expert].pair_count + LINEAR_MAXIMUM_ROWS - 1u) / LINEAR_MAXIMUM_ROWS;
-    }
-    __syncthreads();
-    wide_jobs_block(arguments, arena, job_starts, scratch);
 }
 ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_wide_jobs, router_wide_arguments);
 
 /* grid (1): the count, the place and the jobs of at most ROUTER_SORT_ROWS rows in one block (the reference's
  * router_wide_small, source/kernel_router.cu there): the same pairs, runs, tiles and jobs; the counts scratch is
- * not written */
+ * not written.
+ *
+ * One block's time is its round trips: everything it reads from memory is asked for at its start (the picks of all the rows
+ * there is room for, beside the number of the live ones), a thread owns an expert and takes the starts of its pairs, tiles
+ * and jobs from one scan of the three side by side, the jobs find their expert and their pairs in LDS: five barriers, two
+ * waits for memory. 64 rows of 256 experts, 8 picks: 17.4 -> 6.0 us (three scans of nine barriers, searches, the runs and
+ * the sorted pairs read back from memory, a job's pairs by way of scratch memory). */
 extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
     router_wide_small(struct router_wide_arguments arguments, unsigned char *arena)
 {
-    __shared__ __attribute__((aligned(16))) uint32_t block_experts[ROUTER_SORT_ROWS * ROUTER_MOST_PICKS];
-    __shared__ uint32_t place_of[ROUTER_SORT_ROWS * ROUTER_MOST_PICKS];
-    __shared__ uint32_t totals[ROUTER_MOST_EXPERTS], starts[ROUTER_MOST_EXPERTS], before[ROUTER_MOST_EXPERTS];
-    __shared__ uint32_t tile_starts[ROUTER_MOST_EXPERTS + 1u], scratch[ROUTER_MOST_EXPERTS], job_starts[ROUTER_MOST_EXPERTS + 1u];
-    __shared__ uint32_t first_places[ROUTER_MOST_EXPERTS], cursors[SORT_MOST_WAVES * ROUTER_MOST_EXPERTS];
-    const uint32_t experts = arguments.expert_count;
+    constexpr uint32_t MOST_PAIRS = ROUTER_SORT_ROWS * ROUTER_MOST_PICKS;
+    static_assert(WIDE_SORT_THREADS == SORT_MOST_WAVES * SORT_WAVE && WIDE_SORT_THREADS >= ROUTER_MOST_EXPERTS, "a thread an expert");
+    /* a scan's word: pairs in 12 bits, tiles and jobs in 10 each */
+    static_assert(MOST_PAIRS < 4096u && MOST_PAIRS / WIDE_TILE_PAIRS + ROUTER_MOST_EXPERTS < 1024u &&
+                      MOST_PAIRS / LINEAR_MAXIMUM_ROWS + ROUTER_MOST_EXPERTS < 1024u, "the three sums fit their bits");
+    __shared__ uint32_t block_experts[MOST_PAIRS], sorted_index[MOST_PAIRS], cursors[SORT_MOST_WAVES * ROUTER_MOST_EXPERTS];
+    __shared__ float weights[MOST_PAIRS];
+    __shared__ uint64_t expert_offsets[ROUTER_MOST_EXPERTS * MODEL_EXPERT_MATRICES];
+    __shared__ uint32_t starts[ROUTER_MOST_EXPERTS], totals[ROUTER_MOST_EXPERTS], job_starts[ROUTER_MOST_EXPERTS], scratch[SORT_MOST_WAVES];
+    __shared__ uint16_t job_expert[1024];
+    const uint32_t experts = arguments.expert_count, picks = arguments.pick_count, room = arguments.row_count * picks;
+    const uint32_t wave = threadIdx.x / SORT_WAVE, expert = threadIdx.x;
+    const struct router_pick *all_picks = (const struct router_pick *)(arena + arguments.picks_offset);
+    const uint64_t *offsets = (const uint64_t *)(arena + arguments.expert_offsets_offset) + (uint64_t)expert * MODEL_EXPERT_MATRICES;
     const uint32_t live_rows = wide_live_rows(arguments, arena);
-    const uint32_t pairs = wide_block_picks(arguments, arena, 0u, live_rows, block_experts);
+    struct router_pick mine[MOST_PAIRS / WIDE_SORT_THREADS];
+    uint64_t own_offsets[MODEL_EXPERT_MATRICES] = {0, 0, 0};
+#pragma unroll
+    for (uint32_t k = 0; k < MOST_PAIRS / WIDE_SORT_THREADS; k++) {
+        const uint32_t index = k * WIDE_SORT_THREADS + threadIdx.x;
+        if (index < room) {
+            mine[k] = all_picks[index];
+        }
+    }
+    if (expert < experts) {
+#pragma unroll
+        for (uint32_t matrix = 0; matrix < MODEL_EXPERT_MATRICES; matrix++) {
+            own_offsets[matrix] = offsets[matrix];
+        }
+    }
+    for (uint32_t at = threadIdx.x; at < SORT_MOST_WAVES * experts; at += WIDE_SORT_THREADS) {
+        cursors[at] = 0u;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < MOST_PAIRS / WIDE_SORT_THREADS; k++) {
+        const uint32_t index = k * WIDE_SORT_THREADS + threadIdx.x;
+        if (index < room) { /* past the live rows: whatever the array holds, read no further */
+            block_experts[index] = mine[k].expert;
+            weights[index] = mine[k].route_weight;
+        }
+    }
+    const uint32_t pairs = live_rows * picks;
+    uint32_t begin, end;
+    sort_share(pairs, wave, begin, end);
     __syncthreads();
-    sort_count_picks(block_experts, pairs, experts, totals);
-    for (uint32_t expert = threadIdx.x; expert < experts; expert += blockDim.x) {
-        const uint32_t count = totals[expert];
-        starts[expert] = count;
-        before[expert] = 0u;
-        tile_starts[expert] = (count + WIDE_TILE_PAIRS - 1u) / WIDE_TILE_PAIRS;
-        job_starts[expert] = (count + LINEAR_MAXIMUM_ROWS - 1u) / LINEAR_MAXIMUM_ROWS;
+    sort_count_share(block_experts, begin, end, cursors + wave * experts);
+    __syncthreads();
+    uint32_t counts[SORT_MOST_WAVES], total = 0, sums;
+    if (expert < experts) {
+        total = sort_counts_of(cursors, experts, expert, counts);
+    }
+    const uint32_t own_tiles = (total + WIDE_TILE_PAIRS - 1u) / WIDE_TILE_PAIRS, own_jobs = (total + LINEAR_MAXIMUM_ROWS - 1u) / LINEAR_MAXIMUM_ROWS;
+    const uint32_t before = block_sum_before(total | own_tiles << 12 | own_jobs << 22, scratch, sums);
+    const uint32_t start = before & 4095u, first_tile = before >> 12 & 1023u, first_job = before >> 22;
+    const uint32_t used_tiles = sums >> 12 & 1023u, used_jobs = sums >> 22;
+    struct wide_expert_tile *tiles = (struct wide_expert_tile *)(arena + arguments.tiles_offset);
+    if (expert < experts) {
+        sort_cursors_of(cursors, experts, expert, counts, start);
+        starts[expert] = start;
+        totals[expert] = total;
+        job_starts[expert] = first_job;
+#pragma unroll
+        for (uint32_t matrix = 0; matrix < MODEL_EXPERT_MATRICES; matrix++) {
+            expert_offsets[expert * MODEL_EXPERT_MATRICES + matrix] = own_offsets[matrix];
+        }
+        for (uint32_t k = 0; k < own_jobs; k++) {
+            job_expert[first_job + k] = (uint16_t)expert;
+        }
+        ((struct wide_run *)(arena + arguments.runs_offset))[expert] = (struct wide_run){start, total};
+        for (uint32_t k = 0; k < own_tiles; k++) {
+            const uint32_t taken = k * WIDE_TILE_PAIRS, left = total - taken;
+            tiles[first_tile + k] = (struct wide_expert_tile){own_offsets[0], own_offsets[1], own_offsets[2], start + taken,
+                                                              left < WIDE_TILE_PAIRS ? left : WIDE_TILE_PAIRS};
+        }
+    }
+    for (uint32_t tile = used_tiles + threadIdx.x; tile < ROUTER_WIDE_TILES_OF(arguments.row_count, picks, experts); tile += WIDE_SORT_THREADS) {
+        tiles[tile] = (struct wide_expert_tile){0, 0, 0, 0, 0};
     }
     __syncthreads();
-    wide_place_block(arguments, arena, 0u, block_experts, place_of, pairs, totals, starts, before, tile_starts, scratch, first_places, cursors);
-    __threadfence_block();
-    __syncthreads(); /* the runs and the sorted pairs, written by this block, are read by its jobs */
-    wide_jobs_block(arguments, arena, job_starts, scratch);
+    struct wide_pair *sorted = (struct wide_pair *)(arena + arguments.pairs_offset);
+    sort_place_share(block_experts, begin, end, experts, cursors + wave * experts, [&](uint32_t index, uint32_t place) {
+        sorted_index[place] = index;
+        sorted[place] = (struct wide_pair){index, weights[index]};
+    });
+    __syncthreads();
+    struct expert_job_record *jobs = (struct expert_job_record *)(arena + arguments.jobs_offset);
+    for (uint32_t job = threadIdx.x; job < ROUTER_WIDE_JOBS_OF(arguments.row_count, picks, experts); job += WIDE_SORT_THREADS) {
+        struct expert_job_record value = {};
+        if (job < used_jobs) {
+            const uint32_t owner = job_expert[job];
+            wide_job(job, job_starts[owner], owner, starts[owner], totals[owner], expert_offsets + owner * MODEL_EXPERT_MATRICES, value,
+                     [&](uint32_t place, uint32_t &index, float &weight) {
+                         index = sorted_index[place];
+                         weight = weights[index];
+                     });
+        }
+        jobs[job] = value;
+    }
 }
 ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_wide_small, router_wide_arguments);

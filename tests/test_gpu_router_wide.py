@@ -127,8 +127,20 @@ def test_wide_select_skewed_and_hand_case(amd, card):
     assert counts.max() > 400
 
 
+@pytest.mark.parametrize("experts_n,picks,rows,live,busy", [
+    (512, 8, 384, 384, 0),  # the most experts and pairs: the scan's three sums at their widest
+    (512, 8, 384, 383, 8),  # eight experts take every row: runs of six tiles and 48 jobs, 504 experts without a pair
+    (64, 1, 384, 65, 1),    # one run, its second tile of one pair; most of the room not live
+    (512, 8, 9, 9, 0), (64, 8, 64, 64, 8),
+])
+def test_wide_small_at_its_limits(amd, card, experts_n, picks, rows, live, busy):
+    bias = np.zeros(experts_n, dtype=np.float32)
+    bias[7:7 + 5 * busy:5] = 100.0
+    test_wide_small_equals_the_four_launches(amd, card, experts_n, picks, rows, live, bias)
+
+
 @pytest.mark.parametrize("experts_n,picks,rows,live", [(64, 4, 40, 37), (256, 8, 384, 384), (384, 6, 130, 130), (128, 3, 1, 1)])
-def test_wide_small_equals_the_four_launches(amd, card, experts_n, picks, rows, live):
+def test_wide_small_equals_the_four_launches(amd, card, experts_n, picks, rows, live, bias=None):
     """router_wide_small (count, place and jobs of at most 384 rows in one block) writes the pairs, runs, tiles and
     jobs of the four launches, byte for byte (include/anemone/router.h:117-119 of the reference), and those are held to
     the oracle by the tests above."""
@@ -136,7 +148,7 @@ def test_wide_small_equals_the_four_launches(amd, card, experts_n, picks, rows, 
     layer, _ = small_layer(amd, card, experts_n, picks, rows)
     scores = (normals(123, rows * experts_n) * 1.5).astype(np.float32).reshape(rows, experts_n)
     card.upload(layer.scores_offset, scores)
-    card.upload(layer.bias_offset, np.zeros(experts_n, dtype=np.float32))
+    card.upload(layer.bias_offset, np.zeros(experts_n, dtype=np.float32) if bias is None else bias)
     card.upload(layer.step_offset, amd.step_block(live))
     wide = layer.wide_router()
     names = ("pairs", "runs", "tiles", "jobs")
