@@ -97,42 +97,93 @@ __device__ static __forceinline__ float det_silu(float gate)
     return __fdiv_rn(gate, __fadd_rn(1.0f, det_exp_sequence(x)));
 }
 
-/* One block of 128 values across a wavefront: lane l holds values l (v0) and l + 64 (v1). Seven stages, the
- * distance doubling from 1; a pair (lower, upper) becomes (lower + upper, lower - upper). No normalisation here. */
-__device__ static __forceinline__ void wave_hadamard128(float &v0, float &v1, uint32_t lane)
+/* The 128-point transform: seven stages, the distance doubling from 1; a pair (lower, upper) becomes (lower + upper, lower -
+ * upper), each rounded once. No normalisation here. Two lay-outs: a block across a wavefront, two values a lane
+ * (wave_hadamard128: the fewest instructions for one block), and across a row of sixteen lanes, eight consecutive values a
+ * lane (row_hadamard128: the fewest for many).
+ *
+ * Lanes meet by the data-parallel primitives of a vector instruction, without LDS. Inside a row those reach lane ^ 1 and ^ 2 (a
+ * permutation of four lanes), ^ 7 (the mirror of eight) and ^ 8 (a rotation by eight of sixteen) in one step, so lane L of a
+ * row stands for place r = row_group_of(L), whose four bits are then the four pairings. A pair's sum and difference are one
+ * fused multiply-add each, own + s x other, with s = +1 in the lower lane and -1 in the upper, which is left with upper - lower,
+ * the difference's exact negative; two lanes that meet in a later pairing carry the same sign, so every value ends as its own or
+ * its exact negative, by the parity of r, and row_normalized takes the sign out with the factor it multiplies by (a zero becomes
+ * +0 there). Rows meet by v_permlane16_swap and v_permlane32_swap of a lane's two values. */
+__device__ static __forceinline__ uint32_t row_group_of(uint32_t lane)
+{
+    return (lane % 16u) ^ ((lane & 4u) != 0u ? 3u : 0u);
+}
+
+__device__ static __forceinline__ void row_signs(uint32_t lane, float (&signs)[4])
 {
 #pragma unroll
-    for (uint32_t distance = 1; distance < WAVE; distance *= 2u) {
-        const float o0 = __shfl_xor(v0, (int)distance, WAVE);
-        const float o1 = __shfl_xor(v1, (int)distance, WAVE);
-        /* the lower of a pair becomes lower + upper, the upper lower - upper: other + own or other - own, one
-         * rounding either way: a fused multiply-add of own by +1 or -1 (the product is exact) */
-        const float sign = (lane & distance) == 0u ? 1.0f : -1.0f;
-        v0 = __fmaf_rn(sign, v0, o0);
-        v1 = __fmaf_rn(sign, v1, o1);
+    for (uint32_t bit = 0; bit < 4u; bit++) {
+        signs[bit] = ((row_group_of(lane) >> bit) & 1u) == 0u ? 1.0f : -1.0f;
     }
-    const float sum = __fadd_rn(v0, v1), difference = __fsub_rn(v0, v1);
-    v0 = sum;
-    v1 = difference;
 }
 
-/* The same transform with a block of 128 values across SIXTEEN lanes (a row of the wavefront): lane r of the row holds
- * values 8 r .. 8 r + 7. Distances 1, 2, 4 stay inside the lane; 8, 16, 32, 64 pair lane r with r ^ 1, ^ 2, ^ 4, ^ 8 of
- * the row, which the data-parallel primitives of a vector instruction reach without LDS: a permutation of four lanes
- * (^ 1, ^ 2), the mirror of eight lanes followed by the reversal of four (^ 4), the mirror of sixteen followed by the
- * mirror of eight (^ 8). Every pair (lower, upper) becomes (lower + upper, lower - upper), each one rounding: the bits of
- * wave_hadamard128. A row's sixteen lanes are all active or all idle. */
-template <int control>
-__device__ static __forceinline__ float row_lane_of(float value)
+/* EXL3_NORMALIZATION with the sign that row_hadamard128 leaves the lane's values with */
+__device__ static __forceinline__ float row_normalization(uint32_t lane)
 {
-    /* every lane of an active row has a source lane in it: what a lane without one would keep is never read */
-    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, value), control, 0xF, 0xF, true));
+    return (__builtin_popcount(row_group_of(lane)) & 1) == 0 ? EXL3_NORMALIZATION : -EXL3_NORMALIZATION;
 }
 
+/* value x EXL3_NORMALIZATION of a value of row_hadamard128, rounded once; a zero becomes +0 */
+__device__ static __forceinline__ float row_normalized(float value, float normalization)
+{
+    return __fmaf_rn(value, normalization, 0.0f);
+}
+
+/* A block across a wavefront: lane l begins with the values wave_channel<SWAPPED>(l) (v0) and 64 on (v1) and ends with those of
+ * wave_channel<!SWAPPED>(l): the exchanges of the rows leave the two upper bits of a lane's number the other way round. */
+template <bool SWAPPED>
+__device__ static __forceinline__ uint32_t wave_channel(uint32_t lane)
+{
+    const uint32_t row = lane / 16u % 2u, half = lane / 32u;
+    return row_group_of(lane) + 16u * (SWAPPED ? half : row) + 32u * (SWAPPED ? row : half);
+}
+
+/* Seventeen instructions and their waits: 14 exchanges through LDS, each waited for, and 14 additions before. A launch of one
+ * row a block of channels is its wavefront's instructions: exl3_tc_activate 6.8 -> 5.6 us (8 rows of 4096 x 2048, 8 picks), 13.1 ->
+ * 11.8 (37 rows), exl3_tc_operands 9.5 -> 8.5 (37 rows); a lane-row form of these launches (eight values a lane) was slower at
+ * one row a job, where eight hidden steps stand one behind the other. */
+template <bool SWAPPED>
+__device__ static __forceinline__ void wave_hadamard128(float &v0, float &v1, uint32_t lane)
+{
+    float signs[4];
+    row_signs(lane, signs);
+    /* written as assembly: the compiler does not fold a lane's move into a multiply-add. Two instructions or waits stand between
+     * a vector write and a lane's read of it, ahead of the first stage and behind the last as well */
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %0, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %1, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\ts_nop 0\n\t"
+        "v_fmac_f32_dpp %0, %0, %3 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %1, %3 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\ts_nop 0\n\t"
+        "v_fmac_f32_dpp %0, %0, %4 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %1, %4 row_half_mirror row_mask:0xf bank_mask:0xf\n\ts_nop 0\n\t"
+        "v_fmac_f32_dpp %0, %0, %5 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %1, %5 row_ror:8 row_mask:0xf bank_mask:0xf\n\ts_nop 1"
+        : "+v"(v0), "+v"(v1)
+        : "v"(signs[0]), "v"(signs[1]), "v"(signs[2]), "v"(signs[3]));
+    /* rows: a lane's two values become the two of one pair; what told them apart moves into the lane's number */
+    const auto pair_rows = [&](bool halves) {
+        const auto swapped = halves ? __builtin_amdgcn_permlane32_swap(__float_as_uint(v0), __float_as_uint(v1), false, false)
+                                    : __builtin_amdgcn_permlane16_swap(__float_as_uint(v0), __float_as_uint(v1), false, false);
+        const float lower = __uint_as_float(swapped[0]), upper = __uint_as_float(swapped[1]);
+        v0 = __fadd_rn(lower, upper);
+        v1 = __fsub_rn(lower, upper);
+    };
+    pair_rows(SWAPPED);  /* 16 */
+    pair_rows(!SWAPPED); /* 32 */
+    pair_rows(SWAPPED);  /* 64 */
+}
+
+/* A block across sixteen lanes: lane L of the row holds the values 8 r .. 8 r + 7 of r = row_group_of(L); distances 1, 2, 4 stay
+ * inside the lane. Seven instructions a value where the lanes' part alone was ten (a sign, moves and an addition a pairing): 32768
+ * pairs of 4096 x 2048: exl3_tcp_operands 148 -> 124 us, exl3_tcp_activate 184 -> 163. A row's sixteen lanes are all active or
+ * all idle. */
 __device__ static __forceinline__ void row_hadamard128(float (&v)[8], uint32_t lane)
 {
-    constexpr int SWAP_PAIRS = 0xB1 /* lanes 1, 0, 3, 2 of four */, SWAP_TWOS = 0x4E /* 2, 3, 0, 1 */, REVERSE_FOUR = 0x1B /* 3, 2, 1, 0 */,
-                  MIRROR_SIXTEEN = 0x140, MIRROR_EIGHT = 0x141;
 #pragma unroll
     for (uint32_t distance = 1; distance < 8u; distance *= 2u) {
 #pragma unroll
@@ -144,26 +195,19 @@ __device__ static __forceinline__ void row_hadamard128(float (&v)[8], uint32_t l
             }
         }
     }
-    /* other + own for the lower lane of a pair, other - own for the upper: own by +1 or -1 (exact), then one addition
-     * whose first operand comes from the other lane inside the instruction */
-    const float sign1 = (lane & 1u) == 0u ? 1.0f : -1.0f, sign2 = (lane & 2u) == 0u ? 1.0f : -1.0f;
-    const float sign4 = (lane & 4u) == 0u ? 1.0f : -1.0f, sign8 = (lane & 8u) == 0u ? 1.0f : -1.0f;
-#pragma unroll
-    for (uint32_t i = 0; i < 8u; i++) {
-        v[i] = __fadd_rn(row_lane_of<SWAP_PAIRS>(v[i]), __fmul_rn(sign1, v[i]));
-    }
-#pragma unroll
-    for (uint32_t i = 0; i < 8u; i++) {
-        v[i] = __fadd_rn(row_lane_of<SWAP_TWOS>(v[i]), __fmul_rn(sign2, v[i]));
-    }
-#pragma unroll
-    for (uint32_t i = 0; i < 8u; i++) {
-        v[i] = __fadd_rn(row_lane_of<REVERSE_FOUR>(row_lane_of<MIRROR_EIGHT>(v[i])), __fmul_rn(sign4, v[i]));
-    }
-#pragma unroll
-    for (uint32_t i = 0; i < 8u; i++) {
-        v[i] = __fadd_rn(row_lane_of<MIRROR_EIGHT>(row_lane_of<MIRROR_SIXTEEN>(v[i])), __fmul_rn(sign8, v[i]));
-    }
+    float signs[4];
+    row_signs(lane, signs);
+    /* as in wave_hadamard128; a value's next instruction is eight behind its last */
+#define ROW_STAGE(control, sign)                                                                                           \
+    "v_fmac_f32_dpp %0, %0, %" sign " " control "\n\tv_fmac_f32_dpp %1, %1, %" sign " " control "\n\t"                     \
+    "v_fmac_f32_dpp %2, %2, %" sign " " control "\n\tv_fmac_f32_dpp %3, %3, %" sign " " control "\n\t"                     \
+    "v_fmac_f32_dpp %4, %4, %" sign " " control "\n\tv_fmac_f32_dpp %5, %5, %" sign " " control "\n\t"                     \
+    "v_fmac_f32_dpp %6, %6, %" sign " " control "\n\tv_fmac_f32_dpp %7, %7, %" sign " " control "\n\t"
+    asm("s_nop 1\n\t" ROW_STAGE("quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf", "8") ROW_STAGE("quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf", "9")
+            ROW_STAGE("row_half_mirror row_mask:0xf bank_mask:0xf", "10") ROW_STAGE("row_ror:8 row_mask:0xf bank_mask:0xf", "11")
+        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])
+        : "v"(signs[0]), "v"(signs[1]), "v"(signs[2]), "v"(signs[3]));
+#undef ROW_STAGE
 }
 
 /* eight bfloat16 or fp16 values of a 16-byte load as float32; eight float32 as fp16, one rounding each */
@@ -191,6 +235,50 @@ __device__ static __forceinline__ uint4_t pack_half8(const float (&values)[8])
         packed[word] = (uint32_t)float_to_half_bits(values[2u * word]) | ((uint32_t)float_to_half_bits(values[2u * word + 1u]) << 16);
     }
     return packed;
+}
+
+/* eight values of a row (row_hadamard128's lanes) as an operand of one matrix: fp16(H128(x suh) / sqrt(128)) */
+__device__ static __forceinline__ uint4_t row_operand(uint4_t load, const float (&scale)[8], uint32_t lane)
+{
+    float v[8];
+    unpack_bf16x8(load, v);
+#pragma unroll
+    for (uint32_t j = 0; j < 8u; j++) {
+        v[j] = __fmul_rn(v[j], scale[j]);
+    }
+    row_hadamard128(v, lane);
+    const float normalization = row_normalization(lane);
+#pragma unroll
+    for (uint32_t j = 0; j < 8u; j++) {
+        v[j] = row_normalized(v[j], normalization);
+    }
+    return pack_half8(v);
+}
+
+/* eight gate and eight up products (g, u) as a down operand: gate = H128(gate products) / sqrt(128) x svh, up the same, the
+ * SwiGLU with its limit, x the down matrix's suh, H128, fp16 */
+__device__ static __forceinline__ uint4_t row_activated(float (&g)[8], float (&u)[8], const float (&gs)[8], const float (&us)[8],
+                                                        const float (&ds)[8], float limit, uint32_t lane)
+{
+    float v[8];
+    row_hadamard128(g, lane);
+    row_hadamard128(u, lane);
+    const float normalization = row_normalization(lane);
+#pragma unroll
+    for (uint32_t j = 0; j < 8u; j++) {
+        const float gate = __fmul_rn(__fmul_rn(g[j], normalization), gs[j]);
+        const float up = __fmul_rn(__fmul_rn(u[j], normalization), us[j]);
+        const float bounded_gate = limit > 0.0f ? fminf(gate, limit) : gate;
+        const float bounded_up = limit > 0.0f ? fminf(fmaxf(up, -limit), limit) : up;
+        const float hidden = __fmul_rn(det_silu(bounded_gate), bounded_up);
+        v[j] = __fmul_rn(hidden, ds[j]);
+    }
+    row_hadamard128(v, lane);
+#pragma unroll
+    for (uint32_t j = 0; j < 8u; j++) {
+        v[j] = row_normalized(v[j], normalization);
+    }
+    return pack_half8(v);
 }
 
 /* mul1: two 16-bit states -> two fp16 weights in one register (low half: first) */

@@ -56,7 +56,8 @@ extern "C" __global__ void exl3_input(struct exl3_expert_record record, unsigned
         return;
     }
     const uint32_t lane = threadIdx.x, projection = blockIdx.z;
-    const uint32_t channel = blockIdx.x * EXL3_TRANSFORM + lane;
+    const uint32_t channel = blockIdx.x * EXL3_TRANSFORM + wave_channel<false>(lane), to = blockIdx.x * EXL3_TRANSFORM + wave_channel<true>(lane);
+    const float normalization = row_normalization(lane);
     const uint64_t matrix = projection == 0u ? job->gate_offset : job->up_offset;
     const uint32_t bits_x2 = exl3_bits_x2(chain_width(record, arena, job->expert, projection));
     const uint16_t *suh = (const uint16_t *)(arena + matrix + exl3_code_bytes(record.input_size, record.inner_size, bits_x2));
@@ -68,10 +69,10 @@ extern "C" __global__ void exl3_input(struct exl3_expert_record record, unsigned
         const uint64_t row = pair / record.pairs_per_row;
         float v0 = __fmul_rn(bf16_to_float(input[row * record.input_size + channel]), s0);
         float v1 = __fmul_rn(bf16_to_float(input[row * record.input_size + channel + WAVE]), s1);
-        wave_hadamard128(v0, v1, lane);
+        wave_hadamard128<false>(v0, v1, lane);
         uint16_t *out = operands + ((uint64_t)projection * record.pair_count + pair) * record.input_size;
-        out[channel] = float_to_half_bits(__fmul_rn(v0, EXL3_NORMALIZATION));
-        out[channel + WAVE] = float_to_half_bits(__fmul_rn(v1, EXL3_NORMALIZATION));
+        out[to] = float_to_half_bits(row_normalized(v0, normalization));
+        out[to + WAVE] = float_to_half_bits(row_normalized(v1, normalization));
     }
 }
 ANEMONE_KERNEL(EXL3_KERNEL_FILE, exl3_input, exl3_expert_record);
@@ -192,7 +193,10 @@ extern "C" __global__ void exl3_activate(struct exl3_expert_record record, unsig
     if (job->row_count == 0u) {
         return;
     }
-    const uint32_t lane = threadIdx.x, channel = blockIdx.x * EXL3_TRANSFORM + lane;
+    /* the products by channel, the hidden values by the channels their transforms leave a lane with, the operand by channel again */
+    const uint32_t lane = threadIdx.x;
+    const uint32_t channel = blockIdx.x * EXL3_TRANSFORM + wave_channel<false>(lane), between = blockIdx.x * EXL3_TRANSFORM + wave_channel<true>(lane);
+    const float normalization = row_normalization(lane);
     const uint32_t H = record.input_size, I = record.inner_size;
     const uint16_t *gate_svh = (const uint16_t *)(arena + job->gate_offset +
                                                   exl3_code_bytes(H, I, exl3_bits_x2(chain_width(record, arena, job->expert, 0u)))) + H;
@@ -200,9 +204,9 @@ extern "C" __global__ void exl3_activate(struct exl3_expert_record record, unsig
                                                 exl3_code_bytes(H, I, exl3_bits_x2(chain_width(record, arena, job->expert, 1u)))) + H;
     const uint16_t *down_suh = (const uint16_t *)(arena + job->down_offset +
                                                   exl3_code_bytes(I, H, exl3_bits_x2(chain_width(record, arena, job->expert, 2u))));
-    const float gs0 = half_bits_to_float(gate_svh[channel]), gs1 = half_bits_to_float(gate_svh[channel + WAVE]);
-    const float us0 = half_bits_to_float(up_svh[channel]), us1 = half_bits_to_float(up_svh[channel + WAVE]);
-    const float ds0 = half_bits_to_float(down_suh[channel]), ds1 = half_bits_to_float(down_suh[channel + WAVE]);
+    const float gs0 = half_bits_to_float(gate_svh[between]), gs1 = half_bits_to_float(gate_svh[between + WAVE]);
+    const float us0 = half_bits_to_float(up_svh[between]), us1 = half_bits_to_float(up_svh[between + WAVE]);
+    const float ds0 = half_bits_to_float(down_suh[between]), ds1 = half_bits_to_float(down_suh[between + WAVE]);
     const float limit = record.activation_limit;
     const float *products = (const float *)(arena + record.products_offset);
     for (uint32_t column = 0; column < job->row_count; column++) {
@@ -210,11 +214,11 @@ extern "C" __global__ void exl3_activate(struct exl3_expert_record record, unsig
         float g0 = products[(uint64_t)pair * I + channel], g1 = products[(uint64_t)pair * I + channel + WAVE];
         float u0 = products[((uint64_t)record.pair_count + pair) * I + channel];
         float u1 = products[((uint64_t)record.pair_count + pair) * I + channel + WAVE];
-        wave_hadamard128(g0, g1, lane);
-        wave_hadamard128(u0, u1, lane);
+        wave_hadamard128<false>(g0, g1, lane);
+        wave_hadamard128<false>(u0, u1, lane);
         float hidden[2];
-        const float gate[2] = {__fmul_rn(__fmul_rn(g0, EXL3_NORMALIZATION), gs0), __fmul_rn(__fmul_rn(g1, EXL3_NORMALIZATION), gs1)};
-        const float up[2] = {__fmul_rn(__fmul_rn(u0, EXL3_NORMALIZATION), us0), __fmul_rn(__fmul_rn(u1, EXL3_NORMALIZATION), us1)};
+        const float gate[2] = {__fmul_rn(row_normalized(g0, normalization), gs0), __fmul_rn(row_normalized(g1, normalization), gs1)};
+        const float up[2] = {__fmul_rn(row_normalized(u0, normalization), us0), __fmul_rn(row_normalized(u1, normalization), us1)};
 #pragma unroll
         for (uint32_t i = 0; i < 2u; i++) {
             const float bounded_gate = fminf(gate[i], limit);
@@ -222,13 +226,13 @@ extern "C" __global__ void exl3_activate(struct exl3_expert_record record, unsig
             hidden[i] = __fmul_rn(det_silu(bounded_gate), bounded_up);
         }
         uint16_t *hidden_out = (uint16_t *)(arena + record.hidden_offset) + (uint64_t)pair * I;
-        hidden_out[channel] = float_to_bf16(hidden[0]);
-        hidden_out[channel + WAVE] = float_to_bf16(hidden[1]);
+        hidden_out[between] = float_to_bf16(hidden[0]);
+        hidden_out[between + WAVE] = float_to_bf16(hidden[1]);
         float v0 = __fmul_rn(hidden[0], ds0), v1 = __fmul_rn(hidden[1], ds1);
-        wave_hadamard128(v0, v1, lane);
+        wave_hadamard128<true>(v0, v1, lane);
         uint16_t *operand = (uint16_t *)(arena + record.operands_offset) + (uint64_t)pair * I;
-        operand[channel] = float_to_half_bits(__fmul_rn(v0, EXL3_NORMALIZATION));
-        operand[channel + WAVE] = float_to_half_bits(__fmul_rn(v1, EXL3_NORMALIZATION));
+        operand[channel] = float_to_half_bits(row_normalized(v0, normalization));
+        operand[channel + WAVE] = float_to_half_bits(row_normalized(v1, normalization));
     }
 }
 ANEMONE_KERNEL(EXL3_KERNEL_FILE, exl3_activate, exl3_expert_record);
@@ -239,20 +243,22 @@ extern "C" __global__ void exl3_finish(struct exl3_expert_record record, unsigne
     if (job->row_count == 0u) {
         return;
     }
-    const uint32_t lane = threadIdx.x, channel = blockIdx.x * EXL3_TRANSFORM + lane;
+    const uint32_t lane = threadIdx.x;
+    const uint32_t channel = blockIdx.x * EXL3_TRANSFORM + wave_channel<false>(lane), to = blockIdx.x * EXL3_TRANSFORM + wave_channel<true>(lane);
+    const float normalization = row_normalization(lane);
     const uint32_t H = record.input_size, I = record.inner_size;
     const uint16_t *svh = (const uint16_t *)(arena + job->down_offset +
                                              exl3_code_bytes(I, H, exl3_bits_x2(chain_width(record, arena, job->expert, 2u)))) + I;
-    const float s0 = half_bits_to_float(svh[channel]), s1 = half_bits_to_float(svh[channel + WAVE]);
+    const float s0 = half_bits_to_float(svh[to]), s1 = half_bits_to_float(svh[to + WAVE]);
     for (uint32_t column = 0; column < job->row_count; column++) {
         const uint32_t pair = job->pair_index[column];
         float *values = (float *)(arena + record.products_offset) + (uint64_t)pair * H;
         float v0 = values[channel], v1 = values[channel + WAVE];
-        wave_hadamard128(v0, v1, lane);
+        wave_hadamard128<false>(v0, v1, lane); /* the whole block's loads have landed: the output may take the products' place */
         const float weight = job->route_weight[column];
         float *out = (float *)(arena + record.output_offset) + (uint64_t)pair * H;
-        out[channel] = __fmul_rn(__fmul_rn(__fmul_rn(v0, EXL3_NORMALIZATION), s0), weight);
-        out[channel + WAVE] = __fmul_rn(__fmul_rn(__fmul_rn(v1, EXL3_NORMALIZATION), s1), weight);
+        out[to] = __fmul_rn(__fmul_rn(row_normalized(v0, normalization), s0), weight);
+        out[to + WAVE] = __fmul_rn(__fmul_rn(row_normalized(v1, normalization), s1), weight);
     }
 }
 ANEMONE_KERNEL(EXL3_KERNEL_FILE, exl3_finish, exl3_expert_record);

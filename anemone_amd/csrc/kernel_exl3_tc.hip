@@ -65,7 +65,9 @@ extern "C" __global__ void exl3_tc_operands(struct exl3_tc_record record, unsign
         return;
     }
     const tc_shape shape = tc_shape_of(record);
-    const uint32_t lane = threadIdx.x, projection = blockIdx.z, channel = blockIdx.x * EXL3_TRANSFORM + lane;
+    const uint32_t lane = threadIdx.x, projection = blockIdx.z;
+    const uint32_t channel = blockIdx.x * EXL3_TRANSFORM + wave_channel<false>(lane), to = blockIdx.x * EXL3_TRANSFORM + wave_channel<true>(lane);
+    const float normalization = row_normalization(lane);
     const uint64_t matrix = projection == 0u ? job->gate_offset : job->up_offset;
     const uint16_t *suh = (const uint16_t *)(arena + matrix + exl3_code_bytes(shape.hidden, shape.intermediate,
                                                                                tc_bits_x2(record, arena, job->expert, projection)));
@@ -77,10 +79,10 @@ extern "C" __global__ void exl3_tc_operands(struct exl3_tc_record record, unsign
         const uint64_t row = pair / shape.picks;
         float v0 = __fmul_rn(bf16_to_float(rows[row * shape.hidden + channel]), s0);
         float v1 = __fmul_rn(bf16_to_float(rows[row * shape.hidden + channel + WAVE]), s1);
-        wave_hadamard128(v0, v1, lane);
+        wave_hadamard128<false>(v0, v1, lane);
         uint16_t *out = operands + ((uint64_t)projection * shape.pairs + pair) * shape.hidden;
-        out[channel] = float_to_half_bits(__fmul_rn(v0, EXL3_NORMALIZATION));
-        out[channel + WAVE] = float_to_half_bits(__fmul_rn(v1, EXL3_NORMALIZATION));
+        out[to] = float_to_half_bits(row_normalized(v0, normalization));
+        out[to + WAVE] = float_to_half_bits(row_normalized(v1, normalization));
     }
 }
 ANEMONE_KERNEL(EXL3_TC_KERNEL_FILE, exl3_tc_operands, exl3_tc_record);
@@ -197,20 +199,24 @@ extern "C" __global__ void exl3_tc_activate(struct exl3_tc_record record, unsign
         return;
     }
     const tc_shape shape = tc_shape_of(record);
-    const uint32_t lane = threadIdx.x, channel = blockIdx.x * EXL3_TRANSFORM + lane;
+    /* the sums by channel, the hidden values by the channels their transforms leave a lane with, the operand by channel again */
+    const uint32_t lane = threadIdx.x;
+    const uint32_t channel = blockIdx.x * EXL3_TRANSFORM + wave_channel<false>(lane), between = blockIdx.x * EXL3_TRANSFORM + wave_channel<true>(lane);
+    const float normalization = row_normalization(lane);
     const uint32_t H = shape.hidden, I = shape.intermediate;
     const uint16_t *gate_svh = (const uint16_t *)(arena + job->gate_offset + exl3_code_bytes(H, I, tc_bits_x2(record, arena, job->expert, 0u))) + H;
     const uint16_t *up_svh = (const uint16_t *)(arena + job->up_offset + exl3_code_bytes(H, I, tc_bits_x2(record, arena, job->expert, 1u))) + H;
     const uint16_t *down_suh = (const uint16_t *)(arena + job->down_offset + exl3_code_bytes(I, H, tc_bits_x2(record, arena, job->expert, 2u)));
-    const float gs[2] = {half_bits_to_float(gate_svh[channel]), half_bits_to_float(gate_svh[channel + WAVE])};
-    const float us[2] = {half_bits_to_float(up_svh[channel]), half_bits_to_float(up_svh[channel + WAVE])};
-    const float ds[2] = {half_bits_to_float(down_suh[channel]), half_bits_to_float(down_suh[channel + WAVE])};
+    const float gs[2] = {half_bits_to_float(gate_svh[between]), half_bits_to_float(gate_svh[between + WAVE])};
+    const float us[2] = {half_bits_to_float(up_svh[between]), half_bits_to_float(up_svh[between + WAVE])};
+    const float ds[2] = {half_bits_to_float(down_suh[between]), half_bits_to_float(down_suh[between + WAVE])};
     const float limit = record.activation_limit;
     unsigned char *workspace = arena + record.workspace_offset;
     const float *partials = (const float *)(workspace + exl3_tc_operand_bytes(shape.pairs, H));
     for (uint32_t column = 0; column < job->row_count; column++) {
         const uint32_t pair = job->pair_index[column];
         float g[2] = {0.0f, 0.0f}, u[2] = {0.0f, 0.0f};
+#pragma unroll
         for (uint32_t slice = 0; slice < EXL3_TC_GATE_UP_SLICES; slice++) { /* in slice order from +0 */
             const float *gate = partials + ((uint64_t)slice * 2u * shape.pairs + pair) * I;
             const float *up = partials + (((uint64_t)slice * 2u + 1u) * shape.pairs + pair) * I;
@@ -219,22 +225,22 @@ extern "C" __global__ void exl3_tc_activate(struct exl3_tc_record record, unsign
             u[0] = __fadd_rn(u[0], up[channel]);
             u[1] = __fadd_rn(u[1], up[channel + WAVE]);
         }
-        wave_hadamard128(g[0], g[1], lane);
-        wave_hadamard128(u[0], u[1], lane);
+        wave_hadamard128<false>(g[0], g[1], lane);
+        wave_hadamard128<false>(u[0], u[1], lane);
         float v[2];
 #pragma unroll
         for (uint32_t i = 0; i < 2u; i++) {
-            const float gate = __fmul_rn(__fmul_rn(g[i], EXL3_NORMALIZATION), gs[i]);
-            const float up = __fmul_rn(__fmul_rn(u[i], EXL3_NORMALIZATION), us[i]);
+            const float gate = __fmul_rn(row_normalized(g[i], normalization), gs[i]);
+            const float up = __fmul_rn(row_normalized(u[i], normalization), us[i]);
             const float bounded_gate = limit > 0.0f ? fminf(gate, limit) : gate;
             const float bounded_up = limit > 0.0f ? fminf(fmaxf(up, -limit), limit) : up;
             const float hidden = __fmul_rn(det_silu(bounded_gate), bounded_up);
             v[i] = __fmul_rn(hidden, ds[i]);
         }
-        wave_hadamard128(v[0], v[1], lane);
+        wave_hadamard128<true>(v[0], v[1], lane);
         uint16_t *operand = (uint16_t *)workspace + (uint64_t)pair * I;
-        operand[channel] = float_to_half_bits(__fmul_rn(v[0], EXL3_NORMALIZATION));
-        operand[channel + WAVE] = float_to_half_bits(__fmul_rn(v[1], EXL3_NORMALIZATION));
+        operand[channel] = float_to_half_bits(row_normalized(v[0], normalization));
+        operand[channel + WAVE] = float_to_half_bits(row_normalized(v[1], normalization));
     }
 }
 ANEMONE_KERNEL(EXL3_TC_KERNEL_FILE, exl3_tc_activate, exl3_tc_record);
@@ -249,7 +255,8 @@ extern "C" __global__ void __launch_bounds__(COMBINE_THREADS) exl3_tc_combine(st
     __shared__ uint32_t is_held[ROUTER_MOST_PICKS];
     const tc_shape shape = tc_shape_of(record);
     const uint32_t lane = threadIdx.x % WAVE, slot = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const uint32_t channel = blockIdx.x * EXL3_TRANSFORM + lane, row = blockIdx.y;
+    const uint32_t first_channel = blockIdx.x * EXL3_TRANSFORM, channel = first_channel + wave_channel<false>(lane), to = wave_channel<true>(lane);
+    const uint32_t row = blockIdx.y;
     const uint32_t H = shape.hidden, I = shape.intermediate;
     const struct expert_job_record *jobs = (const struct expert_job_record *)(arena + record.jobs_offset);
     const unsigned char *workspace = arena + record.workspace_offset;
@@ -308,20 +315,21 @@ extern "C" __global__ void __launch_bounds__(COMBINE_THREADS) exl3_tc_combine(st
         }
         if (held) {
             const uint16_t *svh = (const uint16_t *)(arena + down_offset + exl3_code_bytes(I, H, tc_bits_x2(record, arena, expert, 2u))) + I;
-            const float scale0 = half_bits_to_float(svh[channel]), scale1 = half_bits_to_float(svh[channel + WAVE]);
+            const float scale0 = half_bits_to_float(svh[first_channel + to]), scale1 = half_bits_to_float(svh[first_channel + to + WAVE]);
             float v0 = 0.0f, v1 = 0.0f;
 #pragma unroll
             for (uint32_t slice = 0; slice < EXL3_TC_DOWN_SLICES; slice++) { /* in slice order from +0 */
                 v0 = __fadd_rn(v0, partial0[slice]);
                 v1 = __fadd_rn(v1, partial1[slice]);
             }
-            wave_hadamard128(v0, v1, lane);
-            y0 = __fmul_rn(__fmul_rn(__fmul_rn(v0, EXL3_NORMALIZATION), scale0), weight);
-            y1 = __fmul_rn(__fmul_rn(__fmul_rn(v1, EXL3_NORMALIZATION), scale1), weight);
+            wave_hadamard128<false>(v0, v1, lane);
+            const float normalization = row_normalization(lane);
+            y0 = __fmul_rn(__fmul_rn(row_normalized(v0, normalization), scale0), weight);
+            y1 = __fmul_rn(__fmul_rn(row_normalized(v1, normalization), scale1), weight);
         }
     }
-    values[slot][lane] = y0;
-    values[slot][lane + WAVE] = y1;
+    values[slot][to] = y0;
+    values[slot][to + WAVE] = y1;
     if (lane == 0u) {
         is_held[slot] = held ? 1u : 0u;
     }
@@ -340,13 +348,13 @@ extern "C" __global__ void __launch_bounds__(COMBINE_THREADS) exl3_tc_combine(st
         /* the sum joins the shared expert's bfloat16 row, in place: bfloat16(sum + row), one rounding of the float32
          * addition's result (source/kernel_exl3_tc.cu:468-471 of the reference); output_offset is not written */
         uint16_t *shared = (uint16_t *)(arena + record.shared_offset) + (uint64_t)row * H;
-        shared[channel] = float_to_bf16(__fadd_rn(sum0, bf16_to_float(shared[channel])));
-        shared[channel + WAVE] = float_to_bf16(__fadd_rn(sum1, bf16_to_float(shared[channel + WAVE])));
+        shared[first_channel + lane] = float_to_bf16(__fadd_rn(sum0, bf16_to_float(shared[first_channel + lane])));
+        shared[first_channel + lane + WAVE] = float_to_bf16(__fadd_rn(sum1, bf16_to_float(shared[first_channel + lane + WAVE])));
         return;
     }
     float *out = (float *)(arena + record.output_offset) + (uint64_t)row * H;
-    out[channel] = sum0;
-    out[channel + WAVE] = sum1;
+    out[first_channel + lane] = sum0;
+    out[first_channel + lane + WAVE] = sum1;
 }
 ANEMONE_KERNEL(EXL3_TC_KERNEL_FILE, exl3_tc_combine, exl3_tc_record);
 

@@ -173,31 +173,14 @@ __device__ static __forceinline__ struct exl3_tcp_chunk tcp_chunk_of(const tcp_s
     return chunk;
 }
 
-/* The element-wise launches take a block of 128 values in a row of sixteen lanes, eight consecutive values a lane
- * (one 16-byte load of bfloat16 or fp16, two of float32): a wavefront is four adjacent blocks of one vector, 1 KB of
+/* The element-wise launches take a block of 128 values in a row of sixteen lanes, eight consecutive values a lane in
+ * row_hadamard128's order (one 16-byte load of bfloat16 or fp16, two of float32): a wavefront is four adjacent blocks of one vector, 1 KB of
  * bfloat16 a load. this lane's block of 128 channels and its first channel, or false past the width */
 __device__ static __forceinline__ bool tcp_lane_channels(uint32_t width, uint32_t &channel)
 {
     const uint32_t lane = threadIdx.x;
-    channel = (blockIdx.x * TCP_WAVE_BLOCKS + lane / 16u) * EXL3_TRANSFORM + 8u * (lane % 16u);
+    channel = (blockIdx.x * TCP_WAVE_BLOCKS + lane / 16u) * EXL3_TRANSFORM + 8u * row_group_of(lane);
     return channel < width;
-}
-
-/* eight values of a row as an operand of one matrix: fp16(H128(x suh) / sqrt(128)) */
-__device__ static __forceinline__ uint4_t tcp_operand(uint4_t load, const float (&scale)[8], uint32_t lane)
-{
-    float v[8];
-    unpack_bf16x8(load, v);
-#pragma unroll
-    for (uint32_t j = 0; j < 8u; j++) {
-        v[j] = __fmul_rn(v[j], scale[j]);
-    }
-    row_hadamard128(v, lane);
-#pragma unroll
-    for (uint32_t j = 0; j < 8u; j++) {
-        v[j] = __fmul_rn(v[j], EXL3_NORMALIZATION);
-    }
-    return pack_half8(v);
 }
 
 /* launch 2: grid (ceil(hidden / 512), chunk capacity, EXL3_TCP_COLUMN_PARTS), block 64: the gate and the up operands of
@@ -242,7 +225,7 @@ extern "C" __global__ void exl3_tcp_operands(struct exl3_tcp_record record, unsi
             const bool kept = first + i < last_column;
 #pragma unroll
             for (uint32_t projection = 0; projection < 2u; projection++) {
-                const uint4_t operand = tcp_operand(loads[i], scale[projection], lane);
+                const uint4_t operand = row_operand(loads[i], scale[projection], lane);
                 if (kept) {
                     *(uint4_t *)(operands + ((uint64_t)projection * shape.pairs + place[i]) * shape.hidden + channel) = operand;
                 }
@@ -263,7 +246,7 @@ __device__ static __forceinline__ bool tcp_thin_place(const tcp_shape &shape, co
 {
     lane = threadIdx.x % WAVE;
     place = blockIdx.y * TCP_THIN_PLACES + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    channel = (blockIdx.x * TCP_WAVE_BLOCKS + lane / 16u) * EXL3_TRANSFORM + 8u * (lane % 16u);
+    channel = (blockIdx.x * TCP_WAVE_BLOCKS + lane / 16u) * EXL3_TRANSFORM + 8u * row_group_of(lane);
     if (place >= shape.pairs || channel >= width) {
         return false;
     }
@@ -291,7 +274,7 @@ extern "C" __global__ void __launch_bounds__(TCP_THIN_PLACES * WAVE) exl3_tcp_op
     for (uint32_t projection = 0; projection < 2u; projection++) {
         float scale[8];
         unpack_half8(scales[projection], scale);
-        *(uint4_t *)(operands + ((uint64_t)projection * shape.pairs + place) * shape.hidden + channel) = tcp_operand(load, scale, lane);
+        *(uint4_t *)(operands + ((uint64_t)projection * shape.pairs + place) * shape.hidden + channel) = row_operand(load, scale, lane);
     }
 }
 ANEMONE_KERNEL(EXL3_TCP_KERNEL_FILE, exl3_tcp_operands_thin, exl3_tcp_record);
@@ -773,34 +756,17 @@ extern "C" __global__ void __launch_bounds__(TCP_GEMM_THREADS, 4) exl3_tcp_gemm_
 }
 ANEMONE_KERNEL(EXL3_TCP_KERNEL_FILE, exl3_tcp_gemm_thin, exl3_tcp_record);
 
-/* eight gate and eight up products as a down operand: gate = H128(gate products) / sqrt(128) x svh, up the same, the SwiGLU
- * with its limit, x the down matrix's suh, H128, fp16 */
+/* a pair's gate and up products (gate's eight, then up's) as its down operand */
 __device__ static __forceinline__ uint4_t tcp_activated(const float4_t (&loads)[4], const float (&gs)[8], const float (&us)[8], const float (&ds)[8],
                                                         float limit, uint32_t lane)
 {
-    float g[8], u[8], v[8];
+    float g[8], u[8];
 #pragma unroll
     for (uint32_t j = 0; j < 8u; j++) {
         g[j] = loads[j / 4u][j % 4u];
         u[j] = loads[2u + j / 4u][j % 4u];
     }
-    row_hadamard128(g, lane);
-    row_hadamard128(u, lane);
-#pragma unroll
-    for (uint32_t j = 0; j < 8u; j++) {
-        const float gate = __fmul_rn(__fmul_rn(g[j], EXL3_NORMALIZATION), gs[j]);
-        const float up = __fmul_rn(__fmul_rn(u[j], EXL3_NORMALIZATION), us[j]);
-        const float bounded_gate = limit > 0.0f ? fminf(gate, limit) : gate;
-        const float bounded_up = limit > 0.0f ? fminf(fmaxf(up, -limit), limit) : up;
-        const float hidden = __fmul_rn(det_silu(bounded_gate), bounded_up);
-        v[j] = __fmul_rn(hidden, ds[j]);
-    }
-    row_hadamard128(v, lane);
-#pragma unroll
-    for (uint32_t j = 0; j < 8u; j++) {
-        v[j] = __fmul_rn(v[j], EXL3_NORMALIZATION);
-    }
-    return pack_half8(v);
+    return row_activated(g, u, gs, us, ds, limit, lane);
 }
 
 /* launch 4: grid (ceil(intermediate / 512), chunk capacity, EXL3_TCP_COLUMN_PARTS), block 64: per pair of a part of the chunk, gate = H128(gate products) /
@@ -892,6 +858,7 @@ extern "C" __global__ void exl3_tcp_combine(struct exl3_tcp_record record, unsig
     const struct router_pick *picks = (const struct router_pick *)(arena + record.picks_offset) + (uint64_t)row * shape.picks;
     const uint32_t *place_of = (const uint32_t *)(workspace + shape.layout.place_of);
     const float *down = (const float *)(workspace + shape.layout.down);
+    const float normalization = row_normalization(lane);
     float sum[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     for (uint32_t slot = 0; slot < shape.picks; slot++) {
         const struct router_pick pick = picks[slot];
@@ -905,7 +872,7 @@ extern "C" __global__ void exl3_tcp_combine(struct exl3_tcp_record record, unsig
         row_hadamard128(v, lane);
 #pragma unroll
         for (uint32_t j = 0; j < 8u; j++) {
-            sum[j] = __fadd_rn(sum[j], __fmul_rn(__fmul_rn(__fmul_rn(v[j], EXL3_NORMALIZATION), scale[j]), pick.route_weight));
+            sum[j] = __fadd_rn(sum[j], __fmul_rn(__fmul_rn(row_normalized(v[j], normalization), scale[j]), pick.route_weight));
         }
     }
     float4_t *out = (float4_t *)((float *)(arena + record.output_offset) + (uint64_t)row * H + channel);
