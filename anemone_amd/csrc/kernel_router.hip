@@ -415,8 +415,8 @@ ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_select_entry, router_select_arguments)
  * Four launches of one record, in this order (include/anemone/router_records.h:31-47 of the reference; the kernels
  * at source/kernel_router.cu:97-459 there): the picks of every live row; the pairs of each expert counted in blocks
  * of ROUTER_SORT_ROWS rows; every pair placed (a pair's place: the pairs of lower experts, and of its expert in
- * lower rows), the runs and the tiles of at most 64 pairs; the job table of at most 8 pairs a job. No atomic
- * operation: a thread owns an expert and walks the block's picks in row order. */
+ * lower rows), the runs and the tiles of at most 64 pairs; the job table of at most 8 pairs a job. The only atomic
+ * operations count in LDS; the order is the rows' (sort_device.cuh). */
 #define WIDE_SORT_THREADS 512u
 
 __device__ static __forceinline__ uint32_t wide_live_rows(const struct router_wide_arguments &arguments, const unsigned char *arena)
