@@ -44,9 +44,9 @@ __device__ static __forceinline__ void native_vectors_of(const struct wide_pair 
 
 /* grid (ceil(output_size / (4 strips)), tile_count), block 256; a strip is STRIP tiles of gate and STRIP of up */
 /* sets of weight registers and stages of columns: 4-bit weights 2 and 2, with strips of four gate and four up tiles (eight
- * of down) at two wavefronts a SIMD (243 registers, 128 of them sums): a column block's operand read from LDS and its
- * preparation serve eight matrix instructions and not four (8192 rows of 4096 x 2048 x 256 experts: gate/up 1157 -> 1096
- * us, down 651 -> 625, against strips of half as many, three sets and three wavefronts). One-byte weights: gate/up 2 and 2
+ * of down) at two wavefronts a SIMD (232 registers, 128 of them sums): a column block's operand read from LDS and its
+ * permutations serve eight matrix instructions and not four (8192 rows of 4096 x 2048 x 256 experts: gate/up 1157 -> 1096
+ * us, down 651 -> 625, against strips of half as many, three sets and three wavefronts; both with columns turned in place). One-byte weights: gate/up 2 and 2
  * at three wavefronts a SIMD (143 registers, 165 with float32 scales), down 3 and 3 at two (215 and 222): 2048 rows of
  * 4096 x 2048 x 256 experts, gate/up 880 us against 900 (float32 scales 850 / 864), down 433 against 444 (444 / 453). */
 template <bool BYTES, bool DOWN, uint32_t TILES> /* tiles of a wavefront, of its matrices together */
@@ -63,7 +63,7 @@ __device__ static __forceinline__ void native_expert_gate_up(const struct wide_e
     typedef native_chain<2, BYTES, STRIP, COLUMN_BLOCKS, depths::SLOTS, depths::DEPTH, B128> chain_type;
     constexpr uint32_t TILES = chain_type::TILES;
     static_assert(STRIP == 1u || STRIP % 2u == 0u, "a quantizer block of 32 outputs is two strips, or strips are whole blocks");
-    extern __shared__ __attribute__((aligned(16))) unsigned char window[];
+    extern __shared__ __attribute__((aligned(128))) unsigned char window[];
     __shared__ struct wide_pair columns[COLUMN_BLOCKS * 16u];
     const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     struct wide_expert_tile tile;
@@ -98,7 +98,7 @@ __device__ static __forceinline__ void native_expert_down(const struct wide_expe
     typedef native_depths<BYTES, true, DOWN_STRIP> depths;
     typedef native_chain<1, BYTES, DOWN_STRIP, COLUMN_BLOCKS, depths::SLOTS, depths::DEPTH, B128> chain_type;
     constexpr uint32_t TILES = chain_type::TILES, STRIP = chain_type::STRIP;
-    extern __shared__ __attribute__((aligned(16))) unsigned char window[];
+    extern __shared__ __attribute__((aligned(128))) unsigned char window[];
     __shared__ struct wide_pair columns[COLUMN_BLOCKS * 16u];
     const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     struct wide_expert_tile tile;

@@ -4,8 +4,11 @@
  * v_mfma_scale_f32_16x16x128_f8f6f4, 16 bytes a lane (32 of one-byte weights, as two halves of 16), and goes from memory
  * into the wavefront's registers with one 16-byte load a lane and half: no LDS stage, no vector instruction between the
  * load and the matrix instruction. Only the columns (the vectors' codes, which every wavefront of the block reads) pass
- * through LDS, as in wide_device.cuh: brought by LDS DMA; those of a block of 4-bit weights are turned into the B operand's
- * order in place by the wavefront that brought them, a block of one-byte weights reads them as they landed.
+ * through LDS, as in wide_device.cuh: brought by LDS DMA and read as they landed. (4-bit weights take the B operand's bytes in
+ * another order, eight permutations a column block in every wavefront, which run beside the matrix instructions. Turned
+ * about in place, once a block, by the wavefront that brought them, the columns cost it an LDS round trip ahead of every
+ * step's barrier: 8192 rows of 4096 x 2048 x 256 experts, with the weights asked for in the middle of a step: gate/up 1098
+ * -> 1065 us, down 635 -> 606.)
  *
  * A block is COLUMN_BLOCKS x 16 columns (pairs of one expert) by four wavefronts' strips of weight tiles. A wavefront
  * keeps several sets of weight registers: while one step is multiplied, the loads of the steps behind it are on their way.
@@ -25,10 +28,6 @@
 #include "native_waits.h"
 
 #define NATIVE_WAVES 4u
-/* one-byte weights: a step's next weights are asked for at its top, ahead of the columns' preparation and the barrier
- * (gate/up 953 -> 933 us, down 462 -> 456); 4-bit weights: in the middle of its matrix instructions (at the top: gate/up
- * 1 % shorter, down 3 % longer) */
-#define NATIVE_WEIGHTS_FIRST_OF(bytes) (bytes)
 #define NATIVE_THREADS (NATIVE_WAVES * WAVE)
 
 /* memory into registers, 16 bytes or one byte a lane: the address is a base common to the wavefront plus the lane's own
@@ -94,19 +93,18 @@ struct native_chain {
     static constexpr uint32_t TILES = MATRICES * STRIP;
     static constexpr uint32_t STEP_BYTES = BYTES ? BYTE_STEP_BYTES : NIBBLE_STEP_BYTES;
     static constexpr uint32_t HALVES = STEP_BYTES / 1024u;
-    static constexpr uint32_t WAVE_BLOCKS = COLUMN_BLOCKS / NATIVE_WAVES;     /* column blocks a wavefront brings and prepares */
+    static constexpr uint32_t WAVE_BLOCKS = COLUMN_BLOCKS / NATIVE_WAVES;     /* column blocks whose scale words a wavefront brings */
     static constexpr uint32_t VECTOR_BYTES = COLUMN_BLOCKS * 2048u;            /* a K step of the block's columns' codes */
     static constexpr uint32_t STAGE_BYTES = VECTOR_BYTES;
     static constexpr uint32_t SCALE_STEPS = 4u; /* K steps whose scale words of the columns come together */
     static constexpr uint32_t CHUNK_BYTES = COLUMN_BLOCKS * 16u * SCALE_STEPS * 4u; /* [column][step of the chunk] */
     static constexpr uint32_t SCALES_AT = DEPTH * STAGE_BYTES; /* two chunks behind the stages: one in use, the next on its way */
     static constexpr uint32_t WINDOW_BYTES = SCALES_AT + 2u * CHUNK_BYTES;
-    /* loads of a wavefront for a step's columns of LIVE column blocks: groups of eight columns (one-byte weights: a wavefront
-     * brings the groups wave, wave + 4, ... that LIVE blocks need; 4-bit weights: the two of its own block, which it also
-     * prepares), and one of scale words */
+    /* loads of a wavefront for a step's columns of LIVE column blocks: groups of eight columns (the groups wave, wave + 4, ...
+     * that LIVE blocks need), and one of scale words */
     static constexpr uint32_t groups_of(uint32_t live)
     {
-        return BYTES ? (live + 1u) / 2u : 2u * WAVE_BLOCKS;
+        return (live + 1u) / 2u;
     }
     static constexpr uint32_t vector_loads(uint32_t live)
     {
@@ -132,7 +130,9 @@ struct native_chain {
     const unsigned char *words[MATRICES], *scales[MATRICES], *codes, *exponents;
     uint32_t step_stride, scale_stride; /* from a tile's K step to its next; from a group's scale words to the next group's */
     uint32_t window, wave, tile_bytes, group_bytes, word_offset, scale_offset[BYTES && !B128 ? STRIP : 1], code_shift, codes_offset[2u * WAVE_BLOCKS], exponents_offset[WAVE_BLOCKS];
-    uint32_t vector_at[BYTES ? 8 : 4], vector_scale_at, operand_at, scale_shift, last_step, lane_of;
+    /* 4-bit weights: strips of four tiles have no registers for a place a piece, and add three times a column block instead */
+    static constexpr bool PIECES_HELD = TILES == 8u;
+    uint32_t vector_at[BYTES ? 8 : PIECES_HELD ? 4 : 1], vector_scale_at, scale_shift, last_step, lane_of;
 
     template <typename T>
     __device__ static __forceinline__ T lds_read(uint32_t address)
@@ -160,7 +160,7 @@ struct native_chain {
     /* the group of eight columns that is this wavefront's part `part` */
     __device__ __forceinline__ static uint32_t group_of(uint32_t wave_index, uint32_t part)
     {
-        return BYTES ? wave_index + NATIVE_WAVES * part : 2u * WAVE_BLOCKS * wave_index + part;
+        return wave_index + NATIVE_WAVES * part;
     }
 
     /* the block's columns of K step `at` into stage `stage`, this wavefront's groups; and one load of scale words: the
@@ -235,28 +235,6 @@ struct native_chain {
         }
     }
 
-    /* 4-bit weights: this wavefront's column blocks of a stage, from the codes as they landed (a column's 128 bytes in the
-     * order the quantizer writes them) to the B operand, in place: [half of the operand][lane][16 bytes]; only this wavefront
-     * touches them before the next barrier */
-    __device__ __forceinline__ void prepare_columns(uint32_t stage) const
-    {
-#pragma unroll
-        for (uint32_t i = 0; i < WAVE_BLOCKS; i++) {
-            uint32_t at = window + stage * STAGE_BYTES + (wave * WAVE_BLOCKS + i) * 2048u;
-            asm volatile("" : "+s"(at));
-            int8_vector b;
-#pragma unroll
-            for (uint32_t part = 0; part < 4u; part++) {
-                const uint2_t pair = lds_read<uint2_t>(at + vector_at[part]);
-                b[2u * part] = (int)__builtin_amdgcn_perm(pair.y, pair.x, 0x05010400u);
-                b[2u * part + 1u] = (int)__builtin_amdgcn_perm(pair.y, pair.x, 0x07030602u);
-            }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); /* every lane has read before any lane writes */
-            lds_write<uint4_t>(at + operand_at, (uint4_t){(uint32_t)b[0], (uint32_t)b[1], (uint32_t)b[2], (uint32_t)b[3]});
-            lds_write<uint4_t>(at + operand_at + 1024u, (uint4_t){(uint32_t)b[4], (uint32_t)b[5], (uint32_t)b[6], (uint32_t)b[7]});
-        }
-    }
-
     /* the scale words of step `step` of the columns, this lane's part aside */
     __device__ __forceinline__ uint32_t scales_of(uint32_t step) const
     {
@@ -277,38 +255,58 @@ struct native_chain {
         }
     }
 
-    /* one K step of LIVE column blocks from a stage's columns and a set of weight registers; `between` runs behind the
-     * middle column block's matrix instructions */
-    template <uint32_t LIVE, typename BETWEEN>
-    __device__ __forceinline__ void consume(uint32_t stage, uint32_t step, const slot &set, float4_t (&chain)[TILES][COLUMN_BLOCKS], BETWEEN between) const
+    /* 4-bit weights: a column block's codes, read from the stage as they landed (a column's 128 bytes in the order the
+     * quantizer writes them), and the B operand of them */
+    __device__ static constexpr uint32_t piece_of(uint32_t part) /* pieces 0, 1, 4 and 5 from the lane's first: bits 4 and 6 of the place */
     {
-        uint32_t base = window + stage * STAGE_BYTES, scales = window + scales_of(step);
-        asm volatile("" : "+s"(base), "+s"(scales));
-        uint32_t b_at = base + operand_at, b_scale_at = scales + vector_scale_at;
-        asm volatile("" : "+v"(b_at), "+v"(b_scale_at));
+        return 16u * (part % 2u) + 64u * (part / 2u);
+    }
+
+    __device__ __forceinline__ void read_pieces(uint32_t at, uint32_t scales, uint32_t j, uint2_t (&pieces)[4], uint32_t &scale_b) const
+    {
+        uint32_t first = vector_at[0];
+        if constexpr (!PIECES_HELD) {
+            asm volatile("" : "+v"(first)); /* anew for every block: the compiler keeps no sum of it */
+        }
+#pragma unroll
+        for (uint32_t part = 0; part < 4u; part++) {
+            pieces[part] = lds_read<uint2_t>((PIECES_HELD ? vector_at[part] : first ^ piece_of(part)) + at + j * 2048u);
+        }
+        scale_b = lds_read<unsigned char>(vector_scale_at + scales + j * (16u * SCALE_STEPS * 4u));
+    }
+
+    __device__ static __forceinline__ int8_vector operand_of(const uint2_t (&pieces)[4])
+    {
+        int8_vector b;
+#pragma unroll
+        for (uint32_t part = 0; part < 4u; part++) {
+            b[2u * part] = (int)__builtin_amdgcn_perm(pieces[part].y, pieces[part].x, 0x05010400u);
+            b[2u * part + 1u] = (int)__builtin_amdgcn_perm(pieces[part].y, pieces[part].x, 0x07030602u);
+        }
+        return b;
+    }
+
+    /* one K step of LIVE column blocks from a stage's columns and a set of weight registers */
+    template <uint32_t LIVE>
+    __device__ __forceinline__ void consume(uint32_t stage, uint32_t step, const slot &set, float4_t (&chain)[TILES][COLUMN_BLOCKS]) const
+    {
         uint32_t scale_a[SCALE_LOADS];
 #pragma unroll
         for (uint32_t k = 0; k < SCALE_LOADS; k++) { /* two tiles a strip: the group's upper two tiles' codes down */
             scale_a[k] = set.scale[k] >> scale_shift;
         }
+        const uint32_t at = stage * STAGE_BYTES, scales = scales_of(step);
+        uint2_t pieces[LIVE][4];
+        uint32_t scale_b[LIVE];
         __builtin_amdgcn_s_setprio(1);
-        /* a column block's operand is read while the block before it is multiplied: two blocks' registers, not LIVE */
-        uint4_t low = lds_read<uint4_t>(b_at), high = lds_read<uint4_t>(b_at + 1024u);
-        uint32_t scale_b = lds_read<unsigned char>(b_scale_at);
+        read_pieces(at, scales, 0u, pieces[0], scale_b[0]);
 #pragma unroll
         for (uint32_t j = 0; j < LIVE; j++) {
-            const int8_vector b = {(int)low.x, (int)low.y, (int)low.z, (int)low.w, (int)high.x, (int)high.y, (int)high.z, (int)high.w};
-            const uint32_t scale_now = scale_b;
             asm volatile("" ::: "memory"); /* the reads below stay below the reads above, and above those of the next block */
-            if (j + 1u < LIVE) {
-                low = lds_read<uint4_t>(b_at + (j + 1u) * 2048u);
-                high = lds_read<uint4_t>(b_at + (j + 1u) * 2048u + 1024u);
-                scale_b = lds_read<unsigned char>(b_scale_at + (j + 1u) * (16u * SCALE_STEPS * 4u));
+            if (j + 1u < LIVE) { /* a column block's codes are read while the block before it is multiplied */
+                read_pieces(at, scales, j + 1u, pieces[j + 1u], scale_b[j + 1u]);
             }
-            multiply_tiles<0>(set, scale_a, b, scale_now, j, chain);
-            if (j == (LIVE - 1u) / 2u) {
-                between();
-            }
+            multiply_tiles<0>(set, scale_a, operand_of(pieces[j]), scale_b[j], j, chain);
         }
         __builtin_amdgcn_s_setprio(0);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); /* the stage is read before the next barrier */
@@ -387,7 +385,9 @@ struct native_chain {
     }
 
     /* how many loads may be outstanding at the top of a K step for its columns and weights to have landed: native_waits.h */
-    static constexpr bool WEIGHTS_FIRST = NATIVE_WEIGHTS_FIRST_OF(BYTES); /* inside a step: the weights asked for ahead of the columns */
+    /* inside a step: the weights asked for at its top, ahead of the barrier and the columns (in the middle of the matrix
+     * instructions 4-bit weights take the same time and 18 registers more, one-byte weights a quarter longer) */
+    static constexpr bool WEIGHTS_FIRST = true;
     template <uint32_t LIVE> using waits = native_waits<SLOTS, DEPTH, WEIGHTS_FIRST, vector_loads(LIVE), WEIGHT_LOADS>;
 
     /* s_waitcnt takes its count as a constant: one instruction a count that loads_behind can come to */
@@ -420,30 +420,22 @@ struct native_chain {
                 native_landed(held[k]);
             }
         }
-        const auto ask = [&]() {
+        const auto ask = [&]() { /* a function of its own: the compiler spills registers of the same lines without one */
             if (step + SLOTS - 1u < total) {
                 issue_weights(sets[(K + SLOTS - 1u) % SLOTS], step + SLOTS - 1u);
             }
         };
-        if constexpr (WEIGHTS_FIRST) {
-            ask(); /* into the set the step before this one used: nothing of the block's is waited for */
-        }
+        ask(); /* into the set the step before this one used: nothing of the block's is waited for */
         /* where the sets and the stages go round together the stage is a constant of the instance */
         const uint32_t stage = SLOTS % DEPTH == 0u ? K % DEPTH : step % DEPTH;
-        if constexpr (!BYTES) {
-            prepare_columns(stage);
-        }
-        __syncthreads(); /* every wavefront has read the step before; its columns of this one have landed and are prepared */
+        __syncthreads(); /* every wavefront has read the step before; its columns of this one have landed */
         if (step + DEPTH - 1u < total) {
             issue_vectors<LIVE>((stage + DEPTH - 1u) % DEPTH, step + DEPTH - 1u);
         }
-        /* 4-bit weights: the next weights are asked for in the middle of the step's matrix instructions (a launch 1.7 %
-         * shorter than asking ahead of them: the requests spread over the step); one-byte weights in the middle: a quarter
-         * slower */
-        if constexpr (WEIGHTS_FIRST) {
+        if constexpr (BYTES) {
             consume_bytes<LIVE>(stage, step, sets[K], held, step - round, chain);
         } else {
-            consume<LIVE>(stage, step, sets[K], chain, ask);
+            consume<LIVE>(stage, step, sets[K], chain);
         }
     }
 
@@ -584,13 +576,11 @@ struct native_chain {
             }
         } else {
 #pragma unroll
-            for (uint32_t part = 0; part < 4u; part++) {
-                const uint32_t piece = 4u * (part / 2u) + part % 2u + 2u * (g % 2u);
-                vector_at[part] = group_bytes + 16u * (8u * column + (piece ^ column ^ (o / 8u))) + 8u * (g / 2u);
+            for (uint32_t part = 0; part < (PIECES_HELD ? 4u : 1u); part++) {
+                vector_at[part] = (window + group_bytes + 16u * (8u * column + (2u * (g % 2u) ^ column ^ (o / 8u))) + 8u * (g / 2u)) ^ piece_of(part);
             }
         }
-        vector_scale_at = (BYTES ? window : 0u) + 4u * SCALE_STEPS * o + (B128 ? 0u : g);
-        operand_at = 16u * lane;
+        vector_scale_at = window + 4u * SCALE_STEPS * o + (B128 ? 0u : g);
         scale_shift = 8u * (tile0 % 4u);
     }
 };

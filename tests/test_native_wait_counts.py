@@ -23,6 +23,8 @@ INSTANCES = {
     "E4M3_BLOCK128 down (2 tiles of two halves, 1 scale)": (3, 3, True, 5, 5),
     **{"one-byte gate/up, %d loads of columns" % loads: (2, 2, True, loads, 4) for loads in (2, 3, 4, 5)},
     **{"one-byte down, %d loads of columns" % loads: (3, 3, True, loads, 4) for loads in (2, 3, 4, 5)},
+    **{"E2M1, weights ahead of the columns: %d sets, %d loads of columns, %d of weights" % case: (case[0], 2, True, case[1], case[2])
+       for case in ((2, 2, 10), (2, 3, 10), (3, 2, 6), (3, 3, 6), (3, 2, 5), (3, 3, 5))},
     "four sets of weight registers (measured, not kept)": (4, 3, True, 5, 6),
     "six sets": (6, 3, True, 5, 6),
     "weights behind the columns at three stages": (4, 3, False, 5, 6),
