@@ -130,11 +130,11 @@ __device__ static __forceinline__ void trunk_linear_quantized_wide(const struct 
 /* grid (ceil(output_size[0] / 128) + ceil(output_size[1] / 128), ceil(row_count / 64)), block 256 */
 __device__ static __forceinline__ void trunk_linear_quantized_interleaved(const struct trunk_linear_quantized_arguments &arguments, unsigned char *arena)
 {
-    typedef wide_chain<1, true, 2u, 2u> chain_type;
+    typedef wide_chain<1, true, 2u> chain_type;
     constexpr uint32_t TILES = chain_type::TILES, STRIP = chain_type::STRIP, STRIP_OUTPUTS = STRIP * 16u;
     static_assert(chain_type::WINDOW_BYTES == TRUNK_INTERLEAVED_WINDOW_BYTES && WIDE_WAVES * STRIP_OUTPUTS == TRUNK_INTERLEAVED_BLOCK_OUTPUTS &&
                       WIDE_TILE_PAIRS == TRUNK_INTERLEAVED_ROWS, "the window and the block the host asks for are the kernel's");
-    extern __shared__ __attribute__((aligned(16))) unsigned char wide_window[];
+    extern __shared__ __attribute__((aligned(128))) unsigned char wide_window[];
     uint32_t matrix, block;
     trunk_matrix_of(arguments, blockIdx.x, TRUNK_INTERLEAVED_BLOCK_OUTPUTS, matrix, block);
     const uint32_t outputs = arguments.output_size[matrix];
@@ -148,13 +148,14 @@ __device__ static __forceinline__ void trunk_linear_quantized_interleaved(const 
         const uint32_t column = 8u * (2u * wave + part) + lane / 8u;
         code_vectors[part] = first_row + (column < row_count ? column : 0u);
     }
-    const uint32_t scale_column = 16u * wave + lane % 16u;
+    const uint32_t scale_column = 16u * wave + lane / 4u;
     const uint32_t exponent_vector = first_row + (scale_column < row_count ? scale_column : 0u);
     chain_type chain_of;
     const unsigned char *const matrices[1] = {arena + arguments.weights_offset[matrix]};
     uint32_t tile0 = 0;
     chain_of.place(matrices, outputs, arguments.input_size, block, arena + arguments.codes_offset, arena + arguments.exponents_offset,
-                   code_vectors, exponent_vector, (uint32_t)(uintptr_t)(lds_pointer)wide_window, wave, lane, tile0);
+                   code_vectors, exponent_vector, (uint32_t)(uintptr_t)(lds_pointer)wide_window,
+                   (uint32_t)(uintptr_t)(lds_pointer)wide_window + chain_type::STAGES_BYTES, wave, lane, tile0);
     float4_t chain[TILES][WIDE_COLUMN_BLOCKS];
 #pragma unroll
     for (uint32_t t = 0; t < TILES; t++) {

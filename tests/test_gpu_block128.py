@@ -177,6 +177,12 @@ def test_wide_equals_the_job_table_kernels_byte_for_byte(amd, card, hidden, inne
     assert np.array_equal(wide_values[:pairs * inner * 2], hidden_values[:pairs * inner * 2])
 
 
+@pytest.mark.parametrize("hidden,inner", [(512, 384), (640, 896), (1152, 1024)])
+def test_wide_chunks_of_scale_words(amd, card, hidden, inner):
+    """The columns' float32 scales come four K steps at a time: chains that end inside a chunk, with one, at its first step."""
+    test_wide_equals_the_job_table_kernels_byte_for_byte(amd, card, hidden, inner, 2, 100, 100)
+
+
 def test_wide_layer_against_oracle(amd, card):
     say("block128 wide layer against the oracle")
     from test_gpu_router_wide import oracle_wide

@@ -104,6 +104,16 @@ def test_wide_equals_the_job_table_kernels_byte_for_byte(amd, card, hidden, inne
             assert np.all(b.reshape(-1)[pairs * per:] == 0xEE), name
 
 
+@pytest.mark.parametrize("hidden,inner,picks,rows,fmt", [
+    # the columns' scale words come four K steps at a time: chains that end inside a chunk, with one, at its first step
+    *[(hidden, inner, 2, 100, fmt) for hidden, inner in ((512, 384), (640, 896), (1152, 1024)) for fmt in (E2M1, E4M3)],
+    # one expert's pairs: every number of live column blocks
+    *[(640, 256, 1, rows, -fmt) for rows in (9, 16, 30, 41, 64, 70) for fmt in (E2M1, E4M3)],
+])
+def test_wide_chunks_of_scale_words(amd, card, hidden, inner, picks, rows, fmt):
+    test_wide_equals_the_job_table_kernels_byte_for_byte(amd, card, hidden, inner, 64, picks, rows, rows, fmt)
+
+
 def test_wide_layer_against_oracle(amd, card):
     """The whole layer in its wide form (projection, wide select, quantizer, wide gate/up, wide down, row sum) against
     the CPU oracle's layer of the same picks."""
