@@ -297,7 +297,10 @@ ANEMONE_KERNEL(EXL3_TCP_KERNEL_FILE, exl3_tcp_operands_thin, exl3_tcp_record);
  * read and its first operand is decoded in their shadow, where both stood bare behind a barrier at the step's end.
  * 4096 rows of 4096 x 2048 x 256 experts, Zipf(1.1) loads, builds in turns on one card: gate/up 1525 -> 1475 us, down
  * 855 -> 815. The addresses are kept as a base common to the wavefront and one offset a lane, which makes the registers
- * for that (24 spilled with an address a lane, 2 now, neither in the loop over the steps).
+ * for that (24 spilled with an address a lane, 2 now, neither in the loop over the steps). A wavefront's priority at the
+ * issue rises through its step: without it the two wavefronts of a SIMD run into the same phases (gate/up 1460 -> 1420 us,
+ * down 815 -> 800; 600 rows of even loads 725 -> 672 and 377 -> 356; raised at half the step alone: 1420, 783, 703, 370;
+ * falling instead: no shorter).
  */
 /* 16 bytes a lane from memory straight into LDS (lane L lands at lds_base + 16 L), no register in between. Written as
  * assembly: the compiler keeps no book on it, so the wait that ends a step (every load of the wavefront, then the block's
@@ -450,6 +453,17 @@ tcp_wave_gemm(const uint32_t *__restrict__ codes, uint32_t out_tiles, uint32_t s
             const uint32_t h = k % 2u;
             if (k % 2u == 0u && k + 2u < 8u) {
                 read_operands(parity, k + 2u);
+            }
+            /* the further a wavefront is into its step, the more its instructions go first: the other block's wavefront on the SIMD
+             * falls behind to where its decoding meets this one's products, and this one reaches its barrier */
+            if (k == 0u) {
+                __builtin_amdgcn_s_setprio(0);
+            } else if (k == 2u) {
+                __builtin_amdgcn_s_setprio(1);
+            } else if (k == 4u) {
+                __builtin_amdgcn_s_setprio(2);
+            } else if (k == 6u) {
+                __builtin_amdgcn_s_setprio(3);
             }
             if (k == 6u) {
                 /* every load of this wavefront has landed (the next step's codes and its share of the next stage), and it
