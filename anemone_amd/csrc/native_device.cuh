@@ -298,13 +298,21 @@ struct native_chain {
         const uint32_t at = stage * STAGE_BYTES, scales = scales_of(step);
         uint2_t pieces[LIVE][4];
         uint32_t scale_b[LIVE];
-        __builtin_amdgcn_s_setprio(1);
         read_pieces(at, scales, 0u, pieces[0], scale_b[0]);
 #pragma unroll
         for (uint32_t j = 0; j < LIVE; j++) {
             asm volatile("" ::: "memory"); /* the reads below stay below the reads above, and above those of the next block */
             if (j + 1u < LIVE) { /* a column block's codes are read while the block before it is multiplied */
                 read_pieces(at, scales, j + 1u, pieces[j + 1u], scale_b[j + 1u]);
+            }
+            /* the further a wavefront is into its step, the more its instructions go first: the two of a SIMD then meet in
+             * different phases (gate/up 1115 -> 1087 us at 8192 rows; one priority through the matrix instructions, or none: 1115) */
+            if (j == 1u) {
+                __builtin_amdgcn_s_setprio(1);
+            } else if (j == 2u) {
+                __builtin_amdgcn_s_setprio(2);
+            } else if (j == 3u) {
+                __builtin_amdgcn_s_setprio(3);
             }
             multiply_tiles<0>(set, scale_a, operand_of(pieces[j]), scale_b[j], j, chain);
         }
