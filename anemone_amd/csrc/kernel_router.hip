@@ -240,6 +240,17 @@ extern "C" __global__ void __launch_bounds__(PROJECTION_TILE_THREADS, 3) /* thre
         for (uint32_t i = 0; i < 4u; i++) { /* a group of 32 inputs: eight instructions, each one input further on the four chains it takes */
             const uint32_t w_words[4] = {w_now.x, w_now.y, w_now.z, w_now.w}, x_words[4] = {x_now.x, x_now.y, x_now.z, x_now.w};
             float w_values[8], x_values[8];
+            /* the further a wavefront is into its stage, the more its instructions go first: the three of a SIMD then wait for LDS
+             * and the barrier at different times (8192 rows of 4096 inputs by 256 experts 219 -> 210 us, 2048 rows 66 -> 62) */
+            if (i == 0u) {
+                __builtin_amdgcn_s_setprio(0);
+            } else if (i == 1u) {
+                __builtin_amdgcn_s_setprio(1);
+            } else if (i == 2u) {
+                __builtin_amdgcn_s_setprio(2);
+            } else {
+                __builtin_amdgcn_s_setprio(3);
+            }
             projection_convert(w_words, w_values);
             projection_convert(x_words, x_values);
             __builtin_amdgcn_sched_barrier(0);
