@@ -12,7 +12,7 @@
  * quantization, the router's scores, the select; and streams -> mixes -> post, comb and the site's pre. Blocks of
  * width / 8 threads (a row's block of the mix finish; a quarter of 256 threads of it is the dense product's block) take
  * a ticket each and their part by it:
- *     tickets 0 .. rows - 1           a row: its input, its quantization; publishes rows_ready
+ *     tickets 0 .. rows - 1           a row: its input; publishes rows_ready; its quantization
  *     then site_front_mix_blocks      SITE_FRONT_MIX_OUTPUTS mixes a quarter, every row; publishes arrived; the last to
  *                                     arrive waits for rows_ready = rows (the rows' blocks have read the pre) and forms
  *                                     every row's post, comb and pre, sixteen threads a row
@@ -21,6 +21,11 @@
  * A wait is thread 0 polling the counter (agent scope) with a sleep between polls, at most SITE_FRONT_WAIT_POLLS times;
  * a block whose wait runs out counts itself in gave_up, skips its part and leaves: every wave of the grid ends. The
  * last block to leave (departed) clears the counters.
+ *
+ * What a front costs is its two serial chains, so what nobody in it waits for stands behind what somebody does: a row is
+ * published before it is quantized, the scores' blocks ask for a word of every line of their weights before they wait for
+ * the rows, and the dense product's sums meet by the lanes' own exchanges (ffn_front_8 at 5 rows of 4096 by 256 experts 23.7
+ * -> 22.0 us, ffn_front_1 15.7 -> 13.8; asking for the mixes' weights ahead likewise: 1 us longer at 1 and 5 rows).
  *
  * The two halves need no tickets and no waits: the input front is a row a block (grid rows); the coefficient front is the
  * mix project's blocks (grid site_front_mix_blocks), the last of which to publish arrived forms post, comb and pre and
@@ -94,13 +99,11 @@ __device__ static __forceinline__ bool front_wait(uint32_t *counter, uint32_t ta
     return *word != 0u;
 }
 
-/* a row's block: the row's input, then its quantization, a thread four values at a time */
-__device__ static __forceinline__ void front_row(const struct site_front_arguments &arguments, const struct hyper_finish_arguments &finish,
-                                                 unsigned char *arena, uint32_t row, uint32_t thread, uint32_t threads, float *group_sums)
+/* a row's quantization, a thread four values at a time, by the block that wrote the row */
+__device__ static __forceinline__ void front_row_quantize(const struct site_front_arguments &arguments, unsigned char *arena, uint32_t row,
+                                                          uint32_t thread, uint32_t threads)
 {
     const uint32_t width = threads * HYPER_VALUES_PER_THREAD;
-    hyper_row_input_body(finish, arena, row, thread, threads, group_sums);
-    __syncthreads(); /* the row is written: this block's threads read it */
     const struct activation_quantize_arguments quantize = {arguments.hidden_offset, arguments.codes_offset, arguments.exponents_offset,
                                                            arguments.operands_offset, width};
     for (uint32_t q = thread; q < width / 4u; q += threads) {
@@ -167,9 +170,10 @@ __device__ static __forceinline__ void site_front(const struct site_front_argume
                                                   arguments.base_offset, arguments.post_offset, arguments.comb_offset,
                                                   arguments.norm_weight_offset, arguments.hidden_offset};
     if (ticket < rows) {
-        /* a row: its input, then its quantization, a thread four values at a time */
-        front_row(arguments, finish, arena, ticket, thread, threads, lds.group_sums);
+        /* a row: its input, which the blocks of the scores wait for, then its quantization, which no block of this launch does */
+        hyper_row_input_body(finish, arena, ticket, thread, threads, lds.group_sums);
         front_publish<true, false>(&scratch->rows_ready, thread, &word);
+        front_row_quantize(arguments, arena, ticket, thread, threads);
     } else if (ticket < rows + mix_blocks) {
         /* the mix project: float32 [24][4 width] by the streams as rows of 4 width values, with the row's scale */
         front_mix_project<ROWS>(arguments, arena, rows, ticket - rows, thread, threads, lds.mixes);
@@ -208,6 +212,13 @@ __device__ static __forceinline__ void site_front(const struct site_front_argume
         dense.output_type = DENSE_FLOAT32;
         dense.output_scale = 1.0f;
         const uint32_t groups = experts / SITE_FRONT_SCORE_OUTPUTS, group = (ticket - rows - mix_blocks) * quarters + quarter;
+        if (in_quarter && group < groups) { /* a word of every line of the quarter's weights, on their way while the rows are formed */
+            const uint64_t first = arguments.router_weights_offset + (uint64_t)group * SITE_FRONT_SCORE_OUTPUTS * width * 2u;
+            for (uint32_t line = quarter_thread; line < SITE_FRONT_SCORE_OUTPUTS * width * 2u / 128u; line += DENSE_THREADS_VALUE) {
+                const uint32_t touched = *(const uint32_t *)(arena + first + line * 128u);
+                asm volatile("" ::"v"(touched));
+            }
+        }
         if (front_wait<true>(&scratch->rows_ready, rows, thread, &word, &scratch->gave_up)) {
             dense_linear_body<DENSE_BFLOAT16, ROWS, SITE_FRONT_SCORE_OUTPUTS>(dense, arena, (const uint16_t *)(arena + dense.rows_offset),
                                                                               group * SITE_FRONT_SCORE_OUTPUTS, 0u, quarter_thread,
@@ -239,7 +250,9 @@ __device__ static __forceinline__ void input_front(const struct site_front_argum
                                                   arguments.scratch_offset + offsetof(struct site_front_scratch, mixes), arguments.scale_offset,
                                                   arguments.base_offset, arguments.post_offset, arguments.comb_offset,
                                                   arguments.norm_weight_offset, arguments.hidden_offset};
-    front_row(arguments, finish, arena, blockIdx.x, threadIdx.x, blockDim.x, group_sums);
+    hyper_row_input_body(finish, arena, blockIdx.x, threadIdx.x, blockDim.x, group_sums);
+    __syncthreads(); /* the row is written: this block's threads read it */
+    front_row_quantize(arguments, arena, blockIdx.x, threadIdx.x, blockDim.x);
 }
 
 /* its second half: the mix project's blocks; the last to publish forms every row's post, comb and pre */
