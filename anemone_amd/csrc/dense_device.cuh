@@ -20,27 +20,6 @@ __device__ static __forceinline__ float dense_reciprocal_root(float operand)
     return (float)(1.0 / __dsqrt_rn((double)operand));
 }
 
-/* a value plus that of the lane `distance` away in a group of DENSE_GROUP_LANES, for distances 16, 8, 4, 2 and 1: by the lanes'
- * own exchanges (a shuffle is an LDS round trip, and a thread of 8 rows has up to 72 sums of five distances each: 2000 rows
- * of 16384 inputs by 24 outputs 57 -> 51.5 us) */
-template <uint32_t distance>
-__device__ static __forceinline__ float dense_add_lane(float value)
-{
-    if constexpr (distance == 16u) { /* rows of sixteen lanes change places: one of the two results is the lane's own */
-        const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(value), __float_as_uint(value), false, false);
-        return __fadd_rn(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
-    } else if constexpr (distance == 4u) { /* four lanes on, or four back: banks of four lanes in turn */
-        const int bits = (int)__float_as_uint(value);
-        const int on = __builtin_amdgcn_update_dpp(bits, bits, 0x104, 0xF, 0x5, false); /* row_shl:4 */
-        return __fadd_rn(value, __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(on, bits, 0x114, 0xF, 0xA, false))); /* row_shr:4 */
-    } else {
-        static_assert(distance == 8u || distance == 2u || distance == 1u, "a distance inside a group of 32 lanes");
-        constexpr int control = distance == 8u ? 0x128 : distance == 2u ? 0x4E : 0xB1; /* row_ror:8, quad_perm:[2,3,0,1], [1,0,3,2] */
-        const int bits = (int)__float_as_uint(value);
-        return __fadd_rn(value, __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(bits, bits, control, 0xF, 0xF, false)));
-    }
-}
-
 template <uint32_t distance, uint32_t ROWS, uint32_t OUTPUTS>
 __device__ static __forceinline__ void dense_add_lanes(float (&chain)[OUTPUTS][ROWS], float (&squares)[ROWS], bool scaled)
 {
@@ -48,10 +27,10 @@ __device__ static __forceinline__ void dense_add_lanes(float (&chain)[OUTPUTS][R
     for (uint32_t r = 0; r < ROWS; r++) {
 #pragma unroll
         for (uint32_t o = 0; o < OUTPUTS; o++) {
-            chain[o][r] = dense_add_lane<distance>(chain[o][r]);
+            chain[o][r] = lanes_sum<distance>(chain[o][r]);
         }
         if (scaled) {
-            squares[r] = dense_add_lane<distance>(squares[r]);
+            squares[r] = lanes_sum<distance>(squares[r]);
         }
     }
 }
@@ -134,7 +113,8 @@ __device__ static __forceinline__ void dense_linear_body(const struct dense_line
         }
     }
     const uint32_t group = thread / DENSE_GROUP_LANES, lane = thread % DENSE_GROUP_LANES;
-    /* each chain's additions are the definition's: the distance halving from 16 */
+    /* each chain's additions are the definition's: the distance halving from 16. By the lanes' own exchanges: a thread of 8 rows
+     * has up to 72 sums of five distances each (2000 rows of 16384 inputs by 24 outputs, against shuffles: 57 -> 51.5 us) */
     dense_add_lanes<16u>(chain, squares, scaled);
     dense_add_lanes<8u>(chain, squares, scaled);
     dense_add_lanes<4u>(chain, squares, scaled);

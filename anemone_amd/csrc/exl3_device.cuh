@@ -97,6 +97,44 @@ __device__ static __forceinline__ float det_silu(float gate)
     return __fdiv_rn(gate, __fadd_rn(1.0f, det_exp_sequence(x)));
 }
 
+/* A lane's value and that of the lane `distance` away (lane ^ distance), in some order: for operations whose two sides may
+ * change places. By the lanes' own exchanges: a shuffle is an LDS round trip of some 120 cycles, and the sums and maxima of a
+ * small launch are a chain of them. Every lane of a row of sixteen (of two rows for distance 16) calls. */
+struct lane_pair {
+    float first, second;
+};
+
+template <uint32_t distance>
+__device__ static __forceinline__ lane_pair lanes_apart(float value)
+{
+    const int bits = (int)__float_as_uint(value);
+    if constexpr (distance == 16u) { /* two rows change places */
+        const auto rows = __builtin_amdgcn_permlane16_swap((uint32_t)bits, (uint32_t)bits, false, false);
+        return {__uint_as_float(rows[0]), __uint_as_float(rows[1])};
+    } else if constexpr (distance == 4u) { /* four lanes on, or four back: banks of four lanes in turn */
+        const int on = __builtin_amdgcn_update_dpp(bits, bits, 0x104, 0xF, 0x5, false); /* row_shl:4 */
+        return {value, __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(on, bits, 0x114, 0xF, 0xA, false))}; /* row_shr:4 */
+    } else {
+        static_assert(distance == 8u || distance == 2u || distance == 1u, "a distance inside a group of 32 lanes");
+        constexpr int control = distance == 8u ? 0x128 : distance == 2u ? 0x4E : 0xB1; /* row_ror:8, quad_perm:[2,3,0,1], [1,0,3,2] */
+        return {value, __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(bits, bits, control, 0xF, 0xF, false))};
+    }
+}
+
+template <uint32_t distance>
+__device__ static __forceinline__ float lanes_sum(float value)
+{
+    const lane_pair pair = lanes_apart<distance>(value);
+    return __fadd_rn(pair.first, pair.second);
+}
+
+template <uint32_t distance>
+__device__ static __forceinline__ float lanes_largest(float value)
+{
+    const lane_pair pair = lanes_apart<distance>(value);
+    return fmaxf(pair.first, pair.second);
+}
+
 /* The 128-point transform: seven stages, the distance doubling from 1; a pair (lower, upper) becomes (lower + upper, lower -
  * upper), each rounded once. No normalisation here. Two lay-outs: a block across a wavefront, two values a lane
  * (wave_hadamard128: the fewest instructions for one block), and across a row of sixteen lanes, eight consecutive values a

@@ -44,10 +44,7 @@ extern "C" __global__ void __launch_bounds__(LINEAR_ELEMENT_THREADS)
     const uint32_t bits[4] = {near_pair & 0xFFFFu, near_pair >> 16, far_pair & 0xFFFFu, far_pair >> 16};
     float largest = fmaxf(fmaxf(fabsf(bf16_to_float((uint16_t)bits[0])), fabsf(bf16_to_float((uint16_t)bits[1]))),
                           fmaxf(fabsf(bf16_to_float((uint16_t)bits[2])), fabsf(bf16_to_float((uint16_t)bits[3]))));
-#pragma unroll
-    for (uint32_t distance = 16u; distance != 0u; distance >>= 1u) {
-        largest = fmaxf(largest, __shfl_xor(largest, (int)distance, 32));
-    }
+    largest = lanes_largest<1u>(lanes_largest<2u>(lanes_largest<4u>(lanes_largest<8u>(lanes_largest<16u>(largest)))));
     const float scale = __fdiv_rn(fmaxf(largest, 1e-4f), 448.0f);
     uint32_t code[4];
 #pragma unroll

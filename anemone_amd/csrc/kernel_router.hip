@@ -109,11 +109,8 @@ __device__ static __forceinline__ void router_projection_block(const struct rout
     for (uint32_t r = 0; r < PROJECTION_ROWS; r++) {
         float even = __fadd_rn(0.0f, chain[r][0]), odd = __fadd_rn(0.0f, chain[r][1]);
         /* chain c + distance lies distance / 2 threads on, for the distances 16, 8, 4, 2 */
-#pragma unroll
-        for (uint32_t distance = 8u; distance != 0u; distance >>= 1u) {
-            even = __fadd_rn(even, __shfl_down(even, distance, 16));
-            odd = __fadd_rn(odd, __shfl_down(odd, distance, 16));
-        }
+        even = lanes_sum<1u>(lanes_sum<2u>(lanes_sum<4u>(lanes_sum<8u>(even))));
+        odd = lanes_sum<1u>(lanes_sum<2u>(lanes_sum<4u>(lanes_sum<8u>(odd))));
         const float sum = __fadd_rn(even, odd); /* distance 1: chain 0 + chain 1 */
         if (pair == 0u && expert < arguments.expert_count && first_row + r < arguments.row_count) {
             ((float *)(arena + arguments.output_offset))[(uint64_t)(first_row + r) * arguments.expert_count + expert] = __fadd_rn(0.0f, sum);

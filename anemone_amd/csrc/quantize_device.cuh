@@ -91,10 +91,7 @@ __device__ static __forceinline__ void quantize_value(uint32_t bits, uint32_t in
                                                       uint16_t *operands)
 {
     float largest = fabsf(bf16_to_float((uint16_t)bits));
-#pragma unroll
-    for (uint32_t distance = 16u; distance != 0u; distance >>= 1u) {
-        largest = fmaxf(largest, __shfl_xor(largest, (int)distance, 32));
-    }
+    largest = lanes_largest<1u>(lanes_largest<2u>(lanes_largest<4u>(lanes_largest<8u>(lanes_largest<16u>(largest)))));
     const uint32_t code_exponent = quantize_exponent_code(largest);
     uint32_t code, operand;
     quantize_code(bits, code_exponent, code, operand);
@@ -123,10 +120,7 @@ __device__ static __forceinline__ void activation_quantize_body(const struct act
     const uint32_t bits[4] = {near_pair & 0xFFFFu, near_pair >> 16, far_pair & 0xFFFFu, far_pair >> 16}; /* values +0, +1, +8, +9 */
     float largest = fmaxf(fmaxf(fabsf(bf16_to_float((uint16_t)bits[0])), fabsf(bf16_to_float((uint16_t)bits[1]))),
                           fmaxf(fabsf(bf16_to_float((uint16_t)bits[2])), fabsf(bf16_to_float((uint16_t)bits[3]))));
-#pragma unroll
-    for (uint32_t distance = 4u; distance != 0u; distance >>= 1u) {
-        largest = fmaxf(largest, __shfl_xor(largest, (int)distance, 8));
-    }
+    largest = lanes_largest<1u>(lanes_largest<2u>(lanes_largest<4u>(largest)));
     const uint32_t code_exponent = quantize_exponent_code(largest);
     /* the word's bytes j = 0 .. 3 hold values +0 (j = 0), +8 (1), +1 (2), +9 (3); its operands' halfwords 2 r + h hold
      * value + h + 8 r */
