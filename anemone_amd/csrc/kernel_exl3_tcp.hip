@@ -28,7 +28,7 @@
 #define TCP_COLUMN_BLOCKS (EXL3_TCP_CHUNK_PAIRS / 16u) /* of sixteen columns: two a block of the matrix instruction's 32 */
 #define TCP_STEP_INPUTS 64u
 #define TCP_DIES 8u         /* the card's dies (XCDs), each with a level-2 cache of its own: blocks are dealt to them in turn */
-#define TCP_BATCH 4u        /* columns the element-wise launches take at a time */
+#define TCP_BATCH 4u        /* columns, or slots of a row, the element-wise launches take at a time */
 #define TCP_THIN_PLACES 4u  /* places of a block of a thin call's element-wise launches: one a wavefront */
 #define TCP_WAVE_BLOCKS 4u  /* blocks of 128 channels a wavefront of an element-wise launch takes: a row of sixteen lanes each */
 
@@ -874,19 +874,37 @@ extern "C" __global__ void exl3_tcp_combine(struct exl3_tcp_record record, unsig
     const float *down = (const float *)(workspace + shape.layout.down);
     const float normalization = row_normalization(lane);
     float sum[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t slot = 0; slot < shape.picks; slot++) {
-        const struct router_pick pick = picks[slot];
-        const uint64_t place = place_of[row * shape.picks + slot];
-        const uint16_t *svh = (const uint16_t *)(arena + tcp_matrix_of(record, arena, pick.expert, 2u) +
-                                                 exl3_code_bytes(I, H, tcp_bits_x2(record, arena, pick.expert, 2u))) + I;
-        const float4_t *products = (const float4_t *)(down + place * H + channel);
-        const float4_t low = products[0], high = products[1];
-        float v[8] = {low[0], low[1], low[2], low[3], high[0], high[1], high[2], high[3]}, scale[8];
-        unpack_half8(*(const uint4_t *)(svh + channel), scale);
-        row_hadamard128(v, lane);
+    /* TCP_BATCH slots at a time: their products, and behind them their scales, are asked for together (a slot past the last
+     * repeats it and is not added; one at a time: 203 rows 12.0 us and not 10.7, 4096 rows 120 and not 117; eight: 12.3, 122) */
+    for (uint32_t first = 0; first < shape.picks; first += TCP_BATCH) {
+        float4_t low[TCP_BATCH], high[TCP_BATCH];
+        uint4_t scales[TCP_BATCH];
+        float weight[TCP_BATCH];
 #pragma unroll
-        for (uint32_t j = 0; j < 8u; j++) {
-            sum[j] = __fadd_rn(sum[j], __fmul_rn(__fmul_rn(row_normalized(v[j], normalization), scale[j]), pick.route_weight));
+        for (uint32_t i = 0; i < TCP_BATCH; i++) {
+            const uint32_t slot = first + i < shape.picks ? first + i : shape.picks - 1u;
+            const float4_t *products = (const float4_t *)(down + (uint64_t)place_of[row * shape.picks + slot] * H + channel);
+            low[i] = products[0];
+            high[i] = products[1];
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < TCP_BATCH; i++) {
+            const struct router_pick pick = picks[first + i < shape.picks ? first + i : shape.picks - 1u];
+            weight[i] = pick.route_weight;
+            scales[i] = *(const uint4_t *)((const uint16_t *)(arena + tcp_matrix_of(record, arena, pick.expert, 2u) +
+                                                              exl3_code_bytes(I, H, tcp_bits_x2(record, arena, pick.expert, 2u))) + I + channel);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < TCP_BATCH; i++) {
+            float v[8] = {low[i][0], low[i][1], low[i][2], low[i][3], high[i][0], high[i][1], high[i][2], high[i][3]}, scale[8];
+            unpack_half8(scales[i], scale);
+            row_hadamard128(v, lane);
+            if (first + i < shape.picks) {
+#pragma unroll
+                for (uint32_t j = 0; j < 8u; j++) {
+                    sum[j] = __fadd_rn(sum[j], __fmul_rn(__fmul_rn(row_normalized(v[j], normalization), scale[j]), weight[i]));
+                }
+            }
         }
     }
     float4_t *out = (float4_t *)((float *)(arena + record.output_offset) + (uint64_t)row * H + channel);

@@ -122,6 +122,12 @@ def test_prefill_layer_against_oracle(amd, card, hidden, inner, experts_n, picks
     assert error <= 4e-3
 
 
+@pytest.mark.parametrize("picks", [1, 3, 5, 6, 7])
+def test_prefill_slots_of_a_row(amd, card, picks):
+    """The combine takes a row's slots four at a time: counts that leave some of a batch over."""
+    test_prefill_layer_against_oracle(amd, card, 512, 256, 64, picks, 70, [2, 3, 4], 0.0)
+
+
 @pytest.mark.parametrize("hidden,inner,width_choices", [(512, 384, [2, 3, 4]), (128, 128, [40])])
 def test_thin_gemm_at_the_edges_of_its_blocks(amd, card, hidden, inner, width_choices):
     """A call of few pairs an expert (exl3_tcp_gemm_thin: blocks of 48 pairs, instances of one to three blocks of sixteen):
