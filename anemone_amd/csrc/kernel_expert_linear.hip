@@ -44,7 +44,7 @@ template <uint32_t S, bool BYTES, bool B128 = false, bool NATIVE = false>
 __device__ static __forceinline__ void expert_gate_up(const struct expert_gate_up_arguments &arguments,
                                                       unsigned char *arena, uint16_t *strip_hidden = nullptr)
 {
-    typedef strip_chain<2, BYTES, B128, NATIVE> chain_type;
+    typedef strip_chain<2, BYTES, B128, NATIVE, true> chain_type;
     constexpr uint32_t TILES = chain_type::TILES, STRIP = chain_type::STRIP;
     __shared__ __attribute__((aligned(16))) unsigned char window[S][chain_type::WINDOW_BYTES];
     static_assert(chain_type::WINDOW_BYTES >= TILES * WAVE * 16u, "a wavefront's sums fit its idle window");
@@ -130,7 +130,7 @@ template <uint32_t S, bool BYTES>
 __device__ static __forceinline__ void expert_gate_up_quantize(const struct expert_gate_up_quantize_arguments &arguments,
                                                                unsigned char *arena)
 {
-    typedef strip_chain<2, BYTES> chain_type;
+    typedef strip_chain<2, BYTES, false, false, true> chain_type;
     constexpr uint32_t STRIP_OUTPUTS = chain_type::STRIP * 16u;
     __shared__ uint16_t strip_hidden[LINEAR_MAXIMUM_ROWS][STRIP_OUTPUTS];
     __shared__ uint32_t routed[EXPERT_PRODUCER_MOST_PAIRS / 32u];
@@ -197,7 +197,7 @@ __device__ static __forceinline__ void expert_gate_up_quantize(const struct expe
 template <uint32_t S, bool BYTES, bool B128 = false, bool NATIVE = false>
 __device__ static __forceinline__ void expert_down(const struct expert_down_arguments &arguments, unsigned char *arena)
 {
-    typedef strip_chain<1, BYTES, B128, NATIVE> chain_type;
+    typedef strip_chain<1, BYTES, B128, NATIVE, true> chain_type;
     constexpr uint32_t TILES = chain_type::TILES, STRIP = chain_type::STRIP;
     __shared__ __attribute__((aligned(16))) unsigned char window[S][chain_type::WINDOW_BYTES];
     static_assert(chain_type::WINDOW_BYTES >= TILES * WAVE * 16u, "a wavefront's sums fit its idle window");

@@ -22,7 +22,9 @@
  * tiles are read with one or two 16-byte LDS reads and no arithmetic; the scale codes of 4-bit weights are a word a lane
  * for the strip's four tiles (a group of 64 outputs), its byte picked by the matrix instruction; with B128 the scales are
  * E4M3_BLOCK128's float32 words where they are. */
-template <uint32_t MATRICES, bool BYTES, bool B128 = false, bool NATIVE = false>
+/* ONCE: the launch reads a weight once (the experts' launches, but for an expert of more than eight rows; not the shared matrices
+ * of a step of several groups of rows), and asks for it as a stream */
+template <uint32_t MATRICES, bool BYTES, bool B128 = false, bool NATIVE = false, bool ONCE = false>
 struct strip_chain {
     static_assert(BYTES || !B128, "float32 scales go with one-byte weights");
     static constexpr uint32_t STRIP = BYTES ? 2u : 4u; /* tiles of a strip: 4 KB of every matrix a stage either way */
@@ -64,8 +66,13 @@ struct strip_chain {
             for (uint32_t n = 0; n < STRIP; n++) {
 #pragma unroll
                 for (uint32_t part = 0; part < TILE_LOADS; part++) {
-                    load_to_lds_16(words[m] + (uint64_t)n * tile_bytes + (uint64_t)at * STEP_BYTES + part * 1024u, piece_offset,
-                                   base + (m * STRIP + n) * STEP_BYTES + part * 1024u);
+                    if constexpr (ONCE) {
+                        load_to_lds_16_once(words[m] + (uint64_t)n * tile_bytes + (uint64_t)at * STEP_BYTES + part * 1024u, piece_offset,
+                                            base + (m * STRIP + n) * STEP_BYTES + part * 1024u);
+                    } else {
+                        load_to_lds_16(words[m] + (uint64_t)n * tile_bytes + (uint64_t)at * STEP_BYTES + part * 1024u, piece_offset,
+                                            base + (m * STRIP + n) * STEP_BYTES + part * 1024u);
+                    }
                 }
             }
         }
