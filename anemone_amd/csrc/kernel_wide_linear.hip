@@ -47,7 +47,8 @@ __device__ static __forceinline__ void wide_expert_gate_up(const struct wide_exp
     const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     struct wide_expert_tile tile;
     uint32_t pair_count = 0, block_strip = 0;
-    if (!order_block_of<1u, false, !BYTES>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count)) {
+    bool alone = false;
+    if (!order_block_of<1u, false, !BYTES>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count, &alone)) {
         return;
     }
     const struct wide_pair *pairs = (const struct wide_pair *)(arena + arguments.pairs_offset) + tile.first_pair;
@@ -63,6 +64,7 @@ __device__ static __forceinline__ void wide_expert_gate_up(const struct wide_exp
     const uint32_t word_column = 16u * wave + lane / 4u;
     const uint32_t exponent_vector = pairs[word_column < pair_count ? word_column : 0u].pair_index / arguments.pairs_per_row;
     chain_type chain_of;
+    chain_of.once = alone;
     const unsigned char *const matrices[2] = {arena + tile.gate_offset, arena + tile.up_offset};
     const uint32_t window_address = (uint32_t)(uintptr_t)(lds_pointer)window;
     uint32_t tile0 = 0;
@@ -97,7 +99,8 @@ __device__ static __forceinline__ void wide_expert_down(const struct wide_expert
     const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     struct wide_expert_tile tile;
     uint32_t pair_count = 0, block_strip = 0;
-    if (!order_block_of<1u, true, !BYTES>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count)) {
+    bool alone = false;
+    if (!order_block_of<1u, true, !BYTES>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count, &alone)) {
         return;
     }
     const struct wide_pair *pairs = (const struct wide_pair *)(arena + arguments.pairs_offset) + tile.first_pair;
@@ -113,6 +116,7 @@ __device__ static __forceinline__ void wide_expert_down(const struct wide_expert
     const uint32_t exponent_vector = pairs[word_column < pair_count ? word_column : 0u].pair_index;
     columns[own_column] = own_pair; /* for the finish, behind the chain's barriers */
     chain_type chain_of;
+    chain_of.once = alone;
     const unsigned char *const matrices[1] = {arena + tile.down_offset};
     uint32_t tile0 = 0;
     chain_of.place(matrices, arguments.output_size, arguments.input_size, block_strip, arena + arguments.codes_offset,

@@ -37,6 +37,11 @@ struct wide_chain {
     static_assert(WEIGHT_LOADS < 64u && WINDOW_BYTES <= 160u * 1024u, "vmcnt has six bits; LDS 160 KB");
 
     const unsigned char *words[MATRICES], *scales[MATRICES], *codes, *exponents;
+    /* no other tile of the launch reads these weights: they are asked for as a stream (whoever places the chain sets it). 300
+     * rows of 4096 x 2048 x 256 experts of 4-bit weights: gate/up 387 -> 348 us, down 208 -> 192; 200 rows of float32-scaled FP8
+     * 702 -> 645, 361 -> 335; 2048 rows 975 -> 944, 502 -> 489. Where tiles share an expert a stream is read again: all of
+     * them streamed, 2048 rows took 1050 and 555. */
+    bool once;
     uint32_t tile_bytes, window, chunks, wave, piece_offset, scale_offset, codes_offset[2], exponents_offset;
     uint32_t read_at, scale_at[BYTES ? STRIP : 1], vector_at, vector_scale_at, shift, last_step, lane_of;
 
@@ -69,6 +74,7 @@ struct wide_chain {
 
     /* the wavefront's own weights and their scales of K step `at` into its part of stage `stage` (no other wavefront
      * reads that part: once this one has read it, it may be asked for again) */
+    template <bool ONCE>
     __device__ __forceinline__ void issue_weights(uint32_t stage, uint32_t at) const
     {
         const uint32_t mine = window + stage * STAGE_BYTES + wave * WAVE_BYTES;
@@ -78,8 +84,13 @@ struct wide_chain {
             for (uint32_t n = 0; n < STRIP; n++) {
 #pragma unroll
                 for (uint32_t part = 0; part < TILE_LOADS; part++) {
-                    load_to_lds_16(words[m] + (uint64_t)n * tile_bytes + (uint64_t)at * STEP_BYTES + part * 1024u, piece_offset,
-                                   mine + (m * STRIP + n) * STEP_BYTES + part * 1024u);
+                    const unsigned char *piece = words[m] + (uint64_t)n * tile_bytes + (uint64_t)at * STEP_BYTES + part * 1024u;
+                    const uint32_t to = mine + (m * STRIP + n) * STEP_BYTES + part * 1024u;
+                    if constexpr (ONCE) {
+                        load_to_lds_16_once(piece, piece_offset, to);
+                    } else {
+                        load_to_lds_16(piece, piece_offset, to);
+                    }
                 }
             }
         }
@@ -203,7 +214,7 @@ struct wide_chain {
     }
 
     /* all `total` K steps of LIVE live column blocks; every wavefront of the block calls it (barriers inside) */
-    template <uint32_t LIVE>
+    template <uint32_t LIVE, bool ONCE>
     __device__ __forceinline__ void steps(uint32_t total, float4_t (&chain)[TILES][WIDE_COLUMN_BLOCKS]) const
     {
         /* Two stages. A wavefront's weights of a step are asked for two steps ahead, as soon as the wavefront itself has
@@ -212,9 +223,9 @@ struct wide_chain {
          * chunk of scale words), the weights of k + 1. */
         issue_vector_scales(0u);
         issue_vectors(0u, 0u);
-        issue_weights(0u, 0u);
+        issue_weights<ONCE>(0u, 0u);
         if (total > 1u) {
-            issue_weights(1u, 1u);
+            issue_weights<ONCE>(1u, 1u);
         }
         for (uint32_t step = 0; step < total; step++) {
             if (step + 1u < total) {
@@ -228,7 +239,7 @@ struct wide_chain {
             }
             consume<LIVE>(step % 2u, step, chain);
             if (step + 2u < total) {
-                issue_weights(step % 2u, step + 2u);
+                issue_weights<ONCE>(step % 2u, step + 2u);
             }
         }
     }
@@ -238,18 +249,28 @@ struct wide_chain {
     __device__ __forceinline__ void whole(uint32_t total, uint32_t live_blocks, float4_t (&chain)[TILES][WIDE_COLUMN_BLOCKS]) const
     {
         static_assert(WIDE_COLUMN_BLOCKS == 4u, "one instance a count of live column blocks");
+        if (once) { /* the same in every lane of the block: its own instances, and no test in the steps of the others */
+            run<true>(total, live_blocks, chain);
+        } else {
+            run<false>(total, live_blocks, chain);
+        }
+    }
+
+    template <bool ONCE>
+    __device__ __forceinline__ void run(uint32_t total, uint32_t live_blocks, float4_t (&chain)[TILES][WIDE_COLUMN_BLOCKS]) const
+    {
         switch (live_blocks) {
         case 1u:
-            steps<1>(total, chain);
+            steps<1, ONCE>(total, chain);
             break;
         case 2u:
-            steps<2>(total, chain);
+            steps<2, ONCE>(total, chain);
             break;
         case 3u:
-            steps<3>(total, chain);
+            steps<3, ONCE>(total, chain);
             break;
         default:
-            steps<4>(total, chain);
+            steps<4, ONCE>(total, chain);
             break;
         }
     }

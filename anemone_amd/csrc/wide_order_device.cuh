@@ -54,15 +54,23 @@ __device__ static __forceinline__ uint32_t order_used_tiles(const struct wide_ex
 /* The block's strip of the grid's x and its columns: GROUP consecutive tiles of one run, fewer at the run's end. DOWN:
  * runs are tiles of one down matrix, else of one gate and up. Returns false for a block that has nothing to do. Every
  * lane of a wavefront calls; strips = gridDim.x, tile_count = gridDim.y. Two round trips to the table: the used tiles, and
- * the ORDER_WINDOW tiles around the block's own, a lane a tile (runs are cut where a window ends). */
+ * the ORDER_WINDOW tiles around the block's own, a lane a tile (runs are cut where a window ends). alone_out: whether the
+ * block's tile is a run of its own (as far as the block sees: a matter of speed, not of results). */
 template <uint32_t GROUP, bool DOWN, bool BY_RUN>
 __device__ static __forceinline__ bool order_block_of(const struct wide_expert_tile *tiles, uint32_t tile_count, uint32_t lane, uint32_t &strip_out,
-                                                      struct wide_expert_tile &tile_out, uint32_t &pair_count_out)
+                                                      struct wide_expert_tile &tile_out, uint32_t &pair_count_out, bool *alone_out = nullptr)
 {
     if constexpr (!BY_RUN && GROUP == 1u) {
         strip_out = blockIdx.x;
         tile_out = tiles[blockIdx.y];
         pair_count_out = tile_out.pair_count;
+        if (alone_out != nullptr) { /* the neighbours in the table hold another matrix, or lie past it, or hold nothing */
+            const auto matrix_of = [&](uint32_t index) -> uint64_t { return DOWN ? tiles[index].down_offset : tiles[index].gate_offset; };
+            const uint32_t before = blockIdx.y != 0u ? blockIdx.y - 1u : 0u, behind = blockIdx.y + 1u < tile_count ? blockIdx.y + 1u : blockIdx.y;
+            const uint64_t own = DOWN ? tile_out.down_offset : tile_out.gate_offset;
+            *alone_out = !(before != blockIdx.y && matrix_of(before) == own) &&
+                         !(behind != blockIdx.y && tiles[behind].pair_count != 0u && matrix_of(behind) == own);
+        }
         return tile_out.pair_count != 0u;
     }
     const uint32_t strips = gridDim.x;
@@ -119,6 +127,9 @@ __device__ static __forceinline__ bool order_block_of(const struct wide_expert_t
     tile_out.first_pair = of_lane(mine.first_pair, tile);
     tile_out.pair_count = of_lane(mine.pair_count, tile);
     pair_count_out = tile_out.pair_count;
+    if (alone_out != nullptr) {
+        *alone_out = length == 1u;
+    }
     if constexpr (GROUP == 2u) {
         if (tile + 1u < first + length) {
             pair_count_out += of_lane(mine.pair_count, tile + 1u);
