@@ -80,6 +80,30 @@ def test_quantizer_byte_for_byte(amd, card):
     assert np.all(layer.read("operands") == 0xEE)  # not written
 
 
+@pytest.mark.parametrize("seed,narrow", [(1, False), (2, False), (3, True)])
+def test_quantizer_over_every_bfloat16_magnitude(amd, card, seed, narrow):
+    """Quotients by the scale's rounded reciprocal and a correction: every finite bfloat16 value, in groups of all magnitudes (the
+    smallest beside the largest) or, narrow, of neighbouring ones, against the oracle's divisions."""
+    say("quantizer over every bfloat16 magnitude", seed, narrow)
+    finite = np.array([b for b in range(1 << 16) if (b & 0x7F80) != 0x7F80], dtype=np.uint16)
+    rng = np.random.default_rng(seed)
+    if narrow:
+        finite = finite[np.argsort(finite & 0x7FFF, kind="stable")]
+    else:
+        rng.shuffle(finite)
+    width = 1024
+    rows = -(-finite.size // width)
+    values = np.zeros(rows * width, dtype=np.uint16)
+    values[:finite.size] = finite
+    values = np.ascontiguousarray(values.reshape(rows, width))
+    layer, _ = build(amd, card, width, 128, 64, 2, rows, 1)
+    layer.set_rows(values)
+    card.run(layer.quantize_launch())
+    _, scales, lane = oracle_quantize(values)
+    assert np.array_equal(layer.read("exponents").view(np.uint32).reshape(rows, -1), scales.view(np.uint32))
+    assert np.array_equal(layer.read("codes").reshape(rows, width), lane)
+
+
 @pytest.mark.parametrize("slices", [1, 2, 8])
 def test_products_within_the_bound(amd, card, slices):
     """The down kernel is the plain product: each expert's gate matrix through it, against the exact block sums."""
