@@ -294,10 +294,11 @@ extern "C" __global__ void __launch_bounds__(PROJECTION_TILE_THREADS, 3) /* thre
 }
 ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_projection_tiles, router_projection_arguments);
 
-/* The same scores for steps of 9 to 256 rows, whose tiles of 16 experts by 64 rows are fewer than the card's CUs: a block
- * is one 16 x 16 tile, and its four wavefronts take eight chains each, so that a CU's four vector units work on every
- * score. Instruction t of a group of 32 inputs takes the chains 8 wave + 2 b + t of the blocks b = 0 .. 3: lane (b, n)
- * needs the two inputs 32 i + 8 wave + 2 b + {0, 1} of expert n and of row n, one word each. A stage is the 16 + 16 rows'
+/* The same scores for steps whose tiles of 16 experts by 64 rows leave CUs idle or unevenly loaded (which those are:
+ * PROJECTION_SPLIT_BLOCKS_OF_TILE, with both forms' times): a block is one 16 x 16 tile, and its four wavefronts take eight
+ * chains each, so that a CU's four vector units work on every score. Instruction t of a group of 32 inputs takes the chains
+ * 8 wave + 2 b + t of the blocks b = 0 .. 3: lane (b, n) needs the two inputs 32 i + 8 wave + 2 b + {0, 1} of expert n and
+ * of row n, one word each. A stage is the 16 + 16 rows'
  * 128 inputs (8 KB, laid out and swizzled as above); PROJECTION_SPLIT_STAGES of them are in LDS or on their way (three blocks
  * a CU; five to sixteen measured within 10 %), and a stage is read behind the instructions of the one before it. The
  * wavefronts' sums meet in LDS at the end, each wavefront folding a quarter of the scores. What is left is a wavefront's 256

@@ -7,10 +7,10 @@
  *
  *   launch        kernel                grid                        block
  *   projection    router_projection     (ceil(E / 8), ceil(rows / 4), 1)   128   eight experts and four rows a block
- *                 router_projection_tiles (E / 16, ceil(rows / 64), 1)     256   257 rows and more of a width in whole 128, E in whole 16:
- *                                                                                16 experts by 64 rows a block
- *                 router_projection_split (E / 16, ceil(rows / 16), 1)     256   9 to 256 rows of such a width and E: 16 experts by 16 rows a
- *                                                                                block (beside its kernel: both sides' times)
+ *                 router_projection_split (E / 16, ceil(rows / 16), 1)     256   9 rows and more of a width in whole 128, E in whole 16: 16
+ *                                                                                experts by 16 rows a block
+ *                 router_projection_tiles (E / 16, ceil(rows / 64), 1)     256   such steps where its fewer blocks are as many as the CUs
+ *                                                                                (projection_takes_split): 16 experts by 64 rows a block
  *   select        router_select_entry   (1, 1, 1)                   512   a wavefront a row
  *   wide select   router_wide_select    (ceil(rows / 8), 1, 1)      512   a wavefront a row
  *   wide count    router_wide_count     (ceil(rows / 384), 1, 1)    512   a thread an expert
@@ -72,11 +72,11 @@ result_status router_kernels_prepare(const struct backend_operations *backend, s
     uint32_t tiles = BACKEND_NO_KERNEL, split = BACKEND_NO_KERNEL;
     if (backend->kernel_prepare(card, KERNEL_FILE_ROUTER, KERNEL_ROUTER_PROJECTION_TILES, sizeof(struct router_projection_arguments),
                                 &tiles) != STATUS_OK) {
-        tiles = BACKEND_NO_KERNEL; /* every row count then takes router_projection */
+        tiles = BACKEND_NO_KERNEL; /* router_projection_split then takes its steps */
     }
     if (backend->kernel_prepare(card, KERNEL_FILE_ROUTER, KERNEL_ROUTER_PROJECTION_SPLIT, sizeof(struct router_projection_arguments),
                                 &split) != STATUS_OK) {
-        split = BACKEND_NO_KERNEL; /* so do then 9 to 256 rows */
+        split = BACKEND_NO_KERNEL; /* router_projection_tiles and, to 256 rows, router_projection then take its steps */
     }
     memcpy(kernels_out, handles, sizeof handles);
     kernels_out->projection_tiles = tiles;
@@ -231,6 +231,15 @@ result_status router_select_prepare(const struct router_description *description
     return STATUS_OK;
 }
 
+/* the blocks of the fuller CUs, of each form: see PROJECTION_SPLIT_BLOCKS_OF_TILE for both sides' times */
+static bool projection_takes_split(uint32_t row_count, uint32_t expert_count)
+{
+    const uint64_t strips = expert_count / 16u;
+    const uint64_t split = strips * ((row_count + PROJECTION_SPLIT_ROWS - 1u) / PROJECTION_SPLIT_ROWS);
+    const uint64_t tiles = strips * ((row_count + PROJECTION_TILE_ROWS - 1u) / PROJECTION_TILE_ROWS);
+    return (split + PROJECTION_CUS - 1u) / PROJECTION_CUS <= PROJECTION_SPLIT_BLOCKS_OF_TILE * ((tiles + PROJECTION_CUS - 1u) / PROJECTION_CUS);
+}
+
 result_status router_projection_prepare(const struct router_projection_description *description,
                                         uint64_t arena_byte_count, const struct router_kernels_record *kernels,
                                         struct kernel_launch *launch_out)
@@ -258,21 +267,22 @@ result_status router_projection_prepare(const struct router_projection_descripti
         .hidden = description->hidden,
         .expert_count = description->expert_count,
     };
-    if (kernels->projection_tiles != BACKEND_NO_KERNEL && description->row_count >= PROJECTION_TILE_LEAST_ROWS &&
-        description->expert_count % 16u == 0 &&
-        description->hidden % PROJECTION_STAGE_INPUTS == 0) { /* many rows: the chains on the matrix unit, 16 experts by 64 rows a block */
-        launch_fill(launch_out, kernels->projection_tiles, description->expert_count / 16u,
-                    (description->row_count + PROJECTION_TILE_ROWS - 1u) / PROJECTION_TILE_ROWS, 1, PROJECTION_TILE_THREADS, 0, &record,
-                    sizeof record);
-        return STATUS_OK;
-    }
-    if (kernels->projection_split != BACKEND_NO_KERNEL && description->row_count >= PROJECTION_SPLIT_LEAST_ROWS &&
-        description->row_count < PROJECTION_TILE_LEAST_ROWS && description->expert_count % 16u == 0 &&
-        description->hidden % PROJECTION_STAGE_INPUTS == 0) { /* 16 experts by 16 rows a block, their chains over its wavefronts */
-        launch_fill(launch_out, kernels->projection_split, description->expert_count / 16u,
-                    (description->row_count + PROJECTION_SPLIT_ROWS - 1u) / PROJECTION_SPLIT_ROWS, 1, PROJECTION_TILE_THREADS, 0, &record,
-                    sizeof record);
-        return STATUS_OK;
+    /* from nine rows on, the chains on the matrix unit: 16 experts by 16 rows a block, or by 64 */
+    if (description->row_count >= PROJECTION_SPLIT_LEAST_ROWS && description->expert_count % 16u == 0 &&
+        description->hidden % PROJECTION_STAGE_INPUTS == 0) {
+        const bool has_split = kernels->projection_split != BACKEND_NO_KERNEL, has_tiles = kernels->projection_tiles != BACKEND_NO_KERNEL;
+        if (has_split && (!has_tiles || projection_takes_split(description->row_count, description->expert_count))) {
+            launch_fill(launch_out, kernels->projection_split, description->expert_count / 16u,
+                        (description->row_count + PROJECTION_SPLIT_ROWS - 1u) / PROJECTION_SPLIT_ROWS, 1, PROJECTION_TILE_THREADS, 0, &record,
+                        sizeof record);
+            return STATUS_OK;
+        }
+        if (has_tiles && (has_split || description->row_count >= PROJECTION_TILE_LEAST_ROWS)) {
+            launch_fill(launch_out, kernels->projection_tiles, description->expert_count / 16u,
+                        (description->row_count + PROJECTION_TILE_ROWS - 1u) / PROJECTION_TILE_ROWS, 1, PROJECTION_TILE_THREADS, 0, &record,
+                        sizeof record);
+            return STATUS_OK;
+        }
     }
     /* a thin step: a row a block (the kernel takes the rows its grid leaves it: four a block, or one) */
     const uint32_t expert_blocks = (description->expert_count + PROJECTION_OUTPUTS - 1u) / PROJECTION_OUTPUTS;

@@ -107,10 +107,19 @@ ANEMONE_RECORD_HAS(wide_expert_tile, 32);
 #define KERNEL_ROUTER_PROJECTION_TILES "router_projection_tiles" /* the same scores on the matrix unit: steps of many rows */
 #define PROJECTION_TILE_THREADS 256u
 #define PROJECTION_TILE_ROWS 64u   /* rows of a block of router_projection_tiles: 16 a wavefront */
-#define PROJECTION_TILE_LEAST_ROWS 257u /* fewer rows take router_projection_split or router_projection: their blocks are smaller and more */
-#define KERNEL_ROUTER_PROJECTION_SPLIT "router_projection_split" /* and with a tile's chains over a block's wavefronts: few rows */
+#define PROJECTION_TILE_LEAST_ROWS 257u /* of a backend without router_projection_split; fewer rows then take router_projection */
+#define KERNEL_ROUTER_PROJECTION_SPLIT "router_projection_split" /* and with a tile's chains over a block's wavefronts */
 #define PROJECTION_SPLIT_ROWS 16u       /* rows of a block of router_projection_split */
 #define PROJECTION_SPLIT_LEAST_ROWS 9u  /* up to eight rows router_projection takes a row a block, in blocks of eight experts */
+/* Which of the two takes a step of more rows. A block of router_projection_tiles is a score's 32 chains in one wavefront, so a
+ * launch takes as long as the blocks that fall to one of the 256 CUs, one behind the other in all but the loads; a block of
+ * router_projection_split is a quarter of that, on as many wavefronts, and brings its operands for a quarter of the scores. In
+ * blocks a CU, us, 4096 inputs: tiles 1 / 2 / 3 / 4 blocks 26.6 / 42.8 / 64 / 87; split 1 .. 10 blocks 11.3 / 16.5 / 22.4 / 28.4 /
+ * 33.8 / 39.6 / 45.5 / 51 / 57 / 64: three blocks of the split form are the faster, four the slower (256 experts: 512 rows 26.8 |
+ * 17.0, 768 rows 26.8 | 22.7, 1024 rows 27.1 | 28.5, 1152 rows 42.7 | 33.7, 1536 rows 42.8 | 40.3, 1792 rows 43.4 | 46.1; 64 experts: 3072
+ * rows 27.1 | 23.3, 4096 rows 27.5 | 29.3; 384 experts: 512 rows 27.0 | 22.6, 640 rows 26.9 | 28.5; 2048 and 5120 inputs: the same line). */
+#define PROJECTION_SPLIT_BLOCKS_OF_TILE 3u
+#define PROJECTION_CUS 256u
 #define PROJECTION_STAGE_INPUTS 128u     /* inputs of a stage of router_projection_tiles: the width is a whole number of them */
 #define KERNEL_ROUTER_SELECT "router_select_entry"
 #define KERNEL_ROUTER_WIDE_SELECT "router_wide_select"

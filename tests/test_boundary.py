@@ -287,8 +287,9 @@ def router_description(fake, **changes):
 
 
 def test_router_projection_prepare_geometry(fake):
-    """Which kernel takes a projection: many rows of a width in whole 128 inputs go to the matrix unit (16 experts by 64
-    rows a block); any other width, and thin steps, to router_projection (eight experts a block)."""
+    """Which kernel takes a projection: from nine rows on a width in whole 128 inputs goes to the matrix unit, in blocks of 16
+    experts by 16 rows, or by 64 rows where these are fewer than a third of the others a CU (256 CUs, in whole blocks); any
+    other width, and thin steps, to router_projection (eight experts a block)."""
     lib = amd.library()
     kernels = amd.RouterKernels()
     assert lib.router_kernels_prepare(fake.address, fake.card, C.byref(kernels)) == 0
@@ -300,7 +301,7 @@ def test_router_projection_prepare_geometry(fake):
         status = lib.router_projection_prepare(C.byref(d), ARENA, C.byref(kernels), launch)
         return status, (fake.handles[launch[0].kernel][1] if status == 0 else None), list(launch[0].grid), launch[0].block[0]
 
-    assert prepared(300, 512, 64) == (0, "router_projection_tiles", [4, 5, 1], 256)
+    assert prepared(300, 512, 64) == (0, "router_projection_split", [4, 19, 1], 256)
     assert prepared(4096, 4096, 256) == (0, "router_projection_tiles", [16, 64, 1], 256)
     status, name, grid, block = prepared(300, 160, 64)  # no whole number of stages of 128 inputs
     assert (status, name, grid) == (0, "router_projection", [8, 75, 1])
@@ -308,10 +309,19 @@ def test_router_projection_prepare_geometry(fake):
     assert (status, name, grid) == (0, "router_projection", [9, 75, 1])
     for rows in (9, 16, 17, 203, 256):  # few rows: 16 experts by 16 rows a block
         assert prepared(rows, 4096, 256) == (0, "router_projection_split", [16, (rows + 15) // 16, 1], 256)
-    assert prepared(257, 4096, 256)[1] == "router_projection_tiles"
+    # on both sides of the line: 768 blocks of 16 rows are three a CU and 769 four; where the tiles are two a CU, six and seven
+    for rows, experts_n, split in ((257, 256, True), (768, 256, True), (769, 256, False), (1024, 256, False), (1025, 256, True), (1536, 256, True),
+                                   (1537, 256, False), (2560, 256, False), (3072, 64, True), (3073, 64, False), (512, 384, True), (513, 384, False),
+                                   (65535, 64, False), (256, 768, True), (257, 1024, True), (256, 1024, False), (9, 4096, True)):
+        assert prepared(rows, 128, experts_n) == (0, "router_projection_split" if split else "router_projection_tiles",
+                                                  [experts_n // 16, (rows + (15 if split else 63)) // (16 if split else 64), 1], 256), (rows, experts_n)
     assert prepared(100, 160, 64)[1:3] == ("router_projection", [8, 25, 1]) and prepared(100, 512, 72)[1:3] == ("router_projection", [9, 25, 1])
-    kernels.projection_split = amd.BACKEND_NO_KERNEL  # a backend without it
+    split, kernels.projection_split = kernels.projection_split, amd.BACKEND_NO_KERNEL  # a backend without it
     assert prepared(100, 512, 64)[1:3] == ("router_projection", [8, 25, 1])
+    assert prepared(257, 512, 64) == (0, "router_projection_tiles", [4, 5, 1], 256)
+    tiles, kernels.projection_split, kernels.projection_tiles = kernels.projection_tiles, split, amd.BACKEND_NO_KERNEL  # without the other
+    assert prepared(4096, 512, 64) == (0, "router_projection_split", [4, 256, 1], 256)
+    kernels.projection_split, kernels.projection_tiles = amd.BACKEND_NO_KERNEL, tiles
     status, name, grid, block = prepared(8, 4096, 256)  # a thin step: a row a block
     assert (status, name, grid) == (0, "router_projection", [32, 8, 1])
     assert prepared(300, 48, 64)[0] == 1 and prepared(0, 512, 64)[0] == 1  # a width that is no multiple of 32; no row

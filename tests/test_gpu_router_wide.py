@@ -170,8 +170,8 @@ def test_wide_small_equals_the_four_launches(amd, card, experts_n, picks, rows, 
 
 @pytest.mark.parametrize("experts_n,rows,hidden,scale", [(64, 300, 512, 1.0), (256, 257, 1024, 1.0), (64, 321, 128, 1e-18), (128, 1000, 256, 3e18), (64, 700, 384, 1.0), (64, 300, 192, 1.0), (384, 290, 5120, 1.0)])
 def test_projection_of_many_rows_bit_exact(amd, card, experts_n, rows, hidden, scale):
-    """router_projection_tiles (257 rows and more: the 32 chains of a score as matrix-unit products of one input each)
-    against the oracle's chains, every bit; scales that put products among the subnormals and near overflow among
+    """router_projection_tiles (the 32 chains of a score as matrix-unit products of one input each; of a record without
+    router_projection_split it takes every step of 257 rows and more) against the oracle's chains, every bit; scales that put products among the subnormals and near overflow among
     the cases."""
     say("projection, many rows", experts_n, rows, hidden, scale)
     layer, _ = small_layer(amd, card, experts_n, 2, rows, hidden=hidden)
@@ -179,6 +179,7 @@ def test_projection_of_many_rows_bit_exact(amd, card, experts_n, rows, hidden, s
     x = to_bf16(normals(42, rows * hidden) * scale).reshape(rows, hidden)
     card.upload(layer.router_offset, router)
     layer.set_rows(x, rows)
+    layer.router_kernels.projection_split = amd.BACKEND_NO_KERNEL
     launch = layer.projection_launch()
     if hidden % 128 == 0:  # a stage of the matrix-unit kernel is 128 inputs; any other width takes the thin kernel
         assert list(launch[0].block)[0] == 256 and list(launch[0].grid) == [experts_n // 16, (rows + 63) // 64, 1]
@@ -198,9 +199,10 @@ def test_projection_of_many_rows_bit_exact(amd, card, experts_n, rows, hidden, s
     (64, 9, 128, 1.0),       # one stage: fewer than the kernel keeps on their way
     (64, 16, 640, 1e-18), (128, 17, 768, 1.0), (256, 33, 896, 1.0),  # as many stages as places, and around it; a tile's last rows
     (384, 63, 1024, 3e18), (256, 203, 4096, 1.0), (64, 256, 5120, 1.0),
+    (256, 753, 256, 1.0), (64, 3072, 128, 1.0), (384, 1008, 128, 1.0),  # more rows, where the line is (see test_boundary.py)
 ])
 def test_projection_of_few_rows_bit_exact(amd, card, experts_n, rows, hidden, scale):
-    """router_projection_split (9 to 256 rows: a tile's chains over a block's wavefronts) against the oracle's chains, every
+    """router_projection_split (a tile's chains over a block's wavefronts) against the oracle's chains, every
     bit, nothing written behind the scores."""
     say("projection, few rows", experts_n, rows, hidden, scale)
     layer, _ = small_layer(amd, card, experts_n, 2, rows, hidden=hidden)
