@@ -38,6 +38,20 @@
 #include "quantize_device.cuh"
 #include "strip_device.cuh"
 
+/* Whether no other job of the table has this job's matrices (a matter of speed, not of results): an expert of more than eight
+ * rows has its jobs one behind the other, all but the last of them full. Such a job's blocks read the weights through the caches,
+ * any other's as a stream. 4096 x 2048, gate/up and down, us, every job through the caches | every job as a stream | by this rule:
+ * 256 experts, 64 rows of float32-scaled FP8 592 and 304 | 549 and 281 | 550 and 281; 32 rows of FP4 234 and 125 | 213 and 112 | 213
+ * and 112; 64 experts, 64 rows of FP8 182 and 103 | 193 and 105 | 174 and 100; of FP8 with Zipf(1.1) loads in lane order 192 and
+ * 108 | 209 and 114 | 182 and 103, with eight experts of eight jobs each (2048 x 1024) 38 and 25 | 40 and 25 | 34 and 24; FP4 107 and
+ * 66 | 105 and 65 | 104 and 65. (An expert of exactly eight rows counts as one of more. With both neighbours and the table's end looked at it would not:
+ * the same times, and 0.3 us more in a launch of few jobs.) */
+__device__ static __forceinline__ bool job_alone(const struct expert_job_record *jobs, uint32_t index)
+{
+    const struct expert_job_record *job = jobs + index, *before = jobs + (index != 0u ? index - 1u : 0u);
+    const uint32_t follows = (uint32_t)(before->row_count == LINEAR_MAXIMUM_ROWS) & (uint32_t)(before->expert == job->expert);
+    return (follows | (uint32_t)(job->row_count == LINEAR_MAXIMUM_ROWS)) == 0u;
+}
 
 /* gate and up: block = S wavefronts (slices of the inputs); grid (ceil(output_size / 64), jobs) */
 template <uint32_t S, bool BYTES, bool B128 = false, bool NATIVE = false>
@@ -48,7 +62,7 @@ __device__ static __forceinline__ void expert_gate_up(const struct expert_gate_u
     constexpr uint32_t TILES = chain_type::TILES, STRIP = chain_type::STRIP;
     __shared__ __attribute__((aligned(16))) unsigned char window[S][chain_type::WINDOW_BYTES];
     static_assert(chain_type::WINDOW_BYTES >= TILES * WAVE * 16u, "a wavefront's sums fit its idle window");
-    const struct expert_job_record *job = (const struct expert_job_record *)(arena + arguments.jobs_offset) + blockIdx.y;
+    const struct expert_job_record *jobs = (const struct expert_job_record *)(arena + arguments.jobs_offset), *job = jobs + blockIdx.y;
     if (job->row_count == 0u) {
         return;
     }
@@ -64,6 +78,7 @@ __device__ static __forceinline__ void expert_gate_up(const struct expert_gate_u
     const uint32_t steps = arguments.input_size / 128u;
     const uint32_t first = steps * slice / S, last = steps * (slice + 1u) / S;
     chain_type chain_of;
+    chain_of.once = job_alone(jobs, blockIdx.y);
     const unsigned char *const matrices[2] = {arena + job->gate_offset, arena + job->up_offset};
     chain_of.place(matrices, arguments.output_size, arguments.input_size, blockIdx.x, first, arena + arguments.codes_offset,
                    arena + arguments.exponents_offset, rows, (uint32_t)(uintptr_t)(lds_pointer)&window[slice][0], lane);
@@ -201,7 +216,7 @@ __device__ static __forceinline__ void expert_down(const struct expert_down_argu
     constexpr uint32_t TILES = chain_type::TILES, STRIP = chain_type::STRIP;
     __shared__ __attribute__((aligned(16))) unsigned char window[S][chain_type::WINDOW_BYTES];
     static_assert(chain_type::WINDOW_BYTES >= TILES * WAVE * 16u, "a wavefront's sums fit its idle window");
-    const struct expert_job_record *job = (const struct expert_job_record *)(arena + arguments.jobs_offset) + blockIdx.y;
+    const struct expert_job_record *jobs = (const struct expert_job_record *)(arena + arguments.jobs_offset), *job = jobs + blockIdx.y;
     if (job->row_count == 0u) {
         return;
     }
@@ -216,6 +231,7 @@ __device__ static __forceinline__ void expert_down(const struct expert_down_argu
     const uint32_t steps = arguments.input_size / 128u;
     const uint32_t first = steps * slice / S, last = steps * (slice + 1u) / S;
     chain_type chain_of;
+    chain_of.once = job_alone(jobs, blockIdx.y);
     const unsigned char *const matrices[1] = {arena + job->down_offset};
     chain_of.place(matrices, arguments.output_size, arguments.input_size, blockIdx.x, first, arena + arguments.codes_offset,
                    arena + arguments.exponents_offset, rows, (uint32_t)(uintptr_t)(lds_pointer)&window[slice][0], lane);

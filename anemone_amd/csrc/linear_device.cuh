@@ -28,12 +28,9 @@ __device__ static __forceinline__ void load_to_lds_16(const unsigned char *base,
                  : "memory", "m0");
 }
 
-/* the same of bytes that a launch reads once (a small step's weights): asked for as a stream, they do not pass through the
- * caches as lines to be kept, and memory gives more of them: the experts of 4096 x 2048 x 256, 64 rows of float32-scaled FP8
- * gate/up 600 -> 555 us and down 308 -> 282 (6.7 TB/s), 32 rows of FP4 228 -> 207 and 120 -> 106, 5 rows 55.8 -> 51.6 and
- * 31.1 -> 28.5; 64 rows of Zipf(1.1) loads, where a busy expert's weights are read by several blocks, 333 -> 337 and 180 ->
- * 175. Not where blocks of one launch read the same bytes: the shared matrices by groups of rows 18.0 -> 19.6, the wide
- * products of one-byte weights 930 -> 1050 */
+/* the same of bytes that one block of a launch reads: asked for as a stream, they do not pass through the caches as lines to be
+ * kept, and memory gives more of them. Not where other blocks read them too: the shared matrices by groups of rows 18.0 -> 19.6 us,
+ * the wide products of one-byte weights 930 -> 1050, the jobs of an expert of more than eight rows (job_alone, with both sides) */
 __device__ static __forceinline__ void load_to_lds_16_once(const unsigned char *base, uint32_t lane_offset, uint32_t lds_base)
 {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"

@@ -22,9 +22,9 @@
  * tiles are read with one or two 16-byte LDS reads and no arithmetic; the scale codes of 4-bit weights are a word a lane
  * for the strip's four tiles (a group of 64 outputs), its byte picked by the matrix instruction; with B128 the scales are
  * E4M3_BLOCK128's float32 words where they are. */
-/* ONCE: the launch reads a weight once (the experts' launches, but for an expert of more than eight rows; not the shared matrices
- * of a step of several groups of rows), and asks for it as a stream */
-template <uint32_t MATRICES, bool BYTES, bool B128 = false, bool NATIVE = false, bool ONCE = false>
+/* STREAMS: the chain has an instance that asks for the weights as a stream, taken where `once` says that no other block of the
+ * launch reads them (the experts' launches; the shared matrices of a step of several groups of rows have readers enough) */
+template <uint32_t MATRICES, bool BYTES, bool B128 = false, bool NATIVE = false, bool STREAMS = false>
 struct strip_chain {
     static_assert(BYTES || !B128, "float32 scales go with one-byte weights");
     static constexpr uint32_t STRIP = BYTES ? 2u : 4u; /* tiles of a strip: 4 KB of every matrix a stage either way */
@@ -56,7 +56,9 @@ struct strip_chain {
     uint32_t vector_scale_at;               /* LDS byte offset of its vector's scale byte */
     uint32_t shift;                         /* nibbles: 0 the even ones (outputs 0..7 of a tile), 4 the odd ones;
                                              * bytes: the byte selector of the same choice */
+    bool once = false;                      /* STREAMS: the same in every lane of the block */
 
+    template <bool ONCE>
     __device__ __forceinline__ void issue(uint32_t stage, uint32_t at) const
     {
         const uint32_t base = window + stage * STAGE_BYTES;
@@ -190,11 +192,23 @@ struct strip_chain {
     /* The whole chain of `total` steps (the same in every lane). The window is idle on entry and on return. */
     __device__ __forceinline__ void whole(uint32_t total, float4_t (&chain)[TILES]) const
     {
+        if constexpr (STREAMS) {
+            if (once) {
+                steps<true>(total, chain);
+                return;
+            }
+        }
+        steps<false>(total, chain);
+    }
+
+    template <bool ONCE>
+    __device__ __forceinline__ void steps(uint32_t total, float4_t (&chain)[TILES]) const
+    {
         uint32_t done = 0;
         if (total >= 2u * DEPTH) {
 #pragma unroll
             for (uint32_t i = 0; i < DEPTH; i++) {
-                issue(i, i);
+                issue<ONCE>(i, i);
             }
             /* the steady state: a step consumed has DEPTH - 1 whole stages asked for behind it, and asks for one more */
             for (; done + 2u * DEPTH <= total; done += DEPTH) {
@@ -202,14 +216,14 @@ struct strip_chain {
                 for (uint32_t i = 0; i < DEPTH; i++) {
                     wait_loads<STAGE_LOADS * (DEPTH - 1u)>();
                     consume(i, chain);
-                    issue(i, done + i + DEPTH);
+                    issue<ONCE>(i, done + i + DEPTH);
                 }
             }
         } else {
 #pragma unroll
             for (uint32_t i = 0; i < DEPTH; i++) {
                 if (i < total) {
-                    issue(i, i);
+                    issue<ONCE>(i, i);
                 }
             }
         }
@@ -230,7 +244,7 @@ struct strip_chain {
                     }
                     consume(i, chain);
                     if (at + DEPTH < total) {
-                        issue(i, at + DEPTH);
+                        issue<ONCE>(i, at + DEPTH);
                     }
                 }
             }
@@ -245,7 +259,7 @@ struct strip_chain {
                                           const unsigned char *vector_exponents, const uint32_t (&vector_rows)[8],
                                           uint32_t window_address, uint32_t lane)
     {
-        static_assert(DEPTH == 2u || DEPTH == 3u, "the waits of whole() are written out for two or three stages");
+        static_assert(DEPTH == 2u || DEPTH == 3u, "the waits of steps() are written out for two or three stages");
         const uint32_t tiles = outputs / 16u;
         const uint32_t o = lane % 16u, g = lane / 16u, G = o % 8u, parity = o / 8u, ld = g / 2u, q = g % 2u;
         /* a strip that reaches past the last tile reads the last tiles again; its surplus sums are not stored */

@@ -138,6 +138,40 @@ def test_products_within_the_reference_bound(amd, card, slices, fmt, stress):
     assert worst < (0.2 if stress else 0.02)
 
 
+@pytest.mark.parametrize("slices,fmt", [(1, E2M1), (2, E2M1), (4, E2M1), (8, E2M1), (1, E4M3), (2, E4M3), (4, E4M3), (8, E4M3)])
+def test_jobs_of_one_expert_read_its_weights_either_way(amd, card, slices, fmt):
+    """A job whose neighbours say that its expert has other jobs reads the weights through the caches, any other as a stream: the
+    same jobs one expert behind the other, and so that no job stands beside one of its expert, give the same bytes."""
+    say("jobs of one expert", slices, fmt)
+    hidden, inner, rows = 1152, 1024, 43
+    layer, _, _ = build(amd, card, hidden, inner, 64, 1, rows, 3, fmt=fmt, gate_up_slices=slices, down_slices=slices)
+    layer.set_rows(to_bf16(normals(15, rows * hidden)).reshape(rows, hidden))
+    card.run(layer.quantize_launch())
+    plan, pair = [], 0  # (expert, rows of the job): full jobs and the last one's remainder, a full job alone, short jobs, an empty one
+    for expert, count in ((5, 8), (5, 8), (5, 3), (6, 8), (9, 1), (9, 0), (7, 2), (60, 8), (60, 5)):
+        plan.append((expert, list(range(pair, pair + count))))
+        pair += count
+    assert pair == rows
+
+    def run(order):
+        jobs = np.zeros(rows, dtype=JOB_DTYPE)
+        for j, (expert, members) in enumerate(order):
+            jobs[j]["gate_offset"], jobs[j]["up_offset"], jobs[j]["down_offset"] = layer.expert_offsets[expert]
+            jobs[j]["row_count"], jobs[j]["expert"] = len(members), expert
+            jobs[j]["pair_index"][:len(members)] = members
+            jobs[j]["route_weight"][:len(members)] = 0.5
+        card.upload(layer.jobs_offset, jobs.view(np.uint8))
+        for name in ("hidden", "pair_output"):
+            card.upload(layer.ranges[name].byte_offset, np.full(layer.ranges[name].byte_count, 0xEE, dtype=np.uint8))
+        card.run(layer.expert_launches())
+        return layer.read("hidden").copy(), layer.read("pair_output").copy()
+    behind = run(plan)
+    apart = run([plan[i] for i in (2, 3, 0, 7, 1, 4, 8, 5, 6)])
+    for name, a, b in zip(("hidden", "pair outputs"), behind, apart):
+        assert np.array_equal(a, b), name
+    assert np.all(behind[0].view(np.uint16) != 0xEEEE) and np.all(behind[1].view(np.uint16) != 0xEEEE)
+
+
 @pytest.mark.parametrize("rows,live,picks,fmt", [(8, 8, 4, E2M1), (3, 2, 8, E2M1), (1, 1, 2, E2M1), (8, 7, 4, E4M3), (2, 2, 8, E4M3)])
 def test_layer_against_oracle(amd, card, rows, live, picks, fmt):
     say("layer", rows, live, picks, "format", fmt)
