@@ -46,23 +46,11 @@ extern "C" __global__ void __launch_bounds__(LINEAR_ELEMENT_THREADS)
                           fmaxf(fabsf(bf16_to_float((uint16_t)bits[2])), fabsf(bf16_to_float((uint16_t)bits[3]))));
     largest = lanes_largest<1u>(lanes_largest<2u>(lanes_largest<4u>(lanes_largest<8u>(lanes_largest<16u>(largest)))));
     const float scale = __fdiv_rn(fmaxf(largest, 1e-4f), 448.0f);
-    /* A quotient by one divisor: the product with its rounded reciprocal and a correction by the remainder, which is the division's
-     * own value for every bfloat16 numerator and float32 significand (compared over all 2^30 pairs on the card), where neither the
-     * remainder nor the reciprocal leaves the normal range. Below 2^-100 it may: such a value's magnitude is far under the
-     * smallest code's half either way. A scale of infinity divides. The four divisions a thread were vector issue (16384 vectors of 2048
-     * values 42 -> 37 us, 2048 of 4096 13.2 -> 11.7). */
     const float reciprocal = __fdiv_rn(1.0f, scale);
-    const bool finite = scale <= 3.402823466e38f;
     uint32_t code[4];
 #pragma unroll
     for (uint32_t i = 0; i < 4u; i++) {
-        const float value = bf16_to_float((uint16_t)bits[i]);
-        const float near = __fmul_rn(value, reciprocal);
-        const float scaled = finite ? __fmaf_rn(__fmaf_rn(-near, scale, value), reciprocal, near) : __fdiv_rn(value, scale);
-        const float magnitude = fminf(fabsf(scaled), 448.0f);
-        const uint32_t field = __float_as_uint(fmaxf(magnitude, 0.015625f)) >> 23;
-        const uint32_t units = (uint32_t)__builtin_rintf(__fmul_rn(magnitude, __uint_as_float((257u - field) << 23)));
-        code[i] = (((field - 120u) << 3) + units - 8u) | ((bits[i] >> 8) & 0x80u);
+        code[i] = quantize_quotient_code(quantize_quotient(bf16_to_float((uint16_t)bits[i]), scale, reciprocal), bits[i]);
     }
     *(uint32_t *)(arena + arguments.codes_offset + vector * arguments.width + quantize_word_of(l, s, t)) =
         code[0] | (code[2] << 8) | (code[1] << 16) | (code[3] << 24); /* bytes: values +0, +8, +1, +9 */

@@ -1,7 +1,7 @@
 /*
- * kernel_selfcheck.hip -- the library's check of its own short cuts in arithmetic. Two helpers of the kernels take a
- * shorter way than the arithmetic they are defined by: det_silu and det_sigmoid (no tests around the exponential) and quantize_codes4
- * (the card's FP8 conversions). This kernel runs both ways over every input there is and counts the disagreements, so
+ * kernel_selfcheck.hip -- the library's check of its own short cuts in arithmetic. Some helpers of the kernels take a
+ * shorter way than the arithmetic they are defined by: det_silu and det_sigmoid (no tests around the exponential), quantize_codes4
+ * (the card's FP8 conversions) and quantize_quotient (a reciprocal and a correction in place of a division). This kernel runs both ways over every input there is and counts the disagreements, so
  * that a test on the card proves the two ways equal instead of sampling them. No counterpart in the reference; not on
  * the routed-expert path.
  */
@@ -15,7 +15,8 @@
 
 struct arithmetic_selfcheck_arguments {
     uint64_t output_offset; /* written: uint32 [threads of the grid][2]: disagreements, and the first input that disagreed */
-    uint32_t check;         /* 0: det_silu over all 2^32 float32; 1: quantize_codes4 over all 2^16 values x 2^8 scale codes; 2: det_sigmoid; 3: linear_silu within its bound of det_silu */
+    uint32_t check;         /* 0: det_silu over all 2^32 float32; 1: quantize_codes4 over all 2^16 values x 2^8 scale codes; 2: det_sigmoid; 3: linear_silu within its bound of det_silu;
+                             * 4: quantize_quotient over all 2^16 values under the scales of all 2^15 largest magnitudes */
     uint32_t reserved_zero;
 };
 static_assert(sizeof(struct arithmetic_selfcheck_arguments) == 16, "arithmetic_selfcheck_arguments ABI");
@@ -49,6 +50,21 @@ extern "C" __global__ void arithmetic_selfcheck(struct arithmetic_selfcheck_argu
             const bool same = taken == defined || fabsf(taken - defined) <= __fmaf_rn(LINEAR_SILU_BOUND, fabsf(defined), LINEAR_SILU_FLOOR) ||
                               (defined != defined && taken != taken);
             if (!same && disagreements++ == 0u) {
+                first = (uint32_t)pattern;
+            }
+        }
+    } else if (arguments.check == 4u) {
+        for (uint64_t pattern = thread; pattern < (1ull << 31); pattern += threads) {
+            const uint32_t bits = (uint32_t)pattern & 0xFFFFu, largest_bits = (uint32_t)(pattern >> 16);
+            const float value = bf16_to_float((uint16_t)bits), largest = bf16_to_float((uint16_t)largest_bits);
+            if (fabsf(value) > fmaxf(largest, 1e-4f)) { /* no value of a group is above its largest (not-a-numbers are no largest) */
+                continue;
+            }
+            const float scale = __fdiv_rn(fmaxf(largest, 1e-4f), 448.0f);
+            const float defined = __fdiv_rn(value, scale), taken = quantize_quotient(value, scale, __fdiv_rn(1.0f, scale));
+            const bool same = __float_as_uint(defined) == __float_as_uint(taken) || (defined != defined && taken != taken) ||
+                              ((fabsf(value) < 0x1p-100f || fabsf(defined) < 0x1p-100f) && fabsf(defined) < 0x1p-64f && fabsf(taken) < 0x1p-64f);
+            if (!(same && quantize_quotient_code(defined, bits) == quantize_quotient_code(taken, bits)) && disagreements++ == 0u) {
                 first = (uint32_t)pattern;
             }
         }

@@ -11,7 +11,7 @@ import sys
 import numpy as np
 import pytest
 
-from _oracle import JOB_DTYPE, f32p, f64p, normals, orc, ptr, to_bf16, u8p, u16p, u32p
+from _oracle import JOB_DTYPE, bf16_to_f32, f32p, f64p, normals, orc, ptr, to_bf16, u8p, u16p, u32p
 from test_gpu_linear import ALLOWANCE_GFX950
 
 pytestmark = pytest.mark.gpu
@@ -101,6 +101,42 @@ def test_quantizer_over_every_bfloat16_magnitude(amd, card, seed, narrow):
     card.run(layer.quantize_launch())
     _, scales, lane = oracle_quantize(values)
     assert np.array_equal(layer.read("exponents").view(np.uint32).reshape(rows, -1), scales.view(np.uint32))
+    assert np.array_equal(layer.read("codes").reshape(rows, width), lane)
+
+
+def test_quantizer_of_infinities_and_not_a_numbers(amd, card):
+    """What the definition says of them: a not-a-number is no largest magnitude and its quotient is limited to 448 under its sign; an
+    infinity makes the scale one, under which finite values are zeros and infinities (no number by it) 448."""
+    say("quantizer of 128 values a scale, infinities and not-a-numbers")
+    rows, width = 2, 1024
+    values = to_bf16(normals(4, rows * width).reshape(rows, width) * np.repeat([1e-6, 1.0, 1e5, 1e37, 1.0, 1e-3, 1e38, 1.0], 128))
+    values[0, [3, 130, 257, 300]] = 0x7FC0, 0xFF81, 0x7F81, 0xFFFF  # beside finite values: quiet and signalling, both signs
+    values[0, 384:512] = np.where(np.arange(128) % 2 == 0, 0x7FC1, 0xFFC1)  # nothing else: the floor 1e-4
+    values[0, 600], values[0, 601] = 0x7F80, 0xFF80
+    values[1, 0:128] = np.where(np.arange(128) % 2 == 0, 0x7F80, 0xFF80)
+    values[1, [200, 201, 202]] = 0x7F80, 0xFFC0, 0x8000
+    layer, _ = build(amd, card, width, 128, 64, 2, rows, 1)
+    layer.set_rows(values)
+    card.run(layer.quantize_launch())
+    floats = bf16_to_f32(values).reshape(rows, width // 128, 128)
+    magnitudes = np.where(np.isnan(floats), np.float32(0), np.abs(floats))
+    want_scales = np.maximum(magnitudes.max(axis=2), np.float32(1e-4)) / np.float32(448)
+    with np.errstate(all="ignore"):
+        quotients = floats / want_scales[..., None]
+    quotients = np.where(np.isnan(quotients), np.float32(448), np.abs(quotients)).reshape(rows, width)
+    signs = ((values >> 8) & 0x80).astype(np.uint8)
+    finite = values.copy()
+    finite[~np.isfinite(bf16_to_f32(values))] = 0
+    codes, _, _ = oracle_quantize(finite)  # groups of finite values and not-a-numbers: the oracle's codes of the former
+    unordered = ~np.isfinite(bf16_to_f32(values))
+    scales_of = np.repeat(want_scales, 128, axis=1)
+    codes = np.where(np.isinf(scales_of), signs, codes)  # a finite value by infinity: a zero of its sign
+    codes = np.where(unordered, signs | np.uint8(0x7E), codes).astype(np.uint8)
+    assert np.all(quotients[unordered] == 448) and np.all(quotients[np.isinf(scales_of) & ~unordered] == 0)
+    lane = np.zeros_like(codes)
+    for r in range(rows):
+        orc.orc_codes_lane_order(ptr(np.ascontiguousarray(codes[r]), u8p), width, ptr(lane[r], u8p))
+    assert np.array_equal(layer.read("exponents").view(np.uint32).reshape(rows, -1), want_scales.astype(np.float32).view(np.uint32))
     assert np.array_equal(layer.read("codes").reshape(rows, width), lane)
 
 

@@ -2,7 +2,8 @@
 gate / (1 + det_expf(-gate)) for all 2^32 float32 gates (det_sigmoid likewise against 1 / (1 + det_expf(-score))), and the quantizer by the card's FP8 conversions
 (quantize_codes4) against the quantizer's defining arithmetic (source/kernel_activation_quantize.cuh:52-133 of the
 reference, which tests/test_gpu_linear.py holds byte for byte to the CPU oracle) for all 2^16 bfloat16 values under
-all 2^8 scale codes. A disagreement names its first input."""
+all 2^8 scale codes, and the quotients of the quantizer of 128 values a scale (a reciprocal and a correction) against the divisions
+for all 2^16 values under the scales of all 2^15 largest magnitudes, infinities and not-a-numbers among both. A disagreement names its first input."""
 import ctypes as C
 import struct
 import sys
@@ -14,7 +15,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("check,what", [(0, "det_silu over all float32"), (1, "quantize_codes4 over all values and scale codes"),
-                                        (2, "det_sigmoid over all float32"), (3, "linear_silu within 2^-17 of det_silu over all float32")])
+                                        (2, "det_sigmoid over all float32"), (3, "linear_silu within 2^-17 of det_silu over all float32"),
+                                        (4, "quantize_quotient over all values under the scales of all largest magnitudes")])
 def test_short_cuts_equal_their_definitions(check, what):
     import anemone_amd as amd
     print("selfcheck", check, what, flush=True)
