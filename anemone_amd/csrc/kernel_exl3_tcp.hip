@@ -326,8 +326,6 @@ __device__ static __forceinline__ void tcp_chunk_load(const unsigned char *base,
 
 #define TCP_STAGE_COLUMN_BYTES (TCP_STEP_INPUTS * 2u)
 #define TCP_STAGE_BYTES (EXL3_TCP_CHUNK_PAIRS * TCP_STAGE_COLUMN_BYTES)
-#define TCP_STAGE_GROUPS (EXL3_TCP_CHUNK_PAIRS / 8u) /* groups of eight columns: one 16-byte-a-lane load of a wavefront each */
-#define TCP_WAVE_GROUPS ((TCP_STAGE_GROUPS + TCP_GEMM_WAVES - 1u) / TCP_GEMM_WAVES)
 
 /* A wavefront's product of 64 outputs by the chunk's columns on the matrix instruction of 32 x 32 outputs
  * (v_mfma_f32_32x32x16_f16: A lane l row l % 32, k = 8 (l / 32) + e; B lane l column l % 32, the same k; D lane l

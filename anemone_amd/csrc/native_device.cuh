@@ -30,7 +30,7 @@
 #define NATIVE_WAVES 4u
 #define NATIVE_THREADS (NATIVE_WAVES * WAVE)
 
-/* memory into registers, 16 bytes or one byte a lane: the address is a base common to the wavefront plus the lane's own
+/* memory into registers, 16 bytes or a word a lane: the address is a base common to the wavefront plus the lane's own
  * byte offset (plus 1,024: the second half of a tile of one-byte weights). Assembly, like the loads into LDS beside which
  * they are counted: the compiler keeps no book on them, native_landed is the wait (so a kernel of these loads must spill
  * no vector register: one saved between its load and the wait is saved before it is filled, and the build refuses such
@@ -57,11 +57,6 @@ __device__ static __forceinline__ void load_16_second(uint4_t &into, const unsig
     } else {
         asm volatile("global_load_dwordx4 %0, %1, %2 offset:1024" : "=v"(into) : "v"(lane_offset), "s"(base) : "memory");
     }
-}
-
-__device__ static __forceinline__ void load_1(uint32_t &into, const unsigned char *base, uint32_t lane_offset)
-{
-    asm volatile("global_load_ubyte %0, %1, %2" : "=v"(into) : "v"(lane_offset), "s"(base) : "memory");
 }
 
 __device__ static __forceinline__ void load_4(uint32_t &into, const unsigned char *base, uint32_t lane_offset)
@@ -141,12 +136,6 @@ struct native_chain {
     __device__ static __forceinline__ T lds_read(uint32_t address)
     {
         return *(const __attribute__((address_space(3))) T *)(uintptr_t)address;
-    }
-
-    template <typename T>
-    __device__ static __forceinline__ void lds_write(uint32_t address, T value)
-    {
-        *(__attribute__((address_space(3))) T *)(uintptr_t)address = value;
     }
 
     /* The scale words of a column lie in that column's own row: asked for a step at a time they are a cache line a column for
@@ -395,11 +384,10 @@ struct native_chain {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); /* the stage is read before the next barrier */
     }
 
-    /* how many loads may be outstanding at the top of a K step for its columns and weights to have landed: native_waits.h */
-    /* inside a step: the weights asked for at its top, ahead of the barrier and the columns (in the middle of the matrix
-     * instructions 4-bit weights take the same time and 18 registers more, one-byte weights a quarter longer) */
-    static constexpr bool WEIGHTS_FIRST = true;
-    template <uint32_t LIVE> using waits = native_waits<SLOTS, DEPTH, WEIGHTS_FIRST, vector_loads(LIVE), WEIGHT_LOADS>;
+    /* How many loads may be outstanding at the top of a K step for its columns and weights to have landed. Inside a step the
+     * weights are asked for at its top, ahead of the barrier and the columns (in the middle of the matrix instructions 4-bit
+     * weights take the same time and 18 registers more, one-byte weights a quarter longer). */
+    template <uint32_t LIVE> using waits = native_waits<SLOTS, DEPTH, vector_loads(LIVE), WEIGHT_LOADS>;
 
     /* s_waitcnt takes its count as a constant: one instruction a count that loads_behind can come to */
     template <uint32_t LIVE, uint32_t WEIGHTS = 0, uint32_t VECTORS = 0>

@@ -11,35 +11,32 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
-# (SLOTS, DEPTH, WEIGHTS_FIRST, VECTOR_LOADS, WEIGHT_LOADS) of the instances in kernel_native_linear.hip: VECTOR_LOADS is
-# 2 loads a column block a wavefront brings (one or two) and one of scale words; WEIGHT_LOADS the tiles' halves and the
-# scale loads of a wavefront's strip
+# (SLOTS, DEPTH, VECTOR_LOADS, WEIGHT_LOADS) of the instances in kernel_native_linear.hip: VECTOR_LOADS is a load for each
+# two live column blocks and one of scale words; WEIGHT_LOADS the tiles' halves and, of 4-bit weights, the scale words of a
+# wavefront's strip (one-byte weights' scale words come for many steps together, outside the count)
 INSTANCES = {
-    "E2M1 gate/up of whole strips (8 tiles, 2 scale words; 64 columns)": (2, 2, False, 3, 10),
-    "E2M1 down of whole strips (8 tiles, 2 scale words)": (2, 2, False, 3, 10),
-    "E2M1 gate/up (4 tiles, 2 scale words; 64 columns)": (3, 2, False, 3, 6),
-    "E2M1 down (4 tiles, 1 scale word)": (3, 2, False, 3, 5),
-    "E4M3 gate/up and down (2 tiles of two halves, 2 scale bytes; 128 columns)": (3, 3, True, 5, 6),
-    "E4M3_BLOCK128 down (2 tiles of two halves, 1 scale)": (3, 3, True, 5, 5),
-    **{"one-byte gate/up, %d loads of columns" % loads: (2, 2, True, loads, 4) for loads in (2, 3, 4, 5)},
-    **{"one-byte down, %d loads of columns" % loads: (3, 3, True, loads, 4) for loads in (2, 3, 4, 5)},
-    **{"E2M1, weights ahead of the columns: %d sets, %d loads of columns, %d of weights" % case: (case[0], 2, True, case[1], case[2])
-       for case in ((2, 2, 10), (2, 3, 10), (3, 2, 6), (3, 3, 6), (3, 2, 5), (3, 3, 5))},
-    "four sets of weight registers (measured, not kept)": (4, 3, True, 5, 6),
-    "six sets": (6, 3, True, 5, 6),
-    "weights behind the columns at three stages": (4, 3, False, 5, 6),
+    **{"E2M1 whole strips, gate/up and down (8 tiles, 2 scale words), %d loads of columns" % loads: (2, 2, loads, 10) for loads in (2, 3)},
+    **{"E2M1 narrow gate/up (4 tiles, 2 scale words), %d loads of columns" % loads: (3, 2, loads, 6) for loads in (2, 3)},
+    **{"E2M1 narrow down (4 tiles, 1 scale word), %d loads of columns" % loads: (3, 2, loads, 5) for loads in (2, 3)},
+    **{"one-byte gate/up (2 tiles of two halves), %d loads of columns" % loads: (2, 2, loads, 4) for loads in (2, 3, 4, 5)},
+    **{"one-byte down (2 tiles of two halves), %d loads of columns" % loads: (3, 3, loads, 4) for loads in (2, 3, 4, 5)},
+    # other parameters the formula allows
+    "three sets, three stages, 6 loads of weights": (3, 3, 5, 6),
+    "three sets, three stages, 5 loads of weights": (3, 3, 5, 5),
+    "four sets of weight registers": (4, 3, 5, 6),
+    "six sets": (6, 3, 5, 6),
 }
 MOST_TOTAL = 24
 
 HARNESS = r"""
 #include <cstdio>
 #include "native_waits.h"
-template <uint32_t S, uint32_t D, bool W, uint32_t V, uint32_t L>
+template <uint32_t S, uint32_t D, uint32_t V, uint32_t L>
 static void table(const char *name)
 {
     for (uint32_t total = 1; total <= %d; total++) {
         for (uint32_t step = 0; step < total; step++) {
-            std::printf("%%s %%u %%u %%u\n", name, total, step, native_waits<S, D, W, V, L>::loads_behind(step, total));
+            std::printf("%%s %%u %%u %%u\n", name, total, step, native_waits<S, D, V, L>::loads_behind(step, total));
         }
     }
 }
@@ -54,8 +51,8 @@ int main()
 @pytest.fixture(scope="module")
 def tables(tmp_path_factory):
     folder = tmp_path_factory.mktemp("waits")
-    calls = "\n".join('    table<%du, %du, %s, %du, %du>("%d");' % (s, d, "true" if w else "false", v, l, index)
-                      for index, (s, d, w, v, l) in enumerate(INSTANCES.values()))
+    calls = "\n".join('    table<%du, %du, %du, %du>("%d");' % (s, d, v, l, index)
+                      for index, (s, d, v, l) in enumerate(INSTANCES.values()))
     source = folder / "waits.cpp"
     source.write_text(HARNESS % (MOST_TOTAL, calls))
     program = folder / "waits"
@@ -69,7 +66,7 @@ def tables(tmp_path_factory):
     return found
 
 
-def issue_order(slots, depth, weights_first, total):
+def issue_order(slots, depth, total):
     """The loads of a chain of `total` steps in the order the loop issues them, as (kind, step) with kind "V" (a step's
     columns) or "W" (its weights), and for every step the number of loads issued before its wait."""
     order, before_wait = [], []
@@ -83,16 +80,16 @@ def issue_order(slots, depth, weights_first, total):
         before_wait.append(len(order))
         ask = [("W", step + slots - 1)] if step + slots - 1 < total else []
         columns = [("V", step + depth - 1)] if step + depth - 1 < total else []
-        order += ask + columns if weights_first else columns + ask
+        order += ask + columns
     return order, before_wait
 
 
 @pytest.mark.parametrize("index,name", list(enumerate(INSTANCES)))
 def test_a_steps_wait_leaves_its_loads_landed_and_no_more(tables, index, name):
-    slots, depth, weights_first, vector_loads, weight_loads = INSTANCES[name]
+    slots, depth, vector_loads, weight_loads = INSTANCES[name]
     size = {"V": vector_loads, "W": weight_loads}
     for total in range(1, MOST_TOTAL + 1):
-        order, before_wait = issue_order(slots, depth, weights_first, total)
+        order, before_wait = issue_order(slots, depth, total)
         assert sorted(order) == sorted([("V", k) for k in range(total)] + [("W", k) for k in range(total)]), "every step's loads are asked for once"
         for step in range(total):
             issued = order[:before_wait[step]]
@@ -106,7 +103,7 @@ def test_a_steps_wait_leaves_its_loads_landed_and_no_more(tables, index, name):
 def test_the_counts_are_ones_the_kernel_has_an_instruction_for(tables):
     """wait_behind() of native_device.cuh has one s_waitcnt for W x WEIGHT_LOADS + V x VECTOR_LOADS with W below SLOTS and V
     below DEPTH - 1 (at least one): every count the formula gives is one of them."""
-    for index, (slots, depth, weights_first, vector_loads, weight_loads) in enumerate(INSTANCES.values()):
+    for index, (slots, depth, vector_loads, weight_loads) in enumerate(INSTANCES.values()):
         reachable = {w * weight_loads + v * vector_loads for w in range(slots) for v in range(max(1, depth - 1))}
         counts = {count for (i, _, _), count in tables.items() if i == index}
         assert counts <= reachable, (index, sorted(counts - reachable))
