@@ -231,6 +231,14 @@ result_status router_select_prepare(const struct router_description *description
     return STATUS_OK;
 }
 
+/* Whether the record names a kernel of its own there. A member that a caller left zero is the handle of whatever kernel was
+ * prepared first: where that is another of the record's, it is not this one. */
+static bool projection_has(const struct router_kernels_record *kernels, uint32_t handle)
+{
+    return handle != BACKEND_NO_KERNEL && handle != kernels->select && handle != kernels->wide_select && handle != kernels->wide_count &&
+           handle != kernels->wide_place && handle != kernels->wide_jobs && handle != kernels->wide_small && handle != kernels->projection;
+}
+
 /* the blocks of the fuller CUs, of each form: see PROJECTION_SPLIT_BLOCKS_OF_TILE for both sides' times */
 static bool projection_takes_split(uint32_t row_count, uint32_t expert_count)
 {
@@ -270,7 +278,8 @@ result_status router_projection_prepare(const struct router_projection_descripti
     /* from nine rows on, the chains on the matrix unit: 16 experts by 16 rows a block, or by 64 */
     if (description->row_count >= PROJECTION_SPLIT_LEAST_ROWS && description->expert_count % 16u == 0 &&
         description->hidden % PROJECTION_STAGE_INPUTS == 0) {
-        const bool has_split = kernels->projection_split != BACKEND_NO_KERNEL, has_tiles = kernels->projection_tiles != BACKEND_NO_KERNEL;
+        const bool has_tiles = projection_has(kernels, kernels->projection_tiles);
+        const bool has_split = projection_has(kernels, kernels->projection_split) && kernels->projection_split != kernels->projection_tiles;
         if (has_split && (!has_tiles || projection_takes_split(description->row_count, description->expert_count))) {
             launch_fill(launch_out, kernels->projection_split, description->expert_count / 16u,
                         (description->row_count + PROJECTION_SPLIT_ROWS - 1u) / PROJECTION_SPLIT_ROWS, 1, PROJECTION_TILE_THREADS, 0, &record,

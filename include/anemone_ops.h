@@ -12,6 +12,9 @@
  *   expert_producer_prepare              include/anemone/expert_fused.h:51-101         (source/expert_fused.c)
  * Contract of every prepare function (include/anemone/linear.h:17-48): arithmetic on a description, the arena is a
  * number; pure and reentrant; a refusal is a status with one error line on stderr and the launch table untouched.
+ * A record of kernel handles (*_kernels) is filled by its *_kernels_prepare of the same build and by nothing else: zero is
+ * a kernel's handle, and a kernel that is not there is BACKEND_NO_KERNEL. A program built against a header whose record
+ * is shorter is built again.
  * What differs from the reference: shapes (experts, picks, hidden, widths) are run-time members instead of one
  * model's compile-time constants, and the arithmetic class accepted is ARITHMETIC_CLASS_GFX950.
  */

@@ -321,6 +321,12 @@ def test_router_projection_prepare_geometry(fake):
     assert prepared(257, 512, 64) == (0, "router_projection_tiles", [4, 5, 1], 256)
     tiles, kernels.projection_split, kernels.projection_tiles = kernels.projection_tiles, split, amd.BACKEND_NO_KERNEL  # without the other
     assert prepared(4096, 512, 64) == (0, "router_projection_split", [4, 256, 1], 256)
+    # a member left zero: the first handle there is, here the select's, which never runs as a projection
+    assert kernels.select == 0
+    kernels.projection_split, kernels.projection_tiles = 0, tiles
+    assert prepared(100, 512, 64)[1:3] == ("router_projection", [8, 25, 1]) and prepared(300, 512, 64)[1] == "router_projection_tiles"
+    kernels.projection_split = kernels.projection_tiles = 0
+    assert prepared(300, 512, 64)[1:3] == ("router_projection", [8, 75, 1])
     kernels.projection_split, kernels.projection_tiles = amd.BACKEND_NO_KERNEL, tiles
     status, name, grid, block = prepared(8, 4096, 256)  # a thin step: a row a block
     assert (status, name, grid) == (0, "router_projection", [32, 8, 1])
