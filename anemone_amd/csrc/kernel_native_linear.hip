@@ -44,7 +44,7 @@ __device__ static __forceinline__ void native_vectors_of(const struct wide_pair 
 
 /* grid (ceil(output_size / (4 strips)), tile_count), block 256; a strip is STRIP tiles of gate and STRIP of up */
 /* sets of weight registers and stages of columns: 4-bit weights 2 and 2, with strips of four gate and four up tiles (eight
- * of down) at two wavefronts a SIMD (232 registers, 128 of them sums): a column block's operand read from LDS and its
+ * of down) at two wavefronts a SIMD (241 registers, 128 of them sums): a column block's operand read from LDS and its
  * permutations serve eight matrix instructions and not four (8192 rows of 4096 x 2048 x 256 experts: gate/up 1157 -> 1096
  * us, down 651 -> 625, against strips of half as many, three sets and three wavefronts; both with columns turned in place). One-byte weights: gate/up 2 and 2
  * at three wavefronts a SIMD (143 registers, 165 with float32 scales), down 3 and 3 at two (215 and 222): 2048 rows of
@@ -68,13 +68,15 @@ __device__ static __forceinline__ void native_expert_gate_up(const struct wide_e
     const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     struct wide_expert_tile tile;
     uint32_t pair_count = 0, block_strip = 0;
-    if (!order_block_of<GROUP, false, !BYTES>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count)) {
+    bool alone = false;
+    if (!order_block_of<GROUP, false, !BYTES>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count, &alone)) {
         return;
     }
     const struct wide_pair *pairs = (const struct wide_pair *)(arena + arguments.pairs_offset) + tile.first_pair;
     uint32_t code_vectors[2u * chain_type::WAVE_BLOCKS], exponent_vectors[chain_type::WAVE_BLOCKS];
     native_vectors_of<chain_type>(pairs, pair_count, arguments.pairs_per_row, wave, lane, code_vectors, exponent_vectors, columns);
     chain_type chain_of;
+    chain_of.once = alone;
     const unsigned char *const matrices[2] = {arena + tile.gate_offset, arena + tile.up_offset};
     uint32_t tile0 = 0;
     chain_of.place(matrices, arguments.output_size, arguments.input_size, block_strip, arena + arguments.codes_offset,
@@ -103,13 +105,15 @@ __device__ static __forceinline__ void native_expert_down(const struct wide_expe
     const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     struct wide_expert_tile tile;
     uint32_t pair_count = 0, block_strip = 0;
-    if (!order_block_of<GROUP, true, BY_RUN>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count)) {
+    bool alone = false;
+    if (!order_block_of<GROUP, true, BY_RUN>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count, &alone)) {
         return;
     }
     const struct wide_pair *pairs = (const struct wide_pair *)(arena + arguments.pairs_offset) + tile.first_pair;
     uint32_t code_vectors[2u * chain_type::WAVE_BLOCKS], exponent_vectors[chain_type::WAVE_BLOCKS]; /* the vectors are the pairs' hidden vectors */
     native_vectors_of<chain_type>(pairs, pair_count, 1u, wave, lane, code_vectors, exponent_vectors, columns);
     chain_type chain_of;
+    chain_of.once = alone;
     const unsigned char *const matrices[1] = {arena + tile.down_offset};
     uint32_t tile0 = 0;
     chain_of.place(matrices, arguments.output_size, arguments.input_size, block_strip, arena + arguments.codes_offset,

@@ -35,10 +35,7 @@
  * they are counted: the compiler keeps no book on them, native_landed is the wait (so a kernel of these loads must spill
  * no vector register: one saved between its load and the wait is saved before it is filled, and the build refuses such
  * a kernel). ONCE: the bytes are read by this
- * block alone (an expert's one-byte weights in a block that holds all its pairs; 4-bit weights where an expert has few
- * pairs: 700 rows of 4096 x 2048 x 256 experts gate/up 413 -> 381 us, down 225 -> 212, 300 rows 390 -> 351, 208 -> 189, 500
- * rows of Zipf(1.1) loads 408 -> 389, 217 -> 209): asked for as a stream, so that they do not push the columns, which every
- * block of the expert reads, out of the level-2 cache. */
+ * block alone, and are asked for as a stream (native_chain::once). */
 template <bool ONCE>
 __device__ static __forceinline__ void load_16(uint4_t &into, const unsigned char *base, uint32_t lane_offset)
 {
@@ -88,7 +85,7 @@ struct native_chain {
     static_assert(COLUMN_BLOCKS == 4u || COLUMN_BLOCKS == 8u, "a wavefront brings one or two column blocks");
     static constexpr uint32_t STRIP = STRIP_TILES;
     static constexpr uint32_t TILES = MATRICES * STRIP;
-    static constexpr bool ONCE = BYTES || TILES != 8u; /* the narrow strips of 4-bit weights are for experts of few pairs, as a rule one tile */
+    static constexpr bool STREAMS = BYTES || TILES != 8u; /* whole strips of 4-bit weights are for experts of many tiles: no instance of them streams */
     static constexpr uint32_t STEP_BYTES = BYTES ? BYTE_STEP_BYTES : NIBBLE_STEP_BYTES;
     static constexpr uint32_t HALVES = STEP_BYTES / 1024u;
     static constexpr uint32_t WAVE_BLOCKS = COLUMN_BLOCKS / NATIVE_WAVES;     /* column blocks whose scale words a wavefront brings */
@@ -125,6 +122,15 @@ struct native_chain {
         uint32_t scale[BYTES ? 1 : SCALE_LOADS]; /* 4-bit weights */
     };
 
+    /* STREAMS: whether the block holds all of its expert's pairs (the same in every lane). Then no other block reads these weights,
+     * and they are asked for as a stream, so that they do not push the columns, which every strip's block reads, out of the level-2
+     * cache; where an expert has more blocks, a streamed line is read from memory again. 4096 x 2048, gate/up and down, us, no weight
+     * as a stream | every weight | by this rule: FP8 of 2048 rows, 256 experts 919 and 446 | 880 and 430 | 887 and 430; 4096 rows 1160
+     * and 605 | 1350 and 658 | 1138 and 600; 4096 rows of Zipf(1.1) loads 1251 and 656 | 1414 and 700 | 1222 and 652; 2048 rows of 64
+     * experts 463 and 257 | 572 and 282 | 470 and 260; 500 Zipf rows of 128 experts 421 and 219 | 410 and 211 | 403 and 209 (float32 scales:
+     * the same picture). 4-bit weights in narrow strips, 300 rows of 256 experts 386 and 210 | 361 and 196 | 360 and 195; 700
+     * Zipf rows 431 and 228 | 434 and 233 | 410 and 221. */
+    bool once = false;
     const unsigned char *words[MATRICES], *scales[MATRICES], *codes, *exponents;
     uint32_t step_stride, scale_stride; /* from a tile's K step to its next; from a group's scale words to the next group's */
     uint32_t window, wave, tile_bytes, group_bytes, word_offset, scale_offset[BYTES && !B128 ? STRIP : 1], code_shift, codes_offset[2u * WAVE_BLOCKS], exponents_offset[WAVE_BLOCKS];
@@ -175,6 +181,7 @@ struct native_chain {
     }
 
     /* the wavefront's weights and scale codes of K step `at` into a set of registers */
+    template <bool ONCE>
     __device__ __forceinline__ void issue_weights(slot &into, uint32_t at) const
     {
 #pragma unroll
@@ -408,7 +415,7 @@ struct native_chain {
 
     /* K step `step` of `total` out of set K of the wavefront's sets of weight registers; the weights of step
      * `step` + SLOTS - 1 take the set the step before this one used */
-    template <uint32_t LIVE, uint32_t K>
+    template <uint32_t LIVE, bool ONCE, uint32_t K>
     __device__ __forceinline__ void one_step(uint32_t step, uint32_t total, slot (&sets)[SLOTS], uint32_t (&held)[SCALE_LOADS], uint32_t round, float4_t (&chain)[TILES][COLUMN_BLOCKS]) const
     {
         wait_behind<LIVE>(waits<LIVE>::loads_behind(step, total));
@@ -421,7 +428,7 @@ struct native_chain {
         }
         const auto ask = [&]() { /* a function of its own: the compiler spills registers of the same lines without one */
             if (step + SLOTS - 1u < total) {
-                issue_weights(sets[(K + SLOTS - 1u) % SLOTS], step + SLOTS - 1u);
+                issue_weights<ONCE>(sets[(K + SLOTS - 1u) % SLOTS], step + SLOTS - 1u);
             }
         };
         ask(); /* into the set the step before this one used: nothing of the block's is waited for */
@@ -438,29 +445,29 @@ struct native_chain {
         }
     }
 
-    template <uint32_t LIVE, uint32_t K>
+    template <uint32_t LIVE, bool ONCE, uint32_t K>
     __device__ __forceinline__ void round_of_steps(uint32_t step, uint32_t total, slot (&sets)[SLOTS], uint32_t (&held)[SCALE_LOADS], uint32_t round, float4_t (&chain)[TILES][COLUMN_BLOCKS]) const
     {
         if (step + K < total) {
-            one_step<LIVE, K>(step + K, total, sets, held, round, chain);
+            one_step<LIVE, ONCE, K>(step + K, total, sets, held, round, chain);
         }
         if constexpr (K + 1u < SLOTS) {
-            round_of_steps<LIVE, K + 1u>(step, total, sets, held, round, chain);
+            round_of_steps<LIVE, ONCE, K + 1u>(step, total, sets, held, round, chain);
         }
     }
 
-    template <uint32_t K>
+    template <bool ONCE, uint32_t K>
     __device__ __forceinline__ void first_weights(uint32_t total, slot (&sets)[SLOTS]) const
     {
         if (K < total) {
-            issue_weights(sets[K], K);
+            issue_weights<ONCE>(sets[K], K);
         }
         if constexpr (K + 2u < SLOTS) {
-            first_weights<K + 1u>(total, sets);
+            first_weights<ONCE, K + 1u>(total, sets);
         }
     }
 
-    template <uint32_t LIVE>
+    template <uint32_t LIVE, bool ONCE>
     __device__ __forceinline__ void steps(uint32_t total, float4_t (&chain)[TILES][COLUMN_BLOCKS]) const
     {
         slot sets[SLOTS];
@@ -478,15 +485,27 @@ struct native_chain {
                 issue_vectors<LIVE>(k, k);
             }
         }
-        first_weights<0>(total, sets);
+        first_weights<ONCE, 0>(total, sets);
         for (uint32_t step = 0; step < total; step += SLOTS) {
             if (BYTES && step == round + SCALE_ROUND) { /* inputs past 128 SCALE_ROUND */
                 round = step;
                 issue_weight_scales(held, round);
                 wait_loads<0>();
             }
-            round_of_steps<LIVE, 0>(step, total, sets, held, round, chain);
+            round_of_steps<LIVE, ONCE, 0>(step, total, sets, held, round, chain);
         }
+    }
+
+    template <uint32_t LIVE>
+    __device__ __forceinline__ void steps_of(uint32_t total, float4_t (&chain)[TILES][COLUMN_BLOCKS]) const
+    {
+        if constexpr (STREAMS) {
+            if (once) {
+                steps<LIVE, true>(total, chain);
+                return;
+            }
+        }
+        steps<LIVE, false>(total, chain);
     }
 
     /* live_blocks: the column blocks that hold a pair, the same in every lane of the block */
@@ -494,21 +513,21 @@ struct native_chain {
     {
         if constexpr (COLUMN_BLOCKS == 4u) {
             switch (live_blocks) {
-            case 1u: steps<1>(total, chain); break;
-            case 2u: steps<2>(total, chain); break;
-            case 3u: steps<3>(total, chain); break;
-            default: steps<4>(total, chain); break;
+            case 1u: steps_of<1>(total, chain); break;
+            case 2u: steps_of<2>(total, chain); break;
+            case 3u: steps_of<3>(total, chain); break;
+            default: steps_of<4>(total, chain); break;
             }
         } else {
             switch (live_blocks) {
-            case 1u: steps<1>(total, chain); break;
-            case 2u: steps<2>(total, chain); break;
-            case 3u: steps<3>(total, chain); break;
-            case 4u: steps<4>(total, chain); break;
-            case 5u: steps<5>(total, chain); break;
-            case 6u: steps<6>(total, chain); break;
-            case 7u: steps<7>(total, chain); break;
-            default: steps<8>(total, chain); break;
+            case 1u: steps_of<1>(total, chain); break;
+            case 2u: steps_of<2>(total, chain); break;
+            case 3u: steps_of<3>(total, chain); break;
+            case 4u: steps_of<4>(total, chain); break;
+            case 5u: steps_of<5>(total, chain); break;
+            case 6u: steps_of<6>(total, chain); break;
+            case 7u: steps_of<7>(total, chain); break;
+            default: steps_of<8>(total, chain); break;
             }
         }
     }

@@ -15,7 +15,7 @@
  *
  * The 4-bit launches take this order, but for the narrow down's (BY_RUN; 8192 rows of 4096 x 2048 x 256 experts in gfx950's lane order: 5.5 -> 3.4 GB
  * fetched by a gate/up launch). One-byte launches keep the blocks as dealt: their tiles are taken two at a time, so that
- * an expert's matrix is read about once either way, and the second look at the table costs more (2 to 4 %).
+ * the matrix of an expert of up to 128 pairs is read once either way, and the second look at the table costs more (2 to 4 %).
  *
  * Where the runs begin follows from the tile table alone: tiles follow each other in a run where their offsets agree and
  * the pairs of the second follow a full first. A table's unused tiles lie behind its used ones, so the launch's work is
@@ -55,7 +55,7 @@ __device__ static __forceinline__ uint32_t order_used_tiles(const struct wide_ex
  * runs are tiles of one down matrix, else of one gate and up. Returns false for a block that has nothing to do. Every
  * lane of a wavefront calls; strips = gridDim.x, tile_count = gridDim.y. Two round trips to the table: the used tiles, and
  * the ORDER_WINDOW tiles around the block's own, a lane a tile (runs are cut where a window ends). alone_out: whether the
- * block's tile is a run of its own (as far as the block sees: a matter of speed, not of results). */
+ * block's tiles are all of their run (as far as the block sees: a matter of speed, not of results). */
 template <uint32_t GROUP, bool DOWN, bool BY_RUN>
 __device__ static __forceinline__ bool order_block_of(const struct wide_expert_tile *tiles, uint32_t tile_count, uint32_t lane, uint32_t &strip_out,
                                                       struct wide_expert_tile &tile_out, uint32_t &pair_count_out, bool *alone_out = nullptr)
@@ -128,7 +128,7 @@ __device__ static __forceinline__ bool order_block_of(const struct wide_expert_t
     tile_out.pair_count = of_lane(mine.pair_count, tile);
     pair_count_out = tile_out.pair_count;
     if (alone_out != nullptr) {
-        *alone_out = length == 1u;
+        *alone_out = length <= GROUP;
     }
     if constexpr (GROUP == 2u) {
         if (tile + 1u < first + length) {

@@ -139,6 +139,8 @@ def test_native_equals_the_reference_lay_out_byte_for_byte(amd, card, hidden, in
     (8320, 128, 2, 70, B128), (128, 8320, 2, 70, B128),
     # one expert's pairs: every number of column blocks of a block of two tiles, each with its own share of a wavefront's loads
     *[(512, 256, 1, rows, -fmt) for rows in (9, 30, 41, 64, 70, 96, 100, 128) for fmt in (E4M3, B128)],
+    # the same where the expert has a full block before it: weights that two blocks read are not asked for as a stream
+    *[(512, 256, 1, 128 + rows, -fmt) for rows in (9, 30, 41, 64, 70, 96, 100, 128) for fmt in (E4M3, B128)],
 ])
 def test_native_chunks_of_scale_words(amd, card, hidden, inner, picks, rows, fmt):
     test_native_equals_the_reference_lay_out_byte_for_byte(amd, card, hidden, inner, 64, picks, rows, rows, fmt)
