@@ -325,7 +325,7 @@ struct strip_chain {
                 /* lane L of a 16-byte load lands at bytes 16 L of the tile's stage and asks for the piece
                  * p = L ^ ((L / 8) % 4) of the step: LDS has 32 banks of 4 bytes, and the pieces of one T (p = 32 ld + 4 G + T,
                  * G = 0 .. 7) then lie in eight different groups of four banks for the sixteen lanes that read them together
-                 * (measured: SQ_LDS_BANK_CONFLICT of the wide gate/up launch 1.68e8 -> 1.9e7 cycles); every 16 lanes still read
+                 * (SQ_LDS_BANK_CONFLICT of a wide gate/up launch with nothing else in conflict: 1.68e8 -> 1.9e7 cycles); every 16 lanes still read
                  * 256 contiguous bytes of memory */
                 piece_offset = 16u * (lane ^ ((lane >> 3) & 3u));
                 /* scales: uint32 [tile][load][G]; lane L of the 4-byte load: tile L / 16, word L % 16 = 8 ld + G */

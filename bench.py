@@ -31,31 +31,22 @@ HBM_PEAK_GBS = 8000.0
 MEASURED_TRAFFIC_BYTES = {
     ("exl3_decode", 8): 375.1e6 + 4.2e6,
     ("exl3_linear", 1): 8.601e6 + 0.016e6,
-    ("fp4_decode", 32): 1434.7e6 + 1.0e6,
-    ("fp8_decode", 32): 2746.8e6 + 1.0e6,
-    ("fp4_prefill", 8192): 3104.1e6 + 421.3e6,
-    ("fp8_prefill", 2048): 5655.0e6 + 117.1e6,
-    ("expert_join", 8192): 877.7e6 + 402.7e6,
-    ("fp8_decode_block128", 64): 3713.0e6 + 2.1e6,
-    ("fp8_prefill_block128", 2048): 5386.8e6 + 67.2e6,
-    ("fp4_prefill_native", 8192): 3445.3e6 + 413.7e6,
-    ("exl3_prefill", 4096): 2858.6e6 + 538.5e6,
-    ("fp8_prefill_native", 2048): 4725.5e6 + 113.1e6,
-    ("fp8_prefill_block128_native", 2048): 4706.1e6 + 67.1e6,
-    ("fp4_decode_native", 32): 1434.2e6 + 1.0e6,
-    ("fp8_decode_native", 32): 2746.7e6 + 1.0e6,
+    ("fp4_decode", 32): 1428.3e6 + 1.0e6,
+    ("fp8_decode", 32): 2739.0e6 + 1.0e6,
+    ("fp4_prefill", 8192): 3261.9e6 + 470.8e6,
+    ("fp8_prefill", 2048): 5231.7e6 + 116.8e6,
+    ("expert_join", 8192): 877.8e6 + 402.7e6,
+    ("fp8_decode_block128", 1): 134.6e6,
+    ("fp8_decode_block128", 64): 3697.4e6 + 2.1e6,
+    ("fp8_prefill_block128", 2048): 5227.1e6 + 67.1e6,
+    ("fp4_prefill_native", 8192): 3681.1e6 + 415.0e6,
+    ("exl3_prefill", 4096): 2735.2e6 + 536.9e6,
+    ("fp8_prefill_native", 2048): 4723.5e6 + 112.4e6,
+    ("fp8_prefill_block128_native", 2048): 4704.8e6 + 67.1e6,
+    ("fp4_decode_native", 32): 1428.2e6 + 1.0e6,
+    ("fp8_decode_native", 32): 2739.0e6 + 1.0e6,
 }
-TRAFFIC_SOURCE = {
-    "exl3_linear": "profiles/exl3_down_k4_thin_single_linear.md",
-    "exl3_decode": "profiles/exl3_tc_products_decode8.md", "exl3_prefill": "profiles/exl3_tcp_gemm_prefill4096.md", "fp4_decode": "profiles/expert_gate_up_fp4_fp8_decode32.md",
-    "fp8_decode": "profiles/expert_gate_up_fp4_fp8_decode32.md", "fp4_prefill": "profiles/wide_expert_fp4_fp8_prefill.md",
-    "fp8_prefill": "profiles/wide_expert_fp4_fp8_prefill.md",
-    "fp8_decode_block128": "profiles/expert_b128_fp8_block128_decode64_prefill2048.md",
-    "fp8_prefill_block128": "profiles/expert_b128_fp8_block128_decode64_prefill2048.md",
-    "fp4_prefill_native": "profiles/native_expert_fp4_fp8_gfx950_lane_order.md", "fp8_prefill_native": "profiles/native_expert_fp4_fp8_gfx950_lane_order.md",
-    "fp8_prefill_block128_native": "profiles/native_expert_b128_gfx950_prefill2048.md",
-    "fp4_decode_native": "profiles/native_expert_fp4_fp8_gfx950_lane_order.md", "fp8_decode_native": "profiles/native_expert_fp4_fp8_gfx950_lane_order.md",
-}
+TRAFFIC_SOURCE = "profiles/launch_counters.md (counter bytes of the profiled run, not of this one)"
 HIDDEN, INNER, EXPERTS, PICKS, ROWS = 4096, 2048, 256, 8, 8
 CONFIG = 1
 
@@ -288,7 +279,7 @@ def fp4_decode(amd, workloads, arguments, fp8=False, prefill=False):
         key = (key[0] + "_native", rows)
     if key in MEASURED_TRAFFIC_BYTES and (prefill or (arguments.gate_up_slices, arguments.down_slices) == (4, 2)):
         result["roofline"]["traffic"] = MEASURED_TRAFFIC_BYTES[key]
-        result["roofline"]["traffic_source"] = TRAFFIC_SOURCE[key[0]] + " (counter bytes of the profiled run, not of this one)"
+        result["roofline"]["traffic_source"] = TRAFFIC_SOURCE
     if prefill:
         pairs = rows * PICKS
         gate_up_flops, down_flops = 2.0 * pairs * 2 * HIDDEN * INNER, 2.0 * pairs * HIDDEN * INNER
@@ -496,7 +487,7 @@ def exl3_prefill(amd, workloads, arguments):
     }
     if ("exl3_prefill", rows) in MEASURED_TRAFFIC_BYTES and arguments.zipf_strength <= 0.0:
         result["roofline"]["traffic"] = MEASURED_TRAFFIC_BYTES[("exl3_prefill", rows)]
-        result["roofline"]["traffic_source"] = TRAFFIC_SOURCE["exl3_prefill"] + " (counter bytes of the profiled run, not of this one)"
+        result["roofline"]["traffic_source"] = TRAFFIC_SOURCE
     if not arguments.no_cpu:
         import ctypes as C
         import _oracle as o
@@ -591,7 +582,7 @@ def exl3_decode(amd, workloads, arguments):
         "roofline": {"bound": "hbm", "kernel": "exl3_tc_products (gate/up pass)", "achieved": achieved,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                      "traffic": MEASURED_TRAFFIC_BYTES[("exl3_decode", ROWS)],
-                     "traffic_source": TRAFFIC_SOURCE["exl3_decode"] + " (counter bytes of the profiled run, not of this one)",
+                     "traffic_source": TRAFFIC_SOURCE,
                      "algorithmic_bytes_per_launch": int(gate_up_bytes), "launch_us": gate_up_us},
     }
 
@@ -689,7 +680,7 @@ def exl3_linear(amd, workloads, arguments):
                    "step_GBps": algorithmic / (seconds / arguments.steps) / 1e9},
         "roofline": {"bound": "hbm", "kernel": "exl3_down_k4_thin (the product launch)", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": MEASURED_TRAFFIC_BYTES[("exl3_linear", 1)],
-                     "traffic_source": TRAFFIC_SOURCE["exl3_linear"] + " (counter bytes of the profiled run, not of this one)",
+                     "traffic_source": TRAFFIC_SOURCE,
                      "algorithmic_bytes_per_launch": int(algorithmic), "launch_us": product_us},
     }
     got = card.download(record.output_offset, n * 4, np.float32)
