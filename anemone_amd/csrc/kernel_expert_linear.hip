@@ -44,8 +44,8 @@
  * 256 experts, 64 rows of float32-scaled FP8 592 and 304 | 549 and 281 | 550 and 281; 32 rows of FP4 234 and 125 | 213 and 112 | 213
  * and 112; 64 experts, 64 rows of FP8 182 and 103 | 193 and 105 | 174 and 100; of FP8 with Zipf(1.1) loads in lane order 192 and
  * 108 | 209 and 114 | 182 and 103, with eight experts of eight jobs each (2048 x 1024) 38 and 25 | 40 and 25 | 34 and 24; FP4 107 and
- * 66 | 105 and 65 | 104 and 65. (An expert of exactly eight rows counts as one of more. With both neighbours and the table's end looked at it would not:
- * the same times, and 0.3 us more in a launch of few jobs.) */
+ * 66 | 105 and 65 | 104 and 65. An expert of exactly eight rows counts as one of more; with both neighbours and the table's end
+ * looked at it would not, which gave the same times and 0.3 us more in a launch of few jobs. */
 __device__ static __forceinline__ bool job_alone(const struct expert_job_record *jobs, uint32_t index)
 {
     const struct expert_job_record *job = jobs + index, *before = jobs + (index != 0u ? index - 1u : 0u);
@@ -60,7 +60,7 @@ template <uint32_t S, bool BYTES, bool B128 = false, bool NATIVE = false>
 __device__ static __forceinline__ void expert_gate_up(const struct expert_gate_up_arguments &arguments,
                                                       unsigned char *arena, uint16_t *strip_hidden = nullptr)
 {
-    typedef strip_chain<2, BYTES, B128, NATIVE, true> chain_type;
+    typedef strip_chain<2, BYTES, B128, NATIVE> chain_type;
     constexpr uint32_t TILES = chain_type::TILES, STRIP = chain_type::STRIP;
     __shared__ __attribute__((aligned(16))) unsigned char window[S][chain_type::WINDOW_BYTES];
     static_assert(chain_type::WINDOW_BYTES >= TILES * WAVE * 16u, "a wavefront's sums fit its idle window");
@@ -80,17 +80,26 @@ __device__ static __forceinline__ void expert_gate_up(const struct expert_gate_u
     }
     const uint32_t steps = arguments.input_size / 128u;
     const uint32_t first = steps * slice / S, last = steps * (slice + 1u) / S;
-    chain_type chain_of;
-    chain_of.once = alone;
     const unsigned char *const matrices[2] = {arena + job->gate_offset, arena + job->up_offset};
-    chain_of.place(matrices, arguments.output_size, arguments.input_size, blockIdx.x, first, arena + arguments.codes_offset,
-                   arena + arguments.exponents_offset, rows, (uint32_t)(uintptr_t)(lds_pointer)&window[slice][0], lane);
     float4_t chain[TILES];
 #pragma unroll
     for (uint32_t tile = 0; tile < TILES; tile++) {
         chain[tile] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
     }
-    chain_of.whole(last - first, chain);
+    /* each instance forms the places it reads itself, its first loads among them (formed once ahead of both, the lane's would all
+     * stand in front of the first load: 3 % of a launch of short chains) */
+    const auto run = [&](auto chain_of) {
+        uint32_t own_lane = lane;
+        asm volatile("" : "+v"(own_lane));
+        chain_of.place(matrices, arguments.output_size, arguments.input_size, blockIdx.x, first, arena + arguments.codes_offset,
+                       arena + arguments.exponents_offset, rows, (uint32_t)(uintptr_t)(lds_pointer)&window[slice][0], own_lane);
+        chain_of.whole(last - first, chain);
+    };
+    if (alone) {
+        run(strip_chain<2, BYTES, B128, NATIVE, true>());
+    } else {
+        run(chain_type());
+    }
     /* the S chains meet in the windows, idle now: [slice][tile][lane] float4 */
     float4_t *sums = (float4_t *)&window[slice][0];
 #pragma unroll
@@ -148,7 +157,7 @@ template <uint32_t S, bool BYTES>
 __device__ static __forceinline__ void expert_gate_up_quantize(const struct expert_gate_up_quantize_arguments &arguments,
                                                                unsigned char *arena)
 {
-    typedef strip_chain<2, BYTES, false, false, true> chain_type;
+    typedef strip_chain<2, BYTES> chain_type;
     constexpr uint32_t STRIP_OUTPUTS = chain_type::STRIP * 16u;
     __shared__ uint16_t strip_hidden[LINEAR_MAXIMUM_ROWS][STRIP_OUTPUTS];
     __shared__ uint32_t routed[EXPERT_PRODUCER_MOST_PAIRS / 32u];
@@ -215,7 +224,7 @@ __device__ static __forceinline__ void expert_gate_up_quantize(const struct expe
 template <uint32_t S, bool BYTES, bool B128 = false, bool NATIVE = false>
 __device__ static __forceinline__ void expert_down(const struct expert_down_arguments &arguments, unsigned char *arena)
 {
-    typedef strip_chain<1, BYTES, B128, NATIVE, true> chain_type;
+    typedef strip_chain<1, BYTES, B128, NATIVE> chain_type;
     constexpr uint32_t TILES = chain_type::TILES, STRIP = chain_type::STRIP;
     __shared__ __attribute__((aligned(16))) unsigned char window[S][chain_type::WINDOW_BYTES];
     static_assert(chain_type::WINDOW_BYTES >= TILES * WAVE * 16u, "a wavefront's sums fit its idle window");
@@ -234,17 +243,26 @@ __device__ static __forceinline__ void expert_down(const struct expert_down_argu
     }
     const uint32_t steps = arguments.input_size / 128u;
     const uint32_t first = steps * slice / S, last = steps * (slice + 1u) / S;
-    chain_type chain_of;
-    chain_of.once = alone;
     const unsigned char *const matrices[1] = {arena + job->down_offset};
-    chain_of.place(matrices, arguments.output_size, arguments.input_size, blockIdx.x, first, arena + arguments.codes_offset,
-                   arena + arguments.exponents_offset, rows, (uint32_t)(uintptr_t)(lds_pointer)&window[slice][0], lane);
     float4_t chain[TILES];
 #pragma unroll
     for (uint32_t tile = 0; tile < TILES; tile++) {
         chain[tile] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
     }
-    chain_of.whole(last - first, chain);
+    /* each instance forms the places it reads itself, its first loads among them (formed once ahead of both, the lane's would all
+     * stand in front of the first load: 3 % of a launch of short chains) */
+    const auto run = [&](auto chain_of) {
+        uint32_t own_lane = lane;
+        asm volatile("" : "+v"(own_lane));
+        chain_of.place(matrices, arguments.output_size, arguments.input_size, blockIdx.x, first, arena + arguments.codes_offset,
+                       arena + arguments.exponents_offset, rows, (uint32_t)(uintptr_t)(lds_pointer)&window[slice][0], own_lane);
+        chain_of.whole(last - first, chain);
+    };
+    if (alone) {
+        run(strip_chain<1, BYTES, B128, NATIVE, true>());
+    } else {
+        run(chain_type());
+    }
     float4_t *sums = (float4_t *)&window[slice][0];
 #pragma unroll
     for (uint32_t tile = 0; tile < TILES; tile++) {

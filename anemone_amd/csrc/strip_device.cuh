@@ -22,9 +22,9 @@
  * tiles are read with one or two 16-byte LDS reads and no arithmetic; the scale codes of 4-bit weights are a word a lane
  * for the strip's four tiles (a group of 64 outputs), its byte picked by the matrix instruction; with B128 the scales are
  * E4M3_BLOCK128's float32 words where they are. */
-/* STREAMS: the chain has an instance that asks for the weights as a stream, taken where `once` says that no other block of the
- * launch reads them (the experts' launches; the shared matrices of a step of several groups of rows have readers enough) */
-template <uint32_t MATRICES, bool BYTES, bool B128 = false, bool NATIVE = false, bool STREAMS = false>
+/* ONCE: no other block of the launch reads these weights, and they are asked for as a stream (an expert's of one job; not the
+ * shared matrices of a step of several groups of rows) */
+template <uint32_t MATRICES, bool BYTES, bool B128 = false, bool NATIVE = false, bool ONCE = false>
 struct strip_chain {
     static_assert(BYTES || !B128, "float32 scales go with one-byte weights");
     static constexpr uint32_t STRIP = BYTES ? 2u : 4u; /* tiles of a strip: 4 KB of every matrix a stage either way */
@@ -56,9 +56,7 @@ struct strip_chain {
     uint32_t vector_scale_at;               /* LDS byte offset of its vector's scale byte */
     uint32_t shift;                         /* nibbles: 0 the even ones (outputs 0..7 of a tile), 4 the odd ones;
                                              * bytes: the byte selector of the same choice */
-    bool once = false;                      /* STREAMS: the same in every lane of the block */
 
-    template <bool ONCE>
     __device__ __forceinline__ void issue(uint32_t stage, uint32_t at) const
     {
         const uint32_t base = window + stage * STAGE_BYTES;
@@ -192,23 +190,11 @@ struct strip_chain {
     /* The whole chain of `total` steps (the same in every lane). The window is idle on entry and on return. */
     __device__ __forceinline__ void whole(uint32_t total, float4_t (&chain)[TILES]) const
     {
-        if constexpr (STREAMS) {
-            if (once) {
-                steps<true>(total, chain);
-                return;
-            }
-        }
-        steps<false>(total, chain);
-    }
-
-    template <bool ONCE>
-    __device__ __forceinline__ void steps(uint32_t total, float4_t (&chain)[TILES]) const
-    {
         uint32_t done = 0;
         if (total >= 2u * DEPTH) {
 #pragma unroll
             for (uint32_t i = 0; i < DEPTH; i++) {
-                issue<ONCE>(i, i);
+                issue(i, i);
             }
             /* the steady state: a step consumed has DEPTH - 1 whole stages asked for behind it, and asks for one more */
             for (; done + 2u * DEPTH <= total; done += DEPTH) {
@@ -216,14 +202,14 @@ struct strip_chain {
                 for (uint32_t i = 0; i < DEPTH; i++) {
                     wait_loads<STAGE_LOADS * (DEPTH - 1u)>();
                     consume(i, chain);
-                    issue<ONCE>(i, done + i + DEPTH);
+                    issue(i, done + i + DEPTH);
                 }
             }
         } else {
 #pragma unroll
             for (uint32_t i = 0; i < DEPTH; i++) {
                 if (i < total) {
-                    issue<ONCE>(i, i);
+                    issue(i, i);
                 }
             }
         }
@@ -244,7 +230,7 @@ struct strip_chain {
                     }
                     consume(i, chain);
                     if (at + DEPTH < total) {
-                        issue<ONCE>(i, at + DEPTH);
+                        issue(i, at + DEPTH);
                     }
                 }
             }
@@ -259,7 +245,7 @@ struct strip_chain {
                                           const unsigned char *vector_exponents, const uint32_t (&vector_rows)[8],
                                           uint32_t window_address, uint32_t lane)
     {
-        static_assert(DEPTH == 2u || DEPTH == 3u, "the waits of steps() are written out for two or three stages");
+        static_assert(DEPTH == 2u || DEPTH == 3u, "the waits of whole() are written out for two or three stages");
         const uint32_t tiles = outputs / 16u;
         const uint32_t o = lane % 16u, g = lane / 16u, G = o % 8u, parity = o / 8u, ld = g / 2u, q = g % 2u;
         /* a strip that reaches past the last tile reads the last tiles again; its surplus sums are not stored */
@@ -325,8 +311,8 @@ struct strip_chain {
                 /* lane L of a 16-byte load lands at bytes 16 L of the tile's stage and asks for the piece
                  * p = L ^ ((L / 8) % 4) of the step: LDS has 32 banks of 4 bytes, and the pieces of one T (p = 32 ld + 4 G + T,
                  * G = 0 .. 7) then lie in eight different groups of four banks for the sixteen lanes that read them together
-                 * (SQ_LDS_BANK_CONFLICT of a wide gate/up launch with nothing else in conflict: 1.68e8 -> 1.9e7 cycles); every 16 lanes still read
-                 * 256 contiguous bytes of memory */
+                 * (SQ_LDS_BANK_CONFLICT of a wide gate/up launch with nothing else in conflict: 1.68e8 -> 1.9e7 cycles); every 16
+                 * lanes still read 256 contiguous bytes of memory */
                 piece_offset = 16u * (lane ^ ((lane >> 3) & 3u));
                 /* scales: uint32 [tile][load][G]; lane L of the 4-byte load: tile L / 16, word L % 16 = 8 ld + G */
                 scale_offset = (lane / 16u) * (loads * 32u) + (lane % 16u) * 4u;
