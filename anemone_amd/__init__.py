@@ -273,7 +273,9 @@ class Exl3DescriptorModel(C.Structure):
 class LinearNativeKernels(C.Structure):
     _fields_ = [("native_expert_gate_up", u32), ("native_expert_down", u32), ("native_expert_gate_up_e4m3", u32), ("native_expert_down_e4m3", u32),
                 ("native_expert_gate_up_b128", u32), ("native_expert_down_b128", u32),
-                ("native_expert_gate_up_narrow", u32), ("native_expert_down_narrow", u32)]
+                ("native_expert_gate_up_narrow", u32), ("native_expert_down_narrow", u32),
+                ("native_expert_gate_up_e4m3_whole", u32), ("native_expert_down_e4m3_whole", u32),
+                ("native_expert_gate_up_b128_whole", u32), ("native_expert_down_b128_whole", u32)]
 
 
 class QuantizeDescription(C.Structure):

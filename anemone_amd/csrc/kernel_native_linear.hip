@@ -51,8 +51,8 @@ __device__ static __forceinline__ void native_vectors_of(const struct wide_pair 
  * 4096 x 2048 x 256 experts, gate/up 880 us against 900 (float32 scales 850 / 864), down 433 against 444 (444 / 453). */
 template <bool BYTES, bool DOWN, uint32_t TILES> /* tiles of a wavefront, of its matrices together */
 struct native_depths {
-    static constexpr uint32_t SLOTS = BYTES ? (DOWN ? 3u : 2u) : TILES == 8u ? 2u : 3u;
-    static constexpr uint32_t DEPTH = BYTES ? (DOWN ? NATIVE_E4M3_DOWN_STAGES : NATIVE_E4M3_GATE_UP_STAGES) : NATIVE_E2M1_STAGES;
+    static constexpr uint32_t SLOTS = BYTES ? (DOWN && TILES == 2u ? 3u : 2u) : TILES == 8u ? 2u : 3u;
+    static constexpr uint32_t DEPTH = BYTES ? (TILES == 4u ? NATIVE_E4M3_WHOLE_STAGES : DOWN ? NATIVE_E4M3_DOWN_STAGES : NATIVE_E4M3_GATE_UP_STAGES) : NATIVE_E2M1_STAGES;
 };
 
 template <bool BYTES, uint32_t STRIP, uint32_t GROUP, bool B128 = false>
@@ -69,7 +69,7 @@ __device__ static __forceinline__ void native_expert_gate_up(const struct wide_e
     struct wide_expert_tile tile;
     uint32_t pair_count = 0, block_strip = 0;
     bool alone = false;
-    if (!order_block_of<GROUP, false, !BYTES>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count, &alone)) {
+    if (!order_block_of<GROUP, false, !BYTES || chain_type::TILES == 4u>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count, &alone)) {
         return;
     }
     const struct wide_pair *pairs = (const struct wide_pair *)(arena + arguments.pairs_offset) + tile.first_pair;
@@ -93,7 +93,7 @@ __device__ static __forceinline__ void native_expert_gate_up(const struct wide_e
     wide_gate_up_finish<STRIP, COLUMN_BLOCKS, B128>(arguments, arena, window, columns, pair_count, block_strip, tile0, wave, lane, chain);
 }
 
-template <bool BYTES, uint32_t DOWN_STRIP, uint32_t GROUP, bool B128 = false, bool BY_RUN = !BYTES>
+template <bool BYTES, uint32_t DOWN_STRIP, uint32_t GROUP, bool B128 = false, bool BY_RUN = !BYTES || DOWN_STRIP == 4u>
 __device__ static __forceinline__ void native_expert_down(const struct wide_expert_down_arguments &arguments, unsigned char *arena)
 {
     constexpr uint32_t COLUMN_BLOCKS = 4u * GROUP;
@@ -186,7 +186,37 @@ extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_BYTES_DOWN_W
 }
 ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_down_b128_1, wide_expert_down_arguments);
 
+/* The one-byte launches of whole strips: twice the tiles a wavefront (gate's two and up's two, or four of down), so that a
+ * block's columns, which every strip's block brings into LDS again, are brought half as often and an operand read from LDS
+ * serves four matrix instructions; two sets of weights and two stages at two wavefronts a SIMD (244 to 253 registers, 128 of
+ * them sums); the blocks in the order of runs, where each is a longer piece of work and the look at the table counts less. For
+ * launches of many pairs an expert (native_takes_whole_bytes, with both sides' times): at 64 pairs an expert a launch is near
+ * what memory gives and three wavefronts a SIMD hide more, at 128 half of what passes the level-2 caches were columns (4096
+ * rows of 4096 x 2048 x 256 experts, float32 scales: gate/up 1105 -> 985 us, down 598 -> 539). */
+#define NATIVE_BYTES_WHOLE_WAVES 2
+extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_BYTES_WHOLE_WAVES) native_expert_gate_up_e4m3_whole_1(struct wide_expert_gate_up_arguments arguments, unsigned char *arena)
+{
+    native_expert_gate_up<true, 2u, NATIVE_E4M3_COLUMN_BLOCKS / 4u>(arguments, arena);
+}
+ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_gate_up_e4m3_whole_1, wide_expert_gate_up_arguments);
+extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_BYTES_WHOLE_WAVES) native_expert_down_e4m3_whole_1(struct wide_expert_down_arguments arguments, unsigned char *arena)
+{
+    native_expert_down<true, 4u, NATIVE_E4M3_COLUMN_BLOCKS / 4u>(arguments, arena);
+}
+ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_down_e4m3_whole_1, wide_expert_down_arguments);
+extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_BYTES_WHOLE_WAVES) native_expert_gate_up_b128_whole_1(struct wide_expert_gate_up_arguments arguments, unsigned char *arena)
+{
+    native_expert_gate_up<true, 2u, NATIVE_E4M3_COLUMN_BLOCKS / 4u, true>(arguments, arena);
+}
+ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_gate_up_b128_whole_1, wide_expert_gate_up_arguments);
+extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_BYTES_WHOLE_WAVES) native_expert_down_b128_whole_1(struct wide_expert_down_arguments arguments, unsigned char *arena)
+{
+    native_expert_down<true, 4u, NATIVE_E4M3_COLUMN_BLOCKS / 4u, true>(arguments, arena);
+}
+ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_down_b128_whole_1, wide_expert_down_arguments);
+
 static_assert(native_chain<2, false, 2u, NATIVE_E2M1_COLUMN_BLOCKS, 3u, NATIVE_E2M1_STAGES>::WINDOW_BYTES == NATIVE_WINDOW_BYTES(NATIVE_E2M1_COLUMN_BLOCKS, NATIVE_E2M1_STAGES) &&
                   native_chain<2, true, 1u, NATIVE_E4M3_COLUMN_BLOCKS, 2u, NATIVE_E4M3_GATE_UP_STAGES>::WINDOW_BYTES == NATIVE_WINDOW_BYTES(NATIVE_E4M3_COLUMN_BLOCKS, NATIVE_E4M3_GATE_UP_STAGES) &&
-                  native_chain<1, true, 2u, NATIVE_E4M3_COLUMN_BLOCKS, 3u, NATIVE_E4M3_DOWN_STAGES>::WINDOW_BYTES == NATIVE_WINDOW_BYTES(NATIVE_E4M3_COLUMN_BLOCKS, NATIVE_E4M3_DOWN_STAGES),
+                  native_chain<1, true, 2u, NATIVE_E4M3_COLUMN_BLOCKS, 3u, NATIVE_E4M3_DOWN_STAGES>::WINDOW_BYTES == NATIVE_WINDOW_BYTES(NATIVE_E4M3_COLUMN_BLOCKS, NATIVE_E4M3_DOWN_STAGES) &&
+                  native_chain<2, true, 2u, NATIVE_E4M3_COLUMN_BLOCKS, 2u, NATIVE_E4M3_WHOLE_STAGES>::WINDOW_BYTES == NATIVE_WINDOW_BYTES(NATIVE_E4M3_COLUMN_BLOCKS, NATIVE_E4M3_WHOLE_STAGES),
               "the windows the host asks for are the kernels'");

@@ -332,8 +332,8 @@ struct native_chain {
     }
 
     /* The same step of one-byte weights. A column block's operand is read while the block before it is multiplied (two or
-     * three blocks ahead: the same time, and more registers); under float32 scales a block's products enter its chains while
-     * the next block is multiplied. */
+     * three blocks ahead: the same time, and more registers); under float32 scales products enter their chains while the next
+     * ones are formed. */
     template <uint32_t LIVE>
     __device__ __forceinline__ void consume_bytes(uint32_t stage, uint32_t step, const slot &set, const uint32_t (&held)[SCALE_LOADS], uint32_t holder,
                                                   float4_t (&chain)[TILES][COLUMN_BLOCKS]) const
@@ -347,14 +347,17 @@ struct native_chain {
         const uint32_t at = stage * STAGE_BYTES, scales = scales_of(step);
         int8_vector b[LIVE];
         uint32_t scale_b[LIVE];
-        float4_t products[2][TILES];
-        const auto add = [&](uint32_t j) {
+        /* float32 scales: the tiles whose products wait together (one of four: two's do not fit beside the sums of eight blocks) */
+        constexpr uint32_t PART = TILES > 2u ? 1u : TILES, PARTS = TILES / PART;
+        float4_t products[2][PART];
+        const auto add = [&](uint32_t place) { /* part place % PARTS of column block place / PARTS */
+            const uint32_t j = place / PARTS, first = place % PARTS * PART;
 #pragma unroll
-            for (uint32_t t = 0; t < TILES; t++) {
-                const float scale = __fmul_rn(__uint_as_float(scale_a[t / STRIP]), __uint_as_float(scale_b[j]));
+            for (uint32_t t = 0; t < PART; t++) {
+                const float scale = __fmul_rn(__uint_as_float(scale_a[(first + t) / STRIP]), __uint_as_float(scale_b[j]));
 #pragma unroll
                 for (uint32_t v = 0; v < 4u; v++) {
-                    chain[t][j][v] = __fmaf_rn(products[j % 2u][t][v], scale, chain[t][j][v]);
+                    chain[first + t][j][v] = __fmaf_rn(products[place % 2u][t][v], scale, chain[first + t][j][v]);
                 }
             }
         };
@@ -367,25 +370,30 @@ struct native_chain {
                 read_block(at, scales, j + 1u, b[j + 1u], scale_b[j + 1u]);
             }
 #pragma unroll
-            for (uint32_t t = 0; t < TILES; t++) {
-                const uint4_t first = set.words[t][0], second = set.words[t][HALVES - 1u];
-                const int8_vector a = {(int)first.x, (int)first.y, (int)first.z, (int)first.w, (int)second.x, (int)second.y, (int)second.z, (int)second.w};
+            for (uint32_t part = 0; part < PARTS; part++) {
+#pragma unroll
+                for (uint32_t i = 0; i < PART; i++) {
+                    const uint32_t t = part * PART + i;
+                    const uint4_t first = set.words[t][0], second = set.words[t][HALVES - 1u];
+                    const int8_vector a = {(int)first.x, (int)first.y, (int)first.z, (int)first.w, (int)second.x, (int)second.y, (int)second.z, (int)second.w};
+                    if constexpr (B128) {
+                        products[(j * PARTS + part) % 2u][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[j], (float4_t){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0, 127, 0, 127);
+                    } else {
+                        chain[t][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[j], chain[t][j], 0, 0, 0, (int)scale_a[t], 0, (int)scale_b[j]);
+                    }
+                }
                 if constexpr (B128) {
-                    products[j % 2u][t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[j], (float4_t){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0, 127, 0, 127);
-                } else {
-                    chain[t][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[j], chain[t][j], 0, 0, 0, (int)scale_a[t], 0, (int)scale_b[j]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (j * PARTS + part != 0u) {
+                        add(j * PARTS + part - 1u);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (B128) {
-                if (j != 0u) {
-                    add(j - 1u);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
         }
         if constexpr (B128) {
-            add(LIVE - 1u);
+            add(LIVE * PARTS - 1u);
         }
         __builtin_amdgcn_s_setprio(0);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); /* the stage is read before the next barrier */

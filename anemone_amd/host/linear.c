@@ -615,6 +615,27 @@ static bool native_takes_narrow(const struct matrix_shape_record *shape, uint32_
                                     : pairs <= 48u * experts && 4u * narrow_busy <= 3u * whole;
 }
 
+/* Whether a launch of the one-byte native kernels takes strips of twice the tiles (two blocks a CU) in place of blocks of
+ * `outputs` (`resident` on the card): from NATIVE_WHOLE_PAIRS pairs an expert on, where the bigger blocks fill the card about as
+ * well and the matrix holds a whole strip of a wavefront. A strip's block brings its tile's columns into LDS again, so that the
+ * fewer strips the fewer bytes pass the level-2 caches; but a block of many pairs is a long one, and where a few experts hold most
+ * of them the launch ends on it. Half strips / whole ones, us, float32 scales, gate/up and down: 4096 x 2048 x 256 experts, 64 pairs
+ * an expert 811 / 786 and 422 / 433, under loads of Zipf(1.1) 823 / 879 and 463 / 478; 94 pairs 885 / 798 and 470 / 440; 128 pairs
+ * 1105 / 985 and 598 / 539, Zipf 1123 / 1058 and 627 / 586; 2048 x 2048 x 64 at 87 Zipf 115 / 128 and 77 / 70; 2048 x 896 x 64 at
+ * 141 90 / 77 and 50 / 49; 2048 x 1024 x 256 at 128 Zipf 313 / 276 and 216 / 169; 4096 x 2048 x 64 at 256 Zipf 442 / 399 and 252 /
+ * 214. E8M0 scales: 4096 x 2048 x 256 at 128 1128 / 988 and 570 / 536, Zipf 1164 / 1103 and 613 / 606; 2048 x 1024 x 256 at 128
+ * Zipf 345 / 279 and 208 / 167; 2048 x 2048 x 64 at 87 Zipf 123 / 128 and 74 / 69. */
+#define NATIVE_WHOLE_PAIRS 96u
+static bool native_takes_whole_bytes(const struct matrix_shape_record *shape, uint32_t outputs, uint32_t resident, uint32_t tile_count, uint64_t pairs)
+{
+    const uint64_t pairs_tiles = (pairs + WIDE_TILE_PAIRS - 1u) / WIDE_TILE_PAIRS;
+    const uint64_t experts = tile_count > pairs_tiles ? tile_count - pairs_tiles : 1u;
+    const uint64_t full = (pairs + 2u * WIDE_TILE_PAIRS - 1u) / (2u * WIDE_TILE_PAIRS), groups = full > experts ? full : experts; /* blocks a strip */
+    const uint64_t half_strips = ((uint64_t)shape->output_size + outputs - 1u) / outputs, whole_strips = (half_strips + 1u) / 2u;
+    const uint64_t half = (half_strips * groups + resident - 1u) / resident * resident, whole = (whole_strips * groups + 511u) / 512u * 1024u;
+    return pairs >= NATIVE_WHOLE_PAIRS * experts && shape->output_size >= outputs / 2u && 8u * whole <= 9u * half;
+}
+
 /* block128: the launches of WEIGHT_FORMAT_E4M3_BLOCK128 experts (four: the hidden vectors' quantizer is a launch of its
  * own between the products); else those of the reference's formats (three) */
 static result_status wide_experts_prepare(const struct linear_wide_experts_description *description, uint64_t arena_byte_count,
@@ -724,6 +745,21 @@ static result_status wide_experts_prepare(const struct linear_wide_experts_descr
             block_outputs *= 2u;
         }
     }
+    if (native && bytes) { /* one-byte weights: strips of twice the tiles for many pairs an expert */
+        const uint32_t whole_gate_up = block128 ? native_kernels->native_expert_gate_up_b128_whole : native_kernels->native_expert_gate_up_e4m3_whole;
+        const uint32_t whole_down = block128 ? native_kernels->native_expert_down_b128_whole : native_kernels->native_expert_down_e4m3_whole;
+        if (whole_gate_up != BACKEND_NO_KERNEL &&
+            native_takes_whole_bytes(gate_up, gate_up_outputs, 768u, description->tile_count, pairs)) {
+            gate_up_kernel = whole_gate_up;
+            gate_up_outputs *= 2u;
+            gate_up_window = NATIVE_WINDOW_BYTES(NATIVE_E4M3_COLUMN_BLOCKS, NATIVE_E4M3_WHOLE_STAGES);
+        }
+        if (whole_down != BACKEND_NO_KERNEL && native_takes_whole_bytes(down, block_outputs, 512u, description->tile_count, pairs)) {
+            down_kernel = whole_down;
+            block_outputs *= 2u;
+            down_window = NATIVE_WINDOW_BYTES(NATIVE_E4M3_COLUMN_BLOCKS, NATIVE_E4M3_WHOLE_STAGES);
+        }
+    }
     struct kernel_launch launches[LINEAR_WIDE_EXPERTS_BLOCK128_LAUNCH_COUNT];
     uint32_t at = 0;
     launch_fill(&launches[at++], gate_up_kernel,
@@ -779,8 +815,12 @@ result_status linear_native_kernels_prepare(const struct backend_operations *bac
                   {KERNEL_NATIVE_EXPERT_GATE_UP_STEM "b128_1", sizeof(struct wide_expert_gate_up_arguments)},
                   {KERNEL_NATIVE_EXPERT_DOWN_STEM "b128_1", sizeof(struct wide_expert_down_arguments)},
                   {KERNEL_NATIVE_EXPERT_GATE_UP_STEM "narrow_1", sizeof(struct wide_expert_gate_up_arguments)},
-                  {KERNEL_NATIVE_EXPERT_DOWN_STEM "narrow_1", sizeof(struct wide_expert_down_arguments)}};
-    enum { WANTED = sizeof wanted / sizeof wanted[0], REQUIRED = WANTED - 2 }; /* without the narrow ones every launch is of whole strips */
+                  {KERNEL_NATIVE_EXPERT_DOWN_STEM "narrow_1", sizeof(struct wide_expert_down_arguments)},
+                  {KERNEL_NATIVE_EXPERT_GATE_UP_STEM "e4m3_whole_1", sizeof(struct wide_expert_gate_up_arguments)},
+                  {KERNEL_NATIVE_EXPERT_DOWN_STEM "e4m3_whole_1", sizeof(struct wide_expert_down_arguments)},
+                  {KERNEL_NATIVE_EXPERT_GATE_UP_STEM "b128_whole_1", sizeof(struct wide_expert_gate_up_arguments)},
+                  {KERNEL_NATIVE_EXPERT_DOWN_STEM "b128_whole_1", sizeof(struct wide_expert_down_arguments)}};
+    enum { WANTED = sizeof wanted / sizeof wanted[0], REQUIRED = WANTED - 6 }; /* without the narrow and the whole ones every launch is of one kind of strips */
     uint32_t handles[WANTED];
     _Static_assert(sizeof(struct linear_native_kernels_record) == sizeof handles, "a handle a member, in the members' order");
     for (uint32_t i = 0; i < WANTED; i++) {

@@ -616,6 +616,10 @@ struct linear_native_kernels_record {
     uint32_t native_expert_down_b128;
     uint32_t native_expert_gate_up_narrow; /* E2M1_GFX950, strips of half the tiles; BACKEND_NO_KERNEL: launches of whole strips alone */
     uint32_t native_expert_down_narrow;
+    uint32_t native_expert_gate_up_e4m3_whole; /* E4M3_GFX950, strips of twice the tiles; BACKEND_NO_KERNEL: launches without them */
+    uint32_t native_expert_down_e4m3_whole;
+    uint32_t native_expert_gate_up_b128_whole; /* E4M3_BLOCK128_GFX950, likewise */
+    uint32_t native_expert_down_b128_whole;
 };
 MUST_CHECK result_status linear_native_kernels_prepare(const struct backend_operations *backend, struct device_card *card,
                                                        uint32_t arithmetic_class, struct linear_native_kernels_record *kernels_out);

@@ -531,6 +531,7 @@ ANEMONE_RECORD_HAS(expert_gate_up_quantize_arguments, 96);
 #define NATIVE_E2M1_STAGES 2u /* stages of columns in LDS: a K step in use, the next on its way */
 #define NATIVE_E4M3_GATE_UP_STAGES 2u
 #define NATIVE_E4M3_DOWN_STAGES 3u
+#define NATIVE_E4M3_WHOLE_STAGES 2u /* of the launches of whole strips, gate/up and down */
 /* dynamic LDS: the stages of a K step of the block's columns (128 bytes of codes a column), and two chunks of their scale
  * words (four K steps of 4 bytes a column each) */
 #define NATIVE_WINDOW_BYTES(column_blocks, stages) ((stages) * (column_blocks) * 2048u + 2u * (column_blocks) * 256u)

@@ -918,6 +918,41 @@ def test_native_strips_by_how_full_their_last_round_is(fake, experts_n, rows, do
     assert launches[0].grid[0] == -(-down_input // (128 if "narrow" in gate_up else 256)) and launches[1].grid[0] == -(-4096 // (256 if "narrow" in down else 512))
 
 
+@pytest.mark.parametrize("experts_n,rows,down_input,gate_up,down", [
+    (256, 3071, 2048, "", ""),              # a pair below 96 an expert
+    (256, 3072, 2048, "whole_", "whole_"),
+    (64, 1024, 768, "", "whole_"),          # gate/up: 768 half strips fill one round of three a CU, 384 whole ones a round of two
+    (64, 1024, 896, "whole_", "whole_"),    # two rounds or one
+    (64, 4096, 768, "whole_", "whole_")])
+@pytest.mark.parametrize("infix", ["e4m3", "b128"])
+def test_native_one_byte_strips_by_pairs_and_rounds(fake, infix, experts_n, rows, down_input, gate_up, down):
+    """Launches of many pairs an expert take strips of twice the tiles, where these fill the card about as well: grids, windows."""
+    lib, linear, native, launches = amd.library(), amd.LinearKernels(), amd.LinearNativeKernels(), amd.launches_of(4)
+    block128 = infix == "b128"
+    assert lib.linear_kernels_prepare(fake.address, fake.card, 950, C.byref(linear)) == 0
+    assert lib.linear_native_kernels_prepare(fake.address, fake.card, 950, C.byref(native)) == 0
+    d = wide_experts_description(amd.WEIGHT_FORMAT_E4M3_BLOCK128_GFX950 if block128 else amd.WEIGHT_FORMAT_E4M3_GFX950,
+                                 gate_up_shape=amd.Shape(down_input, 4096, 8, 0), down_shape=amd.Shape(4096, down_input, 8, 0),
+                                 row_count=rows, tile_count=amd.wide_tile_count(rows, 8, experts_n))
+    at = 3 << 30
+    for record, name in [(d.experts, name) for name in ("codes", "exponents", "hidden_codes", "hidden_exponents", "hidden_operands", "pair_output", "row_output")] + \
+            [(d, "tiles"), (d, "pairs")]:  # room for 4096 rows
+        size = 4 * getattr(record, name).byte_count
+        setattr(record, name, amd.Range(at, size))
+        at += size
+    for without in (False, True):  # a backend without the kernels of whole strips takes the others
+        if without:
+            native.native_expert_gate_up_e4m3_whole = native.native_expert_gate_up_b128_whole = amd.BACKEND_NO_KERNEL
+            native.native_expert_down_e4m3_whole = native.native_expert_down_b128_whole = amd.BACKEND_NO_KERNEL
+            gate_up = down = ""
+        assert lib.linear_native_experts_prepare(C.byref(d), 8 << 30, C.byref(linear), C.byref(native), launches) == 0
+        first, second = launches[0], launches[2 if block128 else 1]
+        assert fake.handles[first.kernel][1] == "native_expert_gate_up_%s_%s1" % (infix, gate_up)
+        assert fake.handles[second.kernel][1] == "native_expert_down_%s_%s1" % (infix, down)
+        assert first.grid[0] == -(-down_input // (128 if gate_up else 64)) and second.grid[0] == -(-4096 // (256 if down else 128))
+        assert first.dynamic_shared_byte_count == 36864 and second.dynamic_shared_byte_count == (36864 if down else 53248)
+
+
 def test_native_kernels_without_the_narrow_ones(fake):
     """A backend without the kernels of narrow strips prepares the others, and every launch is of whole strips."""
     lib, linear, native, launches = amd.library(), amd.LinearKernels(), amd.LinearNativeKernels(), amd.launches_of(4)

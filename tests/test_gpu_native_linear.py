@@ -362,3 +362,39 @@ def test_narrow_and_whole_strips_give_the_same_bytes(amd, card, hidden, inner, r
     for name, a, b in zip(NAMES, *outputs):
         assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), name
         assert not np.all(a.view(np.uint8) == 0xEE)
+
+
+@pytest.mark.parametrize("fmt", [E4M3, B128])
+@pytest.mark.parametrize("hidden,inner,experts_n,picks,rows,live,one_expert", [
+    (128, 128, 64, 4, 600, 597, False),   # one K step; a strip of a wavefront alone, three past the matrix
+    (256, 384, 64, 8, 300, 300, False),   # two K steps; a block's last strips past the matrix
+    (512, 256, 64, 8, 1500, 1401, False), # blocks of two tiles of one expert, a run's odd last tile alone
+    (640, 384, 64, 3, 4300, 4287, True),  # a run of 68 tiles among the others: pieces of 16, and where a window of 64 tiles ends
+    (256, 128, 384, 1, 100, 100, False),  # more unused tiles behind the used ones than the first look takes
+])
+def test_whole_and_half_strips_of_one_byte_weights_give_the_same_bytes(amd, card, hidden, inner, experts_n, picks, rows, live, one_expert, fmt):
+    """The one-byte launches of strips of twice the tiles (native_expert_gate_up_e4m3_whole_1 and its like, whose blocks go in the
+    order of runs) and the others, over the same rows: every output byte that a launch writes, and none besides."""
+    say("whole and half strips", fmt, hidden, inner, experts_n, picks, rows, live)
+    router = to_bf16(normals(87, experts_n * hidden) * 0.02).reshape(experts_n, hidden)
+    layer = amd.Fp4Layer(card, hidden, inner, experts_n, picks, rows, matrices_of(hidden, inner, experts_n, 89, fmt),
+                         router_weights_bf16=router, weight_format=NATIVE_OF[fmt])
+    if one_expert:
+        card.upload(layer.bias_offset, np.where(np.arange(experts_n) == 5, 100.0, 0.0).astype(np.float32))
+    x = to_bf16(normals(91, rows * hidden)).reshape(rows, hidden)
+    _, wide = run_wide(card, layer, x, live)
+    native, infix = layer.native_kernels, "b128" if fmt == B128 else "e4m3"
+    launches, outputs = layer.wide_expert_launches(wide), []
+    first, second = launches[0], launches[2 if fmt == B128 else 1]
+    for suffix, tiles, stages in (("", 1, 3), ("_whole", 2, 2)):
+        first.kernel, second.kernel = getattr(native, "native_expert_gate_up_" + infix + suffix), getattr(native, "native_expert_down_" + infix + suffix)
+        first.grid[0], second.grid[0] = -(-inner // (64 * tiles)), -(-hidden // (128 * tiles))
+        first.dynamic_shared_byte_count, second.dynamic_shared_byte_count = 2 * 16384 + 4096, stages * 16384 + 4096
+        for name in NAMES:
+            card.upload(layer.ranges[name].byte_offset, np.full(layer.ranges[name].byte_count, 0xEE, dtype=np.uint8))
+        card.run(launches)
+        outputs.append([layer.read(name).copy() for name in NAMES])
+    for name, a, b in zip(NAMES, *outputs):
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), name
+        if not (fmt == B128 and name == "hidden_operands"):
+            assert not np.all(a.view(np.uint8) == 0xEE)

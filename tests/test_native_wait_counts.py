@@ -20,6 +20,7 @@ INSTANCES = {
     **{"E2M1 narrow down (4 tiles, 1 scale word), %d loads of columns" % loads: (3, 2, loads, 5) for loads in (2, 3)},
     **{"one-byte gate/up (2 tiles of two halves), %d loads of columns" % loads: (2, 2, loads, 4) for loads in (2, 3, 4, 5)},
     **{"one-byte down (2 tiles of two halves), %d loads of columns" % loads: (3, 3, loads, 4) for loads in (2, 3, 4, 5)},
+    **{"one-byte whole strips, gate/up and down (4 tiles of two halves), %d loads of columns" % loads: (2, 2, loads, 8) for loads in (2, 3, 4, 5)},
     # other parameters the formula allows
     "three sets, three stages, 6 loads of weights": (3, 3, 5, 6),
     "three sets, three stages, 5 loads of weights": (3, 3, 5, 5),
