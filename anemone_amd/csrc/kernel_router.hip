@@ -28,19 +28,19 @@
  * A block takes PROJECTION_EXPERTS experts and up to PROJECTION_ROWS rows: it stages the weights and the rows in
  * chunks of PROJECTION_CHUNK inputs through LDS with 16-byte coalesced loads (the next chunk in flight while this
  * one is consumed); a thread owns chains 2 j and 2 j + 1 of one expert for every row, so the fma order of a chain
- * is the definition's whatever the staging. grid (ceil(E / 8), ceil(rows / 4)), block 128; or, for a thin step, grid
- * (ceil(E / 8), rows): a row a block (the rows a block takes are what its grid leaves it, four or one), a quarter of
- * the fused multiply-adds a block and four times the blocks: the launch is a few round trips to memory either way. */
-#define PROJECTION_MOST_ROWS 4u
+ * is the definition's whatever the staging. grid (ceil(E / 8), ceil(rows / 4)), block 128. (A thin step takes a row a
+ * block, router_projection_thin.) */
+#define PROJECTION_ROWS 4u
 #define PROJECTION_EXPERTS 8u
 #define PROJECTION_CHUNK 1024u
 #define PROJECTION_W_LOADS (PROJECTION_EXPERTS * PROJECTION_CHUNK * 2u / 16u / PROJECTION_THREADS)
-template <uint32_t PROJECTION_ROWS>
 __device__ static __forceinline__ void router_projection_block(const struct router_projection_arguments &arguments, unsigned char *arena)
 {
     constexpr uint32_t PROJECTION_X_LOADS = PROJECTION_ROWS * PROJECTION_CHUNK * 2u / 16u / PROJECTION_THREADS;
-    __shared__ __attribute__((aligned(16))) uint16_t w_tile[PROJECTION_EXPERTS][PROJECTION_CHUNK];
-    __shared__ __attribute__((aligned(16))) uint16_t x_tile[PROJECTION_ROWS][PROJECTION_CHUNK];
+    extern __shared__ __attribute__((aligned(1024))) unsigned char projection_window[]; /* PROJECTION_WINDOW_BYTES */
+    static_assert((PROJECTION_EXPERTS + PROJECTION_ROWS) * PROJECTION_CHUNK * 2u == PROJECTION_WINDOW_BYTES, "the window the host asks for");
+    uint16_t (*const w_tile)[PROJECTION_CHUNK] = (uint16_t (*)[PROJECTION_CHUNK])projection_window;
+    uint16_t (*const x_tile)[PROJECTION_CHUNK] = w_tile + PROJECTION_EXPERTS;
     const uint32_t H = arguments.hidden, thread = threadIdx.x;
     const uint32_t first_expert = blockIdx.x * PROJECTION_EXPERTS, first_row = blockIdx.y * PROJECTION_ROWS;
     const uint16_t *weights = (const uint16_t *)(arena + arguments.weights_offset);
@@ -88,11 +88,7 @@ __device__ static __forceinline__ void router_projection_block(const struct rout
             fetch(chunk + PROJECTION_CHUNK);
         }
         __syncthreads();
-        /* one row: the LDS reads of UNROLL groups are on their way together; four at a time and the launch was one LDS round trip
-         * behind the other (one row of 4096 inputs by 256 experts 7.3 -> 6.2 us, eight rows 7.8 -> 6.3; two or four chunks asked for
-         * ahead: no shorter) */
-        constexpr uint32_t UNROLL = PROJECTION_ROWS == 1u ? 16u : 4u;
-#pragma unroll UNROLL
+#pragma unroll 4
         for (uint32_t k = 0; k < PROJECTION_CHUNK; k += PROJECTION_CHAINS) {
             const uint32_t w = *(const uint32_t *)&w_tile[expert_in_block][k + 2u * pair];
             const float w0 = __uint_as_float(w << 16), w1 = __uint_as_float(w & 0xFFFF0000u);
@@ -118,13 +114,135 @@ __device__ static __forceinline__ void router_projection_block(const struct rout
     }
 }
 
-extern "C" __global__ void __launch_bounds__(PROJECTION_THREADS)
+
+typedef __attribute__((address_space(3))) void *lds_bytes;
+
+/* 16 bytes a lane from memory straight into LDS (lane L lands at lds_base + 16 L). Written as assembly: the compiler keeps
+ * no book on it, so the waits for it are written out where a stage is needed. */
+__device__ static __forceinline__ void projection_load_to_lds(const void *lane_address, uint32_t lds_base)
+{
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(lane_address), "s"(lds_base) : "memory", "m0");
+}
+
+/* A thin step's form: a row a block, a wavefront two experts, a lane one chain. The inputs pass through LDS, straight from memory,
+ * all THIN_CHUNK of them asked for at once, so that the launch waits for memory one time. A chain's inputs lie 64 bytes apart: the
+ * LDS's transposing read gives a lane four of them (ds_read_b64_tr_b16: sixteen lanes name four rows of sixteen 16-bit values, and
+ * lane i receives value i of each). A wavefront that has a vector unit to itself issues an instruction in six cycles whatever it
+ * is and has fifteen LDS reads on their way at most, so both are what counts: by single reads of 16 bits 4.9 us, by these 4.0
+ * (one row of 4096 inputs by 256 experts; two chains a lane, through registers and in chunks of 1024: 5.5; eight rows 5.6 -> 4.35,
+ * eight of 5120 by 384 experts 7.2 -> 5.7, three of 2048 by 64 3.6 -> 3.0). grid (ceil(E / 8), rows), block 256. */
+#define THIN_EXPERTS 2u /* of a wavefront */
+#define THIN_CHUNK 4096u
+#define THIN_ROW_VALUES (THIN_CHUNK + 32u) /* 64 bytes more: the two experts' chains lie on different banks */
+#define THIN_LOADS (THIN_CHUNK / 512u) /* of a row's chunk: 64 lanes of eight values */
+typedef short thin_values_t __attribute__((ext_vector_type(4)));
+#define THIN_BATCH 16u /* groups of 32 inputs whose reads go together */
+struct thin_batch {
+    uint2_t w[THIN_BATCH / 4u], x[THIN_BATCH / 4u];
+};
+
+/* the inputs of THIN_BATCH groups of the lane's chain, of its expert and of the row */
+__device__ static __forceinline__ void thin_read(uint32_t w_at, uint32_t x_at, struct thin_batch &into)
+{
+    typedef __attribute__((address_space(3))) thin_values_t *place;
+#pragma unroll
+    for (uint32_t k = 0; k < THIN_BATCH / 4u; k++) {
+        into.w[k] = __builtin_bit_cast(uint2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((place)(uintptr_t)(w_at + k * (4u * PROJECTION_CHAINS * 2u))));
+        into.x[k] = __builtin_bit_cast(uint2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((place)(uintptr_t)(x_at + k * (4u * PROJECTION_CHAINS * 2u))));
+    }
+}
+
+/* the first `groups` of a batch into the chain */
+__device__ static __forceinline__ float thin_add(const struct thin_batch &batch, uint32_t groups, float chain)
+{
+#pragma unroll
+    for (uint32_t k = 0; k < THIN_BATCH; k++) {
+        const uint32_t w = batch.w[k / 4u][k / 2u % 2u], x = batch.x[k / 4u][k / 2u % 2u];
+        const float sum = k % 2u == 0u ? __fmaf_rn(__uint_as_float(w << 16), __uint_as_float(x << 16), chain)
+                                       : __fmaf_rn(__uint_as_float(w & 0xFFFF0000u), __uint_as_float(x & 0xFFFF0000u), chain);
+        chain = k < groups ? sum : chain;
+    }
+    return chain;
+}
+
+__device__ static __forceinline__ void router_projection_thin(const struct router_projection_arguments &arguments, unsigned char *arena)
+{
+    extern __shared__ __attribute__((aligned(1024))) unsigned char projection_window[]; /* PROJECTION_THIN_WINDOW_BYTES: the experts' rows, then the row's */
+    static_assert((PROJECTION_EXPERTS + 1u) * THIN_ROW_VALUES * 2u == PROJECTION_THIN_WINDOW_BYTES, "the window the host asks for");
+    const uint32_t H = arguments.hidden, lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const uint32_t first_expert = blockIdx.x * PROJECTION_EXPERTS + wave * THIN_EXPERTS, chain_of = lane % PROJECTION_CHAINS, mine = lane / PROJECTION_CHAINS;
+    const uint32_t window_address = (uint32_t)(uintptr_t)(lds_bytes)projection_window;
+    const uint16_t *row = (const uint16_t *)(arena + arguments.rows_offset) + (uint64_t)blockIdx.y * H + 8u * lane;
+    const uint16_t *weights[THIN_EXPERTS]; /* an expert past the last repeats the last: its score is not stored */
+#pragma unroll
+    for (uint32_t e = 0; e < THIN_EXPERTS; e++) {
+        const uint32_t expert = first_expert + e < arguments.expert_count ? first_expert + e : arguments.expert_count - 1u;
+        weights[e] = (const uint16_t *)(arena + arguments.weights_offset) + (uint64_t)expert * H + 8u * lane;
+    }
+    /* row lane % 16 / 4 of the four, sixteen chains of the 32, eight bytes a lane */
+    const uint32_t lane_bytes = lane % 16u / 4u * (PROJECTION_CHAINS * 2u) + lane / 16u % 2u * 32u + lane % 4u * 8u;
+    const uint32_t w_at = window_address + (wave * THIN_EXPERTS + mine) * (THIN_ROW_VALUES * 2u) + lane_bytes;
+    const uint32_t x_at = window_address + PROJECTION_EXPERTS * (THIN_ROW_VALUES * 2u) + lane_bytes;
+    float chain = 0.0f;
+    for (uint32_t chunk = 0; chunk < H; chunk += THIN_CHUNK) {
+        if (chunk != 0u) {
+            __syncthreads(); /* the chunk before has been read */
+        }
+#pragma unroll
+        for (uint32_t part = 0; part < THIN_LOADS; part++) {
+            if (chunk + 512u * part + 8u * lane < H) { /* a width is a whole number of groups: no group is brought in part */
+#pragma unroll
+                for (uint32_t e = 0; e < THIN_EXPERTS; e++) {
+                    projection_load_to_lds(weights[e] + chunk + 512u * part, window_address + ((wave * THIN_EXPERTS + e) * THIN_ROW_VALUES + 512u * part) * 2u);
+                }
+                if (part / (THIN_LOADS / (PROJECTION_EXPERTS / THIN_EXPERTS)) == wave) {
+                    projection_load_to_lds(row + chunk + 512u * part, window_address + (PROJECTION_EXPERTS * THIN_ROW_VALUES + 512u * part) * 2u);
+                }
+            }
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        const uint32_t groups = (H - chunk < THIN_CHUNK ? H - chunk : THIN_CHUNK) / PROJECTION_CHAINS;
+        /* a batch is read while the one before it is added; past the chunk's last group the reads stay inside its place, and what
+         * they give is not added (a width that is no whole 512) */
+        constexpr uint32_t BATCH_BYTES = THIN_BATCH * PROJECTION_CHAINS * 2u;
+        struct thin_batch batch[2];
+        thin_read(w_at, x_at, batch[0]);
+        for (uint32_t group = 0; group < groups; group += 2u * THIN_BATCH) {
+            const uint32_t at = group * (PROJECTION_CHAINS * 2u);
+            thin_read(w_at + at + BATCH_BYTES, x_at + at + BATCH_BYTES, batch[1]);
+            if (group + THIN_BATCH <= groups) {
+                chain = thin_add(batch[0], THIN_BATCH, chain);
+            } else {
+                chain = thin_add(batch[0], groups - group, chain);
+            }
+            if (group + THIN_BATCH >= groups) {
+                break;
+            }
+            if (group + 2u * THIN_BATCH < groups) {
+                thin_read(w_at + at + 2u * BATCH_BYTES, x_at + at + 2u * BATCH_BYTES, batch[0]);
+            }
+            if (group + 2u * THIN_BATCH <= groups) {
+                chain = thin_add(batch[1], THIN_BATCH, chain);
+            } else {
+                chain = thin_add(batch[1], groups - group - THIN_BATCH, chain);
+            }
+        }
+    }
+    /* the fold, over the distances 16, 8, 4, 2 and 1 of the expert's 32 lanes */
+    const float sum = lanes_sum<1u>(lanes_sum<2u>(lanes_sum<4u>(lanes_sum<8u>(lanes_sum<16u>(__fadd_rn(0.0f, chain))))));
+    if (chain_of == 0u && first_expert + mine < arguments.expert_count) {
+        ((float *)(arena + arguments.output_offset))[(uint64_t)blockIdx.y * arguments.expert_count + first_expert + mine] = __fadd_rn(0.0f, sum);
+    }
+}
+
+extern "C" __global__ void __launch_bounds__(PROJECTION_THIN_THREADS)
     router_projection(struct router_projection_arguments arguments, unsigned char *arena)
 {
-    if (gridDim.y >= arguments.row_count) { /* the same in every block: a row a block */
-        router_projection_block<1u>(arguments, arena);
+    if (blockDim.x == PROJECTION_THIN_THREADS) { /* the same in every block: a row a block */
+        router_projection_thin(arguments, arena);
     } else {
-        router_projection_block<PROJECTION_MOST_ROWS>(arguments, arena);
+        router_projection_block(arguments, arena);
     }
 }
 ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_projection, router_projection_arguments);
@@ -146,7 +264,6 @@ ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_projection, router_projection_argument
  * three blocks a CU, which measured faster than three stages and two blocks): the next stage is asked for behind the
  * barrier that ends the stage before the current one. */
 typedef __attribute__((ext_vector_type(16))) float float16_t;
-typedef __attribute__((address_space(3))) void *lds_bytes;
 #define PROJECTION_STAGE_ROW_BYTES (PROJECTION_STAGE_INPUTS * 2u)
 #define PROJECTION_STAGE_ROWS (16u + PROJECTION_TILE_ROWS)
 #define PROJECTION_STAGE_BYTES (PROJECTION_STAGE_ROWS * PROJECTION_STAGE_ROW_BYTES)
@@ -166,13 +283,6 @@ __device__ static __forceinline__ void projection_convert(const uint32_t (&words
         values[k] = __uint_as_float(k % 2u == 0u ? words[k / 2u] << 16 : words[k / 2u] & 0xFFFF0000u);
         asm volatile("" : "+v"(values[k]));
     }
-}
-
-/* 16 bytes a lane from memory straight into LDS (lane L lands at lds_base + 16 L). Written as assembly: the compiler keeps
- * no book on it, so the waits for it are written out where a stage is needed. */
-__device__ static __forceinline__ void projection_load_to_lds(const void *lane_address, uint32_t lds_base)
-{
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(lane_address), "s"(lds_base) : "memory", "m0");
 }
 
 extern "C" __global__ void __launch_bounds__(PROJECTION_TILE_THREADS, 3) /* three blocks a CU */

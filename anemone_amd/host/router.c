@@ -6,7 +6,8 @@
  * per-matrix widths table.
  *
  *   launch        kernel                grid                        block
- *   projection    router_projection     (ceil(E / 8), ceil(rows / 4), 1)   128   eight experts and four rows a block
+ *   projection    router_projection     (ceil(E / 8), rows, 1)             256   thin steps: eight experts and a row a block, a lane a chain
+ *                                       (ceil(E / 8), ceil(rows / 4), 1)   128   other sizes: eight experts and four rows a block
  *                 router_projection_split (E / 16, ceil(rows / 16), 1)     256   9 rows and more of a width in whole 128, E in whole 16: 16
  *                                                                                experts by 16 rows a block
  *                 router_projection_tiles (E / 16, ceil(rows / 64), 1)     256   such steps where its fewer blocks are as many as the CUs
@@ -293,12 +294,13 @@ result_status router_projection_prepare(const struct router_projection_descripti
             return STATUS_OK;
         }
     }
-    /* a thin step: a row a block (the kernel takes the rows its grid leaves it: four a block, or one) */
+    /* a thin step: a row a block (the kernel takes one or four by its block's threads) */
     const uint32_t expert_blocks = (description->expert_count + PROJECTION_OUTPUTS - 1u) / PROJECTION_OUTPUTS;
     const bool by_row = description->row_count <= LINEAR_MAXIMUM_ROWS && expert_blocks * description->row_count <= PROJECTION_BY_ROW_MOST_BLOCKS;
     launch_fill(launch_out, kernels->projection, expert_blocks,
-                by_row ? description->row_count : (description->row_count + PROJECTION_ROWS - 1u) / PROJECTION_ROWS, 1, PROJECTION_THREADS, 0,
-                &record, sizeof record);
+                by_row ? description->row_count : (description->row_count + PROJECTION_ROWS - 1u) / PROJECTION_ROWS, 1,
+                by_row ? PROJECTION_THIN_THREADS : PROJECTION_THREADS, by_row ? PROJECTION_THIN_WINDOW_BYTES : PROJECTION_WINDOW_BYTES, &record,
+                sizeof record);
     return STATUS_OK;
 }
 

@@ -104,6 +104,9 @@ ANEMONE_RECORD_HAS(wide_expert_tile, 32);
 /* ---- router ---- */
 #define KERNEL_FILE_ROUTER "kernel_router"
 #define KERNEL_ROUTER_PROJECTION "router_projection"
+#define PROJECTION_THIN_THREADS 256u /* of its blocks of one row; those of four rows are smaller */
+#define PROJECTION_THIN_WINDOW_BYTES (9u * (4096u + 32u) * 2u) /* dynamic shared memory of a block of one row */
+#define PROJECTION_WINDOW_BYTES (12u * 1024u * 2u)             /* and of four */
 #define KERNEL_ROUTER_PROJECTION_TILES "router_projection_tiles" /* the same scores on the matrix unit: steps of many rows */
 #define PROJECTION_TILE_THREADS 256u
 #define PROJECTION_TILE_ROWS 64u   /* rows of a block of router_projection_tiles: 16 a wavefront */

@@ -196,6 +196,31 @@ def test_projection_of_many_rows_bit_exact(amd, card, experts_n, rows, hidden, s
 
 
 @pytest.mark.parametrize("experts_n,rows,hidden,scale", [
+    (64, 1, 32, 1.0), (9, 2, 96, 1.0), (72, 3, 480, 1.0),   # one group of 32 inputs; less than a batch of sixteen; a block's last experts past the last
+    (64, 8, 512, 1e-18), (64, 5, 544, 1.0), (128, 8, 1056, 3e18),  # a batch, and a group more; two batches and a group
+    (256, 1, 4096, 1.0), (256, 8, 4128, 1.0), (384, 7, 5120, 1.0), (64, 4, 8224, 1.0),  # a chunk; a group behind it; two and a group
+])
+def test_projection_of_thin_steps_bit_exact(amd, card, experts_n, rows, hidden, scale):
+    """router_projection's blocks of one row (a lane a chain, by the LDS's transposing reads) against the oracle's chains, every
+    bit, nothing written behind the scores."""
+    say("projection, thin steps", experts_n, rows, hidden, scale)
+    router = to_bf16(normals(61, experts_n * hidden) * scale).reshape(experts_n, hidden)
+    x = to_bf16(normals(62, rows * hidden) * scale).reshape(rows, hidden)
+    weights, inputs, size = card.place(router), card.place(x), rows * experts_n * 4
+    output = card.place(np.full(size + 256, 0xEE, dtype=np.uint8))
+    kernels, launch = amd.RouterKernels(), amd.launches_of(1)
+    amd.check(card.lib.router_kernels_prepare(amd.backend_table(), card.handle, C.byref(kernels)), "router_kernels_prepare")
+    d = amd.RouterProjectionDescription(amd.Range(weights, router.nbytes), amd.Range(inputs, x.nbytes), amd.Range(output, size), rows, hidden, experts_n, 0)
+    amd.check(card.lib.router_projection_prepare(C.byref(d), card.arena_bytes, C.byref(kernels), launch), "router_projection_prepare")
+    assert list(launch[0].grid) == [-(-experts_n // 8), rows, 1]
+    card.run(launch)
+    got = card.download(output, size + 256)
+    want = np.zeros((rows, experts_n), dtype=np.float32)
+    orc.orc_router_projection(ptr(x, u16p), ptr(router, u16p), rows, hidden, experts_n, ptr(want, f32p))
+    assert got[:size].tobytes() == want.tobytes() and np.all(got[size:] == 0xEE)
+
+
+@pytest.mark.parametrize("experts_n,rows,hidden,scale", [
     (64, 9, 128, 1.0),       # one stage: fewer than the kernel keeps on their way
     (64, 16, 640, 1e-18), (128, 17, 768, 1.0), (256, 33, 896, 1.0),  # as many stages as places, and around it; a tile's last rows
     (384, 63, 1024, 3e18), (256, 203, 4096, 1.0), (64, 256, 5120, 1.0),
