@@ -73,6 +73,20 @@ __device__ static __forceinline__ void exl3_chunk_load(const uint32_t *__restric
     }
 }
 
+/* the same of a base common to the wavefront and the lane's own byte offsets from it */
+template <uint32_t bits_x2>
+__device__ static __forceinline__ void exl3_chunk_load_at(const unsigned char *base, uint32_t own, uint32_t front, exl3_chunk_words<bits_x2> &out)
+{
+    typedef exl3_chunk<bits_x2> C;
+    typedef uint32_t words_t __attribute__((ext_vector_type(C::words)));
+    out.z[0] = *(const uint32_t *)(base + front);
+    const words_t load = *(const words_t *)(base + own);
+#pragma unroll
+    for (uint32_t word = 0; word < C::words; word++) {
+        out.z[word + 1u] = load[word];
+    }
+}
+
 /* K 2.5: a chunk of an odd c begins 16 bits into its first word; bring it to the form of an even one */
 template <uint32_t bits_x2>
 __device__ static __forceinline__ void exl3_chunk_align(exl3_chunk_words<bits_x2> &held, bool odd)
@@ -265,12 +279,15 @@ exl3_stream_product(const uint32_t *__restrict__ codes, uint32_t out_tiles, uint
  * half's places (one shift of the chunk a step), so that every lane's fields are constants. Each output's sums run over the
  * same operands in the same order as exl3_stream_product's: the same bits.
  * The loads run STEPS_AHEAD steps ahead (a step is two loads of codes and two of operands): the more, the fewer of a lone
- * chain's waits for memory; each costs 13 to 17 registers, and a launch of several wavefronts a SIMD needs the wavefronts.
+ * chain's waits for memory; each costs 11 to 13 registers, and a launch of several wavefronts a SIMD needs the wavefronts.
+ *   operands     fp16 operand rows of the whole wavefront; operand_at: the lane's column's row, in bytes from there (a column
+ *                that is not live names any live column's)
  *   accumulator  lane 16 g' + j: outputs 4 g' + {0..3} of the tile, column j
  */
 template <uint32_t bits_x2, uint32_t STEPS_AHEAD>
 __device__ static __forceinline__ void exl3_stream_tile_product(const uint32_t *__restrict__ codes, uint32_t out_tiles, uint32_t out_tile, uint32_t first_tile,
-                                                                uint32_t last_tile, const half_t *__restrict__ operand, uint32_t lane, float4_t &accumulator)
+                                                                uint32_t last_tile, const unsigned char *__restrict__ operands, uint32_t operand_at,
+                                                                uint32_t lane, float4_t &accumulator)
 {
     typedef exl3_chunk<bits_x2> C;
     constexpr uint32_t FOUR_SYMBOLS = 2u * bits_x2; /* bits */
@@ -278,59 +295,76 @@ __device__ static __forceinline__ void exl3_stream_tile_product(const uint32_t *
     const bool odd = (c & 1u) != 0u, upper = i >= 8u;
     uint32_t own, front;
     exl3_chunk_place<bits_x2>(c, own, front);
-    const uint64_t step_stride = 4u * (uint64_t)out_tiles * C::tile_words; /* words between steps */
-    const uint32_t *tile = codes + ((uint64_t)(first_tile + g) * out_tiles + out_tile) * C::tile_words;
-    const half_t *x = operand + (first_tile + g) * EXL3_TILE;
+    /* bases common to the wavefront, which scalar instructions move on, and the lane's own byte offsets from them */
+    const uint64_t step_stride = 16u * (uint64_t)out_tiles * C::tile_words;
+    const unsigned char *tile = (const unsigned char *)(codes + ((uint64_t)first_tile * out_tiles + out_tile) * C::tile_words);
+    const unsigned char *x = operands + first_tile * (EXL3_TILE * 2u);
+    const uint32_t lane_tile = g * out_tiles * C::tile_words; /* a K tile's row of tiles is far below 2^30 bytes */
+    own = (own + lane_tile) * 4u;
+    front = (front + lane_tile) * 4u;
+    operand_at += g * (EXL3_TILE * 2u);
     const uint32_t steps = (last_tile - first_tile) / 4u;
     accumulator = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
     exl3_chunk_words<bits_x2> held[STEPS_AHEAD];
     uint4_t values[STEPS_AHEAD][2];
-    const auto load = [&](uint32_t step, uint32_t set) {
-        exl3_chunk_load<bits_x2>(tile + step * step_stride, own, front, held[set]);
-        values[set][0] = *(const uint4_t *)(x + step * 4u * EXL3_TILE);
-        values[set][1] = *(const uint4_t *)(x + step * 4u * EXL3_TILE + 8u);
+    if (steps == 0u) { /* the same in every lane: a slice of a short matrix */
+        return;
+    }
+    uint32_t asked = 0;
+    const auto load = [&](uint32_t set) { /* the next step; past the last the last again, into registers that nobody reads: no branch around the loads */
+        exl3_chunk_load_at<bits_x2>(tile, own, front, held[set]);
+        values[set][0] = *(const uint4_t *)(x + operand_at);
+        values[set][1] = *(const uint4_t *)(x + operand_at + 16u);
+        asked++;
+        tile += asked < steps ? step_stride : 0u;
+        x += asked < steps ? 4u * EXL3_TILE * 2u : 0u;
+    };
+    const auto multiply = [&](uint32_t set) {
+        exl3_chunk_align<bits_x2>(held[set], odd);
+        uint32_t z[C::words + 1u], funnel[C::words];
+#pragma unroll
+        for (uint32_t k = 0; k < C::words; k++) {
+            const uint32_t moved = __builtin_amdgcn_alignbit(held[set].z[k], held[set].z[k + 1u], 32u - FOUR_SYMBOLS);
+            z[k] = upper ? moved : held[set].z[k];
+        }
+        z[C::words] = upper ? held[set].z[C::words] << FOUR_SYMBOLS : held[set].z[C::words];
+#pragma unroll
+        for (uint32_t k = 0; k < C::words; k++) {
+            funnel[k] = __builtin_amdgcn_alignbit(z[k], z[k + 1u], 16u);
+        }
+#pragma unroll
+        for (uint32_t v = 0; v < 2u; v++) {
+            uint32_t a[4];
+#pragma unroll
+            for (uint32_t t = 0; t < 4u; t++) {
+                a[t] = exl3_decode_pair(exl3_chunk_state<bits_x2>(z, funnel, 8u * t + 2u * v), exl3_chunk_state<bits_x2>(z, funnel, 8u * t + 2u * v + 1u));
+            }
+            const uint4_t packed = {a[0], a[1], a[2], a[3]};
+            accumulator = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, packed), __builtin_bit_cast(half8_t, values[set][v]), accumulator, 0, 0, 0);
+        }
     };
 #pragma unroll
     for (uint32_t set = 0; set < STEPS_AHEAD; set++) {
-        if (set < steps) { /* the same in every lane */
-            load(set, set);
+        if (set < steps) {
+            load(set);
         }
     }
-    for (uint32_t first = 0; first < steps; first += STEPS_AHEAD) {
+    uint32_t first = 0;
+    for (; first + STEPS_AHEAD < steps; first += STEPS_AHEAD) {
 #pragma unroll
         for (uint32_t set = 0; set < STEPS_AHEAD; set++) {
-            if (first + set >= steps) {
-                break;
-            }
-            exl3_chunk_words<bits_x2> now = held[set];
-            const uint4_t now_values[2] = {values[set][0], values[set][1]};
-            if (first + set + STEPS_AHEAD < steps) {
-                load(first + set + STEPS_AHEAD, set);
-            }
-            exl3_chunk_align<bits_x2>(now, odd);
-#pragma unroll
-            for (uint32_t k = 0; k < C::words; k++) {
-                const uint32_t moved = __builtin_amdgcn_alignbit(now.z[k], now.z[k + 1u], 32u - FOUR_SYMBOLS);
-                now.z[k] = upper ? moved : now.z[k];
-            }
-            now.z[C::words] = upper ? now.z[C::words] << FOUR_SYMBOLS : now.z[C::words];
-            uint32_t funnel[C::words];
-#pragma unroll
-            for (uint32_t k = 0; k < C::words; k++) {
-                funnel[k] = __builtin_amdgcn_alignbit(now.z[k], now.z[k + 1u], 16u);
-            }
-#pragma unroll
-            for (uint32_t v = 0; v < 2u; v++) {
-                uint32_t a[4];
-#pragma unroll
-                for (uint32_t t = 0; t < 4u; t++) {
-                    a[t] = exl3_decode_pair(exl3_chunk_state<bits_x2>(now.z, funnel, 8u * t + 2u * v),
-                                            exl3_chunk_state<bits_x2>(now.z, funnel, 8u * t + 2u * v + 1u));
-                }
-                const uint4_t packed = {a[0], a[1], a[2], a[3]};
-                accumulator = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, packed), __builtin_bit_cast(half8_t, now_values[v]), accumulator, 0, 0, 0);
-            }
+            multiply(set);
+            __builtin_amdgcn_sched_barrier(0);
+            load(set); /* behind the step and into its own registers: ahead of it the loads took copies of them */
+            __builtin_amdgcn_sched_barrier(0);
         }
+    }
+#pragma unroll
+    for (uint32_t set = 0; set < STEPS_AHEAD; set++) {
+        if (first + set >= steps) {
+            break;
+        }
+        multiply(set);
     }
 }
 

@@ -49,13 +49,16 @@ __device__ static __forceinline__ uint32_t chain_width(const struct exl3_expert_
     return exl3_width_of(((const uint32_t *)(arena + record.widths_offset))[expert], matrix);
 }
 
-extern "C" __global__ void exl3_input(struct exl3_expert_record record, unsigned char *arena)
+/* The element-wise launches (input, activate, finish): a block is 128 channels of one job, a wavefront one of its rows, or more
+ * where the job has more rows than the block wavefronts: rows one behind the other in one wavefront are a chain of their
+ * transforms (one 4096-wide matrix by eight rows: input 4.7 -> 2.3 us, finish 3.4 -> 2.2). */
+extern "C" __global__ void __launch_bounds__(EXL3_ELEMENT_MOST_THREADS) exl3_input(struct exl3_expert_record record, unsigned char *arena)
 {
     const struct expert_job_record *job = (const struct expert_job_record *)(arena + record.jobs_offset) + blockIdx.y;
     if (job->row_count == 0u) {
         return;
     }
-    const uint32_t lane = threadIdx.x, projection = blockIdx.z;
+    const uint32_t lane = threadIdx.x % WAVE, projection = blockIdx.z;
     const uint32_t channel = blockIdx.x * EXL3_TRANSFORM + wave_channel<false>(lane), to = blockIdx.x * EXL3_TRANSFORM + wave_channel<true>(lane);
     const float normalization = row_normalization(lane);
     const uint64_t matrix = projection == 0u ? job->gate_offset : job->up_offset;
@@ -64,7 +67,7 @@ extern "C" __global__ void exl3_input(struct exl3_expert_record record, unsigned
     const float s0 = half_bits_to_float(suh[channel]), s1 = half_bits_to_float(suh[channel + WAVE]);
     const uint16_t *input = (const uint16_t *)(arena + record.input_offset);
     uint16_t *operands = (uint16_t *)(arena + record.operands_offset);
-    for (uint32_t column = 0; column < job->row_count; column++) {
+    for (uint32_t column = threadIdx.x / WAVE; column < job->row_count; column += blockDim.x / WAVE) {
         const uint32_t pair = job->pair_index[column];
         const uint64_t row = pair / record.pairs_per_row;
         float v0 = __fmul_rn(bf16_to_float(input[row * record.input_size + channel]), s0);
@@ -80,13 +83,14 @@ ANEMONE_KERNEL(EXL3_KERNEL_FILE, exl3_input, exl3_expert_record);
 /* Products of one job: block = four wavefronts = the four K slices (whole steps of four K tiles) of one strip of
  * STRIP_TILES output tiles: eight (the stream product), or one in the thin instances, which a launch of few jobs takes so
  * that its blocks cover the card (the same slices and the same order of sums, so the same bits).
- * A thin launch of at most a block a CU has a wavefront a SIMD, so its time is the chain of one wavefront: its codes' loads
- * run eight steps ahead and pass through no LDS. One 4096 x 4096 matrix of K 4 by one vector: 7.8 us (13.4 with two K tiles a
- * step, a step ahead through an LDS window); the input, product and finish launches 10.8 us (16.5).
- * The thin instances of more blocks (_thin_many) run five steps ahead: 108 to 122 registers, four wavefronts a SIMD, where
- * eight ahead take 157 to 177 and leave two or three. K 4, us, eight | five | the LDS form: 512 blocks of 4096 inputs 11.8 |
- * 11.2 | 23.9; 1,024 of 4096 20.3 | 18.7 | 27.9, of 512 5.6 | 4.2 | 5.2; 1,280 of 512 7.1 | 5.3 | 5.9. Four steps ahead are
- * within 3 % of five either way, six (three wavefronts) slower from 1,024 blocks up.
+ * A thin launch of at most a block a CU has a wavefront a SIMD, so its time is the chain of one wavefront, which issues an
+ * instruction every six to seven cycles: its codes' loads run eight steps ahead and pass through no LDS, and a step is its decoding
+ * and little else (exl3_stream_tile_product: no copies of registers, scalar addresses; 103 -> 72 vector instructions a step). One
+ * 4096 x 4096 matrix of K 4 by one vector, launches queued back to back: the product 6.5 -> 5.75 us, the input, product and finish
+ * 10.5 -> 9.85 (in the first form, two K tiles a step through an LDS window, 16.5).
+ * The thin instances of more blocks (_thin_many) run five steps ahead: 80 to 90 registers, five wavefronts a SIMD, where eight
+ * ahead take 110 to 125 and leave three or four. 512 blocks, product alone, us, before | now | seven ahead: 8192 inputs of K 2.5
+ * 16.9 | 15.6 | 15.7, of K 4 17.2 | 16.8 | 17.0; 320 blocks of 5120 inputs, K 3 10.2 | 9.15 | 9.35.
  * The eight-tile instances are held to three wavefronts a SIMD: left to itself the compiler keeps the sums in accumulation
  * registers and copies beside them (175 registers, two wavefronts, for K 4): down of 32 jobs at 1536 x 5120 40.5 -> 39.0 us,
  * of 64 at 2048 x 4096 79.7 -> 74.6. */
@@ -102,16 +106,16 @@ __device__ static __forceinline__ void chain_product(const struct exl3_expert_re
     const uint32_t column = lane % 16u;
     /* a column that is not live reads the first column's operand: its sums are not stored */
     const uint32_t pair = job->pair_index[column < job->row_count ? column : 0u];
-    const half_t *operand = (const half_t *)(arena + record.operands_offset) + ((uint64_t)projection * record.pair_count + pair) * inputs;
+    const unsigned char *operands = arena + record.operands_offset + (uint64_t)projection * record.pair_count * inputs * 2u;
     const uint32_t steps = inputs / (4u * EXL3_TILE), strip_tile = blockIdx.x * STRIP_TILES;
     const uint32_t first_tile = 4u * (steps * slice / PRODUCT_WAVES), last_tile = 4u * (steps * (slice + 1u) / PRODUCT_WAVES);
     const uint32_t *codes = (const uint32_t *)(arena + matrix);
     float4_t sums[STRIP_TILES];
     if constexpr (STRIP_TILES == 1u) {
-        exl3_stream_tile_product<bits_x2, STEPS_AHEAD>(codes, outputs / EXL3_TILE, strip_tile, first_tile, last_tile, operand, lane, sums[0]);
+        exl3_stream_tile_product<bits_x2, STEPS_AHEAD>(codes, outputs / EXL3_TILE, strip_tile, first_tile, last_tile, operands, pair * inputs * 2u, lane, sums[0]);
     } else {
         float4_t accumulator[STRIP_TILES / 2u][2];
-        exl3_stream_product<bits_x2, STRIP_TILES / 2u, true>(codes, outputs / EXL3_TILE, strip_tile, first_tile, last_tile, operand, lane, accumulator);
+        exl3_stream_product<bits_x2, STRIP_TILES / 2u, true>(codes, outputs / EXL3_TILE, strip_tile, first_tile, last_tile, (const half_t *)operands + (uint64_t)pair * inputs, lane, accumulator);
 #pragma unroll
         for (uint32_t n = 0; n < STRIP_TILES; n++) {
             sums[n] = accumulator[n / 2u][n % 2u];
@@ -187,14 +191,14 @@ EXL3_PRODUCT_ENTRIES(k3, 6u);
 EXL3_PRODUCT_ENTRIES(k4, 8u);
 EXL3_PRODUCT_ENTRIES(mixed, 0u); /* the width of each matrix from the record's widths table */
 
-extern "C" __global__ void exl3_activate(struct exl3_expert_record record, unsigned char *arena)
+extern "C" __global__ void __launch_bounds__(EXL3_ELEMENT_MOST_THREADS) exl3_activate(struct exl3_expert_record record, unsigned char *arena)
 {
     const struct expert_job_record *job = (const struct expert_job_record *)(arena + record.jobs_offset) + blockIdx.y;
     if (job->row_count == 0u) {
         return;
     }
     /* the products by channel, the hidden values by the channels their transforms leave a lane with, the operand by channel again */
-    const uint32_t lane = threadIdx.x;
+    const uint32_t lane = threadIdx.x % WAVE;
     const uint32_t channel = blockIdx.x * EXL3_TRANSFORM + wave_channel<false>(lane), between = blockIdx.x * EXL3_TRANSFORM + wave_channel<true>(lane);
     const float normalization = row_normalization(lane);
     const uint32_t H = record.input_size, I = record.inner_size;
@@ -209,7 +213,7 @@ extern "C" __global__ void exl3_activate(struct exl3_expert_record record, unsig
     const float ds0 = half_bits_to_float(down_suh[between]), ds1 = half_bits_to_float(down_suh[between + WAVE]);
     const float limit = record.activation_limit;
     const float *products = (const float *)(arena + record.products_offset);
-    for (uint32_t column = 0; column < job->row_count; column++) {
+    for (uint32_t column = threadIdx.x / WAVE; column < job->row_count; column += blockDim.x / WAVE) {
         const uint32_t pair = job->pair_index[column];
         float g0 = products[(uint64_t)pair * I + channel], g1 = products[(uint64_t)pair * I + channel + WAVE];
         float u0 = products[((uint64_t)record.pair_count + pair) * I + channel];
@@ -237,20 +241,20 @@ extern "C" __global__ void exl3_activate(struct exl3_expert_record record, unsig
 }
 ANEMONE_KERNEL(EXL3_KERNEL_FILE, exl3_activate, exl3_expert_record);
 
-extern "C" __global__ void exl3_finish(struct exl3_expert_record record, unsigned char *arena)
+extern "C" __global__ void __launch_bounds__(EXL3_ELEMENT_MOST_THREADS) exl3_finish(struct exl3_expert_record record, unsigned char *arena)
 {
     const struct expert_job_record *job = (const struct expert_job_record *)(arena + record.jobs_offset) + blockIdx.y;
     if (job->row_count == 0u) {
         return;
     }
-    const uint32_t lane = threadIdx.x;
+    const uint32_t lane = threadIdx.x % WAVE;
     const uint32_t channel = blockIdx.x * EXL3_TRANSFORM + wave_channel<false>(lane), to = blockIdx.x * EXL3_TRANSFORM + wave_channel<true>(lane);
     const float normalization = row_normalization(lane);
     const uint32_t H = record.input_size, I = record.inner_size;
     const uint16_t *svh = (const uint16_t *)(arena + job->down_offset +
                                              exl3_code_bytes(I, H, exl3_bits_x2(chain_width(record, arena, job->expert, 2u)))) + I;
     const float s0 = half_bits_to_float(svh[to]), s1 = half_bits_to_float(svh[to + WAVE]);
-    for (uint32_t column = 0; column < job->row_count; column++) {
+    for (uint32_t column = threadIdx.x / WAVE; column < job->row_count; column += blockDim.x / WAVE) {
         const uint32_t pair = job->pair_index[column];
         float *values = (float *)(arena + record.products_offset) + (uint64_t)pair * H;
         float v0 = values[channel], v1 = values[channel + WAVE];

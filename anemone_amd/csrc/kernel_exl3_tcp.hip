@@ -310,20 +310,6 @@ __device__ static __forceinline__ void tcp_load_to_lds(const unsigned char *base
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_offset), "s"(base), "s"(lds_base) : "memory", "m0");
 }
 
-/* exl3_chunk_load of a base common to the wavefront and the lane's own byte offsets from it */
-template <uint32_t bits_x2>
-__device__ static __forceinline__ void tcp_chunk_load(const unsigned char *base, uint32_t own, uint32_t front, exl3_chunk_words<bits_x2> &out)
-{
-    typedef exl3_chunk<bits_x2> C;
-    typedef uint32_t words_t __attribute__((ext_vector_type(C::words)));
-    out.z[0] = *(const uint32_t *)(base + front);
-    const words_t load = *(const words_t *)(base + own);
-#pragma unroll
-    for (uint32_t word = 0; word < C::words; word++) {
-        out.z[word + 1u] = load[word];
-    }
-}
-
 #define TCP_STAGE_COLUMN_BYTES (TCP_STEP_INPUTS * 2u)
 #define TCP_STAGE_BYTES (EXL3_TCP_CHUNK_PAIRS * TCP_STAGE_COLUMN_BYTES)
 
@@ -379,7 +365,7 @@ tcp_wave_gemm(const uint32_t *__restrict__ codes, uint32_t out_tiles, uint32_t s
     exl3_chunk_words<bits_x2> held[2][2];
 #pragma unroll
     for (uint32_t s = 0; s < 2u; s++) {
-        tcp_chunk_load<bits_x2>(tile + s * half_stride, own, front, held[0][s]);
+        exl3_chunk_load_at<bits_x2>(tile + s * half_stride, own, front, held[0][s]);
     }
 #pragma unroll
     for (uint32_t part = 0; part < wave_groups; part++) {
@@ -422,7 +408,7 @@ tcp_wave_gemm(const uint32_t *__restrict__ codes, uint32_t out_tiles, uint32_t s
         tile += step_stride;
 #pragma unroll
         for (uint32_t s = 0; s < 2u; s++) {
-            tcp_chunk_load<bits_x2>(tile + s * half_stride, own, front, next[s]);
+            exl3_chunk_load_at<bits_x2>(tile + s * half_stride, own, front, next[s]);
         }
 #pragma unroll
         for (uint32_t part = 0; part < wave_groups; part++) {

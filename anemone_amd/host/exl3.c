@@ -4,13 +4,14 @@
  * source/exl3_tp.c:250-290; the launch geometry is gfx950's:
  *
  *   launch          kernel                      grid                                  block
- *   input           exl3_input                  (input_size / 128, jobs, 2)           64   one wavefront a transform
+ *   input           exl3_input                  (input_size / 128, jobs, 2)           64 x rows of a job on average (1 to 8): a wavefront a
+ *                                                                                     transform
  *   gate/up         exl3_gate_up_<k>|_mixed     (inner_size / 128, jobs, 2)           256  4 K slices x 8 output tiles
- *   activate        exl3_activate               (inner_size / 128, jobs, 1)           64
+ *   activate        exl3_activate               (inner_size / 128, jobs, 1)           likewise
  *   down            exl3_down_<k>|_mixed        (input_size / 128, jobs, 1)           256
  *   (a product launch of at most EXL3_THIN_BLOCKS, EXL3_THIN_MANY_BLOCKS blocks of one output tile: the _thin, _thin_many
  *   instance, x = size / 16)
- *   finish          exl3_finish                 (input_size / 128, jobs, 1)           64
+ *   finish          exl3_finish                 (input_size / 128, jobs, 1)           likewise
  *   row sum         exl3_row_sum                (ceil(width / 256), rows, 1)          256
  *
  * <k> is the record's one width; "_mixed" is taken when the record names a per-matrix widths table.
@@ -71,13 +72,17 @@ result_status exl3_reconstruct_prepare(const struct exl3_reconstruct_record *rec
 }
 
 /* the form of a product launch over `projections` matrices of `outputs` outputs for each of `jobs` jobs (the lines:
- * anemone_records.h). Every form gives the same sums. */
+ * anemone_records.h). Every form gives the same sums. operand_bytes: of a projection's operands, which the forms of one tile name
+ * by offsets of 32 bits. */
 static struct product_form {
     const char *suffix;
     uint32_t block_outputs;
-} product_form_of(uint32_t outputs, uint32_t jobs, uint32_t projections)
+} product_form_of(uint32_t outputs, uint32_t jobs, uint32_t projections, uint64_t operand_bytes)
 {
     const uint64_t thin_blocks = (uint64_t)(outputs / (EXL3_THIN_STRIP_TILES * EXL3_TILE)) * jobs * projections;
+    if (operand_bytes > UINT32_MAX) {
+        return (struct product_form){"", STRIP_OUTPUTS};
+    }
     return thin_blocks <= EXL3_THIN_BLOCKS        ? (struct product_form){"_thin", EXL3_THIN_STRIP_TILES * EXL3_TILE}
            : thin_blocks <= EXL3_THIN_MANY_BLOCKS ? (struct product_form){"_thin_many", EXL3_THIN_STRIP_TILES * EXL3_TILE}
                                                   : (struct product_form){"", STRIP_OUTPUTS};
@@ -139,19 +144,22 @@ static result_status chain_prepare(const struct exl3_expert_record *record, uint
     }
     char gate_up_name[40], down_name[40];
     const char *width = mixed ? "mixed" : exl3_width_name(exl3_bits_x2(record->bits_per_weight));
-    const struct product_form gate_up = product_form_of(record->inner_size, record->job_count, 2u);
-    const struct product_form down = product_form_of(record->input_size, record->job_count, 1u);
+    /* the element-wise launches: a wavefront a row of a job, as many as the jobs hold on average */
+    const uint32_t rows_of_job = record->pair_count / record->job_count;
+    const uint32_t element_threads = WAVE_THREADS * (rows_of_job == 0u ? 1u : rows_of_job < LINEAR_MAXIMUM_ROWS ? rows_of_job : LINEAR_MAXIMUM_ROWS);
+    const struct product_form gate_up = product_form_of(record->inner_size, record->job_count, 2u, inputs * 2u);
+    const struct product_form down = product_form_of(record->input_size, record->job_count, 1u, (uint64_t)record->pair_count * record->inner_size * 2u);
     (void)snprintf(gate_up_name, sizeof gate_up_name, "exl3_gate_up_%s%s", width, gate_up.suffix);
     (void)snprintf(down_name, sizeof down_name, "exl3_down_%s%s", width, down.suffix);
     const struct {
         const char *name;
         uint32_t width, threads, projections, block_outputs;
     } stages[EXL3_EXPERT_LAUNCHES] = {
-        {"exl3_input", record->input_size, WAVE_THREADS, 2u, EXL3_TRANSFORM},
+        {"exl3_input", record->input_size, element_threads, 2u, EXL3_TRANSFORM},
         {gate_up_name, record->inner_size, PRODUCT_THREADS, 2u, gate_up.block_outputs},
-        {"exl3_activate", record->inner_size, WAVE_THREADS, 1u, EXL3_TRANSFORM},
+        {"exl3_activate", record->inner_size, element_threads, 1u, EXL3_TRANSFORM},
         {down_name, record->input_size, PRODUCT_THREADS, 1u, down.block_outputs},
-        {"exl3_finish", record->input_size, WAVE_THREADS, 1u, EXL3_TRANSFORM},
+        {"exl3_finish", record->input_size, element_threads, 1u, EXL3_TRANSFORM},
     };
     struct kernel_launch launches[EXL3_EXPERT_LAUNCHES];
     for (uint32_t stage = 0; stage < EXL3_EXPERT_LAUNCHES; stage++) {

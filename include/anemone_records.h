@@ -217,6 +217,7 @@ ANEMONE_RECORD_HAS(router_wide_arguments, 136);
 #define EXL3_NORMALIZATION 0.08838834764831845f
 #define EXL3_EXPERT_LAUNCHES 5u
 #define EXL3_PRODUCT_SLICES 4u
+#define EXL3_ELEMENT_MOST_THREADS 512u /* of a block of the chain's element-wise launches: a wavefront a row of a job */
 #define EXL3_STRIP_TILES 8u      /* output tiles of a block of the chain's product launches: 128 outputs */
 #define EXL3_THIN_STRIP_TILES 1u /* of the _thin and _thin_many instances */
 /* A product launch takes one tile a block while that makes at most this many blocks. By 256 of them, a block a CU, a wavefront
