@@ -544,6 +544,45 @@ __device__ static __forceinline__ uint32_t wide_live_rows(const struct router_wi
     return step_rows < arguments.row_count ? step_rows : arguments.row_count;
 }
 
+/* a lane's values of a row: its `places` experts lie next to each other, from lane * places on (0 past them) */
+__device__ static __forceinline__ void router_lane_values(const float *row, uint32_t lane, uint32_t places, float (&values)[ROUTER_PLACES])
+{
+    typedef float4_t float4_of_words __attribute__((aligned(4)));
+    float4_t four = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (places == 4u) {
+        four = ((const float4_of_words *)row)[lane];
+    }
+#pragma unroll
+    for (uint32_t place = 0; place < ROUTER_PLACES; place++) {
+        values[place] = place < 4u ? four[place % 4u] : 0.0f;
+        if (places != 4u && place < places) {
+            values[place] = row[lane * places + place];
+        }
+    }
+}
+
+/* a row from its scores on: the affinities (LDS and memory), the keys, the picks. places: PLACES, or fewer, where the lane's
+ * others hold key 0 and are never taken */
+template <uint32_t PLACES>
+__device__ static __forceinline__ void router_row_of_scores(const float (&scores)[ROUTER_PLACES], const float (&bias)[ROUTER_PLACES],
+                                                            float *affinities, float *affinities_out, uint32_t lane, uint32_t places, uint32_t affinity_kind,
+                                                            uint32_t picks, uint32_t reference_order, float route_scale, uint32_t &expert_out,
+                                                            float &weight_out)
+{
+    uint32_t keys[PLACES];
+#pragma unroll
+    for (uint32_t place = 0; place < PLACES; place++) {
+        keys[place] = 0u;
+        if (place < places) {
+            const float a = router_affinity(scores[place], affinity_kind);
+            affinities[lane * places + place] = a;
+            affinities_out[lane * places + place] = a;
+            keys[place] = router_key(__fadd_rn(a, bias[place]));
+        }
+    }
+    router_row<PLACES>(affinities, keys, lane, places, picks, reference_order, route_scale, expert_out, weight_out);
+}
+
 /* grid (ceil(row_count / 8)), a wavefront a row: its affinities, as the select writes them, and its picks by slot */
 extern "C" __global__ void __launch_bounds__(SELECT_THREADS)
     router_wide_select(struct router_wide_arguments arguments, unsigned char *arena)
@@ -557,20 +596,19 @@ extern "C" __global__ void __launch_bounds__(SELECT_THREADS)
     const uint32_t live_rows = wide_live_rows(arguments, arena);
     const uint64_t first = (uint64_t)(row < arguments.row_count ? row : 0u) * experts;
     float bias_of[ROUTER_PLACES], scores[ROUTER_PLACES];
-#pragma unroll
-    for (uint32_t place = 0; place < ROUTER_PLACES; place++) {
-        bias_of[place] = place < places ? ((const float *)(arena + arguments.bias_offset))[lane + place * WAVE] : 0.0f;
-        scores[place] = place < places ? ((const float *)(arena + arguments.scores_offset))[first + lane + place * WAVE] : 0.0f;
-    }
+    router_lane_values((const float *)(arena + arguments.bias_offset), lane, places, bias_of);
+    router_lane_values((const float *)(arena + arguments.scores_offset) + first, lane, places, scores);
     if (row >= live_rows) {
         return; /* no barrier in this kernel: a wavefront is a row */
     }
     struct router_pick my_pick;
-    uint32_t my_slot;
-    router_row_any(scores, bias_of, experts, affinities + wave * experts, (float *)(arena + arguments.affinities_offset) + first, lane,
-                   arguments.affinity_kind, picks, arguments.reference_order, arguments.route_scale, my_pick.expert, my_slot, my_pick.route_weight);
-    if (lane < picks) { /* lane p holds pick p */
-        ((struct router_pick *)(arena + arguments.picks_offset))[(uint64_t)row * picks + my_slot] = my_pick;
+    float *own = affinities + wave * experts, *out = (float *)(arena + arguments.affinities_offset) + first;
+    router_by_places(places, [&](auto count) {
+        router_row_of_scores<count.value>(scores, bias_of, own, out, lane, places, arguments.affinity_kind, picks, arguments.reference_order,
+                                          arguments.route_scale, my_pick.expert, my_pick.route_weight);
+    });
+    if (lane < picks) { /* lane s holds the pick of slot s */
+        ((struct router_pick *)(arena + arguments.picks_offset))[(uint64_t)row * picks + lane] = my_pick;
     }
 }
 ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_wide_select, router_wide_arguments);

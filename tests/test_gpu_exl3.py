@@ -118,6 +118,45 @@ def test_router_bit_exact(amd, card, affinity_kind, experts_n, picks, order):
     assert layer.jobs().tobytes() == jobs.tobytes()
 
 
+@pytest.mark.parametrize("experts_n,picks,rows,live,kind", [
+    (64, 8, 8, 8, 1), (128, 1, 1, 1, 0), (192, 7, 3, 2, 1), (256, 8, 1, 1, 1), (256, 8, 8, 8, 0), (320, 5, 2, 2, 1),
+    (384, 8, 8, 5, 0), (448, 6, 4, 4, 1), (512, 8, 8, 8, 1), (512, 2, 1, 0, 0),
+])
+def test_select_of_equal_and_special_keys(amd, card, experts_n, picks, rows, live, kind):
+    """Scores of few values, so that most picks are ties inside a lane's experts and between lanes, and biases of both infinities,
+    both zeros and a not-a-number at the first and last experts: the lowest of equal experts, everywhere, by the thin and the wide
+    select, whose affinities and picks equal the oracle's bit for bit."""
+    say("select of equal keys", experts_n, picks, rows, live, kind)
+    layer, _, _, _ = build_layer(amd, card, 512, 128, experts_n, picks, rows, 5, [2], kind)
+    scores = (np.floor(normals(31 + experts_n, rows * experts_n) * 2.0) * 0.5).astype(np.float32).reshape(rows, experts_n)
+    bias = (np.floor(normals(7 + picks, experts_n)) * 0.25).astype(np.float32)
+    bias[[0, 1, experts_n // 2, experts_n - 2]] = [-0.0, -np.inf, np.inf, 0.0]
+    bias[experts_n - 1] = np.nan if picks > 2 else -np.inf
+    card.upload(layer.bias_offset, bias)
+    card.upload(layer.scores_offset, scores)
+    layer.set_rows(np.zeros((rows, 512), dtype=np.uint16), live)
+    affinities = np.array([[orc.orc_router_affinity(float(v), kind) for v in row] for row in scores], dtype=np.float32)
+    experts, weights = np.zeros((rows, picks), dtype=np.uint32), np.zeros((rows, picks), dtype=np.float32)
+    for r in range(live):
+        orc.orc_router_select(ptr(affinities[r], f32p), ptr(bias, f32p), experts_n, picks, 0, layer.route_scale,
+                              ptr(experts[r], u32p), ptr(weights[r], f32p))
+    card.run(layer.select_launch(0))
+    got = card.download(layer.affinities_offset, rows * experts_n * 4, np.float32).reshape(rows, experts_n)
+    assert np.array_equal(got[:live].view(np.uint32), affinities[:live].view(np.uint32))
+    jobs = layer.jobs()
+    seen = {}
+    for job in jobs:
+        for column in range(job["row_count"]):
+            seen[int(job["pair_index"][column])] = (int(job["expert"]), job["route_weight"][column].tobytes())
+    assert seen == {r * picks + s: (int(experts[r, s]), weights[r, s].tobytes()) for r in range(live) for s in range(picks)}
+    used = [int(job["expert"]) for job in jobs if job["row_count"] > 0]
+    assert used == sorted(set(experts[:live].reshape(-1).tolist())) and not jobs[len(used):].tobytes().strip(b"\0")
+    wide = layer.wide_router()
+    card.run(wide.launches()[:1])
+    chosen = wide.read("picks", np.dtype([("expert", "<u4"), ("route_weight", "<f4")])).reshape(rows, picks)[:live]
+    assert np.array_equal(chosen["expert"], experts[:live]) and chosen["route_weight"].tobytes() == weights[:live].tobytes()
+
+
 def test_router_hand_rows_on_the_card(amd, card):
     """The reference's hand rows (ties, NaN bias, -0 < +0) through the kernel: scores chosen so the affinities are
     the rows' values is not possible (affinity is computed), so the choice is exercised through the bias."""
