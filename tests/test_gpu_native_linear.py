@@ -337,6 +337,13 @@ def test_native_job_table_kernels_equal_the_reference_lay_out(amd, card, hidden,
             assert a.reshape(-1)[:count].tobytes() != bytes([0xEE]) * count, "the launches wrote"
 
 
+@pytest.mark.parametrize("steps", range(1, 8))
+@pytest.mark.parametrize("fmt", [E2M1, E4M3])
+def test_native_thin_chains_of_every_length(amd, card, steps, fmt):
+    """The job-table kernels' last K steps, an instance for every number of them, and the steady state ahead of them."""
+    test_native_job_table_kernels_equal_the_reference_lay_out(amd, card, 128 * steps, 128 * (8 - steps), 2, 5, 5, fmt, 1, 1)
+
+
 @pytest.mark.parametrize("hidden,inner,rows,live", [(512, 384, 100, 100), (640, 128, 70, 67), (256, 128, 2500, 2497)])
 def test_narrow_and_whole_strips_give_the_same_bytes(amd, card, hidden, inner, rows, live):
     """The 4-bit wide launches of strips of half the tiles (native_expert_gate_up_narrow_1, native_expert_down_narrow_1) and

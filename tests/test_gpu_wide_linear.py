@@ -114,6 +114,29 @@ def test_wide_chunks_of_scale_words(amd, card, hidden, inner, picks, rows, fmt):
     test_wide_equals_the_job_table_kernels_byte_for_byte(amd, card, hidden, inner, 64, picks, rows, rows, fmt)
 
 
+@pytest.mark.parametrize("steps", range(1, 8))
+@pytest.mark.parametrize("fmt", [E2M1, E4M3])
+def test_thin_chains_of_every_length(amd, card, steps, fmt):
+    """The job-table kernels' last K steps, an instance for every number of them, and the steady state ahead of them (two stages
+    of gate/up, three of down: 1 to 3 and 1 to 5 steps), byte for byte as the wide kernels add them."""
+    say("thin chains of", steps, "and", 8 - steps, "steps, format", fmt)
+    hidden, inner, rows, picks = 128 * steps, 128 * (8 - steps), 9, 2
+    layer, _ = build(amd, card, hidden, inner, 64, picks, rows, 22, fmt)
+    layer.gate_up_slices = layer.down_slices = 1
+    layer.set_rows(to_bf16(normals(32, rows * hidden)).reshape(rows, hidden), rows)
+    card.run(layer.projection_launch())
+    wide = layer.wide_router()
+    card.run(wide.launches())
+    card.run(layer.quantize_launch())
+    outputs = []
+    for launches in (layer.expert_launches(wide), layer.wide_expert_launches(wide)):
+        for name in ("hidden_codes", "pair_output"):
+            card.upload(layer.ranges[name].byte_offset, np.full(layer.ranges[name].byte_count, 0xEE, dtype=np.uint8))
+        card.run(launches)
+        outputs.append([layer.read(name).tobytes() for name in ("hidden_codes", "hidden_exponents", "pair_output", "row_output")])
+    assert outputs[0] == outputs[1]
+
+
 def test_wide_layer_against_oracle(amd, card):
     """The whole layer in its wide form (projection, wide select, quantizer, wide gate/up, wide down, row sum) against
     the CPU oracle's layer of the same picks."""
