@@ -62,7 +62,7 @@ __device__ static __forceinline__ void hyper_row_input_body(const struct hyper_f
 #pragma unroll
     for (uint32_t stream = 0; stream < MODEL_STREAMS; stream++) {
         float values[HYPER_VALUES_PER_THREAD];
-        join_unpack(loads[stream], values);
+        join_unpack<HYPER_VALUES_PER_THREAD>(loads[stream], values);
 #pragma unroll
         for (uint32_t v = 0; v < HYPER_VALUES_PER_THREAD; v++) {
             hidden[v] = __fadd_rn(hidden[v], __fmul_rn(pre[stream], values[v]));
@@ -83,12 +83,12 @@ __device__ static __forceinline__ void hyper_row_input_body(const struct hyper_f
                                     MODEL_NORM_EPSILON);
     const float factor = (float)(1.0 / __dsqrt_rn((double)operand));
     float weights[HYPER_VALUES_PER_THREAD];
-    join_unpack(weight_load, weights);
+    join_unpack<HYPER_VALUES_PER_THREAD>(weight_load, weights);
 #pragma unroll
     for (uint32_t v = 0; v < HYPER_VALUES_PER_THREAD; v++) {
         hidden[v] = __fmul_rn(weights[v], __fmul_rn(hidden[v], factor));
     }
-    ((uint4_t *)(arena + arguments.hidden_offset))[row * row_threads + thread] = join_pack(hidden);
+    ((uint4_t *)(arena + arguments.hidden_offset))[row * row_threads + thread] = join_pack<HYPER_VALUES_PER_THREAD>(hidden);
 }
 
 /* Row `row`'s post, comb and pre from its mixes, by sixteen threads `thread` 0 .. 15 that are sixteen lanes in a row of one

@@ -27,7 +27,7 @@ extern "C" __global__ void __launch_bounds__(HYPER_PIECE_THREADS) hyper_post_ent
     const float *comb = (const float *)(arena + arguments.comb_offset) + row * MODEL_STREAMS * MODEL_STREAMS;
     uint4_t *streams = (uint4_t *)(arena + arguments.streams_offset) + row * MODEL_STREAMS * row_threads + thread;
     float output[HYPER_VALUES_PER_THREAD];
-    join_unpack(((const uint4_t *)(arena + arguments.output_offset))[row * row_threads + thread], output);
+    join_unpack<HYPER_VALUES_PER_THREAD>(((const uint4_t *)(arena + arguments.output_offset))[row * row_threads + thread], output);
     if (arguments.is_combined != 0u) {
         const float4_t *sums = (const float4_t *)(arena + arguments.sums_offset) + (row * row_threads + thread) * 2u;
         const float4_t low = sums[0], high = sums[1];
@@ -36,7 +36,7 @@ extern "C" __global__ void __launch_bounds__(HYPER_PIECE_THREADS) hyper_post_ent
             output[v] = bf16_to_float(float_to_bf16(__fadd_rn(v < 4u ? low[v % 4u] : high[v % 4u], output[v])));
         }
     }
-    join_post_values(output, post, comb, streams, row_threads);
+    join_write_streams<HYPER_VALUES_PER_THREAD>(output, join_read_streams<HYPER_VALUES_PER_THREAD>(post, comb, streams, row_threads), streams, row_threads);
 }
 ANEMONE_KERNEL(KERNEL_FILE_HYPER_CONNECTION, hyper_post_entry, hyper_post_arguments);
 
@@ -44,15 +44,16 @@ extern "C" __global__ void __launch_bounds__(HYPER_PIECE_THREADS) expert_join(st
 {
     const uint64_t row = blockIdx.y, row_threads = (uint64_t)gridDim.x * blockDim.x, thread = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     float shared_output[HYPER_VALUES_PER_THREAD];
-    join_unpack(((const uint4_t *)(arena + arguments.shared_output_offset))[row * row_threads + thread], shared_output);
-    join_values((const uint4_t *)(arena + arguments.pair_output_offset) + row * arguments.pairs_per_row * row_threads + thread,
-                arguments.pairs_per_row, shared_output, (const float *)(arena + arguments.post_offset) + row * MODEL_STREAMS,
-                (const float *)(arena + arguments.comb_offset) + row * MODEL_STREAMS * MODEL_STREAMS,
-                (uint4_t *)(arena + arguments.streams_offset) + row * MODEL_STREAMS * row_threads + thread,
-                arguments.row_sums_offset == EXPERT_JOIN_NO_ROW_SUMS
-                    ? nullptr
-                    : (float4_t *)(arena + arguments.row_sums_offset) + (row * row_threads + thread) * 2u,
-                row_threads);
+    constexpr uint32_t VALUES = HYPER_VALUES_PER_THREAD;
+    const uint4_t *pairs = (const uint4_t *)(arena + arguments.pair_output_offset) + row * arguments.pairs_per_row * row_threads + thread;
+    uint4_t *streams = (uint4_t *)(arena + arguments.streams_offset) + row * MODEL_STREAMS * row_threads + thread;
+    const join_slots<VALUES> slots = join_read_slots<VALUES>(pairs, arguments.pairs_per_row, row_threads);
+    const join_streams<VALUES> read = join_read_streams<VALUES>((const float *)(arena + arguments.post_offset) + row * MODEL_STREAMS,
+                                                               (const float *)(arena + arguments.comb_offset) + row * MODEL_STREAMS * MODEL_STREAMS, streams, row_threads);
+    join_unpack<VALUES>(((const uint4_t *)(arena + arguments.shared_output_offset))[row * row_threads + thread], shared_output);
+    join_values<VALUES>(pairs, arguments.pairs_per_row, slots, shared_output, read, streams,
+                        arguments.row_sums_offset == EXPERT_JOIN_NO_ROW_SUMS ? nullptr : (float *)(arena + arguments.row_sums_offset) + (row * row_threads + thread) * VALUES,
+                        row_threads);
 }
 ANEMONE_KERNEL(KERNEL_FILE_HYPER_CONNECTION, expert_join, expert_join_arguments);
 

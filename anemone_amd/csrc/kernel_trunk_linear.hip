@@ -189,35 +189,40 @@ __device__ static __forceinline__ void trunk_linear_quantized_interleaved(const 
     }
 }
 
-/* The shared expert's down and the join of its strip: grid (ceil(width / 32), 1), block 64 S. Thread 4 r + h joins
- * values 8 h .. 8 h + 7 of the strip for row r, reading the strip's outputs from the block's copy. */
+/* The shared expert's down and the join of its strip: grid (ceil(width / 32), 1), block 64 S. A thread joins two values of the
+ * strip for one row (four where the block is one wavefront), reading the strip's outputs from the block's copy: eight values a
+ * thread were 700 instructions of a quarter of one wavefront while the others had ended. What the join reads of other launches'
+ * results is asked for ahead of the product and stays in registers (4096 x 2048, five rows of eight pairs: 6.3 -> 4.85 us). */
 template <uint32_t S>
 __device__ static __forceinline__ void expert_shared_join(const struct expert_shared_join_arguments &arguments, unsigned char *arena)
 {
     TRUNK_WINDOW(S);
+    constexpr uint32_t VALUES = S == 1u ? 4u : 2u, PIECES = TRUNK_STRIP_OUTPUTS / VALUES;
+    static_assert(LINEAR_MAXIMUM_ROWS * PIECES <= S * WAVE, "a thread a piece of a row");
     __shared__ __attribute__((aligned(16))) uint16_t copy[LINEAR_MAXIMUM_ROWS][TRUNK_STRIP_OUTPUTS];
     const uint32_t width = arguments.reserved_zero == 0u ? 5120u : arguments.reserved_zero, strip = blockIdx.x;
+    const uint32_t row = threadIdx.x / PIECES, piece = threadIdx.x % PIECES;
+    /* a last strip that reaches past the matrix starts earlier: its first outputs are the strip's before it */
+    const uint32_t tiles = width / 16u, tile0 = strip * 2u + 2u <= tiles ? strip * 2u : tiles - 2u;
+    const uint32_t output = tile0 * 16u + piece * VALUES;
+    const bool joins = row < arguments.row_count && output >= strip * TRUNK_STRIP_OUTPUTS;
+    const uint64_t row_loads = width / VALUES, load = output / VALUES, own_row = row < arguments.row_count ? row : 0u;
+    const join_load<VALUES> *pairs = (const join_load<VALUES> *)(arena + arguments.pair_output_offset) + own_row * arguments.pairs_per_row * row_loads + load;
+    join_load<VALUES> *streams = (join_load<VALUES> *)(arena + arguments.streams_offset) + own_row * MODEL_STREAMS * row_loads + load;
+    const join_slots<VALUES> slots = join_read_slots<VALUES>(pairs, arguments.pairs_per_row, row_loads);
+    const join_streams<VALUES> read = join_read_streams<VALUES>((const float *)(arena + arguments.post_offset) + own_row * MODEL_STREAMS,
+                                                               (const float *)(arena + arguments.comb_offset) + own_row * MODEL_STREAMS * MODEL_STREAMS, streams, row_loads);
     trunk_strip<S>(arena + arguments.weights_offset, width, arguments.input_size, strip, arena + arguments.codes_offset,
                    arena + arguments.exponents_offset, 0u, arguments.row_count, (uint16_t *)(arena + arguments.output_offset), window, &copy[0][0]);
     __syncthreads();
-    const uint32_t row = threadIdx.x / 4u, piece = threadIdx.x % 4u;
-    /* a last strip that reaches past the matrix starts earlier: its first outputs are the strip's before it */
-    const uint32_t tiles = width / 16u, tile0 = strip * 2u + 2u <= tiles ? strip * 2u : tiles - 2u;
-    const uint32_t output = tile0 * 16u + piece * HYPER_VALUES_PER_THREAD;
-    if (row >= arguments.row_count || output < strip * TRUNK_STRIP_OUTPUTS) {
+    if (!joins) {
         return;
     }
-    const uint64_t row_threads = width / HYPER_VALUES_PER_THREAD, thread = output / HYPER_VALUES_PER_THREAD;
-    float shared_output[HYPER_VALUES_PER_THREAD];
-    join_unpack(*(const uint4_t *)&copy[row][piece * HYPER_VALUES_PER_THREAD], shared_output);
-    join_values((const uint4_t *)(arena + arguments.pair_output_offset) + (uint64_t)row * arguments.pairs_per_row * row_threads + thread,
-                arguments.pairs_per_row, shared_output, (const float *)(arena + arguments.post_offset) + (uint64_t)row * MODEL_STREAMS,
-                (const float *)(arena + arguments.comb_offset) + (uint64_t)row * MODEL_STREAMS * MODEL_STREAMS,
-                (uint4_t *)(arena + arguments.streams_offset) + (uint64_t)row * MODEL_STREAMS * row_threads + thread,
-                arguments.row_sums_offset == EXPERT_JOIN_NO_ROW_SUMS
-                    ? nullptr
-                    : (float4_t *)(arena + arguments.row_sums_offset) + ((uint64_t)row * row_threads + thread) * 2u,
-                row_threads);
+    float shared_output[VALUES];
+    join_unpack<VALUES>(*(const join_load<VALUES> *)&copy[row][piece * VALUES], shared_output);
+    join_values<VALUES>(pairs, arguments.pairs_per_row, slots, shared_output, read, streams,
+                        arguments.row_sums_offset == EXPERT_JOIN_NO_ROW_SUMS ? nullptr : (float *)(arena + arguments.row_sums_offset) + own_row * width + output,
+                        row_loads);
 }
 
 #define TRUNK_ENTRIES(S)                                                                                          \
@@ -265,14 +270,14 @@ extern "C" __global__ void trunk_hidden_entry(struct trunk_hidden_arguments argu
     const float limit = arguments.activation_limit;
     if (arguments.width % HYPER_VALUES_PER_THREAD == 0u) {
         float g[HYPER_VALUES_PER_THREAD], u[HYPER_VALUES_PER_THREAD], h[HYPER_VALUES_PER_THREAD];
-        join_unpack(*(const uint4_t *)gate, g);
-        join_unpack(*(const uint4_t *)up, u);
+        join_unpack<HYPER_VALUES_PER_THREAD>(*(const uint4_t *)gate, g);
+        join_unpack<HYPER_VALUES_PER_THREAD>(*(const uint4_t *)up, u);
 #pragma unroll
         for (uint32_t v = 0; v < HYPER_VALUES_PER_THREAD; v++) {
             const float bounded_gate = fminf(g[v], limit), bounded_up = fminf(fmaxf(u[v], -limit), limit);
             h[v] = __fmul_rn(__fmul_rn(det_silu(bounded_gate), bounded_up), 1.0f);
         }
-        *(uint4_t *)hidden = join_pack(h);
+        *(uint4_t *)hidden = join_pack<HYPER_VALUES_PER_THREAD>(h);
         return;
     }
     for (uint32_t v = 0; v < HYPER_VALUES_PER_THREAD && first + v < arguments.width; v++) {

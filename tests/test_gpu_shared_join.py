@@ -248,6 +248,30 @@ def test_shared_join_equals_the_separate_launches(amd, card, rows, slices, hidde
     assert not np.all(fused[1] == streams.view(np.uint8).reshape(-1))
 
 
+@pytest.mark.parametrize("rows,slices,per_row", [(8, 8, 8), (8, 1, 1), (5, 1, 12), (6, 2, 9), (1, 4, 7), (5, 4, 12)])
+def test_shared_join_of_any_slots(amd, card, rows, slices, per_row):
+    """The shared join by two or four values a thread, of fewer pair outputs a row than it asks for together and of more,
+    infinities, not-a-numbers and signed zeros among them, against the separate launches, every byte."""
+    say("shared join of", per_row, "slots", rows, slices)
+    hidden = 1024
+    layer, shared, _ = build(amd, card, hidden, 256, 8, 8, 15, shared_inner=1024, down_slices=slices)
+    routed_step(card, layer, to_bf16(normals(33, 8 * hidden)).reshape(8, hidden))
+    card.run(shared.launches())
+    layer.P = per_row
+    pairs = to_bf16(normals(34, 64 * hidden) * 2.0).reshape(64, hidden)
+    pairs[0, ::3], pairs[rows * per_row - 1, 1::5], pairs[per_row // 2, 2::7] = 0x8000, 0xFF80, 0x7FC1
+    card.upload(layer.ranges["pair_output"].byte_offset, pairs)
+    results = []
+    for launches in ([shared.launches()[3:4], shared.join_launch(rows)], [shared.shared_join_launch(rows)]):
+        shared.set_site(*site_of(35, 8, hidden))
+        card.upload(shared.ranges["row_sums"].byte_offset, np.full(shared.ranges["row_sums"].byte_count, 0xEE, dtype=np.uint8))
+        for launch in launches:
+            card.run(launch)
+        results.append([shared.read("streams").tobytes(), shared.read("row_sums").tobytes(),
+                        shared.read("output", np.uint16).reshape(8, hidden)[:rows].tobytes()])
+    assert results[0] == results[1]
+
+
 def test_layer_with_shared_expert_and_join_against_oracle(amd, card):
     """The whole FFN site of a wide step: routed experts in their wide form, the shared expert in its interleaved form,
     the join; streams against the oracle's join of the oracle's own routed and shared outputs."""
