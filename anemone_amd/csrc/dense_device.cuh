@@ -21,10 +21,13 @@ __device__ static __forceinline__ float dense_reciprocal_root(float operand)
 }
 
 template <uint32_t distance, uint32_t ROWS, uint32_t OUTPUTS>
-__device__ static __forceinline__ void dense_add_lanes(float (&chain)[OUTPUTS][ROWS], float (&squares)[ROWS], bool scaled)
+__device__ static __forceinline__ void dense_add_lanes(float (&chain)[OUTPUTS][ROWS], float (&squares)[ROWS], bool scaled, uint32_t live)
 {
 #pragma unroll
     for (uint32_t r = 0; r < ROWS; r++) {
+        if (ROWS > 1u && r >= live) {
+            break;
+        }
 #pragma unroll
         for (uint32_t o = 0; o < OUTPUTS; o++) {
             chain[o][r] = lanes_sum<distance>(chain[o][r]);
@@ -42,8 +45,10 @@ template <uint32_t ROWS, uint32_t OUTPUTS> struct dense_group_sums {
 
 /* OUTPUTS outputs from first_output on by ROWS rows from first_row on, by the DENSE_THREADS_VALUE threads `thread` 0 ..
  * (every one of them calls, and the others of the block reach the same barrier: `active` false computes and stores
- * nothing that is read). `rows` names row 0 of the rows (memory or LDS). */
-template <uint32_t TYPE, uint32_t ROWS, uint32_t OUTPUTS>
+ * nothing that is read). `rows` names row 0 of the rows (memory or LDS). FRONT, of a launch of few blocks whose time is its
+ * wavefronts' instructions: the places of the eight that hold no row are not computed, and the float32 outputs go through to
+ * where every die sees them, for another block of the launch to read. */
+template <uint32_t TYPE, uint32_t ROWS, uint32_t OUTPUTS, bool FRONT = false>
 __device__ static __forceinline__ void dense_linear_body(const struct dense_linear_arguments &arguments, unsigned char *arena, const uint16_t *rows,
                                                          uint32_t first_output, uint32_t first_row, uint32_t thread, bool active,
                                                          dense_group_sums<ROWS, OUTPUTS> &lds)
@@ -60,37 +65,66 @@ __device__ static __forceinline__ void dense_linear_body(const struct dense_line
             chain[o][r] = 0.0f;
         }
     }
-#pragma unroll(ROWS == 1u ? 4 : 1)
-    for (uint32_t chunk = thread; chunk < chunks; chunk += DENSE_THREADS_VALUE) {
-        /* every row's chunk is asked for before any is used: a chunk costs one trip to memory, not one a row */
-        uint4_t packed[ROWS];
+    const uint32_t live = FRONT && arguments.row_count - first_row < ROWS ? arguments.row_count - first_row : ROWS;
+    constexpr uint32_t WEIGHT_LOADS = TYPE == DENSE_FLOAT32 ? 2u : 1u;
+    struct chunk_loads {
+        uint4_t rows[ROWS], weights[OUTPUTS][WEIGHT_LOADS];
+    };
+    /* every row's chunk and every output's weights are asked for before any is used: a chunk costs one trip to memory, not one a row */
+    const auto ask = [&](uint32_t chunk, chunk_loads &into) {
 #pragma unroll
         for (uint32_t r = 0; r < ROWS; r++) {
             /* a column from row_count on reads row 0 and is stored nowhere */
             const uint32_t row = first_row + r < arguments.row_count ? first_row + r : 0u;
-            packed[r] = *(const uint4_t *)(rows + (uint64_t)row * inputs + chunk * DENSE_CHUNK_INPUTS);
+            into.rows[r] = *(const uint4_t *)(rows + (uint64_t)row * inputs + chunk * DENSE_CHUNK_INPUTS);
         }
-        /* and every output's weights before the first chain runs */
-        float weights[OUTPUTS][DENSE_CHUNK_INPUTS];
 #pragma unroll
         for (uint32_t o = 0; o < OUTPUTS; o++) {
             const uint64_t at = (uint64_t)(first_output + o) * inputs + chunk * DENSE_CHUNK_INPUTS;
-            if constexpr (TYPE == DENSE_FLOAT32) {
-                const float4_t low = *(const float4_t *)((const float *)(arena + arguments.weights_offset) + at);
-                const float4_t high = *(const float4_t *)((const float *)(arena + arguments.weights_offset) + at + 4u);
 #pragma unroll
-                for (uint32_t i = 0; i < 4u; i++) {
-                    weights[o][i] = low[i];
-                    weights[o][4u + i] = high[i];
+            for (uint32_t part = 0; part < WEIGHT_LOADS; part++) {
+                into.weights[o][part] = *(const uint4_t *)(arena + arguments.weights_offset + (TYPE == DENSE_FLOAT32 ? 4u : 2u) * at + 16u * part);
+            }
+        }
+    };
+    const auto add = [&](const chunk_loads &now) {
+        float weights[OUTPUTS][DENSE_CHUNK_INPUTS];
+#pragma unroll
+        for (uint32_t o = 0; o < OUTPUTS; o++) {
+            if constexpr (TYPE == DENSE_FLOAT32) {
+#pragma unroll
+                for (uint32_t i = 0; i < DENSE_CHUNK_INPUTS; i++) {
+                    weights[o][i] = __uint_as_float(now.weights[o][i / 4u][i % 4u]);
                 }
             } else {
-                unpack_bf16x8(*(const uint4_t *)((const uint16_t *)(arena + arguments.weights_offset) + at), weights[o]);
+                unpack_bf16x8(now.weights[o][0], weights[o]);
             }
+        }
+        if constexpr (FRONT) { /* a row at a time, those that are one */
+#pragma unroll
+            for (uint32_t r = 0; r < ROWS; r++) {
+                if (ROWS > 1u && r >= live) {
+                    break;
+                }
+                float values[DENSE_CHUNK_INPUTS];
+                unpack_bf16x8(now.rows[r], values);
+#pragma unroll
+                for (uint32_t i = 0; i < DENSE_CHUNK_INPUTS; i++) {
+                    if (scaled) {
+                        squares[r] = __fmaf_rn(values[i], values[i], squares[r]);
+                    }
+#pragma unroll
+                    for (uint32_t o = 0; o < OUTPUTS; o++) {
+                        chain[o][r] = __fmaf_rn(weights[o][i], values[i], chain[o][r]);
+                    }
+                }
+            }
+            return;
         }
         float values[ROWS][DENSE_CHUNK_INPUTS];
 #pragma unroll
         for (uint32_t r = 0; r < ROWS; r++) {
-            unpack_bf16x8(packed[r], values[r]);
+            unpack_bf16x8(now.rows[r], values[r]);
         }
         if (scaled) {
 #pragma unroll
@@ -111,15 +145,21 @@ __device__ static __forceinline__ void dense_linear_body(const struct dense_line
                 }
             }
         }
+    };
+#pragma unroll(ROWS == 1u ? 4 : 1)
+    for (uint32_t chunk = thread; chunk < chunks; chunk += DENSE_THREADS_VALUE) {
+        chunk_loads now;
+        ask(chunk, now);
+        add(now);
     }
     const uint32_t group = thread / DENSE_GROUP_LANES, lane = thread % DENSE_GROUP_LANES;
     /* each chain's additions are the definition's: the distance halving from 16. By the lanes' own exchanges: a thread of 8 rows
      * has up to 72 sums of five distances each (2000 rows of 16384 inputs by 24 outputs, against shuffles: 57 -> 51.5 us) */
-    dense_add_lanes<16u>(chain, squares, scaled);
-    dense_add_lanes<8u>(chain, squares, scaled);
-    dense_add_lanes<4u>(chain, squares, scaled);
-    dense_add_lanes<2u>(chain, squares, scaled);
-    dense_add_lanes<1u>(chain, squares, scaled);
+    dense_add_lanes<16u>(chain, squares, scaled, live);
+    dense_add_lanes<8u>(chain, squares, scaled, live);
+    dense_add_lanes<4u>(chain, squares, scaled, live);
+    dense_add_lanes<2u>(chain, squares, scaled, live);
+    dense_add_lanes<1u>(chain, squares, scaled, live);
     if (lane == 0u && active) {
 #pragma unroll
         for (uint32_t r = 0; r < ROWS; r++) {
@@ -150,7 +190,10 @@ __device__ static __forceinline__ void dense_linear_body(const struct dense_line
         sum = __fmul_rn(sum, dense_reciprocal_root(operand));
     }
     const uint64_t index = (uint64_t)(first_row + r) * arguments.output_size + first_output + o;
-    if (arguments.output_type == DENSE_FLOAT32) {
+    if constexpr (FRONT) { /* a float32 that another block of this launch reads: through to where every die sees it */
+        __hip_atomic_store((float *)(arena + arguments.output_offset) + index, __fmul_rn(sum, arguments.output_scale), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    } else if (arguments.output_type == DENSE_FLOAT32) {
         ((float *)(arena + arguments.output_offset))[index] = __fmul_rn(sum, arguments.output_scale);
     } else {
         ((uint16_t *)(arena + arguments.output_offset))[index] = float_to_bf16(__fmul_rn(bf16_to_float(float_to_bf16(sum)), arguments.output_scale));

@@ -37,7 +37,9 @@ __device__ static __forceinline__ float hyper_divide(float value, bool rows, flo
 }
 
 /* The sublayer's input of row `row` (the collapse of its streams by the carried pre, and its norm) by the `row_threads` =
- * width / 8 threads `thread` 0 .. of a block (every one of them calls: barriers inside); group_sums: 32 floats of LDS. */
+ * width / 8 threads `thread` 0 .. of a block (every one of them calls: barriers inside); group_sums: 32 floats of LDS. THROUGH:
+ * the row is stored through to where every die sees it, for readers in other blocks of the launch. */
+template <bool THROUGH = false>
 __device__ static __forceinline__ void hyper_row_input_body(const struct hyper_finish_arguments &arguments, unsigned char *arena, uint64_t row,
                                                              uint32_t thread, uint64_t row_threads, float *group_sums)
 {
@@ -88,7 +90,17 @@ __device__ static __forceinline__ void hyper_row_input_body(const struct hyper_f
     for (uint32_t v = 0; v < HYPER_VALUES_PER_THREAD; v++) {
         hidden[v] = __fmul_rn(weights[v], __fmul_rn(hidden[v], factor));
     }
-    ((uint4_t *)(arena + arguments.hidden_offset))[row * row_threads + thread] = join_pack<HYPER_VALUES_PER_THREAD>(hidden);
+    uint4_t *out = (uint4_t *)(arena + arguments.hidden_offset) + row * row_threads + thread;
+    const uint4_t packed = join_pack<HYPER_VALUES_PER_THREAD>(hidden);
+    if constexpr (THROUGH) {
+#pragma unroll
+        for (uint32_t half = 0; half < 2u; half++) {
+            const uint64_t words = (uint64_t)packed[2u * half + 1u] << 32 | packed[2u * half];
+            __hip_atomic_store((uint64_t *)out + half, words, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    } else {
+        *out = packed;
+    }
 }
 
 /* Row `row`'s post, comb and pre from its mixes, by sixteen threads `thread` 0 .. 15 that are sixteen lanes in a row of one

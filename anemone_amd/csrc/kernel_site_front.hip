@@ -24,8 +24,13 @@
  *
  * What a front costs is its two serial chains, so what nobody in it waits for stands behind what somebody does: a row is
  * published before it is quantized, the scores' blocks ask for a word of every line of their weights before they wait for
- * the rows, and the dense product's sums meet by the lanes' own exchanges (ffn_front_8 at 5 rows of 4096 by 256 experts 23.7
- * -> 22.0 us, ffn_front_1 15.7 -> 13.8; asking for the mixes' weights ahead likewise: 1 us longer at 1 and 5 rows).
+ * the rows, a block is counted out ahead of its quantization, coefficients or select, and the dense product's sums meet by the
+ * lanes' own exchanges (ffn_front_8 at 5 rows of 4096 by 256 experts 23.7 -> 22.0 us, ffn_front_1 15.7 -> 13.8; asking for the
+ * mixes' weights ahead likewise: 1 us longer at 1 and 5 rows; a chunk of the dense products on its way while one is added: none).
+ * Leaving early, stores that need no write-back and the eight rows' form without the rows that are not there: at 5 rows 16.3 -> 14.25,
+ * at 2 of 2048 by 384 experts 15.7 -> 13.6, at 8 of 5120 by 384 21.0 -> 19.45, ffn_front_1 10.9 -> 10.5. At 5 rows each of the two
+ * chains by itself takes the launch's time: the tickets, waits and row's input alone are 8.7 us of it, the scores 3.5 and the select
+ * 3; the mixes 7 and the coefficients 3.
  *
  * The two halves need no tickets and no waits: the input front is a row a block (grid rows); the coefficient front is the
  * mix project's blocks (grid site_front_mix_blocks), the last of which to publish arrived forms post, comb and pre and
@@ -45,21 +50,21 @@ __device__ static __forceinline__ uint32_t front_add(uint32_t *counter)
     return __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-/* Every thread of the block calls; the old value of the counter, on every thread. RELEASE: what the block's threads stored
- * is visible at agent scope before the counter moves (every thread's stores are through to the block's level 2 cache
- * before the block meets; thread 0 then writes that cache's lines back once for all). ACQUIRE: what the earlier
- * publishers stored is visible to the block's threads behind the call (thread 0 drops the stale lines once for all). */
+/* Every thread of the block calls; the old value of the counter, on every thread. RELEASE: what the block's threads stored by
+ * relaxed stores of agent scope, which go through the level 2 cache of their die, is there before the counter moves (every
+ * thread waits for its own, then the block meets). What other blocks read is a row, a few mixes or scores: written back with
+ * all else that the die's cache holds, by a release of agent scope, each of a front's two publications in line took 0.7 us
+ * (ffn_front_8 at five rows 15.5 -> 14.1). ACQUIRE: what the earlier publishers stored is visible to the block's threads
+ * behind the call (thread 0 drops the stale lines once for all). */
 template <bool RELEASE, bool ACQUIRE>
 __device__ static __forceinline__ uint32_t front_publish(uint32_t *counter, uint32_t thread, uint32_t *word)
 {
     if (RELEASE) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     }
     __syncthreads();
     if (thread == 0u) {
-        if (RELEASE) {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        }
         *word = front_add(counter);
         if (ACQUIRE) {
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -133,7 +138,7 @@ __device__ static __forceinline__ void front_mix_project(const struct site_front
     dense.epsilon = MODEL_NORM_EPSILON;
     constexpr uint32_t groups = MODEL_MIXES / SITE_FRONT_MIX_OUTPUTS;
     const uint32_t group = block * quarters + quarter;
-    dense_linear_body<DENSE_FLOAT32, ROWS, SITE_FRONT_MIX_OUTPUTS>(dense, arena, (const uint16_t *)(arena + dense.rows_offset),
+    dense_linear_body<DENSE_FLOAT32, ROWS, SITE_FRONT_MIX_OUTPUTS, true>(dense, arena, (const uint16_t *)(arena + dense.rows_offset),
                                                                    group * SITE_FRONT_MIX_OUTPUTS, 0u, thread % DENSE_THREADS_VALUE,
                                                                    in_quarter && group < groups, sums[in_quarter ? quarter : 0u]);
 }
@@ -166,19 +171,26 @@ __device__ static __forceinline__ void site_front(const struct site_front_argume
     }
     __syncthreads();
     const uint32_t ticket = word;
+    /* a block is counted out behind its last use of the counters, ahead of what it does after that: only thread 0 uses them, and
+     * it looks at what the counter said at the very end */
+    uint32_t left = 0u;
+    const auto leave = [&]() { return thread == 0u ? front_add(&scratch->departed) : 0u; };
     const struct hyper_finish_arguments finish = {arguments.streams_offset, arguments.pre_offset, mixes_offset, arguments.scale_offset,
                                                   arguments.base_offset, arguments.post_offset, arguments.comb_offset,
                                                   arguments.norm_weight_offset, arguments.hidden_offset};
     if (ticket < rows) {
         /* a row: its input, which the blocks of the scores wait for, then its quantization, which no block of this launch does */
-        hyper_row_input_body(finish, arena, ticket, thread, threads, lds.group_sums);
+        hyper_row_input_body<true>(finish, arena, ticket, thread, threads, lds.group_sums);
         front_publish<true, false>(&scratch->rows_ready, thread, &word);
+        left = leave();
         front_row_quantize(arguments, arena, ticket, thread, threads);
     } else if (ticket < rows + mix_blocks) {
         /* the mix project: float32 [24][4 width] by the streams as rows of 4 width values, with the row's scale */
         front_mix_project<ROWS>(arguments, arena, rows, ticket - rows, thread, threads, lds.mixes);
-        if (front_publish<true, true>(&scratch->arrived, thread, &word) == mix_blocks - 1u &&
-            front_wait<false>(&scratch->rows_ready, rows, thread, &word, &scratch->gave_up)) {
+        const bool complete = front_publish<true, true>(&scratch->arrived, thread, &word) == mix_blocks - 1u &&
+                              front_wait<false>(&scratch->rows_ready, rows, thread, &word, &scratch->gave_up);
+        left = leave();
+        if (complete) {
             /* every mix is stored and every row's block has read the carried pre */
             if (thread < rows * MODEL_STREAMS * MODEL_STREAMS) {
                 hyper_coefficients_body(finish, arena, thread / (MODEL_STREAMS * MODEL_STREAMS), thread % (MODEL_STREAMS * MODEL_STREAMS));
@@ -219,17 +231,22 @@ __device__ static __forceinline__ void site_front(const struct site_front_argume
                 asm volatile("" ::"v"(touched));
             }
         }
+        bool last = false;
         if (front_wait<true>(&scratch->rows_ready, rows, thread, &word, &scratch->gave_up)) {
-            dense_linear_body<DENSE_BFLOAT16, ROWS, SITE_FRONT_SCORE_OUTPUTS>(dense, arena, (const uint16_t *)(arena + dense.rows_offset),
+            dense_linear_body<DENSE_BFLOAT16, ROWS, SITE_FRONT_SCORE_OUTPUTS, true>(dense, arena, (const uint16_t *)(arena + dense.rows_offset),
                                                                               group * SITE_FRONT_SCORE_OUTPUTS, 0u, quarter_thread,
                                                                               in_quarter && group < groups, lds.scores[slot]);
-            if (front_publish<true, true>(&scratch->scored, thread, &word) == score_blocks - 1u) {
-                router_select_body(select, arena, thread, threads, lds.select);
-            }
+            last = front_publish<true, true>(&scratch->scored, thread, &word) == score_blocks - 1u;
         }
+        left = leave();
+        if (last) {
+            router_select_body(select, arena, thread, threads, lds.select);
+        }
+    } else { /* a ticket past the parts, of a counter that did not start at zero */
+        left = leave();
     }
     /* the last block to leave clears the counters: no block reads them any more */
-    if (front_publish<false, false>(&scratch->departed, thread, &word) == gridDim.x - 1u && thread == 0u) {
+    if (thread == 0u && left == gridDim.x - 1u) {
         scratch->tickets = 0u;
         scratch->arrived = 0u;
         scratch->rows_ready = 0u;
