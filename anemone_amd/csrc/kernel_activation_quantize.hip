@@ -18,7 +18,7 @@
 extern "C" __global__ void __launch_bounds__(LINEAR_ELEMENT_THREADS)
     activation_quantize_entry(struct activation_quantize_arguments arguments, unsigned char *arena)
 {
-    activation_quantize_body(arguments, arena, blockIdx.x * blockDim.x + threadIdx.x, blockIdx.y);
+    activation_quantize_body(arguments, arena, blockIdx.x * LINEAR_ELEMENT_THREADS + threadIdx.x, blockIdx.y);
 }
 ANEMONE_KERNEL(KERNEL_FILE_ACTIVATION_QUANTIZE, activation_quantize_entry, activation_quantize_arguments);
 
@@ -33,7 +33,7 @@ extern "C" __global__ void __launch_bounds__(LINEAR_ELEMENT_THREADS)
 {
     /* the threads' values as in activation_quantize_entry: thread q = 16 l + 4 s + t takes 64 l + 16 s + 2 t + {0, 1, 8, 9},
      * one word of codes; the 128 values of a scale are those of 32 neighbouring threads */
-    const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t q = blockIdx.x * LINEAR_ELEMENT_THREADS + threadIdx.x;
     const uint32_t l = q / 16u, s = (q / 4u) % 4u, t = q % 4u, first = 64u * l + 16u * s + 2u * t;
     if (first >= arguments.width) {
         return; /* the width is a multiple of 128: whole groups of 32 threads leave together */

@@ -38,10 +38,11 @@ __device__ static __forceinline__ void dense_linear(const struct dense_linear_ar
     __shared__ dense_group_sums<ROWS, OUTPUTS> lds;
     uint32_t output_group = blockIdx.x, row_group = blockIdx.y;
     if constexpr (ROWS != 1u) {
-        if (gridDim.y % DENSE_DIES == 0u) {
-            const uint32_t linear = blockIdx.x + gridDim.x * blockIdx.y, place = linear / DENSE_DIES;
-            output_group = place % gridDim.x;
-            row_group = place / gridDim.x * DENSE_DIES + linear % DENSE_DIES;
+        const uint32_t output_groups = arguments.output_size / OUTPUTS, row_groups = (arguments.row_count + ROWS - 1u) / ROWS; /* the grid's */
+        if (row_groups % DENSE_DIES == 0u) {
+            const uint32_t linear = blockIdx.x + output_groups * blockIdx.y, place = linear / DENSE_DIES;
+            output_group = place % output_groups;
+            row_group = place / output_groups * DENSE_DIES + linear % DENSE_DIES;
         }
     }
     dense_linear_body<TYPE, ROWS, OUTPUTS>(arguments, arena, (const uint16_t *)(arena + arguments.rows_offset), output_group * OUTPUTS,

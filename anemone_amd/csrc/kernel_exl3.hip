@@ -18,7 +18,7 @@
 
 extern "C" __global__ void exl3_reconstruct(struct exl3_reconstruct_record record, unsigned char *arena)
 {
-    const uint64_t element = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t element = (uint64_t)blockIdx.x * LINEAR_ELEMENT_THREADS + threadIdx.x;
     if (element >= (uint64_t)record.input_size * record.output_size) {
         return;
     }
@@ -67,7 +67,7 @@ extern "C" __global__ void __launch_bounds__(EXL3_ELEMENT_MOST_THREADS) exl3_inp
     const float s0 = half_bits_to_float(suh[channel]), s1 = half_bits_to_float(suh[channel + WAVE]);
     const uint16_t *input = (const uint16_t *)(arena + record.input_offset);
     uint16_t *operands = (uint16_t *)(arena + record.operands_offset);
-    for (uint32_t column = threadIdx.x / WAVE; column < job->row_count; column += blockDim.x / WAVE) {
+    for (uint32_t column = threadIdx.x / WAVE; column < job->row_count; column += exl3_element_rows(record.pair_count, record.job_count)) {
         const uint32_t pair = job->pair_index[column];
         const uint64_t row = pair / record.pairs_per_row;
         float v0 = __fmul_rn(bf16_to_float(input[row * record.input_size + channel]), s0);
@@ -213,7 +213,7 @@ extern "C" __global__ void __launch_bounds__(EXL3_ELEMENT_MOST_THREADS) exl3_act
     const float ds0 = half_bits_to_float(down_suh[between]), ds1 = half_bits_to_float(down_suh[between + WAVE]);
     const float limit = record.activation_limit;
     const float *products = (const float *)(arena + record.products_offset);
-    for (uint32_t column = threadIdx.x / WAVE; column < job->row_count; column += blockDim.x / WAVE) {
+    for (uint32_t column = threadIdx.x / WAVE; column < job->row_count; column += exl3_element_rows(record.pair_count, record.job_count)) {
         const uint32_t pair = job->pair_index[column];
         float g0 = products[(uint64_t)pair * I + channel], g1 = products[(uint64_t)pair * I + channel + WAVE];
         float u0 = products[((uint64_t)record.pair_count + pair) * I + channel];
@@ -254,7 +254,7 @@ extern "C" __global__ void __launch_bounds__(EXL3_ELEMENT_MOST_THREADS) exl3_fin
     const uint16_t *svh = (const uint16_t *)(arena + job->down_offset +
                                              exl3_code_bytes(I, H, exl3_bits_x2(chain_width(record, arena, job->expert, 2u)))) + I;
     const float s0 = half_bits_to_float(svh[to]), s1 = half_bits_to_float(svh[to + WAVE]);
-    for (uint32_t column = threadIdx.x / WAVE; column < job->row_count; column += blockDim.x / WAVE) {
+    for (uint32_t column = threadIdx.x / WAVE; column < job->row_count; column += exl3_element_rows(record.pair_count, record.job_count)) {
         const uint32_t pair = job->pair_index[column];
         float *values = (float *)(arena + record.products_offset) + (uint64_t)pair * H;
         float v0 = values[channel], v1 = values[channel + WAVE];
@@ -269,7 +269,7 @@ ANEMONE_KERNEL(EXL3_KERNEL_FILE, exl3_finish, exl3_expert_record);
 
 extern "C" __global__ void exl3_row_sum(struct expert_row_sum_arguments record, unsigned char *arena)
 {
-    const uint32_t channel = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t channel = blockIdx.x * LINEAR_ELEMENT_THREADS + threadIdx.x;
     if (channel >= record.width) {
         return;
     }

@@ -75,7 +75,7 @@ extern "C" __global__ void __launch_bounds__(TCP_SORT_THREADS) exl3_tcp_count(st
     __shared__ uint32_t histogram[ROUTER_MOST_EXPERTS];
     sort_count_picks(block_experts, pairs, shape.experts, histogram);
     uint32_t *counts = (uint32_t *)(arena + record.workspace_offset + shape.layout.counts) + (uint64_t)blockIdx.x * shape.experts;
-    for (uint32_t expert = threadIdx.x; expert < shape.experts; expert += blockDim.x) {
+    for (uint32_t expert = threadIdx.x; expert < shape.experts; expert += TCP_SORT_THREADS) {
         counts[expert] = histogram[expert];
     }
 }
@@ -97,7 +97,7 @@ extern "C" __global__ void __launch_bounds__(TCP_SORT_THREADS) exl3_tcp_place(st
     const uint32_t pairs = sort_block_picks((const struct router_pick *)(arena + record.picks_offset), shape.picks, blockIdx.x,
                                             record.row_count, block_experts);
     const uint32_t *counts = (const uint32_t *)(workspace + shape.layout.counts);
-    for (uint32_t expert = threadIdx.x; expert < experts; expert += blockDim.x) {
+    for (uint32_t expert = threadIdx.x; expert < experts; expert += TCP_SORT_THREADS) {
         uint32_t total = 0, lower = 0;
 #pragma unroll 8
         for (uint32_t block = 0; block < blocks; block++) {
@@ -115,12 +115,12 @@ extern "C" __global__ void __launch_bounds__(TCP_SORT_THREADS) exl3_tcp_place(st
     uint32_t *sorted = (uint32_t *)(workspace + shape.layout.sorted), *place_of = (uint32_t *)(workspace + shape.layout.place_of);
     const uint32_t first_pair = blockIdx.x * ROUTER_SORT_ROWS * shape.picks;
     /* every pick's place into LDS; the two tables are written behind it, a thread a pick */
-    for (uint32_t expert = threadIdx.x; expert < experts; expert += blockDim.x) {
+    for (uint32_t expert = threadIdx.x; expert < experts; expert += TCP_SORT_THREADS) {
         first_places[expert] = starts[expert] + before[expert];
     }
     __syncthreads();
     sort_place_picks(block_experts, pairs, experts, first_places, cursors, block_places);
-    for (uint32_t index = threadIdx.x; index < pairs; index += blockDim.x) {
+    for (uint32_t index = threadIdx.x; index < pairs; index += TCP_SORT_THREADS) {
         const uint32_t place = block_places[index];
         sorted[place] = first_pair + index;
         place_of[first_pair + index] = place;
@@ -129,7 +129,7 @@ extern "C" __global__ void __launch_bounds__(TCP_SORT_THREADS) exl3_tcp_place(st
         return;
     }
     struct wide_run *runs = (struct wide_run *)(workspace + shape.layout.runs);
-    for (uint32_t expert = threadIdx.x; expert < experts; expert += blockDim.x) {
+    for (uint32_t expert = threadIdx.x; expert < experts; expert += TCP_SORT_THREADS) {
         runs[expert] = (struct wide_run){starts[expert], totals[expert]};
     }
     const uint32_t used = block_exclusive_scan(chunk_starts, experts, scratch);
@@ -141,7 +141,7 @@ extern "C" __global__ void __launch_bounds__(TCP_SORT_THREADS) exl3_tcp_place(st
     }
     __syncthreads();
     struct exl3_tcp_chunk *chunks = (struct exl3_tcp_chunk *)(workspace + shape.layout.chunks);
-    for (uint32_t chunk = threadIdx.x; chunk < shape.layout.chunk_capacity; chunk += blockDim.x) {
+    for (uint32_t chunk = threadIdx.x; chunk < shape.layout.chunk_capacity; chunk += TCP_SORT_THREADS) {
         struct exl3_tcp_chunk value = {0, 0, 0, 0};
         if (chunk < used) {
             uint32_t low = 0, high = experts; /* the expert whose chunks hold this one */
@@ -507,19 +507,20 @@ extern "C" __global__ void __launch_bounds__(TCP_GEMM_THREADS, 2) exl3_tcp_gemm(
      * chunk's operand columns: the blocks of eight consecutive rows m = y + gy z of the grid are re-assigned so that those
      * a die holds among them are all the strips of one (chunk, projection), which then come from memory into that die's
      * level-2 cache once (a grid whose x is no multiple of eight, and the rows past the last whole eight, stay as dealt). */
-    uint32_t strip = blockIdx.x, place = blockIdx.y + gridDim.y * blockIdx.z;
-    const uint32_t places = gridDim.y * gridDim.z;
-    if (gridDim.x % TCP_DIES == 0u && place < places / TCP_DIES * TCP_DIES) {
-        strip = (place % TCP_DIES) * (gridDim.x / TCP_DIES) + blockIdx.x / TCP_DIES;
+    const bool down = record.pass == EXL3_TCP_DOWN;
+    const uint32_t strips = ((down ? shape.hidden : shape.intermediate) + EXL3_TCP_BLOCK_OUTPUTS - 1u) / EXL3_TCP_BLOCK_OUTPUTS; /* the grid's */
+    const uint32_t capacity = shape.layout.chunk_capacity, places = capacity * (down ? 1u : 2u);
+    uint32_t strip = blockIdx.x, place = blockIdx.y + capacity * blockIdx.z;
+    if (strips % TCP_DIES == 0u && place < places / TCP_DIES * TCP_DIES) {
+        strip = (place % TCP_DIES) * (strips / TCP_DIES) + blockIdx.x / TCP_DIES;
         place = place / TCP_DIES * TCP_DIES + blockIdx.x % TCP_DIES;
     }
-    const struct exl3_tcp_chunk chunk = tcp_chunk_of(shape, workspace, place % gridDim.y);
+    const struct exl3_tcp_chunk chunk = tcp_chunk_of(shape, workspace, place % capacity);
     if (chunk.pair_count == 0u) {
         return;
     }
     const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const bool down = record.pass == EXL3_TCP_DOWN;
-    const uint32_t projection = down ? 2u : place / gridDim.y;
+    const uint32_t projection = down ? 2u : place / capacity;
     const uint32_t inputs = down ? shape.intermediate : shape.hidden, outputs = down ? shape.hidden : shape.intermediate;
     const uint32_t bits_x2 = tcp_bits_x2(record, arena, chunk.expert, projection);
     const uint32_t *codes = (const uint32_t *)(arena + tcp_matrix_of(record, arena, chunk.expert, projection));

@@ -393,7 +393,7 @@ EXPERT_ENTRIES(8);
  * again (width 4096, 8 slots: 8192 rows 121 -> 97 us, 112 of them without the stream; 2048 rows 27.9 -> 25.3, 64 rows 5.8 -> 4.7) */
 extern "C" __global__ void expert_row_sum_entry(struct expert_row_sum_arguments arguments, unsigned char *arena)
 {
-    const uint32_t channel = (blockIdx.x * blockDim.x + threadIdx.x) * EXPERT_ROW_SUM_CHANNELS;
+    const uint32_t channel = (blockIdx.x * LINEAR_ELEMENT_THREADS + threadIdx.x) * EXPERT_ROW_SUM_CHANNELS;
     if (channel >= arguments.width) {
         return;
     }

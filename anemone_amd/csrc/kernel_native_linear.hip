@@ -69,7 +69,8 @@ __device__ static __forceinline__ void native_expert_gate_up(const struct wide_e
     struct wide_expert_tile tile;
     uint32_t pair_count = 0, block_strip = 0;
     bool alone = false;
-    if (!order_block_of<GROUP, false, !BYTES || chain_type::TILES == 4u>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count, &alone)) {
+    const uint32_t strips = (arguments.output_size + NATIVE_WAVES * STRIP * 16u - 1u) / (NATIVE_WAVES * STRIP * 16u);
+    if (!order_block_of<GROUP, false, !BYTES || chain_type::TILES == 4u>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, strips, lane, block_strip, tile, pair_count, &alone)) {
         return;
     }
     const struct wide_pair *pairs = (const struct wide_pair *)(arena + arguments.pairs_offset) + tile.first_pair;
@@ -106,7 +107,8 @@ __device__ static __forceinline__ void native_expert_down(const struct wide_expe
     struct wide_expert_tile tile;
     uint32_t pair_count = 0, block_strip = 0;
     bool alone = false;
-    if (!order_block_of<GROUP, true, BY_RUN>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count, &alone)) {
+    const uint32_t strips = (arguments.output_size + NATIVE_WAVES * DOWN_STRIP * 16u - 1u) / (NATIVE_WAVES * DOWN_STRIP * 16u);
+    if (!order_block_of<GROUP, true, BY_RUN>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, strips, lane, block_strip, tile, pair_count, &alone)) {
         return;
     }
     const struct wide_pair *pairs = (const struct wide_pair *)(arena + arguments.pairs_offset) + tile.first_pair;

@@ -239,7 +239,7 @@ __device__ static __forceinline__ void router_projection_thin(const struct route
 extern "C" __global__ void __launch_bounds__(PROJECTION_THIN_THREADS)
     router_projection(struct router_projection_arguments arguments, unsigned char *arena)
 {
-    if (blockDim.x == PROJECTION_THIN_THREADS) { /* the same in every block: a row a block */
+    if (router_projection_by_row(arguments.row_count, arguments.expert_count)) { /* the same in every block */
         router_projection_thin(arguments, arena);
     } else {
         router_projection_block(arguments, arena);
@@ -526,7 +526,7 @@ extern "C" __global__ void __launch_bounds__(SELECT_THREADS)
     router_select_entry(struct router_select_arguments arguments, unsigned char *arena)
 {
     __shared__ struct router_select_lds lds;
-    router_select_body(arguments, arena, threadIdx.x, blockDim.x, lds);
+    router_select_body(arguments, arena, threadIdx.x, SELECT_THREADS, lds);
 }
 ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_select_entry, router_select_arguments);
 
@@ -634,7 +634,7 @@ extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
     __shared__ uint32_t histogram[ROUTER_MOST_EXPERTS];
     sort_count_picks(block_experts, pairs, arguments.expert_count, histogram);
     uint32_t *counts = (uint32_t *)(arena + arguments.counts_offset) + (uint64_t)blockIdx.x * arguments.expert_count;
-    for (uint32_t expert = threadIdx.x; expert < arguments.expert_count; expert += blockDim.x) {
+    for (uint32_t expert = threadIdx.x; expert < arguments.expert_count; expert += WIDE_SORT_THREADS) {
         counts[expert] = histogram[expert];
     }
 }
@@ -655,19 +655,19 @@ __device__ static __forceinline__ void wide_place_block(const struct router_wide
     struct wide_pair *sorted = (struct wide_pair *)(arena + arguments.pairs_offset);
     const uint32_t first_pair = block * ROUTER_SORT_ROWS * picks;
     /* every pick's place into LDS; the pairs are written behind it, a thread a pick */
-    for (uint32_t expert = threadIdx.x; expert < experts; expert += blockDim.x) {
+    for (uint32_t expert = threadIdx.x; expert < experts; expert += WIDE_SORT_THREADS) {
         first_places[expert] = starts[expert] + before[expert];
     }
     __syncthreads();
     sort_place_picks(block_experts, pairs, experts, first_places, cursors, place_of);
-    for (uint32_t index = threadIdx.x; index < pairs; index += blockDim.x) {
+    for (uint32_t index = threadIdx.x; index < pairs; index += WIDE_SORT_THREADS) {
         sorted[place_of[index]] = (struct wide_pair){first_pair + index, all_picks[first_pair + index].route_weight};
     }
     if (block != 0u) {
         return;
     }
     struct wide_run *runs = (struct wide_run *)(arena + arguments.runs_offset);
-    for (uint32_t expert = threadIdx.x; expert < experts; expert += blockDim.x) {
+    for (uint32_t expert = threadIdx.x; expert < experts; expert += WIDE_SORT_THREADS) {
         runs[expert] = (struct wide_run){starts[expert], totals[expert]};
     }
     const uint32_t used_tiles = block_exclusive_scan(tile_starts, experts, scratch);
@@ -678,7 +678,7 @@ __device__ static __forceinline__ void wide_place_block(const struct router_wide
     const uint32_t all_tiles = ROUTER_WIDE_TILES_OF(arguments.row_count, picks, experts);
     struct wide_expert_tile *tiles = (struct wide_expert_tile *)(arena + arguments.tiles_offset);
     const uint64_t *offsets = (const uint64_t *)(arena + arguments.expert_offsets_offset);
-    for (uint32_t tile = threadIdx.x; tile < all_tiles; tile += blockDim.x) {
+    for (uint32_t tile = threadIdx.x; tile < all_tiles; tile += WIDE_SORT_THREADS) {
         struct wide_expert_tile value = {0, 0, 0, 0, 0};
         if (tile < used_tiles) {
             uint32_t low = 0, high = experts; /* the expert whose tiles hold this one: tile_starts[e] <= tile < [e + 1] */
@@ -718,7 +718,7 @@ extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
         return;
     }
     const uint32_t *counts = (const uint32_t *)(arena + arguments.counts_offset);
-    for (uint32_t expert = threadIdx.x; expert < experts; expert += blockDim.x) {
+    for (uint32_t expert = threadIdx.x; expert < experts; expert += WIDE_SORT_THREADS) {
         uint32_t total = 0, lower = 0;
 #pragma unroll 8
         for (uint32_t block = 0; block < live_blocks; block++) {
@@ -775,7 +775,7 @@ extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
     const struct wide_pair *sorted = (const struct wide_pair *)(arena + arguments.pairs_offset);
     const uint64_t *offsets = (const uint64_t *)(arena + arguments.expert_offsets_offset);
     struct expert_job_record *jobs = (struct expert_job_record *)(arena + arguments.jobs_offset);
-    for (uint32_t job = threadIdx.x; job < all_jobs; job += blockDim.x) {
+    for (uint32_t job = threadIdx.x; job < all_jobs; job += WIDE_SORT_THREADS) {
         struct expert_job_record value = {};
         if (job < used_jobs) {
             uint32_t low = 0, high = experts;

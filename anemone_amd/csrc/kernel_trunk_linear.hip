@@ -151,7 +151,7 @@ __device__ static __forceinline__ void trunk_linear_quantized_interleaved(const 
     const uint32_t scale_column = 16u * wave + lane / 4u;
     const uint32_t exponent_vector = first_row + (scale_column < row_count ? scale_column : 0u);
     chain_type chain_of;
-    chain_of.once = gridDim.y == 1u;
+    chain_of.once = arguments.row_count <= TRUNK_INTERLEAVED_ROWS;
     const unsigned char *const matrices[1] = {arena + arguments.weights_offset[matrix]};
     uint32_t tile0 = 0;
     chain_of.place(matrices, outputs, arguments.input_size, block, arena + arguments.codes_offset, arena + arguments.exponents_offset,
@@ -260,7 +260,7 @@ ANEMONE_KERNEL(KERNEL_FILE_TRUNK_LINEAR, trunk_linear_quantized_interleaved_1, t
  * eight, else one value at a time */
 extern "C" __global__ void trunk_hidden_entry(struct trunk_hidden_arguments arguments, unsigned char *arena)
 {
-    const uint32_t first = (blockIdx.x * blockDim.x + threadIdx.x) * HYPER_VALUES_PER_THREAD;
+    const uint32_t first = (blockIdx.x * LINEAR_ELEMENT_THREADS + threadIdx.x) * HYPER_VALUES_PER_THREAD;
     if (first >= arguments.width) {
         return;
     }

@@ -48,7 +48,8 @@ __device__ static __forceinline__ void wide_expert_gate_up(const struct wide_exp
     struct wide_expert_tile tile;
     uint32_t pair_count = 0, block_strip = 0;
     bool alone = false;
-    if (!order_block_of<1u, false, !BYTES>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count, &alone)) {
+    const uint32_t strips = (arguments.output_size + WIDE_WAVES * STRIP_OUTPUTS - 1u) / (WIDE_WAVES * STRIP_OUTPUTS);
+    if (!order_block_of<1u, false, !BYTES>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, strips, lane, block_strip, tile, pair_count, &alone)) {
         return;
     }
     const struct wide_pair *pairs = (const struct wide_pair *)(arena + arguments.pairs_offset) + tile.first_pair;
@@ -100,7 +101,9 @@ __device__ static __forceinline__ void wide_expert_down(const struct wide_expert
     struct wide_expert_tile tile;
     uint32_t pair_count = 0, block_strip = 0;
     bool alone = false;
-    if (!order_block_of<1u, true, !BYTES>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, lane, block_strip, tile, pair_count, &alone)) {
+    constexpr uint32_t BLOCK_OUTPUTS = WIDE_WAVES * chain_type::STRIP * 16u;
+    const uint32_t strips = (arguments.output_size + BLOCK_OUTPUTS - 1u) / BLOCK_OUTPUTS;
+    if (!order_block_of<1u, true, !BYTES>((const struct wide_expert_tile *)(arena + arguments.tiles_offset), arguments.tile_count, strips, lane, block_strip, tile, pair_count, &alone)) {
         return;
     }
     const struct wide_pair *pairs = (const struct wide_pair *)(arena + arguments.pairs_offset) + tile.first_pair;

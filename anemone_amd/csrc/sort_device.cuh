@@ -12,6 +12,9 @@
 
 #include "anemone_records.h"
 
+#define SORT_WAVE 64u
+#define SORT_MOST_WAVES 8u /* of a block of the sorts: 512 threads */
+
 /* the picked experts of the live rows of block `block` of ROUTER_SORT_ROWS rows, into LDS; returns their number */
 __device__ static __forceinline__ uint32_t sort_block_picks(const struct router_pick *all_picks, uint32_t picks_per_row,
                                                             uint32_t block, uint32_t live_rows, uint32_t *experts_out)
@@ -19,24 +22,21 @@ __device__ static __forceinline__ uint32_t sort_block_picks(const struct router_
     const uint32_t first_row = block * ROUTER_SORT_ROWS;
     const uint32_t rows = live_rows <= first_row ? 0u : live_rows - first_row < ROUTER_SORT_ROWS ? live_rows - first_row : ROUTER_SORT_ROWS;
     const struct router_pick *picks = all_picks + (uint64_t)first_row * picks_per_row;
-    for (uint32_t index = threadIdx.x; index < rows * picks_per_row; index += blockDim.x) {
+    for (uint32_t index = threadIdx.x; index < rows * picks_per_row; index += SORT_MOST_WAVES * SORT_WAVE) {
         experts_out[index] = picks[index].expert;
     }
     return rows * picks_per_row;
 }
 
-#define SORT_WAVE 64u
-#define SORT_MOST_WAVES 8u /* of a block of the sorts: 512 threads */
-
 /* The block's picks of every expert: histogram[expert] in LDS. Integer additions in LDS: the same sums whatever their
  * order. The whole block calls it (barriers inside); block_experts is complete before the call. */
 __device__ static __forceinline__ void sort_count_picks(const uint32_t *block_experts, uint32_t pairs, uint32_t experts, uint32_t *histogram)
 {
-    for (uint32_t expert = threadIdx.x; expert < experts; expert += blockDim.x) {
+    for (uint32_t expert = threadIdx.x; expert < experts; expert += SORT_MOST_WAVES * SORT_WAVE) {
         histogram[expert] = 0u;
     }
     __syncthreads();
-    for (uint32_t index = threadIdx.x; index < pairs; index += blockDim.x) {
+    for (uint32_t index = threadIdx.x; index < pairs; index += SORT_MOST_WAVES * SORT_WAVE) {
         __hip_atomic_fetch_add(&histogram[block_experts[index]], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     __syncthreads();
@@ -135,13 +135,13 @@ __device__ static __forceinline__ void sort_place_picks(const uint32_t *block_ex
     const uint32_t wave = threadIdx.x / SORT_WAVE;
     uint32_t begin, end;
     sort_share(pairs, wave, begin, end);
-    for (uint32_t at = threadIdx.x; at < SORT_MOST_WAVES * experts; at += blockDim.x) {
+    for (uint32_t at = threadIdx.x; at < SORT_MOST_WAVES * experts; at += SORT_MOST_WAVES * SORT_WAVE) {
         cursors[at] = 0u;
     }
     __syncthreads();
     sort_count_share(block_experts, begin, end, cursors + wave * experts);
     __syncthreads();
-    for (uint32_t expert = threadIdx.x; expert < experts; expert += blockDim.x) {
+    for (uint32_t expert = threadIdx.x; expert < experts; expert += SORT_MOST_WAVES * SORT_WAVE) {
         uint32_t counts[SORT_MOST_WAVES];
         (void)sort_counts_of(cursors, experts, expert, counts);
         sort_cursors_of(cursors, experts, expert, counts, first[expert]);

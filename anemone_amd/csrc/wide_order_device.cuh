@@ -53,11 +53,11 @@ __device__ static __forceinline__ uint32_t order_used_tiles(const struct wide_ex
 
 /* The block's strip of the grid's x and its columns: GROUP consecutive tiles of one run, fewer at the run's end. DOWN:
  * runs are tiles of one down matrix, else of one gate and up. Returns false for a block that has nothing to do. Every
- * lane of a wavefront calls; strips = gridDim.x, tile_count = gridDim.y. Two round trips to the table: the used tiles, and
+ * lane of a wavefront calls; strips and tile_count: the grid's. Two round trips to the table: the used tiles, and
  * the ORDER_WINDOW tiles around the block's own, a lane a tile (runs are cut where a window ends). alone_out: whether the
  * block's tiles are all of their run (as far as the block sees: a matter of speed, not of results). */
 template <uint32_t GROUP, bool DOWN, bool BY_RUN>
-__device__ static __forceinline__ bool order_block_of(const struct wide_expert_tile *tiles, uint32_t tile_count, uint32_t lane, uint32_t &strip_out,
+__device__ static __forceinline__ bool order_block_of(const struct wide_expert_tile *tiles, uint32_t tile_count, uint32_t strips, uint32_t lane, uint32_t &strip_out,
                                                       struct wide_expert_tile &tile_out, uint32_t &pair_count_out, bool *alone_out = nullptr)
 {
     if constexpr (!BY_RUN && GROUP == 1u) {
@@ -73,7 +73,6 @@ __device__ static __forceinline__ bool order_block_of(const struct wide_expert_t
         }
         return tile_out.pair_count != 0u;
     }
-    const uint32_t strips = gridDim.x;
     uint32_t used = tile_count, at = blockIdx.y, unit = 0;
     if constexpr (BY_RUN) {
         const uint32_t number = blockIdx.x + strips * blockIdx.y;

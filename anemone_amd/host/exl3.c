@@ -145,8 +145,7 @@ static result_status chain_prepare(const struct exl3_expert_record *record, uint
     char gate_up_name[40], down_name[40];
     const char *width = mixed ? "mixed" : exl3_width_name(exl3_bits_x2(record->bits_per_weight));
     /* the element-wise launches: a wavefront a row of a job, as many as the jobs hold on average */
-    const uint32_t rows_of_job = record->pair_count / record->job_count;
-    const uint32_t element_threads = WAVE_THREADS * (rows_of_job == 0u ? 1u : rows_of_job < LINEAR_MAXIMUM_ROWS ? rows_of_job : LINEAR_MAXIMUM_ROWS);
+    const uint32_t element_threads = WAVE_THREADS * exl3_element_rows(record->pair_count, record->job_count);
     const struct product_form gate_up = product_form_of(record->inner_size, record->job_count, 2u, inputs * 2u);
     const struct product_form down = product_form_of(record->input_size, record->job_count, 1u, (uint64_t)record->pair_count * record->inner_size * 2u);
     (void)snprintf(gate_up_name, sizeof gate_up_name, "exl3_gate_up_%s%s", width, gate_up.suffix);

@@ -27,9 +27,7 @@
 #define SELECT_THREADS (LINEAR_MAXIMUM_ROWS * 64u)
 #define WIDE_SORT_THREADS 512u
 #define PROJECTION_THREADS 128u
-#define PROJECTION_OUTPUTS 8u /* experts a block */
 #define PROJECTION_ROWS 4u    /* rows a block takes at once */
-#define PROJECTION_BY_ROW_MOST_BLOCKS 1024u
 
 result_status router_kernels_prepare(const struct backend_operations *backend, struct device_card *card,
                                      struct router_kernels_record *kernels_out)
@@ -296,7 +294,7 @@ result_status router_projection_prepare(const struct router_projection_descripti
     }
     /* a thin step: a row a block (the kernel takes one or four by its block's threads) */
     const uint32_t expert_blocks = (description->expert_count + PROJECTION_OUTPUTS - 1u) / PROJECTION_OUTPUTS;
-    const bool by_row = description->row_count <= LINEAR_MAXIMUM_ROWS && expert_blocks * description->row_count <= PROJECTION_BY_ROW_MOST_BLOCKS;
+    const bool by_row = router_projection_by_row(description->row_count, description->expert_count) != 0u;
     launch_fill(launch_out, kernels->projection, expert_blocks,
                 by_row ? description->row_count : (description->row_count + PROJECTION_ROWS - 1u) / PROJECTION_ROWS, 1,
                 by_row ? PROJECTION_THIN_THREADS : PROJECTION_THREADS, by_row ? PROJECTION_THIN_WINDOW_BYTES : PROJECTION_WINDOW_BYTES, &record,

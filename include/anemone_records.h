@@ -41,6 +41,12 @@
 #endif
 
 /* ---- shared geometry ---- */
+#ifdef __cplusplus
+#define ANEMONE_INLINE __host__ __device__ static constexpr inline
+#else
+#define ANEMONE_INLINE static inline
+#endif
+
 #define LINEAR_MAXIMUM_ROWS 8u          /* columns of one job; rows of one thin trunk launch, a group of a wide one */
 #define LINEAR_OUTPUTS_PER_TILE 16u
 #define LINEAR_VALUES_PER_BLOCK 32u     /* values that share one scale exponent */
@@ -107,6 +113,13 @@ ANEMONE_RECORD_HAS(wide_expert_tile, 32);
 #define PROJECTION_THIN_THREADS 256u /* of its blocks of one row; those of four rows are smaller */
 #define PROJECTION_THIN_WINDOW_BYTES (9u * (4096u + 32u) * 2u) /* dynamic shared memory of a block of one row */
 #define PROJECTION_WINDOW_BYTES (12u * 1024u * 2u)             /* and of four */
+#define PROJECTION_OUTPUTS 8u /* experts of a block of either */
+#define PROJECTION_BY_ROW_MOST_BLOCKS 1024u
+/* whether router_projection takes a step a row a block */
+ANEMONE_INLINE uint32_t router_projection_by_row(uint32_t row_count, uint32_t expert_count)
+{
+    return row_count <= LINEAR_MAXIMUM_ROWS && (uint64_t)(expert_count / PROJECTION_OUTPUTS + (expert_count % PROJECTION_OUTPUTS != 0u)) * row_count <= PROJECTION_BY_ROW_MOST_BLOCKS;
+}
 #define KERNEL_ROUTER_PROJECTION_TILES "router_projection_tiles" /* the same scores on the matrix unit: steps of many rows */
 #define PROJECTION_TILE_THREADS 256u
 #define PROJECTION_TILE_ROWS 64u   /* rows of a block of router_projection_tiles: 16 a wavefront */
@@ -218,6 +231,17 @@ ANEMONE_RECORD_HAS(router_wide_arguments, 136);
 #define EXL3_EXPERT_LAUNCHES 5u
 #define EXL3_PRODUCT_SLICES 4u
 #define EXL3_ELEMENT_MOST_THREADS 512u /* of a block of the chain's element-wise launches: a wavefront a row of a job */
+/* the wavefronts of such a block: as many as the jobs hold rows on average, one to eight. The kernels form it of the record
+ * as well: a kernel that asks for its block's or grid's size has thirteen arguments more, which the runtime fills in at every
+ * launch (2.7 -> 3.7 us of the calling thread; a single matrix of three launches then waited for the thread) */
+ANEMONE_INLINE uint32_t exl3_element_rows(uint32_t pair_count, uint32_t job_count)
+{
+    uint32_t rows = 1u;
+    for (uint32_t more = 2u; more <= LINEAR_MAXIMUM_ROWS; more++) {
+        rows += more * job_count <= pair_count ? 1u : 0u; /* the jobs are a grid's rows: at most 65,535 */
+    }
+    return rows;
+}
 #define EXL3_STRIP_TILES 8u      /* output tiles of a block of the chain's product launches: 128 outputs */
 #define EXL3_THIN_STRIP_TILES 1u /* of the _thin and _thin_many instances */
 /* A product launch takes one tile a block while that makes at most this many blocks. By 256 of them, a block a CU, a wavefront
@@ -226,12 +250,6 @@ ANEMONE_RECORD_HAS(router_wide_arguments, 136);
  * of 4096 inputs 18.7 | 24.0, 1,408 of 2048 inputs 13.9 | 14.1, 1,536 of 4096 inputs 25.0 | 24.1, 1,984 of 1024 inputs 10.9 | 9.4. */
 #define EXL3_THIN_BLOCKS 256u
 #define EXL3_THIN_MANY_BLOCKS 1408u
-
-#ifdef __cplusplus
-#define ANEMONE_INLINE __host__ __device__ static constexpr inline
-#else
-#define ANEMONE_INLINE static inline
-#endif
 
 /* bits_x2 = 2 K of a stored width; 0 for a value that is no width (whole 1-8, half 1.5-7.5) */
 ANEMONE_INLINE uint32_t exl3_bits_x2(uint32_t stored_width)

@@ -389,11 +389,12 @@ def test_a_slice_of_outputs_gives_the_whole_matrix_bits(amd, card, width):
 @pytest.mark.parametrize("rows_of_jobs", [(8,), (7, 1, 0, 2), (5, 8)])
 def test_chain_rows_by_wavefronts_give_the_same_bits(amd, card, rows_of_jobs):
     """The chain's element-wise launches take as many wavefronts a block as its jobs hold rows on average, a row each; jobs of
-    more rows, of fewer and of none: every byte of the operands, the hidden values and the output is that of blocks of one wavefront."""
+    more rows, of fewer and of none: every byte of the operands, the hidden values and the output is that of blocks of one wavefront,
+    which the same jobs take with empty ones behind them."""
     say("chain rows by wavefronts", rows_of_jobs)
     hidden, inner, width, job_count, pairs = 512, 256, 3, len(rows_of_jobs), sum(rows_of_jobs)
     places = [card.place(exl3_matrix(0x7900 + m, *((inner, hidden) if m < 2 else (hidden, inner)), width), 256) for m in range(3)]
-    jobs, next_pair = np.zeros(job_count, dtype=JOB_DTYPE), 0
+    jobs, next_pair = np.zeros(pairs, dtype=JOB_DTYPE), 0
     for job, rows in zip(jobs, rows_of_jobs):
         job["gate_offset"], job["up_offset"], job["down_offset"] = places
         job["row_count"], job["pair_index"][:rows], job["route_weight"][:rows] = rows, np.arange(next_pair, next_pair + rows)[::-1], 0.25 + np.arange(rows)
@@ -405,13 +406,12 @@ def test_chain_rows_by_wavefronts_give_the_same_bits(amd, card, rows_of_jobs):
     record.operands_offset, record.hidden_offset = at["operands"], at["hidden"]
     record.products_offset = record.output_offset = at["products"]
     record.input_size, record.inner_size = hidden, inner
-    record.pair_count, record.pairs_per_row, record.job_count = pairs, 1, job_count
+    record.pair_count, record.pairs_per_row = pairs, 1
     record.bits_per_weight, record.activation_limit = width, 10.0
     launches, outputs = amd.launches_of(5), []
-    amd.check(card.lib.exl3_experts_prepare(C.byref(record), card.arena_bytes, amd.backend_table(), card.handle, 950, launches), "prepare")
-    assert [launches[i].block[0] for i in (0, 2, 4)] == [64 * (pairs // job_count)] * 3
-    for threads in (launches[0].block[0], 64):
-        launches[0].block[0] = launches[2].block[0] = launches[4].block[0] = threads
+    for record.job_count in (job_count, pairs):
+        amd.check(card.lib.exl3_experts_prepare(C.byref(record), card.arena_bytes, amd.backend_table(), card.handle, 950, launches), "prepare")
+        assert [launches[i].block[0] for i in (0, 2, 4)] == [64 * (pairs // record.job_count)] * 3
         for name, size in sizes.items():
             card.upload(at[name], np.full(size, 0xEE, dtype=np.uint8))
         card.run(launches[0:1])
