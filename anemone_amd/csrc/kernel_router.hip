@@ -405,120 +405,145 @@ extern "C" __global__ void __launch_bounds__(PROJECTION_TILE_THREADS, 3) /* thre
 ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_projection_tiles, router_projection_arguments);
 
 /* The same scores for steps whose tiles of 16 experts by 64 rows leave CUs idle or unevenly loaded (which those are:
- * PROJECTION_SPLIT_BLOCKS_OF_TILE, with both forms' times): a block is one 16 x 16 tile, and its four wavefronts take eight
- * chains each, so that a CU's four vector units work on every score. Instruction t of a group of 32 inputs takes the chains
- * 8 wave + 2 b + t of the blocks b = 0 .. 3: lane (b, n) needs the two inputs 32 i + 8 wave + 2 b + {0, 1} of expert n and
- * of row n, one word each. A stage is the 16 + 16 rows'
- * 128 inputs (8 KB, laid out and swizzled as above); PROJECTION_SPLIT_STAGES of them are in LDS or on their way (three blocks
- * a CU; five to sixteen measured within 10 %), and a stage is read behind the instructions of the one before it. The
- * wavefronts' sums meet in LDS at the end, each wavefront folding a quarter of the scores. What is left is a wavefront's 256
- * instructions of 4096 inputs and their conversions (10,900 cycles, 5 us), the first loads' way from memory and the
- * launch. By router_projection / so, us, 256 experts of 4096 inputs: 203 rows 38 / 13.5, 100 rows 25 / 12.7, 64 rows 14.3 /
- * 12, 37 rows 15 / 13.2, 16 rows 13 / 12.6; up to eight rows router_projection takes a row a block (7 to 11).
- * grid (E / 16, ceil(rows / 16)), block 256. */
+ * PROJECTION_SPLIT_BLOCKS_OF_TILE, with both forms' times): a block is one 16 x 16 tile, and its eight wavefronts take four
+ * chains each, so that a CU's four vector units work on every score, two wavefronts a unit. The instruction of a group of 32
+ * inputs takes the chains 4 wave + b of the blocks b = 0 .. 3: lane (b, n) needs the input 32 i + 4 wave + b of expert n and of
+ * row n, 16 bits each, which LDS reads into the upper half of a register whose lower half is zero: a float32, and no conversion
+ * that the matrix instruction would wait for. A stage is the 16 + 16 rows' 128 inputs (8 KB, laid out and swizzled as above, a
+ * load a wavefront). Stages go in pairs, a barrier a pair; three pairs are in LDS or on their way (three blocks a CU), and a stage
+ * is read behind the instructions of the one before it. The wavefronts' sums meet in LDS at the end, half of them folding the
+ * scores. What bounds it: a unit's 256 instructions of 4096 inputs, 33 cycles each, beside 64 LDS reads a stage; the first loads'
+ * way from memory; the launch. By four wavefronts of eight chains, words converted and a barrier a stage | so, us, 256 experts of
+ * 4096 inputs: 32 rows 10.75 | 9.25, 203 rows 10.85 | 9.45, 300 rows 15.3 | 14.35, 700 rows 21.6 | 20.0 (eight wavefronts with a
+ * barrier a stage 9.95 and 22.6). grid (E / 16, ceil(rows / 16)), block (256, 2). */
 #define PROJECTION_SPLIT_STAGE_BYTES (32u * PROJECTION_STAGE_ROW_BYTES)
-#define PROJECTION_SPLIT_STAGES 6u
-extern "C" __global__ void __launch_bounds__(PROJECTION_TILE_THREADS)
+#define PROJECTION_SPLIT_PAIRS 3u
+#define PROJECTION_SPLIT_WAVES (2u * PROJECTION_TILE_THREADS / WAVE)
+struct split_inputs {
+    float w[4], x[4]; /* of a stage's four groups; the lower halves stay zero */
+};
+
+/* a stage's inputs out of LDS: asked for here, there behind split_landed */
+template <uint32_t STAGE> __device__ static __forceinline__ void split_read(const uint32_t (&at)[4], uint32_t place, struct split_inputs &into)
+{
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; i++) {
+        const uint32_t from = at[i] + place;
+        asm volatile("ds_read_u16_d16_hi %0, %1 offset:%2" : "+v"(into.w[i]) : "v"(from), "n"(STAGE * PROJECTION_SPLIT_STAGE_BYTES) : "memory");
+        asm volatile("ds_read_u16_d16_hi %0, %1 offset:%2" : "+v"(into.x[i]) : "v"(from), "n"(STAGE * PROJECTION_SPLIT_STAGE_BYTES + 4096u) : "memory");
+    }
+}
+
+__device__ static __forceinline__ void split_landed(struct split_inputs &inputs)
+{
+    asm volatile("s_waitcnt lgkmcnt(0)"
+                 : "+v"(inputs.w[0]), "+v"(inputs.w[1]), "+v"(inputs.w[2]), "+v"(inputs.w[3]), "+v"(inputs.x[0]), "+v"(inputs.x[1]), "+v"(inputs.x[2]),
+                   "+v"(inputs.x[3])
+                 :
+                 : "memory");
+}
+
+extern "C" __global__ void __launch_bounds__(2u * PROJECTION_TILE_THREADS)
     router_projection_split(struct router_projection_arguments arguments, unsigned char *arena)
 {
-    __shared__ __attribute__((aligned(1024))) unsigned char window[PROJECTION_SPLIT_STAGES * PROJECTION_SPLIT_STAGE_BYTES];
-    const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), block = lane / 16u, index = lane % 16u;
-    const uint32_t H = arguments.hidden, stages = H / PROJECTION_STAGE_INPUTS;
+    constexpr uint32_t PAIR_BYTES = 2u * PROJECTION_SPLIT_STAGE_BYTES;
+    __shared__ __attribute__((aligned(1024))) unsigned char window[PROJECTION_SPLIT_PAIRS * PAIR_BYTES];
+    const uint32_t lane = threadIdx.x % WAVE, block = lane / 16u, index = lane % 16u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane((threadIdx.x + PROJECTION_TILE_THREADS * threadIdx.y) / WAVE);
+    const uint32_t H = arguments.hidden, stages = H / PROJECTION_STAGE_INPUTS, pairs = (stages + 1u) / 2u;
     const uint32_t first_expert = blockIdx.x * 16u, first_row = blockIdx.y * 16u;
     const uint32_t window_address = (uint32_t)(uintptr_t)(lds_bytes)window;
-    /* this wavefront brings four experts' rows and four rows of a stage (a row past the last repeats the last) */
-    const uint32_t line = 4u * wave + lane / 16u, row = first_row + line < arguments.row_count ? first_row + line : arguments.row_count - 1u;
-    const uint32_t piece_bytes = 16u * ((lane % 16u) ^ line);
-    const unsigned char *w_source = arena + arguments.weights_offset + (uint64_t)(first_expert + line) * H * 2u + piece_bytes;
-    const unsigned char *x_source = arena + arguments.rows_offset + (uint64_t)row * H * 2u + piece_bytes;
-    auto ask = [&](uint32_t stage, uint32_t place) {
-        const uint32_t base = window_address + place * PROJECTION_SPLIT_STAGE_BYTES + wave * 1024u;
-        projection_load_to_lds(w_source + (uint64_t)stage * PROJECTION_STAGE_ROW_BYTES, base);
-        projection_load_to_lds(x_source + (uint64_t)stage * PROJECTION_STAGE_ROW_BYTES, base + 16u * PROJECTION_STAGE_ROW_BYTES);
+    /* this wavefront brings four experts' rows of a stage (the first four) or four rows (a row past the last repeats the last) */
+    const uint32_t line = 4u * (wave % 4u) + lane / 16u, last_row = arguments.row_count - 1u - first_row;
+    const unsigned char *base = arena + (wave < 4u ? arguments.weights_offset + (uint64_t)first_expert * H * 2u : arguments.rows_offset + (uint64_t)first_row * H * 2u);
+    const uint32_t own = 16u * ((lane % 16u) ^ line) + (wave < 4u || line < last_row ? line : last_row) * (H * 2u);
+    const uint32_t lands_at = window_address + wave * 1024u;
+    /* a stage past the last is the last again, into a place that nobody reads any more: every wait counts the same */
+    auto ask = [&](uint32_t pair, uint32_t place) {
+        const uint32_t one = 2u * pair < stages ? 2u * pair : stages - 1u, two = 2u * pair + 1u < stages ? 2u * pair + 1u : stages - 1u;
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %4, %3"
+                     : : "s"(lands_at + place), "s"(lands_at + place + PROJECTION_SPLIT_STAGE_BYTES), "v"(own + one * PROJECTION_STAGE_ROW_BYTES), "s"(base),
+                       "v"(own + two * PROJECTION_STAGE_ROW_BYTES) : "memory", "m0");
     };
-    /* past the last stage the last is asked for again, into a place that nobody reads any more: every wait counts the same */
-    for (uint32_t stage = 0; stage < PROJECTION_SPLIT_STAGES; stage++) {
-        ask(stage < stages ? stage : stages - 1u, stage);
+    for (uint32_t pair = 0; pair < PROJECTION_SPLIT_PAIRS; pair++) {
+        ask(pair, pair * PAIR_BYTES);
     }
-    float16_t chain[2];
+    float16_t chain;
 #pragma unroll
     for (uint32_t v = 0; v < 16u; v++) {
-        chain[0][v] = chain[1][v] = 0.0f;
+        chain[v] = 0.0f;
     }
-    uint32_t w_words[4], x_words[4];
-    auto read = [&](uint32_t place) {
-        const unsigned char *now = window + place * PROJECTION_SPLIT_STAGE_BYTES + index * PROJECTION_STAGE_ROW_BYTES + 4u * block;
+    /* input 32 i + 4 wave + block of line `index`: piece 4 i + wave / 2, its value 4 (wave % 2) + block */
+    uint32_t at[4];
+    struct split_inputs inputs[2];
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; i++) {
+        at[i] = window_address + index * PROJECTION_STAGE_ROW_BYTES + 16u * ((4u * i + wave / 2u) ^ index) + 2u * (4u * (wave % 2u) + block);
+        inputs[0].w[i] = inputs[0].x[i] = inputs[1].w[i] = inputs[1].x[i] = 0.0f;
+    }
+    /* this wavefront's loads of the first pair have landed, then every wavefront's */
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2u * (PROJECTION_SPLIT_PAIRS - 1u)) : "memory");
+    __syncthreads();
+    split_read<0>(at, 0u, inputs[0]);
+    uint32_t place = 0;
+    for (uint32_t pair = 0; pair < pairs; pair++) {
+        split_landed(inputs[0]);
+        split_read<1>(at, place, inputs[1]);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (uint32_t i = 0; i < 4u; i++) {
-            const uint32_t slot = 16u * ((4u * i + wave) ^ index);
-            w_words[i] = *(const uint32_t *)(now + slot);
-            x_words[i] = *(const uint32_t *)(now + 16u * PROJECTION_STAGE_ROW_BYTES + slot);
+            chain = __builtin_amdgcn_mfma_f32_16x16x1f32(inputs[0].w[i], inputs[0].x[i], chain, 0, 0, 0);
         }
-    };
-    /* this wavefront's loads of the oldest stage have landed, then every wavefront's */
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2u * (PROJECTION_SPLIT_STAGES - 1u)) : "memory");
-    __syncthreads();
-    read(0u);
-    uint32_t place = 0;
-    for (uint32_t stage = 0; stage < stages; stage++) {
-        float w_values[8], x_values[8];
-        projection_convert(w_words, w_values);
-        projection_convert(x_words, x_values);
-        /* the next stage is read behind this one's instructions; every wavefront has read this one, whose place the one to
-         * ask for takes */
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2u * (PROJECTION_SPLIT_STAGES - 2u)) : "memory");
-        __syncthreads();
-        const uint32_t ahead = stage + PROJECTION_SPLIT_STAGES;
-        ask(ahead < stages ? ahead : stages - 1u, place);
-        place = place + 1u < PROJECTION_SPLIT_STAGES ? place + 1u : 0u;
-        read(place);
         __builtin_amdgcn_sched_barrier(0);
+        /* every wavefront has read the pair, whose place the one to ask for takes; the next pair has landed */
+        split_landed(inputs[1]);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2u * (PROJECTION_SPLIT_PAIRS - 2u)) : "memory");
+        __syncthreads();
+        ask(pair + PROJECTION_SPLIT_PAIRS, place);
+        place = place + PAIR_BYTES < PROJECTION_SPLIT_PAIRS * PAIR_BYTES ? place + PAIR_BYTES : 0u;
+        split_read<0>(at, place, inputs[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (2u * pair + 1u < stages) {
 #pragma unroll
-        for (uint32_t k = 0; k < 8u; k++) {
-            chain[k % 2u] = __builtin_amdgcn_mfma_f32_16x16x1f32(w_values[k], x_values[k], chain[k % 2u], 0, 0, 0);
+            for (uint32_t i = 0; i < 4u; i++) {
+                chain = __builtin_amdgcn_mfma_f32_16x16x1f32(inputs[1].w[i], inputs[1].x[i], chain, 0, 0, 0);
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-    /* register v = 4 b + r of chain[t] is chain 8 wave + 2 b + t of expert 4 (lane / 16) + r and row lane % 16. Every
-     * wavefront leaves its eight chains of the experts r, [r][b][t] a lane; wavefront r then folds those of expert 4 (lane / 16) + r
-     * as the definition orders it: + 0 first, then the distances 16 and 8 (wavefronts), 4 and 2 (blocks), 1 (instructions) */
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* the last stage's repeats */
+    split_landed(inputs[0]);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* the last pairs' repeats */
     __syncthreads();
-    float *exchange = (float *)window; /* [wavefront][r][lane][8] */
+    /* register v = 4 b + r is chain 4 wave + b of expert 4 (lane / 16) + r and row lane % 16. Every wavefront leaves its four
+     * chains of the experts r; wavefront r then folds those of expert 4 (lane / 16) + r as the definition orders it: + 0 first, then
+     * the distances 16, 8 and 4 (wavefronts), 2 and 1 (blocks) */
+    float4_t *exchange = (float4_t *)window; /* [wavefront][r][lane] */
 #pragma unroll
     for (uint32_t r = 0; r < 4u; r++) {
-        float *to = exchange + ((wave * 4u + r) * WAVE + lane) * 8u;
-#pragma unroll
-        for (uint32_t b = 0; b < 4u; b += 2u) {
-            *(float4_t *)(to + 2u * b) = (float4_t){__fadd_rn(0.0f, chain[0][4u * b + r]), __fadd_rn(0.0f, chain[1][4u * b + r]),
-                                                   __fadd_rn(0.0f, chain[0][4u * b + 4u + r]), __fadd_rn(0.0f, chain[1][4u * b + 4u + r])};
-        }
+        exchange[(wave * 4u + r) * WAVE + lane] = (float4_t){__fadd_rn(0.0f, chain[r]), __fadd_rn(0.0f, chain[4u + r]), __fadd_rn(0.0f, chain[8u + r]),
+                                                             __fadd_rn(0.0f, chain[12u + r])};
     }
     __syncthreads();
-    float sums[8];
+    if (wave >= 4u || first_row + index >= arguments.row_count) {
+        return;
+    }
+    float4_t part[PROJECTION_SPLIT_WAVES];
 #pragma unroll
-    for (uint32_t k = 0; k < 8u; k += 4u) {
-        float4_t part[4];
-#pragma unroll
-        for (uint32_t from = 0; from < 4u; from++) {
-            part[from] = *(const float4_t *)(exchange + ((from * 4u + wave) * WAVE + lane) * 8u + k);
-        }
-#pragma unroll
-        for (uint32_t v = 0; v < 4u; v++) {
-            sums[k + v] = __fadd_rn(__fadd_rn(part[0][v], part[2][v]), __fadd_rn(part[1][v], part[3][v]));
-        }
+    for (uint32_t from = 0; from < PROJECTION_SPLIT_WAVES; from++) {
+        part[from] = exchange[(from * 4u + wave) * WAVE + lane];
     }
 #pragma unroll
-    for (uint32_t distance = 4u; distance != 0u; distance >>= 1u) {
+    for (uint32_t distance = PROJECTION_SPLIT_WAVES / 2u; distance != 0u; distance >>= 1u) {
 #pragma unroll
-        for (uint32_t k = 0; k < distance; k++) {
-            sums[k] = __fadd_rn(sums[k], sums[k + distance]);
+        for (uint32_t from = 0; from < distance; from++) {
+#pragma unroll
+            for (uint32_t b = 0; b < 4u; b++) {
+                part[from][b] = __fadd_rn(part[from][b], part[from + distance][b]);
+            }
         }
     }
-    if (first_row + index < arguments.row_count) {
-        ((float *)(arena + arguments.output_offset))[(uint64_t)(first_row + index) * arguments.expert_count + first_expert + 4u * block + wave] =
-            __fadd_rn(0.0f, sums[0]);
-    }
+    const float sum = __fadd_rn(__fadd_rn(part[0][0], part[0][2]), __fadd_rn(part[0][1], part[0][3]));
+    ((float *)(arena + arguments.output_offset))[(uint64_t)(first_row + index) * arguments.expert_count + first_expert + 4u * block + wave] = __fadd_rn(0.0f, sum);
 }
 ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_projection_split, router_projection_arguments);
 

@@ -8,7 +8,7 @@
  *   launch        kernel                grid                        block
  *   projection    router_projection     (ceil(E / 8), rows, 1)             256   thin steps: eight experts and a row a block, a lane a chain
  *                                       (ceil(E / 8), ceil(rows / 4), 1)   128   other sizes: eight experts and four rows a block
- *                 router_projection_split (E / 16, ceil(rows / 16), 1)     256   9 rows and more of a width in whole 128, E in whole 16: 16
+ *                 router_projection_split (E / 16, ceil(rows / 16), 1)  256, 2   9 rows and more of a width in whole 128, E in whole 16: 16
  *                                                                                experts by 16 rows a block
  *                 router_projection_tiles (E / 16, ceil(rows / 64), 1)     256   such steps where its fewer blocks are as many as the CUs
  *                                                                                (projection_takes_split): 16 experts by 64 rows a block
@@ -283,6 +283,7 @@ result_status router_projection_prepare(const struct router_projection_descripti
             launch_fill(launch_out, kernels->projection_split, description->expert_count / 16u,
                         (description->row_count + PROJECTION_SPLIT_ROWS - 1u) / PROJECTION_SPLIT_ROWS, 1, PROJECTION_TILE_THREADS, 0, &record,
                         sizeof record);
+            launch_out->block[1] = 2u;
             return STATUS_OK;
         }
         if (has_tiles && (has_split || description->row_count >= PROJECTION_TILE_LEAST_ROWS)) {

@@ -129,8 +129,9 @@ ANEMONE_INLINE uint32_t router_projection_by_row(uint32_t row_count, uint32_t ex
 #define PROJECTION_SPLIT_LEAST_ROWS 9u  /* up to eight rows router_projection takes a row a block, in blocks of eight experts */
 /* Which of the two takes a step of more rows. A block of router_projection_tiles is a score's 32 chains in one wavefront, so a
  * launch takes as long as the blocks that fall to one of the 256 CUs, one behind the other in all but the loads; a block of
- * router_projection_split is a quarter of that, on as many wavefronts, and brings its operands for a quarter of the scores. In
- * blocks a CU, us, 4096 inputs: tiles 1 / 2 / 3 / 4 blocks 26.6 / 42.8 / 64 / 87; split 1 .. 10 blocks 11.3 / 16.5 / 22.4 / 28.4 /
+ * router_projection_split is a quarter of that, on twice as many wavefronts, and brings its operands for a quarter of the scores. In
+ * blocks a CU, us, 4096 inputs: tiles 1 / 2 / 3 / 4 blocks 26.6 / 42.8 / 64 / 87; split (by four wavefronts, which drew the line; by
+ * eight 9.3 / 15.1 / 20.6, 31.2 at five, 38 at six) 1 .. 10 blocks 11.3 / 16.5 / 22.4 / 28.4 /
  * 33.8 / 39.6 / 45.5 / 51 / 57 / 64: three blocks of the split form are the faster, four the slower (256 experts: 512 rows 26.8 |
  * 17.0, 768 rows 26.8 | 22.7, 1024 rows 27.1 | 28.5, 1152 rows 42.7 | 33.7, 1536 rows 42.8 | 40.3, 1792 rows 43.4 | 46.1; 64 experts: 3072
  * rows 27.1 | 23.3, 4096 rows 27.5 | 29.3; 384 experts: 512 rows 27.0 | 22.6, 640 rows 26.9 | 28.5; 2048 and 5120 inputs: the same line). */

@@ -249,6 +249,12 @@ def test_projection_of_few_rows_bit_exact(amd, card, experts_n, rows, hidden, sc
     assert np.all(card.download(layer.affinities_offset, rows * experts_n * 4, np.uint8) == 0xEE)
 
 
+@pytest.mark.parametrize("experts_n,rows,hidden,scale", [(64, 9, 256, 1.0), (64, 31, 384, 1e-18), (128, 16, 512, 3e18), (64, 17, 1152, 1.0)])
+def test_projection_of_few_rows_by_pairs_of_stages(amd, card, experts_n, rows, hidden, scale):
+    """router_projection_split's stages go in pairs: one pair, a pair and a half, two, and the places used again, with a half behind."""
+    test_projection_of_few_rows_bit_exact(amd, card, experts_n, rows, hidden, scale)
+
+
 def test_fp4_layer_through_the_wide_job_table(amd, card):
     """40 rows (37 live) routed by the wide select, then the FP4 experts over its job table, against the oracle."""
     say("fp4 layer, wide")
