@@ -1,7 +1,7 @@
 /*
  * kernel_selfcheck.hip -- the library's check of its own short cuts in arithmetic. Some helpers of the kernels take a
- * shorter way than the arithmetic they are defined by: det_silu and det_sigmoid (no tests around the exponential), quantize_codes4
- * (the card's FP8 conversions) and quantize_quotient (a reciprocal and a correction in place of a division). This kernel runs both ways over every input there is and counts the disagreements, so
+ * shorter way than the arithmetic they are defined by: det_silu and det_sigmoid (no tests around the exponential,
+ * quotient_above_one for the division), quantize_codes4 (the card's FP8 conversions) and quantize_quotient (a reciprocal and a correction in place of a division). This kernel runs both ways over every input there is and counts the disagreements, so
  * that a test on the card proves the two ways equal instead of sampling them. No counterpart in the reference; not on
  * the routed-expert path.
  */

@@ -42,7 +42,7 @@ __device__ static __forceinline__ float det_log1pf(float y) /* 0 <= y <= 1 */
 __device__ static __forceinline__ float det_sigmoid(float score)
 {
     const float x = __builtin_amdgcn_fmed3f(-score, -104.0f, 89.5f);
-    const float value = __fdiv_rn(1.0f, __fadd_rn(1.0f, det_exp_sequence(x)));
+    const float value = quotient_above_one(1.0f, __fadd_rn(1.0f, det_exp_sequence(x)));
     return score != score ? score : value;
 }
 

@@ -207,3 +207,62 @@ def test_prefill_equals_fused_decode_on_the_same_rows(amd, card):
     error = float(np.max(np.abs(prefill - decode))) / scale
     say("  max difference %.2e of rms" % error)
     assert error <= 2e-4
+
+
+@pytest.mark.parametrize("limit", [10.0, 0.0])
+def test_activation_of_products_that_are_no_numbers(amd, card, limit):
+    """The activation of gate and up products given to it, among them blocks of infinities and not-a-numbers: with a limit a gate
+    that is not a number is the limit and such an up product the lower one (fminf(gate, limit), fminf(fmaxf(up, -limit), limit));
+    without one they stay what they are. Against the same steps in float64. What float32 moves: a down operand is a sum of 128
+    values, each of some ten roundings, then one to fp16: below 2^-10 of the block's largest value or sum of magnitudes / 128."""
+    hidden, inner, experts_n, picks, rows = 128, 256, 64, 2, 70
+    say("activation", limit)
+    layer, matrices, widths = build_layer(amd, card, hidden, inner, experts_n, picks, rows, 43, [2, 4])
+    layer.limit = limit
+    layer.set_rows(to_bf16(normals(44, rows * hidden)).reshape(rows, hidden), rows)
+    card.upload(layer.bias_offset, np.zeros(experts_n, dtype=np.float32))
+    card.run(layer.projection_launch())
+    wide = layer.wide_router()
+    card.run(wide.launches()[0:1])
+    experts = wide.read("picks", np.dtype([("expert", "<u4"), ("route_weight", "<f4")])).reshape(-1)["expert"]
+    launches = layer.tcp_launches(wide.ranges["picks"].byte_offset)
+    card.run(launches[0:3])
+    pairs, layout = rows * picks, layer.tcp_layout
+    products = (normals(45, 2 * pairs * inner) * 30.0).astype(np.float32).reshape(2, pairs, inner)
+    for place, (gate, up) in enumerate([(np.nan, 1.0), (1.0, np.nan), (np.nan, np.nan), (np.inf, 2.0), (-np.inf, 2.0), (3.0, np.inf),
+                                        (3.0, -np.inf), (3e38, -3e38), (-0.0, 0.0)]):
+        products[0, 7 * place, 128:], products[1, 7 * place, 128:] = gate, up
+    card.upload(layer.tcp_workspace_offset + layout["gate_up"], products)
+    card.run(launches[4:5])
+    got = card.download(layer.tcp_workspace_offset + layout["operands"], pairs * inner * 2, np.float16).reshape(pairs, inner).astype(np.float64)
+    sorted_pairs = card.download(layer.tcp_workspace_offset + layout["sorted"], pairs * 4, np.uint32)
+    signs = np.array([[(-1.0) ** bin(i & j).count("1") for j in range(128)] for i in range(128)])
+
+    def block_sums(values):  # the butterflies in float32, as an infinity meets its like in them
+        values = values.astype(np.float32).reshape(-1, 128).copy()
+        for distance in (1, 2, 4, 8, 16, 32, 64):
+            pair = values.reshape(-1, 64 // distance, 2, distance)
+            values = np.stack([pair[:, :, 0] + pair[:, :, 1], pair[:, :, 0] - pair[:, :, 1]], axis=2).reshape(-1, 128)
+        return values.reshape(-1)
+
+    with np.errstate(all="ignore"):
+        for place in range(pairs):
+            trio = matrices[int(experts[sorted_pairs[place]])]
+            e = int(experts[sorted_pairs[place]])
+            scales = []
+            for matrix, (rows_in, columns_out) in enumerate([(hidden, inner), (hidden, inner), (inner, hidden)]):
+                code_bytes = int(orc.orc_exl3_code_bytes(rows_in, columns_out, int(widths[e, matrix])))
+                halves = np.ascontiguousarray(trio[matrix][code_bytes:code_bytes + 2 * (rows_in + columns_out)]).view(np.float16).astype(np.float64)
+                scales.append(halves[rows_in:] if matrix < 2 else halves[:rows_in])
+            gate, up = [block_sums(products[side, place]).astype(np.float64) / np.sqrt(128.0) * scales[side] for side in (0, 1)]
+            if limit > 0.0:
+                gate, up = np.fmin(gate, limit), np.fmin(np.fmax(up, -limit), limit)
+            values = gate / (1.0 + np.exp(-gate)) * up * scales[2]
+            want = (values.reshape(-1, 128) @ signs / np.sqrt(128.0)).reshape(-1)
+            for block in range(inner // 128):
+                here = slice(128 * block, 128 * block + 128)
+                if not np.isfinite(values[here]).all() or np.abs(want[here]).max() > 6e4:
+                    assert not np.isfinite(got[place, here]).all(), (place, block)
+                    continue
+                bound = 2.0 ** -10 * max(np.abs(want[here]).max(), np.abs(values[here]).mean())
+                assert np.abs(got[place, here] - want[here]).max() <= bound, (place, block)
