@@ -17,6 +17,8 @@
  * outputs, one for every 32 columns. Decoding is the vector unit's work (about 3.7 instructions a weight) and the
  * products the matrix unit's (32 cycles an instruction).
  */
+#include <type_traits>
+
 #include "exl3_stream_device.cuh"
 #include "kernel_registry.h"
 #include "sort_device.cuh"
@@ -29,6 +31,11 @@
 #define TCP_STEP_INPUTS 64u
 #define TCP_DIES 8u         /* the card's dies (XCDs), each with a level-2 cache of its own: blocks are dealt to them in turn */
 #define TCP_BATCH 4u        /* columns, or slots of a row, the element-wise launches take at a time */
+/* values of one of the two operand arrays from which on they are written past the caches (nontemporal): two arrays of 192 MiB and
+ * more leave the 256 MB behind the dies before the products read them, whichever way they are written. 256 experts, 8 picks, hidden
+ * 4096, as before -> nontemporal: 2048 rows 59.0 -> 61.1 us, 2560 73.9 -> 75.4, 3072 (the line) 89.4 -> 88.6, 4096 128.6 -> 112.6,
+ * 6144 208 -> 166; the products behind them take the same */
+#define TCP_STREAMED_OPERANDS (96ull << 20)
 #define TCP_THIN_PLACES 4u  /* places of a block of a thin call's element-wise launches: one a wavefront */
 #define TCP_WAVE_BLOCKS 4u  /* blocks of 128 channels a wavefront of an element-wise launch takes: a row of sixteen lanes each */
 
@@ -208,29 +215,39 @@ extern "C" __global__ void exl3_tcp_operands(struct exl3_tcp_record record, unsi
     const uint16_t *rows = (const uint16_t *)(arena + record.hidden_offset);
     const uint32_t *sorted = (const uint32_t *)(workspace + shape.layout.sorted);
     uint16_t *operands = (uint16_t *)(workspace + shape.layout.operands);
-    /* TCP_BATCH columns at a time: their loads are asked for together, so that one column's latency hides behind
-     * the others' (a column past the part's last repeats it and is not stored) */
-    for (uint32_t first = first_column; first < last_column; first += TCP_BATCH) {
-        uint4_t loads[TCP_BATCH];
-        uint32_t place[TCP_BATCH];
+    const auto write = [&](auto streamed) {
+        /* TCP_BATCH columns at a time: their loads are asked for together, so that one column's latency hides behind
+         * the others' (a column past the part's last repeats it and is not stored) */
+        for (uint32_t first = first_column; first < last_column; first += TCP_BATCH) {
+            uint4_t loads[TCP_BATCH];
+            uint32_t place[TCP_BATCH];
 #pragma unroll
-        for (uint32_t i = 0; i < TCP_BATCH; i++) {
-            const uint32_t column = first + i < last_column ? first + i : last_column - 1u;
-            place[i] = chunk.first_pair + column;
-            const uint64_t row = sorted[place[i]] / shape.picks;
-            loads[i] = *(const uint4_t *)(rows + row * shape.hidden + channel);
-        }
+            for (uint32_t i = 0; i < TCP_BATCH; i++) {
+                const uint32_t column = first + i < last_column ? first + i : last_column - 1u;
+                place[i] = chunk.first_pair + column;
+                const uint64_t row = sorted[place[i]] / shape.picks;
+                loads[i] = *(const uint4_t *)(rows + row * shape.hidden + channel);
+            }
 #pragma unroll
-        for (uint32_t i = 0; i < TCP_BATCH; i++) {
-            const bool kept = first + i < last_column;
+            for (uint32_t i = 0; i < TCP_BATCH; i++) {
+                const bool kept = first + i < last_column;
 #pragma unroll
-            for (uint32_t projection = 0; projection < 2u; projection++) {
-                const uint4_t operand = row_operand(loads[i], scale[projection], lane);
-                if (kept) {
-                    *(uint4_t *)(operands + ((uint64_t)projection * shape.pairs + place[i]) * shape.hidden + channel) = operand;
+                for (uint32_t projection = 0; projection < 2u; projection++) {
+                    const uint4_t operand = row_operand(loads[i], scale[projection], lane);
+                    uint4_t *out = (uint4_t *)(operands + ((uint64_t)projection * shape.pairs + place[i]) * shape.hidden + channel);
+                    if (kept && streamed.value) {
+                        __builtin_nontemporal_store(operand, out);
+                    } else if (kept) {
+                        *out = operand;
+                    }
                 }
             }
         }
+    };
+    if (shape.pairs * (uint64_t)shape.hidden >= TCP_STREAMED_OPERANDS) { /* the same in every block */
+        write(std::true_type{});
+    } else {
+        write(std::false_type{});
     }
 }
 ANEMONE_KERNEL(EXL3_TCP_KERNEL_FILE, exl3_tcp_operands, exl3_tcp_record);

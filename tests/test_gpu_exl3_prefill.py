@@ -266,3 +266,32 @@ def test_activation_of_products_that_are_no_numbers(amd, card, limit):
                     continue
                 bound = 2.0 ** -10 * max(np.abs(want[here]).max(), np.abs(values[here]).mean())
                 assert np.abs(got[place, here] - want[here]).max() <= bound, (place, block)
+
+
+@pytest.mark.parametrize("rows", [3071, 3072])
+def test_operands_about_the_line_of_their_streamed_form(amd, card, rows):
+    """The operands of a step are written past the caches from 96 Mi values an array on (3072 rows of 8 picks by 4096): the row
+    below the line and the line itself, bit for bit the oracle's, the first and the last place among those looked at."""
+    hidden, inner, experts_n, picks = 4096, 128, 64, 8
+    say("streamed operands", rows)
+    layer, matrices, widths = build_layer(amd, card, hidden, inner, experts_n, picks, rows, 61, [2, 4])
+    x = to_bf16(normals(62, rows * hidden)).reshape(rows, hidden)
+    layer.set_rows(x, rows)
+    card.upload(layer.bias_offset, np.zeros(experts_n, dtype=np.float32))
+    card.run(layer.projection_launch())
+    wide = layer.wide_router()
+    card.run(wide.launches()[0:1])
+    experts = wide.read("picks", np.dtype([("expert", "<u4"), ("route_weight", "<f4")])).reshape(-1)["expert"]
+    card.run(layer.tcp_launches(wide.ranges["picks"].byte_offset)[0:3])
+    pairs, layout = rows * picks, layer.tcp_layout
+    sorted_pairs = card.download(layer.tcp_workspace_offset + layout["sorted"], pairs * 4, np.uint32)
+    operands = card.download(layer.tcp_workspace_offset + layout["operands"], 2 * pairs * hidden * 2, np.uint16).reshape(2, pairs, hidden)
+    for place in [0, 1, pairs - 2, pairs - 1] + list(range(97, pairs, pairs // 29)):
+        pair = int(sorted_pairs[place])
+        e = int(experts[pair])
+        for side in range(2):
+            code_bytes = int(orc.orc_exl3_code_bytes(hidden, inner, int(widths[e, side])))
+            suh = np.ascontiguousarray(matrices[e][side][code_bytes:code_bytes + 2 * hidden]).view(np.uint16)
+            expect = np.zeros(hidden, dtype=np.uint16)
+            orc.orc_exl3_operand(ptr(x[pair // picks], u16p), ptr(suh, u16p), hidden, ptr(expect, u16p))
+            assert np.array_equal(operands[side, place], expect), (place, side)
