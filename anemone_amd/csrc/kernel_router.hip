@@ -423,7 +423,10 @@ struct split_inputs {
     float w[4], x[4]; /* of a stage's four groups; the lower halves stay zero */
 };
 
-/* a stage's inputs out of LDS: asked for here, there behind split_landed */
+/* A stage's inputs out of LDS: asked for here, there behind split_landed. Assembly, as the compiler has no read of this form; it
+ * takes the registers for filled where they are asked for, and one that it copied or saved in between would be taken before it
+ * is filled. So the two stand in one run of instructions without a branch or a loop's end between them, with nothing but the
+ * matrix instructions of the other set, and the build refuses the kernel if it spills a vector register. */
 template <uint32_t STAGE> __device__ static __forceinline__ void split_read(const uint32_t (&at)[4], uint32_t place, struct split_inputs &into)
 {
 #pragma unroll
@@ -450,7 +453,7 @@ extern "C" __global__ void __launch_bounds__(2u * PROJECTION_TILE_THREADS)
     __shared__ __attribute__((aligned(1024))) unsigned char window[PROJECTION_SPLIT_PAIRS * PAIR_BYTES];
     const uint32_t lane = threadIdx.x % WAVE, block = lane / 16u, index = lane % 16u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane((threadIdx.x + PROJECTION_TILE_THREADS * threadIdx.y) / WAVE);
-    const uint32_t H = arguments.hidden, stages = H / PROJECTION_STAGE_INPUTS, pairs = (stages + 1u) / 2u;
+    const uint32_t H = arguments.hidden, stages = H / PROJECTION_STAGE_INPUTS;
     const uint32_t first_expert = blockIdx.x * 16u, first_row = blockIdx.y * 16u;
     const uint32_t window_address = (uint32_t)(uintptr_t)(lds_bytes)window;
     /* this wavefront brings four experts' rows of a stage (the first four) or four rows (a row past the last repeats the last) */
@@ -484,16 +487,19 @@ extern "C" __global__ void __launch_bounds__(2u * PROJECTION_TILE_THREADS)
     /* this wavefront's loads of the first pair have landed, then every wavefront's */
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2u * (PROJECTION_SPLIT_PAIRS - 1u)) : "memory");
     __syncthreads();
-    split_read<0>(at, 0u, inputs[0]);
-    uint32_t place = 0;
-    for (uint32_t pair = 0; pair < pairs; pair++) {
-        split_landed(inputs[0]);
-        split_read<1>(at, place, inputs[1]);
-        __builtin_amdgcn_sched_barrier(0);
+    const auto multiply = [&](const struct split_inputs &of) {
 #pragma unroll
         for (uint32_t i = 0; i < 4u; i++) {
-            chain = __builtin_amdgcn_mfma_f32_16x16x1f32(inputs[0].w[i], inputs[0].x[i], chain, 0, 0, 0);
+            chain = __builtin_amdgcn_mfma_f32_16x16x1f32(of.w[i], of.x[i], chain, 0, 0, 0);
         }
+    };
+    split_read<0>(at, 0u, inputs[0]);
+    split_landed(inputs[0]);
+    uint32_t place = 0;
+    for (uint32_t pair = 0; pair < stages / 2u; pair++) {
+        split_read<1>(at, place, inputs[1]);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(inputs[0]);
         __builtin_amdgcn_sched_barrier(0);
         /* every wavefront has read the pair, whose place the one to ask for takes; the next pair has landed */
         split_landed(inputs[1]);
@@ -503,15 +509,13 @@ extern "C" __global__ void __launch_bounds__(2u * PROJECTION_TILE_THREADS)
         place = place + PAIR_BYTES < PROJECTION_SPLIT_PAIRS * PAIR_BYTES ? place + PAIR_BYTES : 0u;
         split_read<0>(at, place, inputs[0]);
         __builtin_amdgcn_sched_barrier(0);
-        if (2u * pair + 1u < stages) {
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; i++) {
-                chain = __builtin_amdgcn_mfma_f32_16x16x1f32(inputs[1].w[i], inputs[1].x[i], chain, 0, 0, 0);
-            }
-        }
+        multiply(inputs[1]);
         __builtin_amdgcn_sched_barrier(0);
+        split_landed(inputs[0]);
     }
-    split_landed(inputs[0]);
+    if (stages % 2u != 0u) { /* a last stage alone */
+        multiply(inputs[0]);
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* the last pairs' repeats */
     __syncthreads();
     /* register v = 4 b + r is chain 4 wave + b of expert 4 (lane / 16) + r and row lane % 16. Every wavefront leaves its four
