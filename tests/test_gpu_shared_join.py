@@ -272,6 +272,27 @@ def test_shared_join_of_any_slots(amd, card, rows, slices, per_row):
     assert results[0] == results[1]
 
 
+@pytest.mark.parametrize("rows,slices,per_row", [(4, 1, 15), (4, 2, 16), (3, 4, 17), (2, 2, 24), (2, 1, 31), (1, 8, 64)])
+def test_joins_of_groups_of_slots(amd, card, rows, slices, per_row):
+    """More slots than are asked for together: whole groups of eight, a part of one behind them. The shared join against the separate
+    launches, and expert_join against the oracle, every bit."""
+    test_shared_join_of_any_slots(amd, card, rows, slices, per_row)
+    card.cursor = 256
+    hidden = 1024
+    layer, shared, _ = build(amd, card, hidden, 256, 8, 8, 15)
+    layer.P = per_row
+    pairs, output = to_bf16(normals(36, 64 * hidden) * 2.0).reshape(64, hidden), to_bf16(normals(37, 8 * hidden)).reshape(8, hidden)
+    streams, post, comb = site_of(38, 8, hidden)
+    card.upload(layer.ranges["pair_output"].byte_offset, pairs)
+    card.upload(shared.ranges["output"].byte_offset, output)
+    shared.set_site(streams, post, comb)
+    card.run(shared.join_launch(rows))
+    want, sums = streams.copy(), np.zeros((rows, hidden), dtype=np.float32)
+    orc.orc_expert_join(ptr(pairs, u16p), ptr(output, u16p), ptr(want, u16p), ptr(post, f32p), ptr(comb, f32p), ptr(sums, f32p), rows, per_row, hidden)
+    assert np.array_equal(shared.read("streams", np.uint16).reshape(8, STREAMS, hidden), want)
+    assert np.array_equal(shared.read("row_sums", np.uint32).reshape(8, hidden)[:rows], sums.view(np.uint32))
+
+
 def test_layer_with_shared_expert_and_join_against_oracle(amd, card):
     """The whole FFN site of a wide step: routed experts in their wide form, the shared expert in its interleaved form,
     the join; streams against the oracle's join of the oracle's own routed and shared outputs."""
