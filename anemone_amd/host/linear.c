@@ -636,6 +636,18 @@ static bool native_takes_whole_bytes(const struct matrix_shape_record *shape, ui
     return pairs >= NATIVE_WHOLE_PAIRS * experts && shape->output_size >= outputs / 2u && 8u * whole <= 9u * half;
 }
 
+/* Whether the record names a kernel of its own there: a member that the others do not repeat. Members that a caller left zero hold the
+ * handle of whatever kernel was prepared first, the same in all of them. */
+static bool native_has(const struct linear_native_kernels_record *kernels, uint32_t handle)
+{
+    uint32_t handles[sizeof *kernels / sizeof(uint32_t)], named = 0;
+    memcpy(handles, kernels, sizeof handles);
+    for (uint32_t i = 0; i < sizeof handles / sizeof handles[0]; i++) {
+        named += handles[i] == handle ? 1u : 0u;
+    }
+    return handle != BACKEND_NO_KERNEL && named == 1u;
+}
+
 /* block128: the launches of WEIGHT_FORMAT_E4M3_BLOCK128 experts (four: the hidden vectors' quantizer is a launch of its
  * own between the products); else those of the reference's formats (three) */
 static result_status wide_experts_prepare(const struct linear_wide_experts_description *description, uint64_t arena_byte_count,
@@ -732,13 +744,13 @@ static result_status wide_experts_prepare(const struct linear_wide_experts_descr
                                                             down->output_size, experts->pairs_per_row};
     uint32_t block_outputs = 4u * strip_outputs, gate_up_outputs = bytes ? WIDE_GATE_UP_E4M3_BLOCK_OUTPUTS : WIDE_GATE_UP_BLOCK_OUTPUTS;
     if (native && !bytes) { /* 4-bit weights in gfx950's lane order: strips of twice the tiles, or of as many */
-        if (native_kernels->native_expert_gate_up_narrow != BACKEND_NO_KERNEL &&
+        if (native_has(native_kernels, native_kernels->native_expert_gate_up_narrow) &&
             native_takes_narrow(gate_up, gate_up_outputs, description->tile_count, pairs)) {
             gate_up_kernel = native_kernels->native_expert_gate_up_narrow;
         } else {
             gate_up_outputs *= 2u;
         }
-        if (native_kernels->native_expert_down_narrow != BACKEND_NO_KERNEL &&
+        if (native_has(native_kernels, native_kernels->native_expert_down_narrow) &&
             native_takes_narrow(down, block_outputs, description->tile_count, pairs)) {
             down_kernel = native_kernels->native_expert_down_narrow;
         } else {
@@ -748,13 +760,13 @@ static result_status wide_experts_prepare(const struct linear_wide_experts_descr
     if (native && bytes) { /* one-byte weights: strips of twice the tiles for many pairs an expert */
         const uint32_t whole_gate_up = block128 ? native_kernels->native_expert_gate_up_b128_whole : native_kernels->native_expert_gate_up_e4m3_whole;
         const uint32_t whole_down = block128 ? native_kernels->native_expert_down_b128_whole : native_kernels->native_expert_down_e4m3_whole;
-        if (whole_gate_up != BACKEND_NO_KERNEL &&
+        if (native_has(native_kernels, whole_gate_up) &&
             native_takes_whole_bytes(gate_up, gate_up_outputs, 768u, description->tile_count, pairs)) {
             gate_up_kernel = whole_gate_up;
             gate_up_outputs *= 2u;
             gate_up_window = NATIVE_WINDOW_BYTES(NATIVE_E4M3_COLUMN_BLOCKS, NATIVE_E4M3_WHOLE_STAGES);
         }
-        if (whole_down != BACKEND_NO_KERNEL && native_takes_whole_bytes(down, block_outputs, 512u, description->tile_count, pairs)) {
+        if (native_has(native_kernels, whole_down) && native_takes_whole_bytes(down, block_outputs, 512u, description->tile_count, pairs)) {
             down_kernel = whole_down;
             block_outputs *= 2u;
             down_window = NATIVE_WINDOW_BYTES(NATIVE_E4M3_COLUMN_BLOCKS, NATIVE_E4M3_WHOLE_STAGES);

@@ -953,6 +953,34 @@ def test_native_one_byte_strips_by_pairs_and_rounds(fake, infix, experts_n, rows
         assert first.dynamic_shared_byte_count == 36864 and second.dynamic_shared_byte_count == (36864 if down else 53248)
 
 
+@pytest.mark.parametrize("rows,weight_format,names", [(1024, "WEIGHT_FORMAT_E4M3_GFX950", ["e4m3_1", "e4m3_1"]), (1024, "WEIGHT_FORMAT_E4M3_BLOCK128_GFX950", ["b128_1", "b128_1"]),
+                                                      (64, "WEIGHT_FORMAT_E2M1_GFX950", ["1", "1"])])
+def test_native_kernels_left_zero_are_never_launched(fake, rows, weight_format, names):
+    """Zero is a kernel's handle: members of the record that a caller left zero count as kernels that are not there, whether
+    the kernel prepared first is one of the record's or of another."""
+    lib = amd.library()
+    fmt, bits = getattr(amd, weight_format), 4 if "E2M1" in weight_format else 8
+    for native_first in (False, True):
+        if native_first:
+            fake.handles.clear()
+        linear, native, launches = amd.LinearKernels(), amd.LinearNativeKernels(), amd.launches_of(4)
+        for prepare, record in ((lib.linear_native_kernels_prepare, native), (lib.linear_kernels_prepare, linear))[::1 if native_first else -1]:
+            assert prepare(fake.address, fake.card, 950, C.byref(record)) == 0
+        for name, _ in amd.LinearNativeKernels._fields_[6:]:
+            setattr(native, name, 0)
+        d = wide_experts_description(fmt, gate_up_shape=amd.Shape(2048, 4096, bits, 0), down_shape=amd.Shape(4096, 2048, bits, 0),
+                                     row_count=rows, tile_count=amd.wide_tile_count(rows, 8, 64))
+        at = 3 << 30
+        for record, name in [(d.experts, name) for name in ("codes", "exponents", "hidden_codes", "hidden_exponents", "hidden_operands", "pair_output", "row_output")] + \
+                [(d, "tiles"), (d, "pairs")]:
+            size = 4 * getattr(record, name).byte_count
+            setattr(record, name, amd.Range(at, size))
+            at += size
+        assert lib.linear_native_experts_prepare(C.byref(d), 8 << 30, C.byref(linear), C.byref(native), launches) == 0
+        got = [fake.handles[launches[i].kernel][1] for i in (0, 2 if "BLOCK128" in weight_format else 1)]
+        assert got == ["native_expert_gate_up_" + names[0], "native_expert_down_" + names[1]], native_first
+
+
 def test_native_kernels_without_the_narrow_ones(fake):
     """A backend without the kernels of narrow strips prepares the others, and every launch is of whole strips."""
     lib, linear, native, launches = amd.library(), amd.LinearKernels(), amd.LinearNativeKernels(), amd.launches_of(4)
