@@ -415,10 +415,11 @@ ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_projection_tiles, router_projection_ar
  * scores. What bounds it: a unit's 256 instructions of 4096 inputs, 33 cycles each, beside 64 LDS reads a stage; the first loads'
  * way from memory; the launch. By four wavefronts of eight chains, words converted and a barrier a stage | so, us, 256 experts of
  * 4096 inputs: 32 rows 10.75 | 9.25, 203 rows 10.85 | 9.45, 300 rows 15.3 | 14.35, 700 rows 21.6 | 20.0 (eight wavefronts with a
- * barrier a stage 9.95 and 22.6). grid (E / 16, ceil(rows / 16)), block (256, 2). */
+ * barrier a stage 9.95 and 22.6). grid (E / 16, ceil(rows / 16)), block (256, 2): 512 threads, the 256
+ * of y = 0 bring the experts' rows of the tile, those of y = 1 the rows. */
 #define PROJECTION_SPLIT_STAGE_BYTES (32u * PROJECTION_STAGE_ROW_BYTES)
 #define PROJECTION_SPLIT_PAIRS 3u
-#define PROJECTION_SPLIT_WAVES (2u * PROJECTION_TILE_THREADS / WAVE)
+#define PROJECTION_SPLIT_WAVES (PROJECTION_SPLIT_SIDES * PROJECTION_TILE_THREADS / WAVE)
 struct split_inputs {
     float w[4], x[4]; /* of a stage's four groups; the lower halves stay zero */
 };
@@ -446,20 +447,21 @@ __device__ static __forceinline__ void split_landed(struct split_inputs &inputs)
                  : "memory");
 }
 
-extern "C" __global__ void __launch_bounds__(2u * PROJECTION_TILE_THREADS)
+extern "C" __global__ void __launch_bounds__(PROJECTION_SPLIT_SIDES * PROJECTION_TILE_THREADS)
     router_projection_split(struct router_projection_arguments arguments, unsigned char *arena)
 {
     constexpr uint32_t PAIR_BYTES = 2u * PROJECTION_SPLIT_STAGE_BYTES;
     __shared__ __attribute__((aligned(1024))) unsigned char window[PROJECTION_SPLIT_PAIRS * PAIR_BYTES];
     const uint32_t lane = threadIdx.x % WAVE, block = lane / 16u, index = lane % 16u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane((threadIdx.x + PROJECTION_TILE_THREADS * threadIdx.y) / WAVE);
+    const uint32_t side = __builtin_amdgcn_readfirstlane(threadIdx.y), of_side = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const uint32_t wave = PROJECTION_TILE_THREADS / WAVE * side + of_side;
     const uint32_t H = arguments.hidden, stages = H / PROJECTION_STAGE_INPUTS;
     const uint32_t first_expert = blockIdx.x * 16u, first_row = blockIdx.y * 16u;
     const uint32_t window_address = (uint32_t)(uintptr_t)(lds_bytes)window;
-    /* this wavefront brings four experts' rows of a stage (the first four) or four rows (a row past the last repeats the last) */
-    const uint32_t line = 4u * (wave % 4u) + lane / 16u, last_row = arguments.row_count - 1u - first_row;
-    const unsigned char *base = arena + (wave < 4u ? arguments.weights_offset + (uint64_t)first_expert * H * 2u : arguments.rows_offset + (uint64_t)first_row * H * 2u);
-    const uint32_t own = 16u * ((lane % 16u) ^ line) + (wave < 4u || line < last_row ? line : last_row) * (H * 2u);
+    /* this wavefront brings four experts' rows of a stage (side 0) or four rows (a row past the last repeats the last) */
+    const uint32_t line = 4u * of_side + lane / 16u, last_row = arguments.row_count - 1u - first_row;
+    const unsigned char *base = arena + (side == 0u ? arguments.weights_offset + (uint64_t)first_expert * H * 2u : arguments.rows_offset + (uint64_t)first_row * H * 2u);
+    const uint32_t own = 16u * ((lane % 16u) ^ line) + (side == 0u || line < last_row ? line : last_row) * (H * 2u);
     const uint32_t lands_at = window_address + wave * 1024u;
     /* a stage past the last is the last again, into a place that nobody reads any more: every wait counts the same */
     auto ask = [&](uint32_t pair, uint32_t place) {
@@ -528,7 +530,7 @@ extern "C" __global__ void __launch_bounds__(2u * PROJECTION_TILE_THREADS)
                                                              __fadd_rn(0.0f, chain[12u + r])};
     }
     __syncthreads();
-    if (wave >= 4u || first_row + index >= arguments.row_count) {
+    if (side != 0u || first_row + index >= arguments.row_count) {
         return;
     }
     float4_t part[PROJECTION_SPLIT_WAVES];

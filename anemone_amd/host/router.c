@@ -283,7 +283,7 @@ result_status router_projection_prepare(const struct router_projection_descripti
             launch_fill(launch_out, kernels->projection_split, description->expert_count / 16u,
                         (description->row_count + PROJECTION_SPLIT_ROWS - 1u) / PROJECTION_SPLIT_ROWS, 1, PROJECTION_TILE_THREADS, 0, &record,
                         sizeof record);
-            launch_out->block[1] = 2u;
+            launch_out->block[1] = PROJECTION_SPLIT_SIDES;
             return STATUS_OK;
         }
         if (has_tiles && (has_split || description->row_count >= PROJECTION_TILE_LEAST_ROWS)) {
@@ -293,7 +293,7 @@ result_status router_projection_prepare(const struct router_projection_descripti
             return STATUS_OK;
         }
     }
-    /* a thin step: a row a block (the kernel takes one or four by its block's threads) */
+    /* a thin step: a row a block (the kernel asks router_projection_by_row of the same record) */
     const uint32_t expert_blocks = (description->expert_count + PROJECTION_OUTPUTS - 1u) / PROJECTION_OUTPUTS;
     const bool by_row = router_projection_by_row(description->row_count, description->expert_count) != 0u;
     launch_fill(launch_out, kernels->projection, expert_blocks,

@@ -126,6 +126,7 @@ ANEMONE_INLINE uint32_t router_projection_by_row(uint32_t row_count, uint32_t ex
 #define PROJECTION_TILE_LEAST_ROWS 257u /* of a backend without router_projection_split; fewer rows then take router_projection */
 #define KERNEL_ROUTER_PROJECTION_SPLIT "router_projection_split" /* and with a tile's chains over a block's wavefronts */
 #define PROJECTION_SPLIT_ROWS 16u       /* rows of a block of router_projection_split */
+#define PROJECTION_SPLIT_SIDES 2u       /* block[1] of router_projection_split: PROJECTION_TILE_THREADS threads that bring the experts' rows, as many the rows */
 #define PROJECTION_SPLIT_LEAST_ROWS 9u  /* up to eight rows router_projection takes a row a block, in blocks of eight experts */
 /* Which of the two takes a step of more rows. A block of router_projection_tiles is a score's 32 chains in one wavefront, so a
  * launch takes as long as the blocks that fall to one of the 256 CUs, one behind the other in all but the loads; a block of

@@ -333,6 +333,21 @@ def test_router_projection_prepare_geometry(fake):
     assert prepared(300, 48, 64)[0] == 1 and prepared(0, 512, 64)[0] == 1  # a width that is no multiple of 32; no row
 
 
+@pytest.mark.parametrize("rows,hidden,experts_n,name,block,window", [
+    (8, 4096, 256, "router_projection", [256, 1, 1], 9 * (4096 + 32) * 2),  # a row a block
+    (300, 160, 64, "router_projection", [128, 1, 1], 12 * 1024 * 2),        # four rows a block
+    (300, 512, 64, "router_projection_split", [256, 2, 1], 0),              # 512 threads: the experts' rows by 256, the rows by 256
+    (4096, 4096, 256, "router_projection_tiles", [256, 1, 1], 0)])
+def test_router_projection_threads(fake, rows, hidden, experts_n, name, block, window):
+    """Every dimension of a projection's block, and the shared memory asked for: a kernel forms neither of the launch."""
+    lib, kernels, launch = amd.library(), amd.RouterKernels(), amd.launches_of(1)
+    assert lib.router_kernels_prepare(fake.address, fake.card, C.byref(kernels)) == 0
+    d = amd.RouterProjectionDescription(amd.Range(1 << 20, experts_n * hidden * 2), amd.Range(1 << 24, rows * hidden * 2),
+                                        amd.Range(1 << 27, rows * experts_n * 4), rows, hidden, experts_n, 0)
+    assert lib.router_projection_prepare(C.byref(d), ARENA, C.byref(kernels), launch) == 0
+    assert (fake.handles[launch[0].kernel][1], list(launch[0].block), launch[0].dynamic_shared_byte_count) == (name, block, window)
+
+
 def test_router_prepare(fake):
     lib = amd.library()
     kernels = amd.RouterKernels()
