@@ -10,6 +10,8 @@
 
 #include "exl3_device.cuh"
 
+#include "publish_device.cuh"
+
 #define DENSE_GROUP_LANES 32u
 #define DENSE_GROUPS (DENSE_THREADS_VALUE / DENSE_GROUP_LANES)
 #define DENSE_DIES 8u
@@ -191,8 +193,7 @@ __device__ static __forceinline__ void dense_linear_body(const struct dense_line
     }
     const uint64_t index = (uint64_t)(first_row + r) * arguments.output_size + first_output + o;
     if constexpr (FRONT) { /* a float32 that another block of this launch reads: through to where every die sees it */
-        __hip_atomic_store((float *)(arena + arguments.output_offset) + index, __fmul_rn(sum, arguments.output_scale), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+        store_through((float *)(arena + arguments.output_offset) + index, __fmul_rn(sum, arguments.output_scale));
     } else if (arguments.output_type == DENSE_FLOAT32) {
         ((float *)(arena + arguments.output_offset))[index] = __fmul_rn(sum, arguments.output_scale);
     } else {

@@ -6,6 +6,7 @@
 #define HYPER_DEVICE_CUH
 
 #include "join_device.cuh"
+#include "publish_device.cuh"
 
 __device__ static __forceinline__ float hyper_group_sum(float value)
 {
@@ -96,7 +97,7 @@ __device__ static __forceinline__ void hyper_row_input_body(const struct hyper_f
 #pragma unroll
         for (uint32_t half = 0; half < 2u; half++) {
             const uint64_t words = (uint64_t)packed[2u * half + 1u] << 32 | packed[2u * half];
-            __hip_atomic_store((uint64_t *)out + half, words, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            store_through((uint64_t *)out + half, words);
         }
     } else {
         *out = packed;

@@ -50,16 +50,16 @@ __device__ static __forceinline__ uint32_t front_add(uint32_t *counter)
     return __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-/* Every thread of the block calls; the old value of the counter, on every thread. RELEASE: what the block's threads stored by
- * relaxed stores of agent scope, which go through the level 2 cache of their die, is there before the counter moves (every
- * thread waits for its own, then the block meets). What other blocks read is a row, a few mixes or scores: written back with
+/* Every thread of the block calls; the old value of the counter, on every thread. STORED_THROUGH: what the block's threads published by
+ * store_through, and that alone, is there for every die before the counter moves (every thread waits for its own stores, then
+ * the block meets): this is no release of plain stores. What other blocks read is a row, a few mixes or scores: written back with
  * all else that the die's cache holds, by a release of agent scope, each of a front's two publications in line took 0.7 us
  * (ffn_front_8 at five rows 15.5 -> 14.1). ACQUIRE: what the earlier publishers stored is visible to the block's threads
  * behind the call (thread 0 drops the stale lines once for all). */
-template <bool RELEASE, bool ACQUIRE>
+template <bool STORED_THROUGH, bool ACQUIRE>
 __device__ static __forceinline__ uint32_t front_publish(uint32_t *counter, uint32_t thread, uint32_t *word)
 {
-    if (RELEASE) {
+    if (STORED_THROUGH) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     }

@@ -172,6 +172,49 @@ def test_a_wait_that_cannot_end_gives_up_and_every_block_leaves(amd, card):
     assert not front.read("scratch", np.uint8)[16 + 768:16 + 776].any()
 
 
+@pytest.mark.parametrize("rows,width", [(1, 4096), (5, 4096), (8, 2048)])
+def test_fronts_of_consecutive_steps(amd, card, rows, width):
+    """Fronts of a number of steps in a row, over the same ranges and with other streams in each: what a block reads of another
+    block's (rows, mixes, scores) is this step's, whichever die wrote it. Every output against the separate launches."""
+    say("fronts of consecutive steps", rows, width)
+    experts_n, picks, steps = 64, 4, 6
+    layer = fp4_layer(amd, card, width, 256, experts_n, picks, rows)
+    mix_weights = (normals(80, MIXES * STREAMS * width) * 0.02).astype(np.float32).reshape(MIXES, STREAMS * width)
+    front = amd.SiteFront(card, rows, width, mix_weights, np.array([1.0, 0.8, 1.2], np.float32), (normals(81, MIXES) * 0.5).astype(np.float32),
+                          to_bf16(normals(82, width) * 0.1 + 1.0), hidden_range=amd.Range(layer.x_offset, rows * width * 2))
+    layer.set_rows(np.zeros((rows, width), np.uint16), rows)
+    inputs = [(to_bf16(normals(90 + step, rows * STREAMS * width) * (1.0 + step)).reshape(rows, STREAMS, width),
+               (np.abs(normals(190 + step, rows * STREAMS)) * 0.3 + 0.1).astype(np.float32).reshape(rows, STREAMS)) for step in range(steps)]
+    fused = front.front_launch(rows, layer)
+    scores_range, jobs_range = amd.Range(layer.scores_offset, rows * experts_n * 4), layer.experts_description().jobs
+    scores = front.dense_launch(amd.Range(layer.router_offset, experts_n * width * 2), amd.Range(layer.x_offset, rows * width * 2), scores_range,
+                                experts_n, width, amd.DENSE_BFLOAT16, amd.DENSE_FLOAT32, 0, 1.0, 0.0, rows)
+    kernels = amd.LinearKernels()
+    amd.check(card.lib.linear_kernels_prepare(amd.backend_table(), card.handle, amd.ARITHMETIC_CLASS_GFX950, C.byref(kernels)), "linear_kernels_prepare")
+    q = amd.QuantizeDescription(front.ranges["hidden"], front.ranges["codes"], front.ranges["exponents"], front.ranges["operands"], width, rows)
+    quantize = amd.launches_of(1)
+    amd.check(card.lib.linear_quantize_prepare(C.byref(q), card.arena_bytes, C.byref(kernels), quantize), "linear_quantize_prepare")
+    ranges = dict(front.ranges)
+    ranges["scores"], ranges["affinities"] = scores_range, amd.Range(layer.affinities_offset, rows * experts_n * 4)
+    ranges["jobs"] = amd.Range(jobs_range.byte_offset, jobs_range.byte_count)
+    outputs = SITE_OUTPUTS + ("scores", "affinities", "jobs")
+    separate = [front.mix_project_launch(rows), front.site_launches(rows)[:1], scores, layer.select_launch(0), quantize]
+    wanted = []
+    for streams, carried in inputs:
+        front.set_streams(streams, carried)
+        for launches in separate:
+            card.run(launches)
+        wanted.append(snapshot(card, ranges, outputs))
+    assert wanted[0]["scores"].tobytes() != wanted[1]["scores"].tobytes() and wanted[0]["jobs"].tobytes() != wanted[1]["jobs"].tobytes()
+    for _ in range(2):
+        for (streams, carried), want in zip(inputs, wanted):
+            front.set_streams(streams, carried)
+            card.run(fused)
+            got = snapshot(card, ranges, outputs)
+            for name in outputs:
+                assert got[name].tobytes() == want[name].tobytes(), (name, np.flatnonzero(got[name] != want[name])[:8])
+
+
 def fp4_layer(amd, card, hidden, inner, experts_n, picks, rows, distinct=4, **keywords):
     from anemone_amd import workloads
     trios = [[workloads.fp4_matrix(9000 + 3 * e, inner, hidden), workloads.fp4_matrix(9001 + 3 * e, inner, hidden),
