@@ -620,20 +620,37 @@ static bool native_takes_narrow(const struct matrix_shape_record *shape, uint32_
  * well and the matrix holds a whole strip of a wavefront. A strip's block brings its tile's columns into LDS again, so that the
  * fewer strips the fewer bytes pass the level-2 caches; but a block of many pairs is a long one, and where a few experts hold most
  * of them the launch ends on it. Half strips / whole ones, us, float32 scales, gate/up and down: 4096 x 2048 x 256 experts, 64 pairs
- * an expert 811 / 786 and 422 / 433, under loads of Zipf(1.1) 823 / 879 and 463 / 478; 94 pairs 885 / 798 and 470 / 440; 128 pairs
- * 1105 / 985 and 598 / 539, Zipf 1123 / 1058 and 627 / 586; 2048 x 2048 x 64 at 87 Zipf 115 / 128 and 77 / 70; 2048 x 896 x 64 at
- * 141 90 / 77 and 50 / 49; 2048 x 1024 x 256 at 128 Zipf 313 / 276 and 216 / 169; 4096 x 2048 x 64 at 256 Zipf 442 / 399 and 252 /
- * 214. E8M0 scales: 4096 x 2048 x 256 at 128 1128 / 988 and 570 / 536, Zipf 1164 / 1103 and 613 / 606; 2048 x 1024 x 256 at 128
- * Zipf 345 / 279 and 208 / 167; 2048 x 2048 x 64 at 87 Zipf 123 / 128 and 74 / 69. */
+ * an expert 811 / 786 and 422 / 433, under loads of Zipf(1.1) 823 / 879 and 463 / 478; 96 pairs 893 / 805 and 474 / 441, Zipf 969 /
+ * 965 and 553 / 534; 128 pairs 1105 / 985 and 598 / 539, Zipf 1123 / 1058 and 627 / 586; 2048 x 1024 x 256 at 96 347 / 226 and 218 /
+ * 134, Zipf 268 / 249 and 173 / 148; 3072 x 1024 x 128 at 96 Zipf 196 / 182 and 115 / 109; 4096 x 2048 x 64 at 256 Zipf 447 / 405 and
+ * 254 / 217. E8M0 scales: 4096 x 2048 x 256 at 96 Zipf 1032 / 1020 and 538 / 552, at 128 1128 / 988 and 570 / 536, Zipf 1164 / 1103 and
+ * 613 / 606; 5120 x 1024 x 384 at 96 Zipf 1064 / 940 and 588 / 560.
+ * Strips in whole 32 are dealt evenly to the dies' engines as half strips too (sixteen and fewer leave engines idle beside a run's
+ * second tile, which has no block of its own), so that only the columns are gained, and in launches of few blocks Zipf loads
+ * lose it: those begin at NATIVE_WHOLE_DEALT_PAIRS. Gate/up or down of such strips, float32 scales, Zipf at 96 / 108 / 120 / 128 pairs:
+ * 4096 x 2048 x 64 gate/up 234 / 243, 244 / 245, 259 / 254, 275 / 263 (even loads at 96: 221 / 200); 5120 x 2048 x 64 at 96 294 / 311, at
+ * 128 355 / 348; 2048 x 2048 x 128 at 96 246 / 255, at 128 291 / 284; down of 4096 x 1536 x 64 at 96 105 / 110, at 128 124 / 117. E8M0
+ * scales: 4096 x 2048 x 64 at 96 239 / 246 and 127 / 130, at 128 283 / 265 and 147 / 143.
+ * few_blocks: a launch whose chains are short against their blocks' ends, gate/up of float32 scales and fewer than
+ * NATIVE_WHOLE_LONG_INPUTS inputs, takes whole strips from 24 half strips on only where they are more blocks than this. Zipf,
+ * 64 experts of 2048 inputs: 1536 outputs at 144 (864 blocks), 160 (960) and 224 pairs (1344) 116 / 126, 123 / 136 and 158 / 156; 1792
+ * at 144 (1008), 176 (1232) and 224 (1568) 134 / 147, 150 / 152 and 179 / 177; 2048 at 120 (1024), 160 (1280) and 176 (1408) 131 / 139, 158 /
+ * 162 and 168 / 164; of 4096 inputs 1536 outputs at 160 242 / 230; E8M0 scales, 2048 inputs, 1536 outputs at 160 143 / 139. */
 #define NATIVE_WHOLE_PAIRS 96u
-static bool native_takes_whole_bytes(const struct matrix_shape_record *shape, uint32_t outputs, uint32_t resident, uint32_t tile_count, uint64_t pairs)
+#define NATIVE_WHOLE_DEALT_PAIRS 128u
+#define NATIVE_WHOLE_LONG_INPUTS 4096u
+#define NATIVE_WHOLE_FEW_BLOCKS 1280u
+static bool native_takes_whole_bytes(const struct matrix_shape_record *shape, uint32_t outputs, uint32_t resident, uint32_t tile_count, uint64_t pairs,
+                                     uint32_t few_blocks)
 {
     const uint64_t pairs_tiles = (pairs + WIDE_TILE_PAIRS - 1u) / WIDE_TILE_PAIRS;
     const uint64_t experts = tile_count > pairs_tiles ? tile_count - pairs_tiles : 1u;
     const uint64_t full = (pairs + 2u * WIDE_TILE_PAIRS - 1u) / (2u * WIDE_TILE_PAIRS), groups = full > experts ? full : experts; /* blocks a strip */
     const uint64_t half_strips = ((uint64_t)shape->output_size + outputs - 1u) / outputs, whole_strips = (half_strips + 1u) / 2u;
     const uint64_t half = (half_strips * groups + resident - 1u) / resident * resident, whole = (whole_strips * groups + 511u) / 512u * 1024u;
-    return pairs >= NATIVE_WHOLE_PAIRS * experts && shape->output_size >= outputs / 2u && 8u * whole <= 9u * half;
+    const bool dealt = half_strips % 32u == 0u && whole_strips * groups < 8u * 512u;
+    return pairs >= (dealt ? NATIVE_WHOLE_DEALT_PAIRS : NATIVE_WHOLE_PAIRS) * experts && shape->output_size >= outputs / 2u && 8u * whole <= 9u * half &&
+           (half_strips < 24u || whole_strips * groups > few_blocks);
 }
 
 /* Whether the record names a kernel of its own there: a member that the others do not repeat. Members that a caller left zero hold the
@@ -760,13 +777,14 @@ static result_status wide_experts_prepare(const struct linear_wide_experts_descr
     if (native && bytes) { /* one-byte weights: strips of twice the tiles for many pairs an expert */
         const uint32_t whole_gate_up = block128 ? native_kernels->native_expert_gate_up_b128_whole : native_kernels->native_expert_gate_up_e4m3_whole;
         const uint32_t whole_down = block128 ? native_kernels->native_expert_down_b128_whole : native_kernels->native_expert_down_e4m3_whole;
+        const uint32_t few_blocks = block128 && gate_up->input_size < NATIVE_WHOLE_LONG_INPUTS ? NATIVE_WHOLE_FEW_BLOCKS : 0u;
         if (native_has(native_kernels, whole_gate_up) &&
-            native_takes_whole_bytes(gate_up, gate_up_outputs, 768u, description->tile_count, pairs)) {
+            native_takes_whole_bytes(gate_up, gate_up_outputs, 768u, description->tile_count, pairs, few_blocks)) {
             gate_up_kernel = whole_gate_up;
             gate_up_outputs *= 2u;
             gate_up_window = NATIVE_WINDOW_BYTES(NATIVE_E4M3_COLUMN_BLOCKS, NATIVE_E4M3_WHOLE_STAGES);
         }
-        if (native_has(native_kernels, whole_down) && native_takes_whole_bytes(down, block_outputs, 512u, description->tile_count, pairs)) {
+        if (native_has(native_kernels, whole_down) && native_takes_whole_bytes(down, block_outputs, 512u, description->tile_count, pairs, 0u)) {
             down_kernel = whole_down;
             block_outputs *= 2u;
             down_window = NATIVE_WINDOW_BYTES(NATIVE_E4M3_COLUMN_BLOCKS, NATIVE_E4M3_WHOLE_STAGES);

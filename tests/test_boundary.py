@@ -996,6 +996,37 @@ def test_native_kernels_left_zero_are_never_launched(fake, rows, weight_format, 
         assert got == ["native_expert_gate_up_" + names[0], "native_expert_down_" + names[1]], native_first
 
 
+@pytest.mark.parametrize("experts_n,rows,hidden,inner,gate_up,gate_up_b128,down", [
+    (64, 1023, 4096, 2048, "", "", ""),                     # 32 half strips either way: a pair below 128 an expert
+    (64, 1024, 4096, 2048, "whole_", "whole_", "whole_"),
+    (128, 1536, 4096, 2048, "", "", ""),                    # 96 pairs an expert: 2048 whole blocks; 256 experts, 4096 blocks, take them
+    (64, 768, 2048, 2048, "", "", "whole_"),                # down: sixteen half strips
+    (64, 768, 4096, 1024, "whole_", "whole_", ""),          # and gate/up
+    (64, 1280, 2048, 1536, "whole_", "", ""),               # short chains of 960 whole blocks
+    (64, 1792, 2048, 1536, "whole_", "whole_", "whole_"),   # of 1344
+    (64, 1280, 2048, 2048, "whole_", "", ""),               # of 1280
+    (64, 1280, 4096, 1536, "whole_", "whole_", "")])        # chains of 32 steps
+@pytest.mark.parametrize("infix", ["e4m3", "b128"])
+def test_native_one_byte_strips_under_uneven_loads(fake, infix, experts_n, rows, hidden, inner, gate_up, gate_up_b128, down):
+    """Where loads of Zipf lose what even ones gain, strips of twice the tiles begin later (host/linear.c has both sides' times)."""
+    lib, linear, native, launches = amd.library(), amd.LinearKernels(), amd.LinearNativeKernels(), amd.launches_of(4)
+    block128 = infix == "b128"
+    assert lib.linear_kernels_prepare(fake.address, fake.card, 950, C.byref(linear)) == 0
+    assert lib.linear_native_kernels_prepare(fake.address, fake.card, 950, C.byref(native)) == 0
+    d = wide_experts_description(amd.WEIGHT_FORMAT_E4M3_BLOCK128_GFX950 if block128 else amd.WEIGHT_FORMAT_E4M3_GFX950,
+                                 gate_up_shape=amd.Shape(inner, hidden, 8, 0), down_shape=amd.Shape(hidden, inner, 8, 0),
+                                 row_count=rows, tile_count=amd.wide_tile_count(rows, 8, experts_n))
+    at = 3 << 30
+    for record, name in [(d.experts, name) for name in ("codes", "exponents", "hidden_codes", "hidden_exponents", "hidden_operands", "pair_output", "row_output")] + \
+            [(d, "tiles"), (d, "pairs")]:
+        size = 4 * getattr(record, name).byte_count
+        setattr(record, name, amd.Range(at, size))
+        at += size
+    assert lib.linear_native_experts_prepare(C.byref(d), 8 << 30, C.byref(linear), C.byref(native), launches) == 0
+    got = [fake.handles[launches[i].kernel][1] for i in (0, 2 if block128 else 1)]
+    assert got == ["native_expert_gate_up_%s_%s1" % (infix, gate_up_b128 if block128 else gate_up), "native_expert_down_%s_%s1" % (infix, down)]
+
+
 def test_native_kernels_without_the_narrow_ones(fake):
     """A backend without the kernels of narrow strips prepares the others, and every launch is of whole strips."""
     lib, linear, native, launches = amd.library(), amd.LinearKernels(), amd.LinearNativeKernels(), amd.launches_of(4)
