@@ -238,11 +238,10 @@ ANEMONE_RECORD_HAS(router_wide_arguments, 136);
  * launch (2.7 -> 3.7 us of the calling thread; a single matrix of three launches then waited for the thread) */
 ANEMONE_INLINE uint32_t exl3_element_rows(uint32_t pair_count, uint32_t job_count)
 {
-    uint32_t rows = 1u;
-    for (uint32_t more = 2u; more <= LINEAR_MAXIMUM_ROWS; more++) {
-        rows += more * job_count <= pair_count ? 1u : 0u; /* the jobs are a grid's rows: at most 65,535 */
-    }
-    return rows;
+    const uint32_t four = 4u * job_count <= pair_count ? 4u : 0u;
+    const uint32_t two = four + ((four + 2u) * job_count <= pair_count ? 2u : 0u);
+    const uint32_t one = two + ((two + 1u) * job_count <= pair_count ? 1u : 0u);
+    return 8u * job_count <= pair_count ? 8u : one != 0u ? one : 1u; /* the jobs are a grid's rows: at most 65,535 */
 }
 #define EXL3_STRIP_TILES 8u      /* output tiles of a block of the chain's product launches: 128 outputs */
 #define EXL3_THIN_STRIP_TILES 1u /* of the _thin and _thin_many instances */

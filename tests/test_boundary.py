@@ -118,6 +118,18 @@ def chain_record(**changes):
     return r
 
 
+def test_chain_element_wise_blocks(fake):
+    """A wavefront a row of a job, as many as the jobs hold on average, one to eight: the block of the three element-wise launches."""
+    lib, launches = amd.library(), amd.launches_of(5)
+    for jobs in (1, 2, 3, 7, 64, 1000, 65535):
+        for pairs in sorted({max(1, jobs * rows + beside) for rows in range(0, 11) for beside in (-1, 0, 1)}):
+            r = chain_record(job_count=jobs, pair_count=pairs, pairs_per_row=1, input_size=128, inner_size=128, hidden_offset=8 << 30,
+                             input_offset=2 << 30, operands_offset=4 << 30, products_offset=6 << 30, output_offset=6 << 30)
+            assert lib.exl3_experts_prepare(C.byref(r), 16 << 30, fake.address, fake.card, 950, launches) == 0
+            want = 64 * min(8, max(1, pairs // jobs))
+            assert [launches[i].block[0] for i in (0, 2, 4)] == [want] * 3, (jobs, pairs)
+
+
 def test_chain_prepare_geometry(fake):
     lib = amd.library()
     launches = amd.launches_of(5)
