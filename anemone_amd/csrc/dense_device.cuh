@@ -72,7 +72,9 @@ __device__ static __forceinline__ void dense_linear_body(const struct dense_line
     struct chunk_loads {
         uint4_t rows[ROWS], weights[OUTPUTS][WEIGHT_LOADS];
     };
-    /* every row's chunk and every output's weights are asked for before any is used: a chunk costs one trip to memory, not one a row */
+    /* every row's chunk and every output's weights are asked for before any is used: a chunk costs one trip to memory, not one a row.
+     * Asked for and added in two functions: written as one loop body, the front's row loop took 129 registers in place of 116
+     * (ffn_front_8 at 5 rows 14.3 -> 15.95 us, at 8 of 5120 by 384 experts 19.3 -> 25.7) */
     const auto ask = [&](uint32_t chunk, chunk_loads &into) {
 #pragma unroll
         for (uint32_t r = 0; r < ROWS; r++) {

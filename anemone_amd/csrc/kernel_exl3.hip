@@ -52,8 +52,8 @@ __device__ static __forceinline__ uint32_t chain_width(const struct exl3_expert_
 /* The element-wise launches (input, activate, finish): a block is 128 channels of one job, a wavefront one of its rows, or more
  * where the job has more rows than the block wavefronts: rows one behind the other in one wavefront are a chain of their
  * transforms (one 4096-wide matrix by eight rows: input 4.7 -> 2.3 us, finish 3.4 -> 2.2). The step to a wavefront's next row is
- * formed behind a row: ahead of the first it stood in the chain of a launch of one row (input 2.23 -> 2.16 us, the matrix's three
- * launches 10.0 -> 9.85). */
+ * formed behind a row: ahead of the first it stood in the chain of a launch of one row (input 2.22 -> 2.17 us, the matrix's three
+ * launches 10.1 -> 10.0). */
 __device__ static __forceinline__ uint32_t element_stride(const struct exl3_expert_record &record)
 {
     uint32_t jobs = record.job_count;

@@ -193,8 +193,9 @@ ANEMONE_KERNEL(KERNEL_FILE_NATIVE_LINEAR, native_expert_down_b128_1, wide_expert
  * serves four matrix instructions; two sets of weights and two stages at two wavefronts a SIMD (244 to 253 registers, 128 of
  * them sums); the blocks in the order of runs, where each is a longer piece of work and the look at the table counts less. For
  * launches of many pairs an expert (native_takes_whole_bytes, with both sides' times): at 64 pairs an expert a launch is near
- * what memory gives and three wavefronts a SIMD hide more, at 128 half of what passes the level-2 caches were columns (4096
- * rows of 4096 x 2048 x 256 experts, float32 scales: gate/up 1105 -> 985 us, down 598 -> 539). */
+ * what memory gives and three wavefronts a SIMD hide more, at 128 columns were 45 % of the lines that passed the level-2 caches
+ * (4096 rows of 4096 x 2048 x 256 experts, float32 scales: gate/up 1105 -> 985 us, 9.4e7 -> 7.3e7 lines, 7.3 -> 5.2 GB fetched; down
+ * 598 -> 539 us, 4.8e7 -> 3.7e7 lines). */
 #define NATIVE_BYTES_WHOLE_WAVES 2
 extern "C" __global__ void __launch_bounds__(NATIVE_THREADS, NATIVE_BYTES_WHOLE_WAVES) native_expert_gate_up_e4m3_whole_1(struct wide_expert_gate_up_arguments arguments, unsigned char *arena)
 {

@@ -130,7 +130,10 @@ __device__ static __forceinline__ void projection_load_to_lds(const void *lane_a
  * lane i receives value i of each). A wavefront that has a vector unit to itself issues an instruction in six cycles whatever it
  * is and has fifteen LDS reads on their way at most, so both are what counts: by single reads of 16 bits 4.9 us, by these 4.0
  * (one row of 4096 inputs by 256 experts; two chains a lane, through registers and in chunks of 1024: 5.5; eight rows 5.6 -> 4.35,
- * eight of 5120 by 384 experts 7.2 -> 5.7, three of 2048 by 64 3.6 -> 3.0). grid (ceil(E / 8), rows), block 256. */
+ * eight of 5120 by 384 experts 7.2 -> 5.7, three of 2048 by 64 3.6 -> 3.0). A wider row is a chunk behind the other, no chunk on its
+ * way while one is added, and still the faster: eight rows of 7168 by 256 8.35 -> 6.05, of 8192 9.3 -> 6.6, of 12288 by 384 14.75 -> 9.6,
+ * of 16384 by 512 18.95 -> 12.4. A narrower one asks for the same 74 KB of LDS, two blocks a CU: eight of 512 by 256 2.75 -> 2.4, of
+ * 1024 by 1024 (four blocks a CU in two rounds) 4.45 -> 4.35. grid (ceil(E / 8), rows), block 256. */
 #define THIN_EXPERTS 2u /* of a wavefront */
 #define THIN_CHUNK 4096u
 #define THIN_ROW_VALUES (THIN_CHUNK + 32u) /* 64 bytes more: the two experts' chains lie on different banks */
@@ -414,8 +417,8 @@ ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_projection_tiles, router_projection_ar
  * is read behind the instructions of the one before it. The wavefronts' sums meet in LDS at the end, half of them folding the
  * scores. What bounds it: a unit's 256 instructions of 4096 inputs, 33 cycles each, beside 64 LDS reads a stage; the first loads'
  * way from memory; the launch. By four wavefronts of eight chains, words converted and a barrier a stage | so, us, 256 experts of
- * 4096 inputs: 32 rows 10.75 | 9.25, 203 rows 10.85 | 9.45, 300 rows 15.3 | 14.35, 700 rows 21.6 | 20.0 (eight wavefronts with a
- * barrier a stage 9.95 and 22.6). grid (E / 16, ceil(rows / 16)), block (256, 2): 512 threads, the 256
+ * 4096 inputs: 32 rows 10.6 | 9.2, 203 rows 10.75 | 9.4, 300 rows 15.2 | 14.2, 700 rows 21.2 | 19.5 (eight wavefronts with a
+ * barrier a stage 9.95 at 32 rows and 22.6 at 700). grid (E / 16, ceil(rows / 16)), block (256, 2): 512 threads, the 256
  * of y = 0 bring the experts' rows of the tile, those of y = 1 the rows. */
 #define PROJECTION_SPLIT_STAGE_BYTES (32u * PROJECTION_STAGE_ROW_BYTES)
 #define PROJECTION_SPLIT_PAIRS 3u

@@ -30,21 +30,21 @@ HBM_PEAK_GBS = 8000.0
 # under profiles/ hold the commands and the counts), reported as roofline.traffic when a run has the same sizes
 MEASURED_TRAFFIC_BYTES = {
     ("exl3_decode", 8): 375.1e6 + 4.2e6,
-    ("exl3_linear", 1): 8.601e6 + 0.016e6,
-    ("fp4_decode", 32): 1428.3e6 + 1.0e6,
+    ("exl3_linear", 1): 8.660e6 + 0.016e6,
+    ("fp4_decode", 32): 1428.2e6 + 1.0e6,
     ("fp8_decode", 32): 2739.0e6 + 1.0e6,
-    ("fp4_prefill", 8192): 3261.9e6 + 470.8e6,
-    ("fp8_prefill", 2048): 5231.7e6 + 116.8e6,
-    ("expert_join", 8192): 877.8e6 + 402.7e6,
+    ("fp4_prefill", 8192): 3276.0e6 + 471.0e6,
+    ("fp8_prefill", 2048): 5229.3e6 + 116.9e6,
+    ("expert_join", 8192): 878.8e6 + 402.7e6,
     ("fp8_decode_block128", 1): 134.6e6,
     ("fp8_decode_block128", 64): 3697.4e6 + 2.1e6,
-    ("fp8_prefill_block128", 2048): 5227.1e6 + 67.1e6,
-    ("fp4_prefill_native", 8192): 3681.1e6 + 415.0e6,
-    ("exl3_prefill", 4096): 2735.2e6 + 536.9e6,
-    ("fp8_prefill_native", 2048): 4723.5e6 + 112.4e6,
-    ("fp8_prefill_block128_native", 2048): 4704.8e6 + 67.1e6,
+    ("fp8_prefill_block128", 2048): 5236.6e6 + 67.1e6,
+    ("fp4_prefill_native", 8192): 3684.0e6 + 414.8e6,
+    ("exl3_prefill", 4096): 2729.0e6 + 536.9e6,
+    ("fp8_prefill_native", 2048): 4723.3e6 + 112.4e6,
+    ("fp8_prefill_block128_native", 2048): 4705.3e6 + 67.1e6,
     ("fp4_decode_native", 32): 1428.2e6 + 1.0e6,
-    ("fp8_decode_native", 32): 2739.0e6 + 1.0e6,
+    ("fp8_decode_native", 32): 2738.9e6 + 1.0e6,
 }
 TRAFFIC_SOURCE = "profiles/launch_counters.md (counter bytes of the profiled run, not of this one)"
 HIDDEN, INNER, EXPERTS, PICKS, ROWS = 4096, 2048, 256, 8, 8

@@ -131,11 +131,12 @@ ANEMONE_INLINE uint32_t router_projection_by_row(uint32_t row_count, uint32_t ex
 /* Which of the two takes a step of more rows. A block of router_projection_tiles is a score's 32 chains in one wavefront, so a
  * launch takes as long as the blocks that fall to one of the 256 CUs, one behind the other in all but the loads; a block of
  * router_projection_split is a quarter of that, on twice as many wavefronts, and brings its operands for a quarter of the scores. In
- * blocks a CU, us, 4096 inputs: tiles 1 / 2 / 3 / 4 blocks 26.6 / 42.8 / 64 / 87; split (by four wavefronts, which drew the line; by
- * eight 9.3 / 15.1 / 20.6, 31.2 at five, 38 at six) 1 .. 10 blocks 11.3 / 16.5 / 22.4 / 28.4 /
- * 33.8 / 39.6 / 45.5 / 51 / 57 / 64: three blocks of the split form are the faster, four the slower (256 experts: 512 rows 26.8 |
- * 17.0, 768 rows 26.8 | 22.7, 1024 rows 27.1 | 28.5, 1152 rows 42.7 | 33.7, 1536 rows 42.8 | 40.3, 1792 rows 43.4 | 46.1; 64 experts: 3072
- * rows 27.1 | 23.3, 4096 rows 27.5 | 29.3; 384 experts: 512 rows 27.0 | 22.6, 640 rows 26.9 | 28.5; 2048 and 5120 inputs: the same line). */
+ * blocks a CU, us, 4096 inputs: tiles 1 / 2 / 3 / 4 blocks 26.5 / 42.6 / 64 / 87; split 1 .. 8 blocks 9.5 / 14.8 / 19.6 / 25.7 / 30.8 /
+ * 35.8 / 41.4 / 46.6: three blocks of the split form to one of tiles are the faster; at four the two are within 5 % of each other
+ * either way, which is no line (tiles | split, 256 experts: 512 rows 26.5 | 14.8, 768 rows 26.5 | 19.6, 1024 rows 26.5 | 25.7, 1152 rows
+ * 42.4 | 30.6, 1536 rows 42.6 | 35.8, 1792 rows 42.9 | 41.4, 2048 rows 43.0 | 46.6; 64 experts: 3072 rows 26.6 | 20.8, 4096 rows 26.9 | 26.7;
+ * 384 experts: 512 rows 26.5 | 19.5, 640 rows 26.5 | 25.6; 256 experts of 2048 inputs: 768 rows 14.6 | 11.7, 1024 rows 15.0 | 15.6; of 5120
+ * inputs: 768 rows 32.2 | 23.3, 1024 rows 32.3 | 30.7). */
 #define PROJECTION_SPLIT_BLOCKS_OF_TILE 3u
 #define PROJECTION_CUS 256u
 #define PROJECTION_STAGE_INPUTS 128u     /* inputs of a stage of router_projection_tiles: the width is a whole number of them */
