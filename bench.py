@@ -291,7 +291,8 @@ def fp4_decode(amd, workloads, arguments, fp8=False, prefill=False):
         result["config"]["step_TFLOPs"] = (gate_up_flops + down_flops) / (seconds / arguments.steps) / 1e12
         # the products are MFMAs of FP8 activations (with FP4 or FP8 weights): the FP8 rate is the instruction's peak.
         # What bounds the launch is read off its arithmetic intensity against the card's balance of the two peaks.
-        kernel = ("native_expert_gate_up_%s1" if native else "wide_expert_gate_up_%s1") % ("b128_" if block128 else "e4m3_" if fp8 else "")
+        record, launched = layer.native_kernels if native else layer.wide_kernels, experts[0].kernel
+        kernel = next(name + "_1" for name, _ in record._fields_ if getattr(record, name) == launched)  # narrow or whole strips as the launch takes
         if gate_up_flops / gate_up_bytes >= MFMA_F8_PEAK_TFLOPS * 1e12 / (HBM_PEAK_GBS * 1e9):
             result["roofline"] = {"bound": "mfma", "kernel": kernel, "achieved": achieved, "peak": MFMA_F8_PEAK_TFLOPS, "unit": "TFLOP/s",
                                   "frac": achieved / MFMA_F8_PEAK_TFLOPS, "traffic": result["roofline"]["traffic"],
