@@ -127,20 +127,27 @@ __device__ static __forceinline__ void trunk_linear_quantized_wide(const struct 
     }
 }
 
-/* grid (ceil(output_size[0] / 128) + ceil(output_size[1] / 128), ceil(row_count / 64)), block 256 */
+template <uint32_t ROWS>
+using trunk_deep_chain = wide_chain<1, true, 1u, false, TRUNK_DEEP_STAGES(ROWS), ROWS>;
+static_assert(trunk_deep_chain<16u>::WINDOW_BYTES + 8u * trunk_deep_chain<16u>::CHUNK_BYTES == TRUNK_DEEP_WINDOW_BYTES(4096u, 16u) &&
+                  trunk_deep_chain<64u>::WINDOW_BYTES + 8u * trunk_deep_chain<64u>::CHUNK_BYTES == TRUNK_DEEP_WINDOW_BYTES(4096u, 64u) &&
+                  WIDE_WAVES * trunk_deep_chain<16u>::STRIP * 16u == TRUNK_DEEP_BLOCK_OUTPUTS && TRUNK_DEEP_WINDOW_BYTES(TRUNK_DEEP_MOST_INPUTS, 64u) <= 160u * 1024u,
+              "the windows and the blocks the host asks for are the kernel's");
+
+/* grid (ceil(output_size[0] / n) + ceil(output_size[1] / n), ceil(row_count / rows)), block 256; n and rows: TRUNK_INTERLEAVED_BLOCK_OUTPUTS and
+ * TRUNK_INTERLEAVED_ROWS, or TRUNK_DEEP_BLOCK_OUTPUTS and the deep instance's rows */
+template <typename chain_type, uint32_t ROWS>
 __device__ static __forceinline__ void trunk_linear_quantized_interleaved(const struct trunk_linear_quantized_arguments &arguments, unsigned char *arena)
 {
-    typedef wide_chain<1, true, 2u> chain_type;
     constexpr uint32_t TILES = chain_type::TILES, STRIP = chain_type::STRIP, STRIP_OUTPUTS = STRIP * 16u;
-    static_assert(chain_type::WINDOW_BYTES == TRUNK_INTERLEAVED_WINDOW_BYTES && WIDE_WAVES * STRIP_OUTPUTS == TRUNK_INTERLEAVED_BLOCK_OUTPUTS &&
-                      WIDE_TILE_PAIRS == TRUNK_INTERLEAVED_ROWS, "the window and the block the host asks for are the kernel's");
+    static_assert(ROWS <= WIDE_TILE_PAIRS && WIDE_TILE_PAIRS == TRUNK_INTERLEAVED_ROWS, "the block the host asks for is the kernel's");
     extern __shared__ __attribute__((aligned(128))) unsigned char wide_window[];
     uint32_t matrix, block;
-    trunk_matrix_of(arguments, blockIdx.x, TRUNK_INTERLEAVED_BLOCK_OUTPUTS, matrix, block);
+    trunk_matrix_of(arguments, blockIdx.x, WIDE_WAVES * STRIP_OUTPUTS, matrix, block);
     const uint32_t outputs = arguments.output_size[matrix];
     const uint32_t lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const uint32_t first_row = blockIdx.y * TRUNK_INTERLEAVED_ROWS;
-    const uint32_t row_count = arguments.row_count - first_row < TRUNK_INTERLEAVED_ROWS ? arguments.row_count - first_row : TRUNK_INTERLEAVED_ROWS;
+    const uint32_t first_row = blockIdx.y * ROWS;
+    const uint32_t row_count = arguments.row_count - first_row < ROWS ? arguments.row_count - first_row : ROWS;
     /* columns past the tile's last row read its first row's vector; their sums are never stored */
     uint32_t code_vectors[2];
 #pragma unroll
@@ -165,7 +172,11 @@ __device__ static __forceinline__ void trunk_linear_quantized_interleaved(const 
             chain[t][j] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
         }
     }
-    chain_of.whole(arguments.input_size / 128u, (row_count + 15u) / 16u, chain);
+    if constexpr (chain_type::DEEP) {
+        chain_of.whole_deep(arguments.input_size / 128u, (row_count + 15u) / 16u, chain);
+    } else {
+        chain_of.whole(arguments.input_size / 128u, (row_count + 15u) / 16u, chain);
+    }
     const uint32_t first_output = (block * WIDE_WAVES + wave) * STRIP_OUTPUTS;
     if (first_output >= outputs) {
         return;
@@ -252,9 +263,23 @@ TRUNK_ENTRIES(8);
 extern "C" __global__ void __launch_bounds__(WIDE_THREADS)
     trunk_linear_quantized_interleaved_1(struct trunk_linear_quantized_arguments arguments, unsigned char *arena)
 {
-    trunk_linear_quantized_interleaved(arguments, arena);
+    typedef wide_chain<1, true, 2u> chain_type;
+    static_assert(chain_type::WINDOW_BYTES == TRUNK_INTERLEAVED_WINDOW_BYTES && WIDE_WAVES * chain_type::STRIP * 16u == TRUNK_INTERLEAVED_BLOCK_OUTPUTS,
+                  "the window and the block the host asks for are the kernel's");
+    trunk_linear_quantized_interleaved<chain_type, TRUNK_INTERLEAVED_ROWS>(arguments, arena);
 }
 ANEMONE_KERNEL(KERNEL_FILE_TRUNK_LINEAR, trunk_linear_quantized_interleaved_1, trunk_linear_quantized_arguments);
+
+#define TRUNK_DEEP_ENTRY(rows)                                                                              \
+    extern "C" __global__ void __launch_bounds__(WIDE_THREADS)                                              \
+        trunk_linear_quantized_deep_##rows(struct trunk_linear_quantized_arguments arguments, unsigned char *arena) \
+    {                                                                                                       \
+        trunk_linear_quantized_interleaved<trunk_deep_chain<rows>, rows>(arguments, arena);                 \
+    }                                                                                                       \
+    ANEMONE_KERNEL(KERNEL_FILE_TRUNK_LINEAR, trunk_linear_quantized_deep_##rows, trunk_linear_quantized_arguments)
+TRUNK_DEEP_ENTRY(16);
+TRUNK_DEEP_ENTRY(32);
+TRUNK_DEEP_ENTRY(64);
 
 /* grid (ceil(width / (8 block[0])), vectors): a thread takes eight consecutive values where the width is a multiple of
  * eight, else one value at a time */

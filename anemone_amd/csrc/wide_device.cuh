@@ -12,11 +12,11 @@
 #define WIDE_COLUMN_BLOCKS (WIDE_TILE_PAIRS / 16u)
 #define WIDE_BLOCKS_A_CU 3 /* as the windows allow: 168 registers */
 #define WIDE_STAGES 2u /* K steps in LDS: one in use, the next on its way */
-#define WIDE_VECTOR_BYTES (WIDE_TILE_PAIRS * 128u) /* a K step of the tile's columns' codes */
 
 /* One block's pipeline: MATRICES matrices x STRIP tiles a wavefront, the tile's columns shared. */
 /* B128: float32 scales of 128 x 128 blocks and of 128 values in place of the E8M0 codes, as in strip_device.cuh. */
-template <uint32_t MATRICES, bool BYTES, uint32_t STRIP_TILES, bool B128 = false>
+/* STAGES: K steps in LDS; more than WIDE_STAGES: for a launch of few blocks (whole_deep), of tiles of ROWS columns at most. */
+template <uint32_t MATRICES, bool BYTES, uint32_t STRIP_TILES, bool B128 = false, uint32_t STAGES = WIDE_STAGES, uint32_t ROWS = WIDE_TILE_PAIRS>
 struct wide_chain {
     static_assert(BYTES || !B128, "float32 scales go with one-byte weights");
     static constexpr uint32_t STRIP = STRIP_TILES;
@@ -27,12 +27,13 @@ struct wide_chain {
     static constexpr uint32_t SCALE_LANES = BYTES ? 16u : STRIP * 16u;           /* a word of the weights' scales each */
     static constexpr uint32_t WAVE_BYTES = SCALES_AT + MATRICES * SCALE_LANES * 4u; /* a wavefront's part of a stage */
     static constexpr uint32_t VECTOR_AT = WIDE_WAVES * WAVE_BYTES;               /* inside a stage */
-    static constexpr uint32_t STAGE_BYTES = VECTOR_AT + WIDE_VECTOR_BYTES;
+    static constexpr uint32_t STAGE_BYTES = VECTOR_AT + ROWS * 128u;             /* and a K step of the tile's columns' codes */
     static constexpr uint32_t SCALE_STEPS = 4u; /* K steps whose scale words of the columns come together */
-    static constexpr uint32_t CHUNK_BYTES = WIDE_TILE_PAIRS * SCALE_STEPS * 4u;  /* [column][step of the chunk] */
-    static constexpr uint32_t STAGES_BYTES = WIDE_STAGES * STAGE_BYTES;
+    static constexpr uint32_t CHUNK_BYTES = ROWS * SCALE_STEPS * 4u;             /* [column][step of the chunk] */
+    static constexpr uint32_t STAGES_BYTES = STAGES * STAGE_BYTES;
+    static constexpr bool DEEP = STAGES != WIDE_STAGES;                          /* every chunk has a place of its own */
     static constexpr uint32_t CHUNKS_BYTES = 2u * CHUNK_BYTES;                   /* one in use, the next on its way */
-    static constexpr uint32_t WINDOW_BYTES = STAGES_BYTES + CHUNKS_BYTES;
+    static constexpr uint32_t WINDOW_BYTES = STAGES_BYTES + (DEEP ? 0u : CHUNKS_BYTES); /* deep: and the chunks of its inputs */
     static constexpr uint32_t WEIGHT_LOADS = TILES * TILE_LOADS + MATRICES;
     static_assert(WEIGHT_LOADS < 64u && WINDOW_BYTES <= 160u * 1024u, "vmcnt has six bits; LDS 160 KB");
 
@@ -54,7 +55,7 @@ struct wide_chain {
     {
         const uint32_t step = SCALE_STEPS * chunk + lane_of % SCALE_STEPS;
         load_to_lds_4(exponents, exponents_offset + 4u * (step < last_step ? step : last_step),
-                      chunks + chunk % 2u * CHUNK_BYTES + wave * (16u * SCALE_STEPS * 4u));
+                      chunks + (DEEP ? chunk : chunk % 2u) * CHUNK_BYTES + wave * (16u * SCALE_STEPS * 4u));
     }
 
     /* the tile's columns of K step `at` into stage `stage` (every wavefront reads them: behind the barrier that ends the
@@ -67,7 +68,7 @@ struct wide_chain {
         for (uint32_t part = 0; part < 2u; part++) {
             load_to_lds_16(codes + (uint64_t)at * 128u, codes_offset[part], base + VECTOR_AT + (2u * wave + part) * 1024u);
         }
-        if (at % SCALE_STEPS == 1u) { /* asked for by the step before it: the waits are for everything older than the weights */
+        if (!DEEP && at % SCALE_STEPS == 1u) { /* asked for by the step before it: the waits are for everything older than the weights */
             issue_vector_scales(at / SCALE_STEPS + 1u);
         }
     }
@@ -114,7 +115,7 @@ struct wide_chain {
     {
         /* the stage's addresses, once a step: every read below is one of them plus a constant */
         uint32_t base = window + stage * STAGE_BYTES, mine = base + wave * WAVE_BYTES;
-        uint32_t vector_scales = chunks + step / SCALE_STEPS % 2u * CHUNK_BYTES + 4u * (step % SCALE_STEPS);
+        uint32_t vector_scales = chunks + (DEEP ? step / SCALE_STEPS : step / SCALE_STEPS % 2u) * CHUNK_BYTES + 4u * (step % SCALE_STEPS);
         asm volatile("" : "+s"(base), "+s"(mine), "+s"(vector_scales));
         /* a lane's pieces differ from its first in bits 4 to 6 of the place (stages and parts are whole 64 and 128 bytes) */
         uint32_t a_at[4], a_scale_at[BYTES ? STRIP : 1], first_a = mine + read_at, first_b = base + VECTOR_AT + vector_at, b_scale_at = vector_scales + vector_scale_at;
@@ -240,6 +241,65 @@ struct wide_chain {
             consume<LIVE>(step % 2u, step, chain);
             if (step + 2u < total) {
                 issue_weights<ONCE>(step % 2u, step + 2u);
+            }
+        }
+    }
+
+    /* The same for a launch whose blocks are so few that each has a CU to itself: a step there is as long as memory takes to answer what
+     * was asked for a step before, so that STAGES - 1 steps are on their way, and the columns' scale words all from the start. A
+     * wavefront brings columns where its two groups are live. */
+    template <uint32_t LIVE>
+    __device__ __forceinline__ void deep_steps(uint32_t total, float4_t (&chain)[TILES][WIDE_COLUMN_BLOCKS]) const
+    {
+        static_assert((STAGES - 2u) * (WEIGHT_LOADS + 2u) < 64u, "vmcnt has six bits");
+        const bool brings = wave < LIVE; /* the same in every lane */
+        const auto ask = [&](uint32_t stage, uint32_t step) {
+            if (brings) {
+                issue_vectors(stage, step);
+            }
+            issue_weights<false>(stage, step);
+        };
+        if (brings) {
+            for (uint32_t chunk = 0; chunk * SCALE_STEPS < total; chunk++) {
+                issue_vector_scales(chunk);
+            }
+        }
+#pragma unroll
+        for (uint32_t step = 0; step + 1u < STAGES; step++) {
+            if (step < total) {
+                ask(step, step);
+            }
+        }
+        uint32_t stage = 0;
+        for (uint32_t step = 0; step < total; step++) {
+            if (step + STAGES - 1u > total) {
+                wait_loads<0>();
+            } else if (brings) { /* but for the steps behind this one */
+                wait_loads<(STAGES - 2u) * (WEIGHT_LOADS + 2u)>();
+            } else {
+                wait_loads<(STAGES - 2u) * WEIGHT_LOADS>();
+            }
+            __syncthreads(); /* every wavefront has read the step before, whose stage is asked for again, and brought its part of this one */
+            if (step + STAGES - 1u < total) {
+                ask(stage == 0u ? STAGES - 1u : stage - 1u, step + STAGES - 1u);
+            }
+            consume<LIVE>(stage, step, chain);
+            stage = stage + 1u == STAGES ? 0u : stage + 1u;
+        }
+    }
+
+    __device__ __forceinline__ void whole_deep(uint32_t total, uint32_t live_blocks, float4_t (&chain)[TILES][WIDE_COLUMN_BLOCKS]) const
+    {
+        constexpr uint32_t MOST = ROWS / 16u; /* live column blocks */
+        if (live_blocks == 1u || MOST == 1u) {
+            deep_steps<1>(total, chain);
+        } else if (live_blocks == 2u || MOST == 2u) {
+            deep_steps<2>(total, chain);
+        } else if constexpr (MOST == 4u) {
+            if (live_blocks == 3u) {
+                deep_steps<3>(total, chain);
+            } else {
+                deep_steps<4>(total, chain);
             }
         }
     }

@@ -613,6 +613,7 @@ ANEMONE_RECORD_HAS(expert_down_arguments, 56);
 #define KERNEL_TRUNK_LINEAR_QUANTIZED_STEM "trunk_linear_quantized_"
 #define KERNEL_TRUNK_LINEAR_QUANTIZED_WIDE_STEM "trunk_linear_quantized_wide_"
 #define KERNEL_TRUNK_LINEAR_QUANTIZED_INTERLEAVED "trunk_linear_quantized_interleaved_1"
+#define KERNEL_TRUNK_LINEAR_QUANTIZED_DEEP_STEM "trunk_linear_quantized_deep_" /* the same in launches of few blocks, by the rows of a block */
 #define KERNEL_TRUNK_HIDDEN "trunk_hidden_entry"
 #define KERNEL_EXPERT_SHARED_JOIN_STEM "expert_shared_join_"
 #define KERNEL_FILE_HYPER_CONNECTION "kernel_hyper_connection"
@@ -623,6 +624,16 @@ ANEMONE_RECORD_HAS(expert_down_arguments, 56);
 #define TRUNK_INTERLEAVED_ROWS 64u          /* rows of a block of the interleaved instance: one tile of vectors */
 #define TRUNK_INTERLEAVED_BLOCK_OUTPUTS 128u /* its outputs: four wavefronts' strips of two tiles */
 #define TRUNK_INTERLEAVED_WINDOW_BYTES 51712u
+/* trunk_linear_quantized_deep_<rows>, the interleaved instance of launches of few blocks: strips of one tile by 16, 32 or 64 rows a block. In
+ * LDS: the K steps that are on their way (8448 bytes of four wavefronts' weights and 128 of a row each), and all of the rows'
+ * scale words (16 bytes a row for four K steps) */
+#define TRUNK_DEEP_INSTANCES 3u
+#define TRUNK_DEEP_ROWS(instance) (16u << (instance))
+#define TRUNK_DEEP_BLOCK_OUTPUTS 64u
+#define TRUNK_DEEP_STAGES(rows) ((rows) < 64u ? 5u : 4u)
+#define TRUNK_DEEP_WINDOW_BYTES(inputs, rows) (TRUNK_DEEP_STAGES(rows) * (8448u + (rows) * 128u) + ((inputs) + 511u) / 512u * ((rows) * 16u))
+#define TRUNK_DEEP_MOST_INPUTS 16384u
+#define TRUNK_DEEP_MOST_BLOCKS 512u /* two a CU */
 #define MODEL_STREAMS 4u
 #define HYPER_VALUES_PER_THREAD 8u /* one 16-byte load of bfloat16 */
 #define HYPER_PIECE_THREADS 128u

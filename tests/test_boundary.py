@@ -751,6 +751,30 @@ def shared_description(rows=8, gate_up_slices=4, down_slices=2, form=amd.LINEAR_
     return d, cursor[0]
 
 
+@pytest.mark.parametrize("rows,taken,groups,windows", [
+    (9, "deep_16", 1, [54528, 53504]), (128, "deep_16", 8, [54528, 53504]), (129, "deep_32", 5, [66816, 64768]), (256, "deep_32", 8, [66816, 64768]),
+    (257, "deep_64", 5, [74752, 70656]), (512, "deep_64", 8, [74752, 70656]), (513, "interleaved_1", 9, [51712, 51712])])
+def test_shared_expert_launches_of_few_blocks(fake, rows, taken, groups, windows):
+    """64 blocks of 64 outputs a product: the instance of the fewest rows that leaves at most 512 blocks, else the other form."""
+    lib = amd.library()
+    kernels = amd.LinearKernels()
+    assert lib.linear_kernels_prepare(fake.address, fake.card, 950, C.byref(kernels)) == 0
+    d, arena = shared_description(rows=rows, gate_up_slices=1, down_slices=1, form=amd.LINEAR_INTERLEAVED_CHUNK_BLOCKS)
+    launches = amd.launches_of(4)
+
+    def prepared():
+        assert lib.linear_shared_expert_prepare(C.byref(d), arena, C.byref(kernels), launches) == 0
+        products = [launches[0], launches[3]]
+        return [fake.handles[l.kernel][1] for l in products], [list(l.grid) for l in products], [l.dynamic_shared_byte_count for l in products]
+    blocks = 32 if taken == "interleaved_1" else 64
+    assert prepared() == (["trunk_linear_quantized_" + taken] * 2, [[blocks, groups, 1]] * 2, windows)
+    for i in range(3):  # a backend without them, and a caller who left the members as zero
+        for handle in (amd.BACKEND_NO_KERNEL, 0):
+            kernels.trunk_linear_quantized_deep[i] = handle
+            if taken == "deep_%d" % (16 << i):
+                assert prepared() == (["trunk_linear_quantized_interleaved_1"] * 2, [[32, (rows + 63) // 64, 1]] * 2, [51712] * 2)
+
+
 def join_description(rows=8, picks=8, width=4096, first=1 << 30, row_sums=True, **changes):
     cursor = [first]
 

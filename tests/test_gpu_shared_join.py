@@ -148,6 +148,29 @@ def test_wide_and_interleaved_instances_have_the_thin_bits(amd, card, slices, ro
             assert differing == 0
 
 
+@pytest.mark.parametrize("hidden,inner,rows,of", [
+    (128, 160, 9, 16), (640, 1056, 33, 16), (768, 64, 16, 16), (4224, 160, 65, 16), (512, 96, 31, 16), (1024, 1056, 475, 32),
+    (512, 2048, 256, 32), (512, 2048, 257, 64), (384, 2048, 512, 64), (512, 2048, 513, 0)])
+def test_instances_for_launches_of_few_blocks_have_the_wide_bits(amd, card, hidden, inner, rows, of):
+    """One step, fewer steps than are on their way, steps and tiles that do not divide, every instance at its last row and block."""
+    say("trunk forms of few blocks, hidden", hidden, "inner", inner, "rows", rows)
+    layer, shared, _ = build(amd, card, hidden, 256, rows, 1, 9, shared_inner=inner)
+    layer.set_rows(to_bf16(normals(10, rows * hidden)).reshape(rows, hidden))
+    card.run(layer.quantize_launch())
+    outputs = [shared.ranges[name] for name in ("gate_output", "up_output")]
+    got = []
+    for form in (amd.LINEAR_WIDE_TILE_BLOCKS, amd.LINEAR_INTERLEAVED_CHUNK_BLOCKS):
+        for output in outputs:
+            card.upload(output.byte_offset, np.full(output.byte_count, 0xEE, dtype=np.uint8))
+        launch = trunk_launch(amd, card, layer, shared, (0, 1), 1, rows, form, outputs)
+        card.run(launch)
+        got.append([shared.read(name, np.uint16).copy() for name in ("gate_output", "up_output")])
+    kernels = layer.kernels
+    assert launch[0].kernel == (kernels.trunk_linear_quantized_deep[of // 32] if of else kernels.trunk_linear_quantized_interleaved)
+    for tiled, deep in zip(*got):
+        assert np.array_equal(tiled, deep)
+
+
 @pytest.mark.parametrize("rows,form,slices", [(6, 0, (4, 2)), (8, 0, (1, 1)), (100, 2, (1, 1)), (37, 0, (2, 4))])
 def test_shared_expert_against_oracle(amd, card, rows, form, slices):
     """The four launches against the oracle's layer of one expert that takes every row with a weight of 1."""
