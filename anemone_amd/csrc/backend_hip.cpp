@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "anemone_backend.h"
+#include "joined_launches.h"
 #include "kernel_registry.h"
 
 namespace {
@@ -36,6 +37,37 @@ std::vector<kernel_entry> &kernel_table()
     static std::vector<kernel_entry> table; /* built by the kernel files' static registrations */
     return table;
 }
+
+struct joined_entry {
+    const char *files[2], *functions[2]; /* of the two launches */
+    const void *host_function;
+};
+
+#define MOST_JOINED_KERNELS 32u /* a bit each */
+
+std::vector<joined_entry> &joined_table()
+{
+    static std::vector<joined_entry> table;
+    return table;
+}
+
+/* the joined kernels that have `entry` as launch 0 or 1, a bit each */
+uint32_t joins_of(const kernel_entry &entry, uint32_t launch)
+{
+    uint32_t joins = 0;
+    const std::vector<joined_entry> &table = joined_table();
+    for (uint32_t index = 0; index < table.size() && index < MOST_JOINED_KERNELS; index++) {
+        if (std::strcmp(table[index].files[launch], entry.file) == 0 && std::strcmp(table[index].functions[launch], entry.function) == 0) {
+            joins |= 1u << index;
+        }
+    }
+    return joins;
+}
+
+struct prepared_kernel {
+    uint32_t index;    /* into kernel_table() */
+    uint32_t joins[2]; /* joins_of its entry */
+};
 
 struct copy_slot {
     hipEvent_t event;
@@ -65,7 +97,7 @@ struct device_card {
     std::mutex mutex;
     bool failed;
     /* prepared kernels: handle = index */
-    std::vector<uint32_t> prepared; /* indices into kernel_table() */
+    std::vector<prepared_kernel> prepared;
     /* copies */
     uint64_t next_ticket, finished_ticket;
     copy_slot slots[BACKEND_MAXIMUM_UPLOADS_IN_FLIGHT];
@@ -178,7 +210,7 @@ result_status launches_check(device_card *card, const kernel_launch *launches, u
             log_error("launch", "a kernel handle that was not prepared on this card");
             return STATUS_INVALID_ARGUMENT;
         }
-        const kernel_entry &entry = kernel_table()[card->prepared[launch.kernel]];
+        const kernel_entry &entry = kernel_table()[card->prepared[launch.kernel].index];
         uint64_t threads = 1;
         for (uint32_t d = 0; d < LAUNCH_DIMENSIONS; d++) {
             if (launch.grid[d] == 0 || launch.block[d] == 0) {
@@ -245,7 +277,7 @@ result_status launches_check(device_card *card, const kernel_launch *launches, u
 
 hipError_t launch_on(device_card *card, const kernel_launch &launch, hipStream_t stream)
 {
-    const kernel_entry &entry = kernel_table()[card->prepared[launch.kernel]];
+    const kernel_entry &entry = kernel_table()[card->prepared[launch.kernel].index];
     /* the record travels by value: the runtime copies record_bytes from the launch's own bytes */
     void *arguments[2] = {(void *)launch.argument, (void *)&card->arena};
     return hipLaunchKernel(entry.host_function, dim3(launch.grid[0], launch.grid[1], launch.grid[2]),
@@ -256,6 +288,26 @@ hipError_t launch_on(device_card *card, const kernel_launch &launch, hipStream_t
 hipError_t launch_one(device_card *card, const kernel_launch &launch)
 {
     return launch_on(card, launch, card->stream);
+}
+
+/* Launch `index` of a list, together with the one behind it where a kernel does both works (joined_launches.h); index is
+ * left at the last launch queued */
+hipError_t launch_next(device_card *card, const kernel_launch *launches, uint32_t count, uint32_t &index)
+{
+    const kernel_launch &first = launches[index];
+    if (index + 1u < count) {
+        const kernel_launch &second = launches[index + 1u];
+        const prepared_kernel &kernel = card->prepared[first.kernel];
+        const uint32_t joins = kernel.joins[0] & card->prepared[second.kernel].joins[1];
+        joined_launch joined;
+        if (joins != 0 && joined_launch_of(kernel_table()[kernel.index].function, first, second, card->arena_bytes, joined)) {
+            index++;
+            void *arguments[6] = {(void *)first.argument, (void *)second.argument, (void *)&card->arena, &joined.numbers[0], &joined.numbers[1], &joined.numbers[2]};
+            return hipLaunchKernel(joined_table()[(uint32_t)__builtin_ctz(joins)].host_function, dim3(joined.grid[0], joined.grid[1], 1), dim3(joined.block, 1, 1),
+                                   arguments, 0, card->stream);
+        }
+    }
+    return launch_one(card, first);
 }
 
 /* A checked list under capture on the card's stream: side runs go to side streams that wait for the fork's event, a
@@ -297,8 +349,9 @@ hipError_t capture_branches(device_card *card, const kernel_launch *launches, ui
             join();
             /* fall through: the launch itself stands on the main line */
         default: /* CHAIN, RESUME: the main line, which stands at the fork while side runs are open */
-            if (status == hipSuccess) {
-                status = launch_on(card, launch, card->stream);
+            if (status == hipSuccess) { /* joined with what is behind it on the main line alone */
+                const bool chained = index + 1u < count && launches[index + 1u].branch == LAUNCH_CHAIN;
+                status = launch_next(card, launches, chained ? index + 2u : index + 1u, index);
             }
             last_is_side = false;
             break;
@@ -339,6 +392,11 @@ void anemone_register_kernel(const char *file, const char *function, const void 
                              uint32_t record_bytes)
 {
     kernel_table().push_back(kernel_entry{file, function, host_function, record_bytes});
+}
+
+void anemone_register_joined_kernel(const char *first_file, const char *first, const char *second_file, const char *second, const void *host_function)
+{
+    joined_table().push_back(joined_entry{{first_file, second_file}, {first, second}, host_function});
 }
 
 uint32_t backend_hip_kernel_table_count(void)
@@ -606,7 +664,7 @@ result_status backend_hip_kernel_prepare(struct device_card *card, const char *k
             return STATUS_INVALID_ARGUMENT;
         }
         for (uint32_t handle = 0; handle < card->prepared.size(); handle++) {
-            if (card->prepared[handle] == index) {
+            if (card->prepared[handle].index == index) {
                 *kernel_out = handle; /* the same kernel again gives the same handle */
                 return STATUS_OK;
             }
@@ -619,9 +677,13 @@ result_status backend_hip_kernel_prepare(struct device_card *card, const char *k
          * the kernel's limit of dynamic shared memory to what the card holds; a refusal shows at the launch that asks */
         if (hipSetDevice(card->device) == hipSuccess) {
             (void)hipFuncSetAttribute(table[index].host_function, hipFuncAttributeMaxDynamicSharedMemorySize, card->max_shared);
+            for (uint32_t joins = joins_of(table[index], 1); joins != 0; joins &= joins - 1u) { /* loaded here too, not by the first pass */
+                hipFuncAttributes attributes;
+                (void)hipFuncGetAttributes(&attributes, joined_table()[(uint32_t)__builtin_ctz(joins)].host_function);
+            }
             (void)hipGetLastError();
         }
-        card->prepared.push_back(index);
+        card->prepared.push_back({index, {joins_of(table[index], 0), joins_of(table[index], 1)}});
         *kernel_out = (uint32_t)card->prepared.size() - 1u;
         return STATUS_OK;
     }
@@ -651,7 +713,7 @@ result_status backend_hip_launch_run(struct device_card *card, const struct kern
         return STATUS_DEVICE_ERROR;
     }
     for (uint32_t index = 0; index < launch_count; index++) {
-        if (card_fail(card, "hipLaunchKernel", launch_one(card, launches[index]))) {
+        if (card_fail(card, "hipLaunchKernel", launch_next(card, launches, launch_count, index))) {
             return STATUS_DEVICE_ERROR;
         }
     }

@@ -1,0 +1,127 @@
+/* joined_launches.cpp -- see joined_launches.h. Host code over the launches' records alone. */
+#include "joined_launches.h"
+
+#include <cstring>
+
+#include <hip/hip_runtime.h> /* what the records mark their functions with */
+
+#include "anemone_records.h"
+
+namespace {
+
+constexpr uint32_t ROUTER_BLOCK = 512u;       /* threads of the router's launches that are joined, and of their joined kernels */
+constexpr uint32_t MOST_BLOCKS = 1u << 22;    /* of 512 threads: the runtime counts a grid's threads in 32 bits */
+
+struct byte_range {
+    uint64_t first, bytes;
+};
+
+bool apart(const byte_range &a, const byte_range &b)
+{
+    return a.bytes == 0 || b.bytes == 0 || (a.first >= b.first ? a.first - b.first >= b.bytes : b.first - a.first >= a.bytes);
+}
+
+template <size_t A, size_t B> bool all_apart(const byte_range (&a)[A], const byte_range (&b)[B])
+{
+    for (const byte_range &x : a) {
+        for (const byte_range &y : b) {
+            if (!apart(x, y)) {
+                return false;
+            }
+        }
+    }
+    return true;
+}
+
+template <typename T> T record_of(const struct kernel_launch &launch)
+{
+    T record;
+    std::memcpy(&record, launch.argument, sizeof record);
+    return record;
+}
+
+bool is_plain(const struct kernel_launch &launch, uint32_t block)
+{
+    return launch.block[0] == block && launch.block[1] == 1 && launch.block[2] == 1 && launch.grid[2] == 1 && launch.dynamic_shared_byte_count == 0;
+}
+
+/* the quantizer's launch: its threads cover the vectors' width, and its values fit the arena (so that no product below wraps) */
+bool quantizer_is_whole(const struct kernel_launch &launch, const struct activation_quantize_arguments &record, uint64_t arena_bytes)
+{
+    return is_plain(launch, LINEAR_ELEMENT_THREADS) && record.width != 0 && (uint64_t)launch.grid[0] * LINEAR_ELEMENT_THREADS * 4u >= record.width &&
+           (uint64_t)launch.grid[1] * record.width <= arena_bytes;
+}
+
+bool join_hidden(const struct kernel_launch &first, const struct kernel_launch &second, uint64_t arena_bytes, struct joined_launch &out)
+{
+    const auto hidden = record_of<trunk_hidden_arguments>(first);
+    const auto quantize = record_of<activation_quantize_arguments>(second);
+    if (!is_plain(first, LINEAR_ELEMENT_THREADS) || !quantizer_is_whole(second, quantize, arena_bytes) || first.grid[1] != second.grid[1] ||
+        hidden.width != quantize.width || hidden.width % 32u != 0 || hidden.hidden_offset != quantize.values_offset ||
+        (uint64_t)first.grid[0] * LINEAR_ELEMENT_THREADS * HYPER_VALUES_PER_THREAD < hidden.width) {
+        return false;
+    }
+    const uint64_t values = (uint64_t)first.grid[1] * hidden.width;
+    const byte_range outputs[] = {{quantize.codes_offset, values}, {quantize.exponents_offset, values / 32u}, {quantize.operands_offset, 2u * values}};
+    const byte_range inputs[] = {{hidden.gate_offset, 2u * values}, {hidden.up_offset, 2u * values}}, own[] = {{hidden.hidden_offset, 2u * values}};
+    if (!all_apart(outputs, inputs) || !all_apart(outputs, own) || !all_apart(inputs, own)) {
+        return false;
+    }
+    out = {{second.grid[0], second.grid[1]}, LINEAR_ELEMENT_THREADS, {0, 0, 0}};
+    return true;
+}
+
+bool join_router(const char *function, const struct kernel_launch &first, const struct kernel_launch &second, uint64_t arena_bytes,
+                 struct joined_launch &out)
+{
+    const auto quantize = record_of<activation_quantize_arguments>(second);
+    if (!is_plain(first, ROUTER_BLOCK) || first.grid[1] != 1 || !quantizer_is_whole(second, quantize, arena_bytes)) {
+        return false;
+    }
+    const uint64_t values = (uint64_t)second.grid[1] * quantize.width;
+    const byte_range read[] = {{quantize.values_offset, 2u * values}};
+    /* the quantizer of 128 values a scale writes no operands: they are kept apart all the same */
+    const byte_range written[] = {{quantize.codes_offset, values}, {quantize.exponents_offset, values / 32u}, {quantize.operands_offset, 2u * values}};
+    if (std::strcmp(function, KERNEL_ROUTER_SELECT) == 0) {
+        const auto select = record_of<router_select_arguments>(first);
+        const uint64_t experts = select.expert_count != 0 ? select.expert_count : ROUTER_DEFAULT_EXPERTS, rows = select.row_count;
+        const uint64_t picks = select.pick_count != 0 ? select.pick_count : ROUTER_DEFAULT_PICKS;
+        const byte_range inputs[] = {{select.step_offset, sizeof(struct step_block)}, {select.scores_offset, rows * experts * 4u},
+                                     {select.bias_offset, experts * 4u}, {select.expert_offsets_offset, experts * MODEL_EXPERT_MATRICES * 8u}};
+        const byte_range outputs[] = {{select.affinities_offset, rows * experts * 4u}, {select.jobs_offset, rows * picks * sizeof(struct expert_job_record)}};
+        if (!all_apart(written, inputs) || !all_apart(written, outputs) || !all_apart(read, outputs)) {
+            return false;
+        }
+    } else {
+        const auto wide = record_of<router_wide_arguments>(first);
+        const uint64_t experts = wide.expert_count != 0 ? wide.expert_count : ROUTER_DEFAULT_EXPERTS, rows = wide.row_count;
+        const uint64_t picks = wide.pick_count != 0 ? wide.pick_count : ROUTER_DEFAULT_PICKS, pairs = rows * picks;
+        const byte_range inputs[] = {{wide.step_offset, sizeof(struct step_block)},
+                                     {wide.expert_offsets_offset, experts * MODEL_EXPERT_MATRICES * 8u},
+                                     {wide.picks_offset, pairs * sizeof(struct router_pick)},
+                                     {wide.counts_offset, (rows + ROUTER_SORT_ROWS - 1u) / ROUTER_SORT_ROWS * experts * 4u}};
+        const byte_range outputs[] = {{wide.pairs_offset, pairs * sizeof(struct wide_pair)},
+                                      {wide.runs_offset, experts * sizeof(struct wide_run)},
+                                      {wide.tiles_offset, ROUTER_WIDE_TILES_OF(rows, picks, experts) * sizeof(struct wide_expert_tile)},
+                                      {wide.jobs_offset, ROUTER_WIDE_JOBS_OF(rows, picks, experts) * sizeof(struct expert_job_record)}};
+        if (!all_apart(written, inputs) || !all_apart(written, outputs) || !all_apart(read, outputs)) {
+            return false;
+        }
+    }
+    constexpr uint32_t TOGETHER = ROUTER_BLOCK / LINEAR_ELEMENT_THREADS;
+    const uint64_t blocks = (uint64_t)first.grid[0] + ((uint64_t)second.grid[0] * second.grid[1] + TOGETHER - 1u) / TOGETHER;
+    if (blocks > MOST_BLOCKS) {
+        return false;
+    }
+    out = {{(uint32_t)blocks, 1}, ROUTER_BLOCK, {first.grid[0], second.grid[0], second.grid[1]}};
+    return true;
+}
+
+} // namespace
+
+extern "C" bool joined_launch_of(const char *first_function, const struct kernel_launch &first, const struct kernel_launch &second, uint64_t arena_bytes,
+                      struct joined_launch &out)
+{
+    return std::strcmp(first_function, KERNEL_TRUNK_HIDDEN) == 0 ? join_hidden(first, second, arena_bytes, out)
+                                                                 : join_router(first_function, first, second, arena_bytes, out);
+}

@@ -31,31 +31,6 @@ ANEMONE_KERNEL(KERNEL_FILE_ACTIVATION_QUANTIZE, activation_quantize_entry, activ
 extern "C" __global__ void __launch_bounds__(LINEAR_ELEMENT_THREADS)
     activation_quantize_128_entry(struct activation_quantize_arguments arguments, unsigned char *arena)
 {
-    /* the threads' values as in activation_quantize_entry: thread q = 16 l + 4 s + t takes 64 l + 16 s + 2 t + {0, 1, 8, 9},
-     * one word of codes; the 128 values of a scale are those of 32 neighbouring threads */
-    const uint32_t q = blockIdx.x * LINEAR_ELEMENT_THREADS + threadIdx.x;
-    const uint32_t l = q / 16u, s = (q / 4u) % 4u, t = q % 4u, first = 64u * l + 16u * s + 2u * t;
-    if (first >= arguments.width) {
-        return; /* the width is a multiple of 128: whole groups of 32 threads leave together */
-    }
-    const uint64_t vector = blockIdx.y;
-    const uint16_t *values = (const uint16_t *)(arena + arguments.values_offset) + vector * arguments.width + first;
-    const uint32_t near_pair = *(const uint32_t *)values, far_pair = *(const uint32_t *)(values + 8);
-    const uint32_t bits[4] = {near_pair & 0xFFFFu, near_pair >> 16, far_pair & 0xFFFFu, far_pair >> 16};
-    float largest = fmaxf(fmaxf(fabsf(bf16_to_float((uint16_t)bits[0])), fabsf(bf16_to_float((uint16_t)bits[1]))),
-                          fmaxf(fabsf(bf16_to_float((uint16_t)bits[2])), fabsf(bf16_to_float((uint16_t)bits[3]))));
-    largest = lanes_largest<1u>(lanes_largest<2u>(lanes_largest<4u>(lanes_largest<8u>(lanes_largest<16u>(largest)))));
-    const float scale = __fdiv_rn(fmaxf(largest, 1e-4f), 448.0f);
-    const float reciprocal = __fdiv_rn(1.0f, scale);
-    uint32_t code[4];
-#pragma unroll
-    for (uint32_t i = 0; i < 4u; i++) {
-        code[i] = quantize_quotient_code(quantize_quotient(bf16_to_float((uint16_t)bits[i]), scale, reciprocal), bits[i]);
-    }
-    *(uint32_t *)(arena + arguments.codes_offset + vector * arguments.width + quantize_word_of(l, s, t)) =
-        code[0] | (code[2] << 8) | (code[1] << 16) | (code[3] << 24); /* bytes: values +0, +8, +1, +9 */
-    if (q % 32u == 0u) {
-        ((float *)(arena + arguments.exponents_offset))[vector * (arguments.width / 128u) + first / 128u] = scale;
-    }
+    activation_quantize_128_body(arguments, arena, blockIdx.x * LINEAR_ELEMENT_THREADS + threadIdx.x, blockIdx.y);
 }
 ANEMONE_KERNEL(KERNEL_FILE_ACTIVATION_QUANTIZE, activation_quantize_128_entry, activation_quantize_arguments);

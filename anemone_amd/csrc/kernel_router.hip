@@ -19,6 +19,7 @@
 #include "router_device.cuh"
 #include "kernel_registry.h"
 #include "sort_device.cuh"
+#include "quantize_device.cuh"
 
 #define PROJECTION_CHAINS 32u
 #define PROJECTION_THREADS 128u
@@ -735,9 +736,8 @@ __device__ static __forceinline__ void wide_place_block(const struct router_wide
     }
 }
 
-/* grid as the count's: the sorted pairs of the block's rows; block 0 also the runs and every tile */
-extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
-    router_wide_place(struct router_wide_arguments arguments, unsigned char *arena)
+/* block `block` of a grid as the count's: the sorted pairs of the block's rows; block 0 also the runs and every tile */
+__device__ static __forceinline__ void wide_place(const struct router_wide_arguments &arguments, unsigned char *arena, uint32_t block)
 {
     __shared__ __attribute__((aligned(16))) uint32_t block_experts[ROUTER_SORT_ROWS * ROUTER_MOST_PICKS];
     __shared__ uint32_t place_of[ROUTER_SORT_ROWS * ROUTER_MOST_PICKS];
@@ -747,18 +747,18 @@ extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
     const uint32_t experts = arguments.expert_count;
     const uint32_t live_rows = wide_live_rows(arguments, arena);
     const uint32_t live_blocks = (live_rows + ROUTER_SORT_ROWS - 1u) / ROUTER_SORT_ROWS;
-    const uint32_t pairs = wide_block_picks(arguments, arena, blockIdx.x, live_rows, block_experts);
-    if (pairs == 0u && blockIdx.x != 0u) {
+    const uint32_t pairs = wide_block_picks(arguments, arena, block, live_rows, block_experts);
+    if (pairs == 0u && block != 0u) {
         return;
     }
     const uint32_t *counts = (const uint32_t *)(arena + arguments.counts_offset);
     for (uint32_t expert = threadIdx.x; expert < experts; expert += WIDE_SORT_THREADS) {
         uint32_t total = 0, lower = 0;
 #pragma unroll 8
-        for (uint32_t block = 0; block < live_blocks; block++) {
-            const uint32_t count = counts[(uint64_t)block * experts + expert];
+        for (uint32_t other = 0; other < live_blocks; other++) {
+            const uint32_t count = counts[(uint64_t)other * experts + expert];
             total += count;
-            lower += block < blockIdx.x ? count : 0u;
+            lower += other < block ? count : 0u;
         }
         totals[expert] = total;
         starts[expert] = total;
@@ -766,8 +766,14 @@ extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
         tile_starts[expert] = (total + WIDE_TILE_PAIRS - 1u) / WIDE_TILE_PAIRS;
     }
     __syncthreads();
-    wide_place_block(arguments, arena, blockIdx.x, block_experts, place_of, pairs, totals, starts, before, tile_starts, scratch, first_places,
+    wide_place_block(arguments, arena, block, block_experts, place_of, pairs, totals, starts, before, tile_starts, scratch, first_places,
                      cursors);
+}
+
+extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
+    router_wide_place(struct router_wide_arguments arguments, unsigned char *arena)
+{
+    wide_place(arguments, arena, blockIdx.x);
 }
 ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_wide_place, router_wide_arguments);
 
@@ -843,8 +849,7 @@ ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_wide_jobs, router_wide_arguments);
  * and jobs from one scan of the three side by side, the jobs find their expert and their pairs in LDS: five barriers, two
  * waits for memory. 64 rows of 256 experts, 8 picks: 17.4 -> 6.0 us (three scans of nine barriers, searches, the runs and
  * the sorted pairs read back from memory, a job's pairs by way of scratch memory). */
-extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
-    router_wide_small(struct router_wide_arguments arguments, unsigned char *arena)
+__device__ static __forceinline__ void wide_small(const struct router_wide_arguments &arguments, unsigned char *arena)
 {
     constexpr uint32_t MOST_PAIRS = ROUTER_SORT_ROWS * ROUTER_MOST_PICKS;
     static_assert(WIDE_SORT_THREADS == SORT_MOST_WAVES * SORT_WAVE && WIDE_SORT_THREADS >= ROUTER_MOST_EXPERTS, "a thread an expert");
@@ -945,4 +950,53 @@ extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
         jobs[job] = value;
     }
 }
+
+extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)
+    router_wide_small(struct router_wide_arguments arguments, unsigned char *arena)
+{
+    wide_small(arguments, arena);
+}
 ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_wide_small, router_wide_arguments);
+
+/* ---- a router's last launch and the quantizer of the step's rows behind it, as one launch ----------------------
+ * Neither reads what the other writes, and the router's is one block, or one for 384 rows: the first `blocks` blocks are its, the
+ * others two of the quantizer's blocks each. The backend runs the pair so where it stands in a list (joined_launches.h, with
+ * what that measured). Bound by the router's block, or by the quantizer's bytes where the rows are many. */
+#define QUANTIZE_JOIN_BLOCKS (WIDE_SORT_THREADS / LINEAR_ELEMENT_THREADS)
+static_assert(SELECT_THREADS == WIDE_SORT_THREADS, "one block size");
+
+template <bool WIDE_SCALES>
+__device__ static __forceinline__ void joined_quantize(const struct activation_quantize_arguments &quantize, unsigned char *arena, uint32_t block, uint32_t columns,
+                                                       uint32_t vectors)
+{
+    const uint32_t part = block * QUANTIZE_JOIN_BLOCKS + threadIdx.x / LINEAR_ELEMENT_THREADS, vector = part / columns;
+    const uint32_t q = part % columns * LINEAR_ELEMENT_THREADS + threadIdx.x % LINEAR_ELEMENT_THREADS;
+    if (vector >= vectors) {
+        return;
+    }
+    if constexpr (WIDE_SCALES) {
+        activation_quantize_128_body(quantize, arena, q, vector);
+    } else {
+        activation_quantize_body(quantize, arena, q, vector);
+    }
+}
+
+#define ROUTER_JOIN(first, record, suffix, wide_scales, ...)                                                                            \
+    extern "C" __global__ void __launch_bounds__(WIDE_SORT_THREADS)                                                                     \
+        first##_quantize##suffix(struct record arguments, struct activation_quantize_arguments quantize, unsigned char *arena, uint32_t blocks, \
+                                 uint32_t columns, uint32_t vectors)                                                                    \
+    {                                                                                                                                   \
+        if (blockIdx.x < blocks) {                                                                                                      \
+            __VA_ARGS__;                                                                                                                \
+        } else {                                                                                                                        \
+            joined_quantize<wide_scales>(quantize, arena, blockIdx.x - blocks, columns, vectors);                                       \
+        }                                                                                                                               \
+    }                                                                                                                                   \
+    ANEMONE_JOINED_KERNEL(KERNEL_FILE_ROUTER, first, KERNEL_FILE_ACTIVATION_QUANTIZE, activation_quantize##suffix##_entry, first##_quantize##suffix);
+#define SELECT_LDS_BODY __shared__ struct router_select_lds lds; router_select_body(arguments, arena, threadIdx.x, SELECT_THREADS, lds)
+ROUTER_JOIN(router_select_entry, router_select_arguments, , false, SELECT_LDS_BODY)
+ROUTER_JOIN(router_select_entry, router_select_arguments, _128, true, SELECT_LDS_BODY)
+ROUTER_JOIN(router_wide_small, router_wide_arguments, , false, wide_small(arguments, arena))
+ROUTER_JOIN(router_wide_small, router_wide_arguments, _128, true, wide_small(arguments, arena))
+ROUTER_JOIN(router_wide_place, router_wide_arguments, , false, wide_place(arguments, arena, blockIdx.x))
+ROUTER_JOIN(router_wide_place, router_wide_arguments, _128, true, wide_place(arguments, arena, blockIdx.x))

@@ -23,6 +23,7 @@
 #include "kernel_registry.h"
 #include "join_device.cuh"
 #include "linear_device.cuh"
+#include "quantize_device.cuh"
 #include "strip_device.cuh"
 #include "wide_device.cuh"
 
@@ -311,3 +312,32 @@ extern "C" __global__ void trunk_hidden_entry(struct trunk_hidden_arguments argu
     }
 }
 ANEMONE_KERNEL(KERNEL_FILE_TRUNK_LINEAR, trunk_hidden_entry, trunk_hidden_arguments);
+
+/* the hidden step and the quantizer of its values behind it as one launch, run so by the backend where the two stand next to
+ * each other in a list (joined_launches.h): a thread forms the four values it quantizes. Both launches' outputs are written. The quantizer's
+ * grid and block. */
+extern "C" __global__ void __launch_bounds__(LINEAR_ELEMENT_THREADS)
+    trunk_hidden_quantize(struct trunk_hidden_arguments arguments, struct activation_quantize_arguments quantize, unsigned char *arena, uint32_t,
+                          uint32_t, uint32_t)
+{
+    const uint32_t q = blockIdx.x * LINEAR_ELEMENT_THREADS + threadIdx.x, first = quantize_first_of(q);
+    if (first >= arguments.width) {
+        return;
+    }
+    const uint64_t at = (uint64_t)blockIdx.y * arguments.width + first;
+    const uint16_t *gate = (const uint16_t *)(arena + arguments.gate_offset) + at, *up = (const uint16_t *)(arena + arguments.up_offset) + at;
+    uint16_t *hidden = (uint16_t *)(arena + arguments.hidden_offset) + at;
+    const uint32_t gates[2] = {*(const uint32_t *)gate, *(const uint32_t *)(gate + 8)}, ups[2] = {*(const uint32_t *)up, *(const uint32_t *)(up + 8)};
+    const float limit = arguments.activation_limit;
+    uint32_t bits[4];
+#pragma unroll
+    for (uint32_t v = 0; v < 4u; v++) {
+        const float g = bf16_to_float((uint16_t)(gates[v / 2u] >> (16u * (v % 2u)))), u = bf16_to_float((uint16_t)(ups[v / 2u] >> (16u * (v % 2u))));
+        const float bounded_gate = fminf(g, limit), bounded_up = fminf(fmaxf(u, -limit), limit);
+        bits[v] = float_to_bf16(__fmul_rn(__fmul_rn(det_silu(bounded_gate), bounded_up), 1.0f));
+    }
+    *(uint32_t *)hidden = bits[0] | (bits[1] << 16);
+    *(uint32_t *)(hidden + 8) = bits[2] | (bits[3] << 16);
+    activation_quantize_values(quantize, arena, q, blockIdx.y, bits);
+}
+ANEMONE_JOINED_KERNEL(KERNEL_FILE_TRUNK_LINEAR, trunk_hidden_entry, KERNEL_FILE_ACTIVATION_QUANTIZE, activation_quantize_entry, trunk_hidden_quantize);

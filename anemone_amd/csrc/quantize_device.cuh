@@ -124,21 +124,20 @@ __device__ static __forceinline__ void quantize_value(uint32_t bits, uint32_t in
     }
 }
 
-/* thread q of a vector's width / 4 (four values, a word of codes) of vector `vector`: activation_quantize_entry's work of
- * one thread; the eight threads of a block of 32 values are neighbours in one wavefront and call together */
-__device__ static __forceinline__ void activation_quantize_body(const struct activation_quantize_arguments &arguments, unsigned char *arena,
-                                                                uint32_t q, uint64_t vector)
+/* the first of the four values +0, +1, +8, +9 of thread q of a vector: thread q = (16 l + 4 s + t) takes 64 l + 16 s + 2 t + {0, 1, 8, 9}, the
+ * four codes of one word of the lane order and the four operands of one pair of words; the 32 values of a block of the
+ * quantization are those of eight neighbouring threads (s = 2 b, 2 b + 1; t = 0 .. 3) */
+__device__ static __forceinline__ uint32_t quantize_first_of(uint32_t q)
 {
-    /* thread q = (16 l + 4 s + t) takes the four values 64 l + 16 s + 2 t + {0, 1, 8, 9}: the four codes of one word of
-     * the lane order and the four operands of one pair of words; the 32 values of a block of the quantization are those
-     * of eight neighbouring threads (s = 2 b, 2 b + 1; t = 0 .. 3) */
-    const uint32_t l = q / 16u, s = (q / 4u) % 4u, t = q % 4u, first = 64u * l + 16u * s + 2u * t;
-    if (first >= arguments.width) {
-        return; /* the width is a multiple of 64: whole groups of sixteen threads leave together */
-    }
-    const uint16_t *values = (const uint16_t *)(arena + arguments.values_offset) + vector * arguments.width + first;
-    const uint32_t near_pair = *(const uint32_t *)values, far_pair = *(const uint32_t *)(values + 8);
-    const uint32_t bits[4] = {near_pair & 0xFFFFu, near_pair >> 16, far_pair & 0xFFFFu, far_pair >> 16}; /* values +0, +1, +8, +9 */
+    return 64u * (q / 16u) + 16u * (q / 4u % 4u) + 2u * (q % 4u);
+}
+
+/* activation_quantize_entry's work of thread q of vector `vector` from its four values on; the eight threads of a block of
+ * 32 values are neighbours in one wavefront and call together */
+__device__ static __forceinline__ void activation_quantize_values(const struct activation_quantize_arguments &arguments, unsigned char *arena,
+                                                                  uint32_t q, uint64_t vector, const uint32_t (&bits)[4])
+{
+    const uint32_t l = q / 16u, s = (q / 4u) % 4u, t = q % 4u, first = quantize_first_of(q);
     float largest = fmaxf(fmaxf(fabsf(bf16_to_float((uint16_t)bits[0])), fabsf(bf16_to_float((uint16_t)bits[1]))),
                           fmaxf(fabsf(bf16_to_float((uint16_t)bits[2])), fabsf(bf16_to_float((uint16_t)bits[3]))));
     largest = lanes_largest<1u>(lanes_largest<2u>(lanes_largest<4u>(largest)));
@@ -154,6 +153,50 @@ __device__ static __forceinline__ void activation_quantize_body(const struct act
         (uint2_t){quantize_operand_pair(carried[0], carried[2], code_exponent), quantize_operand_pair(carried[1], carried[3], code_exponent)};
     if (q % 8u == 0u) {
         (arena + arguments.exponents_offset)[vector * (arguments.width / 32u) + first / 32u] = (unsigned char)code_exponent;
+    }
+}
+
+/* thread q of a vector's width / 4 of vector `vector` */
+__device__ static __forceinline__ void activation_quantize_body(const struct activation_quantize_arguments &arguments, unsigned char *arena,
+                                                                uint32_t q, uint64_t vector)
+{
+    const uint32_t first = quantize_first_of(q);
+    if (first >= arguments.width) {
+        return; /* the width is a multiple of 64: whole groups of sixteen threads leave together */
+    }
+    const uint16_t *values = (const uint16_t *)(arena + arguments.values_offset) + vector * arguments.width + first;
+    const uint32_t near_pair = *(const uint32_t *)values, far_pair = *(const uint32_t *)(values + 8);
+    const uint32_t bits[4] = {near_pair & 0xFFFFu, near_pair >> 16, far_pair & 0xFFFFu, far_pair >> 16};
+    activation_quantize_values(arguments, arena, q, vector, bits);
+}
+
+/* thread q of vector `vector`: activation_quantize_128_entry's work of one thread */
+__device__ static __forceinline__ void activation_quantize_128_body(const struct activation_quantize_arguments &arguments, unsigned char *arena,
+                                                                    uint32_t q, uint64_t vector)
+{
+    /* the threads' values as in activation_quantize_entry: thread q = 16 l + 4 s + t takes 64 l + 16 s + 2 t + {0, 1, 8, 9},
+     * one word of codes; the 128 values of a scale are those of 32 neighbouring threads */
+    const uint32_t l = q / 16u, s = (q / 4u) % 4u, t = q % 4u, first = 64u * l + 16u * s + 2u * t;
+    if (first >= arguments.width) {
+        return; /* the width is a multiple of 128: whole groups of 32 threads leave together */
+    }
+    const uint16_t *values = (const uint16_t *)(arena + arguments.values_offset) + vector * arguments.width + first;
+    const uint32_t near_pair = *(const uint32_t *)values, far_pair = *(const uint32_t *)(values + 8);
+    const uint32_t bits[4] = {near_pair & 0xFFFFu, near_pair >> 16, far_pair & 0xFFFFu, far_pair >> 16};
+    float largest = fmaxf(fmaxf(fabsf(bf16_to_float((uint16_t)bits[0])), fabsf(bf16_to_float((uint16_t)bits[1]))),
+                          fmaxf(fabsf(bf16_to_float((uint16_t)bits[2])), fabsf(bf16_to_float((uint16_t)bits[3]))));
+    largest = lanes_largest<1u>(lanes_largest<2u>(lanes_largest<4u>(lanes_largest<8u>(lanes_largest<16u>(largest)))));
+    const float scale = __fdiv_rn(fmaxf(largest, 1e-4f), 448.0f);
+    const float reciprocal = __fdiv_rn(1.0f, scale);
+    uint32_t code[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; i++) {
+        code[i] = quantize_quotient_code(quantize_quotient(bf16_to_float((uint16_t)bits[i]), scale, reciprocal), bits[i]);
+    }
+    *(uint32_t *)(arena + arguments.codes_offset + vector * arguments.width + quantize_word_of(l, s, t)) =
+        code[0] | (code[2] << 8) | (code[1] << 16) | (code[3] << 24); /* bytes: values +0, +8, +1, +9 */
+    if (q % 32u == 0u) {
+        ((float *)(arena + arguments.exponents_offset))[vector * (arguments.width / 128u) + first / 128u] = scale;
     }
 }
 

@@ -1,0 +1,65 @@
+"""Two launches queued as one (csrc/joined_launches.h) leave the bytes that they leave one after the other, in a queue and in a graph
+that is replayed."""
+import numpy as np
+import pytest
+
+from _oracle import normals, to_bf16
+from test_gpu_shared_join import amd, build, card, fresh_arena, say  # noqa: F401
+from test_joined_launches import rule
+
+pytestmark = pytest.mark.gpu
+
+
+def check(amd, card, launches, ranges, first, name):
+    """launches one by one, in one list and as a graph of three replays, from the same bytes"""
+    assert rule(name, launches[first], launches[first + 1], card.arena_bytes) is not None
+    results = []
+
+    def run(work):
+        for offset, size in ranges:
+            card.upload(offset, np.full(size, 0xEE, dtype=np.uint8))
+        work()
+        results.append([card.download(offset, size) for offset, size in ranges])
+    run(lambda: [card.run([launch]) for launch in launches])
+    run(lambda: card.run(launches))
+    graph = card.capture(launches)
+    for _ in range(3):
+        run(lambda: card.run_graph(graph))
+    assert any(np.any(got != 0xEE) for got in results[0])
+    for other in results[1:]:
+        for index, (one, joined) in enumerate(zip(results[0], other)):
+            assert np.array_equal(one, joined), (name, index)
+
+
+@pytest.mark.parametrize("rows,hidden,form", [(1, 128, "select"), (8, 1280, "select"), (3, 4096, "select"), (9, 256, "small"), (64, 1152, "small"),
+                                              (384, 128, "small"), (1, 1152, "place"), (385, 256, "place"), (1000, 1152, "place")])
+@pytest.mark.parametrize("wide_scales", [False, True])
+def test_router_and_quantizer(amd, card, rows, hidden, form, wide_scales):  # noqa: F811
+    say("joined launches:", form, rows, hidden, wide_scales)
+    layer, _, _ = build(amd, card, hidden, 128, rows, 6, rows + hidden)
+    layer.set_rows(to_bf16(normals(rows, rows * hidden)).reshape(rows, hidden))
+    quantize = layer.quantize_launch()[0]
+    if wide_scales:
+        quantize.kernel = layer.kernels.activation_quantize_128
+    outputs = [layer.ranges[name] for name in ("codes", "exponents", "operands")]
+    if form == "select":
+        launches, name, first = [layer.projection_launch()[0], layer.select_launch(0)[0]], "router_select_entry", 1
+        extra = [(layer.jobs_offset, rows * 6 * 96), (layer.affinities_offset, rows * layer.E * 4)]
+    else:
+        wide = layer.wide_router()
+        routed = list(wide.launches(small=form == "small"))
+        launches, name = [layer.projection_launch()[0]] + routed[:2 if form == "small" else 3], "router_wide_" + form
+        first = len(launches) - 1
+        extra = [(wide.ranges[key].byte_offset, wide.ranges[key].byte_count) for key in ("pairs", "runs", "tiles", "jobs")]
+    check(amd, card, launches + [quantize], [(r.byte_offset, r.byte_count) for r in outputs] + extra, first, name)
+
+
+@pytest.mark.parametrize("rows,inner", [(1, 128), (5, 640), (9, 1152), (70, 2176)])
+def test_hidden_and_quantizer(amd, card, rows, inner):  # noqa: F811
+    say("joined launches: hidden", rows, inner)
+    many = {} if rows <= 8 else {"gate_up_slices": 1, "down_slices": 1, "wide_form": amd.LINEAR_INTERLEAVED_CHUNK_BLOCKS}
+    layer, shared, _ = build(amd, card, 256, 256, rows, 1, rows, shared_inner=inner, **many)
+    layer.set_rows(to_bf16(normals(rows, rows * 256)).reshape(rows, 256))
+    card.run(layer.quantize_launch())
+    names = [name for name in shared.ranges if name not in ("streams", "post", "comb", "pair_output")]
+    check(amd, card, list(shared.launches()), [(shared.ranges[n].byte_offset, shared.ranges[n].byte_count) for n in names], 1, "trunk_hidden_entry")

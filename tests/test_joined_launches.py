@@ -1,0 +1,104 @@
+"""Which pairs of launches the backend queues as one (csrc/joined_launches.cpp): the rule over records alone, on the CPU. A pair whose
+quantizer touches what the other launch writes, or writes what it reads, stays two launches."""
+import ctypes as C
+import struct
+
+import pytest
+
+import anemone_amd as amd
+
+ROWS, E, P, H = 40, 64, 6, 256
+STEP = 1 << 20  # every range begins on a place of its own, further apart than any range is long
+
+
+class Joined(C.Structure):
+    _fields_ = [("grid", C.c_uint32 * 2), ("block", C.c_uint32), ("numbers", C.c_uint32 * 3)]
+
+
+def rule(name, first, second, arena=1 << 34):
+    lib = amd.library()
+    lib.joined_launch_of.restype = C.c_bool
+    lib.joined_launch_of.argtypes = [C.c_char_p, C.c_void_p, C.c_void_p, C.c_uint64, C.c_void_p]
+    out = Joined()
+    joins = lib.joined_launch_of(name.encode(), C.byref(first), C.byref(second), arena, C.byref(out))
+    return (list(out.grid), out.block, list(out.numbers)) if joins else None
+
+
+def launch(grid, block, record):
+    one = amd.launches_of(1)[0]
+    for d in range(3):
+        one.grid[d], one.block[d] = grid[d], (block, 1, 1)[d]
+    one.argument_byte_count = len(record)
+    C.memmove(one.argument, record, len(record))
+    return one
+
+
+def quantizer(values=STEP, codes=2 * STEP, exponents=3 * STEP, operands=4 * STEP, width=H, rows=ROWS, grid=None):
+    return launch(grid or ((width + 1023) // 1024, rows, 1), 256, struct.pack("<4Q2I", values, codes, exponents, operands, width, 0))
+
+
+# name: (offset of the member in the record, its bytes, written or not)
+SELECT = {"step": (0, 16, False), "scores": (1, ROWS * E * 4, False), "bias": (2, E * 4, False), "expert_offsets": (3, E * 24, False),
+          "affinities": (4, ROWS * E * 4, True), "jobs": (5, ROWS * P * 96, True)}
+TILES, JOBS = (ROWS * P + 63) // 64 + E, min(ROWS * P, (ROWS * P + 7 * E) // 8)
+WIDE = {"step": (0, 16, False), "expert_offsets": (3, E * 24, False), "picks": (5, ROWS * P * 8, False), "counts": (6, E * 4, False),
+        "pairs": (7, ROWS * P * 8, True), "runs": (8, E * 8, True), "tiles": (9, TILES * 32, True), "jobs": (10, JOBS * 96, True)}
+
+
+def router(name, **places):
+    wide = name != "router_select_entry"
+    members = [(16 + i) * STEP for i in range(14 if wide else 9)]
+    for member, place in places.items():
+        members[(WIDE if wide else SELECT)[member][0]] = place
+    return launch((1, 1, 1), 512, struct.pack("<%dQ5If" % len(members), *members, ROWS, 0, E, P, 0, 1.5))
+
+
+@pytest.mark.parametrize("name", ["router_select_entry", "router_wide_small", "router_wide_place"])
+def test_router_and_quantizer(name):
+    assert rule(name, router(name), quantizer()) == ([1 + ROWS // 2, 1], 512, [1, 1, ROWS])
+    assert rule(name, router(name), quantizer(width=1280, rows=3)) == ([4, 1], 512, [1, 2, 3])  # two blocks a vector: the last of six alone
+    for member, (_, size, written) in (SELECT if name == "router_select_entry" else WIDE).items():
+        for at, length, is_written in ((STEP, 2 * ROWS * H, False), (2 * STEP, ROWS * H, True), (3 * STEP, ROWS * H // 32, True), (4 * STEP, 2 * ROWS * H, True)):
+            meets = written or is_written
+            for place, overlaps in ((at + length, False), (at + length - 1, True), (at - size, False), (at - size + 1, True)):
+                joined = rule(name, router(name, **{member: place}), quantizer())
+                assert (joined is None) == (overlaps and meets), (name, member, at, place)
+
+
+def test_launches_that_are_not_whole():
+    name = "router_wide_small"
+    first = router(name)
+    assert rule(name, first, quantizer(width=1028, grid=(1, ROWS, 1))) is None  # four values no thread takes
+    assert rule(name, first, quantizer(grid=(1, ROWS, 2))) is None
+    assert rule(name, first, quantizer(width=0, grid=(1, ROWS, 1))) is None
+    assert rule(name, first, quantizer(), arena=ROWS * H - 1) is None
+    wrong = quantizer()
+    wrong.block[0] = 128
+    assert rule(name, first, wrong) is None
+    wrong = router(name)
+    wrong.dynamic_shared_byte_count = 16
+    assert rule(name, wrong, quantizer()) is None
+    many = quantizer(width=32, rows=0xFFFFFFFF)  # more blocks than a grid of 512 threads has
+    assert rule(name, first, many, arena=1 << 62) is None
+
+
+def hidden(gate=8 * STEP, up=9 * STEP, out=STEP, width=H, rows=ROWS):
+    return launch(((width + 2047) // 2048, rows, 1), 256, struct.pack("<3QIf", gate, up, out, width, 10.0))
+
+
+def test_hidden_and_quantizer():
+    name = "trunk_hidden_entry"
+    assert rule(name, hidden(), quantizer()) == ([1, ROWS], 256, [0, 0, 0])
+    assert rule(name, hidden(width=2080), quantizer(width=2080)) == ([3, ROWS], 256, [0, 0, 0])
+    assert rule(name, hidden(out=5 * STEP), quantizer()) is None  # other values
+    assert rule(name, hidden(rows=ROWS - 1), quantizer()) is None
+    assert rule(name, hidden(width=2 * H), quantizer()) is None
+    assert rule(name, hidden(width=264), quantizer(width=264)) is None  # no whole blocks of 32
+    size = 2 * ROWS * H
+    for member in ("gate", "up"):
+        assert rule(name, hidden(**{member: STEP}), quantizer()) is None  # in place
+        for at, length in ((STEP, size), (2 * STEP, ROWS * H), (3 * STEP, ROWS * H // 32), (4 * STEP, size)):
+            for place, overlaps in ((at + length, False), (at + length - 1, True), (at - size, False), (at - size + 1, True)):
+                assert (rule(name, hidden(**{member: place}), quantizer()) is None) == overlaps
+    for member in ("codes", "exponents", "operands"):
+        assert rule(name, hidden(), quantizer(**{member: STEP + size - 1})) is None
