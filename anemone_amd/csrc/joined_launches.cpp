@@ -10,6 +10,7 @@
 namespace {
 
 constexpr uint32_t ROUTER_BLOCK = 512u;       /* threads of the router's launches that are joined, and of their joined kernels */
+constexpr uint32_t MOST_GRID_ROWS = 65534u;
 constexpr uint32_t MOST_BLOCKS = 1u << 22;    /* of 512 threads: the runtime counts a grid's threads in 32 bits */
 
 struct byte_range {
@@ -71,6 +72,29 @@ bool join_hidden(const struct kernel_launch &first, const struct kernel_launch &
     return true;
 }
 
+bool join_gate_up(const struct kernel_launch &first, const struct kernel_launch &second, uint64_t arena_bytes, struct joined_launch &out)
+{
+    const auto gate_up = record_of<expert_gate_up_arguments>(first);
+    const auto quantize = record_of<activation_quantize_arguments>(second);
+    const uint32_t block = first.block[0];
+    if (!is_plain(first, block) || !quantizer_is_whole(second, quantize, arena_bytes) || gate_up.output_size != quantize.width ||
+        gate_up.output_size % 32u != 0 || gate_up.hidden_offset != quantize.values_offset || gate_up.pair_count != second.grid[1] ||
+        gate_up.pair_count > EXPERT_JOINED_MOST_PAIRS || gate_up.pairs_per_row == 0 || gate_up.input_size > arena_bytes || first.grid[1] > MOST_GRID_ROWS) {
+        return false;
+    }
+    const uint64_t values = (uint64_t)second.grid[1] * quantize.width, jobs = first.grid[1];
+    const uint64_t inputs = ((uint64_t)gate_up.pair_count + gate_up.pairs_per_row - 1u) / gate_up.pairs_per_row * gate_up.input_size;
+    const byte_range outputs[] = {{quantize.codes_offset, values}, {quantize.exponents_offset, values / 32u}, {quantize.operands_offset, 2u * values}};
+    /* the matrices, which the jobs name, are nobody's output */
+    const byte_range read[] = {{gate_up.jobs_offset, jobs * sizeof(struct expert_job_record)}, {gate_up.codes_offset, inputs}, {gate_up.exponents_offset, inputs / 32u}};
+    const byte_range own[] = {{gate_up.hidden_offset, 2u * values}};
+    if (!all_apart(outputs, read) || !all_apart(outputs, own) || !all_apart(read, own)) {
+        return false;
+    }
+    out = {{first.grid[0], (uint32_t)jobs + 1u}, block, {(uint32_t)jobs, 0, 0}};
+    return true;
+}
+
 bool join_router(const char *function, const struct kernel_launch &first, const struct kernel_launch &second, uint64_t arena_bytes,
                  struct joined_launch &out)
 {
@@ -122,6 +146,11 @@ bool join_router(const char *function, const struct kernel_launch &first, const 
 extern "C" bool joined_launch_of(const char *first_function, const struct kernel_launch &first, const struct kernel_launch &second, uint64_t arena_bytes,
                       struct joined_launch &out)
 {
-    return std::strcmp(first_function, KERNEL_TRUNK_HIDDEN) == 0 ? join_hidden(first, second, arena_bytes, out)
-                                                                 : join_router(first_function, first, second, arena_bytes, out);
+    if (std::strcmp(first_function, KERNEL_TRUNK_HIDDEN) == 0) {
+        return join_hidden(first, second, arena_bytes, out);
+    }
+    if (std::strncmp(first_function, KERNEL_EXPERT_GATE_UP_STEM, sizeof KERNEL_EXPERT_GATE_UP_STEM - 1u) == 0) {
+        return join_gate_up(first, second, arena_bytes, out);
+    }
+    return join_router(first_function, first, second, arena_bytes, out);
 }

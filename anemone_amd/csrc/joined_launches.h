@@ -3,6 +3,7 @@
  * works (ANEMONE_JOINED_KERNEL):
  *
  *   a router's select, small or place launch, then the quantizer of the step's rows    the two side by side: neither may touch what the other writes
+ *   the experts' gate and up of a few pairs, then the quantizer of the hidden vectors  a block quantizes what it formed (EXPERT_JOINED_MOST_PAIRS)
  *   the shared expert's hidden step, then the quantizer of its values                  the one's values are the other's, a thread both
  *
  * Every byte that the two launches write is written, with the same value. A pair whose records do not show by themselves that this is

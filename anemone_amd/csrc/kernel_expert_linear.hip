@@ -387,6 +387,86 @@ EXPERT_ENTRIES(2);
 EXPERT_ENTRIES(4);
 EXPERT_ENTRIES(8);
 
+/* ---- gate and up, and the quantizer of the hidden vectors behind it, as one launch ---------------------------
+ * Run so by the backend where the two stand next to each other in a list (joined_launches.h): the producer above, for weights of either
+ * lane order. A strip's hidden values pass through LDS to eight threads a block of 32; one more row of blocks quantizes, from memory, the
+ * pairs that stand in no job, which it finds with one trip to the table, a thread a job. Grid (gate and up's, jobs + 1). Bound by
+ * what gate and up are, and a launch less: one row of FP4, 2048 x 896, six picks: a pass 22.7 -> 21.0 us. */
+template <uint32_t S, bool BYTES, bool NATIVE>
+__device__ static __forceinline__ void joined_gate_up_quantize(const struct expert_gate_up_arguments &arguments,
+                                                               const struct activation_quantize_arguments &quantize, unsigned char *arena, uint32_t jobs_number)
+{
+    constexpr uint32_t STRIP = strip_chain<2, BYTES, false, NATIVE>::STRIP, STRIP_OUTPUTS = STRIP * 16u, THREADS = S * WAVE, VECTOR_THREADS = STRIP_OUTPUTS / 4u;
+    __shared__ __attribute__((aligned(16))) uint16_t strip_hidden[LINEAR_MAXIMUM_ROWS][STRIP_OUTPUTS];
+    __shared__ uint32_t routed[EXPERT_JOINED_MOST_PAIRS / 32u];
+    const struct expert_job_record *jobs = (const struct expert_job_record *)(arena + arguments.jobs_offset);
+    const uint32_t tiles = arguments.output_size / 16u, first_output = blockIdx.x * STRIP_OUTPUTS;
+    /* a last strip that reaches past the matrix starts earlier: its first blocks of 32 are the strip's before it */
+    const uint32_t tile0 = blockIdx.x * STRIP + STRIP <= tiles ? blockIdx.x * STRIP : tiles - STRIP;
+    const uint32_t first_q = tile0 * 4u; /* of the quantizer's threads of a vector, four values each */
+    if (blockIdx.y == jobs_number) {
+        for (uint32_t word = threadIdx.x; word < EXPERT_JOINED_MOST_PAIRS / 32u; word += THREADS) {
+            routed[word] = 0u;
+        }
+        __syncthreads();
+        for (uint32_t job = threadIdx.x; job < jobs_number; job += THREADS) {
+            const uint32_t row_count = jobs[job].row_count;
+            uint32_t pairs[LINEAR_MAXIMUM_ROWS];
+#pragma unroll
+            for (uint32_t column = 0; column < LINEAR_MAXIMUM_ROWS; column++) {
+                pairs[column] = jobs[job].pair_index[column];
+            }
+#pragma unroll
+            for (uint32_t column = 0; column < LINEAR_MAXIMUM_ROWS; column++) {
+                if (column < row_count && pairs[column] < EXPERT_JOINED_MOST_PAIRS) {
+                    atomicOr(&routed[pairs[column] / 32u], 1u << (pairs[column] % 32u));
+                }
+            }
+        }
+        __syncthreads();
+        for (uint32_t index = threadIdx.x; index < arguments.pair_count * VECTOR_THREADS; index += THREADS) {
+            const uint32_t pair = index / VECTOR_THREADS, q = first_q + index % VECTOR_THREADS;
+            if (((routed[pair / 32u] >> (pair % 32u)) & 1u) == 0u && quantize_first_of(q) / 32u * 32u >= first_output) {
+                activation_quantize_body(quantize, arena, q, pair);
+            }
+        }
+        return;
+    }
+    const struct expert_job_record *job = jobs + blockIdx.y;
+    if (job->row_count == 0u) {
+        return;
+    }
+    expert_gate_up<S, BYTES, false, NATIVE>(arguments, arena, &strip_hidden[0][0]);
+    __syncthreads();
+    for (uint32_t index = threadIdx.x; index < job->row_count * VECTOR_THREADS; index += THREADS) {
+        const uint32_t column = index / VECTOR_THREADS, q = first_q + index % VECTOR_THREADS, first = quantize_first_of(q);
+        if (first / 32u * 32u >= first_output) {
+            const uint16_t *values = &strip_hidden[column][first - tile0 * 16u];
+            const uint32_t near_pair = *(const uint32_t *)values, far_pair = *(const uint32_t *)(values + 8);
+            const uint32_t bits[4] = {near_pair & 0xFFFFu, near_pair >> 16, far_pair & 0xFFFFu, far_pair >> 16};
+            activation_quantize_values(quantize, arena, q, job->pair_index[column], bits);
+        }
+    }
+}
+
+#define GATE_UP_JOIN(entry, S, bytes, native)                                                                                          \
+    extern "C" __global__ void __launch_bounds__(S * WAVE)                                                                             \
+        entry##_joined(struct expert_gate_up_arguments arguments, struct activation_quantize_arguments quantize, unsigned char *arena, uint32_t jobs, \
+                       uint32_t, uint32_t)                                                                                             \
+    {                                                                                                                                  \
+        joined_gate_up_quantize<S, bytes, native>(arguments, quantize, arena, jobs);                                                   \
+    }                                                                                                                                  \
+    ANEMONE_JOINED_KERNEL(KERNEL_FILE_EXPERT_LINEAR, entry, KERNEL_FILE_ACTIVATION_QUANTIZE, activation_quantize_entry, entry##_joined)
+#define GATE_UP_JOINS(S)                                     \
+    GATE_UP_JOIN(expert_gate_up_##S, S, false, false);       \
+    GATE_UP_JOIN(expert_gate_up_e4m3_##S, S, true, false);   \
+    GATE_UP_JOIN(expert_gate_up_gfx950_##S, S, false, true); \
+    GATE_UP_JOIN(expert_gate_up_e4m3_gfx950_##S, S, true, true)
+GATE_UP_JOINS(1);
+GATE_UP_JOINS(2);
+GATE_UP_JOINS(4);
+GATE_UP_JOINS(8);
+
 /* float32 sum of a row's bfloat16 pair outputs from +0 in ascending slot order; a thread takes
  * EXPERT_ROW_SUM_CHANNELS consecutive outputs (one 16-byte load a slot); grid (ceil(width / (8 x 256)), rows). Bound by
  * memory, and in a small step by its trips: a row's slots are asked for together, and as a stream, since nothing reads them

@@ -516,6 +516,10 @@ ANEMONE_RECORD_HAS(expert_gate_up_arguments, 64);
  * quantization of the hidden vectors in one launch */
 #define KERNEL_EXPERT_GATE_UP_QUANTIZE_STEM "expert_gate_up_quantize_"
 #define EXPERT_PRODUCER_MOST_PAIRS (LINEAR_MAXIMUM_ROWS * ROUTER_MOST_PICKS)
+/* of gate/up and the quantizer in one launch (csrc/joined_launches.h). A pass, us, as two launches -> as one: 6 pairs 22.7 -> 21.0, 4 pairs 30.9 ->
+ * 29.5, 32 pairs 58.9 -> 58.3, 64 pairs 126.0 -> 124.5, a site of 8 pairs 38.4 -> 36.6; 72 pairs 107.2 -> 106.9, 120 pairs 65.9 -> 66.2, 400 pairs 148.0 ->
+ * 149.5: the quantizing of many jobs' blocks stands behind their own products, where a launch of its own has the whole card */
+#define EXPERT_JOINED_MOST_PAIRS 64u
 struct expert_gate_up_quantize_arguments {
     uint64_t jobs_offset;
     uint64_t codes_offset;            /* the rows' quantized input: as expert_gate_up_arguments */

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 from _oracle import normals, to_bf16
+from anemone_amd import workloads
 from test_gpu_shared_join import amd, build, card, fresh_arena, say  # noqa: F401
 from test_joined_launches import rule
 
@@ -63,3 +64,25 @@ def test_hidden_and_quantizer(amd, card, rows, inner):  # noqa: F811
     card.run(layer.quantize_launch())
     names = [name for name in shared.ranges if name not in ("streams", "post", "comb", "pair_output")]
     check(amd, card, list(shared.launches()), [(shared.ranges[n].byte_offset, shared.ranges[n].byte_count) for n in names], 1, "trunk_hidden_entry")
+
+
+@pytest.mark.parametrize("rows,live,inner,slices", [(1, 1, 128, 1), (8, 8, 640, 4), (8, 5, 384, 2), (3, 2, 256, 8)])
+@pytest.mark.parametrize("weights", ["e2m1", "e4m3", "e2m1_gfx950", "e4m3_gfx950"])
+def test_gate_up_and_quantizer(amd, card, rows, live, inner, slices, weights):  # noqa: F811
+    """Every slice instance; pairs that stand in no job, whose hidden values are quantized as they lie."""
+    say("joined launches: gate and up", rows, live, inner, slices, weights)
+    fmt = {"e2m1": amd.WEIGHT_FORMAT_E2M1_SCALED, "e4m3": amd.WEIGHT_FORMAT_E4M3_SCALED, "e2m1_gfx950": amd.WEIGHT_FORMAT_E2M1_GFX950,
+           "e4m3_gfx950": amd.WEIGHT_FORMAT_E4M3_GFX950}[weights]
+    hidden, experts, picks = 1024, 64, 8
+    matrix = workloads.fp4_matrix if weights.startswith("e2m1") else workloads.fp8_matrix
+    trios = [[matrix(3 * e, inner, hidden), matrix(3 * e + 1, inner, hidden), matrix(3 * e + 2, hidden, inner)] for e in range(2)]
+    router = to_bf16(normals(5, experts * hidden) * 0.02).reshape(experts, hidden)
+    layer = amd.Fp4Layer(card, hidden, inner, experts, picks, rows, [trios[e % 2] for e in range(experts)], router_weights_bf16=router, weight_format=fmt)
+    layer.gate_up_slices, layer.down_slices = slices, min(slices, 2)
+    layer.set_rows(to_bf16(normals(rows, rows * hidden)).reshape(rows, hidden))
+    card.upload(layer.step_offset, amd.step_block(live))
+    card.run([layer.projection_launch()[0], layer.select_launch(0)[0], layer.quantize_launch()[0]])
+    names = ("hidden", "hidden_codes", "hidden_exponents", "hidden_operands", "pair_output", "row_output")
+    infix = {"e2m1": "", "e4m3": "e4m3_", "e2m1_gfx950": "gfx950_", "e4m3_gfx950": "e4m3_gfx950_"}[weights]
+    check(amd, card, list(layer.expert_launches()), [(layer.ranges[n].byte_offset, layer.ranges[n].byte_count) for n in names], 0,
+          "expert_gate_up_%s%d" % (infix, slices))

@@ -102,3 +102,26 @@ def test_hidden_and_quantizer():
                 assert (rule(name, hidden(**{member: place}), quantizer()) is None) == overlaps
     for member in ("codes", "exponents", "operands"):
         assert rule(name, hidden(), quantizer(**{member: STEP + size - 1})) is None
+
+
+def gate_up(jobs=8 * STEP, codes=9 * STEP, exponents=10 * STEP, out=STEP, width=H, inputs=384, pairs=ROWS, picks=4, job_count=30, grid_x=None):
+    record = struct.pack("<5Q4IfI", jobs, codes, exponents, 11 * STEP, out, width, inputs, pairs, picks, 10.0, 0)
+    return launch((grid_x or (width + 63) // 64, job_count, 1), 256, record)
+
+
+@pytest.mark.parametrize("name", ["expert_gate_up_4", "expert_gate_up_e4m3_gfx950_4"])
+def test_gate_up_and_quantizer(name):
+    assert rule(name, gate_up(), quantizer()) == ([4, 31], 256, [30, 0, 0])
+    assert rule(name, gate_up(pairs=64), quantizer(rows=64)) is not None
+    assert rule(name, gate_up(pairs=65), quantizer(rows=65)) is None  # more pairs than one launch takes
+    assert rule(name, gate_up(pairs=ROWS - 1), quantizer()) is None
+    assert rule(name, gate_up(out=5 * STEP), quantizer()) is None
+    assert rule(name, gate_up(width=2 * H), quantizer()) is None
+    assert rule(name, gate_up(width=272), quantizer(width=272)) is None  # no whole blocks of 32
+    rows = (ROWS + 3) // 4
+    for member, size in (("jobs", 30 * 96), ("codes", rows * 384), ("exponents", rows * 12)):
+        for at, length in ((STEP, 2 * ROWS * H), (2 * STEP, ROWS * H), (3 * STEP, ROWS * H // 32), (4 * STEP, 2 * ROWS * H)):
+            for place, overlaps in ((at + length, False), (at + length - 1, True), (at - size, False), (at - size + 1, True)):
+                assert (rule(name, gate_up(**{member: place}), quantizer()) is None) == overlaps, (member, at, place)
+    for member in ("codes", "exponents", "operands"):
+        assert rule(name, gate_up(), quantizer(**{member: STEP + 2 * ROWS * H - 1})) is None
