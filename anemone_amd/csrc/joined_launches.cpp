@@ -1,6 +1,7 @@
 /* joined_launches.cpp -- see joined_launches.h. Host code over the launches' records alone. */
 #include "joined_launches.h"
 
+#include <cstdlib>
 #include <cstring>
 
 #include <hip/hip_runtime.h> /* what the records mark their functions with */
@@ -72,12 +73,18 @@ bool join_hidden(const struct kernel_launch &first, const struct kernel_launch &
     return true;
 }
 
-bool join_gate_up(const struct kernel_launch &first, const struct kernel_launch &second, uint64_t arena_bytes, struct joined_launch &out)
+bool join_gate_up(const char *function, const struct kernel_launch &first, const struct kernel_launch &second, uint64_t arena_bytes,
+                  struct joined_launch &out)
 {
     const auto gate_up = record_of<expert_gate_up_arguments>(first);
     const auto quantize = record_of<activation_quantize_arguments>(second);
-    const uint32_t block = first.block[0];
-    if (!is_plain(first, block) || !quantizer_is_whole(second, quantize, arena_bytes) || gate_up.output_size != quantize.width ||
+    /* expert_gate_up_[e4m3_][gfx950_]<S>: the weights' bytes and the slices, a wavefront each */
+    const char *const form = function + sizeof KERNEL_EXPERT_GATE_UP_STEM - 1u;
+    const uint32_t strip = EXPERT_STRIP_OUTPUTS(std::strncmp(form, "e4m3_", 5) == 0);
+    const uint32_t block = 64u * (uint32_t)std::strtoul(std::strrchr(function, '_') + 1, nullptr, 10);
+    /* a block quantizes the outputs of its own strip alone: there is one for every strip */
+    if (!is_plain(first, block) || first.grid[0] != gate_up.output_size / strip + (gate_up.output_size % strip != 0 ? 1u : 0u) ||
+        gate_up.output_size < strip || !quantizer_is_whole(second, quantize, arena_bytes) || gate_up.output_size != quantize.width ||
         gate_up.output_size % 32u != 0 || gate_up.hidden_offset != quantize.values_offset || gate_up.pair_count != second.grid[1] ||
         gate_up.pair_count > EXPERT_JOINED_MOST_PAIRS || gate_up.pairs_per_row == 0 || gate_up.input_size > arena_bytes || first.grid[1] > MOST_GRID_ROWS) {
         return false;
@@ -150,7 +157,7 @@ extern "C" bool joined_launch_of(const char *first_function, const struct kernel
         return join_hidden(first, second, arena_bytes, out);
     }
     if (std::strncmp(first_function, KERNEL_EXPERT_GATE_UP_STEM, sizeof KERNEL_EXPERT_GATE_UP_STEM - 1u) == 0) {
-        return join_gate_up(first, second, arena_bytes, out);
+        return join_gate_up(first_function, first, second, arena_bytes, out);
     }
     return join_router(first_function, first, second, arena_bytes, out);
 }

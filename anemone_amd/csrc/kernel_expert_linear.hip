@@ -397,6 +397,7 @@ __device__ static __forceinline__ void joined_gate_up_quantize(const struct expe
                                                                const struct activation_quantize_arguments &quantize, unsigned char *arena, uint32_t jobs_number)
 {
     constexpr uint32_t STRIP = strip_chain<2, BYTES, false, NATIVE>::STRIP, STRIP_OUTPUTS = STRIP * 16u, THREADS = S * WAVE, VECTOR_THREADS = STRIP_OUTPUTS / 4u;
+    static_assert(STRIP_OUTPUTS == EXPERT_STRIP_OUTPUTS(BYTES), "the strips the host counts are the kernel's");
     __shared__ __attribute__((aligned(16))) uint16_t strip_hidden[LINEAR_MAXIMUM_ROWS][STRIP_OUTPUTS];
     __shared__ uint32_t routed[EXPERT_JOINED_MOST_PAIRS / 32u];
     const struct expert_job_record *jobs = (const struct expert_job_record *)(arena + arguments.jobs_offset);

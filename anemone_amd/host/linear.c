@@ -19,7 +19,6 @@
 
 #define ROW_SUM_BLOCK_OUTPUTS (EXPERT_ROW_SUM_CHANNELS * LINEAR_ELEMENT_THREADS) /* outputs a block of the row sum takes */
 #define QUANTIZE_BLOCK_VALUES (4u * LINEAR_ELEMENT_THREADS) /* a thread of activation_quantize_entry takes four values */
-#define LINEAR_STRIP_OUTPUTS 64u /* a block of the expert kernels: a strip of four tiles of 16 outputs */
 static const uint32_t slice_counts[LINEAR_SLICE_INSTANCES] = {1u, 2u, 4u, 8u, 16u};
 #define BUILT_INSTANCES 4u
 #define MOST_ROWS 4096u /* rows of one call: a wide step's chunk */
@@ -262,7 +261,7 @@ result_status linear_routed_experts_prepare(const struct linear_routed_experts_d
                         description->weight_format == WEIGHT_FORMAT_E4M3_BLOCK128_GFX950;
     const bool bytes = description->weight_format == WEIGHT_FORMAT_E4M3_SCALED || description->weight_format == WEIGHT_FORMAT_E4M3_GFX950 || block128;
     const bool nibbles = description->weight_format == WEIGHT_FORMAT_E2M1_SCALED || description->weight_format == WEIGHT_FORMAT_E2M1_GFX950;
-    const uint32_t strip_outputs = bytes ? LINEAR_STRIP_OUTPUTS / 2u : LINEAR_STRIP_OUTPUTS;
+    const uint32_t strip_outputs = EXPERT_STRIP_OUTPUTS(bytes);
     if (description->reserved_zero != 0 || (!nibbles && !bytes) || format == NULL ||
         format->stored_byte_count(gate_up, &gate_up_bytes) != STATUS_OK ||
         format->stored_byte_count(down, &down_bytes) != STATUS_OK || gate_up->input_size % 128u != 0 ||
@@ -732,7 +731,7 @@ static result_status wide_experts_prepare(const struct linear_wide_experts_descr
     const enum weight_format_code nibbles_format = native ? WEIGHT_FORMAT_E2M1_GFX950 : WEIGHT_FORMAT_E2M1_SCALED;
     const enum weight_format_code bytes_format = native ? WEIGHT_FORMAT_E4M3_GFX950 : WEIGHT_FORMAT_E4M3_SCALED;
     const bool bytes = experts->weight_format == bytes_format || block128;
-    const uint32_t strip_outputs = bytes ? LINEAR_STRIP_OUTPUTS / 2u : LINEAR_STRIP_OUTPUTS;
+    const uint32_t strip_outputs = EXPERT_STRIP_OUTPUTS(bytes);
     uint64_t gate_up_bytes = 0, down_bytes = 0;
     if (description->reserved_zero != 0 || experts->reserved_zero != 0 || (experts->weight_format != nibbles_format && !bytes) ||
         format == NULL || format->stored_byte_count(gate_up, &gate_up_bytes) != STATUS_OK ||

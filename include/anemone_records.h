@@ -486,6 +486,7 @@ ANEMONE_INLINE struct exl3_tcp_layout exl3_tcp_layout_of(uint64_t rows, uint64_t
 #define KERNEL_EXPERT_GATE_UP_STEM "expert_gate_up_"
 #define KERNEL_EXPERT_DOWN_STEM "expert_down_"
 #define KERNEL_EXPERT_ROW_SUM "expert_row_sum_entry"
+#define EXPERT_STRIP_OUTPUTS(one_byte) ((one_byte) ? 32u : 64u) /* outputs of a block of gate/up and of down, of one-byte and of 4-bit weights */
 
 struct activation_quantize_arguments {
     uint64_t values_offset;    /* read: bf16 [V][width] */

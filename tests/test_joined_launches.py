@@ -104,14 +104,16 @@ def test_hidden_and_quantizer():
         assert rule(name, hidden(), quantizer(**{member: STEP + size - 1})) is None
 
 
-def gate_up(jobs=8 * STEP, codes=9 * STEP, exponents=10 * STEP, out=STEP, width=H, inputs=384, pairs=ROWS, picks=4, job_count=30, grid_x=None):
+def whole_gate_up(jobs=8 * STEP, codes=9 * STEP, exponents=10 * STEP, out=STEP, width=H, inputs=384, pairs=ROWS, picks=4, job_count=30, strip=64, grid_x=None, block=256):
     record = struct.pack("<5Q4IfI", jobs, codes, exponents, 11 * STEP, out, width, inputs, pairs, picks, 10.0, 0)
-    return launch((grid_x or (width + 63) // 64, job_count, 1), 256, record)
+    return launch((grid_x or (width + strip - 1) // strip, job_count, 1), block, record)
 
 
-@pytest.mark.parametrize("name", ["expert_gate_up_4", "expert_gate_up_e4m3_gfx950_4"])
-def test_gate_up_and_quantizer(name):
-    assert rule(name, gate_up(), quantizer()) == ([4, 31], 256, [30, 0, 0])
+@pytest.mark.parametrize("name,strip", [("expert_gate_up_4", 64), ("expert_gate_up_e4m3_gfx950_4", 32)])
+def test_gate_up_and_quantizer(name, strip):
+    def gate_up(**changes):
+        return whole_gate_up(strip=strip, **changes)
+    assert rule(name, gate_up(), quantizer()) == ([H // strip, 31], 256, [30, 0, 0])
     assert rule(name, gate_up(pairs=64), quantizer(rows=64)) is not None
     assert rule(name, gate_up(pairs=65), quantizer(rows=65)) is None  # more pairs than one launch takes
     assert rule(name, gate_up(pairs=ROWS - 1), quantizer()) is None
@@ -125,3 +127,19 @@ def test_gate_up_and_quantizer(name):
                 assert (rule(name, gate_up(**{member: place}), quantizer()) is None) == overlaps, (member, at, place)
     for member in ("codes", "exponents", "operands"):
         assert rule(name, gate_up(), quantizer(**{member: STEP + 2 * ROWS * H - 1})) is None
+
+
+@pytest.mark.parametrize("infix,strip", [("", 64), ("gfx950_", 64), ("e4m3_", 32), ("e4m3_gfx950_", 32)])
+@pytest.mark.parametrize("slices", [1, 2, 4, 8])
+def test_gate_up_of_fewer_blocks_than_strips(infix, strip, slices):
+    """The quantizer's launch covers whole vectors, a joined block its own strip alone."""
+    name = "expert_gate_up_%s%d" % (infix, slices)
+    for width in (64, H, 11 * 64):
+        strips = width // strip
+
+        def joins(**changes):
+            launch = whole_gate_up(width=width, strip=strip, **{"block": 64 * slices, **changes})
+            return rule(name, launch, quantizer(width=width)) is not None
+        assert joins()
+        assert not any(joins(grid_x=grid) for grid in (1, strips - 1, strips + 1) if grid not in (0, strips))
+        assert not any(joins(block=block) for block in (32 * slices, 128 * slices))
