@@ -300,7 +300,8 @@ hipError_t launch_next(device_card *card, const kernel_launch *launches, uint32_
         const prepared_kernel &kernel = card->prepared[first.kernel];
         const uint32_t joins = kernel.joins[0] & card->prepared[second.kernel].joins[1];
         joined_launch joined;
-        if (joins != 0 && joined_launch_of(kernel_table()[kernel.index].function, first, second, card->arena_bytes, joined)) {
+        if (joins != 0 && joined_launch_of(kernel_table()[kernel.index].function, kernel_table()[card->prepared[second.kernel].index].function, first, second,
+                                           card->arena_bytes, joined)) {
             index++;
             void *arguments[6] = {(void *)first.argument, (void *)second.argument, (void *)&card->arena, &joined.numbers[0], &joined.numbers[1], &joined.numbers[2]};
             return hipLaunchKernel(joined_table()[(uint32_t)__builtin_ctz(joins)].host_function, dim3(joined.grid[0], joined.grid[1], 1), dim3(joined.block, 1, 1),

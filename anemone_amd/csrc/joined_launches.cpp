@@ -11,6 +11,7 @@
 namespace {
 
 constexpr uint32_t ROUTER_BLOCK = 512u;       /* threads of the router's launches that are joined, and of their joined kernels */
+constexpr uint32_t QUANTIZE_UNIT = 64u, QUANTIZE_128_UNIT = 128u; /* widths of activation_quantize_entry, _128_entry: multiples */
 constexpr uint32_t MOST_GRID_ROWS = 65534u;
 constexpr uint32_t MOST_BLOCKS = 1u << 22;    /* of 512 threads: the runtime counts a grid's threads in 32 bits */
 
@@ -47,19 +48,21 @@ bool is_plain(const struct kernel_launch &launch, uint32_t block)
     return launch.block[0] == block && launch.block[1] == 1 && launch.block[2] == 1 && launch.grid[2] == 1 && launch.dynamic_shared_byte_count == 0;
 }
 
-/* the quantizer's launch: its threads cover the vectors' width, and its values fit the arena (so that no product below wraps) */
-bool quantizer_is_whole(const struct kernel_launch &launch, const struct activation_quantize_arguments &record, uint64_t arena_bytes)
+/* the quantizer's launch: its threads cover the vectors' width, and its values fit the arena (so that no product below wraps). `unit`: the
+ * values that its lane order keeps together; a vector of a width that is no multiple of them is written past its end, into the next one's
+ * place */
+bool quantizer_is_whole(const struct kernel_launch &launch, const struct activation_quantize_arguments &record, uint32_t unit, uint64_t arena_bytes)
 {
-    return is_plain(launch, LINEAR_ELEMENT_THREADS) && record.width != 0 && (uint64_t)launch.grid[0] * LINEAR_ELEMENT_THREADS * 4u >= record.width &&
-           (uint64_t)launch.grid[1] * record.width <= arena_bytes;
+    return is_plain(launch, LINEAR_ELEMENT_THREADS) && record.width != 0 && record.width % unit == 0 &&
+           (uint64_t)launch.grid[0] * LINEAR_ELEMENT_THREADS * 4u >= record.width && (uint64_t)launch.grid[1] * record.width <= arena_bytes;
 }
 
 bool join_hidden(const struct kernel_launch &first, const struct kernel_launch &second, uint64_t arena_bytes, struct joined_launch &out)
 {
     const auto hidden = record_of<trunk_hidden_arguments>(first);
     const auto quantize = record_of<activation_quantize_arguments>(second);
-    if (!is_plain(first, LINEAR_ELEMENT_THREADS) || !quantizer_is_whole(second, quantize, arena_bytes) || first.grid[1] != second.grid[1] ||
-        hidden.width != quantize.width || hidden.width % 32u != 0 || hidden.hidden_offset != quantize.values_offset ||
+    if (!is_plain(first, LINEAR_ELEMENT_THREADS) || !quantizer_is_whole(second, quantize, QUANTIZE_UNIT, arena_bytes) || first.grid[1] != second.grid[1] ||
+        hidden.width != quantize.width || hidden.hidden_offset != quantize.values_offset ||
         (uint64_t)first.grid[0] * LINEAR_ELEMENT_THREADS * HYPER_VALUES_PER_THREAD < hidden.width) {
         return false;
     }
@@ -83,9 +86,8 @@ bool join_gate_up(const char *function, const struct kernel_launch &first, const
     const uint32_t strip = EXPERT_STRIP_OUTPUTS(std::strncmp(form, "e4m3_", 5) == 0);
     const uint32_t block = 64u * (uint32_t)std::strtoul(std::strrchr(function, '_') + 1, nullptr, 10);
     /* a block quantizes the outputs of its own strip alone: there is one for every strip */
-    if (!is_plain(first, block) || first.grid[0] != gate_up.output_size / strip + (gate_up.output_size % strip != 0 ? 1u : 0u) ||
-        gate_up.output_size < strip || !quantizer_is_whole(second, quantize, arena_bytes) || gate_up.output_size != quantize.width ||
-        gate_up.output_size % 32u != 0 || gate_up.hidden_offset != quantize.values_offset || gate_up.pair_count != second.grid[1] ||
+    if (!is_plain(first, block) || gate_up.output_size % strip != 0 || first.grid[0] != gate_up.output_size / strip ||
+        !quantizer_is_whole(second, quantize, QUANTIZE_UNIT, arena_bytes) || gate_up.output_size != quantize.width || gate_up.hidden_offset != quantize.values_offset || gate_up.pair_count != second.grid[1] ||
         gate_up.pair_count > EXPERT_JOINED_MOST_PAIRS || gate_up.pairs_per_row == 0 || gate_up.input_size > arena_bytes || first.grid[1] > MOST_GRID_ROWS) {
         return false;
     }
@@ -102,11 +104,12 @@ bool join_gate_up(const char *function, const struct kernel_launch &first, const
     return true;
 }
 
-bool join_router(const char *function, const struct kernel_launch &first, const struct kernel_launch &second, uint64_t arena_bytes,
+bool join_router(const char *function, const char *second_function, const struct kernel_launch &first, const struct kernel_launch &second, uint64_t arena_bytes,
                  struct joined_launch &out)
 {
+    const uint32_t unit = std::strcmp(second_function, KERNEL_ACTIVATION_QUANTIZE_128) == 0 ? QUANTIZE_128_UNIT : QUANTIZE_UNIT;
     const auto quantize = record_of<activation_quantize_arguments>(second);
-    if (!is_plain(first, ROUTER_BLOCK) || first.grid[1] != 1 || !quantizer_is_whole(second, quantize, arena_bytes)) {
+    if (!is_plain(first, ROUTER_BLOCK) || first.grid[1] != 1 || !quantizer_is_whole(second, quantize, unit, arena_bytes)) {
         return false;
     }
     const uint64_t values = (uint64_t)second.grid[1] * quantize.width;
@@ -150,8 +153,8 @@ bool join_router(const char *function, const struct kernel_launch &first, const 
 
 } // namespace
 
-extern "C" bool joined_launch_of(const char *first_function, const struct kernel_launch &first, const struct kernel_launch &second, uint64_t arena_bytes,
-                      struct joined_launch &out)
+extern "C" bool joined_launch_of(const char *first_function, const char *second_function, const struct kernel_launch &first,
+                                 const struct kernel_launch &second, uint64_t arena_bytes, struct joined_launch &out)
 {
     if (std::strcmp(first_function, KERNEL_TRUNK_HIDDEN) == 0) {
         return join_hidden(first, second, arena_bytes, out);
@@ -159,5 +162,5 @@ extern "C" bool joined_launch_of(const char *first_function, const struct kernel
     if (std::strncmp(first_function, KERNEL_EXPERT_GATE_UP_STEM, sizeof KERNEL_EXPERT_GATE_UP_STEM - 1u) == 0) {
         return join_gate_up(first_function, first, second, arena_bytes, out);
     }
-    return join_router(first_function, first, second, arena_bytes, out);
+    return join_router(first_function, second_function, first, second, arena_bytes, out);
 }

@@ -21,8 +21,8 @@ struct joined_launch {
     uint32_t numbers[3]; /* the kernel's arguments behind the records and the arena: the first launch's blocks, the second's grid */
 };
 
-/* first_function: the first launch's kernel, one of those named by ANEMONE_JOINED_KERNEL together with the second's */
-extern "C" bool joined_launch_of(const char *first_function, const struct kernel_launch &first, const struct kernel_launch &second, uint64_t arena_bytes,
-                      struct joined_launch &out);
+/* the launches' kernels: two of those that ANEMONE_JOINED_KERNEL names together */
+extern "C" bool joined_launch_of(const char *first_function, const char *second_function, const struct kernel_launch &first,
+                                 const struct kernel_launch &second, uint64_t arena_bytes, struct joined_launch &out);
 
 #endif

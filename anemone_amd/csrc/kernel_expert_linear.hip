@@ -396,15 +396,13 @@ template <uint32_t S, bool BYTES, bool NATIVE>
 __device__ static __forceinline__ void joined_gate_up_quantize(const struct expert_gate_up_arguments &arguments,
                                                                const struct activation_quantize_arguments &quantize, unsigned char *arena, uint32_t jobs_number)
 {
-    constexpr uint32_t STRIP = strip_chain<2, BYTES, false, NATIVE>::STRIP, STRIP_OUTPUTS = STRIP * 16u, THREADS = S * WAVE, VECTOR_THREADS = STRIP_OUTPUTS / 4u;
+    constexpr uint32_t STRIP_OUTPUTS = strip_chain<2, BYTES, false, NATIVE>::STRIP * 16u, THREADS = S * WAVE, VECTOR_THREADS = STRIP_OUTPUTS / 4u;
     static_assert(STRIP_OUTPUTS == EXPERT_STRIP_OUTPUTS(BYTES), "the strips the host counts are the kernel's");
     __shared__ __attribute__((aligned(16))) uint16_t strip_hidden[LINEAR_MAXIMUM_ROWS][STRIP_OUTPUTS];
     __shared__ uint32_t routed[EXPERT_JOINED_MOST_PAIRS / 32u];
     const struct expert_job_record *jobs = (const struct expert_job_record *)(arena + arguments.jobs_offset);
-    const uint32_t tiles = arguments.output_size / 16u, first_output = blockIdx.x * STRIP_OUTPUTS;
-    /* a last strip that reaches past the matrix starts earlier: its first blocks of 32 are the strip's before it */
-    const uint32_t tile0 = blockIdx.x * STRIP + STRIP <= tiles ? blockIdx.x * STRIP : tiles - STRIP;
-    const uint32_t first_q = tile0 * 4u; /* of the quantizer's threads of a vector, four values each */
+    /* the matrix is whole strips, a block each. first_q: of the quantizer's threads of a vector, four values each */
+    const uint32_t first_output = blockIdx.x * STRIP_OUTPUTS, first_q = first_output / 4u;
     if (blockIdx.y == jobs_number) {
         for (uint32_t word = threadIdx.x; word < EXPERT_JOINED_MOST_PAIRS / 32u; word += THREADS) {
             routed[word] = 0u;
@@ -427,7 +425,7 @@ __device__ static __forceinline__ void joined_gate_up_quantize(const struct expe
         __syncthreads();
         for (uint32_t index = threadIdx.x; index < arguments.pair_count * VECTOR_THREADS; index += THREADS) {
             const uint32_t pair = index / VECTOR_THREADS, q = first_q + index % VECTOR_THREADS;
-            if (((routed[pair / 32u] >> (pair % 32u)) & 1u) == 0u && quantize_first_of(q) / 32u * 32u >= first_output) {
+            if (((routed[pair / 32u] >> (pair % 32u)) & 1u) == 0u) {
                 activation_quantize_body(quantize, arena, q, pair);
             }
         }
@@ -440,13 +438,11 @@ __device__ static __forceinline__ void joined_gate_up_quantize(const struct expe
     expert_gate_up<S, BYTES, false, NATIVE>(arguments, arena, &strip_hidden[0][0]);
     __syncthreads();
     for (uint32_t index = threadIdx.x; index < job->row_count * VECTOR_THREADS; index += THREADS) {
-        const uint32_t column = index / VECTOR_THREADS, q = first_q + index % VECTOR_THREADS, first = quantize_first_of(q);
-        if (first / 32u * 32u >= first_output) {
-            const uint16_t *values = &strip_hidden[column][first - tile0 * 16u];
-            const uint32_t near_pair = *(const uint32_t *)values, far_pair = *(const uint32_t *)(values + 8);
-            const uint32_t bits[4] = {near_pair & 0xFFFFu, near_pair >> 16, far_pair & 0xFFFFu, far_pair >> 16};
-            activation_quantize_values(quantize, arena, q, job->pair_index[column], bits);
-        }
+        const uint32_t column = index / VECTOR_THREADS, q = first_q + index % VECTOR_THREADS;
+        const uint16_t *values = &strip_hidden[column][quantize_first_of(q) - first_output];
+        const uint32_t near_pair = *(const uint32_t *)values, far_pair = *(const uint32_t *)(values + 8);
+        const uint32_t bits[4] = {near_pair & 0xFFFFu, near_pair >> 16, far_pair & 0xFFFFu, far_pair >> 16};
+        activation_quantize_values(quantize, arena, q, job->pair_index[column], bits);
     }
 }
 

@@ -15,12 +15,12 @@ class Joined(C.Structure):
     _fields_ = [("grid", C.c_uint32 * 2), ("block", C.c_uint32), ("numbers", C.c_uint32 * 3)]
 
 
-def rule(name, first, second, arena=1 << 34):
+def rule(name, first, second, arena=1 << 34, quantize="activation_quantize_entry"):
     lib = amd.library()
     lib.joined_launch_of.restype = C.c_bool
-    lib.joined_launch_of.argtypes = [C.c_char_p, C.c_void_p, C.c_void_p, C.c_uint64, C.c_void_p]
+    lib.joined_launch_of.argtypes = [C.c_char_p, C.c_char_p, C.c_void_p, C.c_void_p, C.c_uint64, C.c_void_p]
     out = Joined()
-    joins = lib.joined_launch_of(name.encode(), C.byref(first), C.byref(second), arena, C.byref(out))
+    joins = lib.joined_launch_of(name.encode(), quantize.encode(), C.byref(first), C.byref(second), arena, C.byref(out))
     return (list(out.grid), out.block, list(out.numbers)) if joins else None
 
 
@@ -78,7 +78,7 @@ def test_launches_that_are_not_whole():
     wrong = router(name)
     wrong.dynamic_shared_byte_count = 16
     assert rule(name, wrong, quantizer()) is None
-    many = quantizer(width=32, rows=0xFFFFFFFF)  # more blocks than a grid of 512 threads has
+    many = quantizer(width=64, rows=0xFFFFFFFF)  # more blocks than a grid of 512 threads has
     assert rule(name, first, many, arena=1 << 62) is None
 
 
@@ -89,7 +89,7 @@ def hidden(gate=8 * STEP, up=9 * STEP, out=STEP, width=H, rows=ROWS):
 def test_hidden_and_quantizer():
     name = "trunk_hidden_entry"
     assert rule(name, hidden(), quantizer()) == ([1, ROWS], 256, [0, 0, 0])
-    assert rule(name, hidden(width=2080), quantizer(width=2080)) == ([3, ROWS], 256, [0, 0, 0])
+    assert rule(name, hidden(width=2112), quantizer(width=2112)) == ([3, ROWS], 256, [0, 0, 0])
     assert rule(name, hidden(out=5 * STEP), quantizer()) is None  # other values
     assert rule(name, hidden(rows=ROWS - 1), quantizer()) is None
     assert rule(name, hidden(width=2 * H), quantizer()) is None
@@ -143,3 +143,19 @@ def test_gate_up_of_fewer_blocks_than_strips(infix, strip, slices):
         assert joins()
         assert not any(joins(grid_x=grid) for grid in (1, strips - 1, strips + 1) if grid not in (0, strips))
         assert not any(joins(block=block) for block in (32 * slices, 128 * slices))
+
+
+@pytest.mark.parametrize("width", [32, 96, 1120, 2080, 264])
+def test_widths_the_quantizer_has_no_order_for(width):
+    """Its words of codes lie in groups of 64 values (one float32 scale: 128): a vector of another width is written past its
+    end, so that the ranges compared are not what is written."""
+    whole = (width + 63) // 64 * 64
+    for name in ("router_select_entry", "router_wide_small", "router_wide_place"):
+        assert rule(name, router(name), quantizer(width=width)) is None
+        assert rule(name, router(name), quantizer(width=whole)) is not None
+        wide = "activation_quantize_128_entry"
+        assert rule(name, router(name), quantizer(width=whole), quantize=wide) is None or whole % 128 == 0
+        assert rule(name, router(name), quantizer(width=2 * whole), quantize=wide) is not None
+    assert rule("trunk_hidden_entry", hidden(width=width), quantizer(width=width)) is None
+    for name, strip in (("expert_gate_up_4", 64), ("expert_gate_up_e4m3_4", 32)):
+        assert rule(name, whole_gate_up(width=width, strip=strip), quantizer(width=width)) is None
