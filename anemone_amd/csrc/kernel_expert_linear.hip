@@ -438,11 +438,14 @@ __device__ static __forceinline__ void joined_gate_up_quantize(const struct expe
     expert_gate_up<S, BYTES, false, NATIVE>(arguments, arena, &strip_hidden[0][0]);
     __syncthreads();
     for (uint32_t index = threadIdx.x; index < job->row_count * VECTOR_THREADS; index += THREADS) {
-        const uint32_t column = index / VECTOR_THREADS, q = first_q + index % VECTOR_THREADS;
+        const uint32_t column = index / VECTOR_THREADS, q = first_q + index % VECTOR_THREADS, pair = job->pair_index[column];
+        if (pair >= arguments.pair_count) {
+            continue; /* no vector of the quantizer's */
+        }
         const uint16_t *values = &strip_hidden[column][quantize_first_of(q) - first_output];
         const uint32_t near_pair = *(const uint32_t *)values, far_pair = *(const uint32_t *)(values + 8);
         const uint32_t bits[4] = {near_pair & 0xFFFFu, near_pair >> 16, far_pair & 0xFFFFu, far_pair >> 16};
-        activation_quantize_values(quantize, arena, q, job->pair_index[column], bits);
+        activation_quantize_values(quantize, arena, q, pair, bits);
     }
 }
 

@@ -66,11 +66,8 @@ def test_hidden_and_quantizer(amd, card, rows, inner):  # noqa: F811
     check(amd, card, list(shared.launches()), [(shared.ranges[n].byte_offset, shared.ranges[n].byte_count) for n in names], 1, "trunk_hidden_entry")
 
 
-@pytest.mark.parametrize("rows,live,inner,slices", [(1, 1, 128, 1), (8, 8, 640, 4), (8, 5, 384, 2), (3, 2, 256, 8)])
-@pytest.mark.parametrize("weights", ["e2m1", "e4m3", "e2m1_gfx950", "e4m3_gfx950"])
-def test_gate_up_and_quantizer(amd, card, rows, live, inner, slices, weights):  # noqa: F811
-    """Every slice instance; pairs that stand in no job, whose hidden values are quantized as they lie."""
-    say("joined launches: gate and up", rows, live, inner, slices, weights)
+def gate_up_layer(amd, card, rows, live, inner, slices, weights):  # noqa: F811
+    """A layer of 8 picks whose job table holds the pairs of `live` of its rows, and the kernel of its gate and up"""
     fmt = {"e2m1": amd.WEIGHT_FORMAT_E2M1_SCALED, "e4m3": amd.WEIGHT_FORMAT_E4M3_SCALED, "e2m1_gfx950": amd.WEIGHT_FORMAT_E2M1_GFX950,
            "e4m3_gfx950": amd.WEIGHT_FORMAT_E4M3_GFX950}[weights]
     hidden, experts, picks = 1024, 64, 8
@@ -82,7 +79,30 @@ def test_gate_up_and_quantizer(amd, card, rows, live, inner, slices, weights):  
     layer.set_rows(to_bf16(normals(rows, rows * hidden)).reshape(rows, hidden))
     card.upload(layer.step_offset, amd.step_block(live))
     card.run([layer.projection_launch()[0], layer.select_launch(0)[0], layer.quantize_launch()[0]])
-    names = ("hidden", "hidden_codes", "hidden_exponents", "hidden_operands", "pair_output", "row_output")
     infix = {"e2m1": "", "e4m3": "e4m3_", "e2m1_gfx950": "gfx950_", "e4m3_gfx950": "e4m3_gfx950_"}[weights]
-    check(amd, card, list(layer.expert_launches()), [(layer.ranges[n].byte_offset, layer.ranges[n].byte_count) for n in names], 0,
-          "expert_gate_up_%s%d" % (infix, slices))
+    return layer, "expert_gate_up_%s%d" % (infix, slices)
+
+
+@pytest.mark.parametrize("rows,live,inner,slices", [(1, 1, 128, 1), (8, 8, 640, 4), (8, 5, 384, 2), (3, 2, 256, 8)])
+@pytest.mark.parametrize("weights", ["e2m1", "e4m3", "e2m1_gfx950", "e4m3_gfx950"])
+def test_gate_up_and_quantizer(amd, card, rows, live, inner, slices, weights):  # noqa: F811
+    """Every slice instance; pairs that stand in no job, whose hidden values are quantized as they lie."""
+    say("joined launches: gate and up", rows, live, inner, slices, weights)
+    layer, kernel = gate_up_layer(amd, card, rows, live, inner, slices, weights)
+    names = ("hidden", "hidden_codes", "hidden_exponents", "hidden_operands", "pair_output", "row_output")
+    check(amd, card, list(layer.expert_launches()), [(layer.ranges[n].byte_offset, layer.ranges[n].byte_count) for n in names], 0, kernel)
+
+
+@pytest.mark.parametrize("pairs", [1, 21, 63])
+@pytest.mark.parametrize("weights", ["e2m1", "e4m3_gfx950"])
+def test_pairs_of_the_table_past_the_quantizer(amd, card, pairs, weights):  # noqa: F811
+    """A table that names 64 pairs, launches of fewer: the quantizer writes the vectors of its grid alone. Every range has
+    room for all 64."""
+    say("joined launches: gate and up, pairs", pairs, weights)
+    layer, kernel = gate_up_layer(amd, card, 8, 8, 384, 2, weights)
+    launches = list(layer.expert_launches())[:2]
+    launches[0].argument[48:52] = list(pairs.to_bytes(4, "little"))  # expert_gate_up_arguments.pair_count
+    launches[1].grid[1] = pairs
+    names = ("hidden", "hidden_codes", "hidden_exponents", "hidden_operands")
+    check(amd, card, launches, [(layer.ranges[n].byte_offset, layer.ranges[n].byte_count) for n in names], 0, kernel)
+    assert np.all(layer.card.download(layer.ranges["hidden_codes"].byte_offset, 64 * 384)[pairs * 384:] == 0xEE)
