@@ -331,6 +331,8 @@ def library():
             "backend_hip_measure_begin": [vp],
             "backend_hip_measure_end": [vp],
             "backend_hip_measure_elapsed_us": [vp, u64, C.POINTER(C.c_double)],
+            "backend_hip_launch_queued_as": [vp, launch_p, u32, C.POINTER(C.c_char_p), C.POINTER(u32)],
+            "backend_hip_joined_table_entry": [u32, C.POINTER(C.c_char_p), C.POINTER(C.c_char_p), C.POINTER(C.c_char_p)],
             "backend_hip_kernel_table_entry": [u32, C.POINTER(C.c_char_p), C.POINTER(C.c_char_p), C.POINTER(u32)],
             "exl3_reconstruct_prepare": [C.POINTER(Exl3ReconstructRecord), u64, u32, launch_p],
             "exl3_experts_prepare": [C.POINTER(Exl3ExpertRecord), u64, vp, vp, u32, launch_p],
@@ -398,6 +400,7 @@ def library():
         lib.backend_hip_format_supported.restype = C.c_bool
         lib.backend_hip_format_supported.argtypes = [u32, C.c_int]
         lib.backend_hip_kernel_table_count.restype = u32
+        lib.backend_hip_joined_table_count.restype = u32
         lib.exl3_scratch_byte_count.restype = u64
         lib.exl3_scratch_byte_count.argtypes = [u32, u32]
         lib.anemone_sha256.restype = None
@@ -545,6 +548,13 @@ class Card:
 
     def wait(self, seconds=60):
         check(self.lib.backend_hip_launch_wait(self.handle, seconds * SECOND), "launch_wait")
+
+    def queued_as(self, launches):
+        """(the kernel that run() queues launches[0] as, how many of the launches that is)."""
+        array = launches if isinstance(launches, C.Array) else (KernelLaunch * len(launches))(*launches)
+        name, count = C.c_char_p(), u32(0)
+        check(self.lib.backend_hip_launch_queued_as(self.handle, array, len(array), C.byref(name), C.byref(count)), "launch_queued_as")
+        return name.value.decode(), count.value
 
     def run_timed(self, launches):
         array = launches if isinstance(launches, C.Array) else (KernelLaunch * len(launches))(*launches)

@@ -40,10 +40,11 @@ std::vector<kernel_entry> &kernel_table()
 
 struct joined_entry {
     const char *files[2], *functions[2]; /* of the two launches */
+    const char *joined;
     const void *host_function;
 };
 
-#define MOST_JOINED_KERNELS 32u /* a bit each */
+#define MOST_JOINED_KERNELS 32u /* a bit each: a registration beyond them is refused */
 
 std::vector<joined_entry> &joined_table()
 {
@@ -56,7 +57,7 @@ uint32_t joins_of(const kernel_entry &entry, uint32_t launch)
 {
     uint32_t joins = 0;
     const std::vector<joined_entry> &table = joined_table();
-    for (uint32_t index = 0; index < table.size() && index < MOST_JOINED_KERNELS; index++) {
+    for (uint32_t index = 0; index < table.size(); index++) {
         if (std::strcmp(table[index].files[launch], entry.file) == 0 && std::strcmp(table[index].functions[launch], entry.function) == 0) {
             joins |= 1u << index;
         }
@@ -275,40 +276,51 @@ result_status launches_check(device_card *card, const kernel_launch *launches, u
     return STATUS_OK;
 }
 
-hipError_t launch_on(device_card *card, const kernel_launch &launch, hipStream_t stream)
-{
-    const kernel_entry &entry = kernel_table()[card->prepared[launch.kernel].index];
-    /* the record travels by value: the runtime copies record_bytes from the launch's own bytes */
-    void *arguments[2] = {(void *)launch.argument, (void *)&card->arena};
-    return hipLaunchKernel(entry.host_function, dim3(launch.grid[0], launch.grid[1], launch.grid[2]),
-                           dim3(launch.block[0], launch.block[1], launch.block[2]), arguments,
-                           launch.dynamic_shared_byte_count, stream);
-}
+/* what launches[0] of `count` is queued as, alone or with launches[1] where a kernel does both works (joined_launches.h) */
+struct queued_launch {
+    const void *host_function;
+    const char *function;
+    uint32_t launches; /* of the list: 1 or 2 */
+    dim3 grid, block;
+    uint32_t shared;
+    uint32_t numbers[3]; /* of two: the joined kernel's, joined_launch */
+};
 
-hipError_t launch_one(device_card *card, const kernel_launch &launch)
+queued_launch queued_as(const device_card *card, const kernel_launch *launches, uint32_t count)
 {
-    return launch_on(card, launch, card->stream);
-}
-
-/* Launch `index` of a list, together with the one behind it where a kernel does both works (joined_launches.h); index is
- * left at the last launch queued */
-hipError_t launch_next(device_card *card, const kernel_launch *launches, uint32_t count, uint32_t &index)
-{
-    const kernel_launch &first = launches[index];
-    if (index + 1u < count) {
-        const kernel_launch &second = launches[index + 1u];
-        const prepared_kernel &kernel = card->prepared[first.kernel];
-        const uint32_t joins = kernel.joins[0] & card->prepared[second.kernel].joins[1];
+    const kernel_launch &first = launches[0];
+    const prepared_kernel &kernel = card->prepared[first.kernel];
+    const kernel_entry &entry = kernel_table()[kernel.index];
+    if (count > 1u) {
+        const prepared_kernel &behind = card->prepared[launches[1].kernel];
+        const uint32_t joins = kernel.joins[0] & behind.joins[1];
         joined_launch joined;
-        if (joins != 0 && joined_launch_of(kernel_table()[kernel.index].function, kernel_table()[card->prepared[second.kernel].index].function, first, second,
-                                           card->arena_bytes, joined)) {
-            index++;
-            void *arguments[6] = {(void *)first.argument, (void *)second.argument, (void *)&card->arena, &joined.numbers[0], &joined.numbers[1], &joined.numbers[2]};
-            return hipLaunchKernel(joined_table()[(uint32_t)__builtin_ctz(joins)].host_function, dim3(joined.grid[0], joined.grid[1], 1), dim3(joined.block, 1, 1),
-                                   arguments, 0, card->stream);
+        if (joins != 0 && joined_launch_of(entry.function, kernel_table()[behind.index].function, first, launches[1], card->arena_bytes, joined)) {
+            const joined_entry &both = joined_table()[(uint32_t)__builtin_ctz(joins)];
+            return {both.host_function, both.joined, 2u, dim3(joined.grid[0], joined.grid[1], 1), dim3(joined.block, 1, 1), 0u,
+                    {joined.numbers[0], joined.numbers[1], joined.numbers[2]}};
         }
     }
-    return launch_one(card, first);
+    return {entry.host_function, entry.function, 1u, dim3(first.grid[0], first.grid[1], first.grid[2]), dim3(first.block[0], first.block[1], first.block[2]),
+            first.dynamic_shared_byte_count, {0, 0, 0}};
+}
+
+/* launches_done: 1, or 2 where launches[1] was queued with it */
+hipError_t launch_on(device_card *card, const kernel_launch *launches, uint32_t count, hipStream_t stream, uint32_t &launches_done)
+{
+    queued_launch queued = queued_as(card, launches, count);
+    launches_done = queued.launches;
+    /* a record travels by value: the runtime copies record_bytes from the launch's own bytes */
+    void *arguments_of_one[2] = {(void *)launches[0].argument, (void *)&card->arena};
+    void *arguments_of_two[6] = {(void *)launches[0].argument, queued.launches == 2u ? (void *)launches[1].argument : nullptr, (void *)&card->arena,
+                                 &queued.numbers[0], &queued.numbers[1], &queued.numbers[2]};
+    return hipLaunchKernel(queued.host_function, queued.grid, queued.block, queued.launches == 2u ? arguments_of_two : arguments_of_one, queued.shared, stream);
+}
+
+hipError_t launch_one(device_card *card, const kernel_launch &launch, hipStream_t stream)
+{
+    uint32_t done;
+    return launch_on(card, &launch, 1u, stream, done);
 }
 
 /* A checked list under capture on the card's stream: side runs go to side streams that wait for the fork's event, a
@@ -342,7 +354,7 @@ hipError_t capture_branches(device_card *card, const kernel_launch *launches, ui
                 open_runs++;
             }
             if (status == hipSuccess) {
-                status = launch_on(card, launch, card->side_streams[open_runs - 1u]);
+                status = launch_one(card, launch, card->side_streams[open_runs - 1u]);
             }
             last_is_side = true;
             break;
@@ -352,7 +364,9 @@ hipError_t capture_branches(device_card *card, const kernel_launch *launches, ui
         default: /* CHAIN, RESUME: the main line, which stands at the fork while side runs are open */
             if (status == hipSuccess) { /* joined with what is behind it on the main line alone */
                 const bool chained = index + 1u < count && launches[index + 1u].branch == LAUNCH_CHAIN;
-                status = launch_next(card, launches, chained ? index + 2u : index + 1u, index);
+                uint32_t done;
+                status = launch_on(card, launches + index, chained ? 2u : 1u, card->stream, done);
+                index += done - 1u;
             }
             last_is_side = false;
             break;
@@ -395,9 +409,33 @@ void anemone_register_kernel(const char *file, const char *function, const void 
     kernel_table().push_back(kernel_entry{file, function, host_function, record_bytes});
 }
 
-void anemone_register_joined_kernel(const char *first_file, const char *first, const char *second_file, const char *second, const void *host_function)
+void anemone_register_joined_kernel(const char *first_file, const char *first, const char *second_file, const char *second, const char *joined,
+                                    const void *host_function)
 {
-    joined_table().push_back(joined_entry{{first_file, second_file}, {first, second}, host_function});
+    if (joined_table().size() == MOST_JOINED_KERNELS) {
+        log_error(joined, "more joined kernels than the backend has bits for");
+        return;
+    }
+    joined_table().push_back(joined_entry{{first_file, second_file}, {first, second}, joined, host_function});
+}
+
+uint32_t backend_hip_joined_table_count(void)
+{
+    return (uint32_t)joined_table().size();
+}
+
+result_status backend_hip_joined_table_entry(uint32_t index, const char **files_out, const char **functions_out, const char **joined_out)
+{
+    if (index >= joined_table().size() || files_out == nullptr || functions_out == nullptr || joined_out == nullptr) {
+        return STATUS_INVALID_ARGUMENT;
+    }
+    const joined_entry &entry = joined_table()[index];
+    for (uint32_t launch = 0; launch < 2u; launch++) {
+        files_out[launch] = entry.files[launch];
+        functions_out[launch] = entry.functions[launch];
+    }
+    *joined_out = entry.joined;
+    return STATUS_OK;
 }
 
 uint32_t backend_hip_kernel_table_count(void)
@@ -713,11 +751,28 @@ result_status backend_hip_launch_run(struct device_card *card, const struct kern
     if (card_fail(card, "hipSetDevice", hipSetDevice(card->device))) {
         return STATUS_DEVICE_ERROR;
     }
-    for (uint32_t index = 0; index < launch_count; index++) {
-        if (card_fail(card, "hipLaunchKernel", launch_next(card, launches, launch_count, index))) {
+    for (uint32_t index = 0, done; index < launch_count; index += done) {
+        if (card_fail(card, "hipLaunchKernel", launch_on(card, launches + index, launch_count - index, card->stream, done))) {
             return STATUS_DEVICE_ERROR;
         }
     }
+    return STATUS_OK;
+}
+
+result_status backend_hip_launch_queued_as(struct device_card *card, const struct kernel_launch *launches, uint32_t launch_count,
+                                           const char **function_out, uint32_t *launches_out)
+{
+    if (card == nullptr || launches == nullptr || launch_count == 0 || function_out == nullptr || launches_out == nullptr) {
+        return STATUS_INVALID_ARGUMENT;
+    }
+    std::lock_guard<std::mutex> guard(card->mutex);
+    const result_status checked = launches_check(card, launches, launch_count);
+    if (checked != STATUS_OK) {
+        return checked;
+    }
+    const queued_launch queued = queued_as(card, launches, launch_count);
+    *function_out = queued.function;
+    *launches_out = queued.launches;
     return STATUS_OK;
 }
 
@@ -753,7 +808,7 @@ result_status backend_hip_launch_run_timed(struct device_card *card, const struc
     result_status status = STATUS_OK;
     for (uint32_t index = 0; index < launch_count && status == STATUS_OK; index++) {
         if (card_fail(card, "hipEventRecord", hipEventRecord(events[index], card->stream)) ||
-            card_fail(card, "hipLaunchKernel", launch_one(card, launches[index]))) {
+            card_fail(card, "hipLaunchKernel", launch_one(card, launches[index], card->stream))) {
             status = STATUS_DEVICE_ERROR;
         }
     }

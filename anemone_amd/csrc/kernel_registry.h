@@ -22,10 +22,10 @@ extern "C" void anemone_register_kernel(const char *file, const char *function, 
 /* a kernel that does the work of two launches that stand next to each other in a list (joined_launches.h): it takes both records,
  * the arena, and the numbers joined_launch_of leaves */
 extern "C" void anemone_register_joined_kernel(const char *first_file, const char *first, const char *second_file, const char *second,
-                                               const void *host_function);
+                                               const char *joined, const void *host_function);
 
 #define ANEMONE_JOINED_KERNEL(first_file, first, second_file, second, joined)                                  \
     static const int anemone_registered_##joined =                                                             \
-        (anemone_register_joined_kernel(first_file, #first, second_file, #second, (const void *)&joined), 0)
+        (anemone_register_joined_kernel(first_file, #first, second_file, #second, #joined, (const void *)&joined), 0)
 
 #endif

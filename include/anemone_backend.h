@@ -202,6 +202,14 @@ MUST_CHECK result_status backend_hip_measure_elapsed_us(struct device_card *card
 MUST_CHECK result_status backend_hip_launch_run_timed(struct device_card *card,
                                                       const struct kernel_launch *launches, uint32_t launch_count,
                                                       double *microseconds_out);
+/* Which kernel launch_run queues launches[0] of a list as, and how many launches of the list that is (2: joined with the one
+ * behind it, by the same rule). Nothing is queued. No counterpart in the reference: for tests and profiles. */
+MUST_CHECK result_status backend_hip_launch_queued_as(struct device_card *card, const struct kernel_launch *launches,
+                                                      uint32_t launch_count, const char **function_out, uint32_t *launches_out);
+/* The kernels that do the work of two launches: how many, and the i-th one's two launches (files_out[2], functions_out[2]) and its name. */
+uint32_t backend_hip_joined_table_count(void);
+MUST_CHECK result_status backend_hip_joined_table_entry(uint32_t index, const char **files_out, const char **functions_out,
+                                                        const char **joined_out);
 /* How many kernels the library was built with, and the i-th one's names and record size: what kernel_prepare checks
  * a request against (the reference reads the same from the module, source/backend_cuda_launch.c:160-186). */
 uint32_t backend_hip_kernel_table_count(void);

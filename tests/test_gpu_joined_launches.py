@@ -6,14 +6,17 @@ import pytest
 from _oracle import normals, to_bf16
 from anemone_amd import workloads
 from test_gpu_shared_join import amd, build, card, fresh_arena, say  # noqa: F401
-from test_joined_launches import rule
 
 pytestmark = pytest.mark.gpu
 
 
-def check(amd, card, launches, ranges, first, name):
-    """launches one by one, in one list and as a graph of three replays, from the same bytes"""
-    assert rule(name, launches[first], launches[first + 1], card.arena_bytes) is not None
+def check(amd, card, launches, ranges, first, joined):
+    """launches one by one, in one list, where launches[first] and the one behind it are queued as the kernel `joined`, and as a
+    graph of three replays, from the same bytes"""
+    assert card.queued_as(launches[first:]) == (joined, 2)
+    for index, launch in enumerate(launches):
+        assert index == first or card.queued_as(launches[index:])[1] == 1
+        assert card.queued_as([launch])[1] == 1
     results = []
 
     def run(work):
@@ -28,8 +31,8 @@ def check(amd, card, launches, ranges, first, name):
         run(lambda: card.run_graph(graph))
     assert any(np.any(got != 0xEE) for got in results[0])
     for other in results[1:]:
-        for index, (one, joined) in enumerate(zip(results[0], other)):
-            assert np.array_equal(one, joined), (name, index)
+        for index, (one, got) in enumerate(zip(results[0], other)):
+            assert np.array_equal(one, got), (joined, index)
 
 
 @pytest.mark.parametrize("rows,hidden,form", [(1, 128, "select"), (8, 1280, "select"), (3, 4096, "select"), (9, 256, "small"), (64, 1152, "small"),
@@ -52,7 +55,7 @@ def test_router_and_quantizer(amd, card, rows, hidden, form, wide_scales):  # no
         launches, name = [layer.projection_launch()[0]] + routed[:2 if form == "small" else 3], "router_wide_" + form
         first = len(launches) - 1
         extra = [(wide.ranges[key].byte_offset, wide.ranges[key].byte_count) for key in ("pairs", "runs", "tiles", "jobs")]
-    check(amd, card, launches + [quantize], [(r.byte_offset, r.byte_count) for r in outputs] + extra, first, name)
+    check(amd, card, launches + [quantize], [(r.byte_offset, r.byte_count) for r in outputs] + extra, first, name + ("_quantize_128" if wide_scales else "_quantize"))
 
 
 @pytest.mark.parametrize("rows,inner", [(1, 128), (5, 640), (9, 1152), (70, 2176)])
@@ -63,7 +66,54 @@ def test_hidden_and_quantizer(amd, card, rows, inner):  # noqa: F811
     layer.set_rows(to_bf16(normals(rows, rows * 256)).reshape(rows, 256))
     card.run(layer.quantize_launch())
     names = [name for name in shared.ranges if name not in ("streams", "post", "comb", "pair_output")]
-    check(amd, card, list(shared.launches()), [(shared.ranges[n].byte_offset, shared.ranges[n].byte_count) for n in names], 1, "trunk_hidden_entry")
+    check(amd, card, list(shared.launches()), [(shared.ranges[n].byte_offset, shared.ranges[n].byte_count) for n in names], 1, "trunk_hidden_quantize")
+
+
+SPECIALS = np.array([0x7F80, 0xFF80, 0x7FC0, 0xFFC1, 0x7F7F, 0xFF7F, 0x0000, 0x8000, 0x0001, 0x8001, 0x7F81, 0x0080], dtype=np.uint16)
+
+
+def with_specials(values, every):
+    """bfloat16 words, some of them infinities, NaNs, the largest, zeros and denormals, in vectors of their own and side by side"""
+    out = values.copy().reshape(-1)
+    out[::every] = np.resize(SPECIALS, out[::every].size)
+    out[1:40] = np.resize(SPECIALS, 39)
+    return out.reshape(values.shape)
+
+
+@pytest.mark.parametrize("wide_scales", [False, True])
+@pytest.mark.parametrize("every", [7, 1000])
+def test_router_and_quantizer_of_specials(amd, card, wide_scales, every):  # noqa: F811
+    say("joined launches: specials of the rows", wide_scales, every)
+    rows, hidden = 8, 1152
+    layer, _, _ = build(amd, card, hidden, 128, rows, 6, 3)
+    layer.set_rows(with_specials(to_bf16(normals(4, rows * hidden)).reshape(rows, hidden), every))
+    quantize = layer.quantize_launch()[0]
+    quantize.kernel = layer.kernels.activation_quantize_128 if wide_scales else quantize.kernel
+    names = ("codes", "exponents", "operands")
+    check(amd, card, [layer.projection_launch()[0], layer.select_launch(0)[0], quantize],
+          [(layer.ranges[n].byte_offset, layer.ranges[n].byte_count) for n in names], 1, "router_select_entry_quantize" + ("_128" if wide_scales else ""))
+
+
+@pytest.mark.parametrize("every", [7, 1000])
+def test_hidden_and_quantizer_of_specials(amd, card, every):  # noqa: F811
+    say("joined launches: specials of gate and up", every)
+    rows, inner = 5, 1152
+    layer, shared, _ = build(amd, card, 256, 256, rows, 1, rows, shared_inner=inner)
+    for seed, name in enumerate(("gate_output", "up_output")):
+        card.upload(shared.ranges[name].byte_offset, with_specials(to_bf16(normals(seed, rows * inner)), every + 4 * seed))
+    names = [name for name in shared.ranges if name.startswith("hidden")]
+    check(amd, card, list(shared.launches())[1:3], [(shared.ranges[n].byte_offset, shared.ranges[n].byte_count) for n in names], 0, "trunk_hidden_quantize")
+
+
+@pytest.mark.parametrize("weights", ["e2m1", "e4m3_gfx950"])
+@pytest.mark.parametrize("every", [7, 1000])
+def test_gate_up_and_quantizer_of_specials(amd, card, weights, every):  # noqa: F811
+    say("joined launches: specials of gate and up's rows", weights, every)
+    layer, kernel = gate_up_layer(amd, card, 8, 5, 384, 2, weights)
+    layer.set_rows(with_specials(to_bf16(normals(6, 8 * 1024)).reshape(8, 1024), every))
+    card.run(layer.quantize_launch())
+    names = ("hidden", "hidden_codes", "hidden_exponents", "hidden_operands")
+    check(amd, card, list(layer.expert_launches())[:2], [(layer.ranges[n].byte_offset, layer.ranges[n].byte_count) for n in names], 0, kernel + "_joined")
 
 
 def gate_up_layer(amd, card, rows, live, inner, slices, weights):  # noqa: F811
@@ -90,7 +140,7 @@ def test_gate_up_and_quantizer(amd, card, rows, live, inner, slices, weights):  
     say("joined launches: gate and up", rows, live, inner, slices, weights)
     layer, kernel = gate_up_layer(amd, card, rows, live, inner, slices, weights)
     names = ("hidden", "hidden_codes", "hidden_exponents", "hidden_operands", "pair_output", "row_output")
-    check(amd, card, list(layer.expert_launches()), [(layer.ranges[n].byte_offset, layer.ranges[n].byte_count) for n in names], 0, kernel)
+    check(amd, card, list(layer.expert_launches()), [(layer.ranges[n].byte_offset, layer.ranges[n].byte_count) for n in names], 0, kernel + "_joined")
 
 
 @pytest.mark.parametrize("pairs", [1, 21, 63])
@@ -104,5 +154,5 @@ def test_pairs_of_the_table_past_the_quantizer(amd, card, pairs, weights):  # no
     launches[0].argument[48:52] = list(pairs.to_bytes(4, "little"))  # expert_gate_up_arguments.pair_count
     launches[1].grid[1] = pairs
     names = ("hidden", "hidden_codes", "hidden_exponents", "hidden_operands")
-    check(amd, card, launches, [(layer.ranges[n].byte_offset, layer.ranges[n].byte_count) for n in names], 0, kernel)
+    check(amd, card, launches, [(layer.ranges[n].byte_offset, layer.ranges[n].byte_count) for n in names], 0, kernel + "_joined")
     assert np.all(layer.card.download(layer.ranges["hidden_codes"].byte_offset, 64 * 384)[pairs * 384:] == 0xEE)

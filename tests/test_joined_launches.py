@@ -159,3 +159,25 @@ def test_widths_the_quantizer_has_no_order_for(width):
     assert rule("trunk_hidden_entry", hidden(width=width), quantizer(width=width)) is None
     for name, strip in (("expert_gate_up_4", 64), ("expert_gate_up_e4m3_4", 32)):
         assert rule(name, whole_gate_up(width=width, strip=strip), quantizer(width=width)) is None
+
+
+def test_every_joined_kernel_is_registered():
+    """Under the names of two kernels of the library: a pair that is missing, or misnamed, would run as two launches without a word."""
+    lib, kernels, joined = amd.library(), set(), []
+    f, g, b = C.c_char_p(), C.c_char_p(), C.c_uint32()
+    for i in range(lib.backend_hip_kernel_table_count()):
+        assert lib.backend_hip_kernel_table_entry(i, C.byref(f), C.byref(g), C.byref(b)) == 0
+        kernels.add((f.value.decode(), g.value.decode()))
+    files, functions = (C.c_char_p * 2)(), (C.c_char_p * 2)()
+    for i in range(lib.backend_hip_joined_table_count()):
+        assert lib.backend_hip_joined_table_entry(i, files, functions, C.byref(g)) == 0
+        launches = [(files[k].decode(), functions[k].decode()) for k in range(2)]
+        assert all(launch in kernels for launch in launches), launches
+        joined.append((launches[0][1], launches[1][1], g.value.decode()))
+    assert lib.backend_hip_joined_table_entry(len(joined), files, functions, C.byref(g)) != 0
+    want = [(name, "activation_quantize%s_entry" % scales, "%s_quantize%s" % (name, scales))
+            for name in ("router_select_entry", "router_wide_small", "router_wide_place") for scales in ("", "_128")]
+    want += [("trunk_hidden_entry", "activation_quantize_entry", "trunk_hidden_quantize")]
+    want += [(name, "activation_quantize_entry", name + "_joined")
+             for infix in ("", "e4m3_", "gfx950_", "e4m3_gfx950_") for slices in (1, 2, 4, 8) for name in ["expert_gate_up_%s%d" % (infix, slices)]]
+    assert sorted(joined) == sorted(want)
