@@ -25,7 +25,7 @@ HIP_SOURCES = ["kernel_exl3.hip", "kernel_exl3_tc.hip", "kernel_exl3_tcp.hip", "
                "kernel_expert_linear.hip", "kernel_trunk_linear.hip", "kernel_hyper_connection.hip", "kernel_site_front.hip"]
 PROBE_SOURCES = ["kernel_calibrate.hip", "kernel_selfcheck.hip"]
 
-BACKEND_SOURCES = ["backend_hip.cpp", "joined_launches.cpp"]  # host C++ over the HIP runtime API: no device code
+BACKEND_SOURCES = ["backend_hip.cpp", "joined_launches.cpp", "trunk_deep.cpp"]  # host C++ over the HIP runtime API: no device code
 BACKEND_FLAGS = ["-std=c++17", "-O2", "-fPIC", "-Wall", "-Wextra", "-D__HIP_PLATFORM_AMD__", "-I", "/opt/rocm/include"]
 HOST_FLAGS = ["-std=c11", "-D_GNU_SOURCE", "-O2", "-fPIC", "-ffp-contract=off", "-Wall", "-Wextra", "-Werror=implicit-function-declaration"]
 # packed-fp32 instructions are switched off for every HIP translation unit; the host pass warns that it does not

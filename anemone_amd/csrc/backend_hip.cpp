@@ -22,6 +22,7 @@
 #include "anemone_backend.h"
 #include "joined_launches.h"
 #include "kernel_registry.h"
+#include "trunk_deep.h"
 
 namespace {
 
@@ -68,7 +69,35 @@ uint32_t joins_of(const kernel_entry &entry, uint32_t launch)
 struct prepared_kernel {
     uint32_t index;    /* into kernel_table() */
     uint32_t joins[2]; /* joins_of its entry */
+    uint32_t deep[TRUNK_DEEP_INSTANCES]; /* into kernel_table(): what takes its launches of few blocks (trunk_deep.h); NO_ENTRY: nothing */
 };
+
+#define NO_ENTRY UINT32_MAX
+
+/* a kernel of the table by its names, or NO_ENTRY */
+uint32_t entry_of(const char *file, const char *function)
+{
+    const std::vector<kernel_entry> &table = kernel_table();
+    for (uint32_t index = 0; index < table.size(); index++) {
+        if (std::strcmp(table[index].file, file) == 0 && std::strcmp(table[index].function, function) == 0) {
+            return index;
+        }
+    }
+    return NO_ENTRY;
+}
+
+prepared_kernel prepared_of(uint32_t index)
+{
+    const kernel_entry &entry = kernel_table()[index];
+    prepared_kernel kernel = {index, {joins_of(entry, 0), joins_of(entry, 1)}, {}};
+    const bool interleaved = std::strcmp(entry.file, KERNEL_FILE_TRUNK_LINEAR) == 0 && std::strcmp(entry.function, KERNEL_TRUNK_LINEAR_QUANTIZED_INTERLEAVED) == 0;
+    for (uint32_t instance = 0; instance < TRUNK_DEEP_INSTANCES; instance++) {
+        char name[48];
+        (void)std::snprintf(name, sizeof name, "%s%u", KERNEL_TRUNK_LINEAR_QUANTIZED_DEEP_STEM, TRUNK_DEEP_ROWS(instance));
+        kernel.deep[instance] = interleaved ? entry_of(KERNEL_FILE_TRUNK_LINEAR, name) : NO_ENTRY;
+    }
+    return kernel;
+}
 
 struct copy_slot {
     hipEvent_t event;
@@ -276,7 +305,8 @@ result_status launches_check(device_card *card, const kernel_launch *launches, u
     return STATUS_OK;
 }
 
-/* what launches[0] of `count` is queued as, alone or with launches[1] where a kernel does both works (joined_launches.h) */
+/* what launches[0] of `count` is queued as: with launches[1] where a kernel does both works (joined_launches.h); a product of few blocks in
+ * smaller ones (trunk_deep.h); else as it stands */
 struct queued_launch {
     const void *host_function;
     const char *function;
@@ -300,6 +330,12 @@ queued_launch queued_as(const device_card *card, const kernel_launch *launches, 
             return {both.host_function, both.joined, 2u, dim3(joined.grid[0], joined.grid[1], 1), dim3(joined.block, 1, 1), 0u,
                     {joined.numbers[0], joined.numbers[1], joined.numbers[2]}};
         }
+    }
+    trunk_deep_launch deep;
+    const uint32_t instance = kernel.deep[0] != NO_ENTRY ? trunk_deep_instance(first, (uint32_t)card->max_shared, deep) : TRUNK_DEEP_INSTANCES;
+    if (instance < TRUNK_DEEP_INSTANCES && kernel.deep[instance] != NO_ENTRY) {
+        const kernel_entry &smaller = kernel_table()[kernel.deep[instance]];
+        return {smaller.host_function, smaller.function, 1u, dim3(deep.grid[0], deep.grid[1], 1), dim3(first.block[0], 1, 1), deep.shared_bytes, {0, 0, 0}};
     }
     return {entry.host_function, entry.function, 1u, dim3(first.grid[0], first.grid[1], first.grid[2]), dim3(first.block[0], first.block[1], first.block[2]),
             first.dynamic_shared_byte_count, {0, 0, 0}};
@@ -714,15 +750,21 @@ result_status backend_hip_kernel_prepare(struct device_card *card, const char *k
         }
         /* as the reference's backend does behind its parameter check (source/backend_cuda_launch.c:160-186): raise
          * the kernel's limit of dynamic shared memory to what the card holds; a refusal shows at the launch that asks */
+        const prepared_kernel kernel = prepared_of(index);
         if (hipSetDevice(card->device) == hipSuccess) {
             (void)hipFuncSetAttribute(table[index].host_function, hipFuncAttributeMaxDynamicSharedMemorySize, card->max_shared);
-            for (uint32_t joins = joins_of(table[index], 1); joins != 0; joins &= joins - 1u) { /* loaded here too, not by the first pass */
+            for (const uint32_t smaller : kernel.deep) {
+                if (smaller != NO_ENTRY) {
+                    (void)hipFuncSetAttribute(table[smaller].host_function, hipFuncAttributeMaxDynamicSharedMemorySize, card->max_shared);
+                }
+            }
+            for (uint32_t joins = kernel.joins[1]; joins != 0; joins &= joins - 1u) { /* loaded here too, not by the first pass */
                 hipFuncAttributes attributes;
                 (void)hipFuncGetAttributes(&attributes, joined_table()[(uint32_t)__builtin_ctz(joins)].host_function);
             }
             (void)hipGetLastError();
         }
-        card->prepared.push_back({index, {joins_of(table[index], 0), joins_of(table[index], 1)}});
+        card->prepared.push_back(kernel);
         *kernel_out = (uint32_t)card->prepared.size() - 1u;
         return STATUS_OK;
     }

@@ -16,6 +16,8 @@
  *     TRUNK_INTERLEAVED_ROWS rows (four MFMA column blocks) by TRUNK_INTERLEAVED_BLOCK_OUTPUTS outputs of one matrix;
  *     grid (blocks of both matrices, tiles of rows). An output's chain is the same MFMAs on the same operands in the
  *     same order as the thin instance's of one slice: the same bits.
+ *   - trunk_linear_quantized_deep_<rows>: the same for launches of few blocks (trunk_deep.h, which the backend asks): tiles of
+ *     16, 32 or 64 rows by TRUNK_DEEP_BLOCK_OUTPUTS outputs, more K steps on their way. The same bits.
  *   - trunk_hidden_entry: bfloat16((g / (1 + exp(-g))) u) of g = min(gate, L), u = clamp(up, +-L), a route weight of 1.
  *   - expert_shared_join_<S>: trunk_linear_quantized_<S> of the shared expert's down and behind it the join
  *     (join_device.cuh) of the strip's outputs, read from where the block keeps them.

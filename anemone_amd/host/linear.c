@@ -131,14 +131,6 @@ result_status linear_kernels_prepare(const struct backend_operations *backend, s
         status = backend->kernel_prepare(card, KERNEL_FILE_TRUNK_LINEAR, KERNEL_TRUNK_LINEAR_QUANTIZED_INTERLEAVED,
                                          sizeof(struct trunk_linear_quantized_arguments), &kernels.trunk_linear_quantized_interleaved);
     }
-    for (uint32_t instance = 0; status == STATUS_OK && instance < TRUNK_DEEP_INSTANCES; instance++) {
-        char name[48];
-        (void)snprintf(name, sizeof name, "%s%u", KERNEL_TRUNK_LINEAR_QUANTIZED_DEEP_STEM, TRUNK_DEEP_ROWS(instance));
-        if (backend->kernel_prepare(card, KERNEL_FILE_TRUNK_LINEAR, name, sizeof(struct trunk_linear_quantized_arguments),
-                                    &kernels.trunk_linear_quantized_deep[instance]) != STATUS_OK) {
-            kernels.trunk_linear_quantized_deep[instance] = BACKEND_NO_KERNEL; /* trunk_linear_quantized_interleaved_1 then takes its launches */
-        }
-    }
     if (status == STATUS_OK) {
         status = backend->kernel_prepare(card, KERNEL_FILE_TRUNK_LINEAR, KERNEL_TRUNK_HIDDEN, sizeof(struct trunk_hidden_arguments),
                                          &kernels.trunk_hidden);
@@ -359,10 +351,9 @@ result_status linear_routed_experts_prepare(const struct linear_routed_experts_d
  *   1..8      trunk_linear_quantized_<S>              (strips of both matrices, 1, 1)                  64 S    static
  *   9..       trunk_linear_quantized_wide_<S>         (strips x n, 1, 1), n = groups of 8 rows or 1    64 S    static
  *   9..       trunk_linear_quantized_interleaved_1    (blocks of both matrices, ceil(rows / 64), 1)    256     TRUNK_INTERLEAVED_WINDOW_BYTES
- *             trunk_linear_quantized_deep_<R>         (blocks of both matrices, ceil(rows / R), 1)     256     TRUNK_DEEP_WINDOW_BYTES
  *   hidden    trunk_hidden_entry                      (ceil(width / 2048), rows, 1)                    256     0
- * strip = TRUNK_STRIP_OUTPUTS outputs of one matrix, block = TRUNK_INTERLEAVED_BLOCK_OUTPUTS, or TRUNK_DEEP_BLOCK_OUTPUTS of a launch of few
- * blocks (trunk_deep_instance).
+ * strip = TRUNK_STRIP_OUTPUTS outputs of one matrix, block = TRUNK_INTERLEAVED_BLOCK_OUTPUTS. The backend queues an interleaved launch of few
+ * blocks as one of smaller ones (trunk_deep.h).
  */
 static bool trunk_matrix_is_valid(const char *what, const struct linear_matrix *matrix, uint64_t *bytes_out, uint32_t *instance_out)
 {
@@ -385,31 +376,6 @@ static bool trunk_matrix_is_valid(const char *what, const struct linear_matrix *
     return true;
 }
 
-/* Which of trunk_linear_quantized_deep's instances takes a launch of the interleaved form, or TRUNK_DEEP_INSTANCES: the one of the fewest rows
- * a block that gives every block a place on the card at once. A block of the other form has 128 outputs by 64 rows, two K steps in
- * LDS and as long a K step as memory takes to answer (0.9 us), so that a launch of a few dozen blocks is a chain of such steps on as
- * many CUs; fewer rows and outputs a block are more blocks, each of a shorter step (a wavefront alone on a SIMD reads its
- * operands out of LDS one instruction at a time), with three or four steps on their way. Gate and up, and down, us by events, that form | these:
- * 85 rows of 4096 x 896 33.2 | 19.7 and 12.3 | 8.9; 70 of 5120 x 2048 39.2 | 23.0 and 19.2 | 12.7; 158 of 3072 x 1664 26.8 | 18.8 and 17.3 |
- * 12.0; 500 of 4096 x 1024 33.0 | 23.2; 700 of 2048 x 768 (64 rows a block) 20.0 | 17.6. With more blocks than places those behind
- * wait for a whole chain: the other form, three blocks a CU, is then the shorter (1100 of 2048 x 768, down 12.6). */
-static uint32_t trunk_deep_instance(const struct linear_kernels_record *kernels, uint32_t blocks, uint32_t inputs, uint32_t rows)
-{
-    uint32_t handles[sizeof *kernels / sizeof(uint32_t)];
-    memcpy(handles, kernels, sizeof handles);
-    for (uint32_t instance = 0; instance < TRUNK_DEEP_INSTANCES && inputs <= TRUNK_DEEP_MOST_INPUTS; instance++) {
-        const uint32_t of = TRUNK_DEEP_ROWS(instance), handle = kernels->trunk_linear_quantized_deep[instance];
-        if ((uint64_t)blocks * ((rows + of - 1u) / of) <= TRUNK_DEEP_MOST_BLOCKS) {
-            uint32_t named = 0; /* members that a caller left zero hold the same handle, that of whatever kernel was prepared first */
-            for (uint32_t i = 0; i < sizeof handles / sizeof handles[0]; i++) {
-                named += handles[i] == handle ? 1u : 0u;
-            }
-            return handle != BACKEND_NO_KERNEL && named == 1u ? instance : TRUNK_DEEP_INSTANCES;
-        }
-    }
-    return TRUNK_DEEP_INSTANCES;
-}
-
 /* the launch of a trunk product whose description is checked: thin up to LINEAR_MAXIMUM_ROWS rows, else the
  * first matrix's wide form; false where that form's kernel is not prepared or takes no such matrix */
 static bool trunk_launch_fill(const char *what, struct kernel_launch *launch, const struct linear_kernels_record *kernels,
@@ -419,14 +385,13 @@ static bool trunk_launch_fill(const char *what, struct kernel_launch *launch, co
 {
     struct trunk_linear_quantized_arguments record;
     memset(&record, 0, sizeof record);
-    uint32_t strips = 0, blocks = 0, deep_blocks = 0;
+    uint32_t strips = 0, blocks = 0;
     for (uint32_t m = 0; m < matrix_count; m++) {
         record.weights_offset[m] = matrices[m].stored.byte_offset;
         record.output_offset[m] = outputs[m].byte_offset;
         record.output_size[m] = matrices[m].shape.output_size;
         strips += (matrices[m].shape.output_size + TRUNK_STRIP_OUTPUTS - 1u) / TRUNK_STRIP_OUTPUTS;
         blocks += (matrices[m].shape.output_size + TRUNK_INTERLEAVED_BLOCK_OUTPUTS - 1u) / TRUNK_INTERLEAVED_BLOCK_OUTPUTS;
-        deep_blocks += (matrices[m].shape.output_size + TRUNK_DEEP_BLOCK_OUTPUTS - 1u) / TRUNK_DEEP_BLOCK_OUTPUTS;
     }
     record.codes_offset = codes->byte_offset;
     record.exponents_offset = exponents->byte_offset;
@@ -448,17 +413,9 @@ static bool trunk_launch_fill(const char *what, struct kernel_launch *launch, co
             REFUSE("%s: the interleaved form takes a matrix of one slice, not %u", what, matrices[0].slice_count);
             return false;
         }
-        const uint32_t deep = trunk_deep_instance(kernels, deep_blocks, record.input_size, row_count);
-        if (deep < TRUNK_DEEP_INSTANCES) {
-            const uint32_t rows = TRUNK_DEEP_ROWS(deep);
-            kernel = kernels->trunk_linear_quantized_deep[deep];
-            launch_fill(launch, kernel, deep_blocks, (row_count + rows - 1u) / rows, 1, WIDE_BLOCK_THREADS, TRUNK_DEEP_WINDOW_BYTES(record.input_size, rows),
-                        &record, sizeof record);
-        } else {
-            kernel = kernels->trunk_linear_quantized_interleaved;
-            launch_fill(launch, kernel, blocks, (row_count + TRUNK_INTERLEAVED_ROWS - 1u) / TRUNK_INTERLEAVED_ROWS, 1, WIDE_BLOCK_THREADS,
-                        TRUNK_INTERLEAVED_WINDOW_BYTES, &record, sizeof record);
-        }
+        kernel = kernels->trunk_linear_quantized_interleaved;
+        launch_fill(launch, kernel, blocks, (row_count + TRUNK_INTERLEAVED_ROWS - 1u) / TRUNK_INTERLEAVED_ROWS, 1, WIDE_BLOCK_THREADS,
+                    TRUNK_INTERLEAVED_WINDOW_BYTES, &record, sizeof record);
     }
     if (kernel == BACKEND_NO_KERNEL) {
         REFUSE("%s: the kernel of its rows and form is not prepared", what);

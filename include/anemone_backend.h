@@ -202,8 +202,8 @@ MUST_CHECK result_status backend_hip_measure_elapsed_us(struct device_card *card
 MUST_CHECK result_status backend_hip_launch_run_timed(struct device_card *card,
                                                       const struct kernel_launch *launches, uint32_t launch_count,
                                                       double *microseconds_out);
-/* Which kernel launch_run queues launches[0] of a list as, and how many launches of the list that is (2: joined with the one
- * behind it, by the same rule). Nothing is queued. No counterpart in the reference: for tests and profiles. */
+/* Which kernel launch_run queues launches[0] of a list as (its own, or one that does the same work in smaller blocks), and how many
+ * launches of the list that is (2: joined with the one behind it). By the rules launch_run goes by. Nothing is queued. No counterpart in the reference: for tests and profiles. */
 MUST_CHECK result_status backend_hip_launch_queued_as(struct device_card *card, const struct kernel_launch *launches,
                                                       uint32_t launch_count, const char **function_out, uint32_t *launches_out);
 /* The kernels that do the work of two launches: how many, and the i-th one's two launches (files_out[2], functions_out[2]) and its name. */

@@ -386,8 +386,6 @@ struct linear_kernels_record { /* include/anemone/linear.h:121-132 of the refere
     uint32_t expert_down_e4m3_gfx950[LINEAR_SLICE_INSTANCES];
     uint32_t expert_gate_up_b128_gfx950[LINEAR_SLICE_INSTANCES]; /* WEIGHT_FORMAT_E4M3_BLOCK128_GFX950 */
     uint32_t expert_down_b128_gfx950[LINEAR_SLICE_INSTANCES];
-    /* extension: the interleaved instance in launches of few blocks, by TRUNK_DEEP_ROWS; BACKEND_NO_KERNEL: such launches take the other */
-    uint32_t trunk_linear_quantized_deep[TRUNK_DEEP_INSTANCES];
 };
 MUST_CHECK result_status linear_kernels_prepare(const struct backend_operations *backend, struct device_card *card,
                                                 uint32_t arithmetic_class, struct linear_kernels_record *kernels_out);

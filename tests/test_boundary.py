@@ -751,28 +751,28 @@ def shared_description(rows=8, gate_up_slices=4, down_slices=2, form=amd.LINEAR_
     return d, cursor[0]
 
 
-@pytest.mark.parametrize("rows,taken,groups,windows", [
-    (9, "deep_16", 1, [54528, 53504]), (128, "deep_16", 8, [54528, 53504]), (129, "deep_32", 5, [66816, 64768]), (256, "deep_32", 8, [66816, 64768]),
-    (257, "deep_64", 5, [74752, 70656]), (512, "deep_64", 8, [74752, 70656]), (513, "interleaved_1", 9, [51712, 51712])])
-def test_shared_expert_launches_of_few_blocks(fake, rows, taken, groups, windows):
-    """64 blocks of 64 outputs a product: the instance of the fewest rows that leaves at most 512 blocks, else the other form."""
+@pytest.mark.parametrize("rows", [9, 64, 85, 512, 8192])
+def test_shared_expert_launches_are_the_record_s(fake, rows):
+    """The interleaved form's launches name the kernel that the record of handles names, whatever the backend queues them as."""
     lib = amd.library()
     kernels = amd.LinearKernels()
     assert lib.linear_kernels_prepare(fake.address, fake.card, 950, C.byref(kernels)) == 0
     d, arena = shared_description(rows=rows, gate_up_slices=1, down_slices=1, form=amd.LINEAR_INTERLEAVED_CHUNK_BLOCKS)
     launches = amd.launches_of(4)
+    assert lib.linear_shared_expert_prepare(C.byref(d), arena, C.byref(kernels), launches) == 0
+    products = [launches[0], launches[3]]
+    assert [fake.handles[l.kernel][1] for l in products] == ["trunk_linear_quantized_interleaved_1"] * 2
+    assert [list(l.grid) for l in products] == [[32, (rows + 63) // 64, 1]] * 2 and [l.dynamic_shared_byte_count for l in products] == [51712] * 2
 
-    def prepared():
-        assert lib.linear_shared_expert_prepare(C.byref(d), arena, C.byref(kernels), launches) == 0
-        products = [launches[0], launches[3]]
-        return [fake.handles[l.kernel][1] for l in products], [list(l.grid) for l in products], [l.dynamic_shared_byte_count for l in products]
-    blocks = 32 if taken == "interleaved_1" else 64
-    assert prepared() == (["trunk_linear_quantized_" + taken] * 2, [[blocks, groups, 1]] * 2, windows)
-    for i in range(3):  # a backend without them, and a caller who left the members as zero
-        for handle in (amd.BACKEND_NO_KERNEL, 0):
-            kernels.trunk_linear_quantized_deep[i] = handle
-            if taken == "deep_%d" % (16 << i):
-                assert prepared() == (["trunk_linear_quantized_interleaved_1"] * 2, [[32, (rows + 63) // 64, 1]] * 2, [51712] * 2)
+
+def test_prepared_kernels_stay_inside_the_record(fake):
+    """The record of handles is as long as callers were built with: 85 words. Nothing is written behind it."""
+    words, guard = 85, 64
+    assert C.sizeof(amd.LinearKernels) == 4 * words
+    buffer = (C.c_uint32 * (words + guard))(*([0x5A5A5A5A] * (words + guard)))
+    record = C.cast(buffer, C.POINTER(amd.LinearKernels))
+    assert amd.library().linear_kernels_prepare(fake.address, fake.card, 950, record) == 0
+    assert 0x5A5A5A5A not in buffer[:words] and buffer[words:] == [0x5A5A5A5A] * guard
 
 
 def join_description(rows=8, picks=8, width=4096, first=1 << 30, row_sums=True, **changes):

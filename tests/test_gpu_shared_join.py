@@ -165,8 +165,7 @@ def test_instances_for_launches_of_few_blocks_have_the_wide_bits(amd, card, hidd
         launch = trunk_launch(amd, card, layer, shared, (0, 1), 1, rows, form, outputs)
         card.run(launch)
         got.append([shared.read(name, np.uint16).copy() for name in ("gate_output", "up_output")])
-    kernels = layer.kernels
-    assert launch[0].kernel == (kernels.trunk_linear_quantized_deep[of // 32] if of else kernels.trunk_linear_quantized_interleaved)
+    assert card.queued_as(launch) == ("trunk_linear_quantized_" + ("deep_%d" % of if of else "interleaved_1"), 1)
     for tiled, deep in zip(*got):
         assert np.array_equal(tiled, deep)
 
