@@ -133,8 +133,10 @@ __device__ static __forceinline__ void trunk_linear_quantized_wide(const struct 
 template <uint32_t ROWS>
 using trunk_deep_chain = wide_chain<1, true, 1u, false, TRUNK_DEEP_STAGES(ROWS), ROWS>;
 static_assert(trunk_deep_chain<16u>::WINDOW_BYTES + 8u * trunk_deep_chain<16u>::CHUNK_BYTES == TRUNK_DEEP_WINDOW_BYTES(4096u, 16u) &&
+                  trunk_deep_chain<32u>::WINDOW_BYTES + 8u * trunk_deep_chain<32u>::CHUNK_BYTES == TRUNK_DEEP_WINDOW_BYTES(4096u, 32u) &&
                   trunk_deep_chain<64u>::WINDOW_BYTES + 8u * trunk_deep_chain<64u>::CHUNK_BYTES == TRUNK_DEEP_WINDOW_BYTES(4096u, 64u) &&
-                  WIDE_WAVES * trunk_deep_chain<16u>::STRIP * 16u == TRUNK_DEEP_BLOCK_OUTPUTS && TRUNK_DEEP_WINDOW_BYTES(TRUNK_DEEP_MOST_INPUTS, 64u) <= 160u * 1024u,
+                  WIDE_WAVES * trunk_deep_chain<16u>::STRIP * 16u == TRUNK_DEEP_BLOCK_OUTPUTS && TRUNK_DEEP_WINDOW_BYTES(TRUNK_DEEP_MOST_INPUTS, 64u) <= 160u * 1024u &&
+                  TRUNK_DEEP_WINDOW_BYTES(TRUNK_DEEP_MOST_INPUTS, 32u) <= 80u * 1024u,
               "the windows and the blocks the host asks for are the kernel's");
 
 /* grid (ceil(output_size[0] / n) + ceil(output_size[1] / n), ceil(row_count / rows)), block 256; n and rows: TRUNK_INTERLEAVED_BLOCK_OUTPUTS and

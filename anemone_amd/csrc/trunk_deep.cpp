@@ -19,7 +19,9 @@ uint64_t blocks_of(uint64_t size, uint64_t block)
  * 85 rows of 4096 x 896 32.6 | 19.0 and 11.8 | 8.4; 70 of 5120 x 2048 39.6 | 23.8 and 19.6 | 13.0; 158 of 3072 x 1664 26.1 | 18.1 and 16.7 |
  * 11.4; 500 of 4096 x 1024 32.6 | 23.3 and 13.1 | 12.9; 700 of 2048 x 768 19.1 | 17.2 and 11.2 | 10.8; 1100 of 2048 x 768 19.4 | 18.2. With
  * more blocks than places those behind wait for a whole chain: the other form, three blocks a CU, is then the shorter (1100 rows of 768 x
- * 2048 12.4 | 16.1 with 576 blocks). */
+ * 2048 12.4 | 16.1 with 576 blocks). So it is where a CU holds one block alone: 64 rows a block, 7680 inputs, 512 blocks 55.8 | 49.4; 8192
+ * inputs, 320 blocks 60.0 | 93.7, 512 blocks 60.2 | 94.2; 16384 inputs, 320 blocks 113.7 | 180.3 (at 256 blocks 112.1 | 93.9, and 32 rows a
+ * block, two a CU, 73.7). */
 extern "C" uint32_t trunk_deep_instance(const struct kernel_launch &launch, uint32_t most_shared_bytes, struct trunk_deep_launch &out)
 {
     struct trunk_linear_quantized_arguments record;
@@ -36,7 +38,7 @@ extern "C" uint32_t trunk_deep_instance(const struct kernel_launch &launch, uint
     for (uint32_t instance = 0; instance < TRUNK_DEEP_INSTANCES; instance++) {
         const uint32_t rows = TRUNK_DEEP_ROWS(instance), window = TRUNK_DEEP_WINDOW_BYTES(record.input_size, rows);
         const uint64_t groups = blocks_of(record.row_count, rows);
-        if (blocks * groups <= TRUNK_DEEP_MOST_BLOCKS) {
+        if (blocks * groups <= TRUNK_DEEP_MOST_BLOCKS(window)) {
             if (window > most_shared_bytes) {
                 break;
             }

@@ -245,7 +245,7 @@ struct wide_chain {
         }
     }
 
-    /* The same for a launch whose blocks are so few that each has a CU to itself: a step there is as long as memory takes to answer what
+    /* The same for a launch whose blocks are so few that a CU has one or two of them: a step there is as long as memory takes to answer what
      * was asked for a step before, so that STAGES - 1 steps are on their way, and the columns' scale words all from the start. A
      * wavefront brings columns where its two groups are live. */
     template <uint32_t LIVE>

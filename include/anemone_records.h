@@ -638,7 +638,9 @@ ANEMONE_RECORD_HAS(expert_down_arguments, 56);
 #define TRUNK_DEEP_STAGES(rows) ((rows) < 64u ? 5u : 4u)
 #define TRUNK_DEEP_WINDOW_BYTES(inputs, rows) (TRUNK_DEEP_STAGES(rows) * (8448u + (rows) * 128u) + ((inputs) + 511u) / 512u * ((rows) * 16u))
 #define TRUNK_DEEP_MOST_INPUTS 16384u
-#define TRUNK_DEEP_MOST_BLOCKS 512u /* two a CU */
+/* blocks of a window that have a place at once on the 256 CUs: two a CU, one where a CU's 160 KB hold one window alone (64 rows of more than
+ * 7,680 inputs) */
+#define TRUNK_DEEP_MOST_BLOCKS(window) ((window) <= 80u * 1024u ? 512u : 256u)
 #define MODEL_STREAMS 4u
 #define HYPER_VALUES_PER_THREAD 8u /* one 16-byte load of bfloat16 */
 #define HYPER_PIECE_THREADS 128u

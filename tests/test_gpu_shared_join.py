@@ -150,7 +150,8 @@ def test_wide_and_interleaved_instances_have_the_thin_bits(amd, card, slices, ro
 
 @pytest.mark.parametrize("hidden,inner,rows,of", [
     (128, 160, 9, 16), (640, 1056, 33, 16), (768, 64, 16, 16), (4224, 160, 65, 16), (512, 96, 31, 16), (1024, 1056, 475, 32),
-    (512, 2048, 256, 32), (512, 2048, 257, 64), (384, 2048, 512, 64), (512, 2048, 513, 0)])
+    (512, 2048, 256, 32), (512, 2048, 257, 64), (384, 2048, 512, 64), (512, 2048, 513, 0),
+    (4736, 160, 2000, 32), (8192, 160, 513, 16), (16384, 672, 500, 32), (7680, 2048, 512, 64), (8192, 2048, 512, 0)])
 def test_instances_for_launches_of_few_blocks_have_the_wide_bits(amd, card, hidden, inner, rows, of):
     """One step, fewer steps than are on their way, steps and tiles that do not divide, every instance at its last row and block."""
     say("trunk forms of few blocks, hidden", hidden, "inner", inner, "rows", rows)

@@ -48,6 +48,16 @@ def test_blocks_of_the_fewest_rows_that_all_have_a_place(rows, of, groups, windo
     assert rule(product(rows, 4096, 4096), window - 1) == NONE  # the card grants a block less
 
 
+@pytest.mark.parametrize("inputs", [4096, 7680, 7808, 8192, 16384])
+def test_places_are_those_of_the_window(inputs):
+    """A CU's 160 KB hold two windows of 64 rows up to 7680 inputs, above them one: 257 to 512 blocks would be two rounds. Two of 32
+    and of 16 rows at any inputs."""
+    assert rule(product(512, inputs, 2048)) == (32, [32, 16], 62720 + (inputs + 511) // 512 * 512)
+    for rows, blocks in ((513, 32), (1024, 32), (1024, 17)):
+        whole = (64, [blocks, (rows + 63) // 64], 66560 + (inputs + 511) // 512 * 1024)
+        assert rule(product(rows, inputs, 64 * blocks)) == (whole if inputs <= 7680 else NONE)
+
+
 def test_ragged_products():
     assert rule(product(9, 128, 160, 32)) == (16, [4, 1], 5 * 10496 + 256)
     assert rule(product(33, 640, 1056)) == (16, [17, 3], 5 * 10496 + 512)
