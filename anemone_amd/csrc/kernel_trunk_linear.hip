@@ -163,7 +163,9 @@ __device__ static __forceinline__ void trunk_linear_quantized_interleaved(const 
     const uint32_t scale_column = 16u * wave + lane / 4u;
     const uint32_t exponent_vector = first_row + (scale_column < row_count ? scale_column : 0u);
     chain_type chain_of;
-    chain_of.once = arguments.row_count <= TRUNK_INTERLEAVED_ROWS;
+    if constexpr (!chain_type::DEEP) {
+        chain_of.once = arguments.row_count <= TRUNK_INTERLEAVED_ROWS;
+    }
     const unsigned char *const matrices[1] = {arena + arguments.weights_offset[matrix]};
     uint32_t tile0 = 0;
     chain_of.place(matrices, outputs, arguments.input_size, block, arena + arguments.codes_offset, arena + arguments.exponents_offset,

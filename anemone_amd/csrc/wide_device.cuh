@@ -247,7 +247,8 @@ struct wide_chain {
 
     /* The same for a launch whose blocks are so few that a CU has one or two of them: a step there is as long as memory takes to answer what
      * was asked for a step before, so that STAGES - 1 steps are on their way, and the columns' scale words all from the start. A
-     * wavefront brings columns where its two groups are live. */
+     * wavefront brings columns where its two groups are live. The weights are asked for through the caches, also where one tile of
+     * rows is all there is (`once` is not read): as a stream has not been measured here. */
     template <uint32_t LIVE>
     __device__ __forceinline__ void deep_steps(uint32_t total, float4_t (&chain)[TILES][WIDE_COLUMN_BLOCKS]) const
     {
