@@ -12,6 +12,14 @@ namespace {
 
 constexpr uint32_t ROUTER_BLOCK = 512u;       /* threads of the router's launches that are joined, and of their joined kernels */
 constexpr uint32_t QUANTIZE_UNIT = 64u, QUANTIZE_128_UNIT = 128u; /* widths of activation_quantize_entry, _128_entry: multiples */
+/* Values that a router's last launch and the quantizer of the rows are joined for. Beside the place launch a quantizer's block holds that
+ * launch's LDS too, so that a CU has three of them: the quantizer alone is bound by memory, joined it takes longer the more values there
+ * are. Back to back, us, place + quantizer -> joined. 32 values a scale, 256 experts and 8 picks: 16 Mi values 25.1 -> 16.7, 32 Mi 38.2 -> 30.1,
+ * 40 Mi 43.8 -> 36.7, 64 Mi 77.7 -> 78.7 and 78.0 -> 81.3, 128 Mi 142.8 -> 153.9; 64 experts and one pick, 32 Mi 31.4 -> 29.4, 128 Mi 130.2 ->
+ * 152.1. A float32 scale: 16 Mi 25.9 -> 19.9, 24 Mi 31.8 -> 28.0, 32 Mi 38.6 -> 36.4, 40 Mi 44.6 -> 45.8, 64 Mi 63.3 -> 72.1; 128 experts and 6
+ * picks, 24 Mi 30.5 -> 28.0, 32 Mi 36.0 -> 36.4; one pick, 8 Mi 12.9 -> 10.4, 16 Mi 19.4 -> 19.6, 24 Mi 24.9 -> 27.5, 128 Mi 123.6 -> 182.0 */
+constexpr uint64_t MOST_VALUES = 40u << 20, MOST_VALUES_128 = 24u << 20, MOST_VALUES_128_FEW_PICKS = 16u << 20;
+constexpr uint32_t FEW_PICKS = 4u; /* fewer */
 constexpr uint32_t MOST_GRID_ROWS = 65534u;
 constexpr uint32_t MOST_BLOCKS = 1u << 22;    /* of 512 threads: the runtime counts a grid's threads in 32 bits */
 
@@ -107,7 +115,8 @@ bool join_gate_up(const char *function, const struct kernel_launch &first, const
 bool join_router(const char *function, const char *second_function, const struct kernel_launch &first, const struct kernel_launch &second, uint64_t arena_bytes,
                  struct joined_launch &out)
 {
-    const uint32_t unit = std::strcmp(second_function, KERNEL_ACTIVATION_QUANTIZE_128) == 0 ? QUANTIZE_128_UNIT : QUANTIZE_UNIT;
+    const bool wide_scales = std::strcmp(second_function, KERNEL_ACTIVATION_QUANTIZE_128) == 0;
+    const uint32_t unit = wide_scales ? QUANTIZE_128_UNIT : QUANTIZE_UNIT;
     const auto quantize = record_of<activation_quantize_arguments>(second);
     if (!is_plain(first, ROUTER_BLOCK) || first.grid[1] != 1 || !quantizer_is_whole(second, quantize, unit, arena_bytes)) {
         return false;
@@ -116,10 +125,15 @@ bool join_router(const char *function, const char *second_function, const struct
     const byte_range read[] = {{quantize.values_offset, 2u * values}};
     /* the quantizer of 128 values a scale writes no operands: they are kept apart all the same */
     const byte_range written[] = {{quantize.codes_offset, values}, {quantize.exponents_offset, values / 32u}, {quantize.operands_offset, 2u * values}};
-    if (std::strcmp(function, KERNEL_ROUTER_SELECT) == 0) {
+    const bool is_select = std::strcmp(function, KERNEL_ROUTER_SELECT) == 0;
+    const uint32_t pick_count = is_select ? record_of<router_select_arguments>(first).pick_count : record_of<router_wide_arguments>(first).pick_count;
+    const uint64_t picks = pick_count != 0 ? pick_count : ROUTER_DEFAULT_PICKS;
+    if (values > (!wide_scales ? MOST_VALUES : picks < FEW_PICKS ? MOST_VALUES_128_FEW_PICKS : MOST_VALUES_128)) {
+        return false;
+    }
+    if (is_select) {
         const auto select = record_of<router_select_arguments>(first);
         const uint64_t experts = select.expert_count != 0 ? select.expert_count : ROUTER_DEFAULT_EXPERTS, rows = select.row_count;
-        const uint64_t picks = select.pick_count != 0 ? select.pick_count : ROUTER_DEFAULT_PICKS;
         const byte_range inputs[] = {{select.step_offset, sizeof(struct step_block)}, {select.scores_offset, rows * experts * 4u},
                                      {select.bias_offset, experts * 4u}, {select.expert_offsets_offset, experts * MODEL_EXPERT_MATRICES * 8u}};
         const byte_range outputs[] = {{select.affinities_offset, rows * experts * 4u}, {select.jobs_offset, rows * picks * sizeof(struct expert_job_record)}};
@@ -129,7 +143,7 @@ bool join_router(const char *function, const char *second_function, const struct
     } else {
         const auto wide = record_of<router_wide_arguments>(first);
         const uint64_t experts = wide.expert_count != 0 ? wide.expert_count : ROUTER_DEFAULT_EXPERTS, rows = wide.row_count;
-        const uint64_t picks = wide.pick_count != 0 ? wide.pick_count : ROUTER_DEFAULT_PICKS, pairs = rows * picks;
+        const uint64_t pairs = rows * picks;
         const byte_range inputs[] = {{wide.step_offset, sizeof(struct step_block)},
                                      {wide.expert_offsets_offset, experts * MODEL_EXPERT_MATRICES * 8u},
                                      {wide.picks_offset, pairs * sizeof(struct router_pick)},

@@ -961,7 +961,9 @@ ANEMONE_KERNEL(KERNEL_FILE_ROUTER, router_wide_small, router_wide_arguments);
 /* ---- a router's last launch and the quantizer of the step's rows behind it, as one launch ----------------------
  * Neither reads what the other writes, and the router's is one block, or one for 384 rows: the first `blocks` blocks are its, the
  * others two of the quantizer's blocks each. The backend runs the pair so where it stands in a list (joined_launches.h, with
- * what that measured). Bound by the router's block, or by the quantizer's bytes where the rows are many. */
+ * what that measured). Bound by the router's block, or by the quantizer's where the rows are many: each of
+ * them holds the router's LDS as well (place 51 KB, small 74 KB), so that a CU has three or two, and 8192 rows of 4096 take 30 us, the quantizer
+ * alone 25.5 (the rule stops joining where that costs more than a launch). */
 #define QUANTIZE_JOIN_BLOCKS (WIDE_SORT_THREADS / LINEAR_ELEMENT_THREADS)
 static_assert(SELECT_THREADS == WIDE_SORT_THREADS, "one block size");
 

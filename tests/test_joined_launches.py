@@ -45,12 +45,12 @@ WIDE = {"step": (0, 16, False), "expert_offsets": (3, E * 24, False), "picks": (
         "pairs": (7, ROWS * P * 8, True), "runs": (8, E * 8, True), "tiles": (9, TILES * 32, True), "jobs": (10, JOBS * 96, True)}
 
 
-def router(name, **places):
+def router(name, pick_count=P, **places):
     wide = name != "router_select_entry"
     members = [(16 + i) * STEP for i in range(14 if wide else 9)]
     for member, place in places.items():
         members[(WIDE if wide else SELECT)[member][0]] = place
-    return launch((1, 1, 1), 512, struct.pack("<%dQ5If" % len(members), *members, ROWS, 0, E, P, 0, 1.5))
+    return launch((1, 1, 1), 512, struct.pack("<%dQ5If" % len(members), *members, ROWS, 0, E, pick_count, 0, 1.5))
 
 
 @pytest.mark.parametrize("name", ["router_select_entry", "router_wide_small", "router_wide_place"])
@@ -181,3 +181,16 @@ def test_every_joined_kernel_is_registered():
     want += [(name, "activation_quantize_entry", name + "_joined")
              for infix in ("", "e4m3_", "gfx950_", "e4m3_gfx950_") for slices in (1, 2, 4, 8) for name in ["expert_gate_up_%s%d" % (infix, slices)]]
     assert sorted(joined) == sorted(want)
+
+
+@pytest.mark.parametrize("quantize,picks,most", [("", 1, 40), ("", 8, 40), ("_128", 1, 16), ("_128", 3, 16), ("_128", 4, 24), ("_128", 0, 24)])
+def test_router_and_quantizer_of_many_values(quantize, picks, most):
+    """Many values: beside the place launch's LDS the quantizer takes longer than by itself and a launch more."""
+    def joins(width, rows):
+        places = {name: (i + 1) << 33 for i, name in enumerate(("values", "codes", "exponents", "operands"))}
+        second = quantizer(width=width, rows=rows, **places)
+        return rule(name, router(name, pick_count=picks), second, arena=1 << 40, quantize="activation_quantize%s_entry" % quantize) is not None
+    for name in ("router_select_entry", "router_wide_small", "router_wide_place"):
+        for width in (1024, 4096):
+            rows = (most << 20) // width
+            assert joins(width, rows) and not joins(width, rows + 1)
