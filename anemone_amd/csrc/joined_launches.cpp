@@ -84,6 +84,21 @@ bool join_hidden(const struct kernel_launch &first, const struct kernel_launch &
     return true;
 }
 
+/* The most blocks of gate and up that are joined with the quantizer. A block's quantizing stands behind its own product: while the card
+ * is not full of blocks that costs less than the launch it saves, with many short ones it holds places that others wait for. 8 picks, 128
+ * experts, us, gate and up + quantizer -> joined. 4-bit, 4 K steps a slice (2048 x 2048, four slices): 1024 blocks 25.1 -> 24.1, 1280 28.7 -> 29.3,
+ * 2048 38.9 -> 41.2; 8 steps (4096 x 2048): 1280 45.7 -> 44.4, 2048 71.6 -> 69.5, in gfx950's order 71.8 -> 69.7. One byte, 4 steps: 1536 blocks
+ * 32.6 -> 32.0, 2048 40.7 -> 41.0, 4096 70.6 -> 72.3; 8 steps: 1536 59.8 -> 58.5, 4096 142.7 -> 142.1; in gfx950's order 1536 56.7 -> 55.2, 2048
+ * 71.5 -> 72.3, 4096 129.0 -> 130.3; one slice of 32 steps: 1536 60.4 -> 58.9, 2048 75.7 -> 80.3, 4096 116.7 -> 123.0 */
+uint64_t most_gate_up_blocks(bool one_byte, bool native, uint32_t slices, uint32_t slice_steps)
+{
+    const bool is_long = slice_steps >= 8u;
+    if (!one_byte) {
+        return is_long ? 2048u : 1024u;
+    }
+    return is_long && !native && slices > 1u ? 4096u : 1536u;
+}
+
 bool join_gate_up(const char *function, const struct kernel_launch &first, const struct kernel_launch &second, uint64_t arena_bytes,
                   struct joined_launch &out)
 {
@@ -91,12 +106,13 @@ bool join_gate_up(const char *function, const struct kernel_launch &first, const
     const auto quantize = record_of<activation_quantize_arguments>(second);
     /* expert_gate_up_[e4m3_][gfx950_]<S>: the weights' bytes and the slices, a wavefront each */
     const char *const form = function + sizeof KERNEL_EXPERT_GATE_UP_STEM - 1u;
-    const uint32_t strip = EXPERT_STRIP_OUTPUTS(std::strncmp(form, "e4m3_", 5) == 0);
-    const uint32_t block = 64u * (uint32_t)std::strtoul(std::strrchr(function, '_') + 1, nullptr, 10);
+    const bool one_byte = std::strncmp(form, "e4m3_", 5) == 0, native = std::strstr(form, "gfx950_") != nullptr;
+    const uint32_t strip = EXPERT_STRIP_OUTPUTS(one_byte), slices = (uint32_t)std::strtoul(std::strrchr(function, '_') + 1, nullptr, 10);
     /* a block quantizes the outputs of its own strip alone: there is one for every strip */
-    if (!is_plain(first, block) || gate_up.output_size % strip != 0 || first.grid[0] != gate_up.output_size / strip ||
+    if (slices == 0 || !is_plain(first, 64u * slices) || gate_up.output_size % strip != 0 || first.grid[0] != gate_up.output_size / strip ||
         !quantizer_is_whole(second, quantize, QUANTIZE_UNIT, arena_bytes) || gate_up.output_size != quantize.width || gate_up.hidden_offset != quantize.values_offset || gate_up.pair_count != second.grid[1] ||
-        gate_up.pair_count > EXPERT_JOINED_MOST_PAIRS || gate_up.pairs_per_row == 0 || gate_up.input_size > arena_bytes || first.grid[1] > MOST_GRID_ROWS) {
+        gate_up.pair_count > EXPERT_JOINED_MOST_PAIRS || gate_up.pairs_per_row == 0 || gate_up.input_size > arena_bytes || first.grid[1] > MOST_GRID_ROWS ||
+        (uint64_t)first.grid[0] * first.grid[1] > most_gate_up_blocks(one_byte, native, slices, gate_up.input_size / 128u / slices)) {
         return false;
     }
     const uint64_t values = (uint64_t)second.grid[1] * quantize.width, jobs = first.grid[1];
@@ -108,7 +124,7 @@ bool join_gate_up(const char *function, const struct kernel_launch &first, const
     if (!all_apart(outputs, read) || !all_apart(outputs, own) || !all_apart(read, own)) {
         return false;
     }
-    out = {{first.grid[0], (uint32_t)jobs + 1u}, block, {(uint32_t)jobs, 0, 0}};
+    out = {{first.grid[0], (uint32_t)jobs + 1u}, 64u * slices, {(uint32_t)jobs, 0, 0}};
     return true;
 }
 

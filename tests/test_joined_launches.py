@@ -194,3 +194,16 @@ def test_router_and_quantizer_of_many_values(quantize, picks, most):
         for width in (1024, 4096):
             rows = (most << 20) // width
             assert joins(width, rows) and not joins(width, rows + 1)
+
+
+@pytest.mark.parametrize("name,strip,inputs,most", [
+    ("expert_gate_up_4", 64, 3968, 1024), ("expert_gate_up_4", 64, 4096, 2048), ("expert_gate_up_gfx950_8", 64, 8192, 2048), ("expert_gate_up_8", 64, 4096, 1024),
+    ("expert_gate_up_1", 64, 1024, 2048), ("expert_gate_up_e4m3_4", 32, 3968, 1536), ("expert_gate_up_e4m3_4", 32, 4096, 4096),
+    ("expert_gate_up_e4m3_1", 32, 4096, 1536), ("expert_gate_up_e4m3_gfx950_4", 32, 4096, 1536)])
+def test_gate_up_of_many_blocks(name, strip, inputs, most):
+    """Many short blocks: quantizing behind each costs more than the launch."""
+    slices = int(name[-1])
+    for pairs in (32, 64):
+        for width, joins in ((most // pairs * strip, True), (most // pairs * strip + 64, False)):
+            places = dict(out=STEP, width=width, inputs=inputs, pairs=pairs, picks=8, job_count=pairs, strip=strip, block=64 * slices)
+            assert (rule(name, whole_gate_up(**places), quantizer(width=width, rows=pairs)) is not None) == joins, (pairs, width)
