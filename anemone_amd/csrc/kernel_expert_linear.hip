@@ -435,17 +435,22 @@ __device__ static __forceinline__ void joined_gate_up_quantize(const struct expe
     if (job->row_count == 0u) {
         return;
     }
+    uint32_t vectors = 0; /* a bit a column whose pair is a vector of the quantizer's; a table may name others */
+#pragma unroll
+    for (uint32_t column = 0; column < LINEAR_MAXIMUM_ROWS; column++) {
+        vectors |= job->pair_index[column] < arguments.pair_count ? 1u << column : 0u;
+    }
     expert_gate_up<S, BYTES, false, NATIVE>(arguments, arena, &strip_hidden[0][0]);
     __syncthreads();
     for (uint32_t index = threadIdx.x; index < job->row_count * VECTOR_THREADS; index += THREADS) {
-        const uint32_t column = index / VECTOR_THREADS, q = first_q + index % VECTOR_THREADS, pair = job->pair_index[column];
-        if (pair >= arguments.pair_count) {
-            continue; /* no vector of the quantizer's */
+        const uint32_t column = index / VECTOR_THREADS, q = first_q + index % VECTOR_THREADS;
+        if (((vectors >> column) & 1u) == 0u) {
+            continue;
         }
         const uint16_t *values = &strip_hidden[column][quantize_first_of(q) - first_output];
         const uint32_t near_pair = *(const uint32_t *)values, far_pair = *(const uint32_t *)(values + 8);
         const uint32_t bits[4] = {near_pair & 0xFFFFu, near_pair >> 16, far_pair & 0xFFFFu, far_pair >> 16};
-        activation_quantize_values(quantize, arena, q, pair, bits);
+        activation_quantize_values(quantize, arena, q, job->pair_index[column], bits);
     }
 }
 
