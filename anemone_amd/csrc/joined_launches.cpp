@@ -110,15 +110,16 @@ bool join_gate_up(const char *function, const struct kernel_launch &first, const
     const uint32_t strip = EXPERT_STRIP_OUTPUTS(one_byte), slices = (uint32_t)std::strtoul(std::strrchr(function, '_') + 1, nullptr, 10);
     /* a block quantizes the outputs of its own strip alone: there is one for every strip */
     if (slices == 0 || !is_plain(first, 64u * slices) || gate_up.output_size % strip != 0 || first.grid[0] != gate_up.output_size / strip ||
-        !quantizer_is_whole(second, quantize, QUANTIZE_UNIT, arena_bytes) || gate_up.output_size != quantize.width || gate_up.hidden_offset != quantize.values_offset || gate_up.pair_count != second.grid[1] ||
-        gate_up.pair_count > EXPERT_JOINED_MOST_PAIRS || gate_up.pairs_per_row == 0 || gate_up.input_size > arena_bytes || first.grid[1] > MOST_GRID_ROWS ||
+        !quantizer_is_whole(second, quantize, QUANTIZE_UNIT, arena_bytes) || gate_up.output_size != quantize.width ||
+        gate_up.hidden_offset != quantize.values_offset || gate_up.pair_count != second.grid[1] || gate_up.pair_count > EXPERT_JOINED_MOST_PAIRS ||
+        gate_up.pairs_per_row == 0 || gate_up.input_size > arena_bytes || first.grid[1] > MOST_GRID_ROWS ||
         (uint64_t)first.grid[0] * first.grid[1] > most_gate_up_blocks(one_byte, native, slices, gate_up.input_size / 128u / slices)) {
         return false;
     }
     const uint64_t values = (uint64_t)second.grid[1] * quantize.width, jobs = first.grid[1];
     const uint64_t inputs = ((uint64_t)gate_up.pair_count + gate_up.pairs_per_row - 1u) / gate_up.pairs_per_row * gate_up.input_size;
     const byte_range outputs[] = {{quantize.codes_offset, values}, {quantize.exponents_offset, values / 32u}, {quantize.operands_offset, 2u * values}};
-    /* the matrices, which the jobs name, are nobody's output */
+    /* the matrices, which the jobs name, are nobody's output (joined_launches.h) */
     const byte_range read[] = {{gate_up.jobs_offset, jobs * sizeof(struct expert_job_record)}, {gate_up.codes_offset, inputs}, {gate_up.exponents_offset, inputs / 32u}};
     const byte_range own[] = {{gate_up.hidden_offset, 2u * values}};
     if (!all_apart(outputs, read) || !all_apart(outputs, own) || !all_apart(read, own)) {

@@ -7,9 +7,12 @@
  *   the shared expert's hidden step, then the quantizer of its values                  the one's values are the other's, a thread both
  *
  * Every byte that the two launches write is written, with the same value. A pair whose records do not show by themselves that this is
- * so stays two launches. A launch costs 1.3 to 1.7 us of a queue beside its work, and the router's last launch is one block, or one for
- * 384 rows, that leaves the card to the quantizer. A pass, before -> after: one row of float32-scaled FP8 50.6 -> 49.0 us, one row
- * of smaller layers 30.5 -> 28.8 and 36.2 -> 34.8, 2048 rows of FP8 1362 -> 1352, 8192 of FP4 1998 -> 1973, a site's five rows 114.9 -> 114.2.
+ * so stays two launches, and so does a pair so large that one kernel for both is the slower (joined_launches.cpp, with both sides'
+ * times). What no record shows, the matrices that the experts' job table names, is taken to be nobody's output:
+ * linear_routed_experts_prepare refuses ranges that share a byte with them. A launch costs 1.3 to 1.7 us of a queue beside its work, and
+ * the router's last launch is one block, or one for 384 rows, that leaves the card to the quantizer. Back to back, us, two -> one: select
+ * and quantizer of one row 6.0 -> 4.1, small of 64 rows 7.0 -> 5.1, place of 2048 rows 18.2 -> 14.3, of 8192 38.2 -> 30.1; hidden and
+ * quantizer of one row 4.5 -> 2.3, of 8192 35.3 -> 27.2; gate and up and quantizer of 8 pairs of FP4 14.6 -> 12.8, of 64 71.6 -> 69.5.
  */
 #ifndef JOINED_LAUNCHES_H
 #define JOINED_LAUNCHES_H

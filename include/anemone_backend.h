@@ -98,7 +98,9 @@ struct device_card;
  * SIDE_MORE is another side run, of one launch, behind the same fork; RESUME stands behind the fork, not the side runs;
  * JOIN behind the launch before it and every side run's last. A list's first launch may open a side run: its fork is
  * then the graph's root. launch_run runs a list in its serial order whatever the branches say. A list's neighbours
- * that one kernel can do are queued as one launch, there and in a graph; launch_run_timed runs every launch by itself. */
+ * that one kernel can do are queued as one launch, there and in a graph, where their records show that neither touches what the
+ * other writes (the experts' matrices stand in a job table, not in a record: the quantizer behind gate and up may not write over them,
+ * a list that the prepare functions refuse too); launch_run_timed runs every launch by itself. */
 #define LAUNCH_CHAIN 0u
 #define LAUNCH_SIDE 1u
 #define LAUNCH_RESUME 2u
